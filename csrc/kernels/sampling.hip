@@ -24,27 +24,32 @@ template <typename T> __device__ __forceinline__ float ld1(const T* p);
 template <> __device__ __forceinline__ float ld1<bf16_t>(const bf16_t* p) { return bf2f(*p); }
 template <> __device__ __forceinline__ float ld1<float>(const float* p) { return *p; }
 
-template <typename T>
-__global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logits, long ld, int V, float inv_temp,
-                                                     int top_k, float top_p, int greedy, uint64_t seed,
-                                                     const int64_t* __restrict__ offset_ptr,
-                                                     const uint8_t* __restrict__ row_active, long* __restrict__ out_tok,
-                                                     float* __restrict__ out_logp) {
-  __shared__ float hist_f[256];
-  __shared__ unsigned hist_c[256];
-  __shared__ float redf[8];
-  __shared__ int redi[8];
-  __shared__ uint32_t sh_key;
-  __shared__ float sh_f;
+struct SampleShared {
+  float hist_f[256];
+  unsigned hist_c[256];
+  float redf[16];
+  int redi[16];
+  uint32_t key;
+  float f;
+};
 
-  const long row = blockIdx.x;
-  const T* x = logits + row * ld;
+// one row by NT threads: radix-select thresholds over the row as it lies in memory, any V and stride
+template <typename T, int NT>
+__device__ void sample_row(const T* x, long row, int V, float inv_temp, int top_k, float top_p, int greedy, uint64_t seed,
+                           const int64_t* __restrict__ offset_ptr, const uint8_t* __restrict__ row_active,
+                           long* __restrict__ out_tok, float* __restrict__ out_logp, SampleShared& sh) {
+  float* hist_f = sh.hist_f;
+  unsigned* hist_c = sh.hist_c;
+  float* redf = sh.redf;
+  int* redi = sh.redi;
+  uint32_t& sh_key = sh.key;
+  float& sh_f = sh.f;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
 
   // pass 1: max of tempered logits (and argmax for greedy)
   float mx = -INFINITY;
   int amx = 0;
-  for (int i = tid; i < V; i += 256) {
+  for (int i = tid; i < V; i += NT) {
     const float f = ld1<T>(x + i) * inv_temp;
     if (f > mx) { mx = f; amx = i; }
   }
@@ -58,12 +63,12 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
   __syncthreads();
   float M = redf[0];
   int AM = redi[0];
-  for (int w = 1; w < 4; ++w)
+  for (int w = 1; w < NT / 64; ++w)
     if (redf[w] > M || (redf[w] == M && redi[w] < AM)) { M = redf[w]; AM = redi[w]; }
   __syncthreads();
   // pass 2: sum of exp
   float s = 0.f;
-  for (int i = tid; i < V; i += 256) s += __expf(ld1<T>(x + i) * inv_temp - M);
+  for (int i = tid; i < V; i += NT) s += __expf(ld1<T>(x + i) * inv_temp - M);
   const float S = block_sum(s, redf);
   const float lse = M + __logf(S);
 
@@ -76,9 +81,9 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
       uint32_t prefix = 0, mask = 0;
       unsigned remaining = top_k;
       for (int shift = 24; shift >= 0; shift -= 8) {
-        hist_c[tid] = 0;
+        if (tid < 256) hist_c[tid] = 0;
         __syncthreads();
-        for (int i = tid; i < V; i += 256) {
+        for (int i = tid; i < V; i += NT) {
           const uint32_t k = fkey(ld1<T>(x + i));
           if ((k & mask) == prefix) atomicAdd(&hist_c[(k >> shift) & 255], 1u);
         }
@@ -104,7 +109,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
     uint32_t pth = kth;
     if (top_p < 1.f) {
       float sk = 0.f;
-      for (int i = tid; i < V; i += 256) {
+      for (int i = tid; i < V; i += NT) {
         const float f = ld1<T>(x + i);
         if (fkey(f) >= kth) sk += __expf(f * inv_temp - M);
       }
@@ -113,9 +118,9 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
       uint32_t prefix = 0, mask = 0;
       float above = 0.f;
       for (int shift = 24; shift >= 0; shift -= 8) {
-        hist_f[tid] = 0.f;
+        if (tid < 256) hist_f[tid] = 0.f;
         __syncthreads();
-        for (int i = tid; i < V; i += 256) {
+        for (int i = tid; i < V; i += NT) {
           const float f = ld1<T>(x + i);
           const uint32_t k = fkey(f);
           if (k >= kth && (k & mask) == prefix) atomicAdd(&hist_f[(k >> shift) & 255], __expf(f * inv_temp - M));
@@ -143,7 +148,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
     const uint64_t off = offset_ptr ? (uint64_t)offset_ptr[0] : 0ull;
     float best = -INFINITY;
     int bi = AM;
-    for (int i = tid; i < V; i += 256) {
+    for (int i = tid; i < V; i += NT) {
       const float f = ld1<T>(x + i);
       if (fkey(f) >= pth) {
         const uint4 r = Philox::gen(seed, (uint64_t)row, off * (uint64_t)V + (uint64_t)i);
@@ -165,7 +170,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
     if (tid == 0) {
       float B = redf[0];
       int BI = redi[0];
-      for (int w = 1; w < 4; ++w)
+      for (int w = 1; w < NT / 64; ++w)
         if (redf[w] > B || (redf[w] == B && redi[w] < BI)) { B = redf[w]; BI = redi[w]; }
       redi[0] = BI;
     }
@@ -176,6 +181,17 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
     out_tok[row] = tok;
     if (out_logp) out_logp[row] = ld1<T>(x + tok) * inv_temp - lse;
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logits, long ld, int V, float inv_temp,
+                                                     int top_k, float top_p, int greedy, uint64_t seed,
+                                                     const int64_t* __restrict__ offset_ptr,
+                                                     const uint8_t* __restrict__ row_active, long* __restrict__ out_tok,
+                                                     float* __restrict__ out_logp) {
+  __shared__ SampleShared sh;
+  sample_row<T, 256>(logits + blockIdx.x * ld, blockIdx.x, V, inv_temp, top_k, top_p, greedy, seed, offset_ptr, row_active,
+                     out_tok, out_logp, sh);
 }
 
 
@@ -866,6 +882,193 @@ __global__ __launch_bounds__(1024) void sample_topk_search_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// top-k (+ top-p) sampler for fp32 logits, one 1024-thread workgroup per row
+// ---------------------------------------------------------------------------------------------
+// Bound by latency: the row (128 KB at V = 32000) passes one CU once, in 16-byte loads that all are in flight
+// together, and stays in registers (RV chunks a thread; what lies beyond is read again from L2). The k-th largest
+// of the 1024 threads' own maxima is a lower bound of the row's k-th largest logit that hardly any surplus
+// elements reach, whatever the logits' distribution: those that do (about K + K^2 / 2048) are the candidates, and
+// one wave finds the exact threshold among them with ballots instead of 4 histogram passes over the row. Same kept
+// set and same Philox stream (seed, row, offset * V + token) as sample_row, which takes the rows whose candidates
+// do not fit (plateaus of equal logits). V = 32000, top-k 50: 16 rows 177 -> 22 us, 64 rows 173 -> 23 us.
+constexpr int F32_RV = 8, F32_CAP = 1024, F32_TOPK = 256;
+
+// largest t such that at least K of the n (<= 64 * R) keys are >= t; the keys lie R to a lane, absent ones are 0.
+// Every lane of the wave returns it.
+template <int R>
+__device__ __forceinline__ uint32_t wave_kth(const uint32_t (&k)[R], int K) {
+  uint32_t t = 0;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t cnd = t | (1u << b);
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) c += (int)__popcll(__ballot(k[i] >= cnd));
+    if (c >= K) t = cnd;
+  }
+  return t;
+}
+
+__global__ __launch_bounds__(1024) void sample_topk_f32_kernel(
+    const float* __restrict__ logits, long ld, int V, float inv_temp, int top_k, float top_p, uint64_t seed,
+    const int64_t* __restrict__ offset_ptr, const uint8_t* __restrict__ row_active, long* __restrict__ out_tok,
+    float* __restrict__ out_logp) {
+  __shared__ uint32_t tmax[1024];
+  __shared__ uint32_t ckey[F32_CAP];
+  __shared__ int cidx[F32_CAP];
+  __shared__ float redf[16], redi_f[16];
+  __shared__ int redi[16];
+  __shared__ uint32_t thr;
+  __shared__ SampleShared sh;
+  const long row = blockIdx.x;
+  const float* x = logits + row * ld;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nv = V / 4;
+
+  float4 v[F32_RV];
+#pragma unroll
+  for (int i = 0; i < F32_RV; ++i) {
+    const int c = tid + i * 1024;
+    v[i] = c < nv ? *(const float4*)(x + (long)c * 4) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  }
+  // f(value, index) over this thread's elements, in index order
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int i = 0; i < F32_RV; ++i) {
+      const int c = tid + i * 1024;
+      if (c < nv) { f(v[i].x, c * 4); f(v[i].y, c * 4 + 1); f(v[i].z, c * 4 + 2); f(v[i].w, c * 4 + 3); }
+    }
+    for (int c = tid + F32_RV * 1024; c < nv; c += 1024) {
+      const float4 w = *(const float4*)(x + (long)c * 4);
+      f(w.x, c * 4); f(w.y, c * 4 + 1); f(w.z, c * 4 + 2); f(w.w, c * 4 + 3);
+    }
+  };
+  float mx = -INFINITY;
+  int amx = 0;
+  uint32_t km = 0;
+  each([&](float f, int i) {
+    const float t = f * inv_temp;
+    if (t > mx) { mx = t; amx = i; }
+    km = max(km, fkey(f));
+  });
+  tmax[tid] = km;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float om = __shfl_xor(mx, off, 64);
+    const int oi = __shfl_xor(amx, off, 64);
+    if (om > mx || (om == mx && oi < amx)) { mx = om; amx = oi; }
+  }
+  if (lane == 0) { redf[wid] = mx; redi[wid] = amx; }
+  __syncthreads();
+  float M = redf[0];
+  int AM = redi[0];
+#pragma unroll
+  for (int w = 1; w < 16; ++w)
+    if (redf[w] > M || (redf[w] == M && redi[w] < AM)) { M = redf[w]; AM = redi[w]; }
+  float s = 0.f;
+  each([&](float f, int) { s += __expf(f * inv_temp - M); });
+  s = wave_sum_f(s);
+  if (lane == 0) redi_f[wid] = s;
+  const bool active = row_active ? row_active[row] != 0 : true;
+  const int K = min(top_k, V);
+  if (wid == 0 && active) {
+    uint32_t k[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) k[i] = tmax[lane + 64 * i];
+    const uint32_t t = wave_kth(k, K);
+    if (lane == 0) thr = t;
+  }
+  __syncthreads();
+  float S = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) S += redi_f[w];
+  const float lse = M + __logf(S);
+  if (!active) {
+    if (tid == 0) {
+      out_tok[row] = AM;
+      if (out_logp) out_logp[row] = x[AM] * inv_temp - lse;
+    }
+    return;
+  }
+  // candidates in a fixed order: counted, prefix-summed over the workgroup, placed. Most threads have none
+  const uint32_t lo = thr;
+  int n = 0;
+  if (km >= lo) each([&](float f, int) { n += fkey(f) >= lo; });
+  int incl = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += t;
+  }
+  if (lane == 63) redi[wid] = incl;  // AM was read by every wave before the barrier above
+  __syncthreads();
+  int at = incl - n, total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w < wid) at += redi[w];
+    total += redi[w];
+  }
+  if (total > F32_CAP) {
+    sample_row<float, 1024>(x, row, V, inv_temp, top_k, top_p, 0, seed, offset_ptr, row_active, out_tok, out_logp, sh);
+    return;
+  }
+  if (n) each([&](float f, int i) {
+    if (fkey(f) >= lo) { ckey[at] = fkey(f); cidx[at] = i; ++at; }
+  });
+  __syncthreads();
+  if (wid != 0) return;
+  // one wave: exact k-th key, nucleus cut, Gumbel draw
+  constexpr int R = F32_CAP / 64;
+  uint32_t kth = 0;
+  if (total <= 256) {
+    uint32_t k[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) k[i] = lane + 64 * i < total ? ckey[lane + 64 * i] : 0u;
+    kth = wave_kth(k, K);
+  } else {
+    uint32_t k[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) k[i] = lane + 64 * i < total ? ckey[lane + 64 * i] : 0u;
+    kth = wave_kth(k, K);
+  }
+  auto val = [](uint32_t k) { return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k); };
+  float target = 0.f;
+  if (top_p < 1.f) {
+    float sk = 0.f;
+    for (int j = lane; j < total; j += 64)
+      if (ckey[j] >= kth) sk += __expf(val(ckey[j]) * inv_temp - M);
+    target = top_p * wave_sum_f(sk);
+  }
+  const uint64_t off = offset_ptr ? (uint64_t)offset_ptr[0] : 0ull;
+  float best = -INFINITY;
+  int bi = AM;
+  for (int j = lane; j < total; j += 64) {
+    const uint32_t k = ckey[j];
+    bool keep = k >= kth;
+    if (keep && top_p < 1.f) {  // kept: the probability mass above this token stays short of the target
+      float above = 0.f;
+      for (int i = 0; i < total; ++i)
+        if (ckey[i] > k) above += __expf(val(ckey[i]) * inv_temp - M);
+      keep = above < target;
+    }
+    if (keep) {
+      const int i = cidx[j];
+      const uint4 r = Philox::gen(seed, (uint64_t)row, off * (uint64_t)V + (uint64_t)i);
+      const float sc = val(k) * inv_temp - __logf(-__logf(u32_to_unit(r.x)));
+      if (sc > best || (sc == best && i < bi)) { best = sc; bi = i; }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ob = __shfl_xor(best, o, 64);
+    const int oi = __shfl_xor(bi, o, 64);
+    if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+  }
+  if (lane == 0) {
+    out_tok[row] = bi;
+    if (out_logp) out_logp[row] = x[bi] * inv_temp - lse;
+  }
+}
+
 }  // namespace rt
 
 using namespace rt;
@@ -886,6 +1089,13 @@ extern "C" int rt_sample(const void* logits, int is_f32, long ld, long B, int V,
     const size_t shm = ((size_t)V * 2 + 15) / 16 * 16;
     hipLaunchKernelGGL(sample_bf16_lds_kernel, dim3(B), dim3(256), shm, stream, (const bf16_t*)logits, ld, V, inv_temp,
                        top_k, top_p, greedy, seed, offset_ptr, row_active, out_tok, out_logp);
+    RT_LAUNCH_CHECK();
+    return 0;
+  }
+  // top_k over F32_TOPK would bring too many surplus candidates (the general kernel takes 175 us whatever it is)
+  if (is_f32 && !greedy && top_k > 0 && top_k <= F32_TOPK && V % 4 == 0 && ld % 4 == 0 && (uintptr_t)logits % 16 == 0) {
+    hipLaunchKernelGGL(sample_topk_f32_kernel, dim3(B), dim3(1024), 0, stream, (const float*)logits, ld, V, inv_temp,
+                       top_k, top_p, seed, offset_ptr, row_active, out_tok, out_logp);
     RT_LAUNCH_CHECK();
     return 0;
   }
