@@ -66,7 +66,7 @@ int rt_attn_decode_fused(const void*, long, void*, void*, int, const int*, const
                          int, float, const float*, int, float*, float*, int, long long*, hipStream_t);
 int rt_attn_decode_fused_ps(int, int);
 int rt_kv_store_fp8(const void*, long, void*, void*, float*, float*, int, int, int, int, int, int, int, hipStream_t);
-int rt_attn_decode_mfma_ok(int, int, int, int, int);
+int rt_attn_decode_slabs_ok(int, int, int, int, int, int, int);
 int rt_attn_bwd(const void*, long, const void*, long, const void*, long, const void*, long, const void*, long,
                 const float*, float*, float*, void*, long, void*, long, void*, long, const int*, int, int, int, int,
                 int, int, int, float, const int*, const float*, const float*, hipStream_t);
@@ -113,6 +113,8 @@ struct TuningField {
 };
 static const TuningField kTuningFields[] = {
     {"decode_mw_bh", &rt::Tuning::decode_mw_bh, nullptr},
+    {"decode_w4_bh", &rt::Tuning::decode_w4_bh, nullptr},
+    {"decode_w4_smax", &rt::Tuning::decode_w4_smax, nullptr},
     {"attn_lpt", &rt::Tuning::attn_lpt, nullptr},
     {"decode_mw_kpp", &rt::Tuning::decode_mw_kpp, nullptr},
     {"decode_mw_smax", &rt::Tuning::decode_mw_smax, nullptr},
@@ -980,7 +982,8 @@ bool attn_decode_fused_slabs(const Tensor& slabs, int64_t nsplit, Tensor kc, Ten
   const int64_t B = kc.size(0), Hkv = kc.size(1), Smax = kc.size(2), D = kc.size(3);
   const int64_t NP = (Smax + PS - 1) / PS, G = Hq / Hkv;
   TORCH_CHECK(G * Hkv == Hq, "attn_decode_fused_slabs: Hq must be a multiple of Hkv");
-  if (!rt_attn_decode_mfma_ok((int)B, (int)Hq, (int)Hkv, (int)D, (int)NP)) return false;  // caller reduces first
+  if (!rt_attn_decode_slabs_ok((int)B, (int)Hq, (int)Hkv, (int)D, (int)Smax, (int)NP, ksc.has_value() && ksc->defined()))
+    return false;  // caller reduces first  // caller reduces first
   const int64_t W = (Hq + 2 * Hkv) * D;
   TORCH_CHECK(slabs.is_contiguous() && slabs.numel() >= nsplit * B * W && nsplit >= 1, "attn_decode_fused_slabs: slabs");
   TORCH_CHECK(out.size(0) == B && slot.numel() == B && attn_len.numel() == B && out.size(1) >= Hq * D,

@@ -1111,9 +1111,11 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 //   * O += P·V: 8 MFMAs (K = 32: k-slots 4..7 are P = 0 against zero LDS rows), P = the packed
 //     S^T accumulator, V through an LDS image (whole 256-B rows stored by ds_write_b128, read by
 //     ds_read_b64_tr_b16).
-// K and V of the next tile are prefetched into a second register set (plain loads only: no
-// LDS-DMA, so hipcc's counted waits keep the prefetch in flight; 178 VGPRs = 2 waves per SIMD:
-// all 2048 waves of a batch-256 layer are resident at once). The prologue issues every q / k_new /
+// Three tiles are in flight in register sets of their own (plain loads only: no LDS-DMA, so hipcc's
+// counted waits keep the prefetch in flight). The launch bound holds every form to 256 registers, 2
+// waves per SIMD: all 2048 waves of a batch-256 layer, or two workgroups of 4 waves per CU, are resident
+// (unbounded, the 4-wave form took 268 with its accumulators and ran one workgroup per CU: 48 rows of
+// 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every q / k_new /
 // v_new / rotary-table load at once (one round trip) behind the first tile's loads. RoPE of q /
 // k_new and the cache append are fused; lanes whose (clamped) key is the new token's slot use
 // k_new / v_new from registers. Measured at batch 256 (Mistral-7B, 174..301 keys): 51 us per
@@ -1129,7 +1131,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 // write-through stores and takes a ticket, and the last of the row's NP partitions merges them —
 // at 4k keys one workgroup per (batch, kv head) would stream 2 MB from one CU.
 template <int G, int W, bool KV8 = false>
-__global__ __launch_bounds__(64 * W) void attn_decode_mfma_kernel(DecodeFusedArgs a) {
+__global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFusedArgs a) {
   constexpr int D = 128, DS = D / 32, DT = D / 16;
   __shared__ __attribute__((aligned(16))) char vimg_all[W][32 * D * 2];  // per wave; rows 16..31 stay zero
   __shared__ __attribute__((aligned(16))) bf16_t qkv_st[(G + 2) * D];  // slab path (W == 1): reduced q | k | v
@@ -1205,12 +1207,9 @@ __global__ __launch_bounds__(64 * W) void attn_decode_mfma_kernel(DecodeFusedArg
   };
   Tile ta, tb, tc;
   const int cfirst = kbeg + 16 * w, cstep = 16 * W;  // this wave's tiles: cfirst + j * cstep
-  // fp8 tiles carry half the bytes: the single-wave kernel keeps THREE in flight (12 KiB per wave;
-  // a fourth register set would cost the second wave per SIMD)
-  constexpr bool DEEP8 = KV8 && W == 1;
   if (cfirst < len) load(ta, cfirst);
-  if ((W > 1 || DEEP8) && cfirst + cstep < len) load(tb, cfirst + cstep);
-  if ((W > 1 || DEEP8) && cfirst + 2 * cstep < len) load(tc, cfirst + 2 * cstep);
+  if (cfirst + cstep < len) load(tb, cfirst + cstep);
+  if (cfirst + 2 * cstep < len) load(tc, cfirst + 2 * cstep);
 
   // ---- q / k_new / v_new and the rotary tables, all loads at once. D = 128: chunk 4 s + g's
   // rotary partner (chunk ^ 8) is the lane's own chunk 4 (s ^ 2) + g, its table offset
@@ -1434,29 +1433,18 @@ __global__ __launch_bounds__(64 * W) void attn_decode_mfma_kernel(DecodeFusedArg
     }
   };
 
-  if constexpr (W == 1 && !DEEP8) {
-    for (int c0 = cfirst; c0 < len; c0 += 2 * cstep) {
-      if (c0 + cstep < len) load(tb, c0 + cstep);
-      consume(ta, c0);
-      if (c0 + cstep < len) {
-        if (c0 + 2 * cstep < len) load(ta, c0 + 2 * cstep);
-        consume(tb, c0 + cstep);
-      }
+  // three tiles in flight (all of a wave's tiles at up to 48 W keys: one memory round trip); a register
+  // set is refilled right after its tile is consumed
+  for (int c0 = cfirst; c0 < len; c0 += 3 * cstep) {
+    consume(ta, c0);
+    if (c0 + 3 * cstep < len) load(ta, c0 + 3 * cstep);
+    if (c0 + cstep < len) {
+      consume(tb, c0 + cstep);
+      if (c0 + 4 * cstep < len) load(tb, c0 + 4 * cstep);
     }
-  } else {
-    // three tiles in flight (all of a wave's tiles at up to 24 W keys: one memory round trip);
-    // a register set is refilled right after its tile is consumed
-    for (int c0 = cfirst; c0 < len; c0 += 3 * cstep) {
-      consume(ta, c0);
-      if (c0 + 3 * cstep < len) load(ta, c0 + 3 * cstep);
-      if (c0 + cstep < len) {
-        consume(tb, c0 + cstep);
-        if (c0 + 4 * cstep < len) load(tb, c0 + 4 * cstep);
-      }
-      if (c0 + 2 * cstep < len) {
-        consume(tc, c0 + 2 * cstep);
-        if (c0 + 5 * cstep < len) load(tc, c0 + 5 * cstep);
-      }
+    if (c0 + 2 * cstep < len) {
+      consume(tc, c0 + 2 * cstep);
+      if (c0 + 5 * cstep < len) load(tc, c0 + 5 * cstep);
     }
   }
   if constexpr (W == 1) {
@@ -2031,19 +2019,36 @@ extern "C" int rt_attn_decode_fused_ps(int D, int nk) { return 4 * (64 / (D / 8)
 // memory round trip); longer caches split the row into partitions of about RT_DECODE_MW_KPP (512)
 // keys, at most the workspace's NP, merged by the last arriving partition.
 constexpr int DEC_MW = 8;
-static bool rt_attn_decode_mw_ok(int B, int Hq, int Hkv, int D, int Smax) {
-  const int G = Hkv ? Hq / Hkv : 0;
-  return D == 128 && (long)B * Hkv < std::max(256, tuning().decode_mw_bh) && (G == 1 || G == 2 || G == 4 || G == 8);
-}
 static int rt_attn_decode_mw_np(int Smax, int np_ws) {
   const int kpp = std::max(16, tuning().decode_mw_kpp);
   if (Smax <= tuning().decode_mw_smax || np_ws <= 1) return 1;
   return std::max(1, std::min(np_ws, (Smax + kpp - 1) / kpp));
 }
-extern "C" int rt_attn_decode_mfma_ok(int B, int Hq, int Hkv, int D, int NP) {
+// Waves per (batch row, kv head) of the MFMA decode attention; 0: sizes it does not take. A one-wave pair is a
+// serial chain of 16-key tiles (0.8 us each, three in flight), so with few pairs on the chip, long rows or rows of
+// different lengths the pair's keys go round 4 waves that merge through LDS (2.5 us more). us a call, 8 kv heads x
+// 4 queries, rows of 50..80 / 150..300 / 400..600 / 150..1200 keys, one wave | four:
+//    48 rows: 11 / 22 / 40 / 71 | 11 / 17 / 27 / 41     64 rows: 11 / 23 / 42 / 74 | 12 / 19 / 30 / 45
+//    96 rows: 12 / 27 / 47 / 81 | 18 / 29 / 49 / 69    256 rows: 20 / 52 / 99 / 148 | 35 / 61 / 101 / 137
+// The line lies at 512 pairs (two workgroups of four waves per CU) and, beyond it, at caches of 1024 slots, whose
+// rows are past 500 keys when half full. Split-K slabs of the qkv product are summed by the one-wave kernel only: up
+// to 512 pairs that saves a reduce launch (5 us), less than the longer chain costs from about 400 keys on.
+static int rt_attn_decode_waves(int B, int Hq, int Hkv, int D, int Smax, int NP, bool kv8, bool slabs) {
   const int G = Hkv ? Hq / Hkv : 0;
-  return NP == 1 && D == 128 && (long)B * Hkv >= std::max(256, tuning().decode_mw_bh) &&
-         (G == 1 || G == 2 || G == 4 || G == 8 || G == 16);
+  const long pairs = (long)B * Hkv;
+  const bool multi = G == 1 || G == 2 || G == 4 || G == 8;
+  if (D != 128 || !(multi || G == 16)) return 0;
+  if (pairs < 256) return multi ? DEC_MW : 0;
+  const bool many = pairs >= std::max(256, tuning().decode_mw_bh), one = many && NP == 1;
+  if (kv8) return one ? 1 : multi ? DEC_MW : 0;
+  if (!multi || many != one) return one ? 1 : 0;
+  if (!one) return 4;
+  if (pairs <= tuning().decode_w4_bh) return slabs && Smax < 512 ? 1 : 4;
+  return Smax >= tuning().decode_w4_smax && !slabs ? 4 : 1;
+}
+// whether the decode attention sums the qkv product's split-K slabs itself
+extern "C" int rt_attn_decode_slabs_ok(int B, int Hq, int Hkv, int D, int Smax, int NP, int kv8) {
+  return rt_attn_decode_waves(B, Hq, Hkv, D, Smax, NP, kv8 != 0, true) == 1;
 }
 
 // Prompt K / V (rows [b * S + s] of the rotated qkv) -> fp8 cache slots [0, S): one 16-lane group
@@ -2115,17 +2120,18 @@ extern "C" int rt_attn_decode_fused(const void* qkv, long ldq, void* kc, void* v
   if (B == 0) return 0;
   const int G = Hq / Hkv;
   if (G * Hkv != Hq) return -1;
+  const int waves = rt_attn_decode_waves(B, Hq, Hkv, D, Smax, NP, kv8, qkv_slabs != nullptr);
   if (kv8) {
     // fp8 cache: the MFMA kernels only (large batch: one workgroup per (batch, kv head); small
     // batch: 8 waves per (batch, kv head), partitions for long caches)
     if (D != 128 || a.SmaxP < Smax || (G != 1 && G != 2 && G != 4 && G != 8)) return -3;
     // MHA (G = 1) at large batch: the VALU kernel, 2 waves per row (profiles/r3/dec13b_fp8kv_g1_valu_ab.txt)
-    if (G == 1 && !a.qkv_slabs && rt_attn_decode_mfma_ok(B, Hq, Hkv, D, NP)) {
+    if (G == 1 && !a.qkv_slabs && waves == 1) {
       hipLaunchKernelGGL(attn_decode_g1_fp8_kernel<2>, dim3((unsigned)(B * Hkv)), dim3(128), 0, stream, a);
       RT_LAUNCH_CHECK();
       return 0;
     }
-    if (rt_attn_decode_mfma_ok(B, Hq, Hkv, D, NP)) {
+    if (waves == 1) {
       dim3 mgrid((unsigned)(B * Hkv)), mblock(64);
       switch (G) {
         case 1: hipLaunchKernelGGL((attn_decode_mfma_kernel<1, 1, true>), mgrid, mblock, 0, stream, a); break;
@@ -2149,8 +2155,8 @@ extern "C" int rt_attn_decode_fused(const void* qkv, long ldq, void* kc, void* v
     RT_LAUNCH_CHECK();
     return 0;
   }
-  // large batch, one partition per (batch, kv head): the MFMA kernel
-  if (rt_attn_decode_mfma_ok(B, Hq, Hkv, D, NP)) {
+  // one wave per (batch, kv head)
+  if (waves == 1) {
     dim3 mgrid((unsigned)(B * Hkv)), mblock(64);
     switch (G) {
       case 1: hipLaunchKernelGGL((attn_decode_mfma_kernel<1, 1>), mgrid, mblock, 0, stream, a); break;
@@ -2162,16 +2168,13 @@ extern "C" int rt_attn_decode_fused(const void* qkv, long ldq, void* kc, void* v
     RT_LAUNCH_CHECK();
     return 0;
   }
-  // small batch, short caches: 8 waves per (batch, kv head), merged in LDS
-  if (rt_attn_decode_mw_ok(B, Hq, Hkv, D, Smax) && !a.qkv_slabs && (NP <= 1 || (part && tickets))) {
+  // 4 or 8 waves per (batch, kv head), merged in LDS
+  if (waves > 1 && !a.qkv_slabs && (NP <= 1 || (part && tickets))) {
     const int npm = rt_attn_decode_mw_np(Smax, NP);
     a.NP = npm;
     a.PS = npm > 1 ? ((Smax + npm - 1) / npm + 15) / 16 * 16 : Smax;
-    // 8 waves per (row, kv head) up to 256 pairs (one 512-thread workgroup per CU); 4 waves above
-    // (serving at batch 32..127: 1024-2048 waves instead of one chain of tiles per pair)
-    const bool w4 = (long)B * Hkv >= 256;
-    dim3 mgrid((unsigned)(B * Hkv * npm)), mblock(64 * (w4 ? 4 : DEC_MW));
-    if (w4) {
+    dim3 mgrid((unsigned)(B * Hkv * npm)), mblock(64 * waves);
+    if (waves == 4) {
       switch (G) {
         case 1: hipLaunchKernelGGL((attn_decode_mfma_kernel<1, 4>), mgrid, mblock, 0, stream, a); break;
         case 2: hipLaunchKernelGGL((attn_decode_mfma_kernel<2, 4>), mgrid, mblock, 0, stream, a); break;

@@ -65,3 +65,29 @@ def test_gemm_gelu_epilogue(M, N, K):
     assert bool((y[:, 0] == float("inf")).all()) and bool(y[:, 3].isnan().all()) and bool((y[:, 2] == 0).all())
     # the product's own fp32 sum is off by up to K * 2^-24 of its terms' size: 1e-5 here, and gelu's slope is below 1.13
     torch.testing.assert_close(y[:, 4:], e[:, 4:], rtol=2 ** -8, atol=2e-5)
+
+
+# ---------------------------------------------------------------------------------------------- decode attention
+@pytest.mark.parametrize("B,Hq,Hkv,Smax,window", [(33, 32, 8, 300, 0), (64, 32, 8, 1100, 200), (65, 32, 8, 1023, 0),
+                                                  (65, 32, 8, 1024, 0), (70, 64, 8, 1030, 0), (130, 4, 4, 70, 0),
+                                                  (14, 40, 40, 1200, 0), (257, 8, 2, 33, 0)])
+def test_decode_attention_waves_per_pair(B, Hq, Hkv, Smax, window):
+    """One and four waves per (row, kv head) at the lines between them; rows from one key to the whole cache."""
+    D = 128
+    g = torch.Generator(device=DEV).manual_seed(B + Smax)
+    kc = torch.randn(B, Hkv, Smax, D, generator=g, device=DEV).to(torch.bfloat16)
+    vc = torch.randn(B, Hkv, Smax, D, generator=g, device=DEV).to(torch.bfloat16)
+    slot = torch.randint(0, Smax, (B,), generator=g, device=DEV, dtype=torch.int32)
+    slot[:5] = torch.tensor([0, Smax - 1, 15, 16, 17], device=DEV)
+    start = torch.minimum(torch.randint(0, 20, (B,), generator=g, device=DEV, dtype=torch.int32), slot)
+    tail = torch.arange(Smax, device=DEV)[None, None, :, None] >= slot.long()[:, None, None, None]
+    kc.masked_fill_(tail, float("nan"))
+    vc.masked_fill_(tail, float("nan"))
+    cos, sin = ref.rope_tables(D, 4096, 10000.0, DEV)
+    pos = slot - start
+    qkv = torch.randn(B, (Hq + 2 * Hkv) * D, generator=g, device=DEV).to(torch.bfloat16)
+    k2, v2 = kc.clone(), vc.clone()
+    out = ops.decode_step_attention(qkv, kc, vc, slot, slot + 1, Hq, pos, cos, sin, start, window)
+    q = ops.rope_qkv_(qkv.clone(), pos, cos, sin, Hq, Hkv, D, S=1, k_cache=k2, v_cache=v2, slot_base=slot)
+    _close(out, ref.decode_attention(q, k2, v2, slot + 1, Hq, start, window, 1.0 / math.sqrt(D)))
+    assert torch.equal(kc.nan_to_num(), k2.nan_to_num()) and torch.equal(vc.nan_to_num(), v2.nan_to_num())
