@@ -2,7 +2,8 @@
 
 Replaces the reference's per-string ``SentenceTransformer.encode`` calls (1 + k + 2 (+2) separate
 forwards per reward, reinforcement_learning_optimization_after_rag.py:66-67,75-76,102-103): texts
-are tokenised natively in parallel, sorted by length into padded batches, encoded on the GPU.
+are tokenised natively in parallel and sorted by length into padded batches, which go up in one copy and are
+encoded on the GPU.
 """
 from __future__ import annotations
 
@@ -45,13 +46,12 @@ class Encoder:
         out = torch.empty(N, self.dim, dtype=torch.float32, device=self.device)
         if N == 0:
             return out
-        enc = self.tokenizer.encode_batch(texts, True, self.max_length)
-        order = sorted(range(N), key=lambda i: len(enc[i]))
-        for s in range(0, N, self.batch_size):
-            idx = order[s:s + self.batch_size]
-            batch = self.tokenizer.pad([enc[i] for i in idx], side="right", device=self.device)
-            emb = self.model.encode_ids(batch["input_ids"], batch["lengths"], normalize)
-            out[torch.tensor(idx, device=self.device)] = emb.float()
+        # every batch is tokenised, padded and uploaded ahead of the first forward: between them the host only launches
+        order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device)
+        r = 0
+        for ids, lengths in batches:
+            out[order[r:r + len(ids)]] = self.model.encode_ids(ids, lengths, normalize).float()
+            r += len(ids)
         return out
 
     def encode_unique(self, texts: Sequence[str], normalize: bool = True):
