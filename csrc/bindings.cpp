@@ -84,7 +84,7 @@ int rt_adamw_mixed(float*, const void*, long, const float*, float*, float*, void
 int rt_pool_norm(const void*, const int*, int, int, int, int, float*, hipStream_t);
 int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
-int rt_topk(const float*, long, long, int, int, const long*, long, float*, long*, hipStream_t);
+int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
 int rt_segment_mean(const float*, int, const long*, const int*, int, int, float*, hipStream_t);
 int rt_ivf_scan(const void*, int, int, const int*, int, const int*, const int*, const void*, const long*, const float*,
                 int, int, float*, long*,
@@ -1197,15 +1197,15 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   return out;
 }
 
-std::vector<Tensor> topk(const Tensor& scores, int64_t k, const optional<Tensor>& idmap) {
+std::vector<Tensor> topk(const Tensor& scores, int64_t k, const optional<Tensor>& idmap, bool finite) {
   CHECK_CUDA(scores); CHECK_F32(scores); CHECK_ROWS(scores);
   const int64_t nq = scores.size(0), N = scores.size(1);
   auto vals = at::empty({nq, k}, scores.options());
   auto ids = at::empty({nq, k}, scores.options().dtype(at::kLong));
   if (idmap.has_value() && idmap->defined()) { CHECK_I64(*idmap); CHECK_ROWS(*idmap); }
   check_rc(rt_topk(scores.data_ptr<float>(), scores.stride(0), nq, (int)N, (int)k, (const long*)opt_ptr(idmap),
-                   idmap.has_value() && idmap->defined() ? idmap->stride(0) : 0, vals.data_ptr<float>(),
-                   (long*)ids.data_ptr(), cur_stream()),
+                   idmap.has_value() && idmap->defined() ? idmap->stride(0) : 0, finite ? 1 : 0,
+                   vals.data_ptr<float>(), (long*)ids.data_ptr(), cur_stream()),
            "topk");
   return {vals, ids};
 }
@@ -1420,7 +1420,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("adamw_apply", &adamw_apply);
   m.def("grad_sumsq", &grad_sumsq);
   m.def("pool_norm", &pool_norm);
-  m.def("topk", &topk);
+  m.def("topk", &topk, py::arg("scores"), py::arg("k"), py::arg("idmap") = py::none(), py::arg("finite") = false);
   m.def("ivf_scan", &ivf_scan);
   m.def("segment_mean", &segment_mean, "k-means update: per-segment mean of sorted rows (+ L2 normalise)");
   m.def("gae", &gae);

@@ -305,6 +305,21 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// largest t such that at least K of the n (<= 64 * R) keys are >= t; the keys lie R to a lane, absent ones are 0.
+// Every lane of the wave returns it.
+template <int R>
+__device__ __forceinline__ uint32_t wave_kth(const uint32_t (&k)[R], int K) {
+  uint32_t t = 0;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t cnd = t | (1u << b);
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) c += (int)__popcll(__ballot(k[i] >= cnd));
+    if (c >= K) t = cnd;
+  }
+  return t;
+}
+
 // Block-wide sum; `sbuf` must hold blockDim.x/64 floats. Result broadcast to all threads.
 __device__ __forceinline__ float block_sum(float v, float* sbuf) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;

@@ -894,21 +894,6 @@ __global__ __launch_bounds__(1024) void sample_topk_search_kernel(
 // do not fit (plateaus of equal logits). V = 32000, top-k 50: 16 rows 177 -> 22 us, 64 rows 173 -> 23 us.
 constexpr int F32_RV = 8, F32_CAP = 1024, F32_TOPK = 256;
 
-// largest t such that at least K of the n (<= 64 * R) keys are >= t; the keys lie R to a lane, absent ones are 0.
-// Every lane of the wave returns it.
-template <int R>
-__device__ __forceinline__ uint32_t wave_kth(const uint32_t (&k)[R], int K) {
-  uint32_t t = 0;
-  for (int b = 31; b >= 0; --b) {
-    const uint32_t cnd = t | (1u << b);
-    int c = 0;
-#pragma unroll
-    for (int i = 0; i < R; ++i) c += (int)__popcll(__ballot(k[i] >= cnd));
-    if (c >= K) t = cnd;
-  }
-  return t;
-}
-
 __global__ __launch_bounds__(1024) void sample_topk_f32_kernel(
     const float* __restrict__ logits, long ld, int V, float inv_temp, int top_k, float top_p, uint64_t seed,
     const int64_t* __restrict__ offset_ptr, const uint8_t* __restrict__ row_active, long* __restrict__ out_tok,

@@ -158,11 +158,14 @@ def pool_normalize(x: torch.Tensor, lengths=None, normalize: bool = True) -> tor
     return ref.pool_norm(x, lengths, normalize)
 
 
-def topk(scores: torch.Tensor, k: int, idmap=None):
-    """Row-wise top-k (descending) of fp32 scores [nq, N] -> (values, ids)."""
+def topk(scores: torch.Tensor, k: int, idmap=None, finite: bool = False):
+    """Row-wise top-k (descending) of fp32 scores [nq, N] -> (values, ids), mapped through ``idmap`` [nq, N] if given;
+    ``finite``: the ids of scores that are not finite are -1."""
     if on_gpu(scores) and k <= 512:
-        return native().topk(scores.float().contiguous(), k, idmap)
-    return ref.topk(scores, k, idmap)
+        scores = scores.float()
+        return native().topk(scores if scores.stride(-1) == 1 else scores.contiguous(), k, idmap, finite)
+    v, i = ref.topk(scores, k, idmap)
+    return v, torch.where(torch.isfinite(v), i, torch.full_like(i, -1)) if finite else i
 
 
 def ivf_scan(q, probes, lstart, lsize, vecs, ids, maxlen, sqnorm=None, l2: bool = False):

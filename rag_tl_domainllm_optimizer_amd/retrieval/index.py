@@ -160,21 +160,21 @@ class IVFIndex:
     def _set_centroids(self, cen: torch.Tensor):
         self.centroids = cen.float().contiguous()
         n = self.centroids.shape[0]
-        # score(x, c) = x.c - pen[c]: pen = |c|^2 / 2 for l2 (argmax == nearest), 0 for ip;
-        # padding rows of the GEMM operand get +inf so they never win
+        # score(x, c) = x.c - pen[c]: pen = |c|^2 / 2 for l2 (argmax == nearest), 0 for ip
         pen = self.centroids.pow(2).sum(-1) * 0.5 if self.metric == "l2" else torch.zeros(n, device=self.device)
         if self.gpu:
             self._cen_op = _pad_rows(self.centroids.to(self.dtype), 128).contiguous()
-            self._pen = torch.full((self._cen_op.shape[0],), float("inf"), device=self.device)
-            self._pen[:n] = pen
         else:
-            self._cen_op, self._pen = self.centroids, pen
+            self._cen_op = self.centroids
+        self._pen = pen
 
     def _coarse(self, x: torch.Tensor, k: int) -> torch.Tensor:
         """indices [n, k] of the k best centroids per row (x already on device)."""
         if self.gpu:
-            s = ops.gemm(x.to(self.dtype).contiguous(), self._cen_op, out_f32=True)
-            s.sub_(self._pen)
+            # the operand's padding rows stay out of the selection
+            s = ops.gemm(x.to(self.dtype).contiguous(), self._cen_op, out_f32=True)[:, :self.centroids.shape[0]]
+            if self.metric == "l2":
+                s.sub_(self._pen)
             return ops.topk(s, k)[1]
         s = x.float() @ self._cen_op.t() - self._pen
         return torch.topk(s, k, dim=-1).indices
@@ -283,7 +283,7 @@ class IVFIndex:
         if self.gpu:
             cand, cid = ops.ivf_scan(q.to(self.dtype), probes, self.lstart, self.lsize, self.vecs, self.ids, maxlen,
                                      self.sqnorm, l2)
-            v, i = ops.topk(cand, kk)
+            v, out_ids = ops.topk(cand, kk, cid, finite=True)
         else:
             # same algorithm as the list-scan kernel: [nq, nprobe, maxlen] candidate slots
             j = torch.arange(maxlen)
@@ -297,9 +297,7 @@ class IVFIndex:
                 cand = 2 * cand - self.sqnorm[slot] - q.float().pow(2).sum(-1, keepdim=True)
             cand = torch.where(valid, cand, torch.full_like(cand, float("-inf")))
             cid = torch.where(valid, self.ids[slot] if self.ids.numel() else slot, torch.full_like(slot, -1))
-            v, i = torch.topk(cand, kk, dim=-1)
-        out_ids = cid.gather(1, i.clamp(min=0))
-        out_ids = torch.where(torch.isfinite(v), out_ids, torch.full_like(out_ids, -1))
+            v, out_ids = ops.topk(cand, kk, cid, finite=True)
         if kk < k:
             v = torch.cat([v, torch.full((v.shape[0], k - kk), float("-inf"), device=v.device)], 1)
             out_ids = torch.cat([out_ids, torch.full((v.shape[0], k - kk), -1, dtype=torch.long,

@@ -74,3 +74,70 @@ def test_decode_attention_waves_per_pair(B, Hq, Hkv, Smax, window):
     q = ops.rope_qkv_(qkv.clone(), pos, cos, sin, Hq, Hkv, D, S=1, k_cache=k2, v_cache=v2, slot_base=slot)
     _close(out, ref.decode_attention(q, k2, v2, slot + 1, Hq, start, window, 1.0 / math.sqrt(D)))
     assert torch.equal(kc.nan_to_num(), k2.nan_to_num()) and torch.equal(vc.nan_to_num(), v2.nan_to_num())
+
+
+# ---------------------------------------------------------------------------------------------- retrieval
+@pytest.mark.parametrize("nq,N,k", [(1, 40, 40), (3, 512, 16), (2, 1024, 32), (2, 1025, 32), (2, 700, 33), (5, 4097, 128),
+                                    (2, 4096, 128), (2, 300, 129), (4, 9600, 3), (1, 100003, 512), (2, 70, 100), (300, 64, 1)])
+def test_topk_forms(nq, N, k):
+    """Every thread count of the selection, rows that are strided, tied, flat, or short of finite scores, with ids mapped:
+    the order of a stable sort."""
+    g = torch.Generator(device=DEV).manual_seed(N + k)
+    s = torch.randn(nq, N + 3, generator=g, device=DEV)[:, :N]
+    if nq > 1:
+        s[0] = torch.randint(0, 5, (N,), generator=g, device=DEV).float()  # ties
+        s[1, N // 4:] = float("-inf")
+    if nq > 3:
+        s[2] = 0.5                                                         # a plateau
+        s[3] = torch.arange(N, device=DEV).float() / N
+    cid = torch.randint(0, 1 << 40, (nq, N), generator=g, device=DEV)
+    v, i = ops.topk(s, k, cid, finite=True)
+    vs, order = torch.sort(s, dim=-1, descending=True, stable=True)
+    n = min(k, N)
+    fits = torch.tensor([int((s[r] >= vs[r, n - 1]).sum()) <= 1024 for r in range(nq)])  # ties within the candidate list
+    assert torch.equal(v[:, :n], vs[:, :n])
+    want = torch.where(torch.isfinite(vs), cid.gather(1, order), torch.full_like(cid, -1))[:, :n]
+    ok = fits.to(DEV)[:, None] | (v[:, :n] > vs[:, n - 1:n])
+    assert torch.equal(torch.where(ok, i[:, :n], 0), torch.where(ok, want, 0))
+    if k > N:
+        assert bool((v[:, n:] == float("-inf")).all()) and bool((i[:, n:] == -1).all())
+
+
+@pytest.mark.parametrize("d", [8, 72, 384, 1000])
+@pytest.mark.parametrize("l2", [False, True])
+def test_ivf_scan_lists(d, l2):
+    """Lists of 0 to 200 vectors (pieces of 64), an unused probe, odd widths: against the products in float64."""
+    g = torch.Generator(device=DEV).manual_seed(d)
+    size = torch.tensor([0, 1, 63, 64, 65, 200], dtype=torch.int32, device=DEV)
+    start = torch.tensor([0, 0, 5, 70, 140, 210], dtype=torch.int32, device=DEV)
+    vecs = torch.randn(410, d, generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn(3, d, generator=g, device=DEV).to(torch.bfloat16)
+    probes = torch.tensor([[0, 1, 2], [3, 4, 5], [-1, 5, 0]], dtype=torch.int32, device=DEV)
+    sq, ids, maxlen = vecs.float().pow(2).sum(-1), torch.arange(410, device=DEV) + 7, 200
+    cand, cid = ops.ivf_scan(q, probes, start, size, vecs, ids, maxlen, sq, l2)
+    full = q.double() @ vecs.double().t()
+    if l2:
+        full = 2 * full - sq.double() - q.double().pow(2).sum(-1, keepdim=True)
+    want = torch.full((3, 3, maxlen), float("-inf"), dtype=torch.float64, device=DEV)
+    wid = torch.full((3, 3, maxlen), -1, device=DEV)
+    for i in range(3):
+        for p in range(3):
+            L = int(probes[i, p])
+            n = int(size[L]) if L >= 0 else 0
+            if n:
+                b = int(start[L])
+                want[i, p, :n], wid[i, p, :n] = full[i, b:b + n], ids[b:b + n]
+    assert torch.equal(cid, wid.view(3, -1))
+    # d fp32 additions of terms of size 1: d * 2^-24 * sqrt(d) at the very most
+    torch.testing.assert_close(cand.double(), want.view(3, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
+
+
+@pytest.mark.parametrize("B,S,H", [(3, 1, 8), (2, 17, 384), (4, 70, 768), (2, 9, 20), (1, 33, 2056)])
+def test_pool_normalize_forms(B, S, H):
+    g = torch.Generator(device=DEV).manual_seed(S)
+    x = torch.randn(B, S, H, generator=g, device=DEV).to(torch.bfloat16)
+    lens = torch.randint(1, S + 1, (B,), generator=g, device=DEV, dtype=torch.int32)
+    lens[0] = S
+    for n in (True, False):
+        torch.testing.assert_close(ops.pool_normalize(x, lens, n).double(), ref.pool_norm(x.double(), lens, n).double(),
+                                   rtol=1e-5, atol=1e-6)
