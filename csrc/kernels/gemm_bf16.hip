@@ -541,6 +541,290 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Decode products for 16 < M <= 64 rows over tile-ordered weight images
+// ---------------------------------------------------------------------------------------------
+// Both stream each weight fragment once from the image straight into the registers of the wave that multiplies it (1-KiB
+// runs per load, as gemv16_kernel); they differ in how the M rows of X reach the matrix cores. The row-major forms above
+// and below get 2 to 4.6 TB/s of weights at these M: 64-column LDS rings re-read X as often as W, and the 256-row one
+// leaves slabs of half the weight bytes to a second launch. us a call with cold weights, M = 24 / 48 / 64, best
+// row-major form -> image form:
+//   6144 x 4096 with norm    21.6 / 21.5 / 22.5 -> 16.0 / 19.8 / 21.8     28672 x 4096, SwiGLU  55.5 / 53.4 / 56.0 -> 44.2 / 44.3 / 45.5
+//   4096 x 4096 + residual   14.8 / 16.4 / 17.3 -> 10.9 / 14.6 / 16.6     4096 x 14336          29.6 / 30.2 / 31.9 -> 25.5 / 27.6 / 31.0
+//   10304 x 4096             36.0 / 37.4 / 38.8 -> 19.2 / 22.8 / 25.7     14336 x 4096, relu^2  29.8 / 31.3 / 32.6 -> 23.8 / 25.8 / 28.1
+//   32000 x 4096             59.0 / 58.9 / 60.8 -> 47.6 / 50.4 / 54.0     3072 x 2048 with norm 15.5 / 16.7 / 17.7 -> 7.1 / 9.9 / 11.7
+//
+// gemv64_kernel: gemv16_kernel with RT row tiles, for small products (see gemm64_direct): a workgroup owns one 16-row group
+// of the weight over the whole K, its NW waves split K and meet in LDS, and every wave loads its X fragments itself. X is
+// re-read N / 16 times from L2, which costs less than a split's hand-off (about 4 us) up to some 60 MB.
+template <bool OUT_F32, int RT, int NW, int DEPTH>
+__global__ __launch_bounds__(64 * NW) void gemv64_kernel(GemmArgs p) {
+  __shared__ float red[NW][16 * RT][17];
+  __shared__ float rsq[NW][16 * RT];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int frow = lane & 15, g = lane >> 4;
+  const int nc = p.K / 64;
+  const int c_begin = wid * nc / NW, c_end = (wid + 1) * nc / NW;
+  const char* wb = (const char*)p.B + (long)blockIdx.x * nc * 2048 + lane * 16;
+  const bf16_t* xr[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) xr[t] = p.A + (long)min(16 * t + frow, p.M - 1) * p.lda + g * 8;
+  struct Regs { uint4 w[2], x[RT][2]; };
+  auto ld = [&](Regs& r, int c) {
+    r.w[0] = load_nt16(wb + (long)c * 2048);
+    r.w[1] = load_nt16(wb + (long)c * 2048 + 1024);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      r.x[t][0] = *(const uint4*)(xr[t] + c * 64);
+      r.x[t][1] = *(const uint4*)(xr[t] + c * 64 + 32);
+    }
+  };
+  f32x4 acc[RT], sq[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) acc[t] = sq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool normed = p.norm_eps > 0.f;
+  auto mma = [&](const Regs& r) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const bf16x8 x = __builtin_bit_cast(bf16x8, r.x[t][h]);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, r.w[h]), acc[t], 0, 0, 0);
+        if (normed) sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, x, sq[t], 0, 0, 0);
+      }
+  };
+  Regs r[DEPTH];
+#pragma unroll
+  for (int i = 0; i < DEPTH - 1; ++i)
+    if (c_begin + i < c_end) ld(r[i], c_begin + i);
+  int c = c_begin;
+  for (; c + DEPTH <= c_end; c += DEPTH) {
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) {
+      if (c + i + DEPTH - 1 < c_end) ld(r[(i + DEPTH - 1) % DEPTH], c + i + DEPTH - 1);
+      mma(r[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < DEPTH - 1; ++i)
+    if (c + i < c_end) mma(r[i]);
+  // acc[t][e] of lane (frow, g) = C[16 t + 4 g + e][column frow] over this wave's k range; the sums of squares are
+  // the diagonal of X X^T
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      red[wid][16 * t + 4 * g + e][frow] = acc[t][e];
+      if (normed && 4 * g + e == frow) rsq[wid][16 * t + frow] = sq[t][e];
+    }
+  __syncthreads();
+  for (int e = tid; e < 16 * p.M; e += 64 * NW) {
+    const int row = e >> 4, ci = e & 15, col = (int)blockIdx.x * 16 + ci;
+    float ss = 0.f, y = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      if (normed) ss += rsq[w][row];
+      y += red[w][row][ci];
+    }
+    if (normed) y *= rsqrtf(ss / (float)p.K + p.norm_eps);
+    if (p.bias) y += bf2f(p.bias[col]);
+    y = apply_act(y, p.act);
+    if (p.R) y += bf2f(p.R[(long)row * p.ldr + col]);
+    if constexpr (OUT_F32) ((float*)p.C)[(long)row * p.ldc + col] = y;
+    else ((bf16_t*)p.C)[(long)row * p.ldc + col] = f2bf(y);
+  }
+}
+
+// gemm64_image_kernel: 4 waves, one (PAIR: a gate and an up) 16-row weight group each, 64 output columns a workgroup; X goes
+// through LDS in 64-deep chunks (8 KB, double-buffered, one barrier a chunk) and is read N / 64 times. Both X parts
+// and weights come in plain loads, DEPTH - 1 chunks ahead: with LDS-DMA for X the compiler waits for everything in flight
+// wherever it needs a weight register (SwiGLU 28672 x 4096 at M = 24: 49 us instead of 44). Few column groups are split
+// over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order.
+template <bool OUT_F32, int RT, bool PAIR>
+__global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __restrict__ slabs,
+                                                           unsigned* __restrict__ tickets, int split) {
+  constexpr int NG = PAIR ? 2 : 1, DEPTH = 4;
+  constexpr int XQ = (RT + 1) / 2;  // a wave's part of the X tile: 8 rows per load, 8 (cw + 4 q) ..
+  constexpr int SLOT = XQ * 4096, COLS = 64 * NG;
+  __shared__ __attribute__((aligned(16))) char smem[2 * SLOT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int cw = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frow = lane & 15, g = lane >> 4;
+  const int cg = blockIdx.x / split, sp = blockIdx.x % split;
+  const int nc = p.K / 64, ngroups = p.N / 16;
+  const int t0 = (int)((long)sp * nc / split), nt = (int)((long)(sp + 1) * nc / split) - t0;  // its chunks of 64 k
+  const char* wb[NG];
+#pragma unroll
+  for (int j = 0; j < NG; ++j) {
+    const int grp = (j ? p.N / 32 : 0) + 4 * cg + cw;
+    wb[j] = (const char*)p.B + ((long)min(grp, ngroups - 1) * nc + t0) * 2048 + lane * 16;
+  }
+  // X row 8 (cw + 4 q) + lane / 8, 16-B piece lane % 8 of the chunk; it lies at piece ^ lds_swz(row) of its 128-B row
+  const bf16_t* xs[XQ];
+  char* xd[XQ];
+#pragma unroll
+  for (int q = 0; q < XQ; ++q) {
+    const int row = 8 * (cw + 4 * q) + (lane >> 3);
+    xs[q] = p.A + (long)min(row, p.M - 1) * p.lda + t0 * 64 + (lane & 7) * 8;
+    xd[q] = smem + row * 128 + (((lane & 7) ^ lds_swz(row)) << 4);
+  }
+  struct W { uint4 v[NG][2], x[XQ]; };
+  auto load = [&](W& w, int i) {  // chunk t0 + i
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) w.x[q] = *(const uint4*)(xs[q] + (long)i * 64);
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      w.v[j][0] = load_nt16(wb[j] + (long)i * 2048);
+      w.v[j][1] = load_nt16(wb[j] + (long)i * 2048 + 1024);
+    }
+  };
+  f32x4 acc[RT][NG], sq[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    sq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NG; ++j) acc[t][j] = sq[t];
+  }
+  const bool normed = p.norm_eps > 0.f;
+  W w[DEPTH];
+  // chunk i: the wave's part of its X tile goes to LDS, the barrier adds the other waves' (and that the reads of two
+  // chunks ago are done, which the buffer then served)
+  auto step = [&](W& cur, W& nxt, int i, bool all) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) *(uint4*)(xd[q] + (i & 1) * SLOT) = cur.x[q];
+    if (all || i + DEPTH - 1 < nt) load(nxt, i + DEPTH - 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const char* slot = smem + (i & 1) * SLOT;
+    bf16x8 x[2][RT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int row = 16 * t + frow;
+        x[h][t] = *(const bf16x8*)(slot + row * 128 + (((h * 4 + g) ^ lds_swz(row)) << 4));
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+          acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, cur.v[j][h]), x[h][t], acc[t][j], 0, 0, 0);
+    if (normed) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h][t], x[h][t], sq[t], 0, 0, 0);
+    }
+  };
+  int i = 0;
+  if (nt >= 2 * DEPTH - 1) {
+    // no branch between a load and its use: the compiler's counted waits keep DEPTH - 1 chunks in flight
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d) load(w[d], d);
+    do {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) step(w[d], w[(d + DEPTH - 1) % DEPTH], i + d, true);
+      i += DEPTH;
+    } while (i + 2 * DEPTH - 2 < nt);
+  } else {
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (d < nt) load(w[d], d);
+  }
+  for (; i < nt; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (i + d < nt) step(w[d], w[(d + DEPTH - 1) % DEPTH], i + d, false);
+  }
+  // acc[t][j][e] = C[row 16 t + frow][column 4 g + e of group j]; sq[t] = X X^T of the tile, whose diagonal holds the rows'
+  // sums of squares: row frow's in lane (frow, g = frow / 4), element frow % 4
+  float ss[RT];
+  if (normed) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int e = frow & 3;
+      const float v = e == 0 ? sq[t][0] : e == 1 ? sq[t][1] : e == 2 ? sq[t][2] : sq[t][3];
+      ss[t] = __shfl(v, frow + 16 * (frow >> 2), 64);
+    }
+  }
+  if (split > 1) {
+    constexpr int SLAB = 16 * RT * COLS + 64;
+    typedef unsigned long long u64;
+    auto bits = [](float a, float b) -> u64 { return (u64)__float_as_uint(a) | (u64)__float_as_uint(b) << 32; };
+    u64* slab = (u64*)(slabs + ((long)cg * split + sp) * SLAB);
+    // write-through stores, drained before the ticket
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+#pragma unroll
+      for (int j = 0; j < NG; ++j) {
+        u64* d = slab + (((t * NG + j) * 4 + cw) * 64 + lane) * 2;
+        __hip_atomic_store(d, bits(acc[t][j][0], acc[t][j][1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(d + 1, bits(acc[t][j][2], acc[t][j][3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (normed && cw == 0 && g == 0)
+        __hip_atomic_store((float*)slab + 16 * RT * COLS + 16 * t + frow, ss[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* flag = (int*)smem;
+    if (tid == 0)
+      *flag = __hip_atomic_fetch_add(tickets + cg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(split - 1);
+    __syncthreads();
+    if (!*flag) return;
+    if (tid == 0) __hip_atomic_store(tickets + cg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the last one adds all parts in their order, its own among them
+    u64* base = (u64*)(slabs + (long)cg * split * SLAB);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+#pragma unroll
+      for (int j = 0; j < NG; ++j) {
+        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int q = 0; q < split; ++q) {
+          const u64* d = base + (long)q * (SLAB / 2) + (((t * NG + j) * 4 + cw) * 64 + lane) * 2;
+          const u64 a = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const u64 b = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          v += f32x4{__uint_as_float((unsigned)a), __uint_as_float((unsigned)(a >> 32)), __uint_as_float((unsigned)b),
+                     __uint_as_float((unsigned)(b >> 32))};
+        }
+        acc[t][j] = v;
+      }
+      if (normed) {
+        float v = 0.f;
+        for (int q = 0; q < split; ++q)
+          v += __hip_atomic_load((const float*)base + (long)q * SLAB + 16 * RT * COLS + 16 * t + frow, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+        ss[t] = v;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int row = 16 * t + frow;
+    if (row >= p.M) continue;
+    const float rs = normed ? rsqrtf(ss[t] / (float)p.K + p.norm_eps) : 1.f;
+    const int col = 16 * (4 * cg + cw) + 4 * g;
+    if (col >= (PAIR ? p.N / 2 : p.N)) continue;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = acc[t][0][e] * rs;
+      if (p.bias) y[e] += bf2f(p.bias[col + e]);
+      if constexpr (PAIR) {
+        float up = acc[t][1][e] * rs;
+        if (p.bias) up += bf2f(p.bias[p.N / 2 + col + e]);
+        y[e] = glu(y[e], up, p.glu);
+      } else {
+        y[e] = apply_act(y[e], p.act);
+        if (p.R) y[e] += bf2f(p.R[(long)row * p.ldr + col + e]);
+      }
+    }
+    if constexpr (OUT_F32) *(float4*)((float*)p.C + (long)row * p.ldc + col) = make_float4(y[0], y[1], y[2], y[3]);
+    else *(uint2*)((bf16_t*)p.C + (long)row * p.ldc + col) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+  }
+}
+
 // Shared tail of the M <= 64 kernels: split-K hand-off (write-through slabs + ticket, last arriver
 // reduces), in-GEMM RMS-norm scaling, SwiGLU pair / bias + activation + residual epilogues.
 // acc[j][r] = C[16 wid + 4 fq + r][16 j + frow] of the block's 64 columns; sq = sum of squares of
@@ -1110,6 +1394,24 @@ static int decode_split(int N, int K) {
   return split;
 }
 
+// Image products of 16 < M <= 64 rows: re-reading X per 16-row group is the cheaper way while the product is small and its
+// groups fill the chip no more than once. us, direct | best split of the other, M = 24 / 48 / 64: 2048 x 2048 6.7 / 9.3 / 11.1
+// | 8.7 / 10.6 / 12.4; 3072 x 2048 7.1 / 9.9 / 11.7 | 10.1 / 12.8 / 14.3; 4096 x 4096 11.1 / 16.3 / 19.9 | 12.4 / 14.5 / 16.6
+// (M = 32: 12.1 | 12.4); 2048 x 7168, long K, 15.8 / 24 / 30 | 12.9 / 15.6 / 18.0.
+static bool gemm64_direct(int M, int N, int K) {
+  return tuning().decode_split == 0 && N <= 4096 && K <= 4096 && (long)M * N * K <= 1L << 29;
+}
+// Split over K: up to one workgroup per CU, with at least 16 chunks each, 32 for the gated pairs whose partial tiles are
+// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 21.3 / 17.3 / 16.7 / 14.5 / 18.8 / 19.1;
+// 4096 x 14336 63.6 / 40.0 / 32.6 / 27.7 / 35.6 / 32.1; 6144 x 4096 22.1 / 19.3 / 24.3 / 21.7; 10304 x 4096 (161 groups)
+// 22.7 / 27.4; SwiGLU 14336 x 2048 18.0 / 20.8.
+static int gemm64_split(int groups, int K, bool pair) {
+  if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
+  int split = 1;
+  while (split < 8 && groups * (split + 1) <= 256 && K / 64 >= (pair ? 32 : 16) * (split + 1)) ++split;
+  return split;
+}
+
 }  // namespace rt
 
 using namespace rt;
@@ -1197,6 +1499,20 @@ extern "C" int rt_gemm_nt_glu(const void* A, long lda, const void* B, long ldb, 
     dim3 grid(((N + 63) / 64) * split), block(256);
     if (out_f32) hipLaunchKernelGGL((gemm_m64_kernel<true>), grid, block, 0, stream, p, slabs, tickets, split);
     else hipLaunchKernelGGL((gemm_m64_kernel<false>), grid, block, 0, stream, p, slabs, tickets, split);
+  } else if (M > 16 && wshuf && p.Rp == 0 && ldc % 4 == 0) {
+    const bool pair = act == ACT_SWIGLU;
+    const int rt = (M + 15) / 16, groups = pair ? (N + 127) / 128 : (N + 63) / 64;
+    const bool direct = !pair && gemm64_direct(M, N, K);
+    const int split = direct || !slabs || !tickets ? 1 : fit_split(gemm64_split(groups, K, pair), groups, 16 * rt * 64 * (pair ? 2 : 1) + 64);
+    const dim3 grid(direct ? N / 16 : groups * split), block(direct ? 512 : 256);
+#define I64_CASE(F32, RTT)                                                                                              \
+  if (direct) hipLaunchKernelGGL((gemv64_kernel<F32, RTT, 8, 3>), grid, block, 0, stream, p);                           \
+  else if (pair) hipLaunchKernelGGL((gemm64_image_kernel<F32, RTT, true>), grid, block, 0, stream, p, slabs, tickets, split); \
+  else hipLaunchKernelGGL((gemm64_image_kernel<F32, RTT, false>), grid, block, 0, stream, p, slabs, tickets, split);
+#define I64_RT(F32) if (rt == 2) { I64_CASE(F32, 2) } else if (rt == 3) { I64_CASE(F32, 3) } else { I64_CASE(F32, 4) }
+    if (out_f32) { I64_RT(true) } else { I64_RT(false) }
+#undef I64_RT
+#undef I64_CASE
   } else if (M <= gemv16_max_m() && wshuf && tuning().decode_split == 0 && use_gemv16(N, K, act) && p.Rp == 0) {
     const bool pair = act == ACT_SWIGLU;
     dim3 grid(pair ? N / 32 : N / 16), block(256);

@@ -61,7 +61,7 @@ class DecoderLayer(nn.Module):
         self._fp8: Dict[str, ops.Fp8Cache] = {}
         # norm-folded weights of the fused decode path (Llama/Mistral)
         self._fold: Dict[str, ops.FoldCache] = {}
-        # tile-ordered images of the split-K decode projections (qkv, o, down) for batch <= 16
+        # tile-ordered images of the decode projections for batch <= 64
         self._shufc: Dict[str, ops.ShufCache] = {}
 
     # ---------------------------------------------------------------- helpers
@@ -114,7 +114,7 @@ class DecoderLayer(nn.Module):
             if c is not None:
                 c.get(w)
         for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd)):
-            if name in self._shufc:  # images exist once a batch <= 16 decode ran
+            if name in self._shufc:  # images exist once a batch <= 64 decode ran
                 self._shufc[name].get(w)
 
     def decode_fused(self, h, attend):
@@ -203,11 +203,10 @@ class CausalLM(nn.Module):
         if not cfg.tie_embeddings:
             self.lm_head = nn.Parameter(torch.empty(cfg.vocab_size, cfg.hidden_size, **kw))
         self._rope = None
-        self._head_shuf = None  # ShufCache of the LM head for decode at batch <= 16
+        self._head_shuf = None  # ShufCache of the LM head for decode at batch <= 64
         # decode steps run the fused 4-GEMM layer (norms folded into GEMMs, residual epilogues) up to
-        # this batch: bf16 on the no-split tile-ordered GEMVs (M <= 16), then (17..64, serving) on
-        # the 256-row wide kernel / 64-column LDS-DMA ring with the in-GEMM RMS norm — 3 % faster
-        # decode steps than separate norm kernels (profiles/r6/decode_fused_max_ab.log); above it the
+        # this batch: bf16 on the no-split tile-ordered GEMVs (M <= 16), then (17..64, serving) on the
+        # tile-ordered kernels of up to four row tiles, with the in-GEMM RMS norm; above it the
         # bf16 decode layer uses the token-parallel 256x128 split-K GEMMs with the split-K partials
         # summed inside the norm and attention-prologue kernels (``defer_splitk``). With fp8 weights
         # (config 5) the same up to batch 64: W8A16 tile-ordered GEMVs to 16 rows, then the fp8
@@ -272,7 +271,7 @@ class CausalLM(nn.Module):
             return ops.linear(hidden, self.head_weight)
         hw = self.head_weight
         if ops.on_gpu(hidden) and shuffle_enabled(hidden.shape[0]) and hw.shape[0] % 16 == 0 and hw.is_contiguous():
-            # decode at batch <= 16: the tile-ordered image of the LM head (split 8: 52 -> 48 us)
+            # decode at batch <= 64: the tile-ordered image of the LM head (52 -> 48 us at batch 1, 59 -> 50 at 48)
             if self._head_shuf is None:
                 self._head_shuf = ops.ShufCache()
             return ops.native().gemm(hidden.contiguous(), self._head_shuf.get(hw), None, None, None, 0, out_f32,
@@ -513,9 +512,9 @@ def pack_enabled() -> bool:
 
 
 def shuffle_enabled(m: int) -> bool:
-    """Decode GEMMs at batch ``m`` <= 16 stream tile-ordered weight images (ops.ShufCache; the
-    split-K image launches run 5-20 % faster than row-major). RAGTL_DECODE_SHUF=0 turns it off."""
-    return m <= 16 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+    """Decode GEMMs at batch ``m`` <= 64 stream tile-ordered weight images (ops.ShufCache; 5-20 % faster
+    than row-major up to batch 16, 3-50 % above). RAGTL_DECODE_SHUF=0 turns it off."""
+    return m <= 64 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
 
 
 def _normal_(p: torch.Tensor, std: float, g: torch.Generator):

@@ -130,7 +130,7 @@ class Glu:
 
 def project(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, shuf=None, out=None) -> torch.Tensor:
     """x w^T without grad, any shape and dtype: the MFMA kernels where their shape rules hold (bf16;
-    ``shuf``: tile-ordered image at M <= 16), ``gemm_any`` otherwise — also for fp32 operands, which
+    ``shuf``: tile-ordered image at M <= 64), ``gemm_any`` otherwise — also for fp32 operands, which
     stay fp32 throughout. ``out``: rows to write (may be strided)."""
     if not on_gpu(x):
         y = ref.gemm(x, w, out_f32=out_f32)
@@ -151,10 +151,10 @@ def project(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, shuf=None, 
 
 
 def shuffle_decode(m: int) -> bool:
-    """Decode products at ``m`` <= 16 rows stream tile-ordered weight images (RAGTL_DECODE_SHUF=0: off)."""
+    """Decode products at ``m`` <= 64 rows stream tile-ordered weight images (RAGTL_DECODE_SHUF=0: off)."""
     import os
 
-    return m <= 16 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+    return m <= 64 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
 
 
 def glu_project(x: torch.Tensor, w: torch.Tensor, glu: Glu, shuf=None) -> torch.Tensor:
@@ -956,7 +956,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, act: int = 0, residual=None, n
     ``C = act(rstd(x) * x w^T) + residual`` where ``rstd`` (``norm_eps > 0``) is the RMS-norm of
     each input row computed inside the GEMM (the norm weight must already be folded into ``w``)
     and ``act`` may be ACT_SWIGLU (w = [gate; up]). ``fp8`` (Fp8Cache) streams e4m3fn weights;
-    ``shuf`` (ShufCache, M <= 16) streams the tile-ordered image of ``w`` instead."""
+    ``shuf`` (ShufCache, M <= 64) streams the tile-ordered image of ``w`` instead."""
     if on_gpu(x):
         x = x.contiguous()
         if fp8 is not None:
@@ -968,7 +968,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, act: int = 0, residual=None, n
                     return native().gemm_fp8(x, None, qs, sc, None, act, None, residual, norm_eps, True)
                 q, sc = fp8.get(w)
                 return native().gemm_fp8(x, None, q, sc, None, act, None, residual, norm_eps)
-        if shuf is not None and x.shape[0] <= 16 and w.shape[0] % 16 == 0:
+        if shuf is not None and x.shape[0] <= 64 and w.shape[0] % 16 == 0:
             return native().gemm(x, shuf.get(w), None, None, None, act, False, None, residual, norm_eps, True)
         return native().gemm(x, w, None, None, None, act, False, None, residual, norm_eps)
     y = x.float() @ w.float().t()
@@ -986,7 +986,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, act: int = 0, residual=None, n
 
 class ShufCache(dict):
     """Tile-ordered image of a decode weight (native ``shuffle_decode_weight``: each 16-row x 64-k
-    MFMA tile 2 KiB contiguous, so every load instruction of the M <= 16 kernel reads one 1-KiB
+    MFMA tile 2 KiB contiguous, so every load instruction of the M <= 64 kernels reads one 1-KiB
     run), rebuilt in place when the source's data pointer or version changes (graph-safe
     address). Pays on the split-K projections (down 28.5 -> 21.9 us at M = 1)."""
 

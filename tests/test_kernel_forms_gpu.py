@@ -141,3 +141,43 @@ def test_pool_normalize_forms(B, S, H):
     for n in (True, False):
         torch.testing.assert_close(ops.pool_normalize(x, lens, n).double(), ref.pool_norm(x.double(), lens, n).double(),
                                    rtol=1e-5, atol=1e-6)
+
+
+# ---------------------------------------------------------------------------------------------- decode products, 17..64 rows
+@pytest.mark.parametrize("N,K,act", [(16, 64, 0), (80, 192, 0), (2048, 512, 0), (4096, 2048, 0), (4112, 1024, 0),
+                                     (6160, 2112, 0), (4096, 4160, ops.ACT_RELU2), (64, 128, 5), (192, 2048, 5), (4224, 4096, 5)])
+def test_image_products_17_to_64_rows(N, K, act):
+    """Tile-ordered products at 17..64 rows on the rule's own route and at forced splits: odd numbers of row groups and
+    chunks, the in-product norm, bias, activation, residual, fp32 results and strided results. bf16 products are exact in
+    fp32, so fp32 results differ from 64 bits by the sum's order alone: K 2^-24 of sum |x w| bounds it."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    img = C.shuffle_decode_weight(w)
+    bias = torch.randn(N, generator=g, device=DEV).bfloat16()
+    No = N // 2 if act == ops.ACT_SWIGLU else N
+
+    def epi(y, r):
+        if act == ops.ACT_SWIGLU:
+            return torch.nn.functional.silu(y[:, :No]) * y[:, No:]
+        y = ref.apply_act(y, act)
+        return y if r is None else y + r.double()
+
+    for M in (17, 32, 33, 48, 64):
+        x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+        r = torch.randn(M, No, generator=g, device=DEV).bfloat16() if act == 0 else None
+        pre = x.double() @ w.double().t()
+        rstd = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-5)
+        bound = (x.double().abs() @ w.double().abs().t()).max().item() * K * 2.0 ** -24 + 1e-6
+        for split in (0, 1, 2, 3, 7, 8):
+            with ops.tuning(decode_split=split):
+                for _ in range(2):  # the second finds the tickets as the first left them
+                    y = C.gemm(x, img, None, None, None, 0 if act == ops.ACT_RELU2 else act, True, None, None, 0.0, True)
+                e = (y.double() - (epi(pre, None) if act == ops.ACT_SWIGLU else pre)).abs().max().item()
+                assert e <= bound * (8 if act == ops.ACT_SWIGLU else 1), (M, split, e, bound)
+                out = torch.full((M, No + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+                C.gemm(x, img, None, None, bias, act, False, out[:, :No], r, 1e-5, True)
+                want = epi(pre * rstd + bias.double(), r)
+                # a bf16 rounding of the result and, before a square or a product, the fp32 sum's error
+                torch.testing.assert_close(out[:, :No].double(), want, rtol=2.0 ** -8 + 1e-3, atol=4 * bound + 1e-4)
+                assert (out[:, No:] == 7).all()
