@@ -181,3 +181,28 @@ def test_image_products_17_to_64_rows(N, K, act):
                 # a bf16 rounding of the result and, before a square or a product, the fp32 sum's error
                 torch.testing.assert_close(out[:, :No].double(), want, rtol=2.0 ** -8 + 1e-3, atol=4 * bound + 1e-4)
                 assert (out[:, No:] == 7).all()
+
+
+# ---------------------------------------------------------------------------------------------- GELU epilogue
+@pytest.mark.parametrize("M,N,res", [(65, 256, False), (300, 264, True), (4096, 8, False)])
+def test_gelu_epilogue_bits(M, N, res):
+    """The tile epilogue's GELU has the bits of the split-K reduction's (erff throughout). A row's input is the sum of the
+    three bf16 parts of an fp32 value, times a column's power of two: exact, so both see the same values, from denormal
+    results through the negative tail, where the bf16 candidates disagree, to beyond the fitted range."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(M)
+    v = torch.randn(M, generator=g, device=DEV) * torch.where(torch.rand(M, generator=g, device=DEV) < 0.5, 1.0, 4.0)
+    v[:8] = torch.tensor([-3.8, -5.2, 5.2, -9.0, 0.0, 1e-30, -2.125, 40.0], device=DEV)
+    x = torch.zeros(M, 64, device=DEV, dtype=torch.bfloat16)
+    rest = v.clone()
+    for k in range(3):
+        x[:, k] = rest.bfloat16()
+        rest = rest - x[:, k].float()
+    w = torch.zeros(N, 64, device=DEV, dtype=torch.bfloat16)
+    w[:, :3] = (2.0 ** (torch.arange(N, device=DEV) % 5 - 3).float())[:, None].bfloat16()
+    bias = torch.zeros(N, device=DEV, dtype=torch.bfloat16)
+    r = torch.randn(M, N, generator=g, device=DEV).bfloat16() if res else None
+    y = C.gemm_big(x, w, 0, 0, None, None, bias, 2, 0, 1, None, None, r)
+    slabs = torch.empty(M * N, dtype=torch.float32, device=DEV)
+    z = C.gemm_splitk(x, w, 1, slabs, bias, 2, None, r)
+    assert torch.equal(y.view(torch.int16), z.view(torch.int16))
