@@ -59,6 +59,8 @@ int rt_embed(const void*, const long*, const void*, const long*, void*, long, in
 int rt_rows_scatter(const void*, long, const int*, void*, long, int, long, hipStream_t);
 int rt_attn_fwd(const void*, long, const void*, long, const void*, long, void*, long, float*, const int*, const int*,
                 const float*, int, int, int, int, int, int, int, int, int, float, hipStream_t);
+int rt_attn_packed(const void*, long, const void*, long, const void*, long, void*, long, const long*, const float*, int, int,
+                   int, int, int, int, float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
                    void*, long, int, int, int, int, float, hipStream_t);
 int rt_attn_decode_fused(const void*, long, void*, void*, int, const int*, const int*, const int*, const int*,
@@ -81,7 +83,7 @@ int rt_adamw(float*, const float*, float*, float*, void*, long, float, float, fl
 int rt_grad_sumsq_mixed(const void*, long, const float*, long, float*, int, hipStream_t);
 int rt_adamw_mixed(float*, const void*, long, const float*, float*, float*, void*, long, float, float, float, float,
                    float, int, float, const float*, int, float*, int*, hipStream_t);
-int rt_pool_norm(const void*, const int*, int, int, int, int, float*, hipStream_t);
+int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, hipStream_t);
 int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
@@ -867,6 +869,29 @@ std::vector<Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, 
   return {o, lse};
 }
 
+// bidirectional self-attention of sequences whose rows lie one behind the other: off [B + 1] int64 row offsets on the
+// device, longest >= every length
+Tensor attn_packed(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& off, int64_t longest, int64_t H, int64_t D,
+                   double scale, const optional<Tensor>& rel_bias, int64_t rb_L) {
+  CHECK_CUDA(q); CHECK_BF16(q); CHECK_BF16(k); CHECK_BF16(v); CHECK_ROWS(q); CHECK_ROWS(k); CHECK_ROWS(v);
+  CHECK_ALIGN16(q); CHECK_ALIGN16(k); CHECK_ALIGN16(v);
+  CHECK_CUDA(off); CHECK_I64(off);
+  TORCH_CHECK(off.dim() == 1 && off.is_contiguous() && off.size(0) >= 1, "attn_packed: offsets [B + 1]");
+  TORCH_CHECK(q.size(1) == H * D && k.sizes() == q.sizes() && v.sizes() == q.sizes(), "attn_packed: q, k, v [rows, H D]");
+  TORCH_CHECK(q.stride(0) % 8 == 0 && k.stride(0) % 8 == 0 && v.stride(0) % 8 == 0, "attn_packed: strides % 8");
+  TORCH_CHECK(longest >= 0 && longest <= q.size(0), "attn_packed: longest ", longest, " of ", q.size(0), " rows");
+  auto o = at::empty({q.size(0), H * D}, q.options());
+  if (rel_bias.has_value() && rel_bias->defined()) {
+    CHECK_F32(*rel_bias);
+    TORCH_CHECK(rel_bias->is_contiguous() && rel_bias->size(0) == H && rel_bias->size(1) == 2 * rb_L - 1 && rb_L >= longest);
+  }
+  check_rc(rt_attn_packed(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), o.data_ptr(),
+                          o.stride(0), (const long*)off.data_ptr<int64_t>(), (const float*)opt_ptr(rel_bias), (int)rb_L,
+                          (int)off.size(0) - 1, (int)q.size(0), (int)longest, (int)H, (int)D, (float)scale, cur_stream()),
+           "attn_packed");
+  return o;
+}
+
 void attn_decode(const Tensor& q, const Tensor& kc, const Tensor& vc, const Tensor& kv_len,
                  const optional<Tensor>& kv_start, int64_t window, double scale, int64_t Hq, Tensor part, int64_t PS,
                  Tensor out) {
@@ -1186,13 +1211,19 @@ Tensor grad_norm(const Tensor& g, Tensor partials) {
 }
 
 // ---------------------------------------------------------------------------------------------
-Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normalize) {
-  CHECK_CUDA(x); CHECK_BF16(x); TORCH_CHECK(x.dim() == 3 && x.is_contiguous());
-  const int64_t B = x.size(0), S = x.size(1), H = x.size(2);
+// x [B, S, H] with lengths [B], or [rows, H] with row offsets off [B + 1]
+Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normalize, const optional<Tensor>& off) {
+  const bool packed = off.has_value() && off->defined();
+  CHECK_CUDA(x); CHECK_BF16(x); TORCH_CHECK(x.dim() == (packed ? 2 : 3) && x.is_contiguous());
+  if (packed) {
+    CHECK_CUDA(*off); CHECK_I64(*off);
+    TORCH_CHECK(off->dim() == 1 && off->is_contiguous() && off->size(0) >= 1, "pool_norm: offsets [B + 1]");
+  }
+  const int64_t B = packed ? off->size(0) - 1 : x.size(0), S = packed ? 0 : x.size(1), H = x.size(-1);
   auto out = at::empty({B, H}, x.options().dtype(at::kFloat));
   if (lengths.has_value() && lengths->defined()) CHECK_I32(*lengths);
-  check_rc(rt_pool_norm(x.data_ptr(), (const int*)opt_ptr(lengths), (int)B, (int)S, (int)H, normalize ? 1 : 0,
-                        out.data_ptr<float>(), cur_stream()),
+  check_rc(rt_pool_norm(x.data_ptr(), (const int*)opt_ptr(lengths), (const long*)opt_ptr(off), packed ? x.size(0) : 0, (int)B,
+                        (int)S, (int)H, normalize ? 1 : 0, out.data_ptr<float>(), cur_stream()),
            "pool_norm");
   return out;
 }
@@ -1402,6 +1433,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_fwd", &swiglu_fwd);
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("embed", &embed);
+  m.def("attn_packed", &attn_packed, "bidirectional self-attention of packed sequences", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("off"), py::arg("longest"), py::arg("H"), py::arg("D"), py::arg("scale"),
+        py::arg("rel_bias") = py::none(), py::arg("rb_L") = 0);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_decode", &attn_decode);
   m.def("attn_bwd", &attn_bwd, "flash attention backward (RoPE backward optionally fused into dQ / dK)",
@@ -1419,7 +1453,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grad_norm", &grad_norm);
   m.def("adamw_apply", &adamw_apply);
   m.def("grad_sumsq", &grad_sumsq);
-  m.def("pool_norm", &pool_norm);
+  m.def("pool_norm", &pool_norm, py::arg("x"), py::arg("lengths"), py::arg("normalize"), py::arg("off") = py::none());
   m.def("topk", &topk, py::arg("scores"), py::arg("k"), py::arg("idmap") = py::none(), py::arg("finite") = false);
   m.def("ivf_scan", &ivf_scan);
   m.def("segment_mean", &segment_mean, "k-means update: per-segment mean of sorted rows (+ L2 normalise)");

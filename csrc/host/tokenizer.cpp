@@ -143,12 +143,13 @@ class Tokenizer {
   }
 
   // A batch for an encoder in one buffer: every text as front | its tokens | back, cut to max_length (keep_last: the
-  // last token stays), sorted by length, ascending and stable, in groups of `batch`. Layout of the int64 buffer: the
-  // texts' indices in that order [N], their lengths [N], then each group's ids [rows, longest], padded with pad_id on
-  // the right. Returns it (pinned on request, for an asynchronous copy) with the groups' (rows, longest).
-  std::pair<at::Tensor, std::vector<std::pair<int64_t, int64_t>>> encode_sorted(
+  // last token stays), sorted by length, ascending and stable, in groups of `batch`, without padding. Layout of the int64
+  // buffer: the texts' indices in that order [N], then for each group the row offsets of its texts [texts + 1], their
+  // tokens [rows] and these tokens' positions [rows], counted from pos0. Returns it (pinned on request, for an
+  // asynchronous copy) with the groups' (texts, rows, longest text).
+  std::pair<at::Tensor, std::vector<std::tuple<int64_t, int64_t, int64_t>>> encode_sorted(
       const std::vector<std::string>& texts, const std::vector<int64_t>& front, const std::vector<int64_t>& back,
-      bool keep_last, int64_t max_length, int64_t batch, int64_t pad_id, bool pin, int nthreads) const {
+      bool keep_last, int64_t max_length, int64_t batch, int64_t pos0, bool pin, int nthreads) const {
     TORCH_CHECK(batch > 0 && max_length > 0, "encode_sorted: batch ", batch, ", max_length ", max_length);
     std::vector<std::vector<int64_t>> ids = encode_batch(texts, nthreads);
     py::gil_scoped_release release;
@@ -159,27 +160,32 @@ class Tokenizer {
     std::vector<int64_t> order(N);
     for (int64_t i = 0; i < N; ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return len_of(a) < len_of(b); });
-    std::vector<std::pair<int64_t, int64_t>> groups;
-    int64_t total = 2 * N;
+    std::vector<std::tuple<int64_t, int64_t, int64_t>> groups;
+    int64_t total = N;
     for (int64_t r = 0; r < N; r += batch) {
-      const int64_t rows = std::min(batch, N - r), S = std::max<int64_t>(1, len_of(order[r + rows - 1]));
-      groups.emplace_back(rows, S);
-      total += rows * S;
+      const int64_t n = std::min(batch, N - r);
+      int64_t rows = 0;
+      for (int64_t j = r; j < r + n; ++j) rows += len_of(order[j]);
+      groups.emplace_back(n, rows, len_of(order[r + n - 1]));
+      total += n + 1 + 2 * rows;
     }
     at::Tensor buf = at::empty({total}, at::TensorOptions().dtype(at::kLong).pinned_memory(pin));
     int64_t* p = buf.data_ptr<int64_t>();
-    int64_t *len = p + N, *at = p + 2 * N, r = 0;
-    for (const auto& g : groups)
-      for (int64_t j = 0; j < g.first; ++j, ++r, at += g.second) {
+    int64_t *off = p + N, r = 0;
+    for (const auto& [texts_, rows, longest] : groups) {
+      int64_t *id = off + texts_ + 1, *pos = id + rows, at = 0;
+      off[0] = 0;
+      for (int64_t j = 0; j < texts_; ++j, ++r) {
         const int64_t i = order[r], n = len_of(i), nf = (int64_t)front.size(), nt = nf + (int64_t)ids[i].size();
         p[r] = i;
-        len[r] = n;
         auto token = [&](int64_t k) { return k < nf ? front[k] : k < nt ? ids[i][k - nf] : back[k - nt]; };
         const bool cut = nt + (int64_t)back.size() > n;
-        for (int64_t k = 0; k < n; ++k) at[k] = token(k);
-        if (cut && keep_last && n > 0) at[n - 1] = token(nt + (int64_t)back.size() - 1);
-        for (int64_t k = n; k < g.second; ++k) at[k] = pad_id;
+        for (int64_t k = 0; k < n; ++k) { id[at + k] = token(k); pos[at + k] = pos0 + k; }
+        if (cut && keep_last && n > 0) id[at + n - 1] = token(nt + (int64_t)back.size() - 1);
+        off[j + 1] = at += n;
       }
+      off = pos + rows;
+    }
     return {buf, groups};
   }
 
@@ -389,7 +395,7 @@ void bind_tokenizer(py::module& m) {
       .def("encode", &Tokenizer::encode)
       .def("encode_batch", &Tokenizer::encode_batch, py::arg("texts"), py::arg("nthreads") = 8)
       .def("encode_sorted", &Tokenizer::encode_sorted, py::arg("texts"), py::arg("front"), py::arg("back"),
-           py::arg("keep_last"), py::arg("max_length"), py::arg("batch"), py::arg("pad_id"), py::arg("pin"),
+           py::arg("keep_last"), py::arg("max_length"), py::arg("batch"), py::arg("pos0"), py::arg("pin"),
            py::arg("nthreads") = 8)
       .def("decode", &Tokenizer::decode, py::arg("ids"), py::arg("skip_special") = true)
       .def("token_to_id", &Tokenizer::token_to_id)

@@ -8,16 +8,18 @@
 
 namespace rt {
 
-// x [B, S, H] bf16, lengths [B] -> out [B, H] fp32 (L2-normalised if norm != 0). One workgroup a text; a stream
+// x [B, S, H] bf16, lengths [B] (off: text b is rows [off[b], off[b + 1]) of x [rows, H]) -> out [B, H] fp32 (L2-normalised if norm != 0). One workgroup a text; a stream
 // of its tokens, bound by the loads in flight: 256 texts of 162 x 768 115 -> 15.5 us over 2-byte loads one after
 // the other.
 __global__ __launch_bounds__(256) void pool_norm_kernel(const bf16_t* __restrict__ x, const int* __restrict__ lengths,
-                                                        int S, int H, int normalize, float* __restrict__ out) {
+                                                        const long* __restrict__ off, long rows, int S, int H,
+                                                        int normalize, float* __restrict__ out) {
   extern __shared__ float acc[];  // [H]
   __shared__ float sb[4];
   const int b = blockIdx.x;
-  const int len = lengths ? lengths[b] : S;
-  const bf16_t* xb = x + (long)b * S * H;
+  const long first = off ? min(max(off[b], 0L), rows) : (long)b * S;
+  const int len = off ? (int)(min(max(off[b + 1], first), rows) - first) : lengths ? lengths[b] : S;
+  const bf16_t* xb = x + first * H;
   if (H % 8 == 0 && (uintptr_t)x % 16 == 0) {
     // 8 columns a thread in 16-byte loads, 8 tokens' in flight; a column's tokens are summed in order
     for (int c = threadIdx.x; c < H / 8; c += 256) {
@@ -337,11 +339,11 @@ __global__ __launch_bounds__(256) void segment_mean_kernel(const float* __restri
 
 using namespace rt;
 
-extern "C" int rt_pool_norm(const void* x, const int* lengths, int B, int S, int H, int normalize, float* out,
-                            hipStream_t stream) {
+extern "C" int rt_pool_norm(const void* x, const int* lengths, const long* off, long rows, int B, int S, int H,
+                            int normalize, float* out, hipStream_t stream) {
   if (B == 0) return 0;
-  hipLaunchKernelGGL(pool_norm_kernel, dim3(B), dim3(256), H * sizeof(float), stream, (const bf16_t*)x, lengths, S, H,
-                     normalize, out);
+  hipLaunchKernelGGL(pool_norm_kernel, dim3(B), dim3(256), H * sizeof(float), stream, (const bf16_t*)x, lengths, off, rows,
+                     S, H, normalize, out);
   RT_LAUNCH_CHECK();
   return 0;
 }

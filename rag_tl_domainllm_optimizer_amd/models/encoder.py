@@ -99,29 +99,50 @@ class SentenceEncoder(nn.Module):
         cfg = self.cfg
         B, S = input_ids.shape
         dev = input_ids.device
-        H, nh, D = cfg.hidden_size, cfg.num_heads, cfg.head_dim
+        nh, D = cfg.num_heads, cfg.head_dim
         ar = torch.arange(S, device=dev)[None, :].expand(B, S)
         valid = ar < lengths.to(dev).long()[:, None]
         if cfg.arch == "mpnet":
-            pos = torch.where(valid, ar + cfg.pad_token_id + 1, torch.full_like(ar, cfg.pad_token_id))
+            pos = torch.where(valid, ar + self.first_position, torch.full_like(ar, cfg.pad_token_id))
         else:
             pos = ar
-        x = ops.embedding(self.word_embed, input_ids.reshape(-1), self.pos_embed, pos.reshape(-1))
+        lens32 = lengths.to(dev).to(torch.int32)
+        lut, L = self._bias_lut(max(S, 1), dev)
+        return self._states(input_ids.reshape(-1), pos.reshape(-1), lambda q, k, v: ops.attention(
+            q, k, v, B, S, S, nh, nh, D, causal=False, kv_len=lens32, rel_bias_lut=lut, rb_L=L))
+
+    def _states(self, ids, pos, attend):
+        """Token states of the rows ``ids`` at positions ``pos``; ``attend`` mixes them within their texts."""
+        cfg, H = self.cfg, self.cfg.hidden_size
+        x = ops.embedding(self.word_embed, ids, self.pos_embed, pos)
         if cfg.type_vocab_size:
             x = x + self.type_embed[0]
         x, _ = ops.layer_norm(x, self.emb_ln_w, self.emb_ln_b, cfg.norm_eps)
-        lens32 = lengths.to(dev).to(torch.int32)
-        lut, L = self._bias_lut(max(S, 1), dev)
         for layer in self.layers:
             qkv = ops.linear(x, layer.qkv_w, layer.qkv_b)
-            q, k, v = qkv[:, :H], qkv[:, H:2 * H], qkv[:, 2 * H:]
-            a = ops.attention(q, k, v, B, S, S, nh, nh, D, causal=False, kv_len=lens32, rel_bias_lut=lut, rb_L=L)
+            a = attend(qkv[:, :H], qkv[:, H:2 * H], qkv[:, 2 * H:])
             a = ops.linear(a, layer.o_w, layer.o_b)
             x, _ = ops.layer_norm(a, layer.ln1_w, layer.ln1_b, cfg.norm_eps, residual=x)
             f = ops.linear(x, layer.fc1_w, layer.fc1_b, act=cfg.hidden_act)
             d = ops.linear(f, layer.fc2_w, layer.fc2_b)
             x, _ = ops.layer_norm(d, layer.ln2_w, layer.ln2_b, cfg.norm_eps, residual=x)
         return x
+
+    @property
+    def first_position(self) -> int:
+        return self.cfg.pad_token_id + 1 if self.cfg.arch == "mpnet" else 0
+
+    @torch.no_grad()
+    def encode_packed(self, ids: torch.Tensor, pos: torch.Tensor, off: torch.Tensor, longest: int,
+                      normalize: bool = True) -> torch.Tensor:
+        """:meth:`encode_ids` of texts without padding: rows [off[b], off[b + 1]) of ``ids`` are text b, none longer than
+        ``longest``, at positions ``pos`` (from ``first_position``)."""
+        nh, D = self.cfg.num_heads, self.cfg.head_dim
+        if longest == 0:
+            return torch.zeros(len(off) - 1, self.cfg.hidden_size, device=ids.device)
+        lut, L = self._bias_lut(longest, ids.device)
+        x = self._states(ids, pos, lambda q, k, v: ops.attention_packed(q, k, v, off, longest, nh, D, rel_bias_lut=lut, rb_L=L))
+        return ops.pool_normalize_packed(x, off, longest, normalize)
 
     @torch.no_grad()
     def encode_ids(self, input_ids: torch.Tensor, lengths: torch.Tensor, normalize: bool = True) -> torch.Tensor:

@@ -223,6 +223,20 @@ def attention(q, k, v, B, Sq, Sk, Hq, Hkv, D, causal=False, window=0, scale=None
                          rb_L)[0]
 
 
+def attention_packed(q, k, v, off, longest: int, H: int, D: int, scale=None,
+                     rel_bias_lut: Optional[torch.Tensor] = None, rb_L: int = 0):
+    """Bidirectional :func:`attention` within sequences that lie one behind the other: rows [off[b], off[b + 1])
+    of q / k / v [rows, H D] are sequence b, none longer than ``longest``."""
+    scale = scale if scale is not None else 1.0 / math.sqrt(D)
+    if on_gpu(q):
+        return native().attn_packed(q, k, v, off, longest, H, D, scale, rel_bias_lut, rb_L)
+    idx, lengths = ref.packed_grid(off, longest)
+    B = len(lengths)
+    o = ref.attention(*(t[idx.view(-1).clamp(min=0)] for t in (q, k, v)), B, longest, longest, H, H, D, False, 0, scale, None,
+                      lengths, rel_bias_lut, rb_L)[0]
+    return o[idx.view(-1) >= 0]
+
+
 # ------------------------------------------------------------------------------ decode attention
 def decode_partition(batch_heads: int, D: int = 128, Smax: int = 4096) -> int:
     """Keys per split-K partition of the fused decode kernel. A partition is a whole number of

@@ -158,6 +158,14 @@ def pool_normalize(x: torch.Tensor, lengths=None, normalize: bool = True) -> tor
     return ref.pool_norm(x, lengths, normalize)
 
 
+def pool_normalize_packed(x: torch.Tensor, off: torch.Tensor, longest: int, normalize: bool = True) -> torch.Tensor:
+    """:func:`pool_normalize` of texts that lie one behind the other: rows [off[b], off[b + 1]) of x [rows, H]."""
+    if on_gpu(x):
+        return native().pool_norm(x.contiguous(), None, normalize, off)
+    idx, lengths = ref.packed_grid(off, longest)
+    return ref.pool_norm(x[idx.clamp(min=0)], lengths, normalize)
+
+
 def topk(scores: torch.Tensor, k: int, idmap=None, finite: bool = False):
     """Row-wise top-k (descending) of fp32 scores [nq, N] -> (values, ids), mapped through ``idmap`` [nq, N] if given;
     ``finite``: the ids of scores that are not finite are -1."""

@@ -217,6 +217,13 @@ def pool_norm(x, lengths=None, normalize=True):
     return F.normalize(m, dim=-1, eps=1e-12) if normalize else m
 
 
+def packed_grid(off, longest):
+    """-> (idx [B, longest]: the row of each sequence's position, -1 behind its end; lengths [B] int32)."""
+    n = off[1:] - off[:-1]
+    ar = torch.arange(longest, device=off.device)[None, :]
+    return torch.where(ar < n[:, None], off[:-1, None] + ar, torch.full_like(ar, -1)), n.int()
+
+
 def topk(scores, k, idmap=None):
     v, i = torch.topk(scores.float(), k, dim=-1)
     if idmap is not None:

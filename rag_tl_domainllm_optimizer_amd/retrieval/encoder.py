@@ -2,8 +2,8 @@
 
 Replaces the reference's per-string ``SentenceTransformer.encode`` calls (1 + k + 2 (+2) separate
 forwards per reward, reinforcement_learning_optimization_after_rag.py:66-67,75-76,102-103): texts
-are tokenised natively in parallel and sorted by length into padded batches, which go up in one copy and are
-encoded on the GPU.
+are tokenised natively in parallel and sorted by length into batches without padding, which go up in one copy and
+are encoded on the GPU.
 """
 from __future__ import annotations
 
@@ -46,12 +46,14 @@ class Encoder:
         out = torch.empty(N, self.dim, dtype=torch.float32, device=self.device)
         if N == 0:
             return out
-        # every batch is tokenised, padded and uploaded ahead of the first forward: between them the host only launches
-        order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device)
+        # every batch is tokenised and uploaded ahead of the first forward: between them the host only launches
+        order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device,
+                                                      self.model.first_position)
         r = 0
-        for ids, lengths in batches:
-            out[order[r:r + len(ids)]] = self.model.encode_ids(ids, lengths, normalize).float()
-            r += len(ids)
+        for ids, pos, off, longest in batches:
+            n = len(off) - 1
+            out[order[r:r + n]] = self.model.encode_packed(ids, pos, off, longest, normalize).float()
+            r += n
         return out
 
     def encode_unique(self, texts: Sequence[str], normalize: bool = True):

@@ -159,24 +159,24 @@ class Tokenizer:
             out.append(ids)
         return out
 
-    def encode_sorted(self, texts: Sequence[str], max_length: int, batch: int, device):
-        """:meth:`encode_batch` and :meth:`pad` (right) for an encoder, natively and with one upload: the texts sorted by
-        length in groups of ``batch`` -> (order [N]: the texts' indices, [(input_ids [rows, longest], lengths [rows])]),
-        on ``device``; the copy is not waited for."""
+    def encode_sorted(self, texts: Sequence[str], max_length: int, batch: int, device, first_position: int = 0):
+        """:meth:`encode_batch` for an encoder, natively and with one upload: the texts sorted by length in groups of
+        ``batch`` without padding -> (order [N]: the texts' indices, [(ids [rows], positions [rows] from
+        ``first_position``, offsets [texts + 1]: each text's first row, the longest text's length)]), on ``device``; the
+        copy is not waited for."""
         front, back = self._wrap([], True), []
         if self.template == "cls_sep":
             front, back = front[:1], front[1:]
         gpu = torch.device(device).type == "cuda"
         buf, groups = self._impl.encode_sorted(list(texts), front, back, self.template == "cls_sep", max_length, batch,
-                                               self.pad_token_id, gpu)
+                                               first_position, gpu)
         buf = buf.to(device, non_blocking=True)
-        n, r, out = len(texts), 0, []
-        at = 2 * n
-        for rows, longest in groups:
-            out.append((buf[at:at + rows * longest].view(rows, longest), buf[n + r:n + r + rows]))
-            at += rows * longest
-            r += rows
-        return buf[:n], out
+        at, out = len(texts), []
+        for n, rows, longest in groups:
+            off, ids, pos = buf[at:at + n + 1 + 2 * rows].split([n + 1, rows, rows])
+            out.append((ids, pos, off, longest))
+            at += n + 1 + 2 * rows
+        return buf[:len(texts)], out
 
     def decode(self, ids, skip_special_tokens: bool = True) -> str:
         if isinstance(ids, torch.Tensor):

@@ -1,9 +1,11 @@
-"""The encoders' native batch preparation against encode_batch and pad."""
+"""The encoders' native batch preparation against encode_batch, and encoding without padding."""
 import random
 
 import pytest
 import torch
 
+from rag_tl_domainllm_optimizer_amd import models
+from rag_tl_domainllm_optimizer_amd.models import PRESETS
 from rag_tl_domainllm_optimizer_amd.tokenizer import Tokenizer
 
 
@@ -15,11 +17,29 @@ def test_encode_sorted(arch, n, batch, max_length):
     texts = ["", *(" ".join(r.choices(words, k=r.randint(0, 12))) for _ in range(n - 1))]
     enc = tok.encode_batch(texts, True, max_length)
     order = sorted(range(n), key=lambda i: len(enc[i]))
-    got, groups = tok.encode_sorted(texts, max_length, batch, "cpu")
+    got, groups = tok.encode_sorted(texts, max_length, batch, "cpu", 2)
     assert got.tolist() == order and len(groups) == (n + batch - 1) // batch
-    for g, (ids, lengths) in enumerate(groups):
-        want = tok.pad([enc[i] for i in order[g * batch:(g + 1) * batch]], side="right")
-        assert torch.equal(ids, want["input_ids"]) and torch.equal(lengths, want["lengths"])
+    for g, (ids, pos, off, longest) in enumerate(groups):
+        want = [enc[i] for i in order[g * batch:(g + 1) * batch]]
+        assert ids.tolist() == sum(want, []) and pos.tolist() == [2 + k for w in want for k in range(len(w))]
+        assert off.tolist() == [sum(map(len, want[:k])) for k in range(len(want) + 1)]
+        assert longest == len(want[-1])
+
+
+@pytest.mark.parametrize("preset", ["tiny-bert", "tiny-mpnet"])
+def test_encode_packed_equals_padded(preset):
+    """Texts without padding give what the padded batch gives, a text of no tokens among them."""
+    cfg = PRESETS[preset]
+    m = models.SentenceEncoder(cfg, dtype=torch.float32, seed=1)
+    lens = torch.tensor([0, 1, 3, 9, 17])
+    g = torch.Generator().manual_seed(0)
+    ids = torch.randint(5, cfg.vocab_size, (5, 17), generator=g)
+    off = torch.nn.functional.pad(lens.cumsum(0), (1, 0))
+    flat = torch.cat([ids[b, :n] for b, n in enumerate(lens)])
+    pos = torch.cat([torch.arange(n) for n in lens]) + m.first_position
+    torch.testing.assert_close(m.encode_packed(flat, pos, off, 17), m.encode_ids(ids, lens), rtol=1e-5, atol=1e-6)
+    none = torch.zeros(0, dtype=torch.long)
+    assert torch.equal(m.encode_packed(none, none, torch.zeros(3, dtype=torch.long), 0), torch.zeros(2, cfg.hidden_size))
 
 
 def test_encode_sorted_refuses():

@@ -206,3 +206,31 @@ def test_gelu_epilogue_bits(M, N, res):
     slabs = torch.empty(M * N, dtype=torch.float32, device=DEV)
     z = C.gemm_splitk(x, w, 1, slabs, bias, 2, None, r)
     assert torch.equal(y.view(torch.int16), z.view(torch.int16))
+
+
+# ---------------------------------------------------------------------------------------------- encoders without padding
+@pytest.mark.parametrize("D,H,bias", [(32, 3, False), (64, 2, False), (64, 12, True), (128, 1, False), (32, 2, True)])
+@pytest.mark.parametrize("lens", [[1], [64, 65, 0, 127], [128, 129, 63, 1, 300], [2] * 40])
+def test_packed_attention_equals_padded(D, H, bias, lens):
+    """Sequences one behind the other against the padded form, around the tile edges. Without a bias the arithmetic per
+    row is the same, down to probabilities below 2^-126; the bias is added to the rounded or to the exact scaled score
+    (one rounding of an exponent of at most 2^7: 2^-17 of a probability, below the results' bf16)."""
+    g = torch.Generator(device=DEV).manual_seed(D + len(lens))
+    B, S = len(lens), max(lens)
+    n = torch.tensor(lens, device=DEV)
+    qkv = torch.randn(B, S, 3 * H * D, generator=g, device=DEV).bfloat16()
+    lut = torch.randn(H, 2 * S + 5, generator=g, device=DEV) if bias else None
+    rb = S + 3 if bias else 0
+    keep = torch.arange(S, device=DEV)[None, :] < n[:, None]
+    flat = qkv[keep]
+    off = torch.nn.functional.pad(n.cumsum(0), (1, 0))
+    cut = lambda t: (t[:, :H * D], t[:, H * D:2 * H * D], t[:, 2 * H * D:])
+    got = ops.attention_packed(*cut(flat), off, S, H, D, rel_bias_lut=lut, rb_L=rb)
+    want = ops.attention(*cut(qkv.view(B * S, -1)), B, S, S, H, H, D, kv_len=n.int(), rel_bias_lut=lut, rb_L=rb)
+    want = want.view(B, S, -1)[keep]
+    if bias:
+        _close(got, want, rtol=2.0 ** -7, atol=2.0 ** -8)
+    else:
+        assert torch.equal(got, want)
+    x = torch.randn(B, S, 384, generator=g, device=DEV).bfloat16()
+    assert torch.equal(ops.pool_normalize_packed(x[keep], off, S), ops.pool_normalize(x, n))
