@@ -59,6 +59,7 @@ int rt_embed(const void*, const long*, const void*, const long*, void*, long, in
 int rt_rows_scatter(const void*, long, const int*, void*, long, int, long, hipStream_t);
 int rt_attn_fwd(const void*, long, const void*, long, const void*, long, void*, long, float*, const int*, const int*,
                 const float*, int, int, int, int, int, int, int, int, int, float, hipStream_t);
+int rt_gemm_image(const void*, long, const void*, void*, long, int, int, int, int, int, int, const float*, hipStream_t);
 int rt_attn_packed(const void*, long, const void*, long, const void*, long, void*, long, const long*, const float*, int, int,
                    int, int, int, int, float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
@@ -572,6 +573,50 @@ Tensor gemm_splitk(const Tensor& a, const Tensor& w, int64_t nsplit, Tensor slab
                                  has_r ? residual->data_ptr() : nullptr, has_r ? residual->stride(0) : 0, c.data_ptr(),
                                  c.stride(0), GluArg(glu).ptr(), cur_stream()),
            "gemm_splitk_reduce");
+  return c;
+}
+
+// act(a w^T) for 64 < M <= 128 rows over a tile-ordered weight image. nsplit > 1: over K, through the fp32 slabs [nsplit, M,
+// N]; raw leaves them unreduced (plain product) and returns nothing
+optional<Tensor> gemm_image(const Tensor& a, const Tensor& w, int64_t act, bool out_f32, optional<Tensor> out, int64_t nsplit,
+                            optional<Tensor> slabs, bool raw, const std::vector<double>& glu) {
+  CHECK_CUDA(a); CHECK_CUDA(w); CHECK_BF16(a); CHECK_BF16(w); CHECK_ROWS(a);
+  CHECK_ALIGN16(a); CHECK_ALIGN16(w);
+  const int64_t M = a.size(0), K = a.size(1), N = w.size(0);
+  TORCH_CHECK(M > 64 && M <= 128, "gemm_image: 65 to 128 rows, got ", M);
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && w.is_contiguous() && N % 16 == 0 && K % 64 == 0 && K > 0, "gemm_image: image [N, K]");
+  TORCH_CHECK(a.stride(0) % 8 == 0, "gemm_image: row stride % 8");
+  const bool pair = act == 5;
+  TORCH_CHECK(!pair || N % 32 == 0, "gemm_image: SwiGLU needs N % 32 == 0");
+  const int64_t Nout = pair ? N / 2 : N;
+  const bool split = nsplit > 1 || raw;
+  if (split) {
+    TORCH_CHECK(slabs.has_value() && slabs->defined() && nsplit >= 1 && nsplit <= K / 64 && !out_f32 && (!raw || act == 0),
+                "gemm_image: a split of 1 to K / 64 parts into slabs, bf16 results");
+    CHECK_F32(*slabs);
+    TORCH_CHECK(slabs->is_cuda() && slabs->is_contiguous() && slabs->numel() >= nsplit * M * N, "gemm_image: workspace too small");
+    check_rc(rt_gemm_image(a.data_ptr(), a.stride(0), w.data_ptr(), slabs->data_ptr(), N, (int)M, (int)N, (int)K, 0, 3,
+                           (int)nsplit, nullptr, cur_stream()),
+             "gemm_image");
+    if (raw) return {};
+  }
+  Tensor c;
+  if (out.has_value() && out->defined()) {
+    c = *out;
+    TORCH_CHECK(c.is_cuda() && c.size(0) == M && c.size(1) == Nout && c.stride(1) == 1 && c.stride(0) % 8 == 0, "gemm_image: out");
+    TORCH_CHECK(c.scalar_type() == (out_f32 ? at::kFloat : at::kBFloat16), "gemm_image: out dtype");
+    CHECK_ALIGN16(c);
+  } else {
+    c = at::empty({M, Nout}, a.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  }
+  if (split)
+    check_rc(rt_gemm_splitk_reduce_glu(slabs->data_ptr<float>(), (int)nsplit, (int)M, (int)N, nullptr, (int)act, nullptr, 0,
+                                       c.data_ptr(), c.stride(0), GluArg(glu).ptr(), cur_stream()),
+             "gemm_splitk_reduce");
+  else
+    check_rc(rt_gemm_image(a.data_ptr(), a.stride(0), w.data_ptr(), c.data_ptr(), c.stride(0), (int)M, (int)N, (int)K, (int)act,
+                           out_f32 ? 1 : 0, 1, GluArg(glu).ptr(), cur_stream()),
+             "gemm_image");
   return c;
 }
 
@@ -1433,6 +1478,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_fwd", &swiglu_fwd);
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("embed", &embed);
+  m.def("gemm_image", &gemm_image, "act(A W^T) of 65..128 rows over a tile-ordered image", py::arg("a"), py::arg("w"),
+        py::arg("act") = 0, py::arg("out_f32") = false, py::arg("out") = py::none(), py::arg("nsplit") = 1,
+        py::arg("slabs") = py::none(), py::arg("raw") = false, py::arg("glu") = std::vector<double>());
   m.def("attn_packed", &attn_packed, "bidirectional self-attention of packed sequences", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("off"), py::arg("longest"), py::arg("H"), py::arg("D"), py::arg("scale"),
         py::arg("rel_bias") = py::none(), py::arg("rb_L") = 0);

@@ -825,6 +825,138 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Decode products for 64 < M <= 128 rows over tile-ordered weight images
+// ---------------------------------------------------------------------------------------------
+// The 256x128 LDS tiles of gemm_big_kernel take 1.2 us a K-step at these M, for 0.2 us of matrix work: their 8 waves
+// read A four times and B twice from LDS, and four barriers a step keep them in step. Here a wave owns 32 columns (PAIR: 16
+// gate and 16 up) of all rows and takes its weights from the image straight into registers, three 64-k chunks ahead, so only
+// X goes through LDS, with one barrier a chunk. A workgroup is 128 columns; few column groups are split over K into slabs.
+// us with cold weights at 65 / 128 rows, before -> now (split): SwiGLU 28672 x 4096 77.3 / 74.7 -> 46.4 / 56.6; 32000 x 4096
+// 75.3 / 75.9 -> 49.9 / 59.9; 6144 x 4096 20.9 / 22.8 -> 14.2 / 17.5 (5); 4096 x 4096 15.2 / 18.8 -> 10.7 / 13.4 (8); 4096 x
+// 14336 34.7 / 39.5 -> 24.1 / 28.1 (8); 10304 x 4096 28.9 / 30.5 -> 20.1 / 23.1 (3). At 256 rows, as two row halves or as waves
+// of 64 columns, the same loads keep LDS, L1 and the matrix cores equally busy and it was slower (SwiGLU 78.5 -> 87 and 100).
+template <int OUT, int RT, bool PAIR>  // OUT 0 bf16, 1 fp32, 3 fp32 slabs [split][M][N]; 16 RT rows
+__global__ __launch_bounds__(256, 2) void gemm128_image_kernel(GemmArgs p, int split) {
+  constexpr int DEPTH = 4, NG = 2, XQ = RT / 2, SLOT = 16 * RT * 128;
+  static_assert(RT % 2 == 0, "8 rows per X load and wave");
+  __shared__ __attribute__((aligned(16))) char smem[2 * SLOT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frow = lane & 15, g = lane >> 4;
+  const int cg = blockIdx.x / split, sp = blockIdx.x % split;
+  const int nc = p.K / 64, ngroups = p.N / 16;
+  const int t0 = (int)((long)sp * nc / split), nt = (int)((long)(sp + 1) * nc / split) - t0;  // its chunks of 64 k
+  auto group = [&](int j) {
+    return PAIR ? (j ? p.N / 32 : 0) + 4 * cg + wid : 8 * cg + 2 * wid + j;
+  };
+  const char* wb[NG];
+#pragma unroll
+  for (int j = 0; j < NG; ++j)
+    wb[j] = (const char*)p.B + ((long)min(group(j), ngroups - 1) * nc + t0) * 2048 + lane * 16;
+  // X row 8 (wid + 4 q) + lane / 8, 16-B piece lane % 8 of the chunk; it lies at piece ^ lds_swz(row) of its 128-B row
+  const bf16_t* xs[XQ];
+  char* xd[XQ];
+#pragma unroll
+  for (int q = 0; q < XQ; ++q) {
+    const int row = 8 * (wid + 4 * q) + (lane >> 3);
+    xs[q] = p.A + (long)min(row, p.M - 1) * p.lda + t0 * 64 + (lane & 7) * 8;
+    xd[q] = smem + row * 128 + (((lane & 7) ^ lds_swz(row)) << 4);
+  }
+  struct W { u32x4 v[NG][2]; };
+  struct X { u32x4 v[XQ]; };
+  auto load_w = [&](W& w, int i) {  // chunk t0 + i
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      w.v[j][0] = __builtin_bit_cast(u32x4, load_nt16(wb[j] + (long)i * 2048));
+      w.v[j][1] = __builtin_bit_cast(u32x4, load_nt16(wb[j] + (long)i * 2048 + 1024));
+    }
+  };
+  auto load_x = [&](X& x, int i) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) x.v[q] = *(const u32x4*)(xs[q] + (long)i * 64);
+  };
+  f32x4 acc[RT][NG];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int j = 0; j < NG; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  W w[DEPTH];
+  X xr[2];
+  // chunk i: the wave's part of its X tile goes to LDS, the barrier adds the other waves' (and that the reads of two
+  // chunks ago are done, which the buffer then served)
+  auto step = [&](W& cur, W& nxt, X& x, int i, bool all) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) *(u32x4*)(xd[q] + (i & 1) * SLOT) = x.v[q];
+    if (all || i + 2 < nt) load_x(x, i + 2);
+    if (all || i + DEPTH - 1 < nt) load_w(nxt, i + DEPTH - 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const char* slot = smem + (i & 1) * SLOT;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 f[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int row = 16 * t + frow;
+        f[t] = *(const bf16x8*)(slot + row * 128 + (((h * 4 + g) ^ lds_swz(row)) << 4));
+      }
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+          acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, cur.v[j][h]), f[t], acc[t][j], 0, 0, 0);
+    }
+  };
+  int i = 0;
+  if (nt >= 2 * DEPTH - 1) {
+    // no branch between a load and its use: the compiler's counted waits keep the chunks in flight
+    load_x(xr[0], 0);
+    load_x(xr[1], 1);
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d) load_w(w[d], d);
+    do {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) step(w[d], w[(d + DEPTH - 1) % DEPTH], xr[d & 1], i + d, true);
+      i += DEPTH;
+    } while (i + 2 * DEPTH - 2 < nt);
+  } else {
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      if (d < nt) load_x(xr[d], d);
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (d < nt) load_w(w[d], d);
+  }
+  for (; i < nt; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (i + d < nt) step(w[d], w[(d + DEPTH - 1) % DEPTH], xr[d & 1], i + d, false);
+  }
+  // acc[t][j][e] = C[row 16 t + frow][column 4 g + e of group j]
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int row = 16 * t + frow;
+    if (row >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < (PAIR ? 1 : NG); ++j) {
+      const int col = 16 * group(j) + 4 * g;
+      if (col >= (PAIR ? p.N / 2 : p.N)) continue;
+      if constexpr (OUT == 3) {
+        *(f32x4*)((float*)p.C + ((long)sp * p.M + row) * p.ldc + col) = acc[t][j];
+        continue;
+      }
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (PAIR) y[e] = glu(acc[t][0][e], acc[t][1][e], p.glu);
+        else y[e] = apply_act(acc[t][j][e], p.act);
+      }
+      if constexpr (OUT == 1) *(float4*)((float*)p.C + (long)row * p.ldc + col) = make_float4(y[0], y[1], y[2], y[3]);
+      else *(uint2*)((bf16_t*)p.C + (long)row * p.ldc + col) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+    }
+  }
+}
+
 // Shared tail of the M <= 64 kernels: split-K hand-off (write-through slabs + ticket, last arriver
 // reduces), in-GEMM RMS-norm scaling, SwiGLU pair / bias + activation + residual epilogues.
 // acc[j][r] = C[16 wid + 4 fq + r][16 j + frow] of the block's 64 columns; sq = sum of squares of
@@ -1694,6 +1826,28 @@ extern "C" int rt_shuffle_decode_weight_fp8(const void* src, void* dst, long N, 
   const int blocks = (int)std::min<long>((total + 255) / 256, 8192);
   hipLaunchKernelGGL(shuffle_decode_weight_fp8_kernel, dim3(blocks), dim3(256), 0, stream, (const uint4*)src,
                      (uint4*)dst, N, K);
+  RT_LAUNCH_CHECK();
+  return 0;
+}
+
+// act(A W^T) of 64 < M <= 128 rows over the tile-ordered image W of N % 16 == 0 weight rows, K % 64 == 0. out 0 bf16, 1
+// fp32, 3 the split's fp32 partial sums [split][M][ldc]. act ACT_SWIGLU: W = [gate; up], N % 32 == 0, N / 2 columns.
+extern "C" int rt_gemm_image(const void* A, long lda, const void* W, void* C, long ldc, int M, int N, int K, int act, int out,
+                             int split, const float* glu_p, hipStream_t stream) {
+  const bool pair = act == ACT_SWIGLU;
+  if (M <= 64 || M > 128 || N % (pair ? 32 : 16) || K % 64 || K <= 0 || lda % 8 || ldc % 4) return -1;
+  if (split < 1 || split > K / 64 || (out == 3 ? act != 0 : split != 1)) return -2;
+  GemmArgs p = {};
+  p.A = (const bf16_t*)A; p.lda = lda; p.B = (const bf16_t*)W; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.act = act;
+  if (glu_p) { p.glu.limit = glu_p[0]; p.glu.alpha = glu_p[1]; p.glu.offset = glu_p[2]; }
+  const dim3 grid((N + 127) / 128 * split), block(256);
+#define IMG(OUT, P)                                                                                       \
+  if (M <= 96) hipLaunchKernelGGL((gemm128_image_kernel<OUT, 6, P>), grid, block, 0, stream, p, split);   \
+  else hipLaunchKernelGGL((gemm128_image_kernel<OUT, 8, P>), grid, block, 0, stream, p, split)
+  if (out == 3) { IMG(3, false); }
+  else if (out == 1) { if (pair) { IMG(1, true); } else { IMG(1, false); } }
+  else { if (pair) { IMG(0, true); } else { IMG(0, false); } }
+#undef IMG
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -61,7 +61,7 @@ class DecoderLayer(nn.Module):
         self._fp8: Dict[str, ops.Fp8Cache] = {}
         # norm-folded weights of the fused decode path (Llama/Mistral)
         self._fold: Dict[str, ops.FoldCache] = {}
-        # tile-ordered images of the decode projections for batch <= 64
+        # tile-ordered images of the decode projections for batch <= 128
         self._shufc: Dict[str, ops.ShufCache] = {}
 
     # ---------------------------------------------------------------- helpers
@@ -90,6 +90,10 @@ class DecoderLayer(nn.Module):
             return None, None
         return None, self._shufc.setdefault(shufname, ops.ShufCache())
 
+    def _img(self, name: str, m: int):
+        """ShufCache of an unfolded decode weight at batch 65..128, if images are on."""
+        return self._shufc.setdefault(name, ops.ShufCache()) if 64 < m <= 128 and shuffle_enabled(m) else None
+
     # ---------------------------------------------------------------- fused decode step (M <= 64)
     def _w_eff(self, wname: str, gname: str):
         w = getattr(self, wname)
@@ -113,8 +117,9 @@ class DecoderLayer(nn.Module):
             c = self._f8(name)
             if c is not None:
                 c.get(w)
-        for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd)):
-            if name in self._shufc:  # images exist once a batch <= 64 decode ran
+        for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd),
+                        ("qkv_plain", self._w_eff("qkv_w", "qkv")), ("gate_up_plain", self._w_eff("gate_up_w", "gate_up"))):
+            if name in self._shufc:  # images exist once a decode of their batch sizes ran
                 self._shufc[name].get(w)
 
     def decode_fused(self, h, attend):
@@ -137,8 +142,8 @@ class DecoderLayer(nn.Module):
         f8, sh = self._dec_caches("down", "down", wd, m)
         return ops.gemm_decode(f, wd, residual=h, fp8=f8, shuf=sh)
 
-    def attn_in(self, x, residual, defer: bool = False):
-        """``defer`` (no-grad decode, batch > 64): the qkv GEMM may return unreduced split-K
+    def attn_in(self, x, residual, defer: Optional[bool] = None):
+        """``defer`` (given in no-grad decode, batch > 64) True: the qkv GEMM may return unreduced split-K
         partials (ops.SplitK) for the attention kernel to sum; ``x`` may itself be the previous
         layer's unreduced down projection (summed inside the norm)."""
         cfg = self.cfg
@@ -146,9 +151,11 @@ class DecoderLayer(nn.Module):
             h, residual = ops.layer_norm(x, self.ln1_w, self.ln1_b, cfg.norm_eps, residual)
         else:
             h, residual = ops.rms_norm(x, self.ln1_w, cfg.norm_eps, residual)
-        lin = ops.linear_deferred if (defer and cfg.arch != "opt") else ops.linear
-        qkv = lin(h, self.qkv_w, self._b("qkv_b"), lora=self._lg("qkv"), fp8=self._f8("qkv"))
-        return qkv, residual
+        kw = dict(lora=self._lg("qkv"), fp8=self._f8("qkv"))
+        if defer is not None and cfg.arch != "opt":
+            return ops.linear_deferred(h, self.qkv_w, self._b("qkv_b"), shuf=self._img("qkv_plain", h.shape[0]), raw=defer,
+                                       **kw), residual
+        return ops.linear(h, self.qkv_w, self._b("qkv_b"), **kw), residual
 
     def attn_in_rope(self, x, residual, rope):
         """Token-parallel forms (training / reference forwards, prefill): the qkv projection with the
@@ -164,11 +171,16 @@ class DecoderLayer(nn.Module):
                                        rope=(rope[0], rope[1], rope[2], (cfg.num_heads + cfg.num_kv_heads) * D, D))
         return qkv, residual, rotated
 
-    def mlp(self, a, residual, defer: bool = False):
+    def mlp(self, a, residual, defer: Optional[bool] = None):
         cfg = self.cfg
-        defer = defer and cfg.arch != "opt"
-        lin = ops.linear_deferred if defer else ops.linear
-        a = lin(a, self.o_w, self._b("o_b"), lora=self._lg("o"), fp8=self._f8("o"))
+        m = a.shape[0]
+        if defer is not None and cfg.arch != "opt":
+            img = lambda name: self._img(name, m)
+            lin = lambda x, w, b, name, **kw: ops.linear_deferred(x, w, b, shuf=img(name), raw=defer, **kw)
+        else:
+            img = lambda name: None
+            lin = lambda x, w, b, name, **kw: ops.linear(x, w, b, **kw)
+        a = lin(a, self.o_w, self._b("o_b"), "o", lora=self._lg("o"), fp8=self._f8("o"))
         if cfg.arch == "opt":
             h, residual = ops.layer_norm(a, self.ln2_w, self.ln2_b, cfg.norm_eps, residual)
             f = ops.linear(h, self.fc1_w, self.fc1_b, act=cfg.hidden_act, lora=self._lg("fc1"), fp8=self._f8("fc1"))
@@ -182,8 +194,9 @@ class DecoderLayer(nn.Module):
                 d = ops.swiglu_mlp(h, self.gate_up_w, self.down_w, self._lg("gate_up"), self._lg("down"))
             if d is None:
                 # act="swiglu": one fused skinny GEMM in no-grad decode, GEMM + SwiGLU kernel otherwise
-                f = ops.linear(h, self.gate_up_w, act="swiglu", lora=self._lg("gate_up"), fp8=self._f8("gate_up"))
-                d = lin(f, self.down_w, lora=self._lg("down"), fp8=self._f8("down"))
+                f = ops.linear(h, self.gate_up_w, act="swiglu", lora=self._lg("gate_up"), fp8=self._f8("gate_up"),
+                               shuf=img("gate_up_plain"))
+                d = lin(f, self.down_w, None, "down", lora=self._lg("down"), fp8=self._f8("down"))
         return d, residual
 
 
@@ -203,7 +216,7 @@ class CausalLM(nn.Module):
         if not cfg.tie_embeddings:
             self.lm_head = nn.Parameter(torch.empty(cfg.vocab_size, cfg.hidden_size, **kw))
         self._rope = None
-        self._head_shuf = None  # ShufCache of the LM head for decode at batch <= 64
+        self._head_shuf = None  # ShufCache of the LM head for decode at batch <= 128
         # decode steps run the fused 4-GEMM layer (norms folded into GEMMs, residual epilogues) up to
         # this batch: bf16 on the no-split tile-ordered GEMVs (M <= 16), then (17..64, serving) on the
         # tile-ordered kernels of up to four row tiles, with the in-GEMM RMS norm; above it the
@@ -270,12 +283,19 @@ class CausalLM(nn.Module):
         if torch.is_grad_enabled() and hidden.requires_grad:
             return ops.linear(hidden, self.head_weight)
         hw = self.head_weight
-        if ops.on_gpu(hidden) and shuffle_enabled(hidden.shape[0]) and hw.shape[0] % 16 == 0 and hw.is_contiguous():
-            # decode at batch <= 64: the tile-ordered image of the LM head (52 -> 48 us at batch 1, 59 -> 50 at 48)
-            if self._head_shuf is None:
-                self._head_shuf = ops.ShufCache()
-            return ops.native().gemm(hidden.contiguous(), self._head_shuf.get(hw), None, None, None, 0, out_f32,
-                                     None, None, 0.0, True)
+        m = hidden.shape[0]
+        if ops.on_gpu(hidden) and shuffle_enabled(m) and hw.shape[0] % 16 == 0 and hw.is_contiguous():
+            # decode at batch <= 128: the tile-ordered image of the LM head (52 -> 48 us at batch 1, 59 -> 50 at 48, 76 ->
+            # 60 at 128)
+            hidden = hidden.contiguous()
+            shuf = self._head_shuf if self._head_shuf is not None else ops.ShufCache()
+            image = ops.image_rows(hidden, hw, shuf) and not (out_f32 and ops.image_split(*hw.shape) > 1)
+            if m <= 64 or image:
+                self._head_shuf = shuf
+            if m <= 64:
+                return ops.native().gemm(hidden, shuf.get(hw), None, None, None, 0, out_f32, None, None, 0.0, True)
+            if image:
+                return ops.gemm_image(hidden, hw, shuf, 0, out_f32)
         return ops.gemm(hidden.contiguous(), hw, out_f32=out_f32)
 
     # ------------------------------------------------------------------ full forward
@@ -412,7 +432,7 @@ class CausalLM(nn.Module):
             return y
         residual = None
         # batch > 64: split-K GEMM partials flow unreduced into the attention prologue and the norms
-        defer = x.is_cuda and x.shape[0] > 64 and self.defer_splitk
+        defer = self.defer_splitk if x.is_cuda and x.shape[0] > 64 else None
         kv8 = getattr(cache, "fp8", False)
         for li, layer in enumerate(self.layers):
             qkv, residual = layer.attn_in(x, residual, defer)
@@ -512,9 +532,9 @@ def pack_enabled() -> bool:
 
 
 def shuffle_enabled(m: int) -> bool:
-    """Decode GEMMs at batch ``m`` <= 64 stream tile-ordered weight images (ops.ShufCache; 5-20 % faster
+    """Decode GEMMs at batch ``m`` <= 128 stream tile-ordered weight images (ops.ShufCache; 5-20 % faster
     than row-major up to batch 16, 3-50 % above). RAGTL_DECODE_SHUF=0 turns it off."""
-    return m <= 64 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+    return m <= 128 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
 
 
 def _normal_(p: torch.Tensor, std: float, g: torch.Generator):

@@ -130,7 +130,7 @@ class Glu:
 
 def project(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, shuf=None, out=None) -> torch.Tensor:
     """x w^T without grad, any shape and dtype: the MFMA kernels where their shape rules hold (bf16;
-    ``shuf``: tile-ordered image at M <= 64), ``gemm_any`` otherwise — also for fp32 operands, which
+    ``shuf``: tile-ordered image at M <= 128), ``gemm_any`` otherwise — also for fp32 operands, which
     stay fp32 throughout. ``out``: rows to write (may be strided)."""
     if not on_gpu(x):
         y = ref.gemm(x, w, out_f32=out_f32)
@@ -145,16 +145,48 @@ def project(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, shuf=None, 
         return gemm(x, w, out_f32=out_f32, out=out)
     if M <= 64:
         return native().gemm_big(x, w, ROW, ROW, None, None, None, 0, 1 if out_f32 else 0, 1, out)
+    if image_rows(x, w, shuf) and (not out_f32 or image_split(N, K) == 1):
+        return gemm_image(x, w, shuf, 0, out_f32, out)
     if out_f32 and N <= 512:  # narrow fp32 products (router logits): 64x64 tiles fill the chip
         return native().gemm_small(x, w, ROW, ROW, 1, 1, out, 64)
     return gemm(x, w, out_f32=out_f32, out=out)
 
 
 def shuffle_decode(m: int) -> bool:
-    """Decode products at ``m`` <= 64 rows stream tile-ordered weight images (RAGTL_DECODE_SHUF=0: off)."""
+    """Decode products at ``m`` <= 128 rows stream tile-ordered weight images (RAGTL_DECODE_SHUF=0: off)."""
     import os
 
-    return m <= 64 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+    return m <= 128 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+
+
+def image_rows(x: torch.Tensor, w: torch.Tensor, shuf, act: int = 0) -> bool:
+    """Whether :func:`gemm_image` takes x w^T: 65 to 128 rows, and not where a row's bits must not depend on their number."""
+    N, K = w.shape
+    return (shuf is not None and 64 < x.shape[0] <= 128 and shuffle_decode(x.shape[0]) and not _batch_invariant_on()
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.shape[1] == K and K % 64 == 0
+            and N % (32 if act == ACT_SWIGLU else 16) == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0)
+
+
+def image_split(N: int, K: int) -> int:
+    """K parts of an image product at 65..128 rows: up to a workgroup (128 columns of a part) per CU, of at least 4
+    chunks, at most 8 (4096 x 4096 at 128 rows: 8 parts 13.4 us, 4 15.8, 1 42.4; 10304 x 4096: 3 23.1, 4 28.9)."""
+    groups = (N + 127) // 128
+    return max(1, min(8, 256 // groups, K // 256))
+
+
+def gemm_image(x: torch.Tensor, w: torch.Tensor, shuf, act: int = 0, out_f32: bool = False, out=None, glu=(),
+               raw: bool = False):
+    """act(x w^T) over the tile-ordered image of ``w`` (:func:`image_rows`); ``raw``: the unreduced partial sums
+    (:class:`SplitK`) where it splits."""
+    M, K = x.shape
+    N = w.shape[0]
+    s = image_split(N, K)
+    if s == 1:
+        return native().gemm_image(x, shuf.get(w), act, out_f32, out, glu=glu)
+    slabs = torch.empty(s * M * N, dtype=torch.float32, device=x.device)
+    y = native().gemm_image(x, shuf.get(w), act, out_f32, out, s, slabs, raw, glu)
+    return SplitK(slabs, s, M, N, x.dtype) if raw else y
 
 
 def glu_project(x: torch.Tensor, w: torch.Tensor, glu: Glu, shuf=None) -> torch.Tensor:
@@ -169,6 +201,8 @@ def glu_project(x: torch.Tensor, w: torch.Tensor, glu: Glu, shuf=None) -> torch.
             sh = shuf is not None and shuffle_decode(M)
             return native().gemm(x, shuf.get(w) if sh else w, None, None, None, ACT_SWIGLU, False, None, None, 0.0, sh,
                                  glu.args())
+        if image_rows(x, w, shuf, ACT_SWIGLU):
+            return gemm_image(x, w, shuf, ACT_SWIGLU, glu=glu.args())
         if M > 64 and N % 256 == 0 and K % 8 == 0:
             s, bn = splitk_plan(M, N, K, ACT_SWIGLU)
             if s > 1:
@@ -190,6 +224,8 @@ def act_project(x: torch.Tensor, w: torch.Tensor, act: int, shuf=None) -> torch.
         if M <= 64 and K % 64 == 0:
             sh = shuf is not None and shuffle_decode(M) and N % 16 == 0
             return native().gemm(x, shuf.get(w) if sh else w, None, None, None, act, False, None, None, 0.0, sh)
+        if image_rows(x, w, shuf):
+            return gemm_image(x, w, shuf, act)
         if M > 64:
             return gemm(x, w, act=act)
     return native().act_any(project(x, w, True), act, x.dtype == torch.float32)
@@ -203,6 +239,8 @@ def branch_project(x: torch.Tensor, w: torch.Tensor, shuf=None):
         N = w.shape[0]
         if M <= 64:
             return project(x, w, True, shuf)
+        if image_rows(x, w, shuf):
+            return gemm_image(x, w, shuf, raw=True)
         if K % 8 == 0 and N % 16 == 0:
             s, bn = splitk_plan(M, N, K, 0)
             if s > 1:
@@ -757,9 +795,10 @@ def swiglu_mlp(x: torch.Tensor, w_gu: torch.Tensor, w_d: torch.Tensor, lora_gu: 
     return y.reshape(*shp[:-1], w_d.shape[0])
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, lora: Optional[LoRAGroup] = None, fp8=None):
+def linear(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, lora: Optional[LoRAGroup] = None, fp8=None, shuf=None):
     """y = act(x W^T (+ LoRA) + b) over the last dim of x. ``fp8`` (an ``ops.fp8.Fp8Cache``)
-    enables the fp8 inference path for this weight (no-grad only; LoRA merged first)."""
+    enables the fp8 inference path for this weight (no-grad only; LoRA merged first); ``shuf`` (ShufCache) the
+    tile-ordered image of a no-grad SwiGLU product of 65 to 128 rows."""
     act_id = ACT_IDS[act] if not isinstance(act, int) else act
     shp = x.shape
     x2 = x.reshape(-1, shp[-1])
@@ -809,7 +848,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, lora: Optional
                         q, sc = fp8.get(w_eff)
                         y = gemm_fp8(x2, q, sc, act=ACT_SWIGLU)
                     return y.reshape(*shp[:-1], w.shape[0] // 2)
-            y = gemm(x2, w_eff, None, None, None, ACT_SWIGLU)
+            if fp8 is None and image_rows(x2, w_eff, shuf, ACT_SWIGLU):
+                y = gemm_image(x2, w_eff, shuf, ACT_SWIGLU)
+            else:
+                y = gemm(x2, w_eff, None, None, None, ACT_SWIGLU)
             return y.reshape(*shp[:-1], w.shape[0] // 2)
         from .misc import swiglu
 
@@ -914,12 +956,14 @@ class SplitK:
         return native().splitk_reduce(self.slabs, self.nsplit, self.M, self.N, out)
 
 
-def linear_deferred(x: torch.Tensor, w: torch.Tensor, bias=None, lora: Optional[LoRAGroup] = None, fp8=None):
+def linear_deferred(x: torch.Tensor, w: torch.Tensor, bias=None, lora: Optional[LoRAGroup] = None, fp8=None, shuf=None,
+                    raw: bool = True):
     """``linear`` for no-grad decode steps that may return a :class:`SplitK` (unreduced) when the
     plan splits K (no bias / activation, merged or absent LoRA); else a tensor. ``fp8`` (config 5):
     the W8A8 split-K form — per-token fp8 activations, each split's partial scaled in its epilogue,
     the same slab consumers (the o / down projections of a 13B layer are 40 output tiles: without
-    the split they ran on 40 of 256 CUs)."""
+    the split they ran on 40 of 256 CUs). ``shuf`` (ShufCache): up to 128 rows over the tile-ordered image.
+    ``raw`` False: always reduced, with the same bits."""
     x2 = x.reshape(-1, x.shape[-1])
     use_lora = lora is not None and lora.enabled
     if (not on_gpu(x2) or torch.is_grad_enabled() or bias is not None or w.dtype != torch.bfloat16
@@ -929,6 +973,11 @@ def linear_deferred(x: torch.Tensor, w: torch.Tensor, bias=None, lora: Optional[
     w_eff = lora.merged_weight(w) if use_lora else w
     M, K = x2.shape
     N = w_eff.shape[0]
+    if fp8 is None and image_rows(x2, w_eff, shuf):
+        y = gemm_image(x2, w_eff, shuf, raw=raw)
+        return y if isinstance(y, SplitK) else y.reshape(*x.shape[:-1], N)
+    if not raw:
+        return linear(x, w, bias, None, lora, fp8)
     if fp8 is not None:
         from .fp8 import fp8_supported, quantize_fp8
 
@@ -986,7 +1035,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, act: int = 0, residual=None, n
 
 class ShufCache(dict):
     """Tile-ordered image of a decode weight (native ``shuffle_decode_weight``: each 16-row x 64-k
-    MFMA tile 2 KiB contiguous, so every load instruction of the M <= 64 kernels reads one 1-KiB
+    MFMA tile 2 KiB contiguous, so every load instruction of the M <= 128 kernels reads one 1-KiB
     run), rebuilt in place when the source's data pointer or version changes (graph-safe
     address). Pays on the split-K projections (down 28.5 -> 21.9 us at M = 1)."""
 

@@ -234,3 +234,41 @@ def test_packed_attention_equals_padded(D, H, bias, lens):
         assert torch.equal(got, want)
     x = torch.randn(B, S, 384, generator=g, device=DEV).bfloat16()
     assert torch.equal(ops.pool_normalize_packed(x[keep], off, S), ops.pool_normalize(x, n))
+
+
+# ---------------------------------------------------------------------------------------------- decode products, 65..128 rows
+@pytest.mark.parametrize("N,K,act", [(16, 64, 0), (48, 448, 0), (2048, 1024, 0), (4112, 2112, ops.ACT_RELU2), (33024, 256, 0),
+                                     (64, 128, 5), (1056, 1088, 5), (33024, 320, 5)])
+def test_image_products_65_to_128_rows(N, K, act):
+    """Tile-ordered products at 65..128 rows against 64 bits: odd numbers of row groups and chunks, chosen splits and
+    none, unreduced sums, fp32 and strided results. The bound on fp32 results is that of the sum's order."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    shuf = ops.ShufCache()
+    No = N // 2 if act == ops.ACT_SWIGLU else N
+    for M in (65, 96, 97, 128):
+        x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+        pre = x.double() @ w.double().t()
+        want = torch.nn.functional.silu(pre[:, :No]) * pre[:, No:] if act == ops.ACT_SWIGLU else ref.apply_act(pre, act)
+        bound = (x.double().abs() @ w.double().abs().t()).max().item() * K * 2.0 ** -24 + 1e-6
+        out = torch.full((M, No + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        assert ops.image_rows(x, w, shuf, act)
+        ops.gemm_image(x, w, shuf, act, out=out[:, :No])
+        # a bf16 rounding of the result, and of the pre-activations where a split hands those to the reduction
+        torch.testing.assert_close(out[:, :No].double(), want, rtol=2.0 ** -6, atol=4 * bound + 2.0 ** -8)
+        assert (out[:, No:] == 7).all()
+        if act == 0:
+            for s in {1, min(2, K // 64), min(7, K // 64)}:
+                slabs = torch.empty(s * M * N, dtype=torch.float32, device=DEV)
+                assert C.gemm_image(x, shuf.get(w), 0, False, None, s, slabs, True) is None
+                assert (slabs.view(s, M, N).double().sum(0) - pre).abs().max().item() <= bound
+            y = C.gemm_image(x, shuf.get(w), 0, True)
+            assert (y.double() - pre).abs().max().item() <= bound
+    for M in (64, 129):
+        x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+        assert not ops.image_rows(x, w, shuf, act)
+        with pytest.raises(RuntimeError):
+            C.gemm_image(x, shuf.get(w), act)
+    with ops.batch_invariant():
+        assert not ops.image_rows(torch.zeros(96, K, dtype=torch.bfloat16, device=DEV), w, shuf, act)
