@@ -719,7 +719,7 @@ Tensor gemm_fp8(const Tensor& a, const optional<Tensor>& sa, const Tensor& wq, c
 
 // ---------------------------------------------------------------------------------------------
 std::vector<Tensor> norm_fwd(bool layernorm, const Tensor& x, const optional<Tensor>& res, const Tensor& w,
-                             const optional<Tensor>& b, double eps) {
+                             const optional<Tensor>& b, double eps, bool keep_h) {
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w);
   TORCH_CHECK(x.is_contiguous(), "norm: x must be contiguous");
   const int64_t H = x.size(-1), T = x.numel() / H;
@@ -728,7 +728,7 @@ std::vector<Tensor> norm_fwd(bool layernorm, const Tensor& x, const optional<Ten
   if (res.has_value() && res->defined()) {
     CHECK_BF16(*res);
     TORCH_CHECK(res->is_contiguous() && res->numel() == x.numel(), "norm: residual shape");
-    h = at::empty_like(x);
+    if (keep_h) h = at::empty_like(x);
   }
   auto rstd = at::empty({T}, x.options().dtype(at::kFloat));
   Tensor mean = layernorm ? at::empty({T}, x.options().dtype(at::kFloat)) : Tensor();
@@ -1468,7 +1468,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("sa") = py::none(), py::arg("wq"), py::arg("sw"), py::arg("bias") = py::none(), py::arg("act") = 0,
         py::arg("out") = py::none(), py::arg("residual") = py::none(), py::arg("norm_eps") = 0.0,
         py::arg("w_shuffled") = false);
-  m.def("norm_fwd", &norm_fwd);
+  m.def("norm_fwd", &norm_fwd, py::arg("layernorm"), py::arg("x"), py::arg("res"), py::arg("w"), py::arg("b"), py::arg("eps"),
+        py::arg("keep_h") = true);
   m.def("splitk_reduce", &splitk_reduce, "sum of split-K slabs -> bf16");
   m.def("norm_fwd_slabs", &norm_fwd_slabs, "residual-add + norm whose input is a sum of split-K slabs");
   m.def("gemm_splitk_raw", &gemm_splitk_raw, "split-K NT GEMM into fp32 slabs (reduce fused into the consumer)");

@@ -122,10 +122,10 @@ class SentenceEncoder(nn.Module):
             qkv = ops.linear(x, layer.qkv_w, layer.qkv_b)
             a = attend(qkv[:, :H], qkv[:, H:2 * H], qkv[:, 2 * H:])
             a = ops.linear(a, layer.o_w, layer.o_b)
-            x, _ = ops.layer_norm(a, layer.ln1_w, layer.ln1_b, cfg.norm_eps, residual=x)
+            x, _ = ops.layer_norm(a, layer.ln1_w, layer.ln1_b, cfg.norm_eps, residual=x, keep=False)
             f = ops.linear(x, layer.fc1_w, layer.fc1_b, act=cfg.hidden_act)
             d = ops.linear(f, layer.fc2_w, layer.fc2_b)
-            x, _ = ops.layer_norm(d, layer.ln2_w, layer.ln2_b, cfg.norm_eps, residual=x)
+            x, _ = ops.layer_norm(d, layer.ln2_w, layer.ln2_b, cfg.norm_eps, residual=x, keep=False)
         return x
 
     @property

@@ -65,7 +65,7 @@ class _NormFn(torch.autograd.Function):
         return dx, dres, dw, db, None, None
 
 
-def _norm(x, w, b, eps, residual, layernorm):
+def _norm(x, w, b, eps, residual, layernorm, keep=True):
     from .linear import SplitK
 
     if isinstance(x, SplitK):  # the producing GEMM's split-K reduce fused into this pass
@@ -79,7 +79,7 @@ def _norm(x, w, b, eps, residual, layernorm):
         xs = x.contiguous()
         rs = residual.contiguous() if residual is not None else None
         if on_gpu(x):
-            y, h, _, _ = native().norm_fwd(layernorm, xs, rs, w, b, eps)
+            y, h, _, _ = native().norm_fwd(layernorm, xs, rs, w, b, eps, keep)
         else:
             y, h, _, _ = ref.norm(xs, w, b, eps, rs, layernorm)
         return y, (h if residual is not None else xs)
@@ -93,9 +93,10 @@ def rms_norm(x, w, eps=1e-6, residual=None):
     return _norm(x, w, None, eps, residual, False)
 
 
-def layer_norm(x, w, b=None, eps=1e-5, residual=None):
-    """(y, h): h = x + residual (or x), y = LayerNorm(h) * w + b."""
-    return _norm(x, w, b, eps, residual, True)
+def layer_norm(x, w, b=None, eps=1e-5, residual=None, keep=True):
+    """(y, h): h = x + residual (or x), y = LayerNorm(h) * w + b. ``keep`` False: h may be None where no backward
+    needs it (layers normalised at their end go on from y alone)."""
+    return _norm(x, w, b, eps, residual, True, keep)
 
 
 class MoePairs:

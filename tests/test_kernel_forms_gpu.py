@@ -272,3 +272,25 @@ def test_image_products_65_to_128_rows(N, K, act):
             C.gemm_image(x, shuf.get(w), act)
     with ops.batch_invariant():
         assert not ops.image_rows(torch.zeros(96, K, dtype=torch.bfloat16, device=DEV), w, shuf, act)
+
+
+# ---------------------------------------------------------------------------------------------- norms
+@pytest.mark.parametrize("H", [8, 384, 512, 520, 768, 1024, 1032])
+@pytest.mark.parametrize("T", [1, 5, 1023, 1024, 9001])
+def test_norm_wave_per_row_bits(H, T):
+    """Rows of up to 1024 columns have one bit pattern whichever form the number of rows picks (and up to 512 columns
+    that of the split-K form's workgroup a row), with and without the residual sum written."""
+    g = torch.Generator(device=DEV).manual_seed(H)
+    x, r = (torch.randn(T, H, generator=g, device=DEV).bfloat16() for _ in range(2))
+    w, b = (torch.randn(H, generator=g, device=DEV).bfloat16() for _ in range(2))
+    C = ops.native()
+    for ln in (False, True):
+        y, h, rstd, mean = C.norm_fwd(ln, x, r, w, b if ln else None, 1e-5)
+        y2, h2, rstd2, _ = C.norm_fwd(ln, x, r, w, b if ln else None, 1e-5, False)
+        assert h2 is None and torch.equal(y, y2) and torch.equal(rstd, rstd2)
+        ys, hs = C.norm_fwd_slabs(ln, x.float(), 1, T, H, r, w, b if ln else None, 1e-5)[:2]
+        assert torch.equal(y, ys) and torch.equal(h, hs)
+        hd = h.double()
+        want = hd - hd.mean(-1, keepdim=True) if ln else hd
+        want = want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double() + (b.double() if ln else 0)
+        torch.testing.assert_close(y.double(), want, rtol=2.0 ** -8 + 1e-4, atol=1e-4)
