@@ -50,6 +50,26 @@ def test_sampler_f32_topk_equals_general_form(V, top_k, top_p):
     assert same >= 4 * B - 2
 
 
+@pytest.mark.parametrize("V,top_k,top_p", [(32000, 256, 1.0), (32000, 200, 0.9), (32000, 50, 1.0), (512, 64, 1.0), (8, 8, 1.0),
+                                           (4096, 1024, 0.8), (40000, 500, 1.0)])
+def test_sampler_bf16_bound_from_thread_maxima(V, top_k, top_p):
+    """bf16 rows whose window fits badly (narrow, wide, plateaus, -inf) draw what the full-row search draws."""
+    B = 8
+    g = torch.Generator(device=DEV).manual_seed(V + top_k)
+    x = torch.randn(B, V, generator=g, device=DEV) * torch.tensor([0.01, 0.3, 1, 4, 30, 1, 1, 1], device=DEV)[:, None]
+    x[5] = 0.25
+    x[6, ::2] = float("-inf")
+    x[7] = torch.arange(V, device=DEV) / V
+    x = x.bfloat16()
+    for o in range(3):
+        off = torch.full((1,), o, dtype=torch.long, device=DEV)
+        got = []
+        for window in (1, 0):
+            with ops.tuning(sample_window=window):
+                got.append(ops.sample(x, 1 / 0.7, top_k=top_k, top_p=top_p, seed=3, offset=off))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 # ---------------------------------------------------------------------------------------------- decode attention
 @pytest.mark.parametrize("B,Hq,Hkv,Smax,window", [(33, 32, 8, 300, 0), (64, 32, 8, 1100, 200), (65, 32, 8, 1023, 0),
                                                   (65, 32, 8, 1024, 0), (70, 64, 8, 1030, 0), (130, 4, 4, 70, 0),
