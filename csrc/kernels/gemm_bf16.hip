@@ -11,7 +11,8 @@
 //
 // The weight-streaming kernels for M <= 64 (decode / small batch): gemm_decode_kernel (64 columns
 // per wave, split-K over waves and workgroups with an in-launch last-arriver reduction),
-// gemv16_kernel (M <= 16 on tile-ordered weight images), gemm_m64_kernel (16 < M <= 64, LDS-DMA
+// gemv16_kernel (M <= 16 on tile-ordered weight images), gemv64_kernel / gemm64_image_kernel (16 < M <= 64) and
+// gemm128_image_kernel (64 < M <= 128) on the same images, gemm_m64_kernel (16 < M <= 64, LDS-DMA
 // ring) and the W8A16 forms. M > 64 runs on the token-parallel family of gemm_big.hip.
 //
 // Replaces every projection GEMM of the reference's HF forward passes (reference
