@@ -119,7 +119,7 @@ class DecoderLayer(nn.Module):
                 c.get(w)
         for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd),
                         ("qkv_plain", self._w_eff("qkv_w", "qkv")), ("gate_up_plain", self._w_eff("gate_up_w", "gate_up"))):
-            if name in self._shufc:  # images exist once a decode of their batch sizes ran
+            if self._shufc.get(name):  # images exist once a decode of their batch sizes has used them
                 self._shufc[name].get(w)
 
     def decode_fused(self, h, attend):

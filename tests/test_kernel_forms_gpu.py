@@ -314,3 +314,30 @@ def test_norm_wave_per_row_bits(H, T):
         want = hd - hd.mean(-1, keepdim=True) if ln else hd
         want = want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double() + (b.double() if ln else 0)
         torch.testing.assert_close(y.double(), want, rtol=2.0 ** -8 + 1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("mode", ["bf16", "fp8", "adapters apart"])
+def test_decode_weight_images_only_where_read(mode):
+    """A decode of 80 rows lays out images of the weights that it reads through them; a refresh adds none, for fp8 weights or
+    adapters that are not merged either."""
+    from rag_tl_domainllm_optimizer_amd import models
+    from rag_tl_domainllm_optimizer_amd.generation import Generator, SamplingParams
+    from rag_tl_domainllm_optimizer_amd.models.config import ModelConfig
+
+    cfg = ModelConfig(arch="mistral", vocab_size=512, hidden_size=512, num_layers=1, num_heads=4, num_kv_heads=1,
+                      head_dim=128, intermediate_size=1024, max_position=128, norm_eps=1e-5, name="t-d128")
+    m = models.CausalLM(cfg, device=DEV, dtype=torch.bfloat16, seed=6)
+    if mode == "fp8":
+        m.set_fp8(True)
+    elif mode != "bf16":
+        m.add_lora(8, 16.0, "all")
+    Generator(m, 80, 32, DEV, use_graph=False).generate([[3, 4, 5]] * 80, SamplingParams(max_new_tokens=3, do_sample=False),
+                                                         pad_id=0, eos_ids=[-1])
+    layer = m.layers[0]
+    held = {k for k, c in layer._shufc.items() if c}
+    layer.refresh_decode_weights()
+    assert {k for k, c in layer._shufc.items() if c} == held
+    if mode == "bf16":
+        assert held == {"qkv_plain", "o", "gate_up_plain", "down"}
+    elif mode == "fp8":
+        assert not held
