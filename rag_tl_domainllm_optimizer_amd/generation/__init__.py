@@ -610,9 +610,13 @@ class ContinuousBatcher:
         g._nb = 1
         self._prev_merged = g.model.set_lora_merged(g.merge_lora) if hasattr(g.model, "set_lora_merged") else None
         if hasattr(g.model, "refresh_decode_weights"):
-            g.model.refresh_decode_weights(MB)
+            g.model.refresh_decode_weights()  # of every bucket: a graph of an earlier batcher may be replayed
+        params_of = getattr(g.model, "parameters", None)
+        self._read = [p for p in params_of() if not p.is_inference()] if params_of else []
+        self._adapters = [a for layer in getattr(g.model, "layers", ()) for a in getattr(layer, "lora", {}).values()]
         if T > 1:
             g._ensure_graph(params, self.eos, self.eos_list, pad_id, T)  # captured while no row is active
+        self._seen = self._weight_versions()
         self.rows = {}  # row -> (tag, prompt_len, steps at admission)
         self.free = list(range(MB))
         self.steps = 0
@@ -621,6 +625,10 @@ class ContinuousBatcher:
         if self._prev_merged is not None:
             self.gen.model.set_lora_merged(self._prev_merged)
             self._prev_merged = None
+
+    def _weight_versions(self) -> int:
+        """Grows with each change in place of a weight that decode steps read (25 us for 32 layers)."""
+        return sum(p._version for p in self._read) + sum(a.merged._version for a in self._adapters if a.merged is not None)
 
     def free_rows(self) -> int:
         return len(self.free)
@@ -699,6 +707,13 @@ class ContinuousBatcher:
             g._nb = nb
             if self.T > 1:
                 g._ensure_graph(self.params, self.eos, self.eos_list, self.pad_id, self.T)
+        seen = self._weight_versions()
+        if seen != self._seen:
+            # weights changed in place while requests run (a loaded or updated adapter): a replay reads
+            # images derived from them
+            self._seen = seen
+            if hasattr(g.model, "refresh_decode_weights"):
+                g.model.refresh_decode_weights(nb)
         for _ in range(n):
             if not (self.pending and self._mixed_step()):
                 g._replay(self.params, self.eos, self.pad_id)

@@ -104,23 +104,37 @@ class DecoderLayer(nn.Module):
             g.refresh(dtype=w.dtype)
         return g.merged_weight(w)
 
+    def _w_plain(self, wname: str, gname: str):
+        """The weight that the layer's products without grad multiply by; None where an adapter runs beside it."""
+        g = self._lg(gname)
+        if g is None or not g.enabled:
+            return getattr(self, wname)
+        return self._w_eff(wname, gname) if g.use_merged else None
+
     @torch.no_grad()
-    def refresh_decode_weights(self):
+    def refresh_decode_weights(self, fused: bool = True, plain: bool = True):
         """Bring the merged / folded / fp8 decode weights up to date eagerly (graph replays of a
-        captured decode step only read them)."""
+        captured decode step only read them): those of the ``fused`` layer and of the ``plain`` one at
+        65..128 rows, whose images exist once a decode of such a batch has used them."""
         if self.cfg.arch == "opt":
             return
-        wq = self._fold.setdefault("qkv", ops.FoldCache()).get(self._w_eff("qkv_w", "qkv"), self.ln1_w)
-        wgu = self._fold.setdefault("gate_up", ops.FoldCache()).get(self._w_eff("gate_up_w", "gate_up"), self.ln2_w)
-        wo, wd = self._w_eff("o_w", "o"), self._w_eff("down_w", "down")
-        for name, w in (("qkv_folded", wq), ("gate_up_folded", wgu), ("o", wo), ("down", wd)):
-            c = self._f8(name)
-            if c is not None:
-                c.get(w)
-        for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd),
-                        ("qkv_plain", self._w_eff("qkv_w", "qkv")), ("gate_up_plain", self._w_eff("gate_up_w", "gate_up"))):
-            if self._shufc.get(name):  # images exist once a decode of their batch sizes has used them
-                self._shufc[name].get(w)
+        if fused:
+            wq = self._fold.setdefault("qkv", ops.FoldCache()).get(self._w_eff("qkv_w", "qkv"), self.ln1_w)
+            wgu = self._fold.setdefault("gate_up", ops.FoldCache()).get(self._w_eff("gate_up_w", "gate_up"), self.ln2_w)
+            wo, wd = self._w_eff("o_w", "o"), self._w_eff("down_w", "down")
+            for name, w in (("qkv_folded", wq), ("gate_up_folded", wgu), ("o", wo), ("down", wd)):
+                c = self._f8(name)
+                if c is not None:
+                    c.get(w)
+            for name, w in (("qkv", wq), ("o", wo), ("gate_up", wgu), ("down", wd)):
+                if self._shufc.get(name):
+                    self._shufc[name].get(w)
+        if plain:
+            for name, proj in (("qkv_plain", "qkv"), ("o", "o"), ("gate_up_plain", "gate_up"), ("down", "down")):
+                if self._shufc.get(name) and not (fused and name == proj):  # o, down: the fused layer's too
+                    w = self._w_plain(proj + "_w", proj)
+                    if w is not None:
+                        self._shufc[name].get(w)
 
     def decode_fused(self, h, attend):
         """One Llama/Mistral layer of a decode step in four kernels: [RMSNorm folded into the qkv
@@ -471,19 +485,19 @@ class CausalLM(nn.Module):
         return prev
 
     def refresh_decode_weights(self, batch: Optional[int] = None):
-        """Eagerly refresh the images the fused decode layer's graph replays read (norm-folded /
-        tile-ordered / fp8 weights). ``batch``: the decode batch about to run — above the fused
-        layer's limit none of them is read, so batch-256 rollouts skip the refresh (a later
-        small-batch generation refreshes them before its replays). Same-box A/B: within noise
+        """Eagerly refresh the derived weights that graph replays of a decode step read (norm-folded /
+        tile-ordered / fp8). ``batch``: the decode batch about to run, None for any. Up to the fused
+        layer's limit its weights, from there to 128 rows the images of the unfolded ones, and the
+        head's image in both; above, a step reads none of them, so batch-256 rollouts skip the refresh
+        (a later small-batch generation refreshes them before its replays). Same-box A/B: within noise
         (profiles/r6/bench_decode_refresh_gating_ab.log)."""
-        if batch is not None:
-            fp8 = bool(self.layers) and self.layers[0].fp8_enabled
-            if batch > (self.fused_decode_max_batch_fp8 if fp8 else self.fused_decode_max_batch):
-                return
-        if self.fused_decode:
-            for layer in self.layers:
-                layer.refresh_decode_weights()
-        if self._head_shuf is not None:
+        fp8 = bool(self.layers) and self.layers[0].fp8_enabled
+        limit = self.fused_decode_max_batch_fp8 if fp8 else self.fused_decode_max_batch
+        fused = self.fused_decode and (batch is None or batch <= limit)
+        plain = batch is None or (not fused and 64 < batch <= 128)
+        for layer in self.layers if fused or plain else ():
+            layer.refresh_decode_weights(fused, plain)
+        if self._head_shuf is not None and (batch is None or batch <= 128):
             self._head_shuf.get(self.head_weight)
 
     def set_fp8(self, on: bool = True, train: Optional[bool] = None):

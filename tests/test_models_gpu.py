@@ -6,8 +6,8 @@ import pytest
 import torch
 
 from rag_tl_domainllm_optimizer_amd import models, ops
-from rag_tl_domainllm_optimizer_amd.generation import Generator, SamplingParams
-from rag_tl_domainllm_optimizer_amd.models.config import PRESETS
+from rag_tl_domainllm_optimizer_amd.generation import ContinuousBatcher, Generator, SamplingParams
+from rag_tl_domainllm_optimizer_amd.models.config import PRESETS, ModelConfig
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -97,6 +97,84 @@ def test_fused_decode_follows_adapter_updates():
             m.set_lora_merged(prev)
         err = float((lp - out.logprobs).abs().max())
         assert err <= 1e-2, (step, err)
+
+def _d128_lora():
+    cfg = ModelConfig(arch="mistral", vocab_size=512, hidden_size=512, num_layers=2, num_heads=4, num_kv_heads=1,
+                      head_dim=128, intermediate_size=1024, max_position=128, norm_eps=1e-5, name="t-d128")
+    m = models.CausalLM(cfg, device=DEV, dtype=torch.bfloat16, seed=4)
+    m.add_lora(8, 16.0, "all", seed=1)
+    return m
+
+
+def _new_adapters(m, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    with torch.no_grad():
+        for q in m.lora_parameters():
+            q.copy_(torch.randn(q.shape, device=DEV, generator=g, dtype=q.dtype) * 0.08)
+    m.refresh_lora()
+
+
+def _off_policy(m, prompt_ids, start, tokens, lengths, logprobs):
+    """Largest distance of recorded log-probs from teacher forcing on the model's merged weights of now."""
+    from rag_tl_domainllm_optimizer_amd.train.common import score_sequences
+
+    prev = m.set_lora_merged(True)
+    try:
+        with torch.no_grad():
+            lp, _, _, mask = score_sequences(m, prompt_ids, start, tokens, lengths, 1 / 0.7)
+    finally:
+        m.set_lora_merged(prev)
+    return float(((lp - logprobs) * mask).abs().max())
+
+
+# Two engines apart: logits of up to 4 rounded to bf16 on both sides (2^-7 each) over the temperature, and as much from the
+# hidden states' rounding.
+OFF_POLICY = 4 * 2.0 ** -7 / 0.7
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("rows", [20, 48, 65, 80, 128, 140])
+def test_decode_graphs_follow_adapter_updates(rows, fused):
+    """A graph captured before an adapter update replays with the new adapters, whichever derived weights its batch reads:
+    folded images up to 64 rows, plain ones to 128 (and the head's), the merged weights above."""
+    m = _d128_lora()
+    m.fused_decode = fused
+    gen = Generator(m, rows, 64, DEV)
+    p = SamplingParams(max_new_tokens=8, temperature=0.7, top_k=0, seed=5)
+    prompts = [[5 + b % 7, 9, 33, 41, 7, 8, 9, 10 + b] for b in range(rows)]
+    for step in range(3):
+        _new_adapters(m, step)
+        out = gen.generate(prompts, p, pad_id=0, eos_ids=[-1])
+        err = _off_policy(m, out.prompt_ids, out.prompt_start, out.tokens, out.lengths, out.logprobs)
+        assert err <= OFF_POLICY, (step, err)
+
+
+@pytest.mark.parametrize("rows", [1, 40, 72, 100])
+def test_batcher_graphs_follow_adapter_updates(rows):
+    """Requests admitted after an adapter update decode with the new adapters: in a batcher that lives on, and in a new one
+    that finds its bucket's graph captured."""
+    m = _d128_lora()
+    gen = Generator(m, 128, 64, DEV)
+    p = SamplingParams(max_new_tokens=8, temperature=0.7, top_k=0, seed=5)
+    prompts = [[5 + b % 7, 9, 33, 41, 7, 8, 9, 10 + b] for b in range(rows)]
+
+    def serve(cb):
+        cb.admit_many(prompts, list(range(rows)))
+        cb.step(8)
+        done = sorted(cb.collect(), key=lambda r: r.tag)
+        assert len(done) == rows
+        toks, lps = (torch.tensor([getattr(r, n) for r in done], device=DEV) for n in ("tokens", "logprobs"))
+        err = _off_policy(m, torch.tensor(prompts, device=DEV), torch.zeros(rows, dtype=torch.int32, device=DEV), toks,
+                          torch.full((rows,), 8, device=DEV), lps)
+        assert err <= OFF_POLICY, err
+
+    for batcher in range(2):
+        cb = ContinuousBatcher(gen, p, eos_ids=[-1])
+        for update in range(2):
+            _new_adapters(m, 2 * batcher + update)
+            serve(cb)
+        cb.close()
+        _new_adapters(m, 9)  # between two batchers, too
 
 
 def test_shuffled_decode_weights_match_row_major(monkeypatch):
