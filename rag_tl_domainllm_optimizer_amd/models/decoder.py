@@ -546,9 +546,8 @@ def pack_enabled() -> bool:
 
 
 def shuffle_enabled(m: int) -> bool:
-    """Decode GEMMs at batch ``m`` <= 128 stream tile-ordered weight images (ops.ShufCache; 5-20 % faster
-    than row-major up to batch 16, 3-50 % above). RAGTL_DECODE_SHUF=0 turns it off."""
-    return m <= 128 and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
+    """``ops.shuffle_decode``: whether decode GEMMs at batch ``m`` stream tile-ordered weight images."""
+    return ops.shuffle_decode(m)
 
 
 def _normal_(p: torch.Tensor, std: float, g: torch.Generator):

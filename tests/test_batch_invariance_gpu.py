@@ -205,3 +205,37 @@ def test_ppo_resume_bitwise(tmp_path, full):
         if "time" in k or "per_s" in k or k.endswith("_s") or not isinstance(v, (int, float)):
             continue
         assert v == m_b[k] or (v != v and m_b[k] != m_b[k]), (k, v, m_b[k])
+
+
+@pytest.mark.parametrize("N,K", [(4096, 4096), (1040, 512), (10304, 1024)])
+def test_products_with_weight_images_across_rows(N, K):
+    """Inside ``ops.batch_invariant()`` a row's bits are the same at 17 to 140 rows, also where a tile-ordered image of the
+    weight is at hand: plain products and logits over the whole range, gated and activated ones at 17 to 64 rows (their
+    kernel's K order depends on the weight's shape alone there)."""
+    g = torch.Generator(device=DEV).manual_seed(N)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    x = torch.randn(140, K, generator=g, device=DEV).bfloat16()
+    shuf = ops.ShufCache()
+    with ops.batch_invariant():
+        full = ops.project(x, w, shuf=shuf)
+        full32 = ops.project(x, w, True, shuf)
+        for m in (17, 24, 33, 48, 64, 65, 80, 128):
+            assert torch.equal(ops.project(x[:m], w, shuf=shuf), full[:m]), m
+            assert torch.equal(ops.project(x[:m], w, True, shuf), full32[:m]), m
+        glu = ops.Glu()
+        for f in (lambda y: ops.glu_project(y, w, glu, shuf), lambda y: ops.act_project(y, w, ops.ACT_RELU2, shuf)):
+            if N % 64 == 0:
+                y = f(x[:64])
+                for m in (17, 24, 33, 48):
+                    assert torch.equal(f(x[:m]), y[:m]), m
+
+
+def test_logits_across_rows():
+    cfg = PRESETS["tiny-mistral"]
+    m = models.CausalLM(cfg, device=DEV, dtype=torch.bfloat16, seed=1)
+    h = torch.randn(140, cfg.hidden_size, generator=torch.Generator(device=DEV).manual_seed(0), device=DEV).bfloat16()
+    with torch.no_grad(), ops.batch_invariant():
+        for f32 in (False, True):
+            full = m.logits(h, f32)
+            for n in (17, 24, 48, 64, 65, 80, 128):
+                assert torch.equal(m.logits(h[:n], f32), full[:n]), (n, f32)
