@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(1024) void sample_topk_f32_kernel(
       float above = 0.f;
       for (int i = 0; i < total; ++i)
         if (ckey[i] > k) above += __expf(val(ckey[i]) * inv_temp - M);
-      keep = above < target;
+      keep = !(above >= target);  // a NaN leaves nothing to compare: all stay, as in sample_row
     }
     if (keep) {
       const int i = cidx[j];

@@ -50,6 +50,32 @@ def test_sampler_f32_topk_equals_general_form(V, top_k, top_p):
     assert same >= 4 * B - 2
 
 
+def test_sampler_f32_nan_logits_keep_general_draw():
+    """A NaN among the logits leaves no nucleus mass to compare with: every top-k token stays in the draw, as in the
+    general form. NaNs count as the largest logits on both sides; infinities of both signs beside them."""
+    V, B = 4096, 8
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(B, V, generator=g, device=DEV) * 3
+    x[0, 17] = float("nan")
+    x[1, ::5] = float("nan")
+    x[2, 3], x[2, 9] = float("nan"), float("inf")
+    x[3, 100:] = float("-inf")
+    x[4] = float("-inf")
+    x[5, 7] = float("inf")
+    wide = torch.empty(B, V + 1, device=DEV)
+    wide[:, :V] = x
+    for top_p in (1.0, 0.9):
+        drawn = set()
+        for o in range(8):
+            off = torch.full((1,), o, dtype=torch.long, device=DEV)
+            t1, l1 = ops.sample(x, 1 / 0.7, top_k=40, top_p=top_p, seed=3, offset=off)
+            t0, l0 = ops.sample(wide[:, :V], 1 / 0.7, top_k=40, top_p=top_p, seed=3, offset=off)
+            assert torch.equal(t1, t0), (top_p, o, t1, t0)
+            assert torch.equal(l1.isnan(), l0.isnan())
+            drawn.add(int(t1[0]))
+        assert len(drawn) > 1
+
+
 @pytest.mark.parametrize("V,top_k,top_p", [(32000, 256, 1.0), (32000, 200, 0.9), (32000, 50, 1.0), (512, 64, 1.0), (8, 8, 1.0),
                                            (4096, 1024, 0.8), (40000, 500, 1.0)])
 def test_sampler_bf16_bound_from_thread_maxima(V, top_k, top_p):
