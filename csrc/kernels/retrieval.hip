@@ -66,7 +66,7 @@ __device__ __forceinline__ uint32_t okey(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-constexpr int TOPK_CAND = 1024;  // max survivors sorted in LDS (k + ties)
+constexpr int TOPK_CAND = 1024;  // candidates of a row held in LDS
 
 struct TopkShared {
   unsigned hist[256];
@@ -85,16 +85,14 @@ __device__ __forceinline__ void topk_write(float v, int idx, int k, int at, long
   out_i[row * k + at] = id;
 }
 
-// one row of any length and content: 4-pass radix select, sort of what reaches the k-th key
+// A row with more candidates than the list holds (plateaus, fewer than K finite scores): 4-pass radix select of the K-th
+// key, then exactly K entries in cv / ci: the fewer than K above it, and of its ties those of the lowest indices
 template <int NT>
-__device__ void topk_row(const float* s, long row, int N, int k, const long* __restrict__ idmap, long ldmap, int finite,
-                         float* __restrict__ out_v, long* __restrict__ out_i, TopkShared& sh) {
+__device__ void topk_select(const float* s, int N, int K, TopkShared& sh) {
   unsigned* hist = sh.hist;
-  float* cv = sh.cv;
-  int* ci = sh.ci;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   uint32_t prefix = 0, mask = 0;
-  unsigned remaining = (unsigned)min(k, N);
+  unsigned remaining = (unsigned)K;
   for (int shift = 24; shift >= 0; shift -= 8) {
     for (int b = tid; b < 256; b += NT) hist[b] = 0;
     __syncthreads();
@@ -119,35 +117,33 @@ __device__ void topk_row(const float* s, long row, int N, int k, const long* __r
     mask |= 255u << shift;
     __syncthreads();
   }
-  // gather survivors (key >= prefix): strictly-greater first guaranteed < k, ties fill the rest
   if (tid == 0) sh.cnt = 0;
-  for (int i = tid; i < TOPK_CAND; i += NT) { cv[i] = -INFINITY; ci[i] = 0x7fffffff; }
   __syncthreads();
   for (int i = tid; i < N; i += NT) {
     const float v = s[i];
-    if (okey(v) >= prefix) {
+    if (okey(v) > prefix) {
       const unsigned slot = atomicAdd(&sh.cnt, 1u);
-      if (slot < TOPK_CAND) { cv[slot] = v; ci[slot] = i; }
+      if (slot < TOPK_CAND) { sh.cv[slot] = v; sh.ci[slot] = i; }
     }
   }
   __syncthreads();
-  // bitonic sort descending by value, ascending index on ties
-  for (int size = 2; size <= TOPK_CAND; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = tid; i < TOPK_CAND; i += NT) {
-        const int j = i ^ stride;
-        if (j > i) {
-          const bool desc = (i & size) == 0;
-          const float vi = cv[i], vj = cv[j];
-          const int ii = ci[i], ij = ci[j];
-          const bool i_first = vi > vj || (vi == vj && ii < ij);
-          if (desc != i_first) { cv[i] = vj; cv[j] = vi; ci[i] = ij; ci[j] = ii; }
-        }
-      }
-      __syncthreads();
+  int at = (int)sh.cnt;
+  for (int i0 = 0; i0 < N && at < K; i0 += NT) {
+    const int i = i0 + tid;
+    const float v = i < N ? s[i] : 0.f;
+    const bool tie = i < N && okey(v) == prefix;
+    const unsigned long long in_wave = __ballot(tie);
+    if (lane == 0) hist[wid] = (unsigned)__popcll(in_wave);
+    __syncthreads();
+    int slot = at + (int)__popcll(in_wave & ((1ull << lane) - 1ull));
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      if (w < wid) slot += (int)hist[w];
+      at += (int)hist[w];
     }
+    if (tie && slot < K) { sh.cv[slot] = v; sh.ci[slot] = i; }
+    __syncthreads();
   }
-  for (int i = tid; i < k; i += NT) topk_write(cv[i], ci[i], k, i, row, idmap, ldmap, finite, out_v, out_i);
 }
 
 // scores [nq, N] fp32 (row stride ld) -> vals/ids [nq, k] sorted descending (ties: lower index first); ids optionally
@@ -157,7 +153,7 @@ __device__ void topk_row(const float* s, long row, int N, int k, const long* __r
 // the row's k-th largest score that few surplus elements reach: the threads that hold one place theirs in LDS, and
 // every candidate counts the candidates ahead of it, which is its place in the result. Two passes over the row at
 // most, no histogram, no sort (four passes and a sort of 1024 before): top 16 of 512 and top 3 of 9600, one row,
-// 88 -> 8.3 and 10.8 us each. Rows with more than TOPK_CAND candidates (plateaus) go through topk_row.
+// 88 -> 8.3 and 10.8 us each. Rows with more than TOPK_CAND candidates go through topk_select first.
 // NT: a wave where its 64 maxima suffice (k <= 32) and hold 16 elements each at most (k-means assignment: 65536 rows
 // of 512), 1024 threads for long rows, 256 between.
 template <int NT>
@@ -201,13 +197,13 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
       }
     }
   __syncthreads();
-  const int n = (int)sh.cnt;
+  int n = (int)sh.cnt;
   if (n > TOPK_CAND) {
     __syncthreads();  // every thread has read cnt
-    topk_row<NT>(s, row, N, k, idmap, ldmap, finite, out_v, out_i, sh);
-    return;
+    topk_select<NT>(s, N, K, sh);
+    n = K;
   }
-  // those with fewer than K keys above their own, then their places by value and index (as topk_row's sort)
+  // those with fewer than K keys above their own, then their places by value and index
   for (int j = tid; j < n; j += NT) {
     const uint32_t key = okey(sh.cv[j]);
     int above = 0;

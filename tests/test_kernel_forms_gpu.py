@@ -149,6 +149,49 @@ def test_topk_forms(nq, N, k):
         assert bool((v[:, n:] == float("-inf")).all()) and bool((i[:, n:] == -1).all())
 
 
+@pytest.mark.parametrize("N,k", [(1500, 3), (5000, 3), (5000, 128), (9600, 40), (100003, 512)])
+def test_topk_rows_with_more_ties_than_candidates(N, k):
+    """Rows whose k-th score is shared by more entries than the candidate list holds: all larger scores come first, then the
+    ties of the lowest indices; the same for fewer than k finite scores. The order of a stable sort, each time."""
+    g = torch.Generator(device=DEV).manual_seed(N + k)
+    s = torch.full((7, N), 0.5, device=DEV)
+    s[0, -1] = 1.0
+    s[1, torch.randperm(N, generator=g, device=DEV)[:k - 1]] = 0.75 + torch.rand(k - 1, generator=g, device=DEV)
+    s[2] = float("-inf")
+    s[2, N - k // 2 - 1:] = torch.randn(k // 2 + 1, generator=g, device=DEV)
+    s[3] = torch.where(torch.rand(N, generator=g, device=DEV) < 0.5, 0.5, 0.25)
+    s[3, N // 2] = 2.0
+    s[4] = float("-inf")
+    s[5] = torch.where(torch.rand(N, generator=g, device=DEV) < 0.9, 0.0, -1.0)
+    s[5, -1] = 1e-30
+    cid = torch.randint(0, 1 << 40, s.shape, generator=g, device=DEV)
+    vs, order = torch.sort(s, dim=-1, descending=True, stable=True)
+    want = torch.where(torch.isfinite(vs), cid.gather(1, order), torch.full_like(cid, -1))[:, :k]
+    for _ in range(3):
+        v, i = ops.topk(s, k, cid, finite=True)
+        assert torch.equal(v, vs[:, :k])
+        assert torch.equal(i, want)
+
+
+def test_ivf_search_with_fewer_documents_than_asked():
+    """Fewer than k documents in the probed lists, whose slots are more than the candidate list holds: all are found."""
+    from rag_tl_domainllm_optimizer_amd.retrieval.index import IVFIndex
+
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(1500, 64, generator=g)
+    x[:1400] = x[0] + 0.01 * torch.randn(1400, 64, generator=g)  # one list holds most documents
+    x = torch.nn.functional.normalize(x, dim=-1)
+    ix = IVFIndex(64, nlist=24, device=DEV)
+    ix.train(x, niter=4)
+    ix.add(x)
+    q = x[1400:].to(DEV)
+    for nprobe in (2, 4, 24):
+        held = ix.lsize[ix._coarse(q, nprobe).long()].sum(1).clamp(max=500).tolist()
+        _, ids = ix.search(q, 500, nprobe=nprobe)
+        found = [len(row[row >= 0].unique()) for row in ids]
+        assert found == held, nprobe
+
+
 @pytest.mark.parametrize("d", [8, 72, 384, 1000])
 @pytest.mark.parametrize("l2", [False, True])
 def test_ivf_scan_lists(d, l2):
