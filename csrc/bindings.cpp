@@ -117,7 +117,6 @@ struct TuningField {
 static const TuningField kTuningFields[] = {
     {"decode_mw_bh", &rt::Tuning::decode_mw_bh, nullptr},
     {"decode_w4_bh", &rt::Tuning::decode_w4_bh, nullptr},
-    {"decode_w4_smax", &rt::Tuning::decode_w4_smax, nullptr},
     {"attn_lpt", &rt::Tuning::attn_lpt, nullptr},
     {"decode_mw_kpp", &rt::Tuning::decode_mw_kpp, nullptr},
     {"decode_mw_smax", &rt::Tuning::decode_mw_smax, nullptr},

@@ -17,7 +17,6 @@ struct Tuning {
   // waves per (row, kv head) pair (attention.hip, rt_attn_decode_waves):
   int decode_mw_bh = 320;     // pairs below which there are always several (8 below 256, 4 from there)
   int decode_w4_bh = 512;     // pairs up to which there are 4 (bf16 caches)
-  int decode_w4_smax = 1024;  // cache slots from which there are 4 whatever the pairs (bf16 caches)
   int decode_mw_kpp = 512;    // keys per partition of the 8-wave small-batch kernel past decode_mw_smax cache slots
   int decode_mw_smax = 1024;  // cache slots up to which it runs one partition per kv head (fewer: measured slower
                               // at 456 slots, profiles/r5/decode_b1_deferred_partition_merge.log)

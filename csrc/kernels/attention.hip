@@ -2080,13 +2080,20 @@ static int rt_attn_decode_mw_np(int Smax, int np_ws) {
 }
 // Waves per (batch row, kv head) of the MFMA decode attention; 0: sizes it does not take. A one-wave pair is a
 // serial chain of 16-key tiles (0.8 us each, three in flight), so with few pairs on the chip, long rows or rows of
-// different lengths the pair's keys go round 4 waves that merge through LDS (2.5 us more). us a call, 8 kv heads x
-// 4 queries, rows of 50..80 / 150..300 / 400..600 / 150..1200 keys, one wave | four:
-//    48 rows: 11 / 22 / 40 / 71 | 11 / 17 / 27 / 41     64 rows: 11 / 23 / 42 / 74 | 12 / 19 / 30 / 45
-//    96 rows: 12 / 27 / 47 / 81 | 18 / 29 / 49 / 69    256 rows: 20 / 52 / 99 / 148 | 35 / 61 / 101 / 137
-// The line lies at 512 pairs (two workgroups of four waves per CU) and, beyond it, at caches of 1024 slots, whose
-// rows are past 500 keys when half full. Split-K slabs of the qkv product are summed by the one-wave kernel only: up
-// to 512 pairs that saves a reduce launch (5 us), less than the longer chain costs from about 400 keys on.
+// different lengths the pair's keys go round 4 waves that merge through LDS (2.5 us more). us a call in caches of 1088 and
+// (last) 1280 slots, rows of 50..80 / 150..300 / 400..600 / 150..1200 keys, one wave | four:
+//    400 pairs, 40 kv heads, 1 query:   9.3 / 20.8 / 38.0 / 63.1  | 10.5 / 16.6 / 26.6 / 33.1
+//    512 pairs, 16 kv heads, 2 queries: 10.2 / 21.8 / 40.2 / 68.0 | 11.5 / 17.9 / 29.6 / 41.6
+//    512 pairs,  8 kv heads, 4 queries: 11.5 / 23.4 / 42.0 / 73.4 | 12.3 / 19.1 / 30.4 / 44.6
+//    640 pairs, 40 kv heads, 1 query:   10.9 / 23.1 / 42.7 / 71.1 | 15.2 / 23.0 / 36.8 / 52.2
+//    640 pairs,  8 kv heads, 4 queries: 12.7 / 24.6 / 45.0 / 77.9 | 17.5 / 25.3 / 41.2 / 55.9
+//    960 pairs,  8 kv heads, 4 queries: 14.5 / 28.4 / 53.4 / 86.0 | 20.8 / 31.6 / 53.3 / 73.9
+//   2560 pairs, 40 kv heads, 1 query:   24.8 / 58.9 / 125 / 188   | 37.7 / 68.1 / 117 / 165
+//   2560 pairs,  8 kv heads, 4 queries: 27.0 / 62.8 / 129 / 177   | 43.2 / 72.1 / 125 / 163
+// The line lies at 512 pairs, two workgroups of four waves per CU. Beyond it four waves gain only where the rows are
+// long, which neither the host nor the size of the cache tells: short answers in a long cache lost up to 60 %. Split-K
+// slabs of the qkv product are summed by the one-wave kernel only: up to 512 pairs that saves a reduce launch (5 us),
+// less than the longer chain costs from about 400 keys on.
 static int rt_attn_decode_waves(int B, int Hq, int Hkv, int D, int Smax, int NP, bool kv8, bool slabs) {
   const int G = Hkv ? Hq / Hkv : 0;
   const long pairs = (long)B * Hkv;
@@ -2097,8 +2104,7 @@ static int rt_attn_decode_waves(int B, int Hq, int Hkv, int D, int Smax, int NP,
   if (kv8) return one ? 1 : multi ? DEC_MW : 0;
   if (!multi || many != one) return one ? 1 : 0;
   if (!one) return 4;
-  if (pairs <= tuning().decode_w4_bh) return slabs && Smax < 512 ? 1 : 4;
-  return Smax >= tuning().decode_w4_smax && !slabs ? 4 : 1;
+  return pairs > tuning().decode_w4_bh || (slabs && Smax < 512) ? 1 : 4;
 }
 // whether the decode attention sums the qkv product's split-K slabs itself
 extern "C" int rt_attn_decode_slabs_ok(int B, int Hq, int Hkv, int D, int Smax, int NP, int kv8) {

@@ -122,6 +122,22 @@ def test_decode_attention_waves_per_pair(B, Hq, Hkv, Smax, window):
     assert torch.equal(kc.nan_to_num(), k2.nan_to_num()) and torch.equal(vc.nan_to_num(), v2.nan_to_num())
 
 
+@pytest.mark.parametrize("B,Hkv,G", [(13, 40, 1), (33, 16, 2), (65, 8, 4), (65, 8, 8)])
+def test_decode_attention_form_whatever_the_free_slots(B, Hkv, G):
+    """Beyond 512 (row, kv head) pairs short rows cost no more in a cache of many slots: the same form, so the same bits."""
+    D, n = 128, 70
+    g = torch.Generator(device=DEV).manual_seed(B)
+    kv = torch.randn(2, B, Hkv, n, D, generator=g, device=DEV).to(torch.bfloat16)
+    qkv = torch.randn(B, (G + 2) * Hkv * D, generator=g, device=DEV).to(torch.bfloat16)
+    slot = torch.randint(0, n, (B,), generator=g, device=DEV, dtype=torch.int32)
+    outs = []
+    for Smax in (n, 1023, 1024, 2048):
+        kc, vc = torch.zeros(2, B, Hkv, Smax, D, dtype=torch.bfloat16, device=DEV)
+        kc[:, :, :n], vc[:, :, :n] = kv[0], kv[1]
+        outs.append(ops.decode_step_attention(qkv, kc, vc, slot, slot + 1, G * Hkv))
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
 # ---------------------------------------------------------------------------------------------- retrieval
 @pytest.mark.parametrize("nq,N,k", [(1, 40, 40), (3, 512, 16), (2, 1024, 32), (2, 1025, 32), (2, 700, 33), (5, 4097, 128),
                                     (2, 4096, 128), (2, 300, 129), (4, 9600, 3), (1, 100003, 512), (2, 70, 100), (300, 64, 1)])
