@@ -1039,19 +1039,39 @@ class ShufCache(dict):
     """Tile-ordered image of a decode weight (native ``shuffle_decode_weight``: each 16-row x 64-k
     MFMA tile 2 KiB contiguous, so every load instruction of the M <= 128 kernels reads one 1-KiB
     run), rebuilt in place when the source's data pointer or version changes (graph-safe
-    address). Pays on the split-K projections (down 28.5 -> 21.9 us at M = 1)."""
+    address). Pays on the split-K projections (down 28.5 -> 21.9 us at M = 1).
+
+    A write that leaves the version alone (``p.data.copy_``, a kernel's own) has to advance it
+    (``torch.autograd.graph.increment_version``). Calls on other streams wait for the image where it is
+    still being laid out; a stream capture that finds none of the source's current version records one
+    of its own, since what it records runs at the replays only. Copies start empty."""
 
     @torch.no_grad()
     def get(self, w: torch.Tensor) -> torch.Tensor:
         key = (w.data_ptr(), w._version)
         if dict.get(self, "key") != key:
+            if torch.cuda.is_current_stream_capturing():
+                return native().shuffle_decode_weight(w.contiguous(), None)
             buf = dict.get(self, "w")
             if buf is None or buf.shape != w.shape or buf.device != w.device:
                 buf = torch.empty_like(w, memory_format=torch.contiguous_format)
                 self["w"] = buf
+            stream = torch.cuda.current_stream(w.device)
             native().shuffle_decode_weight(w.contiguous(), buf)
+            self["laid"] = (stream, stream.record_event())
             self["key"] = key
+        laid = dict.get(self, "laid")
+        if laid is not None and not torch.cuda.is_current_stream_capturing():  # a capture begins with a synchronisation
+            stream, event = laid
+            here = torch.cuda.current_stream(w.device)
+            if event.query():
+                self.pop("laid", None)
+            elif here != stream:
+                here.wait_event(event)
         return self["w"]
+
+    def __reduce__(self):
+        return type(self), ()
 
 
 class FoldCache(dict):

@@ -379,6 +379,45 @@ def test_image_products_65_to_128_rows(N, K, act):
         assert not ops.image_rows(torch.zeros(96, K, dtype=torch.bfloat16, device=DEV), w, shuf, act)
 
 
+def test_weight_images_across_streams_captures_and_copies():
+    """An image that one stream is still laying out is waited for on another, also after the weight has changed; a capture
+    without a warm-up leaves no image behind that only its replay fills; copies and pickles start empty."""
+    import copy
+    import pickle
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    w = (torch.randn(4096, 4096, generator=g, device=DEV) / 64).bfloat16()
+    x = torch.randn(100, 4096, generator=g, device=DEV).bfloat16()
+    shuf, a, b = ops.ShufCache(), torch.cuda.Stream(), torch.cuda.Stream()
+
+    def check(y):
+        torch.testing.assert_close(y.double(), x.double() @ w.double().t(), rtol=2.0 ** -6, atol=2.0 ** -6)
+
+    for _ in range(2):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(100_000_000)
+            shuf.get(w)
+        with torch.cuda.stream(b):
+            y = ops.project(x, w, shuf=shuf)
+        torch.cuda.synchronize()
+        check(y)
+        w.mul_(-0.5)
+    for m in (16, 48, 100):
+        shuf = ops.ShufCache()
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            y = ops.project(x[:m], w, shuf=shuf)
+        check(torch.cat([ops.project(x[:m], w, shuf=shuf), x.double()[m:] @ w.double().t()]))
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            check(torch.cat([y, x.double()[m:] @ w.double().t()]))
+    assert shuf and not copy.deepcopy(shuf) and not copy.copy(shuf) and not pickle.loads(pickle.dumps(shuf))
+
+
 # ---------------------------------------------------------------------------------------------- norms
 @pytest.mark.parametrize("H", [8, 384, 512, 520, 768, 1024, 1032])
 @pytest.mark.parametrize("T", [1, 5, 1023, 1024, 9001])
