@@ -177,6 +177,19 @@ def test_batcher_graphs_follow_adapter_updates(rows):
         _new_adapters(m, 9)  # between two batchers, too
 
 
+@pytest.mark.parametrize("hidden", [96, 128])
+def test_logits_of_widths_without_images(hidden):
+    """Heads whose width is no multiple of 64 have no tile-ordered image: their logits come from the row-major weight."""
+    cfg = ModelConfig(arch="mistral", vocab_size=512, hidden_size=hidden, num_layers=1, num_heads=2, num_kv_heads=1,
+                      head_dim=32, intermediate_size=128, max_position=64, norm_eps=1e-5, name="t-narrow")
+    m = models.CausalLM(cfg, device=DEV, dtype=torch.bfloat16, seed=4)
+    h = torch.randn(140, hidden, generator=torch.Generator(device=DEV).manual_seed(0), device=DEV).bfloat16()
+    want = h.double() @ m.head_weight.double().t()
+    with torch.no_grad():
+        for n in (32, 48, 64, 65, 128, 140):
+            torch.testing.assert_close(m.logits(h[:n]).double(), want[:n], rtol=2.0 ** -7, atol=1e-4)
+
+
 def test_shuffled_decode_weights_match_row_major(monkeypatch):
     """Batch-1 decode on the tile-ordered weight images (qkv, o, gate_up, down, lm_head) == the
     row-major weights, bitwise at a common split-K, including after an adapter update (the images
