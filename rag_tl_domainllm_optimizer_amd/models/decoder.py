@@ -298,12 +298,12 @@ class CausalLM(nn.Module):
             return ops.linear(hidden, self.head_weight)
         hw = self.head_weight
         m = hidden.shape[0]
-        if ops.on_gpu(hidden) and shuffle_enabled(m) and hw.shape[0] % 16 == 0 and (m <= 16 or hw.shape[1] % 64 == 0) \
-                and hw.is_contiguous():
+        shuf = self._head_shuf if self._head_shuf is not None else ops.ShufCache()
+        if ops.on_gpu(hidden) and ops.image_held(shuf, hw, m) and hw.shape[0] % 16 == 0 and \
+                (m <= 16 or hw.shape[1] % 64 == 0) and hw.is_contiguous():
             # decode at batch <= 128: the tile-ordered image of the LM head (52 -> 48 us at batch 1, 59 -> 50 at 48, 76 ->
             # 60 at 128)
             hidden = hidden.contiguous()
-            shuf = self._head_shuf if self._head_shuf is not None else ops.ShufCache()
             image = ops.image_rows(hidden, hw, shuf) and not (out_f32 and ops.image_split(*hw.shape) > 1)
             if m <= 64 or image:
                 self._head_shuf = shuf

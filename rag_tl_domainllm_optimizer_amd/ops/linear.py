@@ -140,7 +140,7 @@ def project(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, shuf=None, 
     if x.dtype != torch.bfloat16 or K % 8 or N % 8 or x.stride(0) % 8 or x.data_ptr() % 16 or M == 0:
         return native().gemm_any(x, w, out_f32, out)
     if M <= 64 and K % 64 == 0:
-        if shuf is not None and shuffle_decode(M) and N % 16 == 0:
+        if image_held(shuf, w, M) and N % 16 == 0:
             return native().gemm(x, shuf.get(w), None, None, None, 0, out_f32, out, None, 0.0, True)
         return gemm(x, w, out_f32=out_f32, out=out)
     if M <= 64:
@@ -161,10 +161,16 @@ def shuffle_decode(m: int) -> bool:
     return m <= (16 if _batch_invariant_on() else 128) and os.environ.get("RAGTL_DECODE_SHUF", "1") != "0"
 
 
+def image_held(shuf, w: torch.Tensor, m: int) -> bool:
+    """Whether a product of ``m`` rows streams the image of ``w`` that ``shuf`` holds. Weights made in inference mode tell
+    nothing of their changes: above 16 rows they are read as they lie."""
+    return shuf is not None and shuffle_decode(m) and (m <= 16 or not w.is_inference())
+
+
 def image_rows(x: torch.Tensor, w: torch.Tensor, shuf, act: int = 0) -> bool:
     """Whether :func:`gemm_image` takes x w^T: 65 to 128 rows, and not where a row's bits must not depend on their number."""
     N, K = w.shape
-    return (shuf is not None and 64 < x.shape[0] <= 128 and shuffle_decode(x.shape[0])
+    return (64 < x.shape[0] <= 128 and image_held(shuf, w, x.shape[0])
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.shape[1] == K and K % 64 == 0
             and N % (32 if act == ACT_SWIGLU else 16) == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0)
@@ -200,7 +206,7 @@ def glu_project(x: torch.Tensor, w: torch.Tensor, glu: Glu, shuf=None) -> torch.
     N = w.shape[0]
     if x.dtype == torch.bfloat16 and x.is_contiguous() and M > 0:
         if M <= 64 and K % 64 == 0 and N % 64 == 0:
-            sh = shuf is not None and shuffle_decode(M)
+            sh = image_held(shuf, w, M)
             return native().gemm(x, shuf.get(w) if sh else w, None, None, None, ACT_SWIGLU, False, None, None, 0.0, sh,
                                  glu.args())
         if image_rows(x, w, shuf, ACT_SWIGLU):
@@ -224,7 +230,7 @@ def act_project(x: torch.Tensor, w: torch.Tensor, act: int, shuf=None) -> torch.
     N = w.shape[0]
     if x.dtype == torch.bfloat16 and M > 0 and K % 8 == 0 and N % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
         if M <= 64 and K % 64 == 0:
-            sh = shuf is not None and shuffle_decode(M) and N % 16 == 0
+            sh = image_held(shuf, w, M) and N % 16 == 0
             return native().gemm(x, shuf.get(w) if sh else w, None, None, None, act, False, None, None, 0.0, sh)
         if image_rows(x, w, shuf):
             return gemm_image(x, w, shuf, act)

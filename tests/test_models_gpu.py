@@ -190,6 +190,32 @@ def test_logits_of_widths_without_images(hidden):
             torch.testing.assert_close(m.logits(h[:n]).double(), want[:n], rtol=2.0 ** -7, atol=1e-4)
 
 
+@pytest.mark.parametrize("rows", [80, 128])
+def test_decode_of_weights_made_in_inference_mode(rows):
+    """Weights without a version counter have no image that could follow them: decode of 65 to 128 rows, logits and
+    products of 17 to 128 read them as they lie."""
+    cfg = PRESETS["tiny-mistral"]
+    p = SamplingParams(max_new_tokens=6, do_sample=False)
+    prompts = [[3, 4, 5 + b] for b in range(rows)]
+    outs = []
+    for mode in (True, False):
+        with torch.inference_mode(mode):
+            m = models.CausalLM(cfg, device=DEV, dtype=torch.bfloat16, seed=4)
+            w = torch.zeros(512, 256, device=DEV, dtype=torch.bfloat16) + 0.5
+            assert m.head_weight.is_inference() == w.is_inference() == mode
+            outs.append(Generator(m, rows, 64, DEV, use_graph=False).generate(prompts, p, pad_id=0, eos_ids=[-1]))
+            h = torch.ones(rows, cfg.hidden_size, device=DEV, dtype=torch.bfloat16)
+            for n in (17, 64, rows):
+                assert bool((ops.project(h[:n], w, shuf=ops.ShufCache()) == 128).all())
+                with torch.no_grad():
+                    torch.testing.assert_close(m.logits(h[:n]).double(), h[:n].double() @ m.head_weight.double().t(),
+                                               rtol=2.0 ** -7, atol=1e-3)
+    # the same products in another K order: a row may part where two tokens are as likely to within that
+    same = (outs[0].tokens == outs[1].tokens).all(1)
+    assert int(same.sum()) >= 0.9 * rows
+    torch.testing.assert_close(outs[0].logprobs[same], outs[1].logprobs[same], rtol=0.0, atol=OFF_POLICY)
+
+
 def test_shuffled_decode_weights_match_row_major(monkeypatch):
     """Batch-1 decode on the tile-ordered weight images (qkv, o, gate_up, down, lm_head) == the
     row-major weights, bitwise at a common split-K, including after an adapter update (the images
