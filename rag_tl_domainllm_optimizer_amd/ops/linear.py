@@ -163,8 +163,10 @@ def shuffle_decode(m: int) -> bool:
 
 def image_held(shuf, w: torch.Tensor, m: int) -> bool:
     """Whether a product of ``m`` rows streams the image of ``w`` that ``shuf`` holds. Weights made in inference mode tell
-    nothing of their changes: above 16 rows they are read as they lie."""
-    return shuf is not None and shuffle_decode(m) and (m <= 16 or not w.is_inference())
+    nothing of their changes: above 16 rows they are read as they lie, and weights that the row-major kernels refuse
+    (column strides, rows off 16 bytes) are left to them."""
+    return shuf is not None and shuffle_decode(m) and (
+        m <= 16 or (not w.is_inference() and w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0))
 
 
 def image_rows(x: torch.Tensor, w: torch.Tensor, shuf, act: int = 0) -> bool:
@@ -1025,7 +1027,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, act: int = 0, residual=None, n
                     return native().gemm_fp8(x, None, qs, sc, None, act, None, residual, norm_eps, True)
                 q, sc = fp8.get(w)
                 return native().gemm_fp8(x, None, q, sc, None, act, None, residual, norm_eps)
-        if shuf is not None and x.shape[0] <= 64 and w.shape[0] % 16 == 0:
+        if image_held(shuf, w, x.shape[0]) and x.shape[0] <= 64 and w.shape[0] % 16 == 0:
             return native().gemm(x, shuf.get(w), None, None, None, act, False, None, residual, norm_eps, True)
         return native().gemm(x, w, None, None, None, act, False, None, residual, norm_eps)
     y = x.float() @ w.float().t()

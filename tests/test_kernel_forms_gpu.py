@@ -379,6 +379,21 @@ def test_image_products_65_to_128_rows(N, K, act):
         assert not ops.image_rows(torch.zeros(96, K, dtype=torch.bfloat16, device=DEV), w, shuf, act)
 
 
+@pytest.mark.parametrize("m", [17, 48, 64, 65, 128])
+def test_weights_that_row_major_products_refuse(m):
+    """Column strides and rows off 16 bytes are refused with an image at hand as without one; rows further apart are not."""
+    K, N = 256, 512
+    x = torch.ones(m, K, dtype=torch.bfloat16, device=DEV)
+    buf = torch.ones(N * (K + 8) + 8, dtype=torch.bfloat16, device=DEV)
+    for w in (buf[:N * K].view(K, N).t(), buf[1:1 + N * K].view(N, K), buf[:N * (K + 4)].view(N, K + 4)[:, :K]):
+        with pytest.raises(RuntimeError):
+            ops.project(x, w, shuf=ops.ShufCache())
+        with pytest.raises(RuntimeError):
+            ops.act_project(x, w, ops.ACT_RELU2, ops.ShufCache())
+    w = buf[:N * (K + 8)].view(N, K + 8)[:, :K]
+    assert bool((ops.project(x, w, shuf=ops.ShufCache()) == K).all())
+
+
 def test_weight_images_across_streams_captures_and_copies():
     """An image that one stream is still laying out is waited for on another, also after the weight has changed; a capture
     without a warm-up leaves no image behind that only its replay fills; copies and pickles start empty."""
