@@ -6,6 +6,8 @@
 // of a row ranks the few scores that reach a bound from its threads' maxima (no full sort of N = 100k scores).
 #include "rt_common.h"
 
+#include <algorithm>
+
 namespace rt {
 
 // x [B, S, H] bf16, lengths [B] (off: text b is rows [off[b], off[b + 1]) of x [rows, H]) -> out [B, H] fp32 (L2-normalised if norm != 0). One workgroup a text; a stream
@@ -243,14 +245,15 @@ __global__ __launch_bounds__(64) void ivf_scan_kernel(const bf16_t* __restrict__
                                                       int l2, int maxlen, float* __restrict__ cand,
                                                       long* __restrict__ cand_ids) {
   extern __shared__ float qs[];
-  const int p = blockIdx.x, qi = blockIdx.y, j = blockIdx.z * 64 + threadIdx.x;
+  const int p = blockIdx.x, qi = blockIdx.y;
+  const long j0 = blockIdx.z * 64L, step = gridDim.z * 64L;
   const int L = probes[(long)qi * nprobe + p];
   const int b0 = L >= 0 ? lstart[L] : 0;
   const int len = L >= 0 ? min(lsize[L], maxlen) : 0;
   float* out = cand + ((long)qi * nprobe + p) * maxlen;
   long* oid = cand_ids + ((long)qi * nprobe + p) * maxlen;
-  if ((int)blockIdx.z * 64 >= len) {
-    if (j < maxlen) { out[j] = -INFINITY; oid[j] = -1; }
+  if (j0 >= len) {
+    for (long j = j0 + threadIdx.x; j < maxlen; j += step) { out[j] = -INFINITY; oid[j] = -1; }
     return;
   }
   // |q|^2 in four interleaved parts, added in order
@@ -271,9 +274,13 @@ __global__ __launch_bounds__(64) void ivf_scan_kernel(const bf16_t* __restrict__
     for (int w = 0; w < 4; ++w) qn += wave_sum(part[w]);
   }
   __syncthreads();
-  if (j >= maxlen) return;
-  if (j < len) {
-    const bf16_t* vr = vecs + (long)(b0 + j) * d;
+  for (long j = j0 + threadIdx.x; j < maxlen; j += step) {
+    if (j >= len) {
+      out[j] = -INFINITY;
+      oid[j] = -1;
+      continue;
+    }
+    const bf16_t* vr = vecs + (b0 + j) * d;
     float s = 0.f;
     int c = 0;
     for (; c + 64 <= d; c += 64) {
@@ -296,9 +303,6 @@ __global__ __launch_bounds__(64) void ivf_scan_kernel(const bf16_t* __restrict__
     }
     out[j] = l2 ? 2.f * s - sqnorm[b0 + j] - qn : s;
     oid[j] = ids[b0 + j];
-  } else {
-    out[j] = -INFINITY;
-    oid[j] = -1;
   }
 }
 
@@ -365,8 +369,10 @@ extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int 
   if (d % 8 != 0 || (l2 && !sqnorm)) return -1;
   if (nq == 0) return 0;
   if (maxlen <= 0) return 0;
-  hipLaunchKernelGGL(ivf_scan_kernel, dim3(nprobe, nq, (maxlen + 63) / 64), dim3(64), d * sizeof(float), stream, (const bf16_t*)q, d,
-                     probes, nprobe, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, cand, cand_ids);
+  // a grid's third dimension ends at 65535: longer lists (over 4 million vectors) go round
+  const unsigned pieces = (unsigned)std::min((maxlen + 63L) / 64, 65535L);
+  hipLaunchKernelGGL(ivf_scan_kernel, dim3(nprobe, nq, pieces), dim3(64), d * sizeof(float), stream, (const bf16_t*)q, d, probes,
+                     nprobe, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, cand, cand_ids);
   RT_LAUNCH_CHECK();
   return 0;
 }

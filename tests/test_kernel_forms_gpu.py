@@ -237,6 +237,26 @@ def test_ivf_scan_lists(d, l2):
     torch.testing.assert_close(cand.double(), want.view(3, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
 
 
+def test_ivf_scan_of_a_list_longer_than_a_grid():
+    """A list of more 64-vector pieces than a grid's third dimension holds, and a short one beside it."""
+    d, n = 8, 65535 * 64 + 1000
+    g = torch.Generator(device=DEV).manual_seed(0)
+    vecs = torch.randn(n + 70, d, generator=g, device=DEV).to(torch.bfloat16)
+    size = torch.tensor([n, 70], dtype=torch.int32, device=DEV)
+    start = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    q = torch.randn(1, d, generator=g, device=DEV).to(torch.bfloat16)
+    ids = torch.arange(n + 70, device=DEV) + 7
+    maxlen = n + 30
+    cand, cid = ops.ivf_scan(q, torch.tensor([[1, 0]], dtype=torch.int32, device=DEV), start, size, vecs, ids, maxlen)
+    want = torch.full((1, 2, maxlen), float("-inf"), dtype=torch.float64, device=DEV)
+    wid = torch.full((1, 2, maxlen), -1, device=DEV)
+    full = (vecs.double() @ q[0].double())
+    want[0, 0, :70], want[0, 1, :n] = full[n:], full[:n]
+    wid[0, 0, :70], wid[0, 1, :n] = ids[n:], ids[:n]
+    assert torch.equal(cid.view(1, 2, maxlen), wid)
+    torch.testing.assert_close(cand.view(1, 2, maxlen).double(), want, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("B,S,H", [(3, 1, 8), (2, 17, 384), (4, 70, 768), (2, 9, 20), (1, 33, 2056)])
 def test_pool_normalize_forms(B, S, H):
     g = torch.Generator(device=DEV).manual_seed(S)
