@@ -38,6 +38,13 @@ class Encoder:
     def dim(self) -> int:
         return self.model.cfg.hidden_size
 
+    def _as_made(self) -> bool:
+        """Whether model and tokenizer do their parts of a padded batch as this package has them do: others (a pooling of
+        one's own, another tokenizer) are called for each."""
+        return all(getattr(type(o), n, None) is getattr(c, n) and n not in vars(o) for o, c, names in (
+            (self.model, SentenceEncoder, ("forward", "encode_ids")), (self.tokenizer, Tokenizer, ("encode_batch", "pad", "_wrap")))
+            for n in names)
+
     @torch.no_grad()
     def encode(self, texts: Sequence[str], normalize: bool = True) -> torch.Tensor:
         """-> fp32 [N, dim] on the model's device (unit vectors when normalize)."""
@@ -45,6 +52,15 @@ class Encoder:
         N = len(texts)
         out = torch.empty(N, self.dim, dtype=torch.float32, device=self.device)
         if N == 0:
+            return out
+        if not self._as_made():
+            enc = self.tokenizer.encode_batch(texts, True, self.max_length)
+            order = sorted(range(N), key=lambda i: len(enc[i]))
+            for s in range(0, N, self.batch_size):
+                idx = order[s:s + self.batch_size]
+                batch = self.tokenizer.pad([enc[i] for i in idx], side="right", device=self.device)
+                emb = self.model.encode_ids(batch["input_ids"], batch["lengths"], normalize)
+                out[torch.tensor(idx, device=self.device)] = emb.float()
             return out
         # every batch is tokenised and uploaded ahead of the first forward: between them the host only launches
         order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device,

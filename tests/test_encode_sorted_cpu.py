@@ -47,3 +47,35 @@ def test_encode_sorted_refuses():
     for batch, max_length in ((0, 4), (4, 0)):
         with pytest.raises(RuntimeError):
             tok.encode_sorted(["a"], max_length, batch, "cpu")
+
+
+def test_encoder_calls_parts_of_ones_own():
+    """A model that pools in its own way, another tokenizer and patched objects are called as for padded batches."""
+    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder
+
+    class FirstToken(models.SentenceEncoder):
+        def encode_ids(self, input_ids, lengths, normalize=True):
+            B, S = input_ids.shape
+            return self.forward(input_ids, lengths).view(B, S, -1)[:, 0]
+
+    class Letters:
+        def encode_batch(self, texts, special=True, max_length=None):
+            return [[5 + ord(c) % 300 for c in t][:max_length] for t in texts]
+
+        def pad(self, seqs, side=None, max_length=None, device=None):
+            return tok.pad(seqs, side, max_length, device)
+
+    cfg = PRESETS["tiny-bert"]
+    tok = Tokenizer.synthetic(cfg.vocab_size, "bert")
+    words = tok.words()
+    texts = [" ".join(words[i:i + 1 + i % 5]) for i in range(9)]
+    plain, first = (c(cfg, dtype=torch.float32, seed=1) for c in (models.SentenceEncoder, FirstToken))
+
+    def padded(model, t):
+        batch = t.pad(t.encode_batch(texts, True, 16), side="right")
+        return model.encode_ids(batch["input_ids"], batch["lengths"])
+
+    for model, t in ((first, tok), (plain, Letters()), (plain, tok)):
+        torch.testing.assert_close(Encoder(model, t, 16, batch_size=4).encode(texts), padded(model, t), rtol=1e-5, atol=1e-6)
+    plain.encode_ids = lambda ids, lengths, normalize=True: torch.full((len(ids), cfg.hidden_size), 0.5)
+    assert bool((Encoder(plain, tok, 16).encode(texts) == 0.5).all())
