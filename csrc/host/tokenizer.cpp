@@ -145,11 +145,12 @@ class Tokenizer {
   // A batch for an encoder in one buffer: every text as front | its tokens | back, cut to max_length (keep_last: the
   // last token stays), sorted by length, ascending and stable, in groups of `batch`, without padding. Layout of the int64
   // buffer: the texts' indices in that order [N], then for each group the row offsets of its texts [texts + 1], their
-  // tokens [rows] and these tokens' positions [rows], counted from pos0. Returns it (pinned on request, for an
-  // asynchronous copy) with the groups' (texts, rows, longest text).
+  // tokens [rows] and these tokens' positions [rows], counted from pos0. Returns it with the groups' (texts, rows, longest
+  // text); up to `pin` elements it is pinned, for an asynchronous copy. Torch keeps pinned blocks until the process ends,
+  // so that a corpus of any size must not go through them.
   std::pair<at::Tensor, std::vector<std::tuple<int64_t, int64_t, int64_t>>> encode_sorted(
       const std::vector<std::string>& texts, const std::vector<int64_t>& front, const std::vector<int64_t>& back,
-      bool keep_last, int64_t max_length, int64_t batch, int64_t pos0, bool pin, int nthreads) const {
+      bool keep_last, int64_t max_length, int64_t batch, int64_t pos0, int64_t pin, int nthreads) const {
     TORCH_CHECK(batch > 0 && max_length > 0, "encode_sorted: batch ", batch, ", max_length ", max_length);
     std::vector<std::vector<int64_t>> ids = encode_batch(texts, nthreads);
     py::gil_scoped_release release;
@@ -169,7 +170,7 @@ class Tokenizer {
       groups.emplace_back(n, rows, len_of(order[r + n - 1]));
       total += n + 1 + 2 * rows;
     }
-    at::Tensor buf = at::empty({total}, at::TensorOptions().dtype(at::kLong).pinned_memory(pin));
+    at::Tensor buf = at::empty({total}, at::TensorOptions().dtype(at::kLong).pinned_memory(pin > 0 && total <= pin));
     int64_t* p = buf.data_ptr<int64_t>();
     int64_t *off = p + N, r = 0;
     for (const auto& [texts_, rows, longest] : groups) {

@@ -65,6 +65,10 @@ class BatchEncoding(dict):
         return BatchEncoding({k: (v.to(device) if isinstance(v, torch.Tensor) else v) for k, v in self.items()})
 
 
+# int64 elements that encode_sorted sends from pinned memory (32 MiB: 2 million tokens and their positions)
+PINNED_TOKENS = 1 << 22
+
+
 class Tokenizer:
     def __init__(self, kind: str, vocab: Dict[str, int], merges=None, specials: Optional[dict] = None,
                  lowercase: bool = False, continuing_prefix: str = "##", add_prefix_space: bool = False,
@@ -163,14 +167,14 @@ class Tokenizer:
         """:meth:`encode_batch` for an encoder, natively and with one upload: the texts sorted by length in groups of
         ``batch`` without padding -> (order [N]: the texts' indices, [(ids [rows], positions [rows] from
         ``first_position``, offsets [texts + 1]: each text's first row, the longest text's length)]), on ``device``; the
-        copy is not waited for."""
+        copy is not waited for up to ``PINNED_TOKENS`` integers."""
         front, back = self._wrap([], True), []
         if self.template == "cls_sep":
             front, back = front[:1], front[1:]
-        gpu = torch.device(device).type == "cuda"
+        pin = PINNED_TOKENS if torch.device(device).type == "cuda" else 0
         buf, groups = self._impl.encode_sorted(list(texts), front, back, self.template == "cls_sep", max_length, batch,
-                                               first_position, gpu)
-        buf = buf.to(device, non_blocking=True)
+                                               first_position, pin)
+        buf = buf.to(device, non_blocking=pin > 0 and buf.is_pinned())
         at, out = len(texts), []
         for n, rows, longest in groups:
             off, ids, pos = buf[at:at + n + 1 + 2 * rows].split([n + 1, rows, rows])

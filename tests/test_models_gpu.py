@@ -247,6 +247,24 @@ def test_shuffled_decode_weights_match_row_major(monkeypatch):
         assert torch.equal(l1, l0)
 
 
+def test_encoder_pins_no_corpus(monkeypatch):
+    """Tokens go up from pinned memory only as far as torch may keep that for good; beyond, with the same embeddings."""
+    from rag_tl_domainllm_optimizer_amd import tokenizer
+    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder
+
+    cfg = PRESETS["tiny-bert"]
+    tok = tokenizer.Tokenizer.synthetic(cfg.vocab_size, "bert")
+    words = tok.words()
+    texts = [" ".join(words[i:i + 1 + i % 9]) for i in range(50)]
+    enc = Encoder(models.SentenceEncoder(cfg, device=DEV, seed=1), tok, 32, batch_size=16)
+    want = enc.encode(texts)
+    total = len(tok._impl.encode_sorted(texts, [1], [2], True, 32, 16, 0, 0)[0])
+    for pin in (0, total - 1, total):
+        assert tok._impl.encode_sorted(texts, [1], [2], True, 32, 16, 0, pin)[0].is_pinned() == (pin == total)
+    monkeypatch.setattr(tokenizer, "PINNED_TOKENS", total - 1)
+    assert torch.equal(enc.encode(texts), want)
+
+
 def test_encoder_gpu_matches_cpu():
     cfg = PRESETS["tiny-mpnet"]
     cpu = models.SentenceEncoder(cfg, dtype=torch.float32, seed=3)
