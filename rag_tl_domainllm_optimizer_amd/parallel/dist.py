@@ -118,6 +118,8 @@ def broadcast_module_(module: torch.nn.Module, src: int = 0):
         return
     for p in module.parameters():
         dist.broadcast(p.data, src)
+        if not p.is_inference():  # p.data counts its own changes: images derived from the weight go by p's count
+            torch.autograd.graph.increment_version(p)
 
 
 def all_gather_object(obj):

@@ -214,3 +214,25 @@ def test_sft_fit_reports_each_steps_grad_norm():
     assert len(na) == 8
     assert len(set(round(x, 6) for x in na)) > 1  # not one repeated value
     torch.testing.assert_close(torch.tensor(na), torch.tensor(nb), rtol=1e-5, atol=1e-7)
+
+
+def _broadcast_worker(rank, world, port):
+    os.environ.update(RANK=str(rank), WORLD_SIZE=str(world), LOCAL_RANK=str(rank), MASTER_ADDR="127.0.0.1",
+                      MASTER_PORT=str(port))
+    from rag_tl_domainllm_optimizer_amd import parallel
+    from rag_tl_domainllm_optimizer_amd.parallel.dist import broadcast_module_
+
+    parallel.init(device="cpu")
+    m = torch.nn.Linear(4, 3)
+    with torch.no_grad():
+        m.weight.fill_(rank + 1.0)
+    before = [p._version for p in m.parameters()]
+    broadcast_module_(m, 1)
+    assert bool((m.weight == 2).all())
+    assert all(p._version > v for p, v in zip(m.parameters(), before))
+    parallel.shutdown()
+
+
+def test_broadcast_counts_as_a_change():
+    """Derived decode weights are kept by the parameters' version counters: a broadcast advances them."""
+    mp.spawn(_broadcast_worker, args=(2, _free_port()), nprocs=2, join=True)
