@@ -1052,7 +1052,7 @@ bool attn_decode_fused_slabs(const Tensor& slabs, int64_t nsplit, Tensor kc, Ten
   const int64_t NP = (Smax + PS - 1) / PS, G = Hq / Hkv;
   TORCH_CHECK(G * Hkv == Hq, "attn_decode_fused_slabs: Hq must be a multiple of Hkv");
   if (!rt_attn_decode_slabs_ok((int)B, (int)Hq, (int)Hkv, (int)D, (int)Smax, (int)NP, ksc.has_value() && ksc->defined()))
-    return false;  // caller reduces first  // caller reduces first
+    return false;  // caller reduces first
   const int64_t W = (Hq + 2 * Hkv) * D;
   TORCH_CHECK(slabs.is_contiguous() && slabs.numel() >= nsplit * B * W && nsplit >= 1, "attn_decode_fused_slabs: slabs");
   TORCH_CHECK(out.size(0) == B && slot.numel() == B && attn_len.numel() == B && out.size(1) >= Hq * D,
