@@ -494,7 +494,7 @@ class CausalLM(nn.Module):
         (profiles/r6/bench_decode_refresh_gating_ab.log)."""
         fp8 = bool(self.layers) and self.layers[0].fp8_enabled
         limit = self.fused_decode_max_batch_fp8 if fp8 else self.fused_decode_max_batch
-        fused = self.fused_decode and (batch is None or batch <= limit)
+        fused = self.fused_decode and self.embed.is_cuda and (batch is None or batch <= limit)
         plain = batch is None or (not fused and 64 < batch <= 128)
         for layer in self.layers if fused or plain else ():
             layer.refresh_decode_weights(fused, plain)
