@@ -234,8 +234,9 @@ class CausalLM(nn.Module):
         # decode steps run the fused 4-GEMM layer (norms folded into GEMMs, residual epilogues) up to
         # this batch: bf16 on the no-split tile-ordered GEMVs (M <= 16), then (17..64, serving) on the
         # tile-ordered kernels of up to four row tiles, with the in-GEMM RMS norm; above it the
-        # bf16 decode layer uses the token-parallel 256x128 split-K GEMMs with the split-K partials
-        # summed inside the norm and attention-prologue kernels (``defer_splitk``). With fp8 weights
+        # bf16 decode layer uses tile-ordered images to 128 rows and the token-parallel 256x128 GEMMs
+        # beyond, split over K with the partials summed inside the norm and attention-prologue
+        # kernels (``defer_splitk``). With fp8 weights
         # (config 5) the same up to batch 64: W8A16 tile-ordered GEMVs to 16 rows, then the fp8
         # LDS-DMA kernels with the same folded-norm / SwiGLU / residual epilogues
         self.fused_decode = True

@@ -63,7 +63,8 @@ def batch_invariant(on: bool = True):
     """Row-invariant GEMM numerics inside the block: every token-parallel GEMM (``gemm``) runs the
     gemm_big kernel without a K split whatever M is, so a row's output bits do not depend on how
     many other rows share the launch (no M-dependent split-K / skinny-kernel choice; gemm_big's
-    256- and 128-column tiles accumulate every element in the same K order). The PPO scoring
+    256- and 128-column tiles accumulate every element in the same K order; products with a weight
+    image at hand leave it alone above 16 rows). The PPO scoring
     forwards (``train.common.score_sequences``) run under it: reference log-probs, the optional
     theta_old recompute and the update forward then agree bitwise across minibatch sizes,
     padding and packing. Costs nothing at scoring sizes (M in the thousands never splits)."""

@@ -495,6 +495,7 @@ def test_decode_weight_images_only_where_read(mode):
     layer = m.layers[0]
     held = {k for k, c in layer._shufc.items() if c}
     layer.refresh_decode_weights()
+    m.refresh_decode_weights(80)
     assert {k for k, c in layer._shufc.items() if c} == held
     if mode == "bf16":
         assert held == {"qkv_plain", "o", "gate_up_plain", "down"}
