@@ -149,6 +149,24 @@ def test_decode_graphs_follow_adapter_updates(rows, fused):
         assert err <= OFF_POLICY, (step, err)
 
 
+@pytest.mark.parametrize("preset", ["tiny-llama", "tiny-opt", "tiny-vezatar", "tiny-pafolorn"])
+@pytest.mark.parametrize("rows", [20, 48, 72, 128])
+def test_decode_graphs_follow_weights_changed_in_place(preset, rows):
+    """Replays after a change of the weights themselves (a checkpoint loaded into the model) draw the bits of eager steps."""
+    m = models.build_model(preset + ":random", device=DEV, seed=1)
+    p = SamplingParams(max_new_tokens=6, do_sample=False)
+    prompts = [[3 + b % 50, 4, 5 + b % 7] for b in range(rows)]
+    graph, eager = (Generator(m, rows, 64, DEV, use_graph=on) for on in (True, False))
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    for step in range(2):
+        a, b = (gen.generate(prompts, p, pad_id=0, eos_ids=[-1]) for gen in (graph, eager))
+        assert torch.equal(a.tokens, b.tokens) and torch.equal(a.logprobs, b.logprobs), step
+        with torch.no_grad():
+            for q in m.parameters():
+                if q.dim() == 2:
+                    q.add_(torch.randn(q.shape, device=DEV, generator=g).to(q.dtype) * 0.02)
+
+
 @pytest.mark.parametrize("rows", [1, 40, 72, 100])
 def test_batcher_graphs_follow_adapter_updates(rows):
     """Requests admitted after an adapter update decode with the new adapters: in a batcher that lives on, and in a new one
