@@ -99,7 +99,28 @@ class StreamPair:
         self.main = torch.cuda.current_stream() if self.enabled else None
         # default priority, like every stream here: work on streams of different priorities has hung
         # MI355X hosts for good
-        self.side = torch.cuda.Stream() if self.enabled else None
+        self.side = self._beside(self.main) if self.enabled else None
+
+    @staticmethod
+    def _beside(main, tries: int = 8):
+        """A stream whose work runs beside ``main``'s. HIP deals streams out to a few hardware queues (4 here), and every
+        fourth one of torch's pool shares the default stream's: whatever it is given waits for all that main has queued.
+        Each candidate is tried behind 1 ms of waiting on main."""
+        main.synchronize()
+        for _ in range(tries):
+            side = torch.cuda.Stream()
+            side.record_event().synchronize()  # the stream's own start-up
+            with torch.cuda.stream(main):
+                torch.cuda._sleep(2_400_000)
+            busy, free = main.record_event(), side.record_event()
+            while not free.query():
+                if busy.query():
+                    break
+            else:
+                if not busy.query():
+                    return side
+            main.synchronize()
+        return side
 
     @contextlib.contextmanager
     def on_side(self, wait: bool = False):

@@ -230,6 +230,27 @@ def test_reward_stream_overlap_matches_serial(monkeypatch):
         assert abs(a[k] - b[k]) < 1e-5, (k, a[k], b[k])
 
 
+def test_stream_pair_runs_beside_the_main_stream():
+    """The side stream of a pair does not wait for the main one, whichever of torch's pooled streams come first (HIP gives
+    every fourth one the main stream's hardware queue)."""
+    from rag_tl_domainllm_optimizer_amd.runtime import StreamPair
+
+    x = torch.zeros(8, device=DEV)
+    for _ in range(8):
+        torch.cuda.Stream()
+        pair = StreamPair()
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(3)]
+        torch.cuda.synchronize()
+        ev[0].record()
+        torch.cuda._sleep(50_000_000)
+        ev[1].record()
+        with pair.on_side():
+            x.add_(1)
+            ev[2].record()
+        torch.cuda.synchronize()
+        assert ev[0].elapsed_time(ev[2]) < ev[0].elapsed_time(ev[1])
+
+
 def test_cli_pipeline_config5_fp8_gpu(tmp_path):
     """BASELINE config 5 through the CLI preset: Llama-2-13B-shaped RAG -> LoRA SFT -> PPO with the
     fp8 knob on (``model.fp8``): rollout prefill / decode and reference scoring stream e4m3fn
