@@ -105,11 +105,11 @@ class DecoderLayer(nn.Module):
         return g.merged_weight(w)
 
     def _w_plain(self, wname: str, gname: str):
-        """The weight that the layer's products without grad multiply by; None where an adapter runs beside it."""
+        """The weight that the layer's products without grad multiply by; None where an adapter has only run beside it."""
         g = self._lg(gname)
         if g is None or not g.enabled:
             return getattr(self, wname)
-        return self._w_eff(wname, gname) if g.use_merged else None
+        return self._w_eff(wname, gname) if g.use_merged or g.merged is not None else None
 
     @torch.no_grad()
     def refresh_decode_weights(self, fused: bool = True, plain: bool = True):

@@ -167,6 +167,22 @@ def test_decode_graphs_follow_weights_changed_in_place(preset, rows):
                     q.add_(torch.randn(q.shape, device=DEV, generator=g).to(q.dtype) * 0.02)
 
 
+@pytest.mark.parametrize("rows", [40, 80])
+def test_refresh_outside_generation_brings_merged_images_up_to_date(rows):
+    """Between generations adapters run apart from the weights; a refresh there still prepares the next replays."""
+    m = _d128_lora()
+    _new_adapters(m, 0)
+    Generator(m, rows, 32, DEV).generate([[3, 4, 5]] * rows, SamplingParams(max_new_tokens=3, do_sample=False), pad_id=0,
+                                         eos_ids=[-1])
+    _new_adapters(m, 1)
+    m.refresh_decode_weights(rows)
+    for layer in m.layers:
+        assert layer._shufc["o"] and not layer.lora["o"].use_merged
+        for name in ("o", "down"):
+            want = layer.lora[name].merged_weight(getattr(layer, name + "_w")).clone()
+            assert torch.equal(layer._shufc[name]["w"], ops.native().shuffle_decode_weight(want, None)), name
+
+
 @pytest.mark.parametrize("rows", [1, 40, 72, 100])
 def test_batcher_graphs_follow_adapter_updates(rows):
     """Requests admitted after an adapter update decode with the new adapters: in a batcher that lives on, and in a new one
