@@ -134,6 +134,7 @@ static const TuningField kTuningFields[] = {
     {"wide_split", &rt::Tuning::wide_split, nullptr},
     {"m64_wide", &rt::Tuning::m64_wide, nullptr},
     {"gemm_bn128_cost", nullptr, &rt::Tuning::gemm_bn128_cost},
+    {"gemm_duo", &rt::Tuning::gemm_duo, nullptr},
     {"gemm_group_m", &rt::Tuning::gemm_group_m, nullptr},
     {"sample_window", &rt::Tuning::sample_window, nullptr},
     {"sample_fast64", &rt::Tuning::sample_fast64, nullptr},

@@ -34,6 +34,7 @@
 #include "rt_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rt {
 
@@ -122,7 +123,8 @@ __device__ __forceinline__ float act_fn(float x, int act) {
 // 5e-7 less enclose act_fn's fp32 result; both rounding to the same bf16, that is the answer, else erff decides: about 1 pair of
 // 2500 for x around 0, every second one at -3.8. 41.5k rows, 768 -> 3072, inputs of
 // standard deviation 0.55 / 1.1: 389 / 467 -> 290 / 307 us (without GELU 242); 24k rows, 384 -> 1536: 108 / 144 -> 82 / 82 (49).
-__device__ __forceinline__ uint32_t gelu2_bf16(float x0, float x1) {
+// gelu2_fast: the packed results and whether they are the answer.
+__device__ __forceinline__ bool gelu2_fast(float x0, float x1, uint32_t& y) {
   float hi[2], lo[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -147,8 +149,12 @@ __device__ __forceinline__ uint32_t gelu2_bf16(float x0, float x1) {
     hi[k] = h * fmaf(z, q, 1.f + 5e-7f);
     lo[k] = fmaf(h, -1e-6f, hi[k]);
   }
-  uint32_t y = pack2bf(hi[0], hi[1]);
-  if (__builtin_expect(y != pack2bf(lo[0], lo[1]), 0)) y = pack2bf(act_fn(x0, E_GELU), act_fn(x1, E_GELU));
+  y = pack2bf(hi[0], hi[1]);
+  return y == pack2bf(lo[0], lo[1]);
+}
+__device__ __forceinline__ uint32_t gelu2_bf16(float x0, float x1) {
+  uint32_t y;
+  if (__builtin_expect(!gelu2_fast(x0, x1, y), 0)) y = pack2bf(act_fn(x0, E_GELU), act_fn(x1, E_GELU));
   return y;
 }
 
@@ -542,20 +548,24 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Args p) {
     // 16 lanes in 16 rows hit 16 distinct bank pairs) for 16-B coalesced global stores
     constexpr int LDT = BN + 4;
     bf16_t* tile = (bf16_t*)smem;
-    float bcol[2 * NB][4];
+    float bcol[2 * NB][4] = {};
     float scol[2 * NB][4];  // F8: per-output-channel weight scale of the lane's columns
+    if (EPI != E_SWIGLU && p.bias) {
+      // all loads in flight together (with a check per column each waited for the one before it)
 #pragma unroll
-    for (int j = 0; j < 2 * NB; ++j) {
-      const int col = n0 + col_of(j) + fq * 4;
+      for (int j = 0; j < 2 * NB; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        bcol[j][r] = (EPI != E_SWIGLU && p.bias && col < p.N) ? bf2f(p.bias[col + r]) : 0.f;
-        if constexpr (F8) {
+        for (int r = 0; r < 4; ++r) bcol[j][r] = bf2f(p.bias[min(n0 + col_of(j) + fq * 4 + r, p.N - 1)]);
+    }
+    if constexpr (F8) {
+#pragma unroll
+      for (int j = 0; j < 2 * NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
           const int c = col_of(j) + fq * 4 + r;  // tile column -> weight row
           const int wrow = EPI == E_SWIGLU ? (c < HALF ? tn * HALF + c : Fh + tn * HALF + c - HALF) : min(n0 + c, p.N - 1);
           scol[j][r] = p.sb[wrow];
         }
-      }
     }
     auto ld16 = [&](int row, int c8) -> uint4 {  // 8 bf16 at tile[row][8 c8], 8-B aligned
       const uint2 lo = *(const uint2*)(tile + row * LDT + c8 * 8);
@@ -700,6 +710,248 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Args p) {
       }
       __syncthreads();
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// NT products with a short reduction: two independent workgroups per CU
+// ---------------------------------------------------------------------------------------------
+// C = act(A B^T + bias) (+ R) in bf16, K % 64 == 0. With one 128-KiB workgroup per CU a 256 x 256 tile of K = 768 computes for
+// 17 us and then stores (and GELUs) for 10 to 25 with idle matrix cores, every CU at the same time. Here a workgroup is 4 waves
+// (128 x 64 each of a 256 x 128 tile) over a ring of five 16-KiB granules, 80 KiB: two run per CU, a wave of each on every SIMD.
+// A K-step of 64 has three granules: a0 (A rows with bit 6 = 0), b, a1 (bit 6 = 1), in 128-B rows of gemm_big_kernel's swizzle
+// (32-k steps in 64-B rows ask for as many requests of half the size and are bound by the texture unit: 284 us instead of 225
+// at 8192 x 4096 x 4096). Phase 1 multiplies a0 by b, phase 2 a1 by b's fragments; the barriers stand in the middle of the
+// phases, so that the fragments of the next k half are read under the MFMAs of this one; a granule's place is filled again
+// once the barrier says that all waves have read it, 2 or 3 phases before the next use. The DMA are buffer loads: hipcc takes
+// global_load_lds for flat accesses and waits for all LDS reads instead of the oldest. Per element the MFMAs and their order
+// are gemm_big_kernel's: the same bits. In the K loop it reaches 1.25 PFLOP/s, bound as that kernel is by the matrix cores at
+// the clock they leave; two workgroups that start together also store together, which is what is left around it.
+// us, gemm_big_kernel -> this: 23500 x 2304 x 768: 102 -> 88, 23500 x 768 x 768: 45 -> 39, 23500 x 3072 x 768 with GELU:
+// 189 -> 154 (without: 122 -> 114), 20000 x 1152 x 384: 32 -> 26, 1000 x 1536 x 384 with GELU: 32 -> 20.
+constexpr int DUO_G = 16384;
+
+// 16 GELUs of one accumulator row block; the pairs that gelu2_bf16 could not decide are redone with erff in ONE copy of its
+// code, picked by lane from the 8 pairs (about one row block in five has any).
+__device__ __forceinline__ void gelu16_bf16(const float (&x)[16], uint32_t (&y)[8]) {
+  unsigned open = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) open |= gelu2_fast(x[2 * k], x[2 * k + 1], y[k]) ? 0u : 1u << k;
+  while (__any(open != 0)) {
+    float a = 0.f, b = 0.f;
+    const int k0 = open ? __ffs(open) - 1 : 8;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      a = k == k0 ? x[2 * k] : a;
+      b = k == k0 ? x[2 * k + 1] : b;
+    }
+    const uint32_t v = pack2bf(act_fn(a, E_GELU), act_fn(b, E_GELU));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) y[k] = k == k0 ? v : y[k];
+    open &= open - 1;
+  }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_duo_kernel(Args p) {
+  constexpr int LDT = 128 + 4;  // row of the epilogue's bf16 tile
+  static_assert(256 * LDT * 2 <= 5 * DUO_G, "the tile fits the ring");
+  __shared__ __attribute__((aligned(16))) char smem[5 * DUO_G];
+  const int tiles_m = (p.M + 255) / 256, tiles_n = (p.N + 127) / 128;
+  const int nk = p.K / 64;  // K % 64 == 0 (launcher)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wid >> 1, wc = wid & 1;
+  const int frow = lane & 15, fq = lane >> 4;
+  const int bid = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+  const int GM = p.group_m > 0 ? p.group_m : GROUP_M;
+  const int group = bid / (GM * tiles_n);
+  const int first_m = group * GM;
+  const int gsz = min(tiles_m - first_m, GM);
+  const int m0 = (first_m + bid % gsz) * 256, n0 = bid % (GM * tiles_n) / gsz * 128;
+
+  // LDS-DMA: instruction j of this wave brings rows 8 (4 wid + j) .. + 7 of a granule, 128 B each; lane -> row lane / 8, 16-B
+  // slot lane % 8 holding k-chunk slot ^ row_swz(row)
+  uint32_t oa[2][4], ob[4];  // bytes from the tile's first row
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = (wid * 4 + j) * 8 + (lane >> 3), kc = ((lane & 7) ^ row_swz(row)) * 16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ar = (row >> 6) * 128 + h * 64 + (row & 63);
+      oa[h][j] = (uint32_t)(min(m0 + ar, p.M - 1) - m0) * (uint32_t)p.lda * 2 + kc;
+    }
+    ob[j] = (uint32_t)(min(n0 + row, p.N - 1) - n0) * (uint32_t)p.ldb * 2 + kc;
+  }
+  // granule c (0 a0, 1 b, 2 a1) of K-step t into ring place g
+  const __amdgpu_buffer_rsrc_t Ar = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (long)m0 * p.lda), 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t Br = __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (long)n0 * p.ldb), 0, -1, 0x00020000);
+  auto stage = [&](int c, int t, int g) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(c == 1 ? Br : Ar, (lds_void*)(smem + g * DUO_G + wid * 4096 + j * 1024), 16,
+                                               c == 1 ? ob[j] : oa[c >> 1][j], t * 128, 0, 0);
+  };
+
+  f32x4 acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int sw = row_swz(frow);
+  const int ra[2] = {(wr * 64 + frow) * 128 + ((fq ^ sw) << 4), (wr * 64 + frow) * 128 + (((4 + fq) ^ sw) << 4)};
+  const int rb[2] = {(wc * 64 + frow) * 128 + ((fq ^ sw) << 4), (wc * 64 + frow) * 128 + (((4 + fq) ^ sw) << 4)};
+  bf16x8 fa[2][4], fb[2][4];  // fragments of either k half
+  auto read_a = [&](int kk, int g) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fa[kk][i] = *(const bf16x8*)(smem + g * DUO_G + ra[kk] + i * 2048);
+  };
+  auto read_b = [&](int kk, int g) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) fb[kk][j] = *(const bf16x8*)(smem + g * DUO_G + rb[kk] + j * 2048);
+  };
+  auto mma = [&](int h, int kk) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[h * 4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][j], fa[kk][i], acc[h * 4 + i][j], 0, 0, 0);
+  };
+  // of this wave's DMA only the `newer` youngest granules (4 instructions each) may be under way, its LDS reads are done;
+  // behind the barrier both hold for every wave
+  auto sync = [&](int newer) {
+    if (newer == 3) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
+    else if (newer == 2) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    else if (newer == 1) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    GB_BARRIER();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto at = [](int g, int d) { return g + d >= 5 ? g + d - 5 : g + d; };
+  int t = 0, g0 = 0;  // K-step, place of its a0
+  // One K-step. While a k half is multiplied the next one's fragments are read; the two barriers stand between the halves.
+  // MODE 0: two more steps follow at least; 1: one more; 2: the last.
+  auto step = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    read_a(1, g0);
+    read_b(1, at(g0, 1));
+    mma(0, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    sync(MODE == 2 ? 0 : 2);  // a1 is there, a0 and b have been read
+    if constexpr (MODE == 0) {
+      stage(2, t + 1, g0);
+      stage(0, t + 2, at(g0, 1));
+    } else if constexpr (MODE == 1) {
+      stage(2, t + 1, g0);
+    }
+    read_a(0, at(g0, 2));
+    mma(0, 1);
+    if constexpr (MODE == 0) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(1, at(g0, 2));
+    mma(1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MODE == 2) {
+      mma(1, 1);
+    } else {
+      sync(MODE == 0 ? 2 : 1);  // a0 and b of the next step are there, a1 has been read
+      if constexpr (MODE == 0) stage(1, t + 2, at(g0, 2));
+      read_a(0, at(g0, 3));
+      read_b(0, at(g0, 4));
+      mma(1, 1);
+      if constexpr (MODE == 0) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+          __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      ++t;
+      g0 = at(g0, 3);
+    }
+  };
+  // granules in the order a0, b, a1 of step 0, 1, ...; granule n lies in place n % 5
+  stage(0, 0, 0);
+  stage(1, 0, 1);
+  stage(2, 0, 2);
+  if (nk > 1) {
+    stage(0, 1, 3);
+    stage(1, 1, 4);
+  }
+  sync(nk > 1 ? 3 : 1);
+  read_a(0, 0);
+  read_b(0, 1);
+  while (t + 2 < nk) step(std::integral_constant<int, 0>{});
+  if (t + 1 < nk) step(std::integral_constant<int, 1>{});
+  step(std::integral_constant<int, 2>{});
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  GB_BARRIER();
+
+  // acc[i][j][r] = C[m0 + 128 wr + 16 i + frow][n0 + 64 wc + 16 j + 4 fq + r]
+  bf16_t* tile = (bf16_t*)smem;
+  float bcol[4][4] = {};
+  if (p.bias) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bcol[j][r] = bf2f(p.bias[min(n0 + wc * 64 + j * 16 + fq * 4 + r, p.N - 1)]);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (m0 + wr * 128 + i * 16 >= p.M) break;
+    bf16_t* to = tile + (wr * 128 + i * 16 + frow) * LDT + wc * 64 + fq * 4;
+    if constexpr (EPI == E_GELU) {
+      float x[16];
+      uint32_t y[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[4 * j + r] = acc[i][j][r] + bcol[j][r];
+      gelu16_bf16(x, y);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *(uint2*)(to + j * 16) = make_uint2(y[2 * j], y[2 * j + 1]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = act_fn(acc[i][j][r] + bcol[j][r], EPI);
+        *(uint2*)(to + j * 16) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+      }
+    }
+  }
+  __syncthreads();
+  bf16_t* C = (bf16_t*)p.C;
+  const int cc = tid & 15, gcol = n0 + cc * 8;
+  if (gcol >= p.N) return;
+#pragma unroll 4
+  for (int row = tid >> 4; row < 256; row += 16) {
+    const int grow = m0 + row;
+    if (grow >= p.M) break;
+    const uint2 lo = *(const uint2*)(tile + row * LDT + cc * 8), hi = *(const uint2*)(tile + row * LDT + cc * 8 + 4);
+    uint4 v = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    if (p.R) {  // residual in fp32 on the bf16-rounded GEMM result (= a separate add kernel)
+      float y[8], r[8];
+      unpack8(v, y);
+      unpack8(*(const uint4*)(p.R + (long)grow * p.ldr + gcol), r);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] += r[e];
+      v = pack8(y);
+    }
+    *(uint4*)(C + (long)grow * p.ldc + gcol) = v;
   }
 }
 
@@ -1060,6 +1312,22 @@ extern "C" int rt_gemm_big(int layout_a, int layout_b, const void* A, long lda, 
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream) {
   if (bn != 0) return launch_gemm_big(p, layout_a, layout_b, act, out, bn, stream);
   const int M = p.M, N = p.N, nsplit = p.nsplit;
+  // Two workgroups per CU (gemm_duo_kernel) where the reduction is short. With GELU from any number of rows: 19.6 against 32
+  // us for 1000 x 1536 x 384, 258 against 306 for 26000 x 4096 x 1024, 827 against 880 for 26000 x 8192 x 2048. Without an
+  // activation once every CU has more than one tile (20000 x 1152 x 384: 26.2 against 31.5 us, 10000 x 4096 x 1024: 76 against
+  // 86; 2000 x 768 x 768, 36 tiles: 15.9 against 14.8) and up to K = 1024, where it meets gemm_big_kernel (20000 x 4096 x
+  // 1024: 156 both; 32000 x 2048 x 1536: 187 against 177).
+  const long duo_tiles = (long)((M + 255) / 256) * ((N + 127) / 128);
+  if (tuning().gemm_duo && layout_a == ROW && layout_b == ROW && out == O_BF16 && nsplit == 1 && !p.A2 && p.K >= 64 &&
+      p.K % 64 == 0 && p.lda < (1 << 22) && p.ldb < (1 << 22) &&  // 32-bit byte offsets within a tile
+      (tuning().gemm_duo == 2 ? act == E_NONE || act == E_GELU
+                              : (act == E_GELU && p.K <= 2048) || (act == E_NONE && p.K <= 1024 && duo_tiles > num_cus()))) {
+    const dim3 grid((unsigned)duo_tiles), block(256);
+    if (act == E_GELU) hipLaunchKernelGGL(gemm_duo_kernel<E_GELU>, grid, block, 0, stream, p);
+    else hipLaunchKernelGGL(gemm_duo_kernel<E_NONE>, grid, block, 0, stream, p);
+    RT_LAUNCH_CHECK();
+    return 0;
+  }
   const long lda = p.lda, lda2 = p.lda2, ldc = p.ldc, ldc2 = p.ldc2, ldr = p.ldr;
   void* C = p.C;
   const bool can128 = bn128_supported(layout_a, layout_b, act, out);

@@ -333,6 +333,32 @@ def test_gelu_epilogue_bits(M, N, res):
     assert torch.equal(y.view(torch.int16), z.view(torch.int16))
 
 
+@pytest.mark.parametrize("M,N,K,act,res", [(1, 8, 64, 0, False), (255, 128, 128, 0, True), (256, 136, 192, 2, False),
+                                           (257, 120, 256, 0, False), (513, 264, 64, 2, True), (1300, 1152, 384, 0, True)])
+def test_two_workgroup_product_has_the_tile_kernels_bits(M, N, K, act, res):
+    """The form with two workgroups per CU multiplies in the order of the 256 x 256 tiles: the same bits, with strided
+    operands, around the tile edges and from one K-step on; nothing beyond the columns is written."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device=DEV).bfloat16()
+    x, w, bias = r(M, K + 8)[:, :K], r(N, K + 16)[:, :K] * 0.1, r(N)
+    R = r(M, N) if res else None
+    out = []
+    for duo in (0, 2):
+        y = torch.full((M, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        with ops.tuning(gemm_duo=duo):
+            ops.native().gemm_big(x, w, 0, 0, None, None, bias, act, 0, 1, y[:, :N], None, R)
+        assert (y[:, N:] == 7).all()
+        out.append(y[:, :N])
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+    want = x.double() @ w.double().t() + bias.double()
+    if act:
+        want = torch.nn.functional.gelu(want)
+    # a bf16 rounding before the residual and one after, on an fp32 sum
+    _close(out[1], want + (R.double() if res else 0), rtol=2.0 ** -7, atol=1e-3 * math.sqrt(K))
+
+
 # ---------------------------------------------------------------------------------------------- encoders without padding
 @pytest.mark.parametrize("D,H,bias", [(32, 3, False), (64, 2, False), (64, 12, True), (128, 1, False), (32, 2, True)])
 @pytest.mark.parametrize("lens", [[1], [64, 65, 0, 127], [128, 129, 63, 1, 300], [2] * 40])
