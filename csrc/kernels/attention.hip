@@ -27,6 +27,7 @@
 #include "rt_common.h"
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 namespace rt {
@@ -91,11 +92,8 @@ __device__ __forceinline__ int3 attn_block_xyz(int lpt = 0) {
   return make_int3(0, 0, 0);  // not reached: the counts over v sum to the range length
 }
 
-// 2^x; RAW: the instruction itself, whose results below 2^-126 are 0 (a probability that a sum of at least 1 does not see)
-template <bool RAW>
-__device__ __forceinline__ float exp2_any(float x) {
-  return RAW ? __builtin_amdgcn_exp2f(x) : exp2f(x);
-}
+// 2^x as the instruction gives it: results below 2^-126 are 0 (probabilities beside a sum of at least 1)
+__device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
 struct AttnArgs {
   const bf16_t* q; long ldq;
@@ -111,7 +109,8 @@ struct AttnArgs {
   int causal, window;
   float scale_log2;           // softmax scale * log2(e)
   int lpt;                    // heaviest-first dispatch order (attn_block_xyz; causal grids)
-  const long* off;            // VL: sequence b is rows [off[b], off[b + 1]) of Sq in all
+  int nx, gh, groups;         // packed form: query tiles, heads of a group, groups of all sequences
+  const long* off;            // packed form: sequence b is rows [off[b], off[b + 1]) of Sq in all
 };
 
 // byte offset of 16-B chunk c of row r in a K-style (row-read) tile image
@@ -146,17 +145,9 @@ __device__ __forceinline__ int v_off(int r, int c) {
 //
 // Q64 (NU = 1, 4 waves of 16 rows): 64 positions of one head per workgroup — the same causal
 // saving for heads that share no K / V (MHA, e.g. Llama-2-13B), bitwise the 128-row form too.
-//
-// VL (encoders: bidirectional self-attention, one head per K / V head): the sequences' rows lie one behind the other
-// (a.off), so neither the products around it nor this kernel work on padding; tiles count from each sequence's
-// first row, per row the order and arithmetic of the padded form. The additive bias comes from the 191 differences a
-// 128 x 64 tile can have, brought to LDS with the tile, instead of a gather per score; only a sequence's last tile
-// is masked; waves without rows skip the products. 256 texts of 18 to 162 tokens, 12 heads of 64 with the bias: 230 -> 103
-// us a call; bound by the softmax's vector instructions.
-template <int D, int NU = 2, bool HP = false, bool Q64 = false, bool VL = false>
+template <int D, int NU = 2, bool HP = false, bool Q64 = false>
 __global__ __launch_bounds__(Q64 ? 256 : 64 * 8 / NU, D == 128 ? 2 : (D == 64 ? 3 : 4))
 void attn_fwd_kernel(AttnArgs a) {
-  static_assert(!VL || (NU == 2 && !HP && !Q64), "VL: 4 waves of 32 rows");
   static_assert(!HP || NU == 2, "HP: 4 waves of 32 rows");
   static_assert(!Q64 || (NU == 1 && !HP), "Q64: 4 waves of 16 rows");
   constexpr int NT = Q64 ? 256 : 64 * 8 / NU;  // threads per workgroup
@@ -170,21 +161,11 @@ void attn_fwd_kernel(AttnArgs a) {
   constexpr int NBUF = DB ? 2 : 1;
   constexpr int SMEM = (2 * NBUF * TILE_BYTES > 128 * OROW * 2) ? 2 * NBUF * TILE_BYTES : 128 * OROW * 2;
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  __shared__ float rel[VL ? NBUF * 192 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int g = lane >> 4, r16 = lane & 15;
   const int3 bx = attn_block_xyz(a.lpt);
   const int b = bx.z;
-  long base = (long)b * a.Sk;  // its first K / V row (and, VL, its first row altogether)
-  int len = a.Sk;              // and its rows
-  if constexpr (VL) {
-    base = min(max(a.off[b], 0L), (long)a.Sq);
-    len = (int)(min(max(a.off[b + 1], base), (long)a.Sq) - base);
-    if (bx.x * 128 >= len) return;
-  }
-  const int Sq = VL ? len : a.Sq;
-  const long qbase = VL ? base : (long)b * a.Sq;
   const int h = HP ? bx.y * 4 + wid : bx.y;
   const int hk = HP ? bx.y : h / (a.Hq / a.Hkv);
   constexpr int QROWS = HP ? 32 : (Q64 ? 64 : 128);  // query positions per workgroup
@@ -192,8 +173,8 @@ void attn_fwd_kernel(AttnArgs a) {
   const int q0 = HP ? qblk0 : qblk0 + wid * 16 * NU;
 
   const int start = a.kv_start ? a.kv_start[b] : 0;
-  int kend = VL ? len : a.kv_len ? min(a.kv_len[b], a.Sk) : a.Sk;
-  const int qlast = min(qblk0 + QROWS - 1, Sq - 1);
+  int kend = a.kv_len ? min(a.kv_len[b], a.Sk) : a.Sk;
+  const int qlast = min(qblk0 + QROWS - 1, a.Sq - 1);
   if (a.causal) kend = min(kend, qlast + 1);
   int kbeg = start;
   if (a.window > 0) kbeg = max(kbeg, qblk0 - a.window + 1);
@@ -203,8 +184,8 @@ void attn_fwd_kernel(AttnArgs a) {
   bf16x8 qf[NU][DS];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int qrow = min(q0 + 16 * u + r16, Sq - 1);
-    const bf16_t* qp = a.q + (qbase + qrow) * a.ldq + (long)h * D + 8 * g;
+    const int qrow = min(q0 + 16 * u + r16, a.Sq - 1);
+    const bf16_t* qp = a.q + ((long)b * a.Sq + qrow) * a.ldq + (long)h * D + 8 * g;
 #pragma unroll
     for (int s = 0; s < DS; ++s) qf[u][s] = *(const bf16x8*)(qp + 32 * s);
   }
@@ -231,33 +212,28 @@ void attn_fwd_kernel(AttnArgs a) {
   constexpr int CPT = 64 * NCH / NT;  // chunks per thread per tensor (4 for D=128, 256 threads)
   constexpr int KSTEP = NT / NCH;     // key stride between a thread's chunks
   const int lc = tid % NCH, lkey = tid / NCH;
-  const bf16_t* kb = a.k + base * a.ldk + (long)hk * D + lc * 8;
-  const bf16_t* vb = a.v + base * a.ldv + (long)hk * D + lc * 8;
+  const bf16_t* kb = a.k + (long)b * a.Sk * a.ldk + (long)hk * D + lc * 8;
+  const bf16_t* vb = a.v + (long)b * a.Sk * a.ldv + (long)hk * D + lc * 8;
   u32x4 kreg[CPT], vreg[CPT];
-  float breg = 0.f;
   auto load_tile = [&](int kv0) {
 #pragma unroll
     for (int r = 0; r < CPT; ++r) {
-      const long kk = min(kv0 + lkey + KSTEP * r, len - 1);
+      const long kk = min(kv0 + lkey + KSTEP * r, a.Sk - 1);
       kreg[r] = *(const u32x4*)(kb + kk * a.ldk);
       vreg[r] = *(const u32x4*)(vb + kk * a.ldv);
     }
-    // difference key - query of entry w: kv0 - (qblk0 + 127) + w
-    if (VL && a.rel_bias && tid < 192)
-      breg = a.rel_bias[(long)h * (2 * a.rb_L - 1) + min(max(kv0 - qblk0 - 127 + tid + a.rb_L - 1, 0), 2 * a.rb_L - 2)];
   };
-  auto store_tile = [&](char* kd, char* vd, int buf) {
+  auto store_tile = [&](char* kd, char* vd) {
 #pragma unroll
     for (int r = 0; r < CPT; ++r) {
       *(u32x4*)(kd + k_off<D>(lkey + KSTEP * r, lc)) = kreg[r];
       *(u32x4*)(vd + v_off<D>(lkey + KSTEP * r, lc)) = vreg[r];
     }
-    if (VL && a.rel_bias && tid < 192) rel[buf * 192 + tid] = breg;
   };
 
   if (kbeg < kend) {
     load_tile(kbeg);
-    store_tile(smem, smem + TILE_BYTES, 0);
+    store_tile(smem, smem + TILE_BYTES);
   }
   __syncthreads();
 
@@ -268,7 +244,6 @@ void attn_fwd_kernel(AttnArgs a) {
     char* Ks = DB ? smem + cur * (2 * TILE_BYTES) : smem;
     char* Vs = DB ? Ks + TILE_BYTES : smem + TILE_BYTES;
 
-    if (!VL || q0 < Sq) {
     // ---- S^T[t][u] = K[16t..][:] · Q[u]^T ----
     f32x4 st[4][NU];
 #pragma unroll
@@ -294,16 +269,13 @@ void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float x = st[t][u][i] * a.scale_log2;
-          if constexpr (VL) {
-            if (a.rel_bias) x += rel[cur * 192 + 127 + 16 * (t - u) + 4 * g + i - 32 * wid - r16];
-            if (kv0 + 64 > kend) x = kv0 + 16 * t + 4 * g + i < kend ? x : -INFINITY;
-          } else if (!full) {
+          if (!full) {
             const int kk = kv0 + 16 * t + 4 * g + i;
             const int qq = q0 + 16 * u + r16;
             bool ok = kk >= start && kk < kend;
             if (a.causal) ok = ok && kk <= qq;
             if (a.window > 0) ok = ok && (qq - kk) < a.window;
-            ok = ok && qq < Sq;
+            ok = ok && qq < a.Sq;
             if (a.rel_bias && ok) x += a.rel_bias[(long)h * (2 * a.rb_L - 1) + (kk - qq) + a.rb_L - 1];
             x = ok ? x : -INFINITY;
           }
@@ -323,14 +295,14 @@ void attn_fwd_kernel(AttnArgs a) {
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float mn = fmaxf(m[u], mx);
       const float mu = mn == -INFINITY ? 0.f : mn;
-      alpha[u] = exp2_any<VL>(m[u] - mu);
+      alpha[u] = exp2_raw(m[u] - mu);
       m[u] = mn;
       float rs = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float pv = exp2_any<VL>(st[t][u][i] - mu);
+          const float pv = exp2_raw(st[t][u][i] - mu);
           st[t][u][i] = pv;
           rs += pv;
         }
@@ -366,17 +338,16 @@ void attn_fwd_kernel(AttnArgs a) {
         for (int u = 0; u < NU; ++u) o[u][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[u], vf, o[u][c], 0, 0, 0);
       }
     }
-    }
     if constexpr (DB) {
       // the other buffer was last read in the previous iteration, which every wave has left (its
       // closing barrier): store the next tile there and swap
       char* kn = smem + (cur ^ 1) * (2 * TILE_BYTES);
-      if (has_next) store_tile(kn, kn + TILE_BYTES, cur ^ 1);
+      if (has_next) store_tile(kn, kn + TILE_BYTES);
       __syncthreads();
       cur ^= 1;
     } else {
       __syncthreads();
-      if (has_next) store_tile(Ks, Vs, 0);
+      if (has_next) store_tile(Ks, Vs);
       __syncthreads();
     }
   }
@@ -386,7 +357,7 @@ void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int qq = q0 + 16 * u + r16;
-      if (qq < Sq) {
+      if (qq < a.Sq) {
         const float v = l[u] > 0.f ? (m[u] + __log2f(l[u])) * 0.69314718055994531f : INFINITY;
         a.lse[((long)b * a.Hq + h) * a.Sq + qq] = v;
       }
@@ -409,8 +380,206 @@ void attn_fwd_kernel(AttnArgs a) {
     // HP: staging row 32 w + r = position qblk0 + r of head 4 hk + w
     const int qq = HP ? qblk0 + (row & 31) : qblk0 + row;
     const int hh = HP ? hk * 4 + (row >> 5) : h;
-    if (qq < Sq)
-      *(uint4*)(a.o + (qbase + qq) * a.ldo + (long)hh * D + c * 8) = *(const uint4*)(Os + row * OROW + c * 8);
+    if (qq < a.Sq)
+      *(uint4*)(a.o + ((long)b * a.Sq + qq) * a.ldo + (long)hh * D + c * 8) = *(const uint4*)(Os + row * OROW + c * 8);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// forward, sequences one behind the other (encoders: bidirectional self-attention, one head per K / V head)
+// ---------------------------------------------------------------------------------------------
+// Sequence b is rows [off[b], off[b + 1]), so neither the products around it nor this kernel work on padding. A workgroup is
+// 128 query rows of one (sequence, head), 4 waves x 32 rows (waves without rows skip the products), over 64-key tiles:
+// S^T = K Q^T and O^T = V^T P^T, the query on the lane in both, so maxima, sums and rescaling need no shuffles but one of each
+// maximum (v_permlane swaps; sums stay in the lane until the end). Texts are short, a workgroup lives for one to three tiles,
+// and the chain length -> loads -> barrier -> tile decides: Q and the first two tiles are requested together behind one
+// barrier, further tiles (texts beyond 128 tokens) through registers. The bias of a tile's 191 differences lies in LDS and is
+// read once per difference, not per score. 256 texts of 18 to 162 tokens, 12 heads of 64 with the bias: 90 -> 55 us (before: a branch
+// and a wait per score for the bias; 111 where the texts are sorted); 256 texts of 100 to 122, 12 heads of 32: 33 -> 25.
+// f over the four lanes 16 apart, neighbours first (the order of __shfl_xor 16, 32)
+template <typename F>
+__device__ __forceinline__ float over_groups(float x, F f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+template <int D, bool RB>
+__global__ __launch_bounds__(256, D == 128 ? 2 : D == 64 ? 3 : 4) void attn_packed_kernel(AttnArgs a) {
+  constexpr int NCH = D / 8, DS = D / 32, DT = D / 16;
+  constexpr int TILE = 64 * D * 2;
+  __shared__ __attribute__((aligned(16))) char smem[4 * TILE];  // two K / V tiles
+  __shared__ float rel[RB ? 2 * 192 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int g = lane >> 4, r16 = lane & 15;
+  // groups of heads whose rows share 256 bytes go round the XCDs, a group's workgroups to one of them, the last sequences
+  // first: an encoder's batches are sorted, and in contiguous ranges (attn_block_xyz) one XCD had the longest texts
+  const int slot = blockIdx.x / 8, per = a.nx * a.gh;
+  const int grp = slot / per * 8 + blockIdx.x % 8, in = slot % per;
+  if (grp >= a.groups) return;
+  const int hg = a.Hq / a.gh, b = a.B - 1 - grp / hg, h = grp % hg * a.gh + in / a.nx, x = in % a.nx;
+  const long base = min(max(a.off[b], 0L), (long)a.Sq);
+  const int len = (int)(min(max(a.off[b + 1], base), (long)a.Sq) - base);
+  const int qblk0 = x * 128, q0 = qblk0 + wid * 32;
+  if (qblk0 >= len) return;
+
+  // thread tid always owns chunk tid % NCH of keys tid / NCH + (256 / NCH) r of a tile
+  constexpr int CPT = 64 * NCH / 256, KSTEP = 256 / NCH;
+  const int lc = tid % NCH, lkey = tid / NCH;
+  const bf16_t* const kb = a.k + base * a.ldk + (long)h * D + lc * 8;
+  const bf16_t* const vb = a.v + base * a.ldv + (long)h * D + lc * 8;
+  auto load_tile = [&](int kv0, u32x4 (&kr)[CPT], u32x4 (&vr)[CPT], float& br) {
+#pragma unroll
+    for (int r = 0; r < CPT; ++r) {
+      const long kk = min(kv0 + lkey + KSTEP * r, len - 1);
+      kr[r] = *(const u32x4*)(kb + kk * a.ldk);
+      vr[r] = *(const u32x4*)(vb + kk * a.ldv);
+    }
+    // difference key - query of entry w: kv0 - (qblk0 + 127) + w
+    if (RB && tid < 192)
+      br = a.rel_bias[(long)h * (2 * a.rb_L - 1) + min(max(kv0 - qblk0 - 127 + tid + a.rb_L - 1, 0), 2 * a.rb_L - 2)];
+  };
+  auto store_tile = [&](int buf, const u32x4 (&kr)[CPT], const u32x4 (&vr)[CPT], float br) {
+    char* kd = smem + buf * (2 * TILE);
+#pragma unroll
+    for (int r = 0; r < CPT; ++r) {
+      *(u32x4*)(kd + k_off<D>(lkey + KSTEP * r, lc)) = kr[r];
+      *(u32x4*)(kd + TILE + v_off<D>(lkey + KSTEP * r, lc)) = vr[r];
+    }
+    if (RB && tid < 192) rel[buf * 192 + tid] = br;
+  };
+
+  // Q fragments (B operand of S^T = K Q^T): lane holds Q[q0 + 16 u + r16][32 s + 8 g .. + 8]
+  bf16x8 qf[2][DS];
+  {
+    u32x4 k0[CPT], v0[CPT], k1[CPT], v1[CPT];
+    float b0 = 0.f, b1 = 0.f;
+    load_tile(0, k0, v0, b0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bf16_t* qp = a.q + (base + min(q0 + 16 * u + r16, len - 1)) * a.ldq + (long)h * D + 8 * g;
+#pragma unroll
+      for (int s = 0; s < DS; ++s) qf[u][s] = *(const bf16x8*)(qp + 32 * s);
+    }
+    if (D < 128 && len > 64) load_tile(64, k1, v1, b1);
+    store_tile(0, k0, v0, b0);
+    if (D == 128 && len > 64) load_tile(64, k1, v1, b1);  // registers
+    if (len > 64) store_tile(1, k1, v1, b1);
+  }
+  __syncthreads();
+
+  f32x4 o[2][DT];  // O^T: row d = 16 c + 4 g + i, column q0 + 16 u + r16
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int c = 0; c < DT; ++c) o[u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+  for (int kv0 = 0, cur = 0; kv0 < len; kv0 += 64, cur ^= 1) {
+    const bool more = kv0 + 128 < len;
+    u32x4 kr[CPT], vr[CPT];
+    float br = 0.f;
+    if (more) load_tile(kv0 + 128, kr, vr, br);
+    const char* const Ks = smem + cur * (2 * TILE);
+    const char* const Vs = Ks + TILE;
+    if (q0 < len) {
+      // ---- S^T[t][u] = K[16 t ..][:] Q[u]^T, in log2 units ----
+      f32x4 st[4][2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) st[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int s = 0; s < DS; ++s) {
+          const bf16x8 kf = *(const bf16x8*)(Ks + k_off<D>(16 * t + r16, 4 * s + g));
+#pragma unroll
+          for (int u = 0; u < 2; ++u) st[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[u][s], st[t][u], 0, 0, 0);
+        }
+      float bias[5][4];  // by t - u + 1
+      if constexpr (RB) {
+        const float* const rp = rel + cur * 192 + 127 + 4 * g - 32 * wid - r16;
+#pragma unroll
+        for (int d = 0; d < 5; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) bias[d][i] = rp[16 * (d - 1) + i];
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            st[t][u][i] = RB ? fmaf(st[t][u][i], a.scale_log2, bias[t - u + 1][i]) : st[t][u][i] * a.scale_log2;
+      if (kv0 + 64 > len) {  // the last tile
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st[t][u][i] = kv0 + 16 * t + 4 * g + i < len ? st[t][u][i] : -INFINITY;
+      }
+      // ---- online softmax: the query is the lane's column ----
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float mx = st[0][u][0];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[t][u][i]);
+        const float mn = fmaxf(m[u], over_groups(mx, [](float x, float y) { return fmaxf(x, y); }));
+        const float mu = mn == -INFINITY ? 0.f : mn;
+        const float alpha = exp2_raw(m[u] - mu);
+        m[u] = mn;
+        float rs = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma clang fp contract(off)  // the scaled score is rounded before, as where it is masked
+            st[t][u][i] = exp2_raw(st[t][u][i] - mu);
+            rs += st[t][u][i];
+          }
+        l[u] = l[u] * alpha + over_groups(rs, [](float x, float y) { return x + y; });
+        if (kv0 > 0 && __any(alpha != 1.f)) {
+#pragma unroll
+          for (int c = 0; c < DT; ++c) o[u][c] *= alpha;
+        }
+      }
+      // ---- O^T += V^T P^T ----
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 pa[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) pa[u] = pack_bf16x8(st[2 * ks][u], st[2 * ks + 1][u]);
+        const int key = 32 * ks + 4 * g + (lane >> 2 & 3), pcol = lane & 3;  // tr-read addressing within the 16-lane group
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {
+          const int col = 16 * c + 4 * pcol;
+          const s16x4 lo = ds_tr16(Vs + v_off<D>(key, col >> 3) + ((col & 7) << 1));
+          const s16x4 hi = ds_tr16(Vs + v_off<D>(key + 16, col >> 3) + ((col & 7) << 1));
+          const bf16x8 vf = cat_tr(lo, hi);
+#pragma unroll
+          for (int u = 0; u < 2; ++u) o[u][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pa[u], o[u][c], 0, 0, 0);
+        }
+      }
+    }
+    if (more) {  // the tile after the next one takes this one's place
+      __syncthreads();
+      store_tile(cur, kr, vr, br);
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const float inv = l[u] > 0.f ? 1.f / l[u] : 0.f;
+    const int row = q0 + 16 * u + r16;
+    if (row >= len) continue;
+    bf16_t* const op = a.o + (base + row) * a.ldo + (long)h * D + 4 * g;
+#pragma unroll
+    for (int c = 0; c < DT; ++c)
+      *(uint2*)(op + 16 * c) = make_uint2(pack2bf(o[u][c][0] * inv, o[u][c][1] * inv), pack2bf(o[u][c][2] * inv, o[u][c][3] * inv));
   }
 }
 
@@ -1062,9 +1231,9 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 #pragma unroll
     for (int o2 = 1; o2 < 16; o2 <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o2, 64));
     const float mn = fmaxf(m, mx);  // finite: every tile holds >= 1 valid key
-    const float alpha = exp2f(m - mn);
+    const float alpha = exp2_raw(m - mn);
     m = mn;
-    const float pk = exp2f(sc - mn);
+    const float pk = exp2_raw(sc - mn);
     float rs = pk;
 #pragma unroll
     for (int o2 = 1; o2 < 16; o2 <<= 1) rs += __shfl_xor(rs, o2, 64);
@@ -1436,12 +1605,12 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float mn = fmaxf(m, mx);  // finite: every tile holds >= 1 valid key
-    const float alpha = exp2f(m - mn);
+    const float alpha = exp2_raw(m - mn);
     m = mn;
     float rs = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float pv = exp2f(st[i] - mn);
+      const float pv = exp2_raw(st[i] - mn);
       st[i] = KV8 ? pv * vs[i] : pv;  // fp8: the V scale of key c0 + 4 g + i rides on P
       rs += pv;
     }
@@ -1758,7 +1927,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnBwdArgs a) {
           bool ok = key_valid && qq < a.S;
           if (a.causal) ok = ok && mykey <= qq;
           if (a.window > 0) ok = ok && (qq - mykey) < a.window;
-          const float p = ok ? exp2f(sp[u][i] * a.scale_log2 - lse_s[ql]) : 0.f;
+          const float p = ok ? exp2_raw(sp[u][i] * a.scale_log2 - lse_s[ql]) : 0.f;
           sp[u][i] = p;
           dp[u][i] = p * (dp[u][i] - del_s[ql]);
         }
@@ -1923,7 +2092,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnBwdArgs a) {
         bool ok = kk >= start && kk < a.S && qq < a.S;
         if (a.causal) ok = ok && kk <= qq;
         if (a.window > 0) ok = ok && (qq - kk) < a.window;
-        const float pv = ok ? exp2f(st[t][i] * a.scale_log2 - lse2) : 0.f;
+        const float pv = ok ? exp2_raw(st[t][i] * a.scale_log2 - lse2) : 0.f;
         st[t][i] = pv * (dp[t][i] - del);  // dS^T
       }
     // dQ += dS · K: A = packed dS^T accumulators [q][keys], B = K^T by transposed reads
@@ -2029,13 +2198,25 @@ extern "C" int rt_attn_packed(const void* q, long ldq, const void* k, long ldk, 
   a.o = (bf16_t*)o; a.ldo = ldo; a.rel_bias = rel_bias; a.rb_L = rb_L; a.B = B; a.Sq = rows; a.Sk = rows; a.Hq = H;
   a.Hkv = H; a.scale_log2 = scale * 1.4426950408889634f; a.off = off;
   if (B == 0 || rows == 0) return 0;
-  dim3 grid((longest + 127) / 128, H, B), block(256);
+  a.nx = (longest + 127) / 128;
+  a.gh = std::max(1, 512 / (2 * D));
+  while (H % a.gh) a.gh /= 2;
+  const long groups = (long)B * (H / a.gh), blocks = (groups + 7) / 8 * 8 * a.nx * a.gh;
+  if (blocks > INT_MAX) return -1;
+  a.groups = (int)groups;
+  dim3 grid((unsigned)blocks), block(256);
+#define AP(DD)                                                                                     \
+  case DD:                                                                                         \
+    if (rel_bias) hipLaunchKernelGGL((attn_packed_kernel<DD, true>), grid, block, 0, stream, a);  \
+    else hipLaunchKernelGGL((attn_packed_kernel<DD, false>), grid, block, 0, stream, a);          \
+    break
   switch (D) {
-    case 32: hipLaunchKernelGGL((attn_fwd_kernel<32, 2, false, false, true>), grid, block, 0, stream, a); break;
-    case 64: hipLaunchKernelGGL((attn_fwd_kernel<64, 2, false, false, true>), grid, block, 0, stream, a); break;
-    case 128: hipLaunchKernelGGL((attn_fwd_kernel<128, 2, false, false, true>), grid, block, 0, stream, a); break;
+    AP(32);
+    AP(64);
+    AP(128);
     default: return -1;
   }
+#undef AP
   RT_LAUNCH_CHECK();
   return 0;
 }
