@@ -62,6 +62,10 @@ int rt_attn_fwd(const void*, long, const void*, long, const void*, long, void*, 
 int rt_gemm_image(const void*, long, const void*, void*, long, int, int, int, int, int, int, const float*, hipStream_t);
 int rt_attn_packed(const void*, long, const void*, long, const void*, long, void*, long, const long*, const float*, int, int,
                    int, int, int, int, float, hipStream_t);
+int rt_few_rows(const void*, long, const void*, long, const void*, const void*, void*, const void*, long, const void*, void*, long,
+                int, int, int, int, float, hipStream_t);
+int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
+                       float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
                    void*, long, int, int, int, int, float, hipStream_t);
 int rt_attn_decode_fused(const void*, long, void*, void*, int, const int*, const int*, const int*, const int*,
@@ -84,7 +88,7 @@ int rt_adamw(float*, const float*, float*, float*, void*, long, float, float, fl
 int rt_grad_sumsq_mixed(const void*, long, const float*, long, float*, int, hipStream_t);
 int rt_adamw_mixed(float*, const void*, long, const float*, float*, float*, void*, long, float, float, float, float,
                    float, int, float, const float*, int, float*, int*, hipStream_t);
-int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, hipStream_t);
+int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, const long*, hipStream_t);
 int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
@@ -1268,9 +1272,160 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   auto out = at::empty({B, H}, x.options().dtype(at::kFloat));
   if (lengths.has_value() && lengths->defined()) CHECK_I32(*lengths);
   check_rc(rt_pool_norm(x.data_ptr(), (const int*)opt_ptr(lengths), (const long*)opt_ptr(off), packed ? x.size(0) : 0, (int)B,
-                        (int)S, (int)H, normalize ? 1 : 0, out.data_ptr<float>(), cur_stream()),
+                        (int)S, (int)H, normalize ? 1 : 0, out.data_ptr<float>(), nullptr, cur_stream()),
            "pool_norm");
   return out;
+}
+
+// act(x w^T + bias) of at most 64 rows; with a norm (res, lw, lb) of LN(x + res), which is returned second
+std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Tensor>& bias, int64_t act, const optional<Tensor>& res,
+                             const optional<Tensor>& lw, const optional<Tensor>& lb, double eps) {
+  for (const Tensor* t : {&x, &w}) {
+    CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ROWS(*t); CHECK_ALIGN16(*t);
+    TORCH_CHECK(t->stride(0) % 8 == 0, "few_rows: row strides must be multiples of 8");
+  }
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(w.size(1) == K, "few_rows: K mismatch");
+  auto vec = [&](const optional<Tensor>& t, int64_t n) {
+    if (!t) return;
+    CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ALIGN16(*t);
+    TORCH_CHECK(t->is_contiguous() && t->numel() == n, "few_rows: vectors of ", n);
+  };
+  vec(bias, N); vec(lw, K); vec(lb, K);
+  const bool norm = lw.has_value();
+  TORCH_CHECK(norm == lb.has_value() && norm == res.has_value(), "few_rows: a norm has a residual, a weight and a bias");
+  Tensor xo;
+  if (norm) {
+    CHECK_CUDA(*res); CHECK_BF16(*res); CHECK_ALIGN16(*res);
+    TORCH_CHECK(res->is_contiguous() && res->sizes() == x.sizes(), "few_rows: residual");
+    xo = at::empty({M, K}, x.options());
+  }
+  auto y = at::empty({M, N}, x.options());
+  check_rc(rt_few_rows(x.data_ptr(), x.stride(0), opt_ptr(res), K, opt_ptr(lw), opt_ptr(lb), norm ? xo.data_ptr() : nullptr, w.data_ptr(),
+                       w.stride(0), opt_ptr(bias), y.data_ptr(), N, (int)M, (int)N, (int)K, (int)act, (float)eps, cur_stream()),
+           "few_rows");
+  return {y, xo};
+}
+
+// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it
+static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act) {
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
+  int64_t split = 1, bn = 0;
+  if (M <= 512) {
+    bn = act == 0 ? 128 : 256;
+    const int64_t tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
+    if (tiles < 128 && N % 16 == 0) split = std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles));
+  }
+  if (split > 1) {
+    auto slabs = at::empty({split * M * N}, x.options().dtype(at::kFloat));
+    return gemm_splitk(x, w, split, slabs, b, act, std::nullopt, std::nullopt, bn, {});
+  }
+  return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, 1, std::nullopt, std::nullopt, std::nullopt, bn, {});
+}
+
+// A sentence encoder's forward over texts without padding (see attn_packed), pooled and normalised, written to out[to[b]]:
+// one call for the 40 and more launches, which from Python take longer to issue than a short query's take to run. emb: word and
+// position tables, token type row or null, norm weight, norm bias; layers: qkv, o, ln1, fc1, fc2, ln2, a weight and a bias each.
+// False where something is not as this path needs it (the caller goes op by op, which says what).
+bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int64_t longest,
+                    const std::vector<optional<Tensor>>& emb, const std::vector<Tensor>& layers, int64_t heads, double eps,
+                    const optional<Tensor>& rel_bias, int64_t rb_L, bool normalize, Tensor out, const Tensor& to) {
+  if (emb.size() != 5 || layers.empty() || layers.size() % 12 || !emb[0] || !emb[1] || !emb[3] || !emb[4]) return false;
+  const Tensor &word = *emb[0], &ptab = *emb[1];
+  auto plain = [&](const Tensor& t, std::initializer_list<int64_t> size) {
+    return t.is_cuda() && t.device() == word.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
+           (uintptr_t)t.data_ptr() % 16 == 0 && t.sizes() == at::IntArrayRef(size.begin(), size.size());
+  };
+  if (word.dim() != 2 || ptab.dim() != 2) return false;
+  const int64_t H = word.size(1), F = layers[6].dim() == 2 ? layers[6].size(0) : 0, M = ids.numel(), D = heads ? H / heads : 0;
+  if (H % 16 || H > 1024 || F % 16 || !F || heads * D != H || (D != 32 && D != 64 && D != 128) || M > INT_MAX || M == 0) return false;
+  if (!plain(word, {word.size(0), H}) || !plain(ptab, {ptab.size(0), H}) || !plain(*emb[3], {H}) || !plain(*emb[4], {H}) ||
+      (emb[2] && !plain(*emb[2], {H})))
+    return false;
+  for (size_t l = 0; l < layers.size(); l += 12) {
+    const int64_t rows[6] = {3 * H, H, H, F, H, H}, cols[6] = {H, H, 0, H, F, 0};
+    for (int k = 0; k < 6; ++k) {
+      const Tensor &w = layers[l + 2 * k], &b = layers[l + 2 * k + 1];
+      if (!(cols[k] ? plain(w, {rows[k], cols[k]}) : plain(w, {rows[k]})) || !plain(b, {rows[k]})) return false;
+    }
+  }
+  for (const Tensor* t : {&ids, &pos, &off, &to})
+    if (t->device() != word.device() || t->scalar_type() != at::kLong || t->dim() != 1 || !t->is_contiguous()) return false;
+  const int64_t B = off.numel() - 1;
+  if (pos.numel() != M || B < 1 || to.numel() != B || longest < 0 || longest > M) return false;
+  if (out.device() != word.device() || out.scalar_type() != at::kFloat || out.dim() != 2 || !out.is_contiguous() || out.size(1) != H)
+    return false;
+  if (rel_bias && !(rel_bias->device() == word.device() && rel_bias->scalar_type() == at::kFloat && rel_bias->is_contiguous() &&
+                    rel_bias->dim() == 2 && rel_bias->size(0) == heads && rel_bias->size(1) == 2 * rb_L - 1 && rb_L >= longest))
+    return false;
+
+  hipStream_t st = cur_stream();
+  auto rows = [&](int64_t n) { return at::empty({M, n}, word.options()); };
+  auto attend = [&](const Tensor& qkv, Tensor& a) {
+    const char* q = (const char*)qkv.data_ptr();
+    check_rc(rt_attn_packed(q, 3 * H, q + 2 * H, 3 * H, q + 4 * H, 3 * H, a.data_ptr(), H, (const long*)off.data_ptr(),
+                            (const float*)opt_ptr(rel_bias), (int)rb_L, (int)B, (int)M, (int)longest, (int)heads, (int)D,
+                            (float)(1.0 / std::sqrt((double)D)), st),
+             "encoder: attention");
+  };
+  auto norm = [&](const Tensor& d, const Tensor& res, const Tensor& w, const Tensor& b, Tensor& y) {
+    check_rc(rt_norm_fwd(1, d.data_ptr(), res.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), nullptr, nullptr, nullptr, (int)M,
+                         (int)H, (float)eps, nullptr, 0, st),
+             "encoder: norm");
+  };
+  Tensor x = rows(H), a = rows(H);
+  check_rc(rt_embed_norm_rows(word.data_ptr(), (const long*)ids.data_ptr(), ptab.data_ptr(), (const long*)pos.data_ptr(),
+                              emb[2] ? emb[2]->data_ptr() : nullptr, emb[3]->data_ptr(), emb[4]->data_ptr(), x.data_ptr(), (int)M,
+                              (int)H, (float)eps, st),
+           "encoder: embedding");
+  if (M <= 64 && H % 32 == 0 && F % 32 == 0) {
+    // up to 32 rows the products normalise their input themselves (few_rows.hip): 5 launches a layer instead of 7
+    const bool own = M <= 32;
+    Tensor qkv = rows(3 * H), f = rows(F), d = rows(H), z = rows(H);
+    auto product = [&](const Tensor& in, const Tensor& w, const Tensor& b, int act, Tensor& y) {
+      check_rc(rt_few_rows(in.data_ptr(), in.size(1), nullptr, 0, nullptr, nullptr, nullptr, w.data_ptr(), w.size(1), b.data_ptr(),
+                           y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)w.size(1), act, 0.f, st),
+               "encoder: product");
+    };
+    // y = act(LN(d + x) w^T + b); x becomes LN(d + x)
+    auto norm_product = [&](const Tensor& lw, const Tensor& lb, const Tensor& w, const Tensor& b, int act, Tensor& y) {
+      if (own) {
+        check_rc(rt_few_rows(d.data_ptr(), H, x.data_ptr(), H, lw.data_ptr(), lb.data_ptr(), z.data_ptr(), w.data_ptr(), H,
+                             b.data_ptr(), y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)H, act, (float)eps, st),
+                 "encoder: norm and product");
+      } else {
+        norm(d, x, lw, lb, z);
+        product(z, w, b, act, y);
+      }
+      std::swap(x, z);
+    };
+    for (size_t l = 0; l < layers.size(); l += 12) {
+      const Tensor* t = &layers[l];
+      if (l == 0) product(x, t[0], t[1], 0, qkv);
+      else norm_product(t[-2], t[-1], t[0], t[1], 0, qkv);
+      attend(qkv, a);
+      product(a, t[2], t[3], 0, d);
+      norm_product(t[4], t[5], t[6], t[7], 2, f);
+      product(f, t[8], t[9], 0, d);
+    }
+    const Tensor* t = &layers[layers.size() - 2];
+    norm(d, x, t[0], t[1], z);
+    std::swap(x, z);
+  } else {
+    for (size_t l = 0; l < layers.size(); l += 12) {
+      const Tensor* t = &layers[l];
+      attend(encoder_linear(x, t[0], t[1], 0), a);
+      Tensor d = encoder_linear(a, t[2], t[3], 0), y = rows(H);
+      norm(d, x, t[4], t[5], y);
+      d = encoder_linear(encoder_linear(y, t[6], t[7], 2), t[8], t[9], 0);
+      norm(d, y, t[10], t[11], x);
+    }
+  }
+  check_rc(rt_pool_norm(x.data_ptr(), nullptr, (const long*)off.data_ptr(), M, (int)B, 0, (int)H, normalize ? 1 : 0,
+                        out.data_ptr<float>(), (const long*)to.data_ptr(), st),
+           "encoder: pooling");
+  return true;
 }
 
 std::vector<Tensor> topk(const Tensor& scores, int64_t k, const optional<Tensor>& idmap, bool finite) {
@@ -1485,6 +1640,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_packed", &attn_packed, "bidirectional self-attention of packed sequences", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("off"), py::arg("longest"), py::arg("H"), py::arg("D"), py::arg("scale"),
         py::arg("rel_bias") = py::none(), py::arg("rb_L") = 0);
+  m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
+        py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
+        py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
+  m.def("few_rows", &few_rows, "act(x w^T + b) of at most 64 rows, x normalised first if asked", py::arg("x"), py::arg("w"),
+        py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
+        py::arg("lb") = py::none(), py::arg("eps") = 0.0);
   m.def("attn_fwd", &attn_fwd);
   m.def("attn_decode", &attn_decode);
   m.def("attn_bwd", &attn_bwd, "flash attention backward (RoPE backward optionally fused into dQ / dK)",

@@ -32,6 +32,7 @@
 // atomic accumulation (narrow outputs with a deep reduction, e.g. LoRA dA / dB).
 // Reduction tails (K % 64 != 0) and the K-extension read a zero page for out-of-range k.
 #include "rt_common.h"
+#include "rt_gelu.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -106,7 +107,7 @@ __device__ __forceinline__ int kmaj_swz(int k) { return ((k >> 3) & 1) << 1; }
 __device__ __forceinline__ float act_fn(float x, int act) {
   switch (act) {
     case E_RELU: return fmaxf(x, 0.f);
-    case E_GELU: return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
+    case E_GELU: return gelu_erf(x);
     case E_GELU_TANH: {
       const float k0 = 0.7978845608028654f, k1 = 0.044715f;
       return 0.5f * x * (1.f + tanhf(k0 * (x + k1 * x * x * x)));
@@ -117,46 +118,6 @@ __device__ __forceinline__ float act_fn(float x, int act) {
   }
 }
 
-// Two GELU results in bf16, the bits of act_fn's. erff computes two ranges per lane, which in the epilogue of a 768 -> 3072
-// product took nearly as long as the product. Here erf(x / sqrt 2) is x P(x^2) on |x| <= 5.2 (degree 13 in v = x^2 / 13.52 - 1, least
-// squares reweighted towards the maximum) and 1 beyond: 3.3e-7 from erff at most, over all x. The results with 5e-7 more and
-// 5e-7 less enclose act_fn's fp32 result; both rounding to the same bf16, that is the answer, else erff decides: about 1 pair of
-// 2500 for x around 0, every second one at -3.8. 41.5k rows, 768 -> 3072, inputs of
-// standard deviation 0.55 / 1.1: 389 / 467 -> 290 / 307 us (without GELU 242); 24k rows, 384 -> 1536: 108 / 144 -> 82 / 82 (49).
-// gelu2_fast: the packed results and whether they are the answer.
-__device__ __forceinline__ bool gelu2_fast(float x0, float x1, uint32_t& y) {
-  float hi[2], lo[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const float x = k ? x1 : x0;
-    const float z = __builtin_amdgcn_fmed3f(x, -5.2f, 5.2f);
-    const float v = fmaf(z * z, 2.f / (5.2f * 5.2f), -1.f);
-    float q = -0.0009625543607398868f;
-    q = fmaf(q, v, 0.0025370221119374037f);
-    q = fmaf(q, v, -0.0024429871700704098f);
-    q = fmaf(q, v, 0.0036002453416585922f);
-    q = fmaf(q, v, -0.009578078053891659f);
-    q = fmaf(q, v, 0.017119934782385826f);
-    q = fmaf(q, v, -0.0250102411955595f);
-    q = fmaf(q, v, 0.03590957447886467f);
-    q = fmaf(q, v, -0.04944726079702377f);
-    q = fmaf(q, v, 0.06397991627454758f);
-    q = fmaf(q, v, -0.07985963672399521f);
-    q = fmaf(q, v, 0.10004904121160507f);
-    q = fmaf(q, v, -0.13548733294010162f);
-    q = fmaf(q, v, 0.2718999981880188f);
-    const float h = 0.5f * x;
-    hi[k] = h * fmaf(z, q, 1.f + 5e-7f);
-    lo[k] = fmaf(h, -1e-6f, hi[k]);
-  }
-  y = pack2bf(hi[0], hi[1]);
-  return y == pack2bf(lo[0], lo[1]);
-}
-__device__ __forceinline__ uint32_t gelu2_bf16(float x0, float x1) {
-  uint32_t y;
-  if (__builtin_expect(!gelu2_fast(x0, x1, y), 0)) y = pack2bf(act_fn(x0, E_GELU), act_fn(x1, E_GELU));
-  return y;
-}
 
 // counted wait: leave the n newest granules (wave-uniform; n = 4, 2, 1 or 0 at the call sites) in
 // flight. BN = 256: every granule is 2 LDS-DMA instructions per lane -> vmcnt(2n). BN = 128: the B
@@ -731,27 +692,6 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Args p) {
 // 189 -> 154 (without: 122 -> 114), 20000 x 1152 x 384: 32 -> 26, 1000 x 1536 x 384 with GELU: 32 -> 20.
 constexpr int DUO_G = 16384;
 
-// 16 GELUs of one accumulator row block; the pairs that gelu2_bf16 could not decide are redone with erff in ONE copy of its
-// code, picked by lane from the 8 pairs (about one row block in five has any).
-__device__ __forceinline__ void gelu16_bf16(const float (&x)[16], uint32_t (&y)[8]) {
-  unsigned open = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) open |= gelu2_fast(x[2 * k], x[2 * k + 1], y[k]) ? 0u : 1u << k;
-  while (__any(open != 0)) {
-    float a = 0.f, b = 0.f;
-    const int k0 = open ? __ffs(open) - 1 : 8;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a = k == k0 ? x[2 * k] : a;
-      b = k == k0 ? x[2 * k + 1] : b;
-    }
-    const uint32_t v = pack2bf(act_fn(a, E_GELU), act_fn(b, E_GELU));
-#pragma unroll
-    for (int k = 0; k < 8; ++k) y[k] = k == k0 ? v : y[k];
-    open &= open - 1;
-  }
-}
-
 template <int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_duo_kernel(Args p) {
   constexpr int LDT = 128 + 4;  // row of the epilogue's bf16 tile
@@ -920,7 +860,10 @@ __global__ __launch_bounds__(256, 2) void gemm_duo_kernel(Args p) {
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) x[4 * j + r] = acc[i][j][r] + bcol[j][r];
-      gelu16_bf16(x, y);
+      unsigned open = 0;  // about one row block in five has any
+#pragma unroll
+      for (int k = 0; k < 8; ++k) open |= gelu2_fast(x[2 * k], x[2 * k + 1], y[k]) ? 0u : 1u << k;
+      gelu2_settle<8>(x, y, open);
 #pragma unroll
       for (int j = 0; j < 4; ++j) *(uint2*)(to + j * 16) = make_uint2(y[2 * j], y[2 * j + 1]);
     } else {

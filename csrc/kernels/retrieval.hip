@@ -15,7 +15,7 @@ namespace rt {
 // the other.
 __global__ __launch_bounds__(256) void pool_norm_kernel(const bf16_t* __restrict__ x, const int* __restrict__ lengths,
                                                         const long* __restrict__ off, long rows, int S, int H,
-                                                        int normalize, float* __restrict__ out) {
+                                                        int normalize, float* __restrict__ out, const long* __restrict__ to) {
   extern __shared__ float acc[];  // [H]
   __shared__ float sb[4];
   const int b = blockIdx.x;
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void pool_norm_kernel(const bf16_t* __restrict
   for (int h = threadIdx.x; h < H; h += 256) ss += acc[h] * acc[h];
   const float tot = block_sum(ss, sb);
   const float inv = normalize ? 1.f / fmaxf(sqrtf(tot), 1e-12f) : 1.f;
-  for (int h = threadIdx.x; h < H; h += 256) out[(long)b * H + h] = acc[h] * inv;
+  for (int h = threadIdx.x; h < H; h += 256) out[(to ? to[b] : (long)b) * H + h] = acc[h] * inv;
 }
 
 __device__ __forceinline__ uint32_t okey(float f) {
@@ -340,10 +340,10 @@ __global__ __launch_bounds__(256) void segment_mean_kernel(const float* __restri
 using namespace rt;
 
 extern "C" int rt_pool_norm(const void* x, const int* lengths, const long* off, long rows, int B, int S, int H,
-                            int normalize, float* out, hipStream_t stream) {
+                            int normalize, float* out, const long* to, hipStream_t stream) {
   if (B == 0) return 0;
   hipLaunchKernelGGL(pool_norm_kernel, dim3(B), dim3(256), H * sizeof(float), stream, (const bf16_t*)x, lengths, off, rows,
-                     S, H, normalize, out);
+                     S, H, normalize, out, to);
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -32,6 +32,10 @@ def relative_position_bucket(rel: torch.Tensor, num_buckets: int = 32, max_dista
     return ret + torch.where(is_small, n, val_large)
 
 
+# a layer's parameters in the native forward's order
+_LAYER = ("qkv_w", "qkv_b", "o_w", "o_b", "ln1_w", "ln1_b", "fc1_w", "fc1_b", "fc2_w", "fc2_b", "ln2_w", "ln2_b")
+
+
 class EncoderLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, device=None, dtype=torch.bfloat16):
         super().__init__()
@@ -132,11 +136,27 @@ class SentenceEncoder(nn.Module):
     def first_position(self) -> int:
         return self.cfg.pad_token_id + 1 if self.cfg.arch == "mpnet" else 0
 
+    def _encode_native(self, ids, pos, off, longest: int, normalize: bool, out, to) -> bool:
+        """The whole of :meth:`encode_packed` in one native call, to rows ``to`` of ``out``; False: not for this model."""
+        if not (ids.is_cuda and self.cfg.hidden_act == "gelu" and type(self)._states is SentenceEncoder._states
+                and "_states" not in vars(self) and all(type(layer) is EncoderLayer for layer in self.layers)
+                and not ops.batch_invariant_on()):
+            return False
+        lut, L = self._bias_lut(longest, ids.device)
+        emb = [self.word_embed, self.pos_embed, self.type_embed[0] if self.cfg.type_vocab_size else None, self.emb_ln_w, self.emb_ln_b]
+        layers = [getattr(layer, name) for layer in self.layers for name in _LAYER]
+        return ops.native().encoder_packed(ids, pos, off, longest, emb, layers, self.cfg.num_heads, self.cfg.norm_eps, lut, L,
+                                           normalize, out, to)
+
     @torch.no_grad()
-    def encode_packed(self, ids: torch.Tensor, pos: torch.Tensor, off: torch.Tensor, longest: int,
-                      normalize: bool = True) -> torch.Tensor:
+    def encode_packed(self, ids: torch.Tensor, pos: torch.Tensor, off: torch.Tensor, longest: int, normalize: bool = True,
+                      out: torch.Tensor | None = None, to: torch.Tensor | None = None) -> torch.Tensor:
         """:meth:`encode_ids` of texts without padding: rows [off[b], off[b + 1]) of ``ids`` are text b, none longer than
-        ``longest``, at positions ``pos`` (from ``first_position``)."""
+        ``longest``, at positions ``pos`` (from ``first_position``). ``out`` (fp32): text b goes to its row ``to[b]``."""
+        if out is not None:
+            if longest == 0 or not self._encode_native(ids, pos, off, longest, normalize, out, to):
+                out[to] = self.encode_packed(ids, pos, off, longest, normalize).float()
+            return out
         nh, D = self.cfg.num_heads, self.cfg.head_dim
         if longest == 0:
             return torch.zeros(len(off) - 1, self.cfg.hidden_size, device=ids.device)

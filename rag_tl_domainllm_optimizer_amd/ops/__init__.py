@@ -5,7 +5,7 @@ from .linear import (  # noqa: F401
     ACT_DSWIGLU, ACT_IDS, ACT_SWIGLU, KMAJ, ROW, FoldCache, LoRAGroup, ShufCache, SplitK, gemm, gemm_big, gemm_decode, gemm_nn, gemm_tn, linear,
     swiglu_mlp, gemm_rope, linear_rope, rope_fusable,
     refresh_lora_batched,
-    linear_deferred, gemm_image, image_held, image_rows, image_split, shuffle_decode, batch_invariant, Glu, project, glu_project, act_project, branch_project, TransposeCache, ACT_RELU2)
+    linear_deferred, gemm_image, image_held, image_rows, image_split, shuffle_decode, batch_invariant, batch_invariant_on, Glu, project, glu_project, act_project, branch_project, TransposeCache, ACT_RELU2)
 from .norm import MoePairs, branch_norm, embed_norm, layer_norm, rms_norm  # noqa: F401
 from .moe import moe_ff, moe_route  # noqa: F401
 from .window import WindowDims, window_attention  # noqa: F401

@@ -58,6 +58,11 @@ def _batch_invariant_on() -> bool:
     return getattr(_BI, "depth", 0) > 0
 
 
+def batch_invariant_on() -> bool:
+    """Whether this thread is inside :func:`batch_invariant`."""
+    return _batch_invariant_on()
+
+
 @contextlib.contextmanager
 def batch_invariant(on: bool = True):
     """Row-invariant GEMM numerics inside the block: every token-parallel GEMM (``gemm``) runs the

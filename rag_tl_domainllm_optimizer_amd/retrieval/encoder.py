@@ -65,10 +65,14 @@ class Encoder:
         # every batch is tokenised and uploaded ahead of the first forward: between them the host only launches
         order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device,
                                                       self.model.first_position)
-        r = 0
+        r, m = 0, self.model
+        placed = type(m).encode_packed is SentenceEncoder.encode_packed and "encode_packed" not in vars(m)
         for ids, pos, off, longest in batches:
             n = len(off) - 1
-            out[order[r:r + n]] = self.model.encode_packed(ids, pos, off, longest, normalize).float()
+            if placed:
+                m.encode_packed(ids, pos, off, longest, normalize, out, order[r:r + n])
+            else:
+                out[order[r:r + n]] = m.encode_packed(ids, pos, off, longest, normalize).float()
             r += n
         return out
 

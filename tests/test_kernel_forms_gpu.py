@@ -387,6 +387,75 @@ def test_packed_attention_equals_padded(D, H, bias, lens):
     assert torch.equal(ops.pool_normalize_packed(x[keep], off, S), ops.pool_normalize(x, n))
 
 
+# ---------------------------------------------------------------------------------------------- encoders, few rows
+@pytest.mark.parametrize("M,N,K,act,norm", [(1, 16, 32, 0, False), (15, 384, 384, 2, True), (16, 1536, 768, 2, True),
+                                            (17, 48, 480, 0, True), (32, 80, 1024, 0, True), (33, 32, 1536, 2, False),
+                                            (64, 1152, 544, 0, False), (48, 16, 3072, 0, False)])
+def test_few_rows(M, N, K, act, norm):
+    """Products of at most 64 rows, the norm ahead of up to 32 among them: around the row tiles, both splits of K (480 / 32 = 15
+    steps on four waves, 544 / 32 = 17 on eight), strided rows."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+
+    def r(*s, m=1.0):
+        return (torch.randn(*s, generator=g, device=DEV) * m).bfloat16()
+    x, w, b = r(M, K + 8)[:, :K], r(N, K + 24, m=K ** -0.5)[:, :K], r(N)
+    xd = x.double()
+    kw = {}
+    if norm:
+        kw = dict(res=r(M, K), lw=r(K), lb=r(K), eps=1e-5)
+    y, xo = ops.native().few_rows(x, w, b, act, **kw)
+    if norm:
+        h = (x + kw["res"]).double()
+        want = torch.nn.functional.layer_norm(h, (K,), kw["lw"].double(), kw["lb"].double(), 1e-5)
+        # fp32 arithmetic, one rounding to bf16
+        torch.testing.assert_close(xo.double(), want, rtol=2.0 ** -8, atol=1e-4)
+        xd = xo.double()
+    want = xd @ w.double().t() + b.double()
+    if act:
+        want = torch.nn.functional.gelu(want)
+    # fp32 sums of K terms, one rounding to bf16
+    torch.testing.assert_close(y.double(), want, rtol=2.0 ** -8, atol=2.0 ** -22 * K ** 0.5 * float(xd.abs().max()) * 4 + 1e-6)
+
+
+@pytest.mark.parametrize("preset", ["minilm-l6", "mpnet-base"])
+@pytest.mark.parametrize("lens", [[1], [3, 9, 2], [17, 11], [33, 30], [20, 41, 64, 7], [120] * 7])
+def test_native_encoder_forward_is_the_ops_forward(preset, lens):
+    """One native call against the same forward op by op, over the ways it goes (norms in the products up to 32 rows, apart up
+    to 64, general products beyond: the same kernels, so the same bits), rows placed in another order."""
+    from rag_tl_domainllm_optimizer_amd import models
+    import dataclasses
+
+    cfg = dataclasses.replace(models.resolve_preset(preset), num_layers=2)
+    m = models.SentenceEncoder(cfg, device=DEV, dtype=torch.bfloat16, init=False).eval()
+    g = torch.Generator(device=DEV).manual_seed(len(lens))
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            p.normal_(1.0 if "ln" in name and name.endswith("_w") else 0.0, 0.05, generator=g)
+    n = torch.tensor(lens, device=DEV)
+    off = torch.nn.functional.pad(n.cumsum(0), (1, 0))
+    rows = int(off[-1])
+    ids = torch.randint(4, cfg.vocab_size, (rows,), generator=g, device=DEV)
+    pos = torch.cat([torch.arange(k, device=DEV) for k in lens]) + m.first_position
+    to = torch.randperm(len(lens), generator=g, device=DEV)
+    out = torch.full((len(lens) + 1, cfg.hidden_size), 7.0, device=DEV)
+    assert m._encode_native(ids, pos, off, max(lens), True, out, to)
+    want = m.encode_packed(ids, pos, off, max(lens))
+    assert (out[-1] == 7).all()
+    if rows > 64:
+        assert torch.equal(out[to], want)
+    else:  # other sums' order before bf16 roundings, over two layers
+        assert float(torch.nn.functional.cosine_similarity(out[to].double(), want.double()).min()) > 1 - 1e-4
+        _close(out[to] * cfg.hidden_size ** 0.5, want * cfg.hidden_size ** 0.5, rtol=0.05, atol=0.05)
+    # not for layers of another make: op by op again
+    class Other(type(m.layers[0])):
+        pass
+    m.layers[0].__class__ = Other
+    assert not m._encode_native(ids, pos, off, max(lens), True, out, to)
+    got = torch.zeros(len(lens), cfg.hidden_size, device=DEV)
+    m.encode_packed(ids, pos, off, max(lens), True, got, to)
+    assert torch.equal(got[to], want)
+
+
 # ---------------------------------------------------------------------------------------------- decode products, 65..128 rows
 @pytest.mark.parametrize("N,K,act", [(16, 64, 0), (48, 448, 0), (2048, 1024, 0), (4112, 2112, ops.ACT_RELU2), (33024, 256, 0),
                                      (64, 128, 5), (1056, 1088, 5), (33024, 320, 5)])
