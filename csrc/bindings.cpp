@@ -63,7 +63,8 @@ int rt_gemm_image(const void*, long, const void*, void*, long, int, int, int, in
 int rt_attn_packed(const void*, long, const void*, long, const void*, long, void*, long, const long*, const float*, int, int,
                    int, int, int, int, float, hipStream_t);
 int rt_few_rows(const void*, long, const void*, long, const void*, const void*, void*, const void*, long, const void*, void*, long,
-                int, int, int, int, float, hipStream_t);
+                int, int, int, int, float, int, int, hipStream_t);
+int rt_gemm_nt_parts(int, int, int, int*);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
                        float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
@@ -1277,12 +1278,28 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   return out;
 }
 
-// act(x w^T + bias) of at most 64 rows; with a norm (res, lw, lb) of LN(x + res), which is returned second
+// The K split of ops.gemm's token-parallel products (splitk_plan there): parts and the columns of a tile
+static std::pair<int64_t, int64_t> token_split(int64_t M, int64_t N, int64_t K, int64_t act) {
+  if (M > 512) return {1, 0};
+  const int64_t bn = act == 0 ? 128 : 256, tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
+  const int64_t split = tiles < 128 && N % 16 == 0 ? std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles)) : 1;
+  return {split, split == 1 && act ? 0 : bn};
+}
+
+// The parts in which the kernel that ops.gemm takes sums K (row-major operands, K % 64 == 0), for rt_few_rows
+struct KParts { int n, grp; };
+static KParts k_parts(int64_t M, int64_t N, int64_t K, int64_t act) {
+  KParts k{(int)token_split(M, N, K, act).first, 1};
+  if (M <= 64) k.n = rt_gemm_nt_parts((int)M, (int)N, (int)K, &k.grp);
+  return k;
+}
+
+// act(x w^T + bias); with a norm (res, lw, lb; at most 32 rows) of LN(x + res), which is returned second
 std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Tensor>& bias, int64_t act, const optional<Tensor>& res,
                              const optional<Tensor>& lw, const optional<Tensor>& lb, double eps) {
   for (const Tensor* t : {&x, &w}) {
     CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ROWS(*t); CHECK_ALIGN16(*t);
-    TORCH_CHECK(t->stride(0) % 8 == 0, "few_rows: row strides must be multiples of 8");
+    TORCH_CHECK(t->stride(0) % 8 == 0 && t->size(0) <= INT_MAX, "few_rows: row strides must be multiples of 8");
   }
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(w.size(1) == K, "few_rows: K mismatch");
@@ -1301,22 +1318,43 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
     xo = at::empty({M, K}, x.options());
   }
   auto y = at::empty({M, N}, x.options());
+  const KParts kp = k_parts(M, N, K, act);
   check_rc(rt_few_rows(x.data_ptr(), x.stride(0), opt_ptr(res), K, opt_ptr(lw), opt_ptr(lb), norm ? xo.data_ptr() : nullptr, w.data_ptr(),
-                       w.stride(0), opt_ptr(bias), y.data_ptr(), N, (int)M, (int)N, (int)K, (int)act, (float)eps, cur_stream()),
+                       w.stride(0), opt_ptr(bias), y.data_ptr(), N, (int)M, (int)N, (int)K, (int)act, (float)eps, kp.n, kp.grp,
+                       cur_stream()),
            "few_rows");
   return {y, xo};
 }
 
-// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it
+// Whether few_rows_kernel takes x w^T of M > 64 rows sooner than the tile kernels: it works in rounds of a workgroup per CU, each
+// 0.45 us per 32 k of a wave's part, 0.6 and 0.9 where a wave has two and four row tiles, behind 2.5 us; a lone 256 x 128 tile takes
+// 0.77 us per 64 k and 4, its GELU 9 more, and up to 512 rows the K split bounds that by 14 (K up to 2048) or 17. us, few_rows /
+// tiles: 400 x 1152 x 384 8.2 / 9.7, 400 x 384 x 1536 10.8 / 16.4, 640 x 384 x 1536 (one part) 23.6 / 22.7, 640 x 1536 x 384 with
+// GELU 14.2 / 18.8, 1500 x 768 x 768 34.5 / 14.3.
+static bool few_rows_pays(int64_t M, int64_t N, int64_t K, int64_t act) {
+  if (N % 16 || K % 64 || k_parts(M, N, K, act).n > 8) return false;
+  // parts of K, the waves over them, a wave's row tiles and the columns of a workgroup, as rt_few_rows has them
+  const int64_t ks = k_parts(M, N, K, act).n, ws = ks > 4 ? 8 : ks > 2 ? 4 : ks, rt = std::max<int64_t>(1, ws / 2), cols = ws > 1 ? 16 : 32;
+  const double rounds = (double)(((N + cols - 1) / cols * ((M + 63) / 64) + 255) / 256), steps = (double)((K / 64 + ks - 1) / ks * 2);
+  double tiles = 4 + 0.77 * K / 64;
+  if (act) tiles += 9;
+  else if (M <= 512) tiles = std::min(tiles, K > 2048 ? 17.0 : 14.0);
+  return 2.5 + (0.3 + 0.15 * rt) * steps * rounds < tiles;
+}
+
+// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it, or few_rows_kernel
 static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
-  int64_t split = 1, bn = 0;
-  if (M <= 512) {
-    bn = act == 0 ? 128 : 256;
-    const int64_t tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
-    if (tiles < 128 && N % 16 == 0) split = std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles));
+  if (M > 64 && few_rows_pays(M, N, K, act)) {
+    auto y = at::empty({M, N}, x.options());
+    const KParts kp = k_parts(M, N, K, act);
+    check_rc(rt_few_rows(x.data_ptr(), x.stride(0), nullptr, 0, nullptr, nullptr, nullptr, w.data_ptr(), w.stride(0), b.data_ptr(),
+                         y.data_ptr(), N, (int)M, (int)N, (int)K, (int)act, 0.f, kp.n, kp.grp, cur_stream()),
+             "encoder: product");
+    return y;
   }
+  if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
+  const auto [split, bn] = token_split(M, N, K, act);
   if (split > 1) {
     auto slabs = at::empty({split * M * N}, x.options().dtype(at::kFloat));
     return gemm_splitk(x, w, split, slabs, b, act, std::nullopt, std::nullopt, bn, {});
@@ -1379,20 +1417,28 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
                               emb[2] ? emb[2]->data_ptr() : nullptr, emb[3]->data_ptr(), emb[4]->data_ptr(), x.data_ptr(), (int)M,
                               (int)H, (float)eps, st),
            "encoder: embedding");
-  if (M <= 64 && H % 32 == 0 && F % 32 == 0) {
+  const int64_t max_parts = M <= 16 ? 16 : 8;
+  if (M <= 64 && H % 64 == 0 && F % 64 == 0 && k_parts(M, 3 * H, H, 0).n <= max_parts && k_parts(M, H, H, 0).n <= max_parts &&
+      k_parts(M, F, H, 2).n <= max_parts && k_parts(M, H, F, 0).n <= max_parts) {
     // up to 32 rows the products normalise their input themselves (few_rows.hip): 5 launches a layer instead of 7
-    const bool own = M <= 32;
+    const bool own = M <= 32 && (M <= 16 || std::max(k_parts(M, 3 * H, H, 0).n, k_parts(M, F, H, 2).n) <= 4);
     Tensor qkv = rows(3 * H), f = rows(F), d = rows(H), z = rows(H);
     auto product = [&](const Tensor& in, const Tensor& w, const Tensor& b, int act, Tensor& y) {
+      if (M > 32 && w.size(1) > 2048) {  // 40 / 64 rows by 768 x 3072: 13.9 / 14.5 us, 15.6 / 18.5 as few rows
+        gemm(in, w, std::nullopt, std::nullopt, b, act, false, y, std::nullopt, 0.0, false, {});
+        return;
+      }
+      const KParts kp = k_parts(M, w.size(0), w.size(1), act);
       check_rc(rt_few_rows(in.data_ptr(), in.size(1), nullptr, 0, nullptr, nullptr, nullptr, w.data_ptr(), w.size(1), b.data_ptr(),
-                           y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)w.size(1), act, 0.f, st),
+                           y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)w.size(1), act, 0.f, kp.n, kp.grp, st),
                "encoder: product");
     };
     // y = act(LN(d + x) w^T + b); x becomes LN(d + x)
     auto norm_product = [&](const Tensor& lw, const Tensor& lb, const Tensor& w, const Tensor& b, int act, Tensor& y) {
       if (own) {
+        const KParts kp = k_parts(M, w.size(0), H, act);
         check_rc(rt_few_rows(d.data_ptr(), H, x.data_ptr(), H, lw.data_ptr(), lb.data_ptr(), z.data_ptr(), w.data_ptr(), H,
-                             b.data_ptr(), y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)H, act, (float)eps, st),
+                             b.data_ptr(), y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)H, act, (float)eps, kp.n, kp.grp, st),
                  "encoder: norm and product");
       } else {
         norm(d, x, lw, lb, z);
@@ -1643,7 +1689,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
         py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
         py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
-  m.def("few_rows", &few_rows, "act(x w^T + b) of at most 64 rows, x normalised first if asked", py::arg("x"), py::arg("w"),
+  m.def("few_rows", &few_rows, "act(x w^T + b) in groups of 64 rows, up to 32 rows normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);
   m.def("attn_fwd", &attn_fwd);

@@ -1,13 +1,17 @@
-// Products of few rows (M <= 64) with weights of an encoder's size, for gfx950: y = act(x W^T + bias), where x may still be
-// LN(d + res). One query through all-MiniLM-L6-v2 is 24 such products of about 15 rows, each a few hundred KB of weights: what
-// they take is launch, one trip to memory and the reduction over K, not bandwidth.
+// Products of few rows with weights of an encoder's size, for gfx950: y = act(x W^T + bias), where x may still be LN(d + res).
+// One query through all-MiniLM-L6-v2 is 24 such products of about 15 rows, each a few hundred KB of weights: what they take is
+// launch, one trip to memory and the reduction over K, not bandwidth.
 //
-// A workgroup is 8 waves over 16 (K >= 512) or 32 columns; 8 (4) waves split K, so that a wave has 3 to 6 steps of 32 and all of
-// its weight loads (MFMA fragments, 16 B a lane straight from the row-major weight) in flight at once. With a norm ahead every
-// workgroup normalises the rows itself, two or four to a wave, under those loads (12 KB from L2, where a kernel of its own costs
-// a launch and another trip); workgroup 0 also writes them. Partial sums meet in LDS. Bound by latency. 15 rows, us,
-// gemm_decode_kernel and the norm ahead -> this: 1152 x 384 6.1 + 2.9 -> 5.2, 1536 x 384 with GELU 6.3 + 2.9 -> 5.9,
-// 384 x 384 5.7 -> 4.4, 384 x 1536 11.3 -> 5.7.
+// K is summed in the parts, and the parts in the order, of the kernel that ops.gemm takes for the shape (see Args), so that the
+// bits are that kernel's: a text's embedding does not depend on the way it went. The 8 waves of a workgroup are parts x row tiles
+// x column groups of 16; a wave has most of its weight loads (MFMA fragments, 16 B a lane straight from the row-major weight) in
+// flight at once, and partial sums meet in LDS. With a norm ahead every workgroup normalises the rows itself, two or four to a
+// wave, under those loads (12 KB from L2, where a kernel of its own costs a launch and another trip); workgroup 0 also writes them.
+// Bound by latency. 15 rows, us,
+// gemm_decode_kernel -> this: 1152 x 384 5.2 -> 4.0, 1536 x 384 with GELU 5.8 -> 4.4, 384 x 1536 9.8 -> 5.2, and 2.9 of the norm
+// with it; 20 rows, gemm_m64_kernel or the wide one: 6.6 -> 4.9, 11.0 -> 5.3, 21.3 -> 7.1; 64 rows: 6.9 -> 7.9, 16.2 -> 8.3, 21.7 ->
+// 10.6. More rows go in groups of 64, a workgroup reading its 64 rows from L2 for 16 or 32 columns: ahead of the tile kernels
+// while that is a workgroup or two per CU (few_rows_pays in bindings.cpp).
 #include "rt_common.h"
 #include "rt_gelu.h"
 
@@ -22,24 +26,35 @@ struct Args {
   const bf16_t* w; long ldw; const bf16_t* bias;  // [N, K], [N] or null
   bf16_t* y; long ldy;
   int M, N, K, act;
+  int parts, grp;  // K parts of whole 64s, part i from i (K / 64) / parts on; summed in groups of grp, then the groups in order
+  int ks, rs;      // of the 8 waves: over parts, over row tiles (powers of two; the rest over column groups of 16)
   float eps;
 };
 
-// RT: row tiles of 16; NW: 16-B vectors of a row a lane normalises (0: no norm ahead)
-template <int RT, int NW>
-__global__ __launch_bounds__(512) void few_rows_kernel(Args p) {
+// RT: row tiles of 16 a wave; NW: 16-B vectors of a row a lane normalises (0: no norm ahead), of up to 16 TR rows
+template <int RT, int NW, int TR>
+__global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
   constexpr int LDX = NW * 512 + 8;  // K <= 512 NW; an odd number of 16-B chunks where K is a multiple of 16
-  __shared__ __attribute__((aligned(16))) bf16_t xs[NW ? RT * 16 * LDX : 8];
-  __shared__ f32x4 red[8][RT][64];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[NW ? TR * 16 * LDX : 8];
+  __shared__ f32x4 red[RT == 4 ? 32 : 16][64];  // [part][column group][row tile]
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
-  const int steps = p.K / 32, CG = steps >= 16 ? 1 : 2, KS = 8 / CG;
-  const int cg = wid / KS, ks = wid % KS;
+  const int nc = p.K / 64, CG = 8 / (p.ks * p.rs), RTS = p.rs * RT;  // column groups, row tiles of the workgroup
+  const int ks = wid % p.ks, rs = wid / p.ks % p.rs, cg = wid / (p.ks * p.rs);
   const int n0 = (blockIdx.x * CG + cg) * 16;
-  const int s0 = ks * steps / KS, s1 = n0 < p.N ? (ks + 1) * steps / KS : s0;
+  if constexpr (NW == 0) {  // 64 rows of more
+    const int r0 = blockIdx.y * 64;
+    p.x += (long)r0 * p.ldx;
+    p.y += (long)r0 * p.ldy;
+    p.M = min(p.M - r0, 64);
+  }
+  const bool on = n0 < p.N && rs * RT * 16 < p.M;
+  auto begin = [&](int part) { return 2 * (part * nc / p.parts); };  // in steps of 32
   const bf16_t* const wp = p.w + (long)min(n0 + r16, p.N - 1) * p.ldw + 8 * g;
-  constexpr int D = 6;  // weight fragments in flight
+  constexpr int D = RT == 1 ? 12 : RT == 2 ? 8 : 4;  // weight fragments in flight (without a norm in 128 registers)
   bf16x8 wf[D];
+  int s0 = 0, s1 = 0;
+  if (on && ks < p.parts) { s0 = begin(ks); s1 = begin(ks + 1); }
 #pragma unroll
   for (int k = 0; k < D; ++k)
     if (s0 + k < s1) wf[k] = *(const bf16x8*)(wp + (s0 + k) * 32);
@@ -47,7 +62,7 @@ __global__ __launch_bounds__(512) void few_rows_kernel(Args p) {
   if constexpr (NW > 0) {
     // rows of the norm: the arithmetic of norm_rows_kernel
     const int nv = p.K / 8;
-    constexpr int RW = RT * 2;  // rows of a wave
+    constexpr int RW = TR * 2;  // rows of a wave
     uint4 a[RW][NW], b[RW][NW];
 #pragma unroll
     for (int k = 0; k < RW; ++k)
@@ -120,39 +135,47 @@ __global__ __launch_bounds__(512) void few_rows_kernel(Args p) {
     }
     __syncthreads();
   }
-  f32x4 acc[RT];
+  for (int part = ks; part < p.parts; part += p.ks) {
+    if (part > ks && on) { s0 = begin(part); s1 = begin(part + 1); }
+    f32x4 acc[RT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int s = s0; s < s1; s += D) {
+    for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += D) {
+      if (s > s0 || part > ks) {
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-      if (s > s0 && s + k < s1) wf[k] = *(const bf16x8*)(wp + (s + k) * 32);
+        for (int k = 0; k < D; ++k)
+          if (s + k < s1) wf[k] = *(const bf16x8*)(wp + (s + k) * 32);
+      }
+      bf16x8 xf[D][RT];
+#pragma unroll
+      for (int k = 0; k < D; ++k)
+        if (s + k < s1)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            const int row = 16 * (rs * RT + t) + r16, col = (s + k) * 32 + 8 * g;
+            if constexpr (NW > 0) xf[k][t] = *(const bf16x8*)(xs + row * LDX + col);
+            else xf[k][t] = *(const bf16x8*)(p.x + (long)min(row, p.M - 1) * p.ldx + col);
+          }
+#pragma unroll
+      for (int k = 0; k < D; ++k)
+        if (s + k < s1)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k], xf[k][t], acc[t], 0, 0, 0);
     }
-    bf16x8 xf[D][RT];
+    // acc[t][e]: row 16 (rs RT + t) + r16, column n0 + 4 g + e
 #pragma unroll
-    for (int k = 0; k < D; ++k)
-      if (s + k < s1)
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          const int row = 16 * t + r16, col = (s + k) * 32 + 8 * g;
-          if constexpr (NW > 0) xf[k][t] = *(const bf16x8*)(xs + row * LDX + col);
-          else xf[k][t] = *(const bf16x8*)(p.x + (long)min(row, p.M - 1) * p.ldx + col);
-        }
-#pragma unroll
-    for (int k = 0; k < D; ++k)
-      if (s + k < s1)
-#pragma unroll
-        for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k], xf[k][t], acc[t], 0, 0, 0);
+    for (int t = 0; t < RT; ++t) red[(part * CG + cg) * RTS + rs * RT + t][lane] = acc[t];
   }
-  // acc[t][e]: row 16 t + r16, column n0 + 4 g + e
-#pragma unroll
-  for (int t = 0; t < RT; ++t) red[wid][t][lane] = acc[t];
   __syncthreads();
-  for (int o = wid; o < CG * RT; o += 8) {
-    const int c = o / RT, t = o % RT, row = 16 * t + r16, col = (blockIdx.x * CG + c) * 16 + 4 * g;
+  for (int o = wid; o < CG * RTS; o += 8) {
+    const int t = o % RTS, row = 16 * t + r16, col = (blockIdx.x * CG + o / RTS) * 16 + 4 * g;
     if (row >= p.M || col >= p.N) continue;
-    f32x4 v = red[c * KS][t][lane];
-    for (int k = 1; k < KS; ++k) v += red[c * KS + k][t][lane];
+    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < p.parts; b += p.grp) {
+      f32x4 u = red[b * CG * RTS + o][lane];
+      for (int k = 1; k < p.grp; ++k) u += red[(b + k) * CG * RTS + o][lane];
+      v = p.parts == p.grp ? u : v + u;
+    }
     if (p.bias) {
       const uint2 b = *(const uint2*)(p.bias + col);
       v += f32x4{__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u)};
@@ -234,31 +257,31 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
 using namespace rt;
 
 // y = act(x w^T + bias), or act(LN(x + res) w^T + bias) with LN(x + res) to xo (lw given; M <= 32, K <= 1024); act 0 or 2
-// (GELU). M <= 64, N % 16 == 0, K % 32 == 0; operands 16-B aligned, leading dimensions multiples of 8. -1: not for this kernel.
+// (GELU). N % 16 == 0, K % 64 == 0; operands 16-B aligned, leading dimensions multiples of 8; up to 8 parts, up to 16 rows 16,
+// a multiple of grp. -1: not for this kernel.
 extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, const void* lw, const void* lb, void* xo, const void* w,
-                           long ldw, const void* bias, void* y, long ldy, int M, int N, int K, int act, float eps, hipStream_t stream) {
+                           long ldw, const void* bias, void* y, long ldy, int M, int N, int K, int act, float eps, int parts, int grp,
+                           hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || N % 16 || K < 32 || K % 32 || (act != 0 && act != 2) || (lw && (M > 32 || K > 1024 || !lb || !res || !xo))) return -1;
+  if (M > 65535 * 64 || N % 16 || K < 64 || K % 64 || (act != 0 && act != 2) || (lw && (M > 32 || K > 1024 || !lb || !res || !xo))) return -1;
+  if (parts < 1 || parts > (M <= 16 ? 16 : 8) || grp < 1 || parts % grp) return -1;
   fr::Args p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.res = (const bf16_t*)res; p.ldr = ldr;
   p.lw = (const bf16_t*)lw; p.lb = (const bf16_t*)lb; p.xo = (bf16_t*)xo;
   p.w = (const bf16_t*)w; p.ldw = ldw; p.bias = (const bf16_t*)bias; p.y = (bf16_t*)y; p.ldy = ldy;
-  p.M = M; p.N = N; p.K = K; p.act = act; p.eps = eps;
-  const int cols = K / 32 >= 16 ? 16 : 32;
-  const dim3 grid((N + cols - 1) / cols), block(512);
-  const int rt = (M + 15) / 16, nw = lw ? (K <= 512 ? 1 : 2) : 0;
-#define FR(R, W) hipLaunchKernelGGL((fr::few_rows_kernel<R, W>), grid, block, 0, stream, p)
-  switch (rt * 4 + nw) {
-    case 4: FR(1, 0); break;
-    case 5: FR(1, 1); break;
-    case 6: FR(1, 2); break;
-    case 8: FR(2, 0); break;
-    case 9: FR(2, 1); break;
-    case 10: FR(2, 2); break;
-    case 12: FR(3, 0); break;
-    case 16: FR(4, 0); break;
-    default: return -1;
-  }
+  p.M = M; p.N = N; p.K = K; p.act = act; p.eps = eps; p.parts = parts; p.grp = grp;
+  const int tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  p.ks = parts > 4 ? 8 : parts > 2 ? 4 : parts;
+  p.rs = std::min(tiles > 1 ? 4 : 1, 8 / p.ks);  // 17..32 rows in one part: rather idle waves than half the workgroups
+  const int rt = std::max(tiles / p.rs, 1), cols = 16 * (8 / (p.ks * p.rs)), nw = lw ? (K <= 512 ? 1 : 2) : 0;
+  if (nw && rt != 1) return -1;
+  const dim3 grid((N + cols - 1) / cols, (M + 63) / 64), block(512);
+#define FR(R, W, T) hipLaunchKernelGGL((fr::few_rows_kernel<R, W, T>), grid, block, 0, stream, p)
+  if (nw == 1) { if (tiles == 1) FR(1, 1, 1); else FR(1, 1, 2); }
+  else if (nw == 2) { if (tiles == 1) FR(1, 2, 1); else FR(1, 2, 2); }
+  else if (rt == 1) FR(1, 0, 0);
+  else if (rt == 2) FR(2, 0, 0);
+  else FR(4, 0, 0);
 #undef FR
   RT_LAUNCH_CHECK();
   return 0;

@@ -1689,6 +1689,18 @@ extern "C" int rt_gemm_nt_glu(const void* A, long lda, const void* B, long ldb, 
   return 0;
 }
 
+// In how many parts rt_gemm_nt sums K for plain row-major operands of K % 64 == 0 (part i from i (K / 64) / parts on), and in
+// groups of how many: the sums of the groups are added in order
+extern "C" int rt_gemm_nt_parts(int M, int N, int K, int* grp) {
+  *grp = 1;
+  if (M > 16) {
+    if (tuning().m64_wide && N % 256 == 0 && N <= 16384) return std::min(fit_split(wide_split(N, K), N / 256, WD_SLAB), std::max(1, K / 64));
+    return fit_split(m64_split(N, K), (N + 63) / 64, 64 * 64 + 64);
+  }
+  *grp = 4;  // the waves of a workgroup
+  return 4 * fit_split(decode_split(N, K), (N + DG_COLS - 1) / DG_COLS, 16 * (DG_COLS + 1));
+}
+
 extern "C" int rt_gemm_nt(const void* A, long lda, const void* B, long ldb, const void* U, long ldu,
                           const void* UB, long ldub, int Rp, const void* bias, void* C, long ldc, int M,
                           int N, int K, int act, int out_f32, float* slabs, unsigned* tickets,
