@@ -33,6 +33,13 @@ __device__ __forceinline__ bf16x8 cat4(const rt_s16x4& lo, const rt_s16x4& hi) {
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// 16 B a lane from base (uniform) + off bytes to LDS at dst + 16 lane. A buffer instruction: behind global_load_lds, a FLAT one,
+// hipcc waits for every LDS read at once instead of counting them
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, void* dst) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)dst, 16, off, 0, 0, 0);
+}
+
 struct Seg { int row, q_off, q_len, kv_off, kv_len, pos0, pad0, pad1; };  // 8 ints
 
 // LDS image of a K (V) tile: rows of DQ (DV) elements, 16-B chunk c of row r at slot c ^ swizzle(r) (an

@@ -2,6 +2,7 @@
 plain implementation (pafolorn_oracle.py): whole prompts, portions, decoding, mixed batches with reused pages
 and state slots, far keys and far memories, greedy generation through the captured decode step and the scheduler."""
 import json
+import math
 import os
 import subprocess
 import sys
@@ -135,6 +136,40 @@ def test_window_attention(dtype, H, G, D, V, rot, size, keep, cap):
     assert float(e.max()) < (2e-5 if dtype == torch.float32 else 4e-2), int(e.argmax())
     assert rel(out[:, :H * V], want) < (1e-5 if dtype == torch.float32 else 1.2e-2)
     assert float(out[:, H * V:].abs().max()) == 0
+
+
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 72), (200, 64)])
+@pytest.mark.parametrize("cap", [2.0, 50.0, 55.4, 55.5, 300.0, 0.0])
+def test_window_prefill_capped_scores(cap, D, V):
+    """The prompt kernel with and without a running maximum: tiles of scores all near zero, some beyond where tanh is a
+    polynomial, rows with every score at one end of the cap; more than 64 tiles of keys."""
+    g = torch.Generator().manual_seed(int(cap) + D)
+    T, H, G = 4300, 4, 2
+    d = ops.WindowDims(H, G, D, V, D ** -0.5, cap, 0, 0)
+    u = torch.randn(1, 1, D, generator=g).sign()
+    q, k, v = torch.randn(T, H, D, generator=g), torch.randn(T, G, D, generator=g) + u, torch.randn(T, G, V, generator=g)
+    q *= (2.0 ** torch.linspace(-4, 5 if cap else 3, T))[torch.randperm(T, generator=g)][:, None, None]
+    q[T // 2:T // 2 + 64] *= 0.01       # whole waves of small scores
+    q[5::97], q[6::97] = 60 * u, -60 * u
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    cache = PagedCache([d.cache_width], 1, T, T + 64, DEV, torch.bfloat16)
+    cache.reserve(0, T)
+    cache.sync()
+    cos, sin = torch.ones(cache.max_seq, D // 2, device=DEV), torch.zeros(cache.max_seq, D // 2, device=DEV)  # no rotation
+    out = torch.zeros(T, H * V, dtype=torch.bfloat16, device=DEV)
+    proj = torch.cat([q.flatten(1), k.flatten(1), v.flatten(1)], 1).to(DEV)
+    ops.window_attention(proj, 0, d, None, None, 1e-6, cos, sin, RaggedBatch.build([(0, [0] * T, 0)], DEV), cache.pool(0),
+                         cache.table, out)
+    rows = torch.cat([torch.arange(0, T, 13), torch.arange(5, T, 97), torch.arange(6, T, 97), torch.arange(T // 2, T // 2 + 64)]).to(DEV)
+    see = torch.arange(T, device=DEV)[None, :] <= rows[:, None]
+    for h in range(H):
+        kd, vd = (t[:, h // 2].to(DEV).double() for t in (k, v))
+        s = q[:, h].to(DEV).double()[rows] @ kd.t() * d.scale
+        s = cap * torch.tanh(s / cap) if cap else s
+        p = torch.softmax(s.masked_fill(~see, -math.inf), -1)
+        want, size = p @ vd, p @ vd.abs()
+        # p and the result round to bf16 (half an ulp: 2^-8 each), scores up to some hundreds carry fp32 sums of D terms
+        assert (((out[rows, h * V:(h + 1) * V].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
