@@ -50,6 +50,25 @@ __device__ __forceinline__ void stf(float* p, const float* o) { ldf<N>(o, p); }
 
 __device__ __forceinline__ float sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + expf(-x)); }
 __device__ __forceinline__ float softplus(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
+// softplus(x) log2(e), to about 2 ulp, infinities and NaN as ever: log1p(y) = 2 artanh(y / (2 + y)) by its series for
+// y = exp(-|x|), at most 1
+__device__ __forceinline__ float softplus_log2(float x) {
+  constexpr float LOG2E = 1.44269502f, LOG2E_LO = 1.92596299e-8f;
+  const float ax = fabsf(x), h = -ax * LOG2E;
+  const float lo = ax < 200.f ? fmaf(-ax, LOG2E_LO, fmaf(-ax, LOG2E, -h)) : 0.f;  // what h has lost
+  float y = __builtin_amdgcn_exp2f(h);
+  y = fmaf(y, lo * 0.693147181f, y);
+  const float q = __builtin_amdgcn_rcpf(2.f + y);
+  float s = y * q;
+  s = fmaf(fmaf(-s, 2.f + y, y), q, s);
+  const float z = s * s;
+  float p = fmaf(z, 1.f / 13.f, 1.f / 11.f);
+  p = fmaf(z, p, 1.f / 9.f);
+  p = fmaf(z, p, 1.f / 7.f);
+  p = fmaf(z, p, 1.f / 5.f);
+  p = fmaf(z, p, 1.f / 3.f);
+  return fmaf(2.f * s, fmaf(z, p, 1.f), fmaxf(x, 0.f)) * LOG2E;
+}
 __device__ __forceinline__ float gate_of(float z, bool silu) { return (silu ? z : 1.f) * sigmoid(z); }
 
 struct Args {
@@ -349,7 +368,9 @@ __device__ __forceinline__ void conv4(const Conv<T>& cv, int p, int n, int c, fl
     for (int e = 0; e < N; ++e) y[i][e] = i < n ? y[i][e] * sigmoid(y[i][e]) : 0.f;
 }
 
-// workgroup = (head, chunk); CHN: a decay per key channel, else per head. N: elements per access
+// workgroup = (head, chunk); CHN: a decay per key channel, else per head. N: elements per access. With decays per channel
+// bound by the VALU (95 % of its cycles), which is why the summed log decays G are to base 2: their exponentials, six a token
+// and channel, are single instructions. 7400 tokens, 32 heads of 128: 420 -> 336 us, a decay per head (16): 140 -> 137.
 template <typename T, int DP, bool CHN, int N, int TAPS>
 __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
   constexpr int LD = DP + 4, R = DP / 16;
@@ -371,7 +392,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
     const T* bp = (const T*)a.b + (long)(t0 + tid) * a.ldb + h;
     beta[tid] = tid < n ? sigmoid(ld(bp)) : 0.f;
     if constexpr (!CHN) {  // summed log decays
-      float g = tid < n ? -A * softplus(ld((const T*)a.a + (long)(t0 + tid) * a.lda + h) + a.dt[h]) : 0.f;
+      float g = tid < n ? -A * softplus_log2(ld((const T*)a.a + (long)(t0 + tid) * a.lda + h) + a.dt[h]) : 0.f;
 #pragma unroll
       for (int o = 1; o < CH; o *= 2) {
         const float up = __shfl_up(g, o, CH);
@@ -413,7 +434,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
       if (i < n) {
         ldn<T, N>((const T*)a.a + (long)(t0 + i) * a.lda + (long)h * D + d, v);
 #pragma unroll
-        for (int k = 0; k < N; ++k) v[k] = -A * softplus(v[k] + a.dt[(long)h * D + d + k]);
+        for (int k = 0; k < N; ++k) v[k] = -A * softplus_log2(v[k] + a.dt[(long)h * D + d + k]);
       }
       stf<N>(&G[i][d], v);
     }
@@ -467,7 +488,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
       const f32x4 g4 = *(const f32x4*)&G[m][d], v4 = *(const f32x4*)&G[piv][d];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float e = expf(-fabsf(g4[i] - v4[i]));
+        const float e = __builtin_amdgcn_exp2f(-fabsf(g4[i] - v4[i]));
         const float x = k4[i] * e, y = q4[i] * e;
         ka = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, ka, 0, 0, 0);
         pa = __builtin_amdgcn_mfma_f32_16x16x4f32(y, x, pa, 0, 0, 0);
@@ -505,7 +526,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * g + i;
-        const float e = expf(fminf(Gs[r] - Gs[m], 0.f));
+        const float e = __builtin_amdgcn_exp2f(fminf(Gs[r] - Gs[m], 0.f));
         As[r][m] = r > m ? beta[r] * ka[i] * e : 0.f;
         Ps[r][m] = pa[i] * e;
       }
@@ -539,7 +560,7 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
     const f32x4 k4 = *(const f32x4*)&kx[em][d], q4 = *(const f32x4*)&qx[em][d];
     f32x4 ex;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ex[j] = (CHN || j == 0) ? expf(gl(em, d + j)) : ex[0];
+    for (int j = 0; j < 4; ++j) ex[j] = (CHN || j == 0) ? __builtin_amdgcn_exp2f(gl(em, d + j)) : ex[0];
     *(f32x4*)(ws + L::KT + 4 * e) = k4 * ex;
     *(f32x4*)(ws + L::QT + 4 * e) = q4 * ex;
   }
@@ -547,32 +568,40 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
     const int d = 16 * (e >> 6) + (e & 15), i = 4 * (e >> 4 & 3);  // channel d, tokens i .. i + 3
     f32x4 y;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) y[j] = kx[i + j][d] * expf(gl(CH - 1, d) - gl(i + j, d));
+    for (int j = 0; j < 4; ++j) y[j] = kx[i + j][d] * __builtin_amdgcn_exp2f(gl(CH - 1, d) - gl(i + j, d));
     *(f32x4*)(ws + L::KE + 4 * e) = y;
   }
-  for (int d = tw; d < DP; d += 192) ws[L::EG + d] = expf(gl(CH - 1, d));
+  for (int d = tw; d < DP; d += 192) ws[L::EG + d] = __builtin_amdgcn_exp2f(gl(CH - 1, d));
 }
 
 // Workgroup = (run, head, 16 value columns); NW waves hold RW 16-row tiles of the state's columns each, as MFMA
 // accumulators (row 16 r + 4 g + i, column lane % 16), which are at once the B operands of the products with S0
-// (k index of step (r, i): row 16 r + 4 g + i for lane group g). The waves' shares of those products meet in LDS,
-// one barrier per chunk; every wave solves for U by itself, and one more finishes the read-outs off the chain from
-// chunk to chunk. Operands go straight to registers, two chunks ahead.
+// (k index of step (r, i): row 16 r + 4 g + i for lane group g). The waves' shares of k e^G S0 meet in LDS, one barrier
+// per chunk; every wave solves for U by itself, and one more finishes the read-outs off the chain from chunk to chunk.
+// Operands go straight to registers, two chunks ahead. Bound by that chain (54 % of its cycles have a matrix instruction
+// on a SIMD): so the products q e^G S0 run while the shares are on their way back from LDS, their own shares meet behind the
+// next barrier, and the loads are buffer loads whose offsets never change. 2 runs of 3700 tokens, 16 heads of 128 x 128
+// (a workgroup per CU): 308 -> 224 us, 32 heads: 441 -> 357.
 // Values stay the 32-bit words they were loaded as until they are used (anything done at the load waits for it); a
 // lane's bf16 value is the word's upper half if `odd`
 template <typename T> __device__ __forceinline__ float of_word(uint32_t r, bool odd) {
   return __uint_as_float(sizeof(T) == 4 || odd ? (sizeof(T) == 4 ? r : r & 0xffff0000u) : r << 16);
 }
 template <int RW> struct ScanOps { f32x4 k[RW], q[RW], e[RW], g[RW], t; uint32_t v[4]; };
-// uniform base, the lane's byte offset
-template <typename V> __device__ __forceinline__ V at(const void* base, uint32_t off) { return *(const V*)((const char*)base + off); }
 struct ReadOps { f32x4 t, p; uint32_t v[4]; };
+// Loads with a uniform base and the lane's own byte offset, which stays the same from chunk to chunk; beyond `bytes` they give 0
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes = 0xffffffffu) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ f32x4 at4(__amdgpu_buffer_rsrc_t r, uint32_t off, int base) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, base, 0));
+}
 
 template <typename T, int DP>
 __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) void delta_scan_kernel(Args a, Work w, const int* first_chunk) {
   constexpr int R = DP / 16, NW = R < 4 ? R : 4, RW = R / NW;
   using L = Lay<DP>;
-  __shared__ f32x4 part[2][NW][2][64];
+  __shared__ f32x4 part[2][NW][64], part_o[2][NW][64];  // the waves' shares of k e^G S0 and of q e^G S0
   const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int VB = (a.V + 15) / 16, lin = xcd_remap(blockIdx.x, gridDim.x);
@@ -582,71 +611,85 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
   const int col = vb * 16 + m, d0 = 16 * RW * wid;
   const bool ok = col < a.V, live = run.x >= 0 && run.x < a.n_rows;
   float* Sp = a.S + ((long)max(run.x, 0) * a.H + h) * a.D * a.V + (ok ? col : 0);
-  const long ldo = (long)a.H * a.V, vc = (long)h * a.V + (ok ? col : 0);
+  const uint32_t ldo = (uint32_t)(a.H * a.V);
+  const long vc = (long)h * a.V + (ok ? col : 0);
   constexpr int PER = 4 / sizeof(T);  // values per word
   const uint32_t* vp = (const uint32_t*)w.v + (long)run.y * w.ldv / PER;
   const uint32_t ldw = (uint32_t)(w.ldv / PER), vw = (uint32_t)(vc / PER);
   const bool odd = vc & 1;
-  float* op = w.o + (long)run.y * ldo;
   const float* wp = w.ws + ((long)h * w.n_chunks + c0) * L::N;
   const uint32_t o_m = 16 * lane, o_s = 16 * (RW * wid * 64 + lane), o_g = 4 * (d0 + 4 * g);  // the wave's row tiles
-  auto load_kq = [&](ScanOps<RW>& s, int c) {
-    const float* p = wp + (long)min(c, nc - 1) * L::N;
+  auto rows = [&](int c) { return (uint32_t)min(CH, run.z - c * CH); };  // c < nc
+  auto load_k = [&](ScanOps<RW>& s, int c) {
+    const auto p = rsrc(wp + (long)min(c, nc - 1) * L::N);
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      s.k[r] = at<f32x4>(p + L::KT + 256 * r, o_s);
-      s.q[r] = at<f32x4>(p + L::QT + 256 * r, o_s);
-    }
+    for (int r = 0; r < RW; ++r) s.k[r] = at4(p, o_s, 4 * L::KT + 1024 * r);
   };
-  auto load_tv = [&](auto& s, int c) {  // c < nc
-    const uint32_t* p = vp + (long)c * CH * ldw;
-    const int last = run.z - 1 - c * CH;
+  auto load_q = [&](ScanOps<RW>& s, int c) {
+    const auto p = rsrc(wp + (long)min(c, nc - 1) * L::N);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)  // past the run: beta is 0
-      s.v[i] = at<uint32_t>(p, 4 * (__umul24((uint32_t)min(4 * g + i, last), ldw) + vw));
-    s.t = at<f32x4>(wp + (long)c * L::N + L::T, o_m);
+    for (int r = 0; r < RW; ++r) s.q[r] = at4(p, o_s, 4 * L::QT + 1024 * r);
+  };
+  uint32_t o_v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o_v[i] = 4 * ((uint32_t)(4 * g + i) * ldw + vw);
+  auto load_tv = [&](auto& s, int c) {  // c < nc. Rows past the run: 0 (and beta is 0)
+    const auto p = rsrc(vp + (long)c * CH * ldw, 4 * rows(c) * ldw);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s.v[i] = __builtin_amdgcn_raw_buffer_load_b32(p, o_v[i], 0, 0);
+    s.t = at4(rsrc(wp + (long)c * L::N), o_m, 4 * L::T);
   };
   auto load_rest = [&](ScanOps<RW>& s, int c) {
     c = min(c, nc - 1);
     load_tv(s, c);
-    const float* p = wp + (long)c * L::N;
+    const auto p = rsrc(wp + (long)c * L::N);
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
-      s.e[r] = at<f32x4>(p + L::KE + 256 * r, o_s);
-      s.g[r] = at<f32x4>(p + L::EG + 16 * r, o_g);
+      s.e[r] = at4(p, o_s, 4 * L::KE + 1024 * r);
+      s.g[r] = at4(p, o_g, 4 * L::EG + 64 * r);
     }
   };
-  // U from the shares of k e^G S0 in buffer b
-  auto solve = [&](auto& s, int b) {
+  auto value = [&](auto& s) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(s.v[i]));  // nothing of this chunk is used ahead of its barrier
-    f32x4 wv = {of_word<T>(s.v[0], odd), of_word<T>(s.v[1], odd), of_word<T>(s.v[2], odd), of_word<T>(s.v[3], odd)}, u = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(s.v[i]));  // not ahead of its chunk
+    return f32x4{of_word<T>(s.v[0], odd), of_word<T>(s.v[1], odd), of_word<T>(s.v[2], odd), of_word<T>(s.v[3], odd)};
+  };
+  auto solve = [&](const f32x4& t, const f32x4& wv) {
+    f32x4 u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < NW; ++j) wv -= part[b][j][0][lane];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(s.t[i], wv[i], u, 0, 0, 0);
+    for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(t[i], wv[i], u, 0, 0, 0);
     return u;
   };
-  if (wid == NW) {  // read-outs
+  if (wid == NW) {  // read-outs: P U of a chunk, and behind the next barrier the shares of q e^G S0
     ReadOps r0, r1;
+    f32x4 oo = {0.f, 0.f, 0.f, 0.f};
     auto load = [&](ReadOps& s, int c) {
       c = min(c, nc - 1);
       load_tv(s, c);
-      s.p = at<f32x4>(wp + (long)c * L::N + L::P, o_m);
+      s.p = at4(rsrc(wp + (long)c * L::N), o_m, 4 * L::P);
+    };
+    float* op = w.o + (long)run.y * ldo;
+    uint32_t o_o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o_o[i] = ok ? 4 * ((uint32_t)(4 * g + i) * ldo + (uint32_t)vc) : 0x7ffffff0u;
+    auto finish = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < NW; ++j) oo += part_o[c & 1][j][lane];
+      const auto p = rsrc(op + (long)c * CH * ldo, 4 * rows(c) * ldo);  // rows past the run and columns past V: not stored
+#pragma unroll
+      for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(oo[i]), p, o_o[i], 0, 0);
     };
     auto read = [&](ReadOps& s, int c) {
-      const int b = c & 1;
       asm volatile("s_barrier" ::: "memory");
-      const f32x4 u = solve(s, b);
-      f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+      if (c > 0) finish(c - 1);
+      f32x4 wv = value(s);
 #pragma unroll
-      for (int j = 0; j < NW; ++j) oo += part[b][j][1][lane];
+      for (int j = 0; j < NW; ++j) wv -= part[c & 1][j][lane];
+      const f32x4 u = solve(s.t, wv);
+      oo = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i) oo = __builtin_amdgcn_mfma_f32_16x16x4f32(s.p[i], u[i], oo, 0, 0, 0);
-      float* oc = op + (long)c * CH * ldo;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (ok && 4 * g + i < run.z - c * CH) *(float*)((char*)oc + 4 * (__umul24((uint32_t)(4 * g + i), (uint32_t)ldo) + (uint32_t)vc)) = oo[i];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the shares have been read
       load(s, c + 2);
     };
     load(r0, 0);
@@ -658,8 +701,11 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
       read(r1, c + 1);
     }
     if (c < nc) read(r0, c);
+    asm volatile("s_barrier" ::: "memory");
+    if (nc > 0) finish(nc - 1);
     return;
   }
+  __builtin_amdgcn_s_setprio(3);  // ahead of the wave of the read-outs, which nothing waits for
   f32x4 S[RW];
   auto chunk = [&](ScanOps<RW>& s, int c) {
     f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -667,18 +713,30 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
     for (int r = 0; r < RW; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.k[r][i], S[r][i], x[i & 1], 0, 0, 0);
+    load_k(s, c + 2);
+    f32x4 wv = value(s);
+    const int b = c & 1;
+    __builtin_amdgcn_sched_barrier(0);
+    part[b][wid][lane] = x[0] + x[1];
+    // the shares are whole; this buffer is written again only behind the next chunk's barrier. Global loads stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 sh[NW];
+#pragma unroll
+    for (int j = 0; j < NW; ++j) sh[j] = part[b][j][lane];
+    __builtin_amdgcn_sched_barrier(0);
+    // while the shares come: the read-outs' products, which nothing of this chunk waits for
 #pragma unroll
     for (int r = 0; r < RW; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.q[r][i], S[r][i], o[i & 1], 0, 0, 0);
-    load_kq(s, c + 2);
-    const int b = c & 1;
-    part[b][wid][0][lane] = x[0] + x[1];
-    part[b][wid][1][lane] = o[0] + o[1];
-    // the shares are whole; this buffer is written again only behind the next chunk's barrier. Global loads stay in flight
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
-    const f32x4 u = solve(s, b);
+    __builtin_amdgcn_sched_barrier(0);
+    load_q(s, c + 2);
+#pragma unroll
+    for (int j = 0; j < NW; ++j) wv -= sh[j];
+    const f32x4 u = solve(s.t, wv);
+    part_o[b][wid][lane] = o[0] + o[1];
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
       asm volatile("" : "+v"(s.g[r]));
@@ -691,8 +749,12 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
     load_rest(s, c + 2);
   };
   ScanOps<RW> s0, s1;
-  load_kq(s0, 0);
-  load_rest(s0, 0);
+  auto load_all = [&](ScanOps<RW>& s, int c) {
+    load_k(s, c);
+    load_q(s, c);
+    load_rest(s, c);
+  };
+  load_all(s0, 0);
 #pragma unroll
   for (int r = 0; r < RW; ++r)
 #pragma unroll
@@ -700,8 +762,7 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
       const int d = d0 + 16 * r + 4 * g + i;
       S[r][i] = live && run.w > 0 && ok && d < a.D ? Sp[(long)d * a.V] : 0.f;
     }
-  load_kq(s1, 1);
-  load_rest(s1, 1);
+  load_all(s1, 1);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the waits in the loop then count from the loop's own order of loads
   int c = 0;
   for (; c + 1 < nc; c += 2) {
@@ -709,6 +770,8 @@ __global__ __launch_bounds__(DP / 16 < 4 ? DP * 4 + 64 : 320, DP > 128 ? 2 : 4) 
     chunk(s1, c + 1);
   }
   if (c < nc) chunk(s0, c);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last shares of the read-outs
+  asm volatile("s_barrier" ::: "memory");
   if (live && ok) {
 #pragma unroll
     for (int r = 0; r < RW; ++r)
