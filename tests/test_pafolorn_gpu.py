@@ -172,6 +172,39 @@ def test_window_prefill_capped_scores(cap, D, V):
         assert (((out[rows, h * V:(h + 1) * V].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6)
 
 
+@pytest.mark.parametrize("T,parts", [(1, 7), (31, 4), (32, 4), (128, 4), (170, 3), (300, 1)])
+@pytest.mark.parametrize("heads", [32, 72])  # one and two tiles of query heads
+def test_window_decode_partitions(T, parts, heads):
+    """single tokens of rows of 1 to 400 keys, some with fewer tiles of keys than partitions"""
+    G, D, V, most = 8 if heads == 32 else 4, 64, 64, 400
+    d = ops.WindowDims(heads, G, D, V, D ** -0.5, 0.0, 0, 0)
+    assert ops.window._np_parts(T * 8 // G, d, most) == parts
+    T = T * 8 // G
+    g = torch.Generator().manual_seed(T)
+    n = torch.randint(1, most + 1, (T,), generator=g)
+    n[0], n[-1] = 1, most
+    cache = PagedCache([d.cache_width], T, most, T * (most + 63) // 64 * 64 + 64 * T, DEV, torch.bfloat16)
+    for b in range(T):
+        cache.reserve(b, int(n[b]))
+    cache.sync()
+    pool = cache.pool(0)
+    pool.normal_()
+    proj = torch.randn(T, heads * D + G * (D + V), generator=g).bfloat16().to(DEV)
+    cos, sin = torch.ones(cache.max_seq, D // 2, device=DEV), torch.zeros(cache.max_seq, D // 2, device=DEV)
+    out = torch.zeros(T, heads * V, dtype=torch.bfloat16, device=DEV)
+    pos = (n - 1).int().to(DEV)
+    batch = RaggedBatch.single(torch.zeros(T, dtype=torch.long, device=DEV), torch.arange(T, dtype=torch.int32, device=DEV), pos, most)
+    ops.window_attention(proj, 0, d, None, None, 1e-6, cos, sin, batch, pool, cache.table, out)
+    for b in range(T):
+        kv = pool.view(-1, G, 64, D + V)[cache.table[b].long()[:(int(n[b]) + 63) // 64]].transpose(1, 2).flatten(0, 1)[:int(n[b])].double()
+        kv = kv.repeat_interleave(heads // G, 1)
+        p = torch.softmax(torch.einsum("hd,khd->hk", proj[b, :heads * D].view(heads, D).double(), kv[..., :D]) * d.scale, -1)
+        v = kv[..., D:].transpose(0, 1)
+        want, size = ((p[:, None] @ t)[:, 0].flatten() for t in (v, v.abs()))
+        # p and the result round to bf16 (half an ulp: 2^-8 each)
+        assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, b
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ch", [True, False])
 @pytest.mark.parametrize("H,K,D,V,taps", [(4, 2, 32, 64, 4), (6, 3, 9, 11, 3), (3, 1, 128, 128, 2), (2, 2, 200, 72, 4), (2, 1, 64, 256, 1),
