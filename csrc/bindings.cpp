@@ -140,6 +140,7 @@ static const TuningField kTuningFields[] = {
     {"m64_wide", &rt::Tuning::m64_wide, nullptr},
     {"gemm_bn128_cost", nullptr, &rt::Tuning::gemm_bn128_cost},
     {"gemm_duo", &rt::Tuning::gemm_duo, nullptr},
+    {"gemm_mid", &rt::Tuning::gemm_mid, nullptr},
     {"gemm_group_m", &rt::Tuning::gemm_group_m, nullptr},
     {"sample_window", &rt::Tuning::sample_window, nullptr},
     {"sample_fast64", &rt::Tuning::sample_fast64, nullptr},
@@ -1278,9 +1279,16 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   return out;
 }
 
+// ops.linear's small_tiles (products with a bias)
+static bool small_tiles(int64_t M, int64_t N, int64_t K, int64_t act) {
+  if (M <= 64 || K % 64 || K > 3072 || (act != 0 && act != 2)) return false;
+  const int64_t rounds = ((M + 63) / 64 * ((N + 63) / 64) + 255) / 256;
+  return 2.6 + rounds * (0.19 * (K / 64) + (act ? 1.7 : 0.4)) < (K > 2048 ? 17 : 14);
+}
+
 // The K split of ops.gemm's token-parallel products (splitk_plan there): parts and the columns of a tile
 static std::pair<int64_t, int64_t> token_split(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (M > 512) return {1, 0};
+  if (M > 512 || small_tiles(M, N, K, act)) return {1, 0};
   const int64_t bn = act == 0 ? 128 : 256, tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
   const int64_t split = tiles < 128 && N % 16 == 0 ? std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles)) : 1;
   return {split, split == 1 && act ? 0 : bn};
@@ -1303,6 +1311,7 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
   }
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(w.size(1) == K, "few_rows: K mismatch");
+  TORCH_CHECK(M <= 64, "few_rows: up to 64 rows");
   auto vec = [&](const optional<Tensor>& t, int64_t n) {
     if (!t) return;
     CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ALIGN16(*t);
@@ -1326,33 +1335,9 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
   return {y, xo};
 }
 
-// Whether few_rows_kernel takes x w^T of M > 64 rows sooner than the tile kernels: it works in rounds of a workgroup per CU, each
-// 0.45 us per 32 k of a wave's part, 0.6 and 0.9 where a wave has two and four row tiles, behind 2.5 us; a lone 256 x 128 tile takes
-// 0.77 us per 64 k and 4, its GELU 9 more, and up to 512 rows the K split bounds that by 14 (K up to 2048) or 17. us, few_rows /
-// tiles: 400 x 1152 x 384 8.2 / 9.7, 400 x 384 x 1536 10.8 / 16.4, 640 x 384 x 1536 (one part) 23.6 / 22.7, 640 x 1536 x 384 with
-// GELU 14.2 / 18.8, 1500 x 768 x 768 34.5 / 14.3.
-static bool few_rows_pays(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (N % 16 || K % 64 || k_parts(M, N, K, act).n > 8) return false;
-  // parts of K, the waves over them, a wave's row tiles and the columns of a workgroup, as rt_few_rows has them
-  const int64_t ks = k_parts(M, N, K, act).n, ws = ks > 4 ? 8 : ks > 2 ? 4 : ks, rt = std::max<int64_t>(1, ws / 2), cols = ws > 1 ? 16 : 32;
-  const double rounds = (double)(((N + cols - 1) / cols * ((M + 63) / 64) + 255) / 256), steps = (double)((K / 64 + ks - 1) / ks * 2);
-  double tiles = 4 + 0.77 * K / 64;
-  if (act) tiles += 9;
-  else if (M <= 512) tiles = std::min(tiles, K > 2048 ? 17.0 : 14.0);
-  return 2.5 + (0.3 + 0.15 * rt) * steps * rounds < tiles;
-}
-
-// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it, or few_rows_kernel
+// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it
 static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  if (M > 64 && few_rows_pays(M, N, K, act)) {
-    auto y = at::empty({M, N}, x.options());
-    const KParts kp = k_parts(M, N, K, act);
-    check_rc(rt_few_rows(x.data_ptr(), x.stride(0), nullptr, 0, nullptr, nullptr, nullptr, w.data_ptr(), w.stride(0), b.data_ptr(),
-                         y.data_ptr(), N, (int)M, (int)N, (int)K, (int)act, 0.f, kp.n, kp.grp, cur_stream()),
-             "encoder: product");
-    return y;
-  }
   if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
   const auto [split, bn] = token_split(M, N, K, act);
   if (split > 1) {

@@ -49,6 +49,8 @@ struct Tuning {
   float gemm_bn128_cost = 0.55f;  // planner: time of a 256x128 tile / a 256x256 tile
   int gemm_duo = 1;           // NT products on two workgroups per CU: 0 never, 1 where they are short (gemm_big.hip), 2
                               // wherever the kernel takes them
+  int gemm_mid = 1;           // ... and on smaller tiles: 0 never, 1 where the larger leave CUs idle, 2 / 3 / 4 always on 64 x 64 /
+                              // 128 x 64 / 128 x 128
   int gemm_group_m = 4;       // rows of 256x256 tiles per L2-reuse group in the tile order
   // ---- sampler (sampling.hip) ----
   int sample_window = 1;      // top-k: candidates from a window below the row max, k-th key in one

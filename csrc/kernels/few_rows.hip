@@ -10,8 +10,7 @@
 // Bound by latency. 15 rows, us,
 // gemm_decode_kernel -> this: 1152 x 384 5.2 -> 4.0, 1536 x 384 with GELU 5.8 -> 4.4, 384 x 1536 9.8 -> 5.2, and 2.9 of the norm
 // with it; 20 rows, gemm_m64_kernel or the wide one: 6.6 -> 4.9, 11.0 -> 5.3, 21.3 -> 7.1; 64 rows: 6.9 -> 7.9, 16.2 -> 8.3, 21.7 ->
-// 10.6. More rows go in groups of 64, a workgroup reading its 64 rows from L2 for 16 or 32 columns: ahead of the tile kernels
-// while that is a workgroup or two per CU (few_rows_pays in bindings.cpp).
+// 10.6.
 #include "rt_common.h"
 #include "rt_gelu.h"
 
@@ -42,12 +41,6 @@ __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
   const int nc = p.K / 64, CG = 8 / (p.ks * p.rs), RTS = p.rs * RT;  // column groups, row tiles of the workgroup
   const int ks = wid % p.ks, rs = wid / p.ks % p.rs, cg = wid / (p.ks * p.rs);
   const int n0 = (blockIdx.x * CG + cg) * 16;
-  if constexpr (NW == 0) {  // 64 rows of more
-    const int r0 = blockIdx.y * 64;
-    p.x += (long)r0 * p.ldx;
-    p.y += (long)r0 * p.ldy;
-    p.M = min(p.M - r0, 64);
-  }
   const bool on = n0 < p.N && rs * RT * 16 < p.M;
   auto begin = [&](int part) { return 2 * (part * nc / p.parts); };  // in steps of 32
   const bf16_t* const wp = p.w + (long)min(n0 + r16, p.N - 1) * p.ldw + 8 * g;
@@ -256,14 +249,14 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
 
 using namespace rt;
 
-// y = act(x w^T + bias), or act(LN(x + res) w^T + bias) with LN(x + res) to xo (lw given; M <= 32, K <= 1024); act 0 or 2
+// y = act(x w^T + bias), or act(LN(x + res) w^T + bias) with LN(x + res) to xo (lw given; M <= 32, K <= 1024); M <= 64, act 0 or 2
 // (GELU). N % 16 == 0, K % 64 == 0; operands 16-B aligned, leading dimensions multiples of 8; up to 8 parts, up to 16 rows 16,
 // a multiple of grp. -1: not for this kernel.
 extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, const void* lw, const void* lb, void* xo, const void* w,
                            long ldw, const void* bias, void* y, long ldy, int M, int N, int K, int act, float eps, int parts, int grp,
                            hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 65535 * 64 || N % 16 || K < 64 || K % 64 || (act != 0 && act != 2) || (lw && (M > 32 || K > 1024 || !lb || !res || !xo))) return -1;
+  if (M > 64 || N % 16 || K < 64 || K % 64 || (act != 0 && act != 2) || (lw && (M > 32 || K > 1024 || !lb || !res || !xo))) return -1;
   if (parts < 1 || parts > (M <= 16 ? 16 : 8) || grp < 1 || parts % grp) return -1;
   fr::Args p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.res = (const bf16_t*)res; p.ldr = ldr;
@@ -275,7 +268,7 @@ extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, c
   p.rs = std::min(tiles > 1 ? 4 : 1, 8 / p.ks);  // 17..32 rows in one part: rather idle waves than half the workgroups
   const int rt = std::max(tiles / p.rs, 1), cols = 16 * (8 / (p.ks * p.rs)), nw = lw ? (K <= 512 ? 1 : 2) : 0;
   if (nw && rt != 1) return -1;
-  const dim3 grid((N + cols - 1) / cols, (M + 63) / 64), block(512);
+  const dim3 grid((N + cols - 1) / cols), block(512);
 #define FR(R, W, T) hipLaunchKernelGGL((fr::few_rows_kernel<R, W, T>), grid, block, 0, stream, p)
   if (nw == 1) { if (tiles == 1) FR(1, 1, 1); else FR(1, 1, 2); }
   else if (nw == 2) { if (tiles == 1) FR(1, 2, 1); else FR(1, 2, 2); }

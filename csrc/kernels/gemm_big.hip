@@ -899,6 +899,175 @@ __global__ __launch_bounds__(256, 2) void gemm_duo_kernel(Args p) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// NT products with fewer tiles of 256 rows than CUs
+// ---------------------------------------------------------------------------------------------
+// gemm_duo_kernel's product and bits on tiles of 32 FM x 32 FN: 4 waves, 2 x 2, of 16 FM x 16 FN. K-steps of 64 (A rows, then
+// B rows of 128 B in one image) go through a ring of SL images by LDS-DMA, SL - 1 ahead, with one barrier a step.
+// A 256 x 128 tile is a chain of 0.73 us a K-step and 5 to begin and end, however many CUs have none; 64 x 64 take 0.19 and 3. They
+// read 4 times the bytes through LDS, which is what bounds them once there are more than three or four on a CU; 128 x 64 and
+// 128 x 128 stand between. us, tiles of 256 rows -> 64 x 64 / 128 x 64 / 128 x 128: 600 x 384 x 1536 22.3 -> 7.4 / 10.4 / 16.0,
+// 4500 x 384 x 1536 23.4 -> 13.0 / 12.3 / 17.0, 2200 x 768 x 3072 40.4 -> 21.6 / 20.3 / 28.4, 4500 x 768 x 3072 41.1 -> 40.8 / 31.8 /
+// 29.3, 1500 x 1536 x 384 with GELU 18.4 -> 10.5 / 9.6 / 11.8, 13000 x 384 x 1536 24.5 -> 27.7 / 26.0 / 32.1.
+// all but the wave's N youngest loads are done, and its LDS reads
+template <int N>
+__device__ __forceinline__ void wait_but() {
+  static_assert(N == 0 || N == 4 || N == 6 || N == 8 || N == 12 || N == 16, "wait_but");
+  if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  else if constexpr (N == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+  else if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+  else if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+  else if constexpr (N == 12) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+}
+
+// no template: hipcc's host pass drops kernels that call the builtin with dependent arguments
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* to, uint32_t off, int base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)to, 16, off, base, 0, 0);
+}
+
+template <int EPI, int FM, int FN, int SL>
+__global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
+  constexpr int TM = 32 * FM, TN = 32 * FN, IMG = (TM + TN) * 128, NI = (TM + TN) / 32;  // LDS-DMA instructions per wave and step
+  constexpr int LDT = TN + 4;  // row of the epilogue's bf16 tile
+  static_assert(TM * LDT * 2 <= SL * IMG, "the tile fits the ring");
+  __shared__ __attribute__((aligned(16))) char smem[SL * IMG];
+  const int tiles_m = (p.M + TM - 1) / TM, tiles_n = (p.N + TN - 1) / TN;
+  const int nk = p.K / 64;  // K % 64 == 0 (launcher)
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wid >> 1, wc = wid & 1;
+  const int frow = lane & 15, fq = lane >> 4;
+  const int bid = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+  const int GM = (p.group_m > 0 ? p.group_m : GROUP_M) * (256 / TM);
+  const int group = bid / (GM * tiles_n), first_m = group * GM, gsz = min(tiles_m - first_m, GM);
+  const int m0 = (first_m + bid % gsz) * TM, n0 = bid % (GM * tiles_n) / gsz * TN;
+
+  // instruction j of this wave: rows 8 (NI wid + j) .. + 7 of the image, as in gemm_duo_kernel
+  uint32_t src[NI];  // bytes from the tile's first row
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int row = (wid * NI + j) * 8 + (lane >> 3), kc = ((lane & 7) ^ row_swz(row)) * 16;
+    src[j] = row < TM ? (uint32_t)(min(m0 + row, p.M - 1) - m0) * (uint32_t)p.lda * 2 + kc
+                      : (uint32_t)(min(n0 + row - TM, p.N - 1) - n0) * (uint32_t)p.ldb * 2 + kc;
+  }
+  const __amdgpu_buffer_rsrc_t Ar = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (long)m0 * p.lda), 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t Br = __builtin_amdgcn_make_buffer_rsrc((void*)(p.B + (long)n0 * p.ldb), 0, -1, 0x00020000);
+  auto stage = [&](int t, int slot) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      dma16((wid * NI + j) * 8 < TM ? Ar : Br, smem + slot * IMG + (wid * NI + j) * 1024, src[j], t * 128);
+    }
+  };
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int sw = row_swz(frow), c0 = (fq ^ sw) << 4, c1 = ((4 + fq) ^ sw) << 4;
+  const int ra = (wr * 16 * FM + frow) * 128, rb = (TM + wc * 16 * FN + frow) * 128;
+  // K-step t in `slot`; `ahead`: steps behind it whose DMA may still be under way
+  auto step = [&](auto ahead, int t, int slot) {
+    constexpr int NEWER = decltype(ahead)::value;
+    // this wave's share of the image has landed and its reads of the last image are done; behind the barrier every wave's
+    wait_but<NEWER * NI>();
+    GB_BARRIER();
+    __builtin_amdgcn_sched_barrier(0);
+    const char* img = smem + slot * IMG;
+    bf16x8 fa[2][FM], fb[2][FN];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[kk][i] = *(const bf16x8*)(img + ra + i * 2048 + (kk ? c1 : c0));
+#pragma unroll
+      for (int j = 0; j < FN; ++j) fb[kk][j] = *(const bf16x8*)(img + rb + j * 2048 + (kk ? c1 : c0));
+    }
+    if constexpr (NEWER == SL - 2) {
+      if (t + SL - 1 < nk) stage(t + SL - 1, slot == 0 ? SL - 1 : slot - 1);  // the image read in the last step
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][j], fa[kk][i], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < SL - 1; ++t)
+    if (t < nk) stage(t, t);
+  int t = 0, slot = 0;
+  auto next = [&] {
+    ++t;
+    slot = slot == SL - 1 ? 0 : slot + 1;
+  };
+  for (; t + SL - 2 < nk; next()) step(std::integral_constant<int, SL - 2>{}, t, slot);
+  // the last ones, whose successors are all under way
+  if constexpr (SL >= 5) if (t + 3 == nk) { step(std::integral_constant<int, 2>{}, t, slot); next(); }
+  if constexpr (SL >= 4) if (t + 2 == nk) { step(std::integral_constant<int, 1>{}, t, slot); next(); }
+  if (t + 1 == nk) step(std::integral_constant<int, 0>{}, t, slot);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  GB_BARRIER();
+
+  // acc[i][j][r] = C[m0 + 16 FM wr + 16 i + frow][n0 + 16 FN wc + 16 j + 4 fq + r]
+  bf16_t* tile = (bf16_t*)smem;
+  float bcol[FN][4] = {};
+  if (p.bias) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bcol[j][r] = bf2f(p.bias[min(n0 + wc * 16 * FN + j * 16 + fq * 4 + r, p.N - 1)]);
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    if (m0 + wr * 16 * FM + i * 16 >= p.M) break;
+    bf16_t* to = tile + (wr * 16 * FM + i * 16 + frow) * LDT + wc * 16 * FN + fq * 4;
+    if constexpr (EPI == E_GELU) {
+      float x[4 * FN];
+      uint32_t y[2 * FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[4 * j + r] = acc[i][j][r] + bcol[j][r];
+      unsigned open = 0;
+#pragma unroll
+      for (int k = 0; k < 2 * FN; ++k) open |= gelu2_fast(x[2 * k], x[2 * k + 1], y[k]) ? 0u : 1u << k;
+      gelu2_settle<2 * FN>(x, y, open);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) *(uint2*)(to + j * 16) = make_uint2(y[2 * j], y[2 * j + 1]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = act_fn(acc[i][j][r] + bcol[j][r], EPI);
+        *(uint2*)(to + j * 16) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+      }
+    }
+  }
+  __syncthreads();
+  bf16_t* C = (bf16_t*)p.C;
+  constexpr int CPR = TN / 8, RPP = 256 / CPR;  // 16-B chunks a row, rows a pass
+  const int cc = tid % CPR, gcol = n0 + cc * 8;
+  if (gcol >= p.N) return;
+#pragma unroll 2
+  for (int row = tid / CPR; row < TM; row += RPP) {
+    const int grow = m0 + row;
+    if (grow >= p.M) break;
+    const uint2 lo = *(const uint2*)(tile + row * LDT + cc * 8), hi = *(const uint2*)(tile + row * LDT + cc * 8 + 4);
+    uint4 v = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    if (p.R) {  // residual in fp32 on the bf16-rounded GEMM result (= a separate add kernel)
+      float y[8], r[8];
+      unpack8(v, y);
+      unpack8(*(const uint4*)(p.R + (long)grow * p.ldr + gcol), r);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] += r[e];
+      v = pack8(y);
+    }
+    *(uint4*)(C + (long)grow * p.ldc + gcol) = v;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // Small-tile GEMM for the narrow LoRA products (SURVEY K1 dA / dB / LoRA down-projection):
 //   U  = X A_pad^T   [M, Rp]   (ROW / ROW)        dU = dY UB   [M, Rp]  (ROW / KMAJ)
 //   dA = dU^T X      [Rp, K]   (KMAJ / KMAJ)      dB = dY^T U  [N, Rp]  (KMAJ / KMAJ)
@@ -1251,6 +1420,41 @@ extern "C" int rt_gemm_big(int layout_a, int layout_b, const void* A, long lda, 
                          N, K, act, out, nsplit, zpage, bn, nullptr, stream);
 }
 
+// us of gemm_mid_kernel for M rows, fitted to 150 shapes with N of 384 to 6144 and K of 384 to 4096, mostly within 10 % (form: 1
+// 64 x 64, 2 128 x 64, 3 128 x 128): rounds of a tile per CU; two on a CU hide some of each other's latency and their epilogues
+static float mid_us(long M, int N, int K, int act, int form) {
+  const long tm = form == 1 ? 64 : 128, tn = form == 3 ? 128 : 64;
+  const long r = ((M + tm - 1) / tm * ((N + tn - 1) / tn) + num_cus() - 1) / num_cus(), pairs = (r + 1) / 2;
+  const float nk = (float)(K / 64);
+  if (form == 1) return 2.6f + (float)r * (0.19f * nk + 0.4f) + (r > 2 ? 0.5f : 0.f) + (act ? 1.3f * (float)pairs : 0.f);
+  if (form == 2) return 2.2f + 0.05f * nk + (float)r * (0.28f * nk + 0.8f) - (r == 2 ? 1.2f : 0.f) + (act ? 2.6f * (float)pairs : 0.f);
+  return (float)r * (0.5f * nk + (act ? 8.5f : 4.7f));
+}
+static float mid_best(long M, int N, int K, int act, int* form) {
+  float best = 1e30f;
+  for (int f = 1; f <= 3; ++f) {
+    const float t = mid_us(M, N, K, act, f);
+    if (t < best) { best = t; *form = f; }
+  }
+  return best;
+}
+// us of a 256 x 256 tile of gemm_big_kernel
+static float big_us(int K) { return 5.3f + 1.37f / 64.f * (float)K; }
+
+template <int EPI>
+static int launch_mid_form(const Args& p, int form, hipStream_t stream) {
+  const int tm = form == 1 ? 64 : 128, tn = form == 3 ? 128 : 64;
+  const dim3 grid((unsigned)((long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn))), block(256);
+  if (form == 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 2, 2, 5>), grid, block, 0, stream, p);
+  else if (form == 2) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 4, 2, 3>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((gemm_mid_kernel<EPI, 4, 4, 4>), grid, block, 0, stream, p);
+  RT_LAUNCH_CHECK();
+  return 0;
+}
+static int launch_mid(const Args& p, int form, int act, hipStream_t stream) {
+  return act == E_GELU ? launch_mid_form<E_GELU>(p, form, stream) : launch_mid_form<E_NONE>(p, form, stream);
+}
+
 // bn = 0: the wave planner over validated arguments p
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream) {
   if (bn != 0) return launch_gemm_big(p, layout_a, layout_b, act, out, bn, stream);
@@ -1261,10 +1465,18 @@ static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, 
   // 86; 2000 x 768 x 768, 36 tiles: 15.9 against 14.8) and up to K = 1024, where it meets gemm_big_kernel (20000 x 4096 x
   // 1024: 156 both; 32000 x 2048 x 1536: 187 against 177).
   const long duo_tiles = (long)((M + 255) / 256) * ((N + 127) / 128);
-  if (tuning().gemm_duo && layout_a == ROW && layout_b == ROW && out == O_BF16 && nsplit == 1 && !p.A2 && p.K >= 64 &&
-      p.K % 64 == 0 && p.lda < (1 << 22) && p.ldb < (1 << 22) &&  // 32-bit byte offsets within a tile
-      (tuning().gemm_duo == 2 ? act == E_NONE || act == E_GELU
-                              : (act == E_GELU && p.K <= 2048) || (act == E_NONE && p.K <= 1024 && duo_tiles > num_cus()))) {
+  const bool plain = layout_a == ROW && layout_b == ROW && out == O_BF16 && nsplit == 1 && !p.A2 && p.K >= 64 && p.K % 64 == 0 &&
+                     p.lda < (1 << 22) && p.ldb < (1 << 22) && (act == E_NONE || act == E_GELU);  // 32-bit byte offsets within a tile
+  if (plain && tuning().gemm_mid > 1) return launch_mid(p, tuning().gemm_mid - 1, act, stream);
+  // Smaller tiles where they are done sooner: with few rows, and for the rows behind the last full wave of large tiles
+  const bool mid = plain && tuning().gemm_mid;
+  int form = 0;
+  if (tuning().gemm_duo && plain &&
+      (tuning().gemm_duo == 2 || (act == E_GELU && p.K <= 2048) || (act == E_NONE && p.K <= 1024 && duo_tiles > num_cus()))) {
+    // one tile on a CU, or pairs: 9000 x 1152 x 384 16.5 us, 6500 x 2304 x 768 26.6, 13000 x 2304 x 768 47.0
+    const float nk = (float)(p.K / 64), pairs = (float)duo_tiles / (2.f * num_cus());
+    const float duo = pairs <= 0.5f ? 5.3f + 0.73f * nk + (act ? 8.f : 0.f) : std::max(pairs, 1.f) * (9.f + 1.47f * nk + (act ? 10.f : 0.f));
+    if (mid && tuning().gemm_duo == 1 && pairs < 4.f && mid_best(M, N, p.K, act, &form) < 0.95f * duo) return launch_mid(p, form, act, stream);
     const dim3 grid((unsigned)duo_tiles), block(256);
     if (act == E_GELU) hipLaunchKernelGGL(gemm_duo_kernel<E_GELU>, grid, block, 0, stream, p);
     else hipLaunchKernelGGL(gemm_duo_kernel<E_NONE>, grid, block, 0, stream, p);
@@ -1290,6 +1502,18 @@ static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, 
       if (cost < best - 1e-3f) { best = cost; m1 = m; }
     }
   }
+  int tail = 0;  // the form of the rows behind m1 row tiles, 0: 256 x 128
+  if (mid) {
+    const float unit = big_us(p.K);
+    best *= 0.97f;
+    for (int m = tiles_m; m >= 0; --m) {
+      const long rest = M - (long)m * 256;
+      if (rest <= 0) continue;
+      if (rest * N > (long)num_cus() * 8 * 4096) break;  // more than eight 64 x 64 tiles per CU
+      const float cost = (float)(((long)m * tn256 + cus - 1) / cus) + mid_best(rest, N, p.K, act, &form) / unit;
+      if (cost < best - 1e-3f) { best = cost; m1 = m; tail = form; }
+    }
+  }
   if (m1 == tiles_m) return launch_gemm_big(p, layout_a, layout_b, act, out, 256, stream);
   const long r0 = (long)m1 * 256;
   if (m1 > 0) {
@@ -1306,7 +1530,7 @@ static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, 
   if (p.C2) q.C2 = p.C2 + r0 * ldc2;
   if (p.R) q.R = p.R + r0 * ldr;
   if (p.rope_pos) q.rope_pos = p.rope_pos + r0;
-  return launch_gemm_big(q, layout_a, layout_b, act, out, 128, stream);
+  return tail ? launch_mid(q, tail, act, stream) : launch_gemm_big(q, layout_a, layout_b, act, out, 128, stream);
 }
 
 // Grouped NT product C[r] = epi(A[row_map[r]] B_g^T) over rows sorted by group g (see GRP above): bf16 out,

@@ -53,6 +53,16 @@ def splitk_plan(M: int, N: int, K: int, act: int = 0):
     return s, 0 if s == 1 and act == ACT_IDS["gelu"] else bn
 
 
+def small_tiles(M: int, N: int, K: int, act: int) -> bool:
+    """Whether 65 to 512 rows of an encoder's product (one with a bias) take 64x64 tiles without a K split (rt_gemm_big's planner
+    picks them): 2.6 us and 0.19 a K-step for every tile of a CU, where a split product and its reduction take 14, from K = 2048
+    on 17. Decoders' products stay with the split, which their norms and attention sum themselves."""
+    if M <= 64 or K % 64 or K > 3072 or act not in (0, ACT_IDS["gelu"]):
+        return False
+    rounds = ((M + 63) // 64 * ((N + 63) // 64) + 255) // 256
+    return 2.6 + rounds * (0.19 * (K // 64) + (1.7 if act else 0.4)) < (17 if K > 2048 else 14)
+
+
 _BI = threading.local()  # per-thread nesting depth of batch_invariant() (a serving thread keeps its plans)
 
 
@@ -108,6 +118,8 @@ def gemm(x: torch.Tensor, w: torch.Tensor, u=None, ub=None, bias=None, act=0, ou
             s, bn = max(s, 2), 128
         if nsplit:
             s = nsplit
+        elif bias is not None and not out_f32 and u is None and M <= 512 and small_tiles(M, N, K, act):
+            s, bn = 1, 0
         if u is not None or out_f32 or N % 16:
             s = 1
         if s > 1:
