@@ -94,7 +94,7 @@ int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
 int rt_segment_mean(const float*, int, const long*, const int*, int, int, float*, hipStream_t);
-int rt_ivf_scan(const void*, int, int, const int*, int, const int*, const int*, const void*, const long*, const float*,
+int rt_ivf_scan(const void*, int, int, const int*, int, int, const int*, const int*, const void*, const long*, const float*,
                 int, int, float*, long*,
                 hipStream_t);
 int rt_gae(const float*, const float*, const float*, int, int, float, float, float*, float*, hipStream_t);
@@ -1472,9 +1472,10 @@ std::vector<Tensor> topk(const Tensor& scores, int64_t k, const optional<Tensor>
   return {vals, ids};
 }
 
-std::vector<Tensor> ivf_scan(const Tensor& q, const Tensor& probes, const Tensor& lstart, const Tensor& lsize,
+std::vector<Tensor> ivf_scan(const Tensor& q_, const Tensor& probes, const Tensor& lstart, const Tensor& lsize,
                              const Tensor& vecs, const Tensor& ids, const optional<Tensor>& sqnorm, bool l2,
                              int64_t maxlen) {
+  const Tensor q = (uintptr_t)q_.data_ptr() % 16 ? q_.clone() : q_;
   CHECK_CUDA(q); CHECK_BF16(q); CHECK_I32(probes); CHECK_I32(lstart); CHECK_I32(lsize); CHECK_BF16(vecs); CHECK_I64(ids);
   TORCH_CHECK(q.is_contiguous() && probes.is_contiguous() && vecs.is_contiguous() && lstart.is_contiguous() &&
               lsize.is_contiguous());
@@ -1482,7 +1483,7 @@ std::vector<Tensor> ivf_scan(const Tensor& q, const Tensor& probes, const Tensor
   const int64_t nq = q.size(0), d = q.size(1), nprobe = probes.size(1);
   auto cand = at::empty({nq, nprobe * maxlen}, q.options().dtype(at::kFloat));
   auto cid = at::empty({nq, nprobe * maxlen}, q.options().dtype(at::kLong));
-  check_rc(rt_ivf_scan(q.data_ptr(), (int)nq, (int)d, probes.data_ptr<int>(), (int)nprobe, lstart.data_ptr<int>(),
+  check_rc(rt_ivf_scan(q.data_ptr(), (int)nq, (int)d, probes.data_ptr<int>(), (int)nprobe, (int)lsize.numel(), lstart.data_ptr<int>(),
                        lsize.data_ptr<int>(), vecs.data_ptr(), (const long*)ids.data_ptr(),
                        l2 ? sqnorm->data_ptr<float>() : nullptr, l2 ? 1 : 0, (int)maxlen, cand.data_ptr<float>(),
                        (long*)cid.data_ptr(), cur_stream()),
@@ -1674,7 +1675,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
         py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
         py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
-  m.def("few_rows", &few_rows, "act(x w^T + b) in groups of 64 rows, up to 32 rows normalised first if asked", py::arg("x"), py::arg("w"),
+  m.def("few_rows", &few_rows, "act(x w^T + b) of up to 64 rows, up to 32 normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);
   m.def("attn_fwd", &attn_fwd);

@@ -155,7 +155,7 @@ __device__ void topk_select(const float* s, int N, int K, TopkShared& sh) {
 // the row's k-th largest score that few surplus elements reach: the threads that hold one place theirs in LDS, and
 // every candidate counts the candidates ahead of it, which is its place in the result. Two passes over the row at
 // most, no histogram, no sort (four passes and a sort of 1024 before): top 16 of 512 and top 3 of 9600, one row,
-// 88 -> 8.3 and 10.8 us each. Rows with more than TOPK_CAND candidates go through topk_select first.
+// 88 -> 8.3 and 10.8 us each; eight loads in flight in either pass, 16 of 512 and 3 of 7800: 7.8 -> 7.2 and 13.0 -> 11.7. Rows with more than TOPK_CAND candidates go through topk_select first.
 // NT: a wave where its 64 maxima suffice (k <= 32) and hold 16 elements each at most (k-means assignment: 65536 rows
 // of 512), 1024 threads for long rows, 256 between.
 template <int NT>
@@ -169,15 +169,17 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
   const float* s = scores + row * ld;
   const int tid = threadIdx.x, lane = tid & 63, K = min(k, N);
   uint32_t km = 0;
-  int i0 = tid;
-  for (; i0 + 7 * NT < N; i0 += 8 * NT) {
-    float v[8];
+  // eight loads in flight, those past the end of the last element
+  auto scan = [&](auto&& use) {
+    for (int i0 = tid; i0 < N; i0 += 8 * NT) {
+      float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = s[i0 + e * NT];
+      for (int e = 0; e < 8; ++e) v[e] = s[min(i0 + e * NT, N - 1)];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) km = max(km, okey(v[e]));
-  }
-  for (; i0 < N; i0 += NT) km = max(km, okey(s[i0]));
+      for (int e = 0; e < 8; ++e) use(v[e], i0 + e * NT);
+    }
+  };
+  scan([&](float v, int i) { km = i < N ? max(km, okey(v)) : km; });  // the maxima are of different elements
   tmax[tid] = km;
   if (tid == 0) sh.cnt = 0;
   __syncthreads();
@@ -191,13 +193,12 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
   __syncthreads();
   const uint32_t thr = sh.sel;
   if (km >= thr)
-    for (int i = tid; i < N; i += NT) {
-      const float v = s[i];
-      if (okey(v) >= thr) {
+    scan([&](float v, int i) {
+      if (i < N && okey(v) >= thr) {
         const unsigned slot = atomicAdd(&sh.cnt, 1u);
         if (slot < TOPK_CAND) { sh.cv[slot] = v; sh.ci[slot] = i; }
       }
-    }
+    });
   __syncthreads();
   int n = (int)sh.cnt;
   if (n > TOPK_CAND) {
@@ -233,76 +234,120 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
 // list (vectors stored contiguously per list from lstart[L], lsize[L] of them; lists may carry
 // spare capacity for incremental adds) and write into cand[qi, p*maxlen + j] (+ ids).
 // Metric: inner product, or (l2) the negated squared distance 2 q.x - |x|^2 - |q|^2 with |x|^2
-// stored per slot — both "higher is better" for the shared top-k. Unused slots get -inf.
-// One wave per 64 vectors of a (probe, query), one thread per vector, query in LDS: a single query's 16 lists of 200 to
-// 800 are a few hundred waves on as many CUs, where one workgroup per list left 240 CUs idle; 8 of a vector's 16-byte
-// pieces are in flight (16 lists of 600 x 384: 12.4 -> 8.6 us). A vector's terms are summed in the order of the
-// dimensions.
-__global__ __launch_bounds__(64) void ivf_scan_kernel(const bf16_t* __restrict__ q, int d, const int* __restrict__ probes,
-                                                      int nprobe, const int* __restrict__ lstart,
-                                                      const int* __restrict__ lsize, const bf16_t* __restrict__ vecs,
-                                                      const long* __restrict__ ids, const float* __restrict__ sqnorm,
-                                                      int l2, int maxlen, float* __restrict__ cand,
-                                                      long* __restrict__ cand_ids) {
-  extern __shared__ float qs[];
-  const int p = blockIdx.x, qi = blockIdx.y;
-  const long j0 = blockIdx.z * 64L, step = gridDim.z * 64L;
-  const int L = probes[(long)qi * nprobe + p];
-  const int b0 = L >= 0 ? lstart[L] : 0;
-  const int len = L >= 0 ? min(lsize[L], maxlen) : 0;
-  float* out = cand + ((long)qi * nprobe + p) * maxlen;
-  long* oid = cand_ids + ((long)qi * nprobe + p) * maxlen;
-  if (j0 >= len) {
-    for (long j = j0 + threadIdx.x; j < maxlen; j += step) { out[j] = -INFINITY; oid[j] = -1; }
-    return;
-  }
-  // |q|^2 in four interleaved parts, added in order
-  float part[4] = {};
-  for (int i0 = threadIdx.x; i0 < d; i0 += 256) {
+// stored per slot — both "higher is better" for the shared top-k. Unused slots get -inf, and so do probes of no list.
+// A wave multiplies 16 vectors, held as MFMA fragments (64 B of 16 vectors a load), with 16 queries at a time; a thread per vector
+// had each 16-byte load of a wave touch 64 lines, of which L1 kept none for the next one. BY_LIST: a workgroup takes 64
+// vectors of a list for every query that probes it, found among the probes, PAIRS at a time; else for one (query, probe).
+// Bound by the bytes read and written (12 a candidate). us, the thread per vector -> this: 64 queries over lists of up to 102108
+// vectors of 384 (200k in all) 9500 -> 724, 100 queries over 30k 2473 -> 202, one query over 16 lists of 200 10.5 -> 8.
+constexpr int PAIRS = 4096;
+struct ScanArgs {
+  const bf16_t* q; int nq, d; const int* probes; int nprobe, nlist;
+  const int* lstart; const int* lsize; const bf16_t* vecs; const long* ids; const float* sqnorm;
+  int l2, maxlen;
+  float* cand; long* cand_ids;
+};
+
+template <int NF, bool BY_LIST>  // NF: 32-element fragments of a vector held at once
+__global__ __launch_bounds__(256) void ivf_scan_kernel(ScanArgs a) {
+  __shared__ int pair[BY_LIST ? PAIRS : 1];  // query * nprobe + probe, from the round's first one
+  __shared__ int count;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long all = BY_LIST ? (long)a.nq * a.nprobe : 1, first = BY_LIST ? 0 : (long)blockIdx.y * a.nprobe + blockIdx.x;
+  const int L = BY_LIST ? blockIdx.x : a.probes[first];  // BY_LIST: nlist stands for no list
+  const bool real = L >= 0 && L < a.nlist;
+  const int b0 = real ? a.lstart[L] : 0, len = real ? min(a.lsize[L], a.maxlen) : 0;
+  const int z0 = blockIdx.z, zn = gridDim.z;
+  for (long base = 0; base < all; base += PAIRS) {
+    int n = 1;
+    if constexpr (BY_LIST) {
+      const int m = (int)min(all - base, (long)PAIRS);
+      __syncthreads();  // the last round's pairs have been read
+      if (tid == 0) count = 0;
+      __syncthreads();
+      for (int i0 = tid; i0 < m; i0 += 256 * 8) {
+        int l[8];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int i = i0 + 64 * w;
-      if (i >= d) continue;
-      const float v = bf2f(q[(long)qi * d + i]);
-      qs[i] = v;
-      part[w] += v * v;
+        for (int e = 0; e < 8; ++e) l[e] = a.probes[base + min(i0 + e * 256, m - 1)];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (i0 + e * 256 < m && (real ? l[e] == L : l[e] < 0 || l[e] >= a.nlist)) pair[atomicAdd(&count, 1)] = i0 + e * 256;
+      }
+      __syncthreads();
+      n = count;
     }
-  }
-  float qn = 0.f;
-  if (l2) {
-#pragma unroll
-    for (int w = 0; w < 4; ++w) qn += wave_sum(part[w]);
-  }
-  __syncthreads();
-  for (long j = j0 + threadIdx.x; j < maxlen; j += step) {
-    if (j >= len) {
-      out[j] = -INFINITY;
-      oid[j] = -1;
-      continue;
-    }
-    const bf16_t* vr = vecs + (b0 + j) * d;
-    float s = 0.f;
-    int c = 0;
-    for (; c + 64 <= d; c += 64) {
-      uint4 v[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = *(const uint4*)(vr + c + 8 * i);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float f[8];
-        unpack8(v[i], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += f[e] * qs[c + 8 * i + e];
+    auto pair_of = [&](int k) { return BY_LIST ? base + pair[k] : first; };
+    for (int k = 0; k < n; ++k) {  // slots behind the list's vectors
+      const long o = pair_of(k) * a.maxlen;
+      for (long j = len + z0 * 256L + tid; j < a.maxlen; j += zn * 256L) {
+        a.cand[o + j] = -INFINITY;
+        a.cand_ids[o + j] = -1;
       }
     }
-    for (; c < d; c += 8) {
-      float f[8];
-      unpack8(*(const uint4*)(vr + c), f);
+    if (n == 0) continue;
+    for (long v0 = z0 * 64L + wid * 16; v0 < len; v0 += zn * 64L) {
+      const bf16_t* vr = a.vecs + (b0 + min(v0 + r16, (long)len - 1)) * a.d + 8 * g;
+      bf16x8 x[NF];
+      auto load = [&](int c0) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s += f[e] * qs[c + e];
+        for (int s = 0; s < NF; ++s) {
+          x[s] = bf16x8{};
+          if (c0 + 32 * s + 8 * g < a.d) x[s] = *(const bf16x8*)(vr + c0 + 32 * s);
+        }
+      };
+      load(0);
+      long id[4];
+      float sq[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // of the vectors whose scores the lane holds
+        const long at = b0 + min(v0 + 4 * g + i, (long)len - 1);
+        id[i] = a.ids[at];
+        sq[i] = a.l2 ? a.sqnorm[at] : 0.f;
+      }
+      for (int t = 0; t < n; t += 16) {
+        const long pr = pair_of(min(t + r16, n - 1));
+        const bf16_t* qr = a.q + pr / a.nprobe * a.d + 8 * g;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        float qq = 0.f;
+        for (int c0 = 0; c0 < a.d; c0 += 32 * NF) {
+          if (a.d > 32 * NF && (t > 0 || c0 > 0)) load(c0);
+          bf16x8 y[NF];
+#pragma unroll
+          for (int s = 0; s < NF; ++s) {
+            y[s] = bf16x8{};
+            if (c0 + 32 * s + 8 * g < a.d) y[s] = *(const bf16x8*)(qr + c0 + 32 * s);
+          }
+#pragma unroll
+          for (int s = 0; s < NF; ++s)
+            if (c0 + 32 * s < a.d) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[s], y[s], acc, 0, 0, 0);
+          if (a.l2) {
+#pragma unroll
+            for (int s = 0; s < NF; ++s) {
+              float f[8];
+              unpack8(__builtin_bit_cast(uint4, y[s]), f);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) qq = fmaf(f[e], f[e], qq);
+            }
+          }
+        }
+        if (a.l2) {
+          qq += __shfl_xor(qq, 16, 64);
+          qq += __shfl_xor(qq, 32, 64);
+        }
+        // acc[i]: vector v0 + 4 g + i, query r16 of the sixteen
+        if (t + r16 < n && (BY_LIST || r16 == 0)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const long j = v0 + 4 * g + i;
+            if (j < len) {
+              a.cand[pr * a.maxlen + j] = a.l2 ? 2.f * acc[i] - sq[i] - qq : acc[i];
+              a.cand_ids[pr * a.maxlen + j] = id[i];
+            }
+          }
+        }
+      }
     }
-    out[j] = l2 ? 2.f * s - sqnorm[b0 + j] - qn : s;
-    oid[j] = ids[b0 + j];
   }
 }
 
@@ -363,16 +408,25 @@ extern "C" int rt_topk(const float* scores, long ld, long nq, int N, int k, cons
   return 0;
 }
 
-extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int nprobe, const int* lstart,
+extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int nprobe, int nlist, const int* lstart,
                            const int* lsize, const void* vecs, const long* ids, const float* sqnorm, int l2,
                            int maxlen, float* cand, long* cand_ids, hipStream_t stream) {
-  if (d % 8 != 0 || (l2 && !sqnorm)) return -1;
-  if (nq == 0) return 0;
+  if (d % 8 != 0 || (l2 && !sqnorm) || (uintptr_t)q % 16 || (uintptr_t)vecs % 16) return -1;
+  if (nq == 0 || nprobe == 0) return 0;
   if (maxlen <= 0) return 0;
-  // a grid's third dimension ends at 65535: longer lists (over 4 million vectors) go round
-  const unsigned pieces = (unsigned)std::min((maxlen + 63L) / 64, 65535L);
-  hipLaunchKernelGGL(ivf_scan_kernel, dim3(nprobe, nq, pieces), dim3(64), d * sizeof(float), stream, (const bf16_t*)q, d, probes,
-                     nprobe, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, cand, cand_ids);
+  const ScanArgs a{(const bf16_t*)q, nq, d, probes, nprobe, nlist, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, cand, cand_ids};
+  // a list's vectors are read once for all its queries as soon as a list has one on average
+  const bool by_list = (long)nq * nprobe >= nlist || nq > 65535;
+  const long pieces = (maxlen + 63L) / 64;  // a grid's third dimension ends at 65535: longer lists go round
+  const dim3 grid = by_list ? dim3(nlist + 1, 1, (unsigned)std::min(pieces, 64L)) : dim3(nprobe, nq, (unsigned)std::min(pieces, 65535L));
+#define SCAN(NF)                                                                                   \
+  do {                                                                                             \
+    if (by_list) hipLaunchKernelGGL((ivf_scan_kernel<NF, true>), grid, dim3(256), 0, stream, a);   \
+    else hipLaunchKernelGGL((ivf_scan_kernel<NF, false>), grid, dim3(256), 0, stream, a);          \
+  } while (0)
+  if (d <= 384) SCAN(12);
+  else SCAN(24);
+#undef SCAN
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -237,6 +237,34 @@ def test_ivf_scan_lists(d, l2):
     torch.testing.assert_close(cand.double(), want.view(3, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
 
 
+@pytest.mark.parametrize("d", [8, 384, 392, 800])
+@pytest.mark.parametrize("l2", [False, True])
+@pytest.mark.parametrize("nq,nlist", [(1, 9), (3, 40), (17, 6), (700, 6)])
+def test_ivf_scan_by_list_and_by_probe(d, l2, nq, nlist):
+    """A workgroup per list or per probe, queries around the tiles of 16, more than 4096 probes, an unaligned first query."""
+    g = torch.Generator(device=DEV).manual_seed(d + nq)
+    size = torch.zeros(nlist, dtype=torch.int32, device=DEV)
+    size[:6] = torch.tensor([0, 1, 15, 16, 17, 150], dtype=torch.int32, device=DEV)
+    start = torch.cumsum(size, 0).int() - size
+    vecs = torch.randn(int(size.sum()), d, generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn(nq * d + 1, generator=g, device=DEV).to(torch.bfloat16)[1:].view(nq, d)
+    nprobe = 6
+    probes = torch.stack([torch.randperm(6, generator=g, device=DEV) for _ in range(nq)]).int()
+    probes[nq // 2, 2] = -1
+    sq, ids, maxlen = vecs.float().pow(2).sum(-1), torch.arange(len(vecs), device=DEV) + 7, 151
+    cand, cid = ops.ivf_scan(q, probes, start, size, vecs, ids, maxlen, sq, l2)
+    full = q.double() @ vecs.double().t()
+    if l2:
+        full = 2 * full - sq.double() - q.double().pow(2).sum(-1, keepdim=True)
+    j = torch.arange(maxlen, device=DEV)
+    L = probes.long().clamp(min=0)
+    ok = (j < size[L][..., None]) & (probes >= 0)[..., None]
+    at = (start[L][..., None] + j).clamp(max=len(vecs) - 1)
+    want = full.gather(1, at.view(nq, -1)).view(nq, nprobe, maxlen).masked_fill(~ok, float("-inf"))
+    assert torch.equal(cid, ids[at].masked_fill(~ok, -1).view(nq, -1))
+    torch.testing.assert_close(cand.double(), want.view(nq, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
+
+
 def test_ivf_scan_of_a_list_longer_than_a_grid():
     """A list of more 64-vector pieces than a grid's third dimension holds, and a short one beside it."""
     d, n = 8, 65535 * 64 + 1000
