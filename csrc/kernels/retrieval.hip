@@ -155,7 +155,8 @@ __device__ void topk_select(const float* s, int N, int K, TopkShared& sh) {
 // the row's k-th largest score that few surplus elements reach: the threads that hold one place theirs in LDS, and
 // every candidate counts the candidates ahead of it, which is its place in the result. Two passes over the row at
 // most, no histogram, no sort (four passes and a sort of 1024 before): top 16 of 512 and top 3 of 9600, one row,
-// 88 -> 8.3 and 10.8 us each; eight loads in flight in either pass, 16 of 512 and 3 of 7800: 7.8 -> 7.2 and 13.0 -> 11.7. Rows with more than TOPK_CAND candidates go through topk_select first.
+// 88 -> 8.3 and 10.8 us each. Loads of both passes go out in blocks: top 3 of 100k, one row and 200 (top 5), 27 -> 20 and 47 -> 30.
+// Rows with more than TOPK_CAND candidates go through topk_select first.
 // NT: a wave where its 64 maxima suffice (k <= 32) and hold 16 elements each at most (k-means assignment: 65536 rows
 // of 512), 1024 threads for long rows, 256 between.
 template <int NT>
@@ -169,17 +170,26 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
   const float* s = scores + row * ld;
   const int tid = threadIdx.x, lane = tid & 63, K = min(k, N);
   uint32_t km = 0;
-  // eight loads in flight, those past the end of the last element
+  // eight loads in flight, at the end four, those past it of the last element
   auto scan = [&](auto&& use) {
-    for (int i0 = tid; i0 < N; i0 += 8 * NT) {
+    int i0 = tid;
+    for (; i0 + 7 * NT < N; i0 += 8 * NT) {
       float v[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = s[min(i0 + e * NT, N - 1)];
+      for (int e = 0; e < 8; ++e) v[e] = s[i0 + e * NT];
 #pragma unroll
       for (int e = 0; e < 8; ++e) use(v[e], i0 + e * NT);
     }
+    for (; i0 < N; i0 += 4 * NT) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = s[min(i0 + e * NT, N - 1)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i0 + e * NT < N) use(v[e], i0 + e * NT);
+    }
   };
-  scan([&](float v, int i) { km = i < N ? max(km, okey(v)) : km; });  // the maxima are of different elements
+  scan([&](float v, int) { km = max(km, okey(v)); });
   tmax[tid] = km;
   if (tid == 0) sh.cnt = 0;
   __syncthreads();
@@ -194,7 +204,7 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
   const uint32_t thr = sh.sel;
   if (km >= thr)
     scan([&](float v, int i) {
-      if (i < N && okey(v) >= thr) {
+      if (okey(v) >= thr) {
         const unsigned slot = atomicAdd(&sh.cnt, 1u);
         if (slot < TOPK_CAND) { sh.cv[slot] = v; sh.ci[slot] = i; }
       }
