@@ -1281,14 +1281,14 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
 
 // ops.linear's small_tiles (products with a bias)
 static bool small_tiles(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (M <= 64 || K % 64 || K > 3072 || (act != 0 && act != 2)) return false;
+  if (M <= 64 || M > 512 || K % 64 || K > 3072 || (act != 0 && act != 2)) return false;
   const int64_t rounds = ((M + 63) / 64 * ((N + 63) / 64) + 255) / 256;
   return 2.6 + rounds * (0.19 * (K / 64) + (act ? 1.7 : 0.4)) < (K > 2048 ? 17 : 14);
 }
 
 // The K split of ops.gemm's token-parallel products (splitk_plan there): parts and the columns of a tile
 static std::pair<int64_t, int64_t> token_split(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (M > 512 || small_tiles(M, N, K, act)) return {1, 0};
+  if (M > 512) return {1, 0};
   const int64_t bn = act == 0 ? 128 : 256, tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
   const int64_t split = tiles < 128 && N % 16 == 0 ? std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles)) : 1;
   return {split, split == 1 && act ? 0 : bn};
@@ -1340,6 +1340,8 @@ static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, 
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
   const auto [split, bn] = token_split(M, N, K, act);
+  if (small_tiles(M, N, K, act))
+    return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, split, std::nullopt, std::nullopt, std::nullopt, 0, {});
   if (split > 1) {
     auto slabs = at::empty({split * M * N}, x.options().dtype(at::kFloat));
     return gemm_splitk(x, w, split, slabs, b, act, std::nullopt, std::nullopt, bn, {});

@@ -925,7 +925,9 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* to, uint32
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)to, 16, off, base, 0, 0);
 }
 
-template <int EPI, int FM, int FN, int SL>
+// PARTS: K is summed in p.nsplit parts of whole steps, part i from i nk / nsplit on, and the parts in their order: the bits of
+// the split product (O_F32_SLAB) and its reduction, without slabs.
+template <int EPI, int FM, int FN, int SL, bool PARTS = false>
 __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
   constexpr int TM = 32 * FM, TN = 32 * FN, IMG = (TM + TN) * 128, NI = (TM + TN) / 32;  // LDS-DMA instructions per wave and step
   constexpr int LDT = TN + 4;  // row of the epilogue's bf16 tile
@@ -963,6 +965,14 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 sum[PARTS ? FM : 1][PARTS ? FN : 1];
+  int part = 0;
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const int sw = row_swz(frow), c0 = (fq ^ sw) << 4, c1 = ((4 + fq) ^ sw) << 4;
   const int ra = (wr * 16 * FM + frow) * 128, rb = (TM + wc * 16 * FN + frow) * 128;
   // K-step t in `slot`; `ahead`: steps behind it whose DMA may still be under way
@@ -991,6 +1001,18 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
 #pragma unroll
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][j], fa[kk][i], acc[i][j], 0, 0, 0);
+    if constexpr (PARTS) {
+      if (t + 1 == (int)((long)(part + 1) * nk / p.nsplit)) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            sum[i][j] += acc[i][j];
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        ++part;
+      }
+    }
   };
 #pragma unroll
   for (int t = 0; t < SL - 1; ++t)
@@ -1008,6 +1030,12 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   GB_BARRIER();
 
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
+  }
   // acc[i][j][r] = C[m0 + 16 FM wr + 16 i + frow][n0 + 16 FN wc + 16 j + 4 fq + r]
   bf16_t* tile = (bf16_t*)smem;
   float bcol[FN][4] = {};
@@ -1285,7 +1313,7 @@ using namespace rt;
 using namespace rt::gb;
 
 // layout_a / layout_b: 0 = ROW (K contiguous), 1 = KMAJ (M / N contiguous).
-// out: 0 bf16 (epilogue bias + act, or SwiGLU), 1 fp32 store (bias + act), 2 fp32 atomic add
+// out: 0 bf16 (epilogue bias + act, or SwiGLU; nsplit > 1: K in parts, see gemm_mid_kernel), 1 fp32 store (bias + act), 2 fp32 atomic add
 // (split-K; C must be initialised by the caller). Requirements (checked): KMAJ operands have
 // M / N % 8 == 0 and 16-B aligned rows; ROW operands 16-B aligned rows; K, K2 % 8 == 0;
 // E_SWIGLU: ROW/ROW, bf16 out, N % 256 == 0, no K-extension of B beyond the weight rows.
@@ -1362,9 +1390,10 @@ static int num_cus() {
 static float bn128_cost() { return tuning().gemm_bn128_cost; }
 
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream);
+static int launch_mid(const Args& p, int form, int act, hipStream_t stream);
 
 // layout_a / layout_b: 0 = ROW (K contiguous), 1 = KMAJ (M / N contiguous).
-// out: 0 bf16 (epilogue bias + act, or SwiGLU), 1 fp32 store (bias + act), 2 fp32 atomic add
+// out: 0 bf16 (epilogue bias + act, or SwiGLU; nsplit > 1: K in parts, see gemm_mid_kernel), 1 fp32 store (bias + act), 2 fp32 atomic add
 // (split-K; C must be initialised by the caller), 3 fp32 split-K slabs. bn: 256, 128, or 0 = plan:
 // the tile rows are cut in two launches — rows [0, 256 m1) on 256x256 tiles, the rest on 256x128
 // tiles — with m1 chosen so that the last, partial wave of workgroups is as short as possible
@@ -1388,7 +1417,10 @@ extern "C" int rt_gemm_big_glu(int layout_a, int layout_b, const void* A, long l
   if (out != O_F32_ATOMIC && (ldc % 8 || (M > 1 && ldc < (long)((Nout + 7) / 8 * 8)))) return -7;
   if ((layout_a == KMAJ && M % 8) || (layout_b == KMAJ && N % 8)) return -1;
   if (nsplit < 1) nsplit = 1;
-  if (nsplit > 1 && out != O_F32_ATOMIC && out != O_F32_SLAB) return -2;
+  const bool parts = nsplit > 1 && out == O_BF16;  // K in parts without slabs, on 64 x 64 tiles (gemm_mid_kernel)
+  if (parts && (layout_a != ROW || layout_b != ROW || A2 || K % 64 || nsplit > K / 64 || lda >= (1 << 22) || ldb >= (1 << 22) ||
+                (act != E_NONE && act != E_GELU) || bn))
+    return -2;
   if (act == E_SWIGLU && (layout_a != ROW || layout_b != ROW || out != O_BF16 || N % 256)) return -3;
   if (act == E_DSWIGLU) {
     // the SwiGLU backward epilogue: NN, bf16 d[gate | up] [M, 2N] from the pre-activation R [M, 2N]
@@ -1409,6 +1441,7 @@ extern "C" int rt_gemm_big_glu(int layout_a, int layout_b, const void* A, long l
   p.M = M; p.N = N; p.K = K; p.act = act; p.nsplit = nsplit; p.zpage = (const bf16_t*)zpage;
   p.group_m = tuning().gemm_group_m;
   if (glu_p) { p.glu.limit = glu_p[0]; p.glu.alpha = glu_p[1]; p.glu.offset = glu_p[2]; }
+  if (parts) return launch_mid(p, 1, act, stream);
   return gemm_big_planned(p, layout_a, layout_b, act, out, bn, stream);
 }
 
@@ -1445,7 +1478,8 @@ template <int EPI>
 static int launch_mid_form(const Args& p, int form, hipStream_t stream) {
   const int tm = form == 1 ? 64 : 128, tn = form == 3 ? 128 : 64;
   const dim3 grid((unsigned)((long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn))), block(256);
-  if (form == 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 2, 2, 5>), grid, block, 0, stream, p);
+  if (p.nsplit > 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 2, 2, 5, true>), grid, block, 0, stream, p);
+  else if (form == 1) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 2, 2, 5>), grid, block, 0, stream, p);
   else if (form == 2) hipLaunchKernelGGL((gemm_mid_kernel<EPI, 4, 2, 3>), grid, block, 0, stream, p);
   else hipLaunchKernelGGL((gemm_mid_kernel<EPI, 4, 4, 4>), grid, block, 0, stream, p);
   RT_LAUNCH_CHECK();

@@ -54,10 +54,10 @@ def splitk_plan(M: int, N: int, K: int, act: int = 0):
 
 
 def small_tiles(M: int, N: int, K: int, act: int) -> bool:
-    """Whether 65 to 512 rows of an encoder's product (one with a bias) take 64x64 tiles without a K split (rt_gemm_big's planner
-    picks them): 2.6 us and 0.19 a K-step for every tile of a CU, where a split product and its reduction take 14, from K = 2048
-    on 17. Decoders' products stay with the split, which their norms and attention sum themselves."""
-    if M <= 64 or K % 64 or K > 3072 or act not in (0, ACT_IDS["gelu"]):
+    """Whether 65 to 512 rows of an encoder's product (one with a bias) take 64x64 tiles, which sum the parts of a K split
+    themselves (the same bits): 2.6 us and 0.19 a K-step for every tile of a CU, where a split product and its reduction take
+    14, from K = 2048 on 17. Decoders' products stay with the split, which their norms and attention sum themselves."""
+    if M <= 64 or M > 512 or K % 64 or K > 3072 or act not in (0, ACT_IDS["gelu"]):
         return False
     rounds = ((M + 63) // 64 * ((N + 63) // 64) + 255) // 256
     return 2.6 + rounds * (0.19 * (K // 64) + (1.7 if act else 0.4)) < (17 if K > 2048 else 14)
@@ -118,10 +118,11 @@ def gemm(x: torch.Tensor, w: torch.Tensor, u=None, ub=None, bias=None, act=0, ou
             s, bn = max(s, 2), 128
         if nsplit:
             s = nsplit
-        elif bias is not None and not out_f32 and u is None and M <= 512 and small_tiles(M, N, K, act):
-            s, bn = 1, 0
         if u is not None or out_f32 or N % 16:
             s = 1
+        if bias is not None and not nsplit and not out_f32 and u is None and max(x.stride(0), w.stride(0)) < 1 << 22 \
+                and small_tiles(M, N, K, act):
+            return native().gemm_big(x, w, ROW, ROW, None, None, bias, act, 0, s, out, None, residual, 0)
         if s > 1:
             slabs = torch.empty(s * M * N, dtype=torch.float32, device=x.device)
             return native().gemm_splitk(x, w, s, slabs, bias, act, out, residual, bn or 256)

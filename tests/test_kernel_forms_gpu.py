@@ -410,20 +410,25 @@ def test_smaller_tiles_have_the_tile_kernels_bits(form, M, N, K, act, res):
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("M,N,K,act", [(65, 384, 384, 0), (300, 384, 1536, 0), (512, 768, 3072, 0), (130, 272, 768, 2),
-                                       (700, 400, 768, 0), (6000, 768, 1536, 0), (22000, 768, 1536, 0)])
-def test_encoder_products_are_summed_alike_from_65_rows_on(M, N, K, act):
-    """No split of K, whatever tiles the planner takes for a product with a bias, or for the rows behind its large tiles."""
+@pytest.mark.parametrize("M,N,K,act,s", [(65, 384, 384, 0, 1), (300, 384, 1536, 0, 3), (512, 768, 3072, 0, 6), (130, 272, 768, 2, 1),
+                                         (500, 272, 1088, 2, 2), (90, 48, 2560, 0, 5), (700, 400, 768, 0, 1), (6000, 768, 1536, 0, 1),
+                                         (22000, 768, 1536, 0, 1)])
+def test_encoder_products_on_smaller_tiles_are_summed_as_before(M, N, K, act, s):
+    """The parts of K in their order up to 512 rows, no parts beyond, whatever tiles the planner takes for a product with a
+    bias, or for the rows behind its large tiles."""
+    from rag_tl_domainllm_optimizer_amd.ops.linear import small_tiles, splitk_plan
     g = torch.Generator(device=DEV).manual_seed(M)
 
     def r(*s):
         return torch.randn(*s, generator=g, device=DEV).bfloat16()
     x, w, b = r(M, K), r(N, K) * 0.1, r(N)
-    from rag_tl_domainllm_optimizer_amd.ops.linear import small_tiles
-    assert M > 512 or small_tiles(M, N, K, act)
+    assert splitk_plan(M, N, K, act)[0] == s and small_tiles(M, N, K, act) == (M <= 512)
     got = ops.linear(x, w, b, act="gelu" if act else None)
     with ops.tuning(gemm_duo=0, gemm_mid=0):
-        want = ops.native().gemm_big(x, w, 0, 0, None, None, b, act, 0, 1, None, None, None)
+        if s > 1:
+            want = ops.native().gemm_splitk(x, w, s, torch.empty(s * M * N, device=DEV), b, act, None, None, 256)
+        else:
+            want = ops.native().gemm_big(x, w, 0, 0, None, None, b, act, 0, 1, None, None, None)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
