@@ -1302,7 +1302,7 @@ static KParts k_parts(int64_t M, int64_t N, int64_t K, int64_t act) {
   return k;
 }
 
-// act(x w^T + bias); with a norm (res, lw, lb; at most 32 rows) of LN(x + res), which is returned second
+// act(x w^T + bias); with a norm (res, lw, lb) of LN(x + res), which is returned second
 std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Tensor>& bias, int64_t act, const optional<Tensor>& res,
                              const optional<Tensor>& lw, const optional<Tensor>& lb, double eps) {
   for (const Tensor* t : {&x, &w}) {
@@ -1311,7 +1311,7 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
   }
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   TORCH_CHECK(w.size(1) == K, "few_rows: K mismatch");
-  TORCH_CHECK(M <= 64, "few_rows: up to 64 rows");
+  TORCH_CHECK(M <= 32, "few_rows: up to 32 rows");
   auto vec = [&](const optional<Tensor>& t, int64_t n) {
     if (!t) return;
     CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ALIGN16(*t);
@@ -1411,11 +1411,16 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
     const bool own = M <= 32 && (M <= 16 || std::max(k_parts(M, 3 * H, H, 0).n, k_parts(M, F, H, 2).n) <= 4);
     Tensor qkv = rows(3 * H), f = rows(F), d = rows(H), z = rows(H);
     auto product = [&](const Tensor& in, const Tensor& w, const Tensor& b, int act, Tensor& y) {
-      if (M > 32 && w.size(1) > 2048) {  // 40 / 64 rows by 768 x 3072: 13.9 / 14.5 us, 15.6 / 18.5 as few rows
-        gemm(in, w, std::nullopt, std::nullopt, b, act, false, y, std::nullopt, 0.0, false, {});
+      const KParts kp = k_parts(M, w.size(0), w.size(1), act);
+      // few rows / 64 x 64 tiles, 64 rows by 1152 x 384, 384 x 1536, 768 x 3072: 7.9 / 4.5, 8.3 / 8.2, 18.5 / 13.4 us; with GELU by
+      // 1536 x 384 (gemm) 16.2 / 5.8
+      if (M > 32) {
+        if (kp.n <= w.size(1) / 64)
+          gemm_big(in, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, kp.n, y, std::nullopt, std::nullopt, 0, {});
+        else
+          gemm(in, w, std::nullopt, std::nullopt, b, act, false, y, std::nullopt, 0.0, false, {});
         return;
       }
-      const KParts kp = k_parts(M, w.size(0), w.size(1), act);
       check_rc(rt_few_rows(in.data_ptr(), in.size(1), nullptr, 0, nullptr, nullptr, nullptr, w.data_ptr(), w.size(1), b.data_ptr(),
                            y.data_ptr(), y.size(1), (int)M, (int)w.size(0), (int)w.size(1), act, 0.f, kp.n, kp.grp, st),
                "encoder: product");
@@ -1677,7 +1682,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
         py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
         py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
-  m.def("few_rows", &few_rows, "act(x w^T + b) of up to 64 rows, up to 32 normalised first if asked", py::arg("x"), py::arg("w"),
+  m.def("few_rows", &few_rows, "act(x w^T + b) of up to 32 rows, normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);
   m.def("attn_fwd", &attn_fwd);

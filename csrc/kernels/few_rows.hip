@@ -9,8 +9,8 @@
 // wave, under those loads (12 KB from L2, where a kernel of its own costs a launch and another trip); workgroup 0 also writes them.
 // Bound by latency. 15 rows, us,
 // gemm_decode_kernel -> this: 1152 x 384 5.2 -> 4.0, 1536 x 384 with GELU 5.8 -> 4.4, 384 x 1536 9.8 -> 5.2, and 2.9 of the norm
-// with it; 20 rows, gemm_m64_kernel or the wide one: 6.6 -> 4.9, 11.0 -> 5.3, 21.3 -> 7.1; 64 rows: 6.9 -> 7.9, 16.2 -> 8.3, 21.7 ->
-// 10.6.
+// with it; 20 rows, gemm_m64_kernel or the wide one: 6.6 -> 4.9, 11.0 -> 5.3, 21.3 -> 7.1. From 33 rows on gemm_mid_kernel's tiles
+// are ahead.
 #include "rt_common.h"
 #include "rt_gelu.h"
 
@@ -35,7 +35,7 @@ template <int RT, int NW, int TR>
 __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
   constexpr int LDX = NW * 512 + 8;  // K <= 512 NW; an odd number of 16-B chunks where K is a multiple of 16
   __shared__ __attribute__((aligned(16))) bf16_t xs[NW ? TR * 16 * LDX : 8];
-  __shared__ f32x4 red[RT == 4 ? 32 : 16][64];  // [part][column group][row tile]
+  __shared__ f32x4 red[16][64];  // [part][column group][row tile]
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int nc = p.K / 64, CG = 8 / (p.ks * p.rs), RTS = p.rs * RT;  // column groups, row tiles of the workgroup
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
   const bool on = n0 < p.N && rs * RT * 16 < p.M;
   auto begin = [&](int part) { return 2 * (part * nc / p.parts); };  // in steps of 32
   const bf16_t* const wp = p.w + (long)min(n0 + r16, p.N - 1) * p.ldw + 8 * g;
-  constexpr int D = RT == 1 ? 12 : RT == 2 ? 8 : 4;  // weight fragments in flight (without a norm in 128 registers)
+  constexpr int D = RT == 1 ? 12 : 8;  // weight fragments in flight (without a norm in 128 registers)
   bf16x8 wf[D];
   int s0 = 0, s1 = 0;
   if (on && ks < p.parts) { s0 = begin(ks); s1 = begin(ks + 1); }
@@ -249,21 +249,21 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
 
 using namespace rt;
 
-// y = act(x w^T + bias), or act(LN(x + res) w^T + bias) with LN(x + res) to xo (lw given; M <= 32, K <= 1024); M <= 64, act 0 or 2
+// y = act(x w^T + bias), or act(LN(x + res) w^T + bias) with LN(x + res) to xo (lw given; K <= 1024); M <= 32, act 0 or 2
 // (GELU). N % 16 == 0, K % 64 == 0; operands 16-B aligned, leading dimensions multiples of 8; up to 8 parts, up to 16 rows 16,
 // a multiple of grp. -1: not for this kernel.
 extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, const void* lw, const void* lb, void* xo, const void* w,
                            long ldw, const void* bias, void* y, long ldy, int M, int N, int K, int act, float eps, int parts, int grp,
                            hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || N % 16 || K < 64 || K % 64 || (act != 0 && act != 2) || (lw && (M > 32 || K > 1024 || !lb || !res || !xo))) return -1;
+  if (M > 32 || N % 16 || K < 64 || K % 64 || (act != 0 && act != 2) || (lw && (K > 1024 || !lb || !res || !xo))) return -1;
   if (parts < 1 || parts > (M <= 16 ? 16 : 8) || grp < 1 || parts % grp) return -1;
   fr::Args p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.res = (const bf16_t*)res; p.ldr = ldr;
   p.lw = (const bf16_t*)lw; p.lb = (const bf16_t*)lb; p.xo = (bf16_t*)xo;
   p.w = (const bf16_t*)w; p.ldw = ldw; p.bias = (const bf16_t*)bias; p.y = (bf16_t*)y; p.ldy = ldy;
   p.M = M; p.N = N; p.K = K; p.act = act; p.eps = eps; p.parts = parts; p.grp = grp;
-  const int tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  const int tiles = M <= 16 ? 1 : 2;
   p.ks = parts > 4 ? 8 : parts > 2 ? 4 : parts;
   p.rs = std::min(tiles > 1 ? 4 : 1, 8 / p.ks);  // 17..32 rows in one part: rather idle waves than half the workgroups
   const int rt = std::max(tiles / p.rs, 1), cols = 16 * (8 / (p.ks * p.rs)), nw = lw ? (K <= 512 ? 1 : 2) : 0;
@@ -273,8 +273,7 @@ extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, c
   if (nw == 1) { if (tiles == 1) FR(1, 1, 1); else FR(1, 1, 2); }
   else if (nw == 2) { if (tiles == 1) FR(1, 2, 1); else FR(1, 2, 2); }
   else if (rt == 1) FR(1, 0, 0);
-  else if (rt == 2) FR(2, 0, 0);
-  else FR(4, 0, 0);
+  else FR(2, 0, 0);
 #undef FR
   RT_LAUNCH_CHECK();
   return 0;

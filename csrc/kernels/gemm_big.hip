@@ -966,7 +966,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 sum[PARTS ? FM : 1][PARTS ? FN : 1];
-  int part = 0;
+  int part = 0, end = PARTS ? nk / p.nsplit : 0;  // nsplit <= nk (launcher)
   if constexpr (PARTS) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -1002,7 +1002,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][j], fa[kk][i], acc[i][j], 0, 0, 0);
     if constexpr (PARTS) {
-      if (t + 1 == (int)((long)(part + 1) * nk / p.nsplit)) {
+      if (t + 1 == end) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -1011,6 +1011,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mid_kernel(Args p) {
             acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
         ++part;
+        end = (part + 1) * nk / p.nsplit;
       }
     }
   };
