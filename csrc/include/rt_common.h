@@ -159,6 +159,15 @@ __device__ __forceinline__ void ds_read_b64_x4_512(uint32_t a, rt_u32x2 (&r)[4])
       : "memory");
 }
 
+// f over the four lanes 16 apart, neighbours first (the order of __shfl_xor 16, 32)
+template <typename F>
+__device__ __forceinline__ float over_groups(float x, F f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // 2 x (2 reads at a_i + {0, O1})
 template <int O1>
 __device__ __forceinline__ void ds_tr16_2x2(uint32_t a0, uint32_t a1, rt_s16x4& r0, rt_s16x4& r1, rt_s16x4& r2,

@@ -396,15 +396,6 @@ void attn_fwd_kernel(AttnArgs a) {
 // barrier, further tiles (texts beyond 128 tokens) through registers. The bias of a tile's 191 differences lies in LDS and is
 // read once per difference, not per score. 256 texts of 18 to 162 tokens, 12 heads of 64 with the bias: 90 -> 55 us (before: a branch
 // and a wait per score for the bias; 111 where the texts are sorted); 256 texts of 100 to 122, 12 heads of 32: 33 -> 25.
-// f over the four lanes 16 apart, neighbours first (the order of __shfl_xor 16, 32)
-template <typename F>
-__device__ __forceinline__ float over_groups(float x, F f) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 template <int D, bool RB>
 __global__ __launch_bounds__(256, D == 128 ? 2 : D == 64 ? 3 : 4) void attn_packed_kernel(AttnArgs a) {
   constexpr int NCH = D / 8, DS = D / 32, DT = D / 16;

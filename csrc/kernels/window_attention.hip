@@ -160,21 +160,20 @@ static Score make_score(float scale, float cap) {
   const float l2e = 1.4426950408889634f;
   return cap > 0.f ? Score{2.f * l2e * scale / cap, cap * l2e} : Score{scale * l2e, 0.f};
 }
-// Scores under a cap (cap2 at most CAP_MAX) lie within +- cap2: p = 2^(s - cap2 / 4) needs no maximum of the row and stays far
-// from both ends of the range. Where |x| scale / cap is at most 0.4 for all of a tile, tanh is t (c0 + c1 t^2 + ..): minimax over
-// that interval, 1.9e-8 from tanh there, where cap2 - 2 cap2 rcp(1 + 2^y) in fp32 is up to 1e-7 off.
-constexpr float CAP_MAX = 80.f, TANH_T = 0.4f;
+// Where |x| scale / cap is at most 0.4 for all of a wave's tile, the capped score is t (c0 + c1 t^2 + ..) cap2: minimax over that
+// interval, 2.1e-8 from tanh there, where cap2 - 2 cap2 rcp(1 + 2^y) in fp32 is up to 1e-7 off. (2^(s - constant) without a row's
+// maximum, which a cap allows, rounds its heaviest probability to bf16, where 2^0 is exact: errors 1.14 to 1.34 times as large.)
+constexpr float TANH_T = 0.4f;
 struct CapScore {
-  float t, c0, c1, c2, c3, shift;  // t = scale / cap; c's times cap2
+  float t, c0, c1, c2, c3;  // t = scale / cap; c's times cap2
   __device__ __forceinline__ float near(float x) const {
     const float y = x * t, z = y * y;
-    return fmaf(y, fmaf(fmaf(fmaf(c3, z, c2), z, c1), z, c0), -shift);
+    return y * fmaf(fmaf(fmaf(c3, z, c2), z, c1), z, c0);
   }
 };
 static CapScore make_cap_score(float scale, float cap) {
   const double c2 = (double)cap * 1.4426950408889634;
-  return {scale / cap, (float)(0.99999957 * c2), (float)(-0.33329726 * c2), (float)(0.13250565 * c2), (float)(-0.04682564 * c2),
-          (float)(c2 / 4)};
+  return {scale / cap, (float)(0.99999957 * c2), (float)(-0.33329726 * c2), (float)(0.13250565 * c2), (float)(-0.04682564 * c2)};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -380,10 +379,9 @@ __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
 // ---------------------------------------------------------------------------------------------
 // Swapped S^T = K Q^T, P straight into the next MFMA (O^T = V^T P^T), double-buffered K / V tiles by LDS-DMA
 // straight from the pages, one barrier per tile. Bound by the VALU's work on the scores beside 64 MFMAs a tile: with a
-// cap two exponentials and a reciprocal each. So capped scores go without the running maximum (CapScore), most of them
-// with a polynomial for tanh; the pages of 64 tiles are read at once instead of a load that every tile waits for; values
-// are read four column tiles to a wait instead of two. 2 requests of 3700 tokens, 32 heads of 128, cap 50: 460 -> 317 us
-// (510 -> 740 TF/s), of which the order of the tiles 19.
+// cap two exponentials and a reciprocal each. So most capped scores take a polynomial for tanh (CapScore); the pages of 64 tiles are read at once instead of a load that every tile waits for; values
+// are read four column tiles to a wait instead of two. 2 requests of 3700 tokens, 32 heads of 128, cap 50: 407 -> 324 us
+// (550 -> 690 TF/s), of which the order of the tiles 19; without a cap 386 -> 320.
 struct PreArgs {
   const bf16_t* q; long ldq;     // [tokens, ldq], head h at h * D, normed and rotated
   const bf16_t* pool; const int* tab; int max_pages, n_pages, n_rows;
@@ -519,7 +517,7 @@ __global__ __launch_bounds__(256, 2) void window_prefill_kernel(PreArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) stt[t][u][e] = a.score(stt[t][u][e]) - (CAP ? a.near.shift : 0.f);
+          for (int e = 0; e < 4; ++e) stt[t][u][e] = a.score(stt[t][u][e]);
     }
     const int w0 = sg.pos0 + q0, w1 = w0 + 31;  // positions of the wave's rows
     if (!(kv0 + 63 <= w0 && (w1 - kv0 < a.mask.size || kv0 + 63 < a.mask.keep))) {  // not all visible
@@ -531,51 +529,34 @@ __global__ __launch_bounds__(256, 2) void window_prefill_kernel(PreArgs a) {
           for (int e = 0; e < 4; ++e)
             if (!a.mask.sees(w0 + 16 * u + r16, kv0 + 16 * t + 4 * g + e)) stt[t][u][e] = -INFINITY;
     }
-    if constexpr (CAP) {
+    float alpha[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        mx = fmaxf(mx, fmaxf(fmaxf(stt[t][u][0], stt[t][u][1]), fmaxf(stt[t][u][2], stt[t][u][3])));
+      const float mn = fmaxf(m[u], over_groups(mx, [](float x, float y) { return fmaxf(x, y); }));
+      const float mz = mn == -INFINITY ? 0.f : mn;  // a row may see nothing of its first tiles
+      alpha[u] = fexp2(m[u] - mz);
+      m[u] = mn;
+      float rs = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p = fexp2(stt[t][u][e] - mz);
+          stt[t][u][e] = p;
+          rs += p;
+        }
+      l[u] = l[u] * alpha[u] + over_groups(rs, [](float x, float y) { return x + y; });
+    }
+    // O^T: the query is the lane's column, as in the scores (most tiles bring no new maximum)
+    if (__any(alpha[0] != 1.f || alpha[1] != 1.f)) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float p = fexp2(stt[t][u][e]);
-            stt[t][u][e] = p;
-            l[u] += p;  // of the lane's keys
-          }
-    } else {
-      float alpha[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          mx = fmaxf(mx, fmaxf(fmaxf(stt[t][u][0], stt[t][u][1]), fmaxf(stt[t][u][2], stt[t][u][3])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float mn = fmaxf(m[u], mx);
-        const float mz = mn == -INFINITY ? 0.f : mn;  // a row may see nothing of its first tiles
-        alpha[u] = fexp2(m[u] - mz);
-        m[u] = mn;
-        float rs = 0.f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float p = fexp2(stt[t][u][e] - mz);
-            stt[t][u][e] = p;
-            rs += p;
-          }
-        rs += __shfl_xor(rs, 16, 64);
-        rs += __shfl_xor(rs, 32, 64);
-        l[u] = l[u] * alpha[u] + rs;
-      }
-      // O^T: the query is the lane's column, as in the scores (most tiles bring no new maximum)
-      if (__any(alpha[0] != 1.f || alpha[1] != 1.f)) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int c = 0; c < DT; ++c) o[u][c] *= alpha[u];
-      }
+        for (int c = 0; c < DT; ++c) o[u][c] *= alpha[u];
     }
     bf16x8 pa[2][2];
 #pragma unroll
@@ -599,13 +580,6 @@ __global__ __launch_bounds__(256, 2) void window_prefill_kernel(PreArgs a) {
 #pragma unroll
           for (int u = 0; u < 2; ++u) o[u][c + k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pa[ks][u], o[u][c + k], 0, 0, 0);
         }
-    }
-  }
-  if constexpr (CAP) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      l[u] += __shfl_xor(l[u], 16, 64);
-      l[u] += __shfl_xor(l[u], 32, 64);
     }
   }
   __syncthreads();  // the last tile's images become the O staging area
@@ -752,7 +726,7 @@ extern "C" int rt_window_prefill(const void* q, long ldq, const void* pool, cons
   if (!rt_window_prefill_ok(D, V) || G < 1 || H % G || ldq % 8 || ldo % 8 || (uintptr_t)o % 16) return -1;
   PreArgs a{(const bf16_t*)q, ldq, (const bf16_t*)pool, tab, max_pages, n_pages, n_rows, (bf16_t*)o, ldo, (const Seg*)segs,
             (const int2*)tiles, n_tiles, H, G, D, V, make_mask(size, keep), make_score(scale, cap), CapScore{}, out_scale};
-  const bool capped = cap > 0.f && cap * 1.4426950408889634f <= CAP_MAX;
+  const bool capped = cap > 0.f;
   if (capped) a.near = make_cap_score(scale, cap);
   dim3 grid((unsigned)((long)n_tiles * H)), block(256);
 #define WP_C(DQ, DV, C) hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, C>), grid, block, 0, stream, a)

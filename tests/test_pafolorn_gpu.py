@@ -172,6 +172,30 @@ def test_window_prefill_capped_scores(cap, D, V):
         assert (((out[rows, h * V:(h + 1) * V].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6)
 
 
+@pytest.mark.parametrize("cap", [50.0, 35.0, 0.0])
+def test_window_prefill_heaviest_key_is_exact(cap):
+    """Every query sees one key whose weight is 1 but for 2^-15. With the row's maximum ahead of the exponential its probability is
+    exactly 1, in bf16 too, and the result is that key's value: the other keys' share is 2^-13 at most, half an ulp 2^-9."""
+    g = torch.Generator().manual_seed(3)
+    T, H, G, D, V = 1000, 4, 2, 128, 128
+    d = ops.WindowDims(H, G, D, V, D ** -0.5, cap, 0, 0)
+    k = torch.randn(T, G, D, generator=g)
+    k = (k / k.norm(dim=-1, keepdim=True) * D ** 0.5).bfloat16()
+    q = (k.float() * torch.linspace(2.5, 4.0, T)[:, None, None]).bfloat16().repeat_interleave(H // G, 1)
+    v = (torch.randn(T, G, V, generator=g).sign() * (1 + torch.rand(T, G, V, generator=g))).bfloat16()
+    cache = PagedCache([d.cache_width], 1, T, T + 64, DEV, torch.bfloat16)
+    cache.reserve(0, T)
+    cache.sync()
+    cos, sin = torch.ones(cache.max_seq, D // 2, device=DEV), torch.zeros(cache.max_seq, D // 2, device=DEV)  # no rotation
+    out = torch.zeros(T, H * V, dtype=torch.bfloat16, device=DEV)
+    ops.window_attention(torch.cat([q.flatten(1), k.flatten(1), v.flatten(1)], 1).to(DEV), 0, d, None, None, 1e-6, cos, sin,
+                         RaggedBatch.build([(0, [0] * T, 0)], DEV), cache.pool(0), cache.table, out)
+    s = torch.matmul(q.double().transpose(0, 1), k.double().repeat_interleave(H // G, 1).permute(1, 2, 0).contiguous()) * d.scale
+    s = (cap * torch.tanh(s / cap) if cap else s).masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -math.inf)
+    assert (1 - torch.softmax(s, -1).diagonal(dim1=1, dim2=2)).max() < 2.0 ** -15
+    assert torch.equal(out.view(T, H, V).cpu(), v.repeat_interleave(H // G, 1))
+
+
 @pytest.mark.parametrize("T,parts", [(1, 7), (31, 4), (32, 4), (128, 4), (170, 3), (300, 1)])
 @pytest.mark.parametrize("heads", [32, 72])  # one and two tiles of query heads
 def test_window_decode_partitions(T, parts, heads):
