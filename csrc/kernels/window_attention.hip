@@ -160,12 +160,12 @@ static Score make_score(float scale, float cap) {
   const float l2e = 1.4426950408889634f;
   return cap > 0.f ? Score{2.f * l2e * scale / cap, cap * l2e} : Score{scale * l2e, 0.f};
 }
-// Where |x| scale / cap is at most 0.4 for all of a wave's tile, the capped score is t (c0 + c1 t^2 + ..) cap2: minimax over that
+// Where |x scale / cap| is at most 0.4 for all of a wave's tile, the capped score is t (c0 + c1 t^2 + ..) cap2: minimax over that
 // interval, 2.1e-8 from tanh there, where cap2 - 2 cap2 rcp(1 + 2^y) in fp32 is up to 1e-7 off. (2^(s - constant) without a row's
 // maximum, which a cap allows, rounds its heaviest probability to bf16, where 2^0 is exact: errors 1.14 to 1.34 times as large.)
 constexpr float TANH_T = 0.4f;
 struct CapScore {
-  float t, c0, c1, c2, c3;  // t = scale / cap; c's times cap2
+  float t, c0, c1, c2, c3;  // t = scale / cap, of either sign; c's times cap2
   __device__ __forceinline__ float near(float x) const {
     const float y = x * t, z = y * y;
     return y * fmaf(fmaf(fmaf(c3, z, c2), z, c1), z, c0);
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256, 2) void window_prefill_kernel(PreArgs a) {
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(stt[t][u][e]));
-      close = !__any(mx * a.near.t > TANH_T);
+      close = !__any(mx * fabsf(a.near.t) > TANH_T);
     }
     if (close) {
 #pragma unroll

@@ -172,6 +172,30 @@ def test_window_prefill_capped_scores(cap, D, V):
         assert (((out[rows, h * V:(h + 1) * V].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6)
 
 
+@pytest.mark.parametrize("cap", [5.0, 50.0, 0.0])
+def test_window_prefill_negative_scale(cap):
+    """A scale below zero is a scale: products of both signs, well beyond where tanh is a polynomial."""
+    g = torch.Generator().manual_seed(7)
+    T, H, G, D, V = 200, 2, 1, 64, 64
+    d = ops.WindowDims(H, G, D, V, -0.5 * D ** -0.5, cap, 0, 0)
+    q, k, v = (torch.randn(T, n, generator=g).bfloat16() for n in (H * D, G * D, G * V))
+    q *= 4
+    cache = PagedCache([d.cache_width], 1, T, T + 64, DEV, torch.bfloat16)
+    cache.reserve(0, T)
+    cache.sync()
+    cos, sin = torch.ones(cache.max_seq, D // 2, device=DEV), torch.zeros(cache.max_seq, D // 2, device=DEV)  # no rotation
+    out = torch.zeros(T, H * V, dtype=torch.bfloat16, device=DEV)
+    ops.window_attention(torch.cat([q, k, v], 1).to(DEV), 0, d, None, None, 1e-6, cos, sin, RaggedBatch.build([(0, [0] * T, 0)], DEV),
+                         cache.pool(0), cache.table, out)
+    for h in range(H):
+        s = q[:, h * D:(h + 1) * D].double() @ k.double().t() * d.scale
+        s = (cap * torch.tanh(s / cap) if cap else s).masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -math.inf)
+        p = torch.softmax(s, -1)
+        # p and the result round to bf16: half an ulp, 2^-8, each
+        e = (out[:, h * V:(h + 1) * V].double().cpu() - p @ v.double()).abs() - (2.0 ** -7 + 2.0 ** -11) * (p @ v.double().abs())
+        assert e.max() < 1e-6
+
+
 @pytest.mark.parametrize("cap", [50.0, 35.0, 0.0])
 def test_window_prefill_heaviest_key_is_exact(cap):
     """Every query sees one key whose weight is 1 but for 2^-15. With the row's maximum ahead of the exponential its probability is
