@@ -65,6 +65,7 @@ int rt_attn_packed(const void*, long, const void*, long, const void*, long, void
 int rt_few_rows(const void*, long, const void*, long, const void*, const void*, void*, const void*, long, const void*, void*, long,
                 int, int, int, int, float, int, int, hipStream_t);
 int rt_gemm_nt_parts(int, int, int, int*);
+int rt_gemm_plan(int, int, int, int, int*);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
                        float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
@@ -1643,6 +1644,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_store_fp8", &kv_store_fp8, "prompt K/V -> fp8 cache (per-slot scales)");
   m.def("attn_decode_fused_ps", &rt_attn_decode_fused_ps, "keys per partition of the fused decode kernel");
   m.def("quant_fp8", &quant_fp8, "per-row absmax e4m3fn quantisation -> (uint8 [R,C], scale fp32 [R])");
+  m.def("gemm_plan", [](int64_t M, int64_t N, int64_t K, int64_t act) {
+    int form = 0;
+    const int rows = rt_gemm_plan((int)M, (int)N, (int)K, (int)act, &form);
+    return std::make_pair(rows, form);
+  }, "rows of a plain NT product on 256 x 256 tiles (-1: two workgroups per CU) and the tiles of the rest");
   m.def("gemm_big", &gemm_big, "token-parallel GEMM family (NT / NN / TN, LoRA K-extension, split-K, SwiGLU)",
         py::arg("a"), py::arg("b"), py::arg("layout_a"), py::arg("layout_b"), py::arg("a2") = py::none(),
         py::arg("b2") = py::none(), py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("out_mode") = 0,

@@ -1490,68 +1490,85 @@ static int launch_mid(const Args& p, int form, int act, hipStream_t stream) {
   return act == E_GELU ? launch_mid_form<E_GELU>(p, form, stream) : launch_mid_form<E_NONE>(p, form, stream);
 }
 
-// bn = 0: the wave planner over validated arguments p
-static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream) {
-  if (bn != 0) return launch_gemm_big(p, layout_a, layout_b, act, out, bn, stream);
-  const int M = p.M, N = p.N, nsplit = p.nsplit;
+// The launches of a product: rows [0, 256 m1) on 256 x 256 tiles, the rest on 256 x 128 ones (form 0) or gemm_mid_kernel's;
+// m1 < 0: one launch of gemm_duo_kernel
+struct Plan { int m1, form; };
+
+// plain: row-major operands, K % 64 == 0, bf16 result, bias and GELU or no activation (what gemm_duo and gemm_mid take)
+static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128) {
+  const long cus = (long)num_cus() * 1;  // one 512-thread, 128-KiB-LDS workgroup per CU
   // Two workgroups per CU (gemm_duo_kernel) where the reduction is short. With GELU from any number of rows: 19.6 against 32
   // us for 1000 x 1536 x 384, 258 against 306 for 26000 x 4096 x 1024, 827 against 880 for 26000 x 8192 x 2048. Without an
   // activation once every CU has more than one tile (20000 x 1152 x 384: 26.2 against 31.5 us, 10000 x 4096 x 1024: 76 against
   // 86; 2000 x 768 x 768, 36 tiles: 15.9 against 14.8) and up to K = 1024, where it meets gemm_big_kernel (20000 x 4096 x
   // 1024: 156 both; 32000 x 2048 x 1536: 187 against 177).
   const long duo_tiles = (long)((M + 255) / 256) * ((N + 127) / 128);
-  const bool plain = layout_a == ROW && layout_b == ROW && out == O_BF16 && nsplit == 1 && !p.A2 && p.K >= 64 && p.K % 64 == 0 &&
-                     p.lda < (1 << 22) && p.ldb < (1 << 22) && (act == E_NONE || act == E_GELU);  // 32-bit byte offsets within a tile
-  if (plain && tuning().gemm_mid > 1) return launch_mid(p, tuning().gemm_mid - 1, act, stream);
+  if (plain && tuning().gemm_mid > 1) return {0, tuning().gemm_mid - 1};
   // Smaller tiles where they are done sooner: with few rows, and for the rows behind the last full wave of large tiles
   const bool mid = plain && tuning().gemm_mid;
   int form = 0;
   if (tuning().gemm_duo && plain &&
-      (tuning().gemm_duo == 2 || (act == E_GELU && p.K <= 2048) || (act == E_NONE && p.K <= 1024 && duo_tiles > num_cus()))) {
+      (tuning().gemm_duo == 2 || (act == E_GELU && K <= 2048) || (act == E_NONE && K <= 1024 && duo_tiles > cus))) {
     // one tile on a CU, or pairs: 9000 x 1152 x 384 16.5 us, 6500 x 2304 x 768 26.6, 13000 x 2304 x 768 47.0
-    const float nk = (float)(p.K / 64), pairs = (float)duo_tiles / (2.f * num_cus());
+    const float nk = (float)(K / 64), pairs = (float)duo_tiles / (2.f * cus);
     const float duo = pairs <= 0.5f ? 5.3f + 0.73f * nk + (act ? 8.f : 0.f) : std::max(pairs, 1.f) * (9.f + 1.47f * nk + (act ? 10.f : 0.f));
-    if (mid && tuning().gemm_duo == 1 && pairs < 4.f && mid_best(M, N, p.K, act, &form) < 0.95f * duo) return launch_mid(p, form, act, stream);
-    const dim3 grid((unsigned)duo_tiles), block(256);
+    if (mid && tuning().gemm_duo == 1 && pairs < 4.f && mid_best(M, N, K, act, &form) < 0.95f * duo) return {0, form};
+    return {-1, 0};
+  }
+  // ---- plan: m1 row tiles at BN = 256, the rest at BN = 128 ----
+  const int tiles_m = (M + 255) / 256;
+  const int tn256 = act == E_SWIGLU ? N / 256 : (N + 255) / 256;
+  const int tn128 = act == E_SWIGLU ? N / 128 : (N + 127) / 128;
+  Plan p{tiles_m, 0};
+  float best = (float)(((long)tiles_m * tn256 + cus - 1) / cus);  // rounds
+  if (can128) {
+    const float r = bn128_cost();
+    best = 1e30f;
+    for (int m = tiles_m; m >= 0; --m) {
+      const long w256 = ((long)m * tn256 + cus - 1) / cus, w128 = ((long)(tiles_m - m) * tn128 + cus - 1) / cus;
+      const float cost = (float)w256 + r * (float)w128;
+      if (cost < best - 1e-3f) { best = cost; p.m1 = m; }
+    }
+  }
+  if (mid) {
+    const float unit = big_us(K);
+    best *= 0.97f;
+    for (int m = tiles_m; m >= 0; --m) {
+      const long rest = M - (long)m * 256;
+      if (rest <= 0) continue;
+      if (rest * N > cus * 8 * 4096) break;  // more than eight 64 x 64 tiles per CU
+      const float cost = (float)(((long)m * tn256 + cus - 1) / cus) + mid_best(rest, N, K, act, &form) / unit;
+      if (cost < best - 1e-3f) { best = cost; p = {m, form}; }
+    }
+  }
+  return p;
+}
+
+// how many rows of a plain product (see plan_tiles) go on 256 x 256 tiles, and the form of the rest; -1: gemm_duo_kernel
+extern "C" int rt_gemm_plan(int M, int N, int K, int act, int* form) {
+  const Plan p = plan_tiles(M, N, K, act, true, bn128_supported(ROW, ROW, act, O_BF16));
+  *form = p.form;
+  return p.m1 < 0 ? -1 : (int)std::min<long>(M, p.m1 * 256L);
+}
+
+// bn = 0: the wave planner over validated arguments p
+static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream) {
+  if (bn != 0) return launch_gemm_big(p, layout_a, layout_b, act, out, bn, stream);
+  const int M = p.M, N = p.N;
+  const bool plain = layout_a == ROW && layout_b == ROW && out == O_BF16 && p.nsplit == 1 && !p.A2 && p.K >= 64 && p.K % 64 == 0 &&
+                     p.lda < (1 << 22) && p.ldb < (1 << 22) && (act == E_NONE || act == E_GELU);  // 32-bit byte offsets within a tile
+  const Plan pl = plan_tiles(M, N, p.K, act, plain, bn128_supported(layout_a, layout_b, act, out) && p.nsplit == 1 && (out == O_BF16 || out == O_F32));
+  if (pl.m1 < 0) {
+    const dim3 grid((unsigned)((M + 255) / 256 * (long)((N + 127) / 128))), block(256);
     if (act == E_GELU) hipLaunchKernelGGL(gemm_duo_kernel<E_GELU>, grid, block, 0, stream, p);
     else hipLaunchKernelGGL(gemm_duo_kernel<E_NONE>, grid, block, 0, stream, p);
     RT_LAUNCH_CHECK();
     return 0;
   }
   const long lda = p.lda, lda2 = p.lda2, ldc = p.ldc, ldc2 = p.ldc2, ldr = p.ldr;
-  void* C = p.C;
-  const bool can128 = bn128_supported(layout_a, layout_b, act, out);
-  // ---- plan: m1 row tiles at BN = 256, the rest at BN = 128 ----
-  const int tiles_m = (M + 255) / 256;
-  const int tn256 = act == E_SWIGLU ? N / 256 : (N + 255) / 256;
-  const int tn128 = act == E_SWIGLU ? N / 128 : (N + 127) / 128;
-  const long cus = (long)num_cus() * 1;  // one 512-thread, 128-KiB-LDS workgroup per CU
-  int m1 = tiles_m;
-  float best = (float)((long)tiles_m * tn256 + cus - 1) / (float)cus;
-  if (can128 && nsplit == 1 && (out == O_BF16 || out == O_F32)) {
-    const float r = bn128_cost();
-    best = 1e30f;
-    for (int m = tiles_m; m >= 0; --m) {
-      const long w256 = ((long)m * tn256 + cus - 1) / cus, w128 = ((long)(tiles_m - m) * tn128 + cus - 1) / cus;
-      const float cost = (float)w256 + r * (float)w128;
-      if (cost < best - 1e-3f) { best = cost; m1 = m; }
-    }
-  }
-  int tail = 0;  // the form of the rows behind m1 row tiles, 0: 256 x 128
-  if (mid) {
-    const float unit = big_us(p.K);
-    best *= 0.97f;
-    for (int m = tiles_m; m >= 0; --m) {
-      const long rest = M - (long)m * 256;
-      if (rest <= 0) continue;
-      if (rest * N > (long)num_cus() * 8 * 4096) break;  // more than eight 64 x 64 tiles per CU
-      const float cost = (float)(((long)m * tn256 + cus - 1) / cus) + mid_best(rest, N, p.K, act, &form) / unit;
-      if (cost < best - 1e-3f) { best = cost; m1 = m; tail = form; }
-    }
-  }
-  if (m1 == tiles_m) return launch_gemm_big(p, layout_a, layout_b, act, out, 256, stream);
-  const long r0 = (long)m1 * 256;
-  if (m1 > 0) {
+  const long r0 = std::min<long>(M, pl.m1 * 256L);
+  if (r0 == M) return launch_gemm_big(p, layout_a, layout_b, act, out, 256, stream);
+  if (r0 > 0) {
     Args q = p;
     q.M = (int)r0;
     const int rc = launch_gemm_big(q, layout_a, layout_b, act, out, 256, stream);
@@ -1561,11 +1578,11 @@ static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, 
   q.M = M - (int)r0;
   q.A = p.A + (layout_a == ROW ? r0 * lda : r0);
   if (p.A2) q.A2 = p.A2 + (layout_a == ROW ? r0 * lda2 : r0);
-  q.C = (char*)C + r0 * ldc * (out == O_BF16 ? 2 : 4);
+  q.C = (char*)p.C + r0 * ldc * (out == O_BF16 ? 2 : 4);
   if (p.C2) q.C2 = p.C2 + r0 * ldc2;
   if (p.R) q.R = p.R + r0 * ldr;
   if (p.rope_pos) q.rope_pos = p.rope_pos + r0;
-  return tail ? launch_mid(q, tail, act, stream) : launch_gemm_big(q, layout_a, layout_b, act, out, 128, stream);
+  return pl.form ? launch_mid(q, pl.form, act, stream) : launch_gemm_big(q, layout_a, layout_b, act, out, 128, stream);
 }
 
 // Grouped NT product C[r] = epi(A[row_map[r]] B_g^T) over rows sorted by group g (see GRP above): bf16 out,

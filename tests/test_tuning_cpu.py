@@ -71,3 +71,19 @@ def test_tuning_roundtrip():
     assert ops.get_tuning() == t0
     with pytest.raises(KeyError):
         ops.set_tuning(no_such_knob=1)
+
+
+def test_gemm_plan_saves_a_round():
+    """GELU products beyond the two-workgroup form's K: rows leave the 256 x 256 tiles only where those then take a round of
+    workgroups fewer; a product that fills whole rounds stays one launch."""
+    from rag_tl_domainllm_optimizer_amd import ops
+
+    def rounds(rows, N):
+        return ((rows + 255) // 256 * ((N + 255) // 256) + 255) // 256
+
+    for K in (2112, 2560, 3072, 4096, 10240):
+        for N in (768, 1024, 2560, 4096, 6144, 10240, 16384):
+            for M in (513, 700, 1000, 1500, 2100, 3000, 4096, 8192, 10000, 16384, 23500):
+                rows, form = ops.native().gemm_plan(M, N, K, ops.ACT_IDS["gelu"])
+                assert 0 <= rows <= M and (rows == M or (form in (1, 2, 3) and rounds(rows, N) < rounds(M, N))), (M, N, K, rows, form)
+    assert ops.native().gemm_plan(4096, 4096, 4096, ops.ACT_IDS["gelu"])[0] == 4096
