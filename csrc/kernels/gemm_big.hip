@@ -1499,26 +1499,29 @@ static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128) {
   const long cus = (long)num_cus() * 1;  // one 512-thread, 128-KiB-LDS workgroup per CU
   // Two workgroups per CU (gemm_duo_kernel) where the reduction is short. With GELU from any number of rows: 19.6 against 32
   // us for 1000 x 1536 x 384, 258 against 306 for 26000 x 4096 x 1024, 827 against 880 for 26000 x 8192 x 2048. Without an
-  // activation once every CU has more than one tile (20000 x 1152 x 384: 26.2 against 31.5 us, 10000 x 4096 x 1024: 76 against
-  // 86; 2000 x 768 x 768, 36 tiles: 15.9 against 14.8) and up to K = 1024, where it meets gemm_big_kernel (20000 x 4096 x
-  // 1024: 156 both; 32000 x 2048 x 1536: 187 against 177).
+  // activation once 256 x 256 tiles take more than a round (20000 x 1152 x 384: 26.2 against 31.5 us, 10000 x 4096 x 1024: 75
+  // against 84; in one round 4096 x 4096 x 1024 33.5 against 31.7, 4500 x 3072 x 768 26.0 against 24.7, 10000 x 1152 x 384 16.5
+  // and 16.4) and up to K = 1024, where it meets gemm_big_kernel (20000 x 4096 x 1024: 156 both; 32000 x 2048 x 1536: 187
+  // against 177).
   const long duo_tiles = (long)((M + 255) / 256) * ((N + 127) / 128);
   if (plain && tuning().gemm_mid > 1) return {0, tuning().gemm_mid - 1};
   // Smaller tiles where they are done sooner: with few rows, and for the rows behind the last full wave of large tiles
   const bool mid = plain && tuning().gemm_mid;
   int form = 0;
+  const int tiles_m = (M + 255) / 256;
+  const int tn256 = act == E_SWIGLU ? N / 256 : (N + 255) / 256;
+  const int tn128 = act == E_SWIGLU ? N / 128 : (N + 127) / 128;
   if (tuning().gemm_duo && plain &&
       (tuning().gemm_duo == 2 || (act == E_GELU && K <= 2048) || (act == E_NONE && K <= 1024 && duo_tiles > cus))) {
     // one tile on a CU, or pairs: 9000 x 1152 x 384 16.5 us, 6500 x 2304 x 768 26.6, 13000 x 2304 x 768 47.0
     const float nk = (float)(K / 64), pairs = (float)duo_tiles / (2.f * cus);
     const float duo = pairs <= 0.5f ? 5.3f + 0.73f * nk + (act ? 8.f : 0.f) : std::max(pairs, 1.f) * (9.f + 1.47f * nk + (act ? 10.f : 0.f));
-    if (mid && tuning().gemm_duo == 1 && pairs < 4.f && mid_best(M, N, K, act, &form) < 0.95f * duo) return {0, form};
-    return {-1, 0};
+    const bool round = act == E_NONE && (long)tiles_m * tn256 <= cus && tuning().gemm_duo == 1;  // 16 us at K = 384, 24, 28 at 1024
+    const float large = round ? 10.f + 0.0185f * (float)K : 0.95f * duo;
+    if (mid && tuning().gemm_duo == 1 && pairs < 4.f && mid_best(M, N, K, act, &form) < large) return {0, form};
+    return {round ? tiles_m : -1, 0};
   }
   // ---- plan: m1 row tiles at BN = 256, the rest at BN = 128 ----
-  const int tiles_m = (M + 255) / 256;
-  const int tn256 = act == E_SWIGLU ? N / 256 : (N + 255) / 256;
-  const int tn128 = act == E_SWIGLU ? N / 128 : (N + 127) / 128;
   Plan p{tiles_m, 0};
   float best = (float)(((long)tiles_m * tn256 + cus - 1) / cus);  // rounds
   if (can128) {

@@ -87,3 +87,16 @@ def test_gemm_plan_saves_a_round():
                 rows, form = ops.native().gemm_plan(M, N, K, ops.ACT_IDS["gelu"])
                 assert 0 <= rows <= M and (rows == M or (form in (1, 2, 3) and rounds(rows, N) < rounds(M, N))), (M, N, K, rows, form)
     assert ops.native().gemm_plan(4096, 4096, 4096, ops.ACT_IDS["gelu"])[0] == 4096
+
+
+@pytest.mark.parametrize("K", [384, 768, 1024])
+def test_gemm_plan_of_one_round(K):
+    """Without an activation a product that 256 x 256 tiles take in one round of workgroups is not cut to the two-workgroup form,
+    which is behind there; beyond a round it is."""
+    from rag_tl_domainllm_optimizer_amd import ops
+
+    for M, N in ((10000, 1024), (16384, 1024), (16384, 768), (4096, 4096), (3000, 4096), (4500, 3072), (10000, 1152)):
+        rows, form = ops.native().gemm_plan(M, N, K, 0)
+        assert rows == M or (rows == 0 and form), (M, N, rows, form)
+    for M, N in ((23500, 1152), (8192, 3072), (8192, 4096), (23500, 1024)):
+        assert ops.native().gemm_plan(M, N, K, 0)[0] == -1, (M, N)
