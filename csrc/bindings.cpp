@@ -95,7 +95,8 @@ int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
 int rt_segment_mean(const float*, int, const long*, const int*, int, int, float*, hipStream_t);
-int rt_ivf_scan(const void*, int, int, const int*, int, int, const int*, const int*, const void*, const long*, const float*,
+int rt_ivf_by_list(int, int, int, int, int, long);
+int rt_ivf_scan(const void*, int, int, const int*, int, int, const int*, const int*, const void*, long, const long*, const float*,
                 int, int, float*, long*,
                 hipStream_t);
 int rt_gae(const float*, const float*, const float*, int, int, float, float, float*, float*, hipStream_t);
@@ -1492,7 +1493,7 @@ std::vector<Tensor> ivf_scan(const Tensor& q_, const Tensor& probes, const Tenso
   auto cand = at::empty({nq, nprobe * maxlen}, q.options().dtype(at::kFloat));
   auto cid = at::empty({nq, nprobe * maxlen}, q.options().dtype(at::kLong));
   check_rc(rt_ivf_scan(q.data_ptr(), (int)nq, (int)d, probes.data_ptr<int>(), (int)nprobe, (int)lsize.numel(), lstart.data_ptr<int>(),
-                       lsize.data_ptr<int>(), vecs.data_ptr(), (const long*)ids.data_ptr(),
+                       lsize.data_ptr<int>(), vecs.data_ptr(), vecs.size(0), (const long*)ids.data_ptr(),
                        l2 ? sqnorm->data_ptr<float>() : nullptr, l2 ? 1 : 0, (int)maxlen, cand.data_ptr<float>(),
                        (long*)cid.data_ptr(), cur_stream()),
            "ivf_scan");
@@ -1711,6 +1712,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pool_norm", &pool_norm, py::arg("x"), py::arg("lengths"), py::arg("normalize"), py::arg("off") = py::none());
   m.def("topk", &topk, py::arg("scores"), py::arg("k"), py::arg("idmap") = py::none(), py::arg("finite") = false);
   m.def("ivf_scan", &ivf_scan);
+  m.def("ivf_by_list", [](int64_t nq, int64_t nprobe, int64_t nlist, int64_t d, int64_t maxlen, int64_t total) {
+    return rt_ivf_by_list((int)nq, (int)nprobe, (int)nlist, (int)d, (int)maxlen, (long)total) != 0;
+  }, "whether a scan reads a list's vectors once for all its queries");
   m.def("segment_mean", &segment_mean, "k-means update: per-segment mean of sorted rows (+ L2 normalise)");
   m.def("gae", &gae);
   m.def("ppo_advantages", &ppo_advantages, "token KL rewards + GAE + advantage whitening in one launch");

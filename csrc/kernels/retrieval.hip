@@ -7,6 +7,7 @@
 #include "rt_common.h"
 
 #include <algorithm>
+#include <climits>
 
 namespace rt {
 
@@ -245,50 +246,200 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
 // spare capacity for incremental adds) and write into cand[qi, p*maxlen + j] (+ ids).
 // Metric: inner product, or (l2) the negated squared distance 2 q.x - |x|^2 - |q|^2 with |x|^2
 // stored per slot — both "higher is better" for the shared top-k. Unused slots get -inf, and so do probes of no list.
-// A wave multiplies 16 vectors, held as MFMA fragments (64 B of 16 vectors a load), with 16 queries at a time; a thread per vector
-// had each 16-byte load of a wave touch 64 lines, of which L1 kept none for the next one. BY_LIST: a workgroup takes 64
-// vectors of a list for every query that probes it, found among the probes, PAIRS at a time; else for one (query, probe).
-// Bound by the bytes read and written (12 a candidate). us, the thread per vector -> this: 64 queries over lists of up to 102108
-// vectors of 384 (200k in all) 9500 -> 724, 100 queries over 30k 2473 -> 202, one query over 16 lists of 200 10.5 -> 8.
-constexpr int PAIRS = 4096;
 struct ScanArgs {
   const bf16_t* q; int nq, d; const int* probes; int nprobe, nlist;
   const int* lstart; const int* lsize; const bf16_t* vecs; const long* ids; const float* sqnorm;
-  int l2, maxlen;
+  int l2, maxlen, per;  // per: vectors of a workgroup at least (by list)
   float* cand; long* cand_ids;
 };
+// 8 elements a lane from a uniform base + off bytes, 0 beyond `bytes` (at most 2^30; FAR lies beyond)
+constexpr uint32_t FAR = 0x60000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t scan_rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ bf16x8 scan_load(__amdgpu_buffer_rsrc_t r, uint32_t off, int base) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, base, 0));
+}
 
-template <int NF, bool BY_LIST>  // NF: 32-element fragments of a vector held at once
-__global__ __launch_bounds__(256) void ivf_scan_kernel(ScanArgs a) {
-  __shared__ int pair[BY_LIST ? PAIRS : 1];  // query * nprobe + probe, from the round's first one
+// By probe: one wave per 64 vectors of a (probe, query), one thread per vector, query in LDS: a single query's 16 lists of 200 to
+// 800 are a few hundred waves on as many CUs, where one workgroup per list left 240 CUs idle; 8 of a vector's 16-byte
+// pieces are in flight (16 lists of 600 x 384: 12.4 -> 8.6 us). A vector's terms are summed in the order of the
+// dimensions.
+__global__ __launch_bounds__(64) void ivf_probe_kernel(const bf16_t* __restrict__ q, int d, const int* __restrict__ probes,
+                                                       int nprobe, int nlist, const int* __restrict__ lstart,
+                                                       const int* __restrict__ lsize, const bf16_t* __restrict__ vecs,
+                                                       const long* __restrict__ ids, const float* __restrict__ sqnorm,
+                                                       int l2, int maxlen, float* __restrict__ cand,
+                                                       long* __restrict__ cand_ids) {
+  extern __shared__ float qs[];
+  const int p = blockIdx.x, qi = blockIdx.y;
+  const long j0 = blockIdx.z * 64L, step = gridDim.z * 64L;
+  const int L = probes[(long)qi * nprobe + p];
+  const bool real = L >= 0 && L < nlist;
+  const int b0 = real ? lstart[L] : 0;
+  const int len = real ? min(lsize[L], maxlen) : 0;
+  float* out = cand + ((long)qi * nprobe + p) * maxlen;
+  long* oid = cand_ids + ((long)qi * nprobe + p) * maxlen;
+  if (j0 >= len) {
+    for (long j = j0 + threadIdx.x; j < maxlen; j += step) { out[j] = -INFINITY; oid[j] = -1; }
+    return;
+  }
+  // |q|^2 in four interleaved parts, added in order
+  float part[4] = {};
+  for (int i0 = threadIdx.x; i0 < d; i0 += 256) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int i = i0 + 64 * w;
+      if (i >= d) continue;
+      const float v = bf2f(q[(long)qi * d + i]);
+      qs[i] = v;
+      part[w] += v * v;
+    }
+  }
+  float qn = 0.f;
+  if (l2) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) qn += wave_sum(part[w]);
+  }
+  __syncthreads();
+  for (long j = j0 + threadIdx.x; j < maxlen; j += step) {
+    if (j >= len) {
+      out[j] = -INFINITY;
+      oid[j] = -1;
+      continue;
+    }
+    const bf16_t* vr = vecs + (b0 + j) * d;
+    float s = 0.f;
+    int c = 0;
+    for (; c + 64 <= d; c += 64) {
+      uint4 v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = *(const uint4*)(vr + c + 8 * i);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float f[8];
+        unpack8(v[i], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += f[e] * qs[c + 8 * i + e];
+      }
+    }
+    for (; c < d; c += 8) {
+      float f[8];
+      unpack8(*(const uint4*)(vr + c), f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += f[e] * qs[c + e];
+    }
+    out[j] = l2 ? 2.f * s - sqnorm[b0 + j] - qn : s;
+    oid[j] = ids[b0 + j];
+  }
+}
+
+// The same of 256 < d <= 384 and lists that are even or at most 4096 long: a wave per 16 vectors, whose pieces are all in flight as MFMA fragments at once, the query as the other
+// operand's sixteen rows. A single query over 16 lists of 200 and of 780, 7.3 -> 5.2 and 7.5 -> 5.8 us; many queries over
+// lists of 100 20.3 -> 16.4 (64 x 16 of 4096), 53 -> 49 (256 x 16). Smaller d leaves the wave with too little in flight (128: 1.3 to 1.5 times
+// the time), 768 takes half the waves away (1.0 to 1.15 times); one and two queries over skewed
+// lists of up to 7909 16.7 against 15.9 and 29.7 against 27.6, over even ones of up to 8735 11.1 against 12.3 and 18.5 against 19.6.
+constexpr int PF = 12;
+__global__ __launch_bounds__(256, 4) void ivf_probe16_kernel(ScanArgs a) {
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long pr = (long)blockIdx.y * a.nprobe + blockIdx.x;
+  const int L = a.probes[pr];
+  const bool real = L >= 0 && L < a.nlist;
+  const int b0 = real ? a.lstart[L] : 0, len = real ? max(min(a.lsize[L], a.maxlen), 0) : 0;
+  const int z0 = blockIdx.z, zn = gridDim.z;
+  if (z0 * 64L >= len && len + z0 * 256L >= a.maxlen) return;  // no vectors here and no slots to fill
+  float* const out = a.cand + pr * a.maxlen;
+  long* const oid = a.cand_ids + pr * a.maxlen;
+  for (long j = len + z0 * 256L + tid; j < a.maxlen; j += zn * 256L) {
+    out[j] = -INFINITY;
+    oid[j] = -1;
+  }
+  bf16x8 y[PF];
+  const auto qr = scan_rsrc(a.q + (long)blockIdx.y * a.d, (uint32_t)a.d * 2);
+#pragma unroll
+  for (int s = 0; s < PF; ++s) y[s] = scan_load(qr, 16 * g, 64 * s);
+  float qq = 0.f;
+  if (a.l2) {
+#pragma unroll
+    for (int s = 0; s < PF; ++s) {
+      float f[8];
+      unpack8(__builtin_bit_cast(uint4, y[s]), f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qq = fmaf(f[e], f[e], qq);
+    }
+    qq += __shfl_xor(qq, 16, 64);
+    qq += __shfl_xor(qq, 32, 64);
+  }
+  for (long v0 = z0 * 64L + wid * 16; v0 < len; v0 += zn * 64L) {
+    const auto vr = scan_rsrc(a.vecs + (b0 + v0) * a.d, (uint32_t)min(16L, len - v0) * a.d * 2);
+    uint32_t vo = (uint32_t)(r16 * a.d + 8 * g) * 2;
+    asm volatile("" : "+v"(vo));  // the offsets below are not worth a register each
+    bf16x8 x[PF];
+#pragma unroll
+    for (int s = 0; s < PF; ++s) x[s] = scan_load(vr, 32 * s + 8 * g < a.d ? vo : FAR, 64 * s);
+    const long at = b0 + min(v0 + r16, (long)len - 1);
+    const long id = a.ids[at];
+    const float sq = a.l2 ? a.sqnorm[at] : 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < PF; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y[s], x[s], acc, 0, 0, 0);
+    // every row of the product is the query's: column r16 is vector v0 + r16
+    if (g == 0 && v0 + r16 < len) {
+      out[v0 + r16] = a.l2 ? 2.f * acc[0] - sq - qq : acc[0];
+      oid[v0 + r16] = id;
+    }
+  }
+}
+
+// By list: 64 vectors of a list and more for every query that probes it, found among the probes; a wave multiplies 16 vectors, held as
+// MFMA fragments, with 16 queries at a time. Bound by the bytes read and written (12 a candidate), by reading the
+// probes where lists are many and short, and by the chain from probe to result where a list has few queries. us, by probe -> by list: 64 queries
+// x 16 of 512 lists, 100k vectors of 384 28.6 -> 20.5, 256 queries 84 -> 27; 4 and 12 queries x 16 of 256 lists of up to 7909 48.8 -> 29.9,
+// 100 -> 36; 4096 queries x 32 of 4096 lists of about 100 1335 -> 555. (With the probes taken 4096 at a time a list of those
+// had one query a round and read its vectors 32 times: 1690.)
+constexpr int PAIRS = 4096;
+// NF: 32-element fragments of a vector held at once; LONG: a vector has more
+template <int NF, bool LONG>
+__global__ __launch_bounds__(256, NF == 12 ? 4 : 2) void ivf_list_kernel(ScanArgs a) {
+  __shared__ uint32_t pair[PAIRS];  // query * nprobe + probe, from the round's first one
   __shared__ int count;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const long all = BY_LIST ? (long)a.nq * a.nprobe : 1, first = BY_LIST ? 0 : (long)blockIdx.y * a.nprobe + blockIdx.x;
-  const int L = BY_LIST ? blockIdx.x : a.probes[first];  // BY_LIST: nlist stands for no list
-  const bool real = L >= 0 && L < a.nlist;
-  const int b0 = real ? a.lstart[L] : 0, len = real ? min(a.lsize[L], a.maxlen) : 0;
-  const int z0 = blockIdx.z, zn = gridDim.z;
-  if (z0 * 64L >= len && len + z0 * 256L >= a.maxlen) return;  // no vectors here and no slots to fill
-  for (long base = 0; base < all; base += PAIRS) {
-    int n = 1;
-    if constexpr (BY_LIST) {
-      const int m = (int)min(all - base, (long)PAIRS);
-      __syncthreads();  // the last round's pairs have been read
-      if (tid == 0) count = 0;
-      __syncthreads();
-      for (int i0 = tid; i0 < m; i0 += 256 * 8) {
-        int l[8];
+  const int L = blockIdx.x;  // nlist stands for no list
+  const bool real = L < a.nlist;
+  const int b0 = real ? a.lstart[L] : 0, len = real ? max(min(a.lsize[L], a.maxlen), 0) : 0;
+  // the list's workgroups, one at least, which fills an empty one's slots; the others need not look for its queries
+  const int z0 = blockIdx.z, zn = min((int)gridDim.z, max((len + a.per - 1) / a.per, 1));
+  if (z0 >= zn) return;
+  // the probes from base on, m of them, that ask for this list: their number, the first PAIRS of them in pair[]
+  auto collect = [&](long base, long m) {
+    __syncthreads();  // the last pairs and their number have been read
+    if (tid == 0) count = 0;
+    __syncthreads();
+    for (long i0 = tid; i0 < m; i0 += 256 * 16) {
+      int l[16];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) l[e] = a.probes[base + min(i0 + e * 256, m - 1)];
+      for (int e = 0; e < 16; ++e) l[e] = a.probes[base + min(i0 + e * 256, m - 1)];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (i0 + e * 256 < m && (real ? l[e] == L : l[e] < 0 || l[e] >= a.nlist)) pair[atomicAdd(&count, 1)] = i0 + e * 256;
-      }
-      __syncthreads();
-      n = count;
+      for (int e = 0; e < 16; ++e)
+        if (i0 + e * 256 < m && (real ? l[e] == L : l[e] < 0 || l[e] >= a.nlist)) {
+          const int at = atomicAdd(&count, 1);
+          if (at < PAIRS) pair[at] = (uint32_t)(i0 + e * 256);
+        }
     }
-    auto pair_of = [&](int k) { return BY_LIST ? base + pair[k] : first; };
+    __syncthreads();
+    return count;
+  };
+  // a round has all probes, unless more than PAIRS of them ask for this list
+  const long all = (long)a.nq * a.nprobe;
+  for (long base = 0, step = min(all, 1L << 30); base < all; base += step) {
+    int n = collect(base, min(all - base, step));
+    if (n > PAIRS) {
+      step = PAIRS;
+      n = collect(base, min(all - base, step));
+    }
+    auto pair_of = [&](int k) { return base + pair[k]; };
     for (int k = 0; k < n; ++k) {  // slots behind the list's vectors
       const long o = pair_of(k) * a.maxlen;
       for (long j = len + z0 * 256L + tid; j < a.maxlen; j += zn * 256L) {
@@ -298,63 +449,64 @@ __global__ __launch_bounds__(256) void ivf_scan_kernel(ScanArgs a) {
     }
     if (n == 0) continue;
     for (long v0 = z0 * 64L + wid * 16; v0 < len; v0 += zn * 64L) {
-      const bf16_t* vr = a.vecs + (b0 + min(v0 + r16, (long)len - 1)) * a.d + 8 * g;
+      const auto vr = scan_rsrc(a.vecs + (b0 + v0) * a.d, (uint32_t)min(16L, len - v0) * a.d * 2);
       bf16x8 x[NF];
       auto load = [&](int c0) {
+        uint32_t vo = (uint32_t)(r16 * a.d + 8 * g) * 2;
+        asm volatile("" : "+v"(vo));  // the offsets below are not worth a register each
 #pragma unroll
-        for (int s = 0; s < NF; ++s) {
-          x[s] = bf16x8{};
-          if (c0 + 32 * s + 8 * g < a.d) x[s] = *(const bf16x8*)(vr + c0 + 32 * s);
-        }
+        for (int s = 0; s < NF; ++s) x[s] = scan_load(vr, c0 + 32 * s + 8 * g < a.d ? vo : FAR, (c0 + 32 * s) * 2);
       };
-      load(0);
-      long id[4];
-      float sq[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {  // of the vectors whose scores the lane holds
-        const long at = b0 + min(v0 + 4 * g + i, (long)len - 1);
-        id[i] = a.ids[at];
-        sq[i] = a.l2 ? a.sqnorm[at] : 0.f;
-      }
+      if constexpr (!LONG) load(0);
+      const long at = b0 + min(v0 + r16, (long)len - 1);
+      const long id = a.ids[at];
+      const float sq = a.l2 ? a.sqnorm[at] : 0.f;
+      const auto qr = scan_rsrc(a.q, (uint32_t)a.nq * a.d * 2);
       for (int t = 0; t < n; t += 16) {
-        const long pr = pair_of(min(t + r16, n - 1));
-        const bf16_t* qr = a.q + pr / a.nprobe * a.d + 8 * g;
+        uint32_t qo = (uint32_t)(pair_of(min(t + r16, n - 1)) / a.nprobe * a.d + 8 * g) * 2;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         float qq = 0.f;
-        for (int c0 = 0; c0 < a.d; c0 += 32 * NF) {
-          if (a.d > 32 * NF && (t > 0 || c0 > 0)) load(c0);
-          bf16x8 y[NF];
+        auto part = [&](int c0) {
 #pragma unroll
-          for (int s = 0; s < NF; ++s) {
-            y[s] = bf16x8{};
-            if (c0 + 32 * s + 8 * g < a.d) y[s] = *(const bf16x8*)(qr + c0 + 32 * s);
-          }
+          for (int s0 = 0; s0 < NF; s0 += 4) {
+            asm volatile("" : "+v"(qo));
+            bf16x8 y[4];
 #pragma unroll
-          for (int s = 0; s < NF; ++s)
-            if (c0 + 32 * s < a.d) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[s], y[s], acc, 0, 0, 0);
-          if (a.l2) {
+            for (int s = 0; s < 4; ++s) y[s] = scan_load(qr, c0 + 32 * (s0 + s) + 8 * g < a.d ? qo : FAR, (c0 + 32 * (s0 + s)) * 2);
 #pragma unroll
-            for (int s = 0; s < NF; ++s) {
-              float f[8];
-              unpack8(__builtin_bit_cast(uint4, y[s]), f);
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y[s], x[s0 + s], acc, 0, 0, 0);
+            if (a.l2) {
 #pragma unroll
-              for (int e = 0; e < 8; ++e) qq = fmaf(f[e], f[e], qq);
+              for (int s = 0; s < 4; ++s) {
+                float f[8];
+                unpack8(__builtin_bit_cast(uint4, y[s]), f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qq = fmaf(f[e], f[e], qq);
+              }
             }
           }
+        };
+        if constexpr (LONG) {
+          for (int c0 = 0; c0 < a.d; c0 += 32 * NF) {
+            load(c0);
+            part(c0);
+          }
+        } else {
+          part(0);
         }
         if (a.l2) {
           qq += __shfl_xor(qq, 16, 64);
           qq += __shfl_xor(qq, 32, 64);
         }
-        // acc[i]: vector v0 + 4 g + i, query r16 of the sixteen
-        if (t + r16 < n && (BY_LIST || r16 == 0)) {
+        // acc[i]: query 4 g + i of the sixteen, vector v0 + r16
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const long j = v0 + 4 * g + i;
-            if (j < len) {
-              a.cand[pr * a.maxlen + j] = a.l2 ? 2.f * acc[i] - sq[i] - qq : acc[i];
-              a.cand_ids[pr * a.maxlen + j] = id[i];
-            }
+        for (int i = 0; i < 4; ++i) {
+          const int k = t + 4 * g + i;
+          const float qn = a.l2 ? __shfl(qq, 4 * g + i, 64) : 0.f;
+          if (k < n && v0 + r16 < len) {
+            const long o = pair_of(k) * a.maxlen + v0 + r16;
+            a.cand[o] = a.l2 ? 2.f * acc[i] - sq - qn : acc[i];
+            a.cand_ids[o] = id;
           }
         }
       }
@@ -419,28 +571,52 @@ extern "C" int rt_topk(const float* scores, long ld, long nq, int N, int k, cons
   return 0;
 }
 
+// Which form a scan takes (total: vectors in all lists, at most). What either takes, in bytes at the rate of a copy: by probe every
+// candidate's vector (and 35 more); by list every vector, 300 for its share of a workgroup's chain, 125 a candidate and a look at
+// every probe for every list. Fitted to 300 calls of 1 to 20000 queries over 1 to 4096 lists, even and skewed, d of 72 to 1024: none
+// of them is slower than by probe. Queries that do not fit a wave's LDS go by list.
+extern "C" int rt_ivf_by_list(int nq, int nprobe, int nlist, int d, int maxlen, long total) {
+  const double P = (double)nq * nprobe, len = std::min(0.7 * maxlen, (double)total);
+  return d > 16384 || (nq > 1 && total * (2. * d + 300) + P * len * 125 + 3.6 * nlist * P + 10e6 < P * len * (2. * d + 35));
+}
+
 extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int nprobe, int nlist, const int* lstart,
-                           const int* lsize, const void* vecs, const long* ids, const float* sqnorm, int l2,
+                           const int* lsize, const void* vecs, long total, const long* ids, const float* sqnorm, int l2,
                            int maxlen, float* cand, long* cand_ids, hipStream_t stream) {
   if (d % 8 != 0 || (l2 && !sqnorm) || (uintptr_t)q % 16 || (uintptr_t)vecs % 16) return -1;
   if (nq == 0 || nprobe == 0) return 0;
   if (maxlen <= 0) return 0;
-  const ScanArgs a{(const bf16_t*)q, nq, d, probes, nprobe, nlist, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, cand, cand_ids};
-  // A list's vectors are read once for all its queries as soon as a list has one on average, or where lists are long: a few
-  // then hold most of the vectors, and every query probes them. Search, us, thread per vector / by probe / by list, longest
-  // lists of 1000 to 4000: 12 queries 125 / 105 / 81, 20 queries 66 / 77 / 60, 24 queries 118 / 148 / 68; by probe it stays where
-  // they are short (8 queries 42 / 42). Long lists go round some thousand workgroups.
-  const bool by_list = (long)nq * nprobe >= nlist || (nq > 4 && maxlen > 1024) || (nq > 1 && maxlen > 4096) || nq > 65535;
-  const long pieces = (maxlen + 63L) / 64, most = by_list ? 64 : std::max(8192L / ((long)nprobe * nq), 8L);
-  const dim3 grid = by_list ? dim3(nlist + 1, 1, (unsigned)std::min(pieces, most)) : dim3(nprobe, nq, (unsigned)std::min(pieces, most));
-#define SCAN(NF)                                                                                   \
-  do {                                                                                             \
-    if (by_list) hipLaunchKernelGGL((ivf_scan_kernel<NF, true>), grid, dim3(256), 0, stream, a);   \
-    else hipLaunchKernelGGL((ivf_scan_kernel<NF, false>), grid, dim3(256), 0, stream, a);          \
-  } while (0)
-  if (d <= 384) SCAN(12);
-  else SCAN(24);
-#undef SCAN
+  if (d > 1 << 24) return -1;
+  const bool by_list = rt_ivf_by_list(nq, nprobe, nlist, d, maxlen, total);
+  // as many queries at once as a grid's second dimension has, or as 32-bit offsets reach
+  const long most_q = by_list ? std::min((1L << 30) / (2L * d), (long)INT_MAX) : 65535;
+  if (nq > most_q) {
+    for (long i = 0; i < nq; i += most_q) {
+      const int rc = rt_ivf_scan((const bf16_t*)q + i * d, (int)std::min(most_q, nq - i), d, probes + i * nprobe, nprobe, nlist, lstart, lsize,
+                                 vecs, total, ids, sqnorm, l2, maxlen, cand + i * nprobe * maxlen, cand_ids + i * nprobe * maxlen, stream);
+      if (rc) return rc;
+    }
+    return 0;
+  }
+  // 64 vectors a workgroup up to some six thousand of them; a long list goes round its own
+  const int per = by_list ? (int)std::max(64L, (total / 6144 + 63) / 64 * 64) : 64;
+  const ScanArgs a{(const bf16_t*)q, nq, d, probes, nprobe, nlist, lstart, lsize, (const bf16_t*)vecs, ids, sqnorm, l2, maxlen, per, cand, cand_ids};
+  // a grid's third dimension ends at 65535: longer lists (over 4 million vectors) go round
+  const long pieces = std::min((maxlen + per - 1L) / per, 65535L);
+  if (!by_list) {
+    const dim3 grid(nprobe, nq, (unsigned)pieces);
+    if (d > 256 && d <= 32 * PF && (maxlen <= 4096 || (double)maxlen * nlist <= 2. * total))
+      hipLaunchKernelGGL(ivf_probe16_kernel, grid, dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL(ivf_probe_kernel, grid, dim3(64), d * sizeof(float), stream, a.q, d, probes, nprobe, nlist, lstart, lsize, a.vecs,
+                         ids, sqnorm, l2, maxlen, cand, cand_ids);
+    RT_LAUNCH_CHECK();
+    return 0;
+  }
+  const dim3 grid(nlist + 1, 1, (unsigned)std::min(pieces, std::max(64L, 16384L / (nlist + 1))));
+  if (d <= 384) hipLaunchKernelGGL((ivf_list_kernel<12, false>), grid, dim3(256), 0, stream, a);
+  else if (d <= 768) hipLaunchKernelGGL((ivf_list_kernel<24, false>), grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((ivf_list_kernel<12, true>), grid, dim3(256), 0, stream, a);
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -265,6 +265,42 @@ def test_ivf_scan_by_list_and_by_probe(d, l2, nq, nlist):
     torch.testing.assert_close(cand.double(), want.view(nq, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
 
 
+@pytest.mark.parametrize("d", [264, 352])
+def test_ivf_scan_width_between_fragments(d):
+    """Widths of the form that multiplies by probe, with a last fragment that is not whole."""
+    for l2 in (False, True):
+        test_ivf_scan_lists(d, l2)
+        test_ivf_scan_by_list_and_by_probe(d, l2, 3, 40)
+
+
+@pytest.mark.parametrize("nq,nlist,nprobe,d,most", [(5000, 2, 2, 384, 70), (4500, 1, 1, 1000, 130), (900, 9, 4, 768, 65), (64, 3, 3, 72, 9000)])
+@pytest.mark.parametrize("l2", [False, True])
+def test_ivf_scan_by_list_rounds(nq, nlist, nprobe, d, most, l2):
+    """By list: more queries of a list than a workgroup holds, vectors in one to three parts, lists of several workgroups that go round,
+    probes of no list."""
+    g = torch.Generator(device=DEV).manual_seed(nq)
+    size = torch.randint(0, most + 1, (nlist,), generator=g, device=DEV, dtype=torch.int32)
+    size[0] = most
+    start = torch.cumsum(size, 0).int() - size
+    vecs = torch.randn(int(size.sum()), d, generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn(nq, d, generator=g, device=DEV).to(torch.bfloat16)
+    probes = torch.rand(nq, nlist, generator=g, device=DEV).topk(nprobe)[1].int()
+    probes[nq // 2, 0], probes[nq // 3, 0] = -1, nlist
+    sq, ids, maxlen = vecs.float().pow(2).sum(-1), torch.arange(len(vecs), device=DEV) + 7, most + 1
+    assert ops.native().ivf_by_list(nq, nprobe, nlist, d, maxlen, len(vecs))
+    cand, cid = ops.ivf_scan(q, probes, start, size, vecs, ids, maxlen, sq, l2)
+    full = q.double() @ vecs.double().t()
+    if l2:
+        full = 2 * full - sq.double() - q.double().pow(2).sum(-1, keepdim=True)
+    j = torch.arange(maxlen, device=DEV)
+    L = probes.long().clamp(0, nlist - 1)
+    ok = (j < size[L][..., None]) & ((probes >= 0) & (probes < nlist))[..., None]
+    at = (start[L][..., None] + j).clamp(max=len(vecs) - 1)
+    want = full.gather(1, at.view(nq, -1)).view(nq, nprobe, maxlen).masked_fill(~ok, float("-inf"))
+    assert torch.equal(cid, ids[at].masked_fill(~ok, -1).view(nq, -1))
+    torch.testing.assert_close(cand.double(), want.view(nq, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
+
+
 def test_ivf_scan_of_a_list_longer_than_a_grid():
     """A list of more 64-vector pieces than a grid's third dimension holds, and a short one beside it."""
     d, n = 8, 65535 * 64 + 1000

@@ -100,3 +100,16 @@ def test_gemm_plan_of_one_round(K):
         assert rows == M or (rows == 0 and form), (M, N, rows, form)
     for M, N in ((23500, 1152), (8192, 3072), (8192, 4096), (23500, 1024)):
         assert ops.native().gemm_plan(M, N, K, 0)[0] == -1, (M, N)
+
+
+@pytest.mark.parametrize("nq,nprobe,nlist,d,maxlen,total,probe,by_list", [
+    (1, 1, 1, 384, 400000, 400000, 63, 105), (1, 3, 3, 384, 133333, 400000, 62, 76), (2, 8, 64, 384, 8735, 400000, 20, 27),
+    (8, 16, 256, 384, 1091, 200000, 20, 29), (256, 16, 4096, 384, 136, 400000, 53, 57), (4, 16, 512, 384, 3539, 200000, 25, 28),
+    (4, 1, 1, 128, 400000, 400000, 61, 69), (512, 16, 4096, 128, 136, 400000, 36, 65), (4096, 32, 4096, 72, 136, 400000, 319, 506),
+    (8, 1, 1, 384, 400000, 400000, 300, 130), (256, 16, 512, 384, 273, 100000, 84, 27), (12, 16, 256, 384, 7909, 200000, 101, 36),
+    (4096, 32, 4096, 384, 136, 400000, 1335, 555), (10000, 8, 1024, 384, 136, 100000, 787, 152), (16, 1, 1, 128, 400000, 400000, 243, 85)])
+def test_ivf_scan_form(nq, nprobe, nlist, d, maxlen, total, probe, by_list):
+    """Scans take the form that was the faster one when both were timed (us)."""
+    from rag_tl_domainllm_optimizer_amd import ops
+
+    assert ops.native().ivf_by_list(nq, nprobe, nlist, d, maxlen, total) == (by_list < probe)
