@@ -265,6 +265,8 @@ __device__ __forceinline__ bf16x8 scan_load(__amdgpu_buffer_rsrc_t r, uint32_t o
 // 800 are a few hundred waves on as many CUs, where one workgroup per list left 240 CUs idle; 8 of a vector's 16-byte
 // pieces are in flight (16 lists of 600 x 384: 12.4 -> 8.6 us). A vector's terms are summed in the order of the
 // dimensions.
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+__device__ __forceinline__ uint4 load2(const bf16_t* p) { return __builtin_bit_cast(uint4, (u32x4)*(const u32x4_any*)p); }  // vectors at any address
 __global__ __launch_bounds__(64) void ivf_probe_kernel(const bf16_t* __restrict__ q, int d, const int* __restrict__ probes,
                                                        int nprobe, int nlist, const int* __restrict__ lstart,
                                                        const int* __restrict__ lsize, const bf16_t* __restrict__ vecs,
@@ -314,7 +316,7 @@ __global__ __launch_bounds__(64) void ivf_probe_kernel(const bf16_t* __restrict_
     for (; c + 64 <= d; c += 64) {
       uint4 v[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = *(const uint4*)(vr + c + 8 * i);
+      for (int i = 0; i < 8; ++i) v[i] = load2(vr + c + 8 * i);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         float f[8];
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(64) void ivf_probe_kernel(const bf16_t* __restrict_
     }
     for (; c < d; c += 8) {
       float f[8];
-      unpack8(*(const uint4*)(vr + c), f);
+      unpack8(load2(vr + c), f);
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += f[e] * qs[c + e];
     }
@@ -583,11 +585,12 @@ extern "C" int rt_ivf_by_list(int nq, int nprobe, int nlist, int d, int maxlen, 
 extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int nprobe, int nlist, const int* lstart,
                            const int* lsize, const void* vecs, long total, const long* ids, const float* sqnorm, int l2,
                            int maxlen, float* cand, long* cand_ids, hipStream_t stream) {
-  if (d % 8 != 0 || (l2 && !sqnorm) || (uintptr_t)q % 16 || (uintptr_t)vecs % 16) return -1;
+  if (d % 8 != 0 || (l2 && !sqnorm)) return -1;
   if (nq == 0 || nprobe == 0) return 0;
   if (maxlen <= 0) return 0;
   if (d > 1 << 24) return -1;
-  const bool by_list = rt_ivf_by_list(nq, nprobe, nlist, d, maxlen, total);
+  const bool aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)vecs % 16 == 0;  // else a thread per vector
+  const bool by_list = aligned && rt_ivf_by_list(nq, nprobe, nlist, d, maxlen, total);
   // as many queries at once as a grid's second dimension has, or as 32-bit offsets reach
   const long most_q = by_list ? std::min((1L << 30) / (2L * d), (long)INT_MAX) : 65535;
   if (nq > most_q) {
@@ -605,7 +608,7 @@ extern "C" int rt_ivf_scan(const void* q, int nq, int d, const int* probes, int 
   const long pieces = std::min((maxlen + per - 1L) / per, 65535L);
   if (!by_list) {
     const dim3 grid(nprobe, nq, (unsigned)pieces);
-    if (d > 256 && d <= 32 * PF && (maxlen <= 4096 || (double)maxlen * nlist <= 2. * total))
+    if (aligned && d > 256 && d <= 32 * PF && (maxlen <= 4096 || (double)maxlen * nlist <= 2. * total))
       hipLaunchKernelGGL(ivf_probe16_kernel, grid, dim3(256), 0, stream, a);
     else
       hipLaunchKernelGGL(ivf_probe_kernel, grid, dim3(64), d * sizeof(float), stream, a.q, d, probes, nprobe, nlist, lstart, lsize, a.vecs,

@@ -265,6 +265,20 @@ def test_ivf_scan_by_list_and_by_probe(d, l2, nq, nlist):
     torch.testing.assert_close(cand.double(), want.view(nq, -1), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
 
 
+@pytest.mark.parametrize("nq,d", [(3, 384), (2000, 384), (3, 72)])
+def test_ivf_scan_of_vectors_off_16_bytes(nq, d):
+    """Vectors that begin at any element: one list of them, for few queries and as many as would go by list."""
+    g = torch.Generator(device=DEV).manual_seed(nq)
+    n = 300
+    vecs = torch.randn(n * d + 1, generator=g, device=DEV).to(torch.bfloat16)[1:].view(n, d)
+    q = torch.randn(nq, d, generator=g, device=DEV).to(torch.bfloat16)
+    size, start = torch.tensor([n], dtype=torch.int32, device=DEV), torch.tensor([0], dtype=torch.int32, device=DEV)
+    ids = torch.arange(n, device=DEV)
+    cand, cid = ops.ivf_scan(q, torch.zeros(nq, 1, dtype=torch.int32, device=DEV), start, size, vecs, ids, n)
+    torch.testing.assert_close(cand.double(), q.double() @ vecs.double().t(), rtol=1e-5, atol=d ** 1.5 * 2 ** -24 + 1e-6)
+    assert torch.equal(cid, ids.expand(nq, n))
+
+
 @pytest.mark.parametrize("d", [264, 352])
 def test_ivf_scan_width_between_fragments(d):
     """Widths of the form that multiplies by probe, with a last fragment that is not whole."""
