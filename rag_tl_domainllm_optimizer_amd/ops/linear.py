@@ -120,8 +120,9 @@ def gemm(x: torch.Tensor, w: torch.Tensor, u=None, ub=None, bias=None, act=0, ou
             s = nsplit
         if u is not None or out_f32 or N % 16:
             s = 1
+        # the split product's reduction writes and adds rows at any address, tiles want 16 bytes
         if bias is not None and not nsplit and not out_f32 and u is None and max(x.stride(0), w.stride(0)) < 1 << 22 \
-                and small_tiles(M, N, K, act):
+                and small_tiles(M, N, K, act) and (s == 1 or all(t is None or t.data_ptr() % 16 == 0 for t in (out, residual))):
             return native().gemm_big(x, w, ROW, ROW, None, None, bias, act, 0, s, out, None, residual, 0)
         if s > 1:
             slabs = torch.empty(s * M * N, dtype=torch.float32, device=x.device)
