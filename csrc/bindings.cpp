@@ -90,7 +90,7 @@ int rt_adamw(float*, const float*, float*, float*, void*, long, float, float, fl
 int rt_grad_sumsq_mixed(const void*, long, const float*, long, float*, int, hipStream_t);
 int rt_adamw_mixed(float*, const void*, long, const float*, float*, float*, void*, long, float, float, float, float,
                    float, int, float, const float*, int, float*, int*, hipStream_t);
-int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, const long*, hipStream_t);
+int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, const long*, long, hipStream_t);
 int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
@@ -1276,7 +1276,7 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   auto out = at::empty({B, H}, x.options().dtype(at::kFloat));
   if (lengths.has_value() && lengths->defined()) CHECK_I32(*lengths);
   check_rc(rt_pool_norm(x.data_ptr(), (const int*)opt_ptr(lengths), (const long*)opt_ptr(off), packed ? x.size(0) : 0, (int)B,
-                        (int)S, (int)H, normalize ? 1 : 0, out.data_ptr<float>(), nullptr, cur_stream()),
+                        (int)S, (int)H, normalize ? 1 : 0, out.data_ptr<float>(), nullptr, 0, cur_stream()),
            "pool_norm");
   return out;
 }
@@ -1463,7 +1463,7 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
     }
   }
   check_rc(rt_pool_norm(x.data_ptr(), nullptr, (const long*)off.data_ptr(), M, (int)B, 0, (int)H, normalize ? 1 : 0,
-                        out.data_ptr<float>(), (const long*)to.data_ptr(), st),
+                        out.data_ptr<float>(), (const long*)to.data_ptr(), out.size(0), st),
            "encoder: pooling");
   return true;
 }

@@ -189,6 +189,7 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
                                                               float eps) {
   const int lane = threadIdx.x & 63, nv = H / 8;
   for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < T; row += (long)gridDim.x * 4) {
+    RT_ASSERT(ids[row] >= 0 && pids[row] >= 0);
     const bf16_t* const wp = word + ids[row] * H;
     const bf16_t* const pp = pos + pids[row] * H;
     float v[NW][8], s[NW];

@@ -152,7 +152,8 @@ class SentenceEncoder(nn.Module):
     def encode_packed(self, ids: torch.Tensor, pos: torch.Tensor, off: torch.Tensor, longest: int, normalize: bool = True,
                       out: torch.Tensor | None = None, to: torch.Tensor | None = None) -> torch.Tensor:
         """:meth:`encode_ids` of texts without padding: rows [off[b], off[b + 1]) of ``ids`` are text b, none longer than
-        ``longest``, at positions ``pos`` (from ``first_position``). ``out`` (fp32): text b goes to its row ``to[b]``."""
+        ``longest``, at positions ``pos`` (from ``first_position``). ``out`` (fp32): text b goes to its row ``to[b]``,
+        which has to be one (the native forward leaves texts out that have none)."""
         if out is not None:
             if longest == 0 or not self._encode_native(ids, pos, off, longest, normalize, out, to):
                 out[to] = self.encode_packed(ids, pos, off, longest, normalize).float()

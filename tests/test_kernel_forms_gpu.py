@@ -593,6 +593,23 @@ def test_native_encoder_forward_is_the_ops_forward(preset, lens):
     assert torch.equal(got[to], want)
 
 
+def test_native_encoder_writes_no_row_beyond_out():
+    """Rows counted from the end go there, texts whose row does not exist go nowhere: the rows around out stay as they are."""
+    from rag_tl_domainllm_optimizer_amd import models
+    import dataclasses
+
+    m = models.SentenceEncoder(dataclasses.replace(models.resolve_preset("minilm-l6"), num_layers=1), device=DEV, dtype=torch.bfloat16).eval()
+    lens = [5, 9, 3, 7]
+    off = torch.nn.functional.pad(torch.tensor(lens, device=DEV).cumsum(0), (1, 0))
+    ids = torch.arange(10, 10 + sum(lens), device=DEV)
+    pos = torch.cat([torch.arange(n, device=DEV) for n in lens])
+    buf = torch.full((12, m.cfg.hidden_size), 7.0, device=DEV)
+    m.encode_packed(ids, pos, off, max(lens), True, buf[4:8], torch.tensor([2, -1, 4, -5], device=DEV))
+    want = m.encode_packed(ids, pos, off, max(lens))
+    assert torch.equal(buf[6], want[0]) and torch.equal(buf[7], want[1])
+    assert (buf[:6] == 7).all() and (buf[8:] == 7).all()
+
+
 # ---------------------------------------------------------------------------------------------- decode products, 65..128 rows
 @pytest.mark.parametrize("N,K,act", [(16, 64, 0), (48, 448, 0), (2048, 1024, 0), (4112, 2112, ops.ACT_RELU2), (33024, 256, 0),
                                      (64, 128, 5), (1056, 1088, 5), (33024, 320, 5)])
