@@ -425,9 +425,9 @@ Tensor latent_gather(const Tensor& pool, const Tensor& tab, const Tensor& segs, 
 
 // q / gate / out rows are the batch's tokens (segments index them); kv [rows, H (dim + vdim) + rot]: unrotated
 // keys, values, shared rotated key part
-void latent_prefill(const Tensor& q, const Tensor& kv, const Tensor& sink, const Tensor& gate, Tensor out,
+void latent_prefill(const Tensor& q, const Tensor& kv_, const Tensor& sink, const Tensor& gate, Tensor out,
                     const Tensor& segs, const Tensor& tiles, int64_t H, int64_t dim, int64_t rot, int64_t vdim, double scale) {
-  for (const Tensor* t : {&q, &kv, &gate}) {
+  for (const Tensor* t : {&q, &kv_, &gate}) {
     rows(*t, "latent_prefill");
     TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && al16(*t), "latent_prefill: bf16 rows, 16-B aligned");
   }
@@ -437,6 +437,11 @@ void latent_prefill(const Tensor& q, const Tensor& kv, const Tensor& sink, const
   ints(tiles, "tiles");
   f32c(sink, "sink");
   TORCH_CHECK(segs.dim() == 2 && segs.size(1) == 8 && tiles.dim() == 2 && tiles.size(1) == 2, "latent_prefill: tables");
+  Tensor kv = kv_;
+  if (kv.stride(0) >= 1 << 24) {  // a tile's rows lie within 2^32 bytes in the kernel: rows further apart are brought together
+    kv = at::empty({kv_.size(0), (kv_.size(1) + 7) / 8 * 8}, kv_.options()).narrow(1, 0, kv_.size(1));
+    kv.copy_(kv_);
+  }
   TORCH_CHECK(q.size(1) >= H * (dim + rot) && kv.size(1) == H * (dim + vdim) + rot && gate.size(1) == H * vdim &&
                   out.size(1) == H * vdim && sink.numel() == H, "latent_prefill: shapes");
   rc_ok(rt_latent_prefill(q.data_ptr(), q.stride(0), kv.data_ptr(), kv.stride(0), (int)(H * dim), (int)(H * (dim + vdim)),

@@ -249,6 +249,23 @@ def test_latent_prefill(H, dim, rot, vdim):
     assert rel(out, want) < 1e-2
 
 
+def test_latent_prefill_rows_far_apart():
+    """Expanded rows 2^24 elements apart, more than a tile of them: the bits of rows that lie together."""
+    H, dim, rot, vdim, n = 2, 64, 64, 64, 70
+    g = torch.Generator().manual_seed(1)
+    kv = torch.randn(n, H * (dim + vdim) + rot, generator=g).bfloat16().to(DEV)
+    q, gate = torch.randn(n, H * (dim + rot), generator=g).bfloat16().to(DEV), torch.randn(n, H * vdim, generator=g).bfloat16().to(DEV)
+    sink = torch.zeros(H, device=DEV)
+    segs, tiles = torch.tensor([[0, 0, n, 0, n, 0, 0, 0]]).int().to(DEV), torch.tensor([[0, 0]]).int().to(DEV)
+    far = torch.empty(n << 24, dtype=torch.bfloat16, device=DEV).view(n, 1 << 24)[:, :kv.shape[1]]
+    far.copy_(kv)
+    out = []
+    for t in (kv, far):
+        out.append(torch.empty(n, H * vdim, dtype=torch.bfloat16, device=DEV))
+        native().latent_prefill(q, t, sink, gate, out[-1], segs, tiles, H, dim, rot, vdim, 0.1)
+    assert torch.equal(out[0], out[1])
+
+
 def test_wrappers_refuse_bad_shapes():
     n = native()
     x = torch.randn(4, 8, device=DEV)
