@@ -172,6 +172,31 @@ def test_window_prefill_capped_scores(cap, D, V):
         assert (((out[rows, h * V:(h + 1) * V].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6)
 
 
+def test_delta_rule_decay_rounding():
+    """The decay of a prompt's state, from the state itself: one token of a portion decays by e^-40 over 3072 inputs from -8 to 8, the
+    others and beta leave the state alone. Relative errors of the exponent around their mean per head (which exp(A) shares): log1p, exp
+    and the product with A round to fp32, 2^-24 / sqrt(3) rms each at most, 2^-24 in all."""
+    g = torch.Generator().manual_seed(0)
+    T, H, D, V, taps = 20, 48, 64, 16, 2
+    x0 = torch.linspace(-8, 8, H)
+    dt = x0[:, None] + 0.4 * torch.rand(H, D, generator=g)
+    A = torch.log(40 / torch.nn.functional.softplus(x0 + 0.2).double()).float()
+    x = torch.zeros(T, 2 * H * D + H * V)
+    x[:, :2 * H * D] = 1.0
+    conv = torch.zeros(x.shape[1], taps)
+    conv[:, -1] = 1.0
+    a, b, z = torch.full((T, H * D), -300.0), torch.full((T, H), -120.0), torch.zeros(T, H * V)
+    a[3] = 0.0
+    S, ring, out = torch.ones(1, H, D, V, device=DEV), torch.zeros(1, taps, x.shape[1], device=DEV), torch.zeros(T, H * V, device=DEV)
+    x, b, a, z, conv = (t.to(DEV) for t in (x, b, a, z, conv))
+    ops.delta_rule(x, b, a, z, conv, A.to(DEV), dt.reshape(-1).to(DEV), torch.ones(V, device=DEV), 1e-6,
+                   RaggedBatch.build([(0, [0] * T, 5)], DEV), S, ring, out, 1.0, H, False)
+    want = -torch.exp(A.double())[:, None] * torch.log1p(torch.exp(dt.double()))
+    e = (torch.log(S[0, :, :, 0].double().cpu()) - want) / want
+    e = e - e.mean(1, keepdim=True)
+    assert e.abs().max() < 4 * 2.0 ** -24 and e[x0 < -1].pow(2).mean().sqrt() < 2.0 ** -24, (e.abs().max(), e[x0 < -1].pow(2).mean().sqrt())
+
+
 @pytest.mark.parametrize("cap", [5.0, 50.0, 0.0])
 def test_window_prefill_negative_scale(cap):
     """A scale below zero is a scale: products of both signs, well beyond where tanh is a polynomial."""
