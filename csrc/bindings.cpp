@@ -66,6 +66,8 @@ int rt_few_rows(const void*, long, const void*, long, const void*, const void*, 
                 int, int, int, int, float, int, int, hipStream_t);
 int rt_gemm_nt_parts(int, int, int, int*);
 int rt_gemm_plan(int, int, int, int, int*);
+int rt_token_plan(int, int, int, int, int*);
+int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
                        float, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
@@ -1281,25 +1283,11 @@ Tensor pool_norm(const Tensor& x, const optional<Tensor>& lengths, bool normaliz
   return out;
 }
 
-// ops.linear's small_tiles (products with a bias)
-static bool small_tiles(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (M <= 64 || M > 512 || K % 64 || K > 3072 || (act != 0 && act != 2)) return false;
-  const int64_t rounds = ((M + 63) / 64 * ((N + 63) / 64) + 255) / 256;
-  return 2.6 + rounds * (0.19 * (K / 64) + (act ? 1.7 : 0.4)) < (K > 2048 ? 17 : 14);
-}
-
-// The K split of ops.gemm's token-parallel products (splitk_plan there): parts and the columns of a tile
-static std::pair<int64_t, int64_t> token_split(int64_t M, int64_t N, int64_t K, int64_t act) {
-  if (M > 512) return {1, 0};
-  const int64_t bn = act == 0 ? 128 : 256, tiles = (M + 255) / 256 * ((N + bn - 1) / bn);
-  const int64_t split = tiles < 128 && N % 16 == 0 ? std::max<int64_t>(1, std::min((K + 63) / 64 / 8, (256 + tiles / 2) / tiles)) : 1;
-  return {split, split == 1 && act ? 0 : bn};
-}
-
 // The parts in which the kernel that ops.gemm takes sums K (row-major operands, K % 64 == 0), for rt_few_rows
 struct KParts { int n, grp; };
 static KParts k_parts(int64_t M, int64_t N, int64_t K, int64_t act) {
-  KParts k{(int)token_split(M, N, K, act).first, 1};
+  int bn = 0;
+  KParts k{rt_token_plan((int)M, (int)N, (int)K, (int)act, &bn), 1};
   if (M <= 64) k.n = rt_gemm_nt_parts((int)M, (int)N, (int)K, &k.grp);
   return k;
 }
@@ -1341,8 +1329,9 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
 static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
-  const auto [split, bn] = token_split(M, N, K, act);
-  if (small_tiles(M, N, K, act))
+  int bn = 0;
+  const int split = rt_token_plan((int)M, (int)N, (int)K, (int)act, &bn);
+  if (rt_small_tiles((int)M, (int)N, (int)K, (int)act))
     return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, split, std::nullopt, std::nullopt, std::nullopt, 0, {});
   if (split > 1) {
     auto slabs = at::empty({split * M * N}, x.options().dtype(at::kFloat));
@@ -1645,6 +1634,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_store_fp8", &kv_store_fp8, "prompt K/V -> fp8 cache (per-slot scales)");
   m.def("attn_decode_fused_ps", &rt_attn_decode_fused_ps, "keys per partition of the fused decode kernel");
   m.def("quant_fp8", &quant_fp8, "per-row absmax e4m3fn quantisation -> (uint8 [R,C], scale fp32 [R])");
+  m.def("token_plan", [](int64_t M, int64_t N, int64_t K, int64_t act) {
+    int bn = 0;
+    const int parts = rt_token_plan((int)M, (int)N, (int)K, (int)act, &bn);
+    return std::make_pair(parts, bn);
+  }, "parts of K and columns of a tile of a token-parallel NT product");
+  m.def("small_tiles", [](int64_t M, int64_t N, int64_t K, int64_t act) { return rt_small_tiles((int)M, (int)N, (int)K, (int)act) != 0; },
+        "whether a product with a bias takes 64 x 64 tiles that sum the parts of K");
   m.def("gemm_plan", [](int64_t M, int64_t N, int64_t K, int64_t act) {
     int form = 0;
     const int rows = rt_gemm_plan((int)M, (int)N, (int)K, (int)act, &form);

@@ -1554,6 +1554,25 @@ extern "C" int rt_gemm_plan(int M, int N, int K, int act, int* form) {
   return p.m1 < 0 ? -1 : (int)std::min<long>(M, p.m1 * 256L);
 }
 
+// The parts in which a token-parallel NT product sums K, and *bn, the columns of its tiles (0: planned), see ops.linear.splitk_plan.
+// An unsplit GELU product is planned: it has a form of its own (300 x 1536 x 384: 18.9 us, 28.8 on 256 x 256 tiles; the same bits)
+extern "C" int rt_token_plan(int M, int N, int K, int act, int* bn) {
+  *bn = 0;
+  if (M > 512) return 1;
+  const bool narrow = act == E_NONE || act == E_SWIGLU || act == E_RELU2;
+  const int cols = narrow ? 128 : 256;
+  const long tiles = std::max(1L, (M + 255L) / 256 * (act == E_SWIGLU ? N / cols : (N + cols - 1) / cols));
+  const int s = tiles >= 128 ? 1 : (int)std::max(1L, std::min((K + 63L) / 64 / 8, (256 + tiles / 2) / tiles));
+  *bn = s == 1 && act == E_GELU ? 0 : cols;
+  return s;
+}
+
+// Whether 65 to 512 rows of a product with a bias take 64 x 64 tiles, which sum those parts themselves: where they are done before a
+// split product and its reduction, 14 us, from K = 2048 on 17
+extern "C" int rt_small_tiles(int M, int N, int K, int act) {
+  return M > 64 && M <= 512 && K % 64 == 0 && K <= 3072 && (act == E_NONE || act == E_GELU) && mid_us(M, N, K, act, 1) < (K > 2048 ? 17.f : 14.f);
+}
+
 // bn = 0: the wave planner over validated arguments p
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream) {
   if (bn != 0) return launch_gemm_big(p, layout_a, layout_b, act, out, bn, stream);

@@ -20,12 +20,14 @@ The reference runs these products through HF/PyTorch (reinforcement_learning_opt
 from __future__ import annotations
 
 import contextlib
+import functools
 import threading
 from dataclasses import dataclass, field
 from typing import List, Optional
 
 import torch
 
+from . import _ext
 from . import reference as ref
 from ._ext import native, on_gpu
 
@@ -35,32 +37,22 @@ ACT_RELU2 = 8  # max(x, 0)^2
 ACT_DSWIGLU = 6  # gemm_big NN epilogue: d[gate | up] from dF and the [gate | up] pre-activation
 
 
+@functools.lru_cache(maxsize=4096)
 def splitk_plan(M: int, N: int, K: int, act: int = 0):
     """(nsplit, bn) for a token-parallel NT GEMM. Up to 512 rows (decode at batch 65..512, small
     prefills) the 256x128 tile doubles the workgroups over the 256x256 one, and the K split fills
     the rest of the chip (qkv 48 tiles x 5, o / down 32 x 8, gate_up 224 x 1 with the SwiGLU in the
     epilogue, lm_head 250 x 1). Larger M: one launch planned by rt_gemm_big (bn 0: 256x256 tiles,
-    the last partial wave on 256x128 tiles)."""
-    if M > 512:
-        return 1, 0
-    bn = 128 if act in (0, ACT_SWIGLU, ACT_RELU2) else 256
-    tiles = ((M + 255) // 256) * (N // bn if act == ACT_SWIGLU else (N + bn - 1) // bn)
-    if tiles >= 128:
-        return 1, bn
-    nk = (K + 63) // 64
-    s = max(1, min(nk // 8, (256 + tiles // 2) // tiles))
-    # an unsplit GELU product has a form of its own (300 x 1536 x 384: 18.9 us, 28.8 on 256x256 tiles; the same bits)
-    return s, 0 if s == 1 and act == ACT_IDS["gelu"] else bn
+    the last partial wave on 256x128 tiles). rt_token_plan, which the sentence encoder's native forward asks too."""
+    return _ext.native().token_plan(M, N, K, act)
 
 
+@functools.lru_cache(maxsize=4096)
 def small_tiles(M: int, N: int, K: int, act: int) -> bool:
-    """Whether 65 to 512 rows of an encoder's product (one with a bias) take 64x64 tiles, which sum the parts of a K split
-    themselves (the same bits): 2.6 us and 0.19 a K-step for every tile of a CU, where a split product and its reduction take
-    14, from K = 2048 on 17. Decoders' products stay with the split, which their norms and attention sum themselves."""
-    if M <= 64 or M > 512 or K % 64 or K > 3072 or act not in (0, ACT_IDS["gelu"]):
-        return False
-    rounds = ((M + 63) // 64 * ((N + 63) // 64) + 255) // 256
-    return 2.6 + rounds * (0.19 * (K // 64) + (1.7 if act else 0.4)) < (17 if K > 2048 else 14)
+    """Whether 65 to 512 rows of a product with a bias (encoders' products, and decoders' where they have biases) take 64x64 tiles, which sum
+    the parts of a K split themselves (the same bits): rt_small_tiles. Products without one stay with the split, which decoders'
+    norms and attention sum themselves."""
+    return _ext.native().small_tiles(M, N, K, act)
 
 
 _BI = threading.local()  # per-thread nesting depth of batch_invariant() (a serving thread keeps its plans)

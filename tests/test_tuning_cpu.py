@@ -113,3 +113,18 @@ def test_ivf_scan_form(nq, nprobe, nlist, d, maxlen, total, probe, by_list):
     from rag_tl_domainllm_optimizer_amd import ops
 
     assert ops.native().ivf_by_list(nq, nprobe, nlist, d, maxlen, total) == (by_list < probe)
+
+
+def test_token_plans():
+    """The plans that ops.gemm and the encoder's native forward share: whole products beyond 512 rows, parts that fill the chip up to
+    there, and the 64 x 64 tiles where their time by the planner's model is below a split product's and its reduction's."""
+    from rag_tl_domainllm_optimizer_amd.ops.linear import small_tiles, splitk_plan
+
+    assert splitk_plan(513, 4096, 4096) == (1, 0) and splitk_plan(256, 6144, 4096) == (5, 128) and splitk_plan(256, 4096, 14336) == (8, 128)
+    assert splitk_plan(256, 28672, 4096, 5) == (1, 128) and splitk_plan(256, 32000, 4096) == (1, 128)
+    assert splitk_plan(300, 1536, 384, 2) == (1, 0) and splitk_plan(400, 16384, 2048, 2) == (1, 0) and splitk_plan(300, 768, 3072, 3) == (6, 256)
+    for act in (0, 2):
+        assert small_tiles(65, 768, 768, act) and small_tiles(512, 768, 3072, act) and small_tiles(512, 2304, 1408, act)
+        assert not small_tiles(64, 768, 768, act) and not small_tiles(513, 768, 768, act) and not small_tiles(300, 768, 776, act)
+        assert not small_tiles(512, 10240, 2560, act) and not small_tiles(300, 768, 3136, act)
+    assert not small_tiles(300, 768, 768, 1)
