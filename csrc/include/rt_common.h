@@ -168,21 +168,6 @@ __device__ __forceinline__ float over_groups(float x, F f) {
   return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// 2 x (2 reads at a_i + {0, O1})
-template <int O1>
-__device__ __forceinline__ void ds_tr16_2x2(uint32_t a0, uint32_t a1, rt_s16x4& r0, rt_s16x4& r1, rt_s16x4& r2,
-                                            rt_s16x4& r3) {
-  asm volatile(
-      "ds_read_b64_tr_b16 %0, %4\n\t"
-      "ds_read_b64_tr_b16 %1, %4 offset:%6\n\t"
-      "ds_read_b64_tr_b16 %2, %5\n\t"
-      "ds_read_b64_tr_b16 %3, %5 offset:%6\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
-      : "v"(a0), "v"(a1), "i"(O1)
-      : "memory");
-}
-
 // D = A.B + D on a 16x16x32 bf16 MFMA with D tied to AGPRs ("+a") and a "memory" clobber that pins
 // surrounding loads / LDS-DMA issues to their source position (gemm_big.hip's 4-wave kernels).
 // The x86 host pass parses kernel bodies too and has no AGPR constraint: the asm is device-pass only.
