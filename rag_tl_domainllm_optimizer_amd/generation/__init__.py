@@ -370,7 +370,7 @@ class Generator:
     def _ragged_prefill(self, prompts) -> torch.Tensor:
         """Prompts of rows 0.. as one ragged step -> the hidden state of each one's last token."""
         batch = RaggedBatch.build([(b, p, 0) for b, p in enumerate(prompts)], self.device)
-        last = torch.tensor([int(batch.offset[b]) + len(p) - 1 for b, p in enumerate(prompts)]).to(self.device)
+        last = ops.upload(torch.tensor([int(batch.offset[b]) + len(p) - 1 for b, p in enumerate(prompts)]), self.device)
         return self.model.step(batch, self.cache, last)
 
     def _ensure_graph(self, params, eos, eos_list, pad_id, T):
@@ -747,7 +747,7 @@ class ContinuousBatcher:
                                   g.device)
         nd = len(dec)
         if nd:
-            idx = torch.tensor(dec).to(g.device)
+            idx = ops.upload(torch.tensor(dec), g.device)
             batch.ids[:nd] = g.tok_in[idx]
             batch.pos[:nd] = g.pos[idx]
             bound = max(self.rows[b][1] + self.T for b in dec)
@@ -764,10 +764,10 @@ class ContinuousBatcher:
                 g.gen_len[b:b + 1].zero_()
                 g.active[b:b + 1].fill_(1)
         self.pending = [e for e in self.pending if e[2] is None or e[2] < len(e[1])]
-        h = g.model.step(batch, g.cache, torch.tensor(want, dtype=torch.long).to(g.device))
+        h = g.model.step(batch, g.cache, ops.upload(torch.tensor(want, dtype=torch.long), g.device))
         if rows:
             full = h.new_zeros(g._bucket(max(self.rows) + 1), h.shape[1])
-            full[torch.tensor(rows).to(g.device)] = h
+            full[ops.upload(torch.tensor(rows), g.device)] = h
             g._emit(full, self.params, self.eos, self.pad_id)
         return True
 

@@ -15,6 +15,8 @@ from typing import List, Optional
 import numpy as np
 import torch
 
+from ..ops import upload
+
 PAGE = 64
 
 
@@ -95,7 +97,7 @@ class PagedCache:
     def sync(self):
         """Upload the page table if it changed (stream-ordered before the step that reads it)."""
         if self._dirty:
-            self.table.copy_(torch.from_numpy(self._host.copy()))
+            self.table.copy_(upload(self._host, self.table.device))
             self._dirty = False
 
     def rows_view(self, row0: int, n: int) -> "PagedRows":

@@ -12,6 +12,8 @@ from typing import List, Sequence, Tuple
 import numpy as np
 import torch
 
+from ..ops import upload
+
 SHORT_TOKENS = 32   # portions up to this many tokens attend token by token, like decoded ones
 QUERY_TILE = 128    # query rows per workgroup of the portions' attention kernel
 CHUNK = 16          # tokens per chunk of a recurrent layer's portions (csrc/kernels/delta_rule.hip)
@@ -73,7 +75,7 @@ class RaggedBatch:
         tables = [np.asarray(segs, np.int32).reshape(-1, 8), np.asarray(runs, np.int32).reshape(-1, 4),
                   np.asarray(tiles, np.int32).reshape(-1, 2), chunks.astype(np.int32), first[:-1].astype(np.int32)]
         flat = np.concatenate(parts_i + parts_r + parts_p + [np.zeros(-3 * n % 4, np.int32)] + [t.reshape(-1) for t in tables])
-        buf = torch.from_numpy(flat).to(device)
+        buf = upload(flat, device)
         at, dev = 3 * n + -3 * n % 4, []
         for t in tables:
             dev.append(buf[at:at + t.size].view(t.shape) if t.size else None)
@@ -123,7 +125,7 @@ class StepEngine:
         self.cache.sync()
         batch = RaggedBatch.build([(r, t, self.length[r]) for r, t, _ in entries], self.device)
         want = [int(batch.offset[e]) + i for e, (_, _, w) in enumerate(entries) for i in w]
-        h = self.model.step(batch, self.cache, torch.tensor(want, dtype=torch.long).to(self.device))
+        h = self.model.step(batch, self.cache, upload(torch.tensor(want, dtype=torch.long), self.device))
         for row, toks, _ in entries:
             self.length[row] += len(toks)
         if not want:

@@ -417,7 +417,7 @@ class CausalLM(nn.Module):
                 # MLP run on B rows (its K/V above still covered the whole prompt)
                 last = torch.arange(B, device=dev) * S + (S - 1)
                 o = o.index_select(0, last)
-                residual = residual.index_select(0, torch.from_numpy(packed[1][1:] - 1).to(dev)
+                residual = residual.index_select(0, ops.upload(packed[1][1:] - 1, dev)
                                                  if idx is not None else last)
             elif idx is not None:
                 o = ops.gather_rows(o, idx, inv)
@@ -539,7 +539,7 @@ def packed_index(lo, hi, L: int, device):
     off = np.zeros(len(n) + 1, dtype=np.int64)
     np.cumsum(n, out=off[1:])
     idx = np.repeat(np.arange(len(n), dtype=np.int64) * L - off[:-1] + lo, n) + np.arange(off[-1], dtype=np.int64)
-    return torch.from_numpy(idx).to(device), off
+    return ops.upload(idx, device), off
 
 
 def pack_enabled() -> bool:

@@ -3,11 +3,32 @@ from __future__ import annotations
 
 from typing import Optional
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
 from . import reference as ref
 from ._ext import native, on_gpu
+
+
+# ------------------------------------------------------------------------------------ tables made on the host
+# Bytes up to which upload() goes through pinned memory. Torch rounds pinned blocks up to a power of two and keeps them until the
+# process ends; the index tables of a minibatch or a step are 1 to 130 KiB.
+UPLOAD_PINNED = 1 << 20
+
+
+def upload(src, device) -> torch.Tensor:
+    """A host array or tensor on ``device``. On a GPU the copy is queued on the current stream, from a pinned block of its own
+    (torch reuses it once the copy is done), so ``src`` may change at once and the host goes on: a copy from pageable memory
+    waits for all that is queued ahead of it, and the GPU then idles while the host catches up (a PPO minibatch of 16 rows, two
+    layers of Mistral-7B: 0.8 of 8.2 ms, prompts 0.3 to 0.5). Larger sources, and captures (which refuse them), take that copy."""
+    t = torch.from_numpy(src) if isinstance(src, np.ndarray) else src
+    device = torch.device(device)
+    if device.type != "cuda" or t.is_cuda or t.numel() * t.element_size() > UPLOAD_PINNED or torch.cuda.is_current_stream_capturing():
+        return t.to(device)
+    buf = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+    buf.copy_(t)
+    return buf.to(device, non_blocking=True)
 
 
 # ------------------------------------------------------------------------------------ SwiGLU

@@ -74,8 +74,8 @@ def _score_sequences(model, prompt_ids: torch.Tensor, start: torch.Tensor, resp:
             idx, off = packed_index(lo, hi, S + T, dev)
             b = np.repeat(np.arange(B, dtype=np.int64), rl)
             t = np.arange(n_sc, dtype=np.int64) - np.repeat(np.cumsum(rl) - rl, rl)
-            sel = torch.from_numpy(off[:-1][b] + (S - 1 + t) - lo[b]).to(dev)
-            dst = torch.from_numpy(b * T + t).to(dev)
+            sel = ops.upload(off[:-1][b] + (S - 1 + t) - lo[b], dev)
+            dst = ops.upload(b * T + t, dev)
             # hidden states of the scored rows only (the last layer's o_proj / MLP skip the rest)
             hs = model(seq, kv_start=start.to(torch.int32), gradient_checkpointing=gradient_checkpointing,
                        packed_idx=idx, out_rows=sel)

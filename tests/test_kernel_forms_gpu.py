@@ -2,6 +2,7 @@
 general form of the same operation."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -750,3 +751,15 @@ def test_decode_weight_images_only_where_read(mode):
         assert held == {"qkv_plain", "o", "gate_up_plain", "down"}
     elif mode == "fp8":
         assert not held
+
+
+@pytest.mark.parametrize("n,dtype", [(0, np.int64), (1, np.int32), (131072, np.int64), (131073, np.int64)])
+def test_upload_holds_the_source_of_the_call(n, dtype):
+    """ops.upload up to its pinned limit and beyond: the values at the call, whatever becomes of the source, behind a busy stream."""
+    src = np.arange(2 * n, dtype=dtype)[::2]
+    want = src.copy()
+    torch.cuda._sleep(2_000_000)
+    got = [ops.upload(src, DEV), ops.upload(torch.from_numpy(src), DEV)]
+    src += 7
+    for g in got:
+        assert g.device.type == "cuda" and g.is_contiguous() and np.array_equal(g.cpu().numpy(), want)
