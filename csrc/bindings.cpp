@@ -39,6 +39,7 @@ int rt_gemm_big_rope(const void*, long, const void*, long, const void*, long, co
                      void*, long, int, int, int, const int*, const float*, const float*, int, int, const void*, int,
                      hipStream_t);
 int rt_gemm_splitk_reduce(const float*, int, int, int, const void*, int, const void*, long, void*, long, hipStream_t);
+int rt_nn_split(int, int, int, int*);
 int rt_gemm_big_fp8_slabs(const void*, long, const float*, const void*, long, const float*, float*, int, int, int, int,
                           int, hipStream_t);
 int rt_gemm_big_fp8(const void*, long, const float*, const void*, long, const float*, const void*, void*, long, int,
@@ -453,6 +454,23 @@ Tensor gemm_big(const Tensor& a, const Tensor& b, int64_t layout_a, int64_t layo
     CHECK_ALIGN16(*residual);
   }
   if (M == 0 || N == 0) return c;
+  if (layout_a == 0 && layout_b == 1 && out_mode == 0 && act == 0 && nsplit <= 1 && bn == 0 && !has_r && !opt_ptr(bias)) {
+    // an NN product of few tiles: K in parts (rt_nn_split)
+    int cols = 0;
+    const int parts = rt_nn_split((int)M, (int)N, (int)((K + 63) / 64 + (K2 + 63) / 64), &cols);
+    if (parts > 1) {
+      auto slabs = at::empty({(int64_t)parts * M * N}, a.options().dtype(at::kFloat));
+      check_rc(rt_gemm_big(0, 1, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), ext ? a2->data_ptr() : nullptr,
+                           ext ? a2->stride(0) : 0, ext ? b2->data_ptr() : nullptr, ext ? b2->stride(0) : 0, (int)K2, nullptr,
+                           slabs.data_ptr(), N, nullptr, 0, nullptr, 0, (int)M, (int)N, (int)K, 0, 3, parts,
+                           zero_page(a).data_ptr(), cols, cur_stream()),
+               "gemm_big(split)");
+      check_rc(rt_gemm_splitk_reduce(slabs.data_ptr<float>(), parts, (int)M, (int)N, nullptr, 0, nullptr, 0, c.data_ptr(),
+                                     c.stride(0), cur_stream()),
+               "gemm_big(reduce)");
+      return c;
+    }
+  }
   check_rc(rt_gemm_big_glu((int)layout_a, (int)layout_b, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
                        ext ? a2->data_ptr() : nullptr, ext ? a2->stride(0) : 0, ext ? b2->data_ptr() : nullptr,
                        ext ? b2->stride(0) : 0, (int)K2, opt_ptr(bias), c.data_ptr(), c.stride(0), c2, ldc2,
@@ -1639,6 +1657,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const int parts = rt_token_plan((int)M, (int)N, (int)K, (int)act, &bn);
     return std::make_pair(parts, bn);
   }, "parts of K and columns of a tile of a token-parallel NT product");
+  m.def("nn_split", [](int64_t M, int64_t N, int64_t steps) {
+    int bn = 0;
+    const int parts = rt_nn_split((int)M, (int)N, (int)steps, &bn);
+    return std::make_pair(parts, bn);
+  }, "parts of the K-steps and columns of a tile of an NN product");
   m.def("small_tiles", [](int64_t M, int64_t N, int64_t K, int64_t act) { return rt_small_tiles((int)M, (int)N, (int)K, (int)act) != 0; },
         "whether a product with a bias takes 64 x 64 tiles that sum the parts of K");
   m.def("gemm_plan", [](int64_t M, int64_t N, int64_t K, int64_t act) {

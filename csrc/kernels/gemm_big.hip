@@ -1332,6 +1332,7 @@ static int launch_gemm_big(const Args& p, int layout_a, int layout_b, int act, i
       case 10: GB_LAUNCH(ROW, ROW, O_F32, E_NONE, 128); break;
       case 30: GB_LAUNCH(ROW, ROW, O_F32_SLAB, E_NONE, 128); break;
       case 100: GB_LAUNCH(ROW, KMAJ, O_BF16, E_NONE, 128); break;
+      case 130: GB_LAUNCH(ROW, KMAJ, O_F32_SLAB, E_NONE, 128); break;
       case 100 + E_DSWIGLU: GB_LAUNCH(ROW, KMAJ, O_BF16, E_DSWIGLU, 128); break;
       default: return -4;
     }
@@ -1358,6 +1359,7 @@ static int launch_gemm_big(const Args& p, int layout_a, int layout_b, int act, i
       case 10: GB_LAUNCH(ROW, KMAJ, O_BF16, E_NONE, 256); break;
       case 11: GB_LAUNCH(ROW, KMAJ, O_F32, E_NONE, 256); break;
       case 12: GB_LAUNCH(ROW, KMAJ, O_F32_ATOMIC, E_NONE, 256); break;
+      case 13: GB_LAUNCH(ROW, KMAJ, O_F32_SLAB, E_NONE, 256); break;
       case 110: GB_LAUNCH(KMAJ, KMAJ, O_BF16, E_NONE, 256); break;
       case 111: GB_LAUNCH(KMAJ, KMAJ, O_F32, E_NONE, 256); break;
       case 112: GB_LAUNCH(KMAJ, KMAJ, O_F32_ATOMIC, E_NONE, 256); break;
@@ -1372,7 +1374,7 @@ static int launch_gemm_big(const Args& p, int layout_a, int layout_b, int act, i
 static bool bn128_supported(int layout_a, int layout_b, int act, int out) {
   const int key = layout_a * 100 + layout_b * 10 + out;
   return (key == 0 && (act == E_NONE || act == E_SWIGLU || act == E_ROPE || act == E_RELU2)) ||
-         (act == E_NONE && (key == 1 || key == 3 || key == 10)) || (key == 10 && act == E_DSWIGLU);
+         (act == E_NONE && (key == 1 || key == 3 || key == 10 || key == 13)) || (key == 10 && act == E_DSWIGLU);
 }
 
 static int query_num_cus() {
@@ -1387,8 +1389,10 @@ static int num_cus() {
   return n;
 }
 
-// Ratio of a 256x128 tile's time to a 256x256 tile's (same K), for the wave planner below.
-static float bn128_cost() { return tuning().gemm_bn128_cost; }
+// Ratio of a 256x128 tile's time to a 256x256 tile's (same K), for the wave planner below. With a K-contiguous A and a
+// column-contiguous B (NN) it is larger, 74 us to 120 at K = 4096: the transposed reads of B wait inside each phase. 4016 x 14336 x
+// 4096, which 0.55 put on seven rounds of 128 columns: 468 us, 391 on 256; with the SwiGLU backward 535, so 467.
+static float bn128_cost(int layout_b = ROW) { return layout_b == KMAJ ? 0.62f : tuning().gemm_bn128_cost; }
 
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream);
 static int launch_mid(const Args& p, int form, int act, hipStream_t stream);
@@ -1495,7 +1499,7 @@ static int launch_mid(const Args& p, int form, int act, hipStream_t stream) {
 struct Plan { int m1, form; };
 
 // plain: row-major operands, K % 64 == 0, bf16 result, bias and GELU or no activation (what gemm_duo and gemm_mid take)
-static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128) {
+static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128, int layout_b) {
   const long cus = (long)num_cus() * 1;  // one 512-thread, 128-KiB-LDS workgroup per CU
   // Two workgroups per CU (gemm_duo_kernel) where the reduction is short. With GELU from any number of rows: 19.6 against 32
   // us for 1000 x 1536 x 384, 258 against 306 for 26000 x 4096 x 1024, 827 against 880 for 26000 x 8192 x 2048. Without an
@@ -1525,7 +1529,7 @@ static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128) {
   Plan p{tiles_m, 0};
   float best = (float)(((long)tiles_m * tn256 + cus - 1) / cus);  // rounds
   if (can128) {
-    const float r = bn128_cost();
+    const float r = bn128_cost(layout_b);
     best = 1e30f;
     for (int m = tiles_m; m >= 0; --m) {
       const long w256 = ((long)m * tn256 + cus - 1) / cus, w128 = ((long)(tiles_m - m) * tn128 + cus - 1) / cus;
@@ -1549,7 +1553,7 @@ static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128) {
 
 // how many rows of a plain product (see plan_tiles) go on 256 x 256 tiles, and the form of the rest; -1: gemm_duo_kernel
 extern "C" int rt_gemm_plan(int M, int N, int K, int act, int* form) {
-  const Plan p = plan_tiles(M, N, K, act, true, bn128_supported(ROW, ROW, act, O_BF16));
+  const Plan p = plan_tiles(M, N, K, act, true, bn128_supported(ROW, ROW, act, O_BF16), ROW);
   *form = p.form;
   return p.m1 < 0 ? -1 : (int)std::min<long>(M, p.m1 * 256L);
 }
@@ -1567,6 +1571,33 @@ extern "C" int rt_token_plan(int M, int N, int K, int act, int* bn) {
   return s;
 }
 
+// The parts in which an NN product (the gradient of a linear layer's input) sums its nk K-steps, and *bn, the columns of its tiles;
+// 1: not split. Its tiles are few where the rows are few, and then each is one long chain: with tiles for half the chip at most
+// the parts of K go to the other CUs, as slabs that rt_gemm_splitk_reduce adds up. us a K-step, fitted to M of 115 to 2048, N of
+// 2048 and 4096 and K of 2048 to 28672 (within 12 %): 0.80 of 256 x 128 and 1.25 of 256 x 256, on more than 128 CUs up to 0.15 and
+// 0.27 more; the slabs are written and read at 2.3 TB/s together. N = 4096, us: 115 rows of K = 28672 360 -> 66, 500 361 -> 122, 1000
+// 384 -> 217, 1656 398 -> 366, 2048 419 -> 379; 500 rows of K = 4096 58 -> 34.
+extern "C" int rt_nn_split(int M, int N, int nk, int* bn) {
+  *bn = 0;
+  const int tiles = (M + 255) / 256 * ((N + 255) / 256), cus = num_cus();
+  if (M <= 0 || N % 8 || tiles > cus / 2 || nk < 16) return 1;
+  auto step = [&](int wgs, int cols) {
+    const float more = std::max(0.f, (float)(wgs - cus / 2) / (float)(cus / 2));
+    return cols == 128 ? 0.80f + 0.15f * more : 1.25f + 0.27f * more;
+  };
+  const int tiles128 = (M + 255) / 256 * ((N + 127) / 128);
+  float best = 0.97f * std::min((float)nk * step(tiles128, 128), (float)nk * step(tiles, 256));
+  int parts = 1;
+  for (int cols : {128, 256})
+    for (int s = 2; s <= 8; ++s) {
+      const int wgs = s * (cols == 128 ? tiles128 : tiles);
+      if (wgs > cus || nk / s < 8) break;
+      const float t = (float)((nk + s - 1) / s) * step(wgs, cols) + 4.f + (float)((long)s * M * N) * (4.f / 2.3e6f);
+      if (t < best) { best = t; parts = s; *bn = cols; }
+    }
+  return parts;
+}
+
 // Whether 65 to 512 rows of a product with a bias take 64 x 64 tiles, which sum those parts themselves: where they are done before a
 // split product and its reduction, 14 us, from K = 2048 on 17
 extern "C" int rt_small_tiles(int M, int N, int K, int act) {
@@ -1579,7 +1610,7 @@ static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, 
   const int M = p.M, N = p.N;
   const bool plain = layout_a == ROW && layout_b == ROW && out == O_BF16 && p.nsplit == 1 && !p.A2 && p.K >= 64 && p.K % 64 == 0 &&
                      p.lda < (1 << 22) && p.ldb < (1 << 22) && (act == E_NONE || act == E_GELU);  // 32-bit byte offsets within a tile
-  const Plan pl = plan_tiles(M, N, p.K, act, plain, bn128_supported(layout_a, layout_b, act, out) && p.nsplit == 1 && (out == O_BF16 || out == O_F32));
+  const Plan pl = plan_tiles(M, N, p.K, act, plain, bn128_supported(layout_a, layout_b, act, out) && p.nsplit == 1 && (out == O_BF16 || out == O_F32), layout_b);
   if (pl.m1 < 0) {
     const dim3 grid((unsigned)((M + 255) / 256 * (long)((N + 127) / 128))), block(256);
     if (act == E_GELU) hipLaunchKernelGGL(gemm_duo_kernel<E_GELU>, grid, block, 0, stream, p);

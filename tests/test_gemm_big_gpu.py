@@ -45,6 +45,22 @@ def test_nn(M, N, K):
     _close(ops.gemm_nn(dy, w), dy.float() @ w.float())
 
 
+@pytest.mark.parametrize("M,N,K,R", [(1, 8, 1024, 0), (65, 520, 1032, 8), (256, 256, 4096, 48), (257, 264, 8200, 64), (1000, 1024, 4096, 16),
+                                     (1656, 4096, 10240, 0)])
+def test_nn_in_parts(M, N, K, R):
+    """Gradients whose K is split: ragged rows, columns and K, the adapter's K-extension in the last part, against fp32. A part's sum
+    and the parts' are fp32, so the result is the fp32 one rounded to bf16 once: 2^-8 of it, and 2^-18 of the terms' absolute sum for
+    the order of the additions."""
+    dy, w = _r(M, K), _r(K, N, s=1 / math.sqrt(K))
+    du, a = (_r(M, R), _r(R, N, s=0.1)) if R else (None, None)
+    want, size = dy.double() @ w.double(), dy.double().abs() @ w.double().abs()
+    if R:
+        want, size = want + du.double() @ a.double(), size + du.double().abs() @ a.double().abs()
+    got = ops.gemm_nn(dy, w, du, a)
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -18 * size).all()
+    assert torch.equal(got, ops.gemm_nn(dy, w, du, a))
+
+
 @pytest.mark.parametrize("T,P,Q,split", [(1000, 64, 512, 0), (4096, 512, 1024, 1), (776, 264, 136, 3)])
 def test_tn_splitk(T, P, Q, split):
     T8 = T

@@ -128,3 +128,16 @@ def test_token_plans():
         assert not small_tiles(64, 768, 768, act) and not small_tiles(513, 768, 768, act) and not small_tiles(300, 768, 776, act)
         assert not small_tiles(512, 10240, 2560, act) and not small_tiles(300, 768, 3136, act)
     assert not small_tiles(300, 768, 768, 1)
+
+
+def test_nn_split():
+    """Products of a gradient with few tiles: K in parts that do not take more than a round, the ones that were the fastest when timed;
+    whole where the tiles fill half the chip, where K is short and where the sums of the parts cost more than they save."""
+    from rag_tl_domainllm_optimizer_amd import ops
+
+    split = ops.native().nn_split
+    for M, N, K, want in ((115, 4096, 28672, (8, 128)), (500, 4096, 28672, (8, 256)), (1000, 4096, 28672, (4, 256)),
+                          (1656, 4096, 28672, (2, 256)), (2048, 4096, 28672, (2, 256)), (1000, 4096, 4096, (2, 128))):
+        assert split(M, N, K // 64) == want, (M, N, K)
+    for M, N, K in ((2049, 4096, 28672), (4016, 4096, 28672), (1656, 4096, 4096), (1656, 4096, 6144), (256, 256, 960), (115, 4092, 28672)):
+        assert split(M, N, K // 64)[0] == 1, (M, N, K)
