@@ -4,13 +4,14 @@
 //
 // K is summed in the parts, and the parts in the order, of the kernel that ops.gemm takes for the shape (see Args), so that the
 // bits are that kernel's: a text's embedding does not depend on the way it went. The 8 waves of a workgroup are parts x row tiles
-// x column groups of 16; a wave has most of its weight loads (MFMA fragments, 16 B a lane straight from the row-major weight) in
-// flight at once, and partial sums meet in LDS. With a norm ahead every workgroup normalises the rows itself, two or four to a
-// wave, under those loads (12 KB from L2, where a kernel of its own costs a launch and another trip); workgroup 0 also writes them.
-// Bound by latency. 15 rows, us,
-// gemm_decode_kernel -> this: 1152 x 384 5.2 -> 4.0, 1536 x 384 with GELU 5.8 -> 4.4, 384 x 1536 9.8 -> 5.2, and 2.9 of the norm
-// with it; 20 rows, gemm_m64_kernel or the wide one: 6.6 -> 4.9, 11.0 -> 5.3, 21.3 -> 7.1. From 33 rows on gemm_mid_kernel's tiles
-// are ahead.
+// x column groups of 16; a wave has most of its weights (and of x) in flight at once, and partial sums meet in LDS. They come by
+// LDS-DMA, eight lanes to a row's 128 B, into places of the wave's own: loads straight in MFMA order, whose adjacent lanes are in
+// different rows, keep the CU's address path busy for 61 cycles each, these for 28. With a norm ahead every workgroup normalises
+// the rows itself, two or four to a wave, over the weights' trip (12 KB from L2, where a kernel of its own costs a launch and
+// another trip); workgroup 0 also writes them.
+// Bound by latency. 15 rows, us, gemm_decode_kernel -> MFMA-order loads -> this: 1152 x 384 5.2 -> 4.5 -> 4.0, 384 x 384 (4.5 -> 4.0),
+// 384 x 1536 9.8 -> 5.8 -> 4.4, and 2.9 of the norm with it. MiniLM over 15 / 32 rows 157 -> 141 / 201 -> 167, mpnet-base (and with
+// wave_reduce) 428 -> 345 / 620 -> 452. From 33 rows on gemm_mid_kernel's tiles are ahead.
 #include "rt_common.h"
 #include "rt_gelu.h"
 
@@ -30,10 +31,18 @@ struct Args {
   float eps;
 };
 
+typedef __attribute__((address_space(3))) void lds_void;
+
+// no template: hipcc's host pass drops kernels that call the builtin with dependent arguments
+__device__ __forceinline__ void dma16(const bf16_t* from, char* to) { __builtin_amdgcn_global_load_lds(from, (lds_void*)to, 16, 0, 0); }
+
 // RT: row tiles of 16 a wave; NW: 16-B vectors of a row a lane normalises (0: no norm ahead), of up to 16 TR rows
 template <int RT, int NW, int TR>
-__global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
+__global__ __launch_bounds__(512, 2) void few_rows_kernel(Args p) {
   constexpr int LDX = NW * 512 + 8;  // K <= 512 NW; an odd number of 16-B chunks where K is a multiple of 16
+  // D chunks of 64 k under way a wave: 16 weight rows, and without a norm 16 RT rows of x, of 128 B each
+  constexpr int XT = NW ? 0 : RT, CH = (1 + XT) * 2048, D = NW == 0 ? (RT == 1 ? 4 : 3) : NW * TR > 2 ? 4 : 6;
+  __shared__ __attribute__((aligned(16))) char ring[8 * D * CH];
   __shared__ __attribute__((aligned(16))) bf16_t xs[NW ? TR * 16 * LDX : 8];
   __shared__ f32x4 red[16][64];  // [part][column group][row tile]
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -42,16 +51,30 @@ __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
   const int ks = wid % p.ks, rs = wid / p.ks % p.rs, cg = wid / (p.ks * p.rs);
   const int n0 = (blockIdx.x * CG + cg) * 16;
   const bool on = n0 < p.N && rs * RT * 16 < p.M;
-  auto begin = [&](int part) { return 2 * (part * nc / p.parts); };  // in steps of 32
-  const bf16_t* const wp = p.w + (long)min(n0 + r16, p.N - 1) * p.ldw + 8 * g;
-  constexpr int D = RT == 1 ? 12 : 8;  // weight fragments in flight (without a norm in 128 registers)
-  bf16x8 wf[D];
-  int s0 = 0, s1 = 0;
-  if (on && ks < p.parts) { s0 = begin(ks); s1 = begin(ks + 1); }
+  auto begin = [&](int part) { return part * nc / p.parts; };  // in chunks
+  // load j of 8 rows: lane -> row 8 j + lane / 8, 16-B slot lane % 8 of it holding k chunk slot ^ (row / 2 % 8)
+  const bf16_t *wp[2], *xp[XT ? 2 * XT : 1];
 #pragma unroll
-  for (int k = 0; k < D; ++k)
-    if (s0 + k < s1) wf[k] = *(const bf16x8*)(wp + (s0 + k) * 32);
-
+  for (int j = 0; j < 2; ++j) {
+    const int row = 8 * j + (lane >> 3), kc = ((lane & 7) ^ (row >> 1)) * 8;
+    wp[j] = p.w + (long)min(n0 + row, p.N - 1) * p.ldw + kc;
+#pragma unroll
+    for (int t = 0; t < XT; ++t) xp[2 * t + j] = p.x + (long)min(16 * (rs * RT + t) + row, p.M - 1) * p.ldx + kc;
+  }
+  char* const mine = ring + wid * D * CH;
+  int c0 = 0, c1 = 0;
+  if (on && ks < p.parts) { c0 = begin(ks); c1 = begin(ks + 1); }
+  auto ask = [&](int c) {
+#pragma unroll
+    for (int k = 0; k < D; ++k)
+      if (c + k < c1)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          dma16(wp[j] + (c + k) * 64, mine + k * CH + j * 1024);
+#pragma unroll
+          for (int t = 0; t < XT; ++t) dma16(xp[2 * t + j] + (c + k) * 64, mine + k * CH + (2 + 2 * t + j) * 1024);
+        }
+  };
   if constexpr (NW > 0) {
     // rows of the norm: the arithmetic of norm_rows_kernel
     const int nv = p.K / 8;
@@ -75,6 +98,7 @@ __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
         wr[i] = *(const uint4*)(p.lw + (lane + 64 * i) * 8);
         br[i] = *(const uint4*)(p.lb + (lane + 64 * i) * 8);
       }
+    ask(c0);  // behind the rows, which the norm waits for
 #pragma unroll
     for (int k = 0; k < RW; ++k) {
       const int row = wid + 8 * k;
@@ -128,32 +152,36 @@ __global__ __launch_bounds__(512, NW ? 2 : 4) void few_rows_kernel(Args p) {
     }
     __syncthreads();
   }
+  if constexpr (NW == 0) ask(c0);
   for (int part = ks; part < p.parts; part += p.ks) {
-    if (part > ks && on) { s0 = begin(part); s1 = begin(part + 1); }
+    if (part > ks && on) { c0 = begin(part); c1 = begin(part + 1); }
     f32x4 acc[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s = s0; s < s1; s += D) {
-      if (s > s0 || part > ks) {
+    for (int c = c0; c < c1; c += D) {
+      if (c > c0 || part > ks) ask(c);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      bf16x8 wf[D][2], xf[D][2][RT];
 #pragma unroll
-        for (int k = 0; k < D; ++k)
-          if (s + k < s1) wf[k] = *(const bf16x8*)(wp + (s + k) * 32);
-      }
-      bf16x8 xf[D][RT];
+      for (int k = 0; k < D; ++k)  // all places, asked for or not: the reads go out together
 #pragma unroll
-      for (int k = 0; k < D; ++k)
-        if (s + k < s1)
+        for (int h = 0; h < 2; ++h) {
+          const char* const img = mine + k * CH + r16 * 128 + (((4 * h + g) ^ (r16 >> 1)) << 4);
+          wf[k][h] = *(const bf16x8*)img;
 #pragma unroll
           for (int t = 0; t < RT; ++t) {
-            const int row = 16 * (rs * RT + t) + r16, col = (s + k) * 32 + 8 * g;
-            if constexpr (NW > 0) xf[k][t] = *(const bf16x8*)(xs + row * LDX + col);
-            else xf[k][t] = *(const bf16x8*)(p.x + (long)min(row, p.M - 1) * p.ldx + col);
+            const int row = 16 * (rs * RT + t) + r16, col = min(c + k, c1 - 1) * 64 + h * 32 + 8 * g;
+            xf[k][h][t] = *(const bf16x8*)(NW > 0 ? (const char*)(xs + row * LDX + col) : img + (1 + t) * 2048);
           }
+        }
 #pragma unroll
       for (int k = 0; k < D; ++k)
-        if (s + k < s1)
+        if (c + k < c1)
 #pragma unroll
-          for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k], xf[k][t], acc[t], 0, 0, 0);
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k][h], xf[k][h][t], acc[t], 0, 0, 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next chunks take their place
     }
     // acc[t][e]: row 16 (rs RT + t) + r16, column n0 + 4 g + e
 #pragma unroll
