@@ -161,6 +161,10 @@ __device__ void topk_select(const float* s, int N, int K, TopkShared& sh) {
 // every candidate counts the candidates ahead of it, which is its place in the result. Two passes over the row at
 // most, no histogram, no sort (four passes and a sort of 1024 before): top 16 of 512 and top 3 of 9600, one row,
 // 88 -> 8.3 and 10.8 us each. Loads of both passes go out in blocks: top 3 of 100k, one row and 200 (top 5), 27 -> 20 and 47 -> 30.
+// Up to k = 32 the bound is the k-th largest of 64 maxima, a wave's lanes' (32 rounds of one ballot, where 16 of them took 3 us of a
+// row's 10; two candidates more at k = 16, 13 at 32); a row of eight elements a thread is read once; and up to 64 candidates, all
+// but rows of many ties, are ranked in the registers of one wave: the two above 7.0 -> 5.5 and 10.7 -> 5.4, of 100k 20 -> 13.6
+// and 30 -> 23, 65536 rows of 512 56 -> 50.
 // Rows with more than TOPK_CAND candidates go through topk_select first.
 // NT: a wave where its 64 maxima suffice (k <= 32) and hold 16 elements each at most (k-means assignment: 65536 rows
 // of 512), 1024 threads for long rows, 256 between.
@@ -194,32 +198,77 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
         if (i0 + e * NT < N) use(v[e], i0 + e * NT);
     }
   };
-  scan([&](float v, int) { km = max(km, okey(v)); });
+  // a row of at most eight a thread is read once
+  float own[8];
+  const bool few = N > 0 && N <= 8 * NT;
+  if (few) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) own[e] = s[min(tid + e * NT, N - 1)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (tid + e * NT < N) km = max(km, okey(own[e]));
+  } else {
+    scan([&](float v, int) { km = max(km, okey(v)); });
+  }
   tmax[tid] = km;
   if (tid == 0) sh.cnt = 0;
   __syncthreads();
   if (tid < 64) {
-    uint32_t t[NT / 64];
+    uint32_t t[NT / 64], one[1] = {0};
 #pragma unroll
-    for (int i = 0; i < NT / 64; ++i) t[i] = tmax[lane + 64 * i];
-    const uint32_t thr = K <= NT ? wave_kth(t, K) : 0;
+    for (int i = 0; i < NT / 64; ++i) {
+      t[i] = tmax[lane + 64 * i];
+      one[0] = max(one[0], t[i]);
+    }
+    const uint32_t thr = K <= 32 ? wave_kth(one, K) : K <= NT ? wave_kth(t, K) : 0;
     if (lane == 0) sh.sel = thr;
   }
   __syncthreads();
   const uint32_t thr = sh.sel;
-  if (km >= thr)
-    scan([&](float v, int i) {
+  if (km >= thr) {
+    auto take = [&](float v, int i) {
       if (okey(v) >= thr) {
         const unsigned slot = atomicAdd(&sh.cnt, 1u);
         if (slot < TOPK_CAND) { sh.cv[slot] = v; sh.ci[slot] = i; }
       }
-    });
+    };
+    if (few) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (tid + e * NT < N) take(own[e], tid + e * NT);
+    } else {
+      scan(take);
+    }
+  }
   __syncthreads();
   int n = (int)sh.cnt;
   if (n > TOPK_CAND) {
     __syncthreads();  // every thread has read cnt
     topk_select<NT>(s, N, K, sh);
     n = K;
+  }
+  for (int i = K + tid; i < k; i += NT) topk_write(-INFINITY, 0x7fffffff, k, i, row, idmap, ldmap, finite, out_v, out_i);
+  if (n <= 64) {  // a candidate a lane, as below
+    if (tid >= 64) return;
+    const bool in = lane < n;
+    const float v = in ? sh.cv[lane] : 0.f;
+    const int idx = in ? sh.ci[lane] : 0;
+    const long id = idmap ? in ? idmap[row * ldmap + idx] : 0 : idx;
+    const uint32_t raw = okey(v), key = okey(v + 0.f);
+    int above = 0, at = 0;
+    for (int i = 0; i < n; ++i) above += (uint32_t)__builtin_amdgcn_readlane((int)raw, i) > raw;
+    const bool keeps = in && above < K;
+    for (unsigned long long left = __ballot(keeps); left; left &= left - 1) {
+      const int i = __builtin_ctzll(left);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)key, i);
+      const int oi = __builtin_amdgcn_readlane(idx, i);
+      at += o > key || (o == key && oi < idx);
+    }
+    if (keeps && at < K) {
+      out_v[row * k + at] = v;
+      out_i[row * k + at] = finite && !(fabsf(v) < INFINITY) ? -1 : id;
+    }
+    return;
   }
   // those with fewer than K keys above their own, then their places by value and index
   for (int j = tid; j < n; j += NT) {
@@ -242,7 +291,6 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
       }
       if (at < K) topk_write(v, idx, k, at, row, idmap, ldmap, finite, out_v, out_i);
     }
-  for (int i = K + tid; i < k; i += NT) topk_write(-INFINITY, 0x7fffffff, k, i, row, idmap, ldmap, finite, out_v, out_i);
 }
 
 // IVF list scan: for query qi and its probe p (list L = probes[qi, p]), score every vector of the

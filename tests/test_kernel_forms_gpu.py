@@ -166,6 +166,22 @@ def test_topk_forms(nq, N, k):
         assert bool((v[:, n:] == float("-inf")).all()) and bool((i[:, n:] == -1).all())
 
 
+@pytest.mark.parametrize("N,k", [(8, 3), (512, 32), (513, 32), (2048, 33), (2049, 20), (8192, 31), (8193, 7)])
+def test_topk_candidates_around_a_wave(N, k):
+    """Rows of at most eight elements a thread and just longer ones, with a wave's worth of candidates and one more or less at
+    the k-th score: the order of a stable sort."""
+    g = torch.Generator(device=DEV).manual_seed(N + k)
+    s = torch.rand(8, N, generator=g, device=DEV) - 2
+    for r, ties in enumerate((1, 3, 62, 63, 64, 65, 66)):
+        at = torch.randperm(N, generator=g, device=DEV)[:ties]
+        s[r, at] = 0.0
+        s[r, at[0]] = 1.0
+    cid = torch.randint(0, 1 << 40, s.shape, generator=g, device=DEV)
+    vs, order = torch.sort(s, dim=-1, descending=True, stable=True)
+    v, i = ops.topk(s, k, cid)
+    assert torch.equal(v, vs[:, :k]) and torch.equal(i, cid.gather(1, order)[:, :k])
+
+
 @pytest.mark.parametrize("N,k", [(1500, 3), (5000, 3), (5000, 128), (9600, 40), (100003, 512)])
 def test_topk_rows_with_more_ties_than_candidates(N, k):
     """Rows whose k-th score is shared by more entries than the candidate list holds: all larger scores come first, then the
