@@ -168,6 +168,13 @@ __device__ __forceinline__ float over_groups(float x, F f) {
   return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+// lane i (0 .. 3, known where it is unrolled) of every row of 16 lanes
+__device__ __forceinline__ float row_lane(float x, int i) {
+#define RT_BCAST(n) __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x150 + n, 0xf, 0xf, false))
+  return i == 0 ? RT_BCAST(0) : i == 1 ? RT_BCAST(1) : i == 2 ? RT_BCAST(2) : RT_BCAST(3);
+#undef RT_BCAST
+}
+
 // D = A.B + D on a 16x16x32 bf16 MFMA with D tied to AGPRs ("+a") and a "memory" clobber that pins
 // surrounding loads / LDS-DMA issues to their source position (gemm_big.hip's 4-wave kernels).
 // The x86 host pass parses kernel bodies too and has no AGPR constraint: the asm is device-pass only.

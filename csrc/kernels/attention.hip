@@ -291,8 +291,7 @@ void attn_fwd_kernel(AttnArgs a) {
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[t][u][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
       const float mn = fmaxf(m[u], mx);
       const float mu = mn == -INFINITY ? 0.f : mn;
       alpha[u] = exp2_raw(m[u] - mu);
@@ -306,8 +305,7 @@ void attn_fwd_kernel(AttnArgs a) {
           st[t][u][i] = pv;
           rs += pv;
         }
-      rs += __shfl_xor(rs, 16, 64);
-      rs += __shfl_xor(rs, 32, 64);
+      rs = over_groups(rs, [](float x, float y) { return x + y; });
       l[u] = l[u] * alpha[u] + rs;
     }
     // rescale O rows (row q = 16u + 4g + i lives in lane 4g+i's alpha)
@@ -752,7 +750,7 @@ struct DecodeFusedArgs {
   // optional: qkv as nsplit fp32 split-K slabs [nsplit][B][ldq] (the qkv GEMM's reduce fused into
   // the MFMA kernel's prologue); qkv above is then unused
   const float* qkv_slabs; int qkv_nsplit; long qkv_sstride;
-  int kv_nt;                        // MFMA kernel: non-temporal K/V cache loads (each read once per step)
+  int kv_nt;                        // non-temporal K/V cache loads (each read once per step)
   long long* stamps;                // debug (W > 1 kernel): [blocks * W][8] s_memrealtime phase stamps, or null
   // fp8 K/V cache (config 5, MFMA kernels only): kc / vc hold OCP e4m3fn bytes, one fp32 scale per
   // (batch, kv head, slot) in ksc / vsc [B, Hkv, SmaxP]; K rows are stored k-permuted (element
@@ -1156,8 +1154,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 #pragma unroll
       for (int e = 0; e < 8; ++e) amk = fmaxf(amk, fabsf(f[e]));
     }
-    amk = fmaxf(amk, __shfl_xor(amk, 16, 64));
-    amk = fmaxf(amk, __shfl_xor(amk, 32, 64));
+    amk = over_groups(amk, [](float x, float y) { return fmaxf(x, y); });
     unpack8(vx, f);
 #pragma unroll
     for (int e = 0; e < 8; ++e) amv = fmaxf(amv, fabsf(f[e]));
@@ -1215,8 +1212,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
       dot = fmaf(q[4 * w2 + 2], hi.x, dot);
       dot = fmaf(q[4 * w2 + 3], hi.y, dot);
     }
-    dot += __shfl_xor(dot, 16, 64);
-    dot += __shfl_xor(dot, 32, 64);
+    dot = over_groups(dot, [](float x, float y) { return x + y; });
     const float sc = c0 + r < len ? dot * ks : -INFINITY;
     float mx = sc;
 #pragma unroll
@@ -1262,8 +1258,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
   // the 4 lane groups hold disjoint key subsets of the same 8 dims
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    o[e] += __shfl_xor(o[e], 16, 64);
-    o[e] += __shfl_xor(o[e], 32, 64);
+    o[e] = over_groups(o[e], [](float x, float y) { return x + y; });
   }
   // merge the waves' (m, l, O) (m = -inf, l = 0 for a wave without tiles)
   if (lane == 0) { mrg[w][0] = m; mrg[w][1] = l; }
@@ -1310,8 +1305,12 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 // counted waits keep the prefetch in flight). The launch bound holds every form to 256 registers, 2
 // waves per SIMD: all 2048 waves of a batch-256 layer, or two workgroups of 4 waves per CU, are resident
 // (unbounded, the 4-wave form took 268 with its accumulators and ran one workgroup per CU: 48 rows of
-// 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every q / k_new /
-// v_new / rotary-table load at once (one round trip) behind the first tile's loads. RoPE of q /
+// 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every rotary-table / q /
+// k_new / v_new (or slab) load at once and the first tiles behind them: loads return in order, so the other way round
+// it waited for 24 KB a wave. All loads are unconditional, refills past the end too: behind a load under a condition
+// the compiler waits for every load at the join, and so had the three tiles arrive before the first was used, each time
+// (and lengths, slot and position one after the other: 3 trips). 1 row of 300 keys 10.5 -> 10.1 us, 48 rows of 150..1200
+// 37.9 -> 36.0, 256 rows of 173..301 (slabs) 58.9 -> 57.1. RoPE of q /
 // k_new and the cache append are fused; lanes whose (clamped) key is the new token's slot use
 // k_new / v_new from registers. Measured at batch 256 (Mistral-7B, 174..301 keys): 51 us per
 // layer vs 80 us for the VALU kernel (profiles/decode_attn_r2_mfma.log).
@@ -1329,7 +1328,7 @@ template <int G, int W, bool KV8 = false>
 __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFusedArgs a) {
   constexpr int D = 128, DS = D / 32, DT = D / 16;
   __shared__ __attribute__((aligned(16))) char vimg_all[W][32 * D * 2];  // per wave; rows 16..31 stay zero
-  __shared__ __attribute__((aligned(16))) bf16_t qkv_st[(G + 2) * D];  // slab path (W == 1): reduced q | k | v
+  __shared__ __attribute__((aligned(16))) bf16_t qkv_st[W == 1 ? (G + 2) * D : 8];  // slab path: reduced q | k | v
   const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
   const int w = W > 1 ? (int)(threadIdx.x >> 6) : 0;
   char* vimg = vimg_all[w];
@@ -1345,15 +1344,16 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
   const int NP = W > 1 ? max(a.NP, 1) : 1;
   const int part = blockIdx.x % NP, bh = blockIdx.x / NP;
   const int b = bh / a.Hkv, hk = bh % a.Hkv;
-  const int len_row = a.attn_len[b];
-  const int s_new = a.slot[b];
+  // in one trip: what is not given is read from another's place
+  const int len_row = a.attn_len[b], s_new = a.slot[b];
+  const int start_b = (a.kv_start ? a.kv_start : a.slot)[b], pos_b = (a.pos ? a.pos : a.slot)[b];
   RT_ASSERT(len_row <= a.Smax && s_new >= 0 && s_new < a.Smax);
-  int kbeg = a.kv_start ? a.kv_start[b] : 0;
+  int kbeg = a.kv_start ? start_b : 0;
   if (a.window > 0) kbeg = max(kbeg, len_row - a.window);
   // this workgroup's keys [kbeg, len): the whole row, or partition `part` of it
   const int len = NP > 1 ? min(len_row, (part + 1) * a.PS) : len_row;
   if (NP > 1) kbeg = max(kbeg, part * a.PS);
-  const int p = a.pos ? a.pos[b] : 0;
+  const int p = a.pos ? pos_b : 0;
   const bf16_t* row = a.qkv + (long)b * a.ldq;
   const bf16_t* kbase = a.kc + ((long)b * a.Hkv + hk) * a.Smax * D;
   const bf16_t* vbase = a.vc + ((long)b * a.Hkv + hk) * a.Smax * D;
@@ -1373,69 +1373,35 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
   struct Tile8 { uint4 k8[2]; uint2 v8[4]; float ks[4], vs[4]; };
   typedef typename std::conditional<KV8, Tile8, Tile16>::type Tile;
   auto load = [&](Tile& T, int c0) {
-    const long keyk = min(c0 + r16, len - 1);
+    const int last = max(len - 1, 0);  // of no keys slot 0, unused
+    const long keyk = min(c0 + r16, last);
     if constexpr (KV8) {
       T.k8[0] = load_nt16(kbase8 + keyk * D + 32 * g);
       T.k8[1] = load_nt16(kbase8 + keyk * D + 32 * g + 16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) T.v8[i] = load_nt8(vbase8 + (long)min(c0 + 4 * i + g, len - 1) * D + 8 * r16);
+      for (int i = 0; i < 4; ++i) T.v8[i] = load_nt8(vbase8 + (long)min(c0 + 4 * i + g, last) * D + 8 * r16);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int key = min(c0 + 4 * g + i, len - 1);
+        const int key = min(c0 + 4 * g + i, last);
         T.ks[i] = ksb[key];
         T.vs[i] = vsb[key];
       }
-    } else if (a.kv_nt) {
-#pragma unroll
-      for (int s2 = 0; s2 < DS; ++s2) T.k[s2] = load_nt16(kbase + keyk * D + 32 * s2 + 8 * g);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) T.v[i] = load_nt16(vbase + (long)min(c0 + 4 * i + g, len - 1) * D + 8 * r16);
     } else {
+      // K plainly: both 64-B halves of a line are read, by two of these
 #pragma unroll
       for (int s2 = 0; s2 < DS; ++s2) T.k[s2] = *(const uint4*)(kbase + keyk * D + 32 * s2 + 8 * g);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const long key = min(c0 + 4 * i + g, len - 1);
-        T.v[i] = *(const uint4*)(vbase + key * D + 8 * r16);
-      }
+      for (int i = 0; i < 4; ++i) T.v[i] = load_nt16(vbase + (long)min(c0 + 4 * i + g, last) * D + 8 * r16);
     }
   };
   Tile ta, tb, tc;
   const int cfirst = kbeg + 16 * w, cstep = 16 * W;  // this wave's tiles: cfirst + j * cstep
-  if (cfirst < len) load(ta, cfirst);
-  if (cfirst + cstep < len) load(tb, cfirst + cstep);
-  if (cfirst + 2 * cstep < len) load(tc, cfirst + 2 * cstep);
-
-  // ---- q / k_new / v_new and the rotary tables, all loads at once. D = 128: chunk 4 s + g's
+  // ---- the rotary tables and q / k_new / v_new, then the first tiles: loads return in order, and the
+  // tiles are many. D = 128: chunk 4 s + g's
   // rotary partner (chunk ^ 8) is the lane's own chunk 4 (s ^ 2) + g, its table offset
   // ((chunk & 7) * 8) depends on s & 1 only ----
   const bool rot = a.cosT != nullptr;
   const bool has_new = s_new >= kbeg && s_new < len;
-  const bf16_t* qrow = row + (long)min(hk * G + r16, a.Hq - 1) * D;
-  const bf16_t* krow = row + (long)(a.Hq + hk) * D;
-  const bf16_t* vrow = row + (long)(a.Hq + a.Hkv + hk) * D;
-  if (a.qkv_slabs) {
-    // split-K slabs of the qkv GEMM: this wave sums its (G + 2) x D slice once (in the order and
-    // with the bf16 rounding of splitk_reduce_kernel) into LDS, and reads q / k / v from there
-    constexpr int NCHK = (G + 2) * (D / 8);
-    for (int ch = lane; ch < NCHK; ch += 64) {
-      const int seg = ch / (D / 8), c8 = ch % (D / 8);
-      const int head = seg < G ? hk * G + seg : (seg == G ? a.Hq + hk : a.Hq + a.Hkv + hk);
-      float t8[8];
-      sum_slabs8(a.qkv_slabs + (long)b * a.ldq + (long)head * D + c8 * 8, a.qkv_sstride, a.qkv_nsplit, t8);
-      *(uint4*)(qkv_st + seg * D + c8 * 8) = pack8(t8);
-    }
-    qrow = qkv_st + min(r16, G - 1) * D;
-    krow = qkv_st + G * D;
-    vrow = qkv_st + (G + 1) * D;
-  }
-  uint4 qraw[DS], kraw[DS];
-#pragma unroll
-  for (int s2 = 0; s2 < DS; ++s2) {
-    qraw[s2] = *(const uint4*)(qrow + (4 * s2 + g) * 8);
-    kraw[s2] = *(const uint4*)(krow + (4 * s2 + g) * 8);
-  }
-  const uint4 vx = *(const uint4*)(vrow + r16 * 8);
   float4 cq[2][2], sq[2][2];
   {
     // unconditional (no branch between load batches): without tables read the qkv row
@@ -1448,6 +1414,63 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
       sq[par][0] = *(const float4*)(stb + j0); sq[par][1] = *(const float4*)(stb + j0 + 4);
     }
   }
+  uint4 qraw[DS], kraw[DS], vx;
+  auto raw = [&](const bf16_t* qrow, const bf16_t* krow, const bf16_t* vrow) {
+#pragma unroll
+    for (int s2 = 0; s2 < DS; ++s2) {
+      qraw[s2] = *(const uint4*)(qrow + (4 * s2 + g) * 8);
+      kraw[s2] = *(const uint4*)(krow + (4 * s2 + g) * 8);
+    }
+    vx = *(const uint4*)(vrow + r16 * 8);
+  };
+  if (W == 1 && a.qkv_slabs) {
+    // split-K slabs of the qkv GEMM: this wave sums its (G + 2) x D slice once (in the order and
+    // with the bf16 rounding of splitk_reduce_kernel) into LDS, and reads q / k / v from there. 4 columns a lane
+    // and pass, three passes' loads (G = 4: all) in flight
+    constexpr int NP4 = (G + 2) * (D / 4), AT_ONCE = 3;
+#pragma unroll
+    for (int u0 = 0; u0 < NP4; u0 += 64 * AT_ONCE) {
+      float4 x[AT_ONCE][8];
+      const float* sp[AT_ONCE];
+#pragma unroll
+      for (int u = 0; u < AT_ONCE; ++u) {
+        const int c = min(u0 + 64 * u + lane, NP4 - 1), seg = c / (D / 4);
+        const int head = seg < G ? hk * G + seg : (seg == G ? a.Hq + hk : a.Hq + a.Hkv + hk);
+        sp[u] = a.qkv_slabs + (long)b * a.ldq + (long)head * D + c % (D / 4) * 4;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[u][q] = *(const float4*)(sp[u] + (long)min(q, a.qkv_nsplit - 1) * a.qkv_sstride);
+      }
+      if (u0 == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        load(ta, cfirst);
+        load(tb, cfirst + cstep);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int u = 0; u < AT_ONCE; ++u) {
+        const int c = u0 + 64 * u + lane;
+        float4 y = x[u][0];
+#pragma unroll
+        for (int q = 1; q < 8; ++q) {  // y + -0 is y
+          const bool in = q < a.qkv_nsplit;
+          y.x += in ? x[u][q].x : -0.f; y.y += in ? x[u][q].y : -0.f; y.z += in ? x[u][q].z : -0.f; y.w += in ? x[u][q].w : -0.f;
+        }
+        for (int q = 8; q < a.qkv_nsplit; ++q) {
+          const float4 z = *(const float4*)(sp[u] + (long)q * a.qkv_sstride);
+          y.x += z.x; y.y += z.y; y.z += z.z; y.w += z.w;
+        }
+        if (c < NP4) *(uint2*)(qkv_st + c * 4) = make_uint2(pack2bf(y.x, y.y), pack2bf(y.z, y.w));
+      }
+    }
+    raw(qkv_st + min(r16, G - 1) * D, qkv_st + G * D, qkv_st + (G + 1) * D);
+  } else {
+    raw(row + (long)min(hk * G + r16, a.Hq - 1) * D, row + (long)(a.Hq + hk) * D, row + (long)(a.Hq + a.Hkv + hk) * D);
+    __builtin_amdgcn_sched_barrier(0);
+    load(ta, cfirst);
+    load(tb, cfirst + cstep);
+  }
+  load(tc, cfirst + 2 * cstep);
+  __builtin_amdgcn_sched_barrier(0);
   // x rotated with partner y: lo half (chunk < 8) x c - y s', hi half x c + y s' (s' = sign sin),
   // rounded to bf16 as the unfused rope kernel stores it
   auto rope8 = [&](const uint4& xv, const uint4& yv, const float4 (&c)[2], const float4 (&sn)[2], bool lo) -> uint4 {
@@ -1487,8 +1510,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
 #pragma unroll
       for (int e = 0; e < 8; ++e) amk = fmaxf(amk, fabsf(f[e]));
     }
-    amk = fmaxf(amk, __shfl_xor(amk, 16, 64));  // lane group g holds chunks 4 s + g
-    amk = fmaxf(amk, __shfl_xor(amk, 32, 64));
+    amk = over_groups(amk, [](float x, float y) { return fmaxf(x, y); });  // lane group g holds chunks 4 s + g
     unpack8(vx, f);
 #pragma unroll
     for (int e = 0; e < 8; ++e) amv = fmaxf(amv, fabsf(f[e]));
@@ -1593,8 +1615,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
       st[i] = x;
       mx = fmaxf(mx, x);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
     const float mn = fmaxf(m, mx);  // finite: every tile holds >= 1 valid key
     const float alpha = exp2_raw(m - mn);
     m = mn;
@@ -1605,14 +1626,13 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
       st[i] = KV8 ? pv * vs[i] : pv;  // fp8: the V scale of key c0 + 4 g + i rides on P
       rs += pv;
     }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
+    rs = over_groups(rs, [](float x, float y) { return x + y; });
     l = l * alpha + rs;
     // O rows are heads 4 g + i: their factors live in lanes 4 g + i. Only rows < G are ever
     // stored or merged (an O row depends on its own P row only), so G < 4 rescales G rows
 #pragma unroll
     for (int i = 0; i < (G < 4 ? G : 4); ++i) {
-      const float al = __shfl(alpha, 4 * g + i, 64);
+      const float al = G <= 4 ? row_lane(alpha, i) : __shfl(alpha, 4 * g + i, 64);
 #pragma unroll
       for (int c = 0; c < DT; ++c) o[c][i] *= al;
     }
@@ -1629,18 +1649,15 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
   };
 
   // three tiles in flight (all of a wave's tiles at up to 48 W keys: one memory round trip); a register
-  // set is refilled right after its tile is consumed
+  // set is refilled right after its tile is consumed, behind the end with the last key: a load under a
+  // condition would make the compiler wait for all of them at every join
   for (int c0 = cfirst; c0 < len; c0 += 3 * cstep) {
     consume(ta, c0);
-    if (c0 + 3 * cstep < len) load(ta, c0 + 3 * cstep);
-    if (c0 + cstep < len) {
-      consume(tb, c0 + cstep);
-      if (c0 + 4 * cstep < len) load(tb, c0 + 4 * cstep);
-    }
-    if (c0 + 2 * cstep < len) {
-      consume(tc, c0 + 2 * cstep);
-      if (c0 + 5 * cstep < len) load(tc, c0 + 5 * cstep);
-    }
+    load(ta, c0 + 3 * cstep);
+    if (c0 + cstep < len) consume(tb, c0 + cstep);
+    load(tb, c0 + 4 * cstep);
+    if (c0 + 2 * cstep < len) consume(tc, c0 + 2 * cstep);
+    load(tc, c0 + 5 * cstep);
   }
   if constexpr (W == 1) {
     // ---- normalise and store: lane holds O[head 4 g + i][d = 16 c + r16] ----

@@ -318,8 +318,7 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
       }
       float mx = fmaxf(fmaxf(fmaxf(s2[0][0], s2[0][1]), fmaxf(s2[0][2], s2[0][3])),
                        fmaxf(fmaxf(s2[1][0], s2[1][1]), fmaxf(s2[1][2], s2[1][3])));
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
       // every tile holds a key of the row, so mn is finite; scale > 0 (launcher)
       const float mn = fmaxf(m[n], mx * a.scale_log2);
       const float alpha = fexp2(m[n] - mn);
@@ -333,8 +332,7 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
           s2[k][i] = p;
           rs += p;
         }
-      rs += __shfl_xor(rs, 16, 64);
-      rs += __shfl_xor(rs, 32, 64);
+      rs = over_groups(rs, [](float x, float y) { return x + y; });
       l[n] = l[n] * alpha + rs;
       pa[n] = pack_p(s2[0], s2[1]);
       // O^T: the head is the lane's column, as in the scores (most tiles bring no new maximum)
@@ -528,8 +526,7 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(PreArgs a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)
         mx = fmaxf(mx, fmaxf(fmaxf(stt[t][u][0], stt[t][u][1]), fmaxf(stt[t][u][2], stt[t][u][3])));
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
       const float mn = fmaxf(m[u], mx * a.scale_log2);  // scale > 0 (launcher); key 0 keeps it finite
       alpha[u] = fexp2(m[u] - mn);
       m[u] = mn;
@@ -542,8 +539,7 @@ __global__ __launch_bounds__(256, 2) void latent_prefill_kernel(PreArgs a) {
           stt[t][u][i] = p;
           rs += p;
         }
-      rs += __shfl_xor(rs, 16, 64);
-      rs += __shfl_xor(rs, 32, 64);
+      rs = over_groups(rs, [](float x, float y) { return x + y; });
       l[u] = l[u] * alpha[u] + rs;
     }
     // O^T: the query is the lane's column, as in the scores (most tiles bring no new maximum)

@@ -321,8 +321,7 @@ __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
       }
       float mx = fmaxf(fmaxf(fmaxf(s2[0][0], s2[0][1]), fmaxf(s2[0][2], s2[0][3])),
                        fmaxf(fmaxf(s2[1][0], s2[1][1]), fmaxf(s2[1][2], s2[1][3])));
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
       const float mn = fmaxf(m[n], mx);  // finite: every listed tile holds a visible key
       const float alpha = fexp2(m[n] - mn);
       m[n] = mn;
@@ -335,8 +334,7 @@ __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
           s2[k][e] = p;
           rs += p;
         }
-      rs += __shfl_xor(rs, 16, 64);
-      rs += __shfl_xor(rs, 32, 64);
+      rs = over_groups(rs, [](float x, float y) { return x + y; });
       l[n] = l[n] * alpha + rs;
       pa[n] = pack_p(s2[0], s2[1]);
       // O^T: the head is the lane's column, as in the scores (most tiles bring no new maximum)
