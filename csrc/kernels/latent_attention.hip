@@ -188,6 +188,9 @@ __global__ __launch_bounds__(256) void head_gemm_kernel(const bf16_t* __restrict
 //   every wave runs the same online softmax, packs P as the next MFMA's B operand, and accumulates
 //   O^T += V^T P^T (head on the lane again) for its own quarter of the latent columns (V = the latent part of the same LDS image,
 //   transposed reads). Two tiles' images are in flight or in use; three barriers per tile.
+// The pages of 64 tiles come in one load: a page's number for each tile, waited for, had all LDS-DMA under way arrive first (loads
+// return in order), so nothing was ahead. Where four or three images fit twice on a CU they are used, one barrier a tile less.
+// 16 rows of 500..1500 keys, 32 heads over 576 columns, 24 partitions of one or two tiles: 15.8 -> 15.0 us.
 // A row's keys are cut in NP equal partitions (multiples of 32) from its own length, so a captured
 // launch with a fixed NP balances every length. Image rows are CPR = 8 QS + 1 16-B chunks (odd: row
 // reads conflict-free); chunks past KD repeat the row's last one.
@@ -207,24 +210,21 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
   constexpr int NIT = (32 * CPR + 63) / 64;          // of the workgroup (the last one may be half used)
   constexpr int BUFB = NIT * 1024;
   constexpr int QF = NH == 1 ? QS : 2 * QS;          // query fragments per wave
-  __shared__ __attribute__((aligned(16))) char smem[2 * BUFB + 4096];
-  float* sx = (float*)(smem + 2 * BUFB);             // [4 waves][64 lanes][4]
+  // images of two workgroups a CU; with more than two the next one is asked for at the top of a tile, into the last tile's place
+  constexpr int NB = 4 * BUFB + 4096 <= 80 * 1024 ? 4 : 3 * BUFB + 4096 <= 80 * 1024 ? 3 : 2;
+  constexpr int AHEAD = NB == 2 ? 2 : NB - 1;        // tiles asked for before the first one's use
+  __shared__ __attribute__((aligned(16))) char smem[NB * BUFB + 4096];
+  float* sx = (float*)(smem + NB * BUFB);            // [4 waves][64 lanes][4]
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
   const int hg = bid % a.HG, part = (bid / a.HG) % a.NP, t = bid / (a.HG * a.NP);
   const int h0 = hg * 16 * NH;
-  // query fragments: lane holds Q[head r16][32 s + 8 g ..]
-  const int kt = w & 1, hi = w >> 1;                 // key half; K-dim half (NH = 1) or head tile (NH = 2)
-  const int qh = h0 + (NH == 2 ? hi * 16 : 0) + r16;
-  const int sbase = NH == 1 ? hi * QS : 0;
-  bf16x8 qf[QF];
-  const bf16_t* qp = a.q + ((long)t * a.H + min(qh, a.H - 1)) * a.KD;  // heads past the last repeat it (not stored)
-#pragma unroll
-  for (int s = 0; s < QF; ++s) qf[s] = *(const bf16x8*)(qp + min(32 * (sbase + s) + 8 * g, a.KD - 8));
-  const int row = min(max(a.row[t], 0), a.n_rows - 1);
-  const int len = min(a.pos[t] + 1, a.max_pages * PAGE);
+  int row = a.row[t], pos = a.pos[t];
+  asm volatile("" : "+s"(row), "+s"(pos));           // in one trip, also if the partition is empty
+  row = min(max(row, 0), a.n_rows - 1);
+  const int len = min(pos + 1, a.max_pages * PAGE);
   const int per = ((len + a.NP - 1) / a.NP + 31) & ~31;
   const int k0 = part * per, k1 = min(len, k0 + per);
   if (k0 >= k1) {  // nothing for this partition (uniform over the workgroup)
@@ -236,6 +236,15 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
     return;
   }
   const int* tab = a.tab + (long)row * a.max_pages;
+  int pages = tab[min(k0 + 32 * lane, k1 - 1) / PAGE];  // of 64 tiles, a tile a lane
+  // query fragments: lane holds Q[head r16][32 s + 8 g ..]
+  const int kt = w & 1, hi = w >> 1;                 // key half; K-dim half (NH = 1) or head tile (NH = 2)
+  const int qh = h0 + (NH == 2 ? hi * 16 : 0) + r16;
+  const int sbase = NH == 1 ? hi * QS : 0;
+  bf16x8 qf[QF];
+  const bf16_t* qp = a.q + ((long)t * a.H + min(qh, a.H - 1)) * a.KD;  // heads past the last repeat it (not stored)
+#pragma unroll
+  for (int s = 0; s < QF; ++s) qf[s] = *(const bf16x8*)(qp + min(32 * (sbase + s) + 8 * g, a.KD - 8));
 
   // LDS-DMA sources: instruction j of wave w covers image chunks (4 j + w) * 64 + lane
   uint32_t src[NI];  // element offset from the tile's first cache row
@@ -244,15 +253,23 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
     const int c = (4 * j + w) * 64 + lane;
     src[j] = (uint32_t)(min(c / CPR, 31) * a.KD + min(c % CPR * 8, a.KD - 8));
   }
-  auto page_of = [&](int key0) { return min(max(tab[key0 / PAGE], 0), a.n_pages - 1); };
-  auto stage = [&](int key0, int page, int buf) {
-    const bf16_t* base = a.pool + ((long)page * PAGE + key0 % PAGE) * a.KD;
+  int next = 0, place = 0;                           // the next tile to ask for, its image
+  auto stage = [&]() {
+    const int key = k0 + 32 * next;
+    if (next % 64 == 0 && next > 0) {
+      pages = tab[min(key + 32 * lane, k1 - 1) / PAGE];
+      asm volatile("" : "+v"(pages));                // waited for here, not by every tile
+    }
+    const int page = min(max(__builtin_amdgcn_readlane(pages, next % 64), 0), a.n_pages - 1);
+    const bf16_t* base = a.pool + ((long)page * PAGE + key % PAGE) * a.KD;
+    char* to = smem + place * BUFB;
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       if (4 * j + w < NIT)  // wave-uniform
-        __builtin_amdgcn_global_load_lds((const void*)(base + src[j]), (lds_void*)(smem + buf * BUFB + (4 * j + w) * 1024),
-                                         16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(base + src[j]), (lds_void*)(to + (4 * j + w) * 1024), 16, 0, 0);
     }
+    ++next;
+    place = place + 1 == NB ? 0 : place + 1;
   };
 
   f32x4 o[NH][RT];
@@ -264,25 +281,31 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
 #pragma unroll
   for (int n = 0; n < NH; ++n) { m[n] = -INFINITY; l[n] = 0.f; }
 
-  const bool more = w < NIT % 4;  // this wave issues NIT / 4 + 1 instructions per tile, else NIT / 4
-  stage(k0, page_of(k0), 0);
-  if (k0 + 32 < k1) stage(k0 + 32, page_of(k0 + 32), 1);
   if (a.KD < 64 * QS) {  // columns past KD: zero in the query, anything finite in the image
 #pragma unroll
     for (int s = 0; s < QF; ++s)
       if (32 * (sbase + s) + 8 * g >= a.KD) qf[s] = bf16x8{};
   }
 #pragma unroll
-  for (int s = 0; s < QF; ++s) asm volatile("" : "+v"(qf[s]));
+  for (int s = 0; s < QF; ++s) asm volatile("" : "+v"(qf[s]));  // waited for ahead of the tiles
+  const bool more = w < NIT % 4;  // this wave issues NIT / 4 + 1 instructions per tile, else NIT / 4
+  const int tiles = (k1 - k0 + 31) / 32;
+  asm volatile("" : "+v"(pages));
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j)
+    if (j < tiles) stage();
   int buf = 0;
-  for (int key0 = k0; key0 < k1; key0 += 32, buf ^= 1) {
-    const bool n1 = key0 + 32 < k1, n2 = key0 + 64 < k1;
-    const int page2 = n2 ? page_of(key0 + 64) : 0;
-    // this tile's image; the next tile's instructions stay in flight
-    if (!n1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4 + 1) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4) : "memory");
-    asm volatile("s_barrier" ::: "memory");           // ... of every wave
+  for (int i = 0; i < tiles; ++i, buf = buf + 1 == NB ? 0 : buf + 1) {
+    const int key0 = k0 + 32 * i;
+    // this tile's image; the next tiles' instructions stay in flight
+    const int newer = min(AHEAD - 1, tiles - 1 - i);
+    if (newer == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (newer == 1 && more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4 + 1) : "memory");
+    else if (newer == 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4) : "memory");
+    else if (more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * (NIT / 4 + 1)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * (NIT / 4)) : "memory");
+    asm volatile("s_barrier" ::: "memory");           // ... of every wave; and all are done with the tile before
+    if (NB > 2 && next < tiles) stage();
     const char* img = smem + buf * BUFB;
     // ---- scores ----
     f32x4 sp[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two independent MFMA chains
@@ -353,9 +376,9 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(DecArgs a) {
 #pragma unroll
       for (int n = 0; n < NH; ++n) o[n][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pa[n], o[n][c], 0, 0, 0);
     }
-    if (n2) {  // every wave is done with this image: the tile after the next one takes its place
+    if (NB == 2 && next < tiles) {  // every wave is done with this image: the tile after the next one takes its place
       asm volatile("s_barrier" ::: "memory");
-      stage(key0 + 64, page2, buf);
+      stage();
     }
   }
   // o[n][c][i]: head h0 + 16 n + r16, latent column 16 (RT w + c) + 4 g + i
