@@ -39,8 +39,9 @@ int rt_latent_prefill(const void*, long, const void*, long, int, int, const floa
 int rt_window_prep(int, void*, long, int, int, int, const void*, const void*, float, const float*, const float*, int, int,
                    const int*, const int*, void*, const int*, int, int, int, int, int, int, int, int, hipStream_t);
 int rt_window_decode_ok(int, int, int, int);
-int rt_window_decode(const void*, long, const void*, const int*, int, int, int, const int*, const int*, float*, float*, int,
-                     int, int, int, int, int, int, int, float, float, hipStream_t);
+int rt_window_decode(const void*, long, const void*, const int*, int, int, int, const int*, const int*, float*, float*, void*, long,
+                     float, int, int, int, int, int, int, int, int, float, float, hipStream_t);
+int rt_window_decode_parts(int, int, int);
 int rt_window_prefill_ok(int, int);
 int rt_window_prefill(const void*, long, const void*, const int*, int, int, int, void*, long, const void*, const void*, int,
                       int, int, int, int, int, int, float, float, float, hipStream_t);
@@ -524,15 +525,21 @@ void window_decode(const Tensor& q, const Tensor& pool, const Tensor& tab, const
   TORCH_CHECK(pool.scalar_type() == at::kBFloat16 && q.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16 &&
                   q.is_cuda() && out.is_cuda() && q.size(1) == (int64_t)w.H * w.D && out.size(0) == T &&
                   out.size(1) == (int64_t)w.H * w.V && NP >= 1 && NP <= 1024 && al16(q), "window_decode: shapes");
-  Tensor part = at::empty({T, w.H, NP, w.V}, q.options().dtype(at::kFloat));
-  Tensor ml = at::empty({T, w.H, NP, 2}, q.options().dtype(at::kFloat));
+  const int np = rt_window_decode_parts((int)T, w.G, (int)NP);
+  Tensor part, ml;
+  if (np > 1) {
+    part = at::empty({T, w.H, np, w.V}, q.options().dtype(at::kFloat));
+    ml = at::empty({T, w.H, np, 2}, q.options().dtype(at::kFloat));
+  }
   rc_ok(rt_window_decode(q.data_ptr(), q.stride(0), pool.data_ptr(), tab.data_ptr<int>(), pl.max_pages(), pl.pages(), pl.rows(),
-                         row.data_ptr<int>(), pos.data_ptr<int>(), part.data_ptr<float>(), ml.data_ptr<float>(), (int)T, w.H, w.G,
-                         w.D, w.V, (int)NP, w.size, w.keep, w.scale, w.cap, stream()),
+                         row.data_ptr<int>(), pos.data_ptr<int>(), np > 1 ? part.data_ptr<float>() : nullptr,
+                         np > 1 ? ml.data_ptr<float>() : nullptr, out.data_ptr(), out.stride(0), (float)out_scale, (int)T, w.H, w.G,
+                         w.D, w.V, np, w.size, w.keep, w.scale, w.cap, stream()),
         "window_decode");
-  rc_ok(rt_partition_merge(part.data_ptr<float>(), ml.data_ptr<float>(), nullptr, out.data_ptr(), out.stride(0), (int)T, w.H, w.V,
-                           (int)NP, (float)out_scale, stream()),
-        "partition_merge");
+  if (np > 1)
+    rc_ok(rt_partition_merge(part.data_ptr<float>(), ml.data_ptr<float>(), nullptr, out.data_ptr(), out.stride(0), (int)T, w.H, w.V, np,
+                             (float)out_scale, stream()),
+          "partition_merge");
 }
 
 void window_prefill(const Tensor& q, const Tensor& pool, const Tensor& tab, Tensor out, const Tensor& segs, const Tensor& tiles,

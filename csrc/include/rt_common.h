@@ -82,6 +82,22 @@ __device__ __forceinline__ void ds_tr16_x4(uint32_t a, rt_s16x4& r0, rt_s16x4& r
       : "v"(a), "i"(O1), "i"(O2), "i"(O3)
       : "memory");
 }
+// eight reads at eight addresses
+__device__ __forceinline__ void ds_tr16_at8(const uint32_t (&a)[8], rt_s16x4 (&r)[8]) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %1, %9\n\t"
+      "ds_read_b64_tr_b16 %2, %10\n\t"
+      "ds_read_b64_tr_b16 %3, %11\n\t"
+      "ds_read_b64_tr_b16 %4, %12\n\t"
+      "ds_read_b64_tr_b16 %5, %13\n\t"
+      "ds_read_b64_tr_b16 %6, %14\n\t"
+      "ds_read_b64_tr_b16 %7, %15\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
+      : "memory");
+}
 // F fragments x 4 reads at a_f + {0, O1, O2, O3}: r[4 f + h]
 template <int O1, int O2, int O3>
 __device__ __forceinline__ void ds_tr16_frag2(uint32_t a0, uint32_t a1, rt_s16x4 (&r)[8]) {

@@ -179,17 +179,22 @@ static CapScore make_cap_score(float scale, float cap) {
 // ---------------------------------------------------------------------------------------------
 // decode: workgroup = (token, key head with its 16 NH query heads at most, partition), 4 waves
 // ---------------------------------------------------------------------------------------------
-// Per 32-key tile one LDS image [K: 64 QS columns | V: 64 RT columns], two buffers, LDS-DMA one tile ahead:
-//   scores S^T = K Q^T (key on the MFMA row, head on the lane) by waves (key half, K-dim half) for NH = 1 and
-//   (key half, head tile) for NH = 2, exchanged through LDS; every wave runs the same online softmax and
-//   accumulates O^T += V^T P^T for its own quarter of the value columns (transposed reads of the image).
+// The waves take the partition's 16-key tiles in turn, each for itself until the end: an LDS image of its own
+// [K: 64 QS columns | V: 64 RT columns] by LDS-DMA, two of them, no barrier. S^T = K Q^T (key on the MFMA row, head on
+// the lane), online softmax of 4 scores a lane, O^T += V^T P^T with 16-key MFMAs (P is their B operand as it is);
+// the waves' (m, l, O) meet in LDS. With a tile of 32 keys shared by the four waves every wave ran the same softmax
+// (H / G of 16 lanes of it needed: 38 of 46 us were its VALU work), with three barriers a tile; and a page's number, loaded
+// for each tile, waited for all LDS-DMA under way (loads return in order): the pages of 64 tiles now come at once.
+// us, before -> this (each at its partitions): 64 rows of 300..1100 keys 50.2 -> 43.5 and no merge, 16 22.6 -> 15.5, 4 of 3000..4000 30 -> 17,
+// 200 of 100..600 81.5 -> 70.8, 256 of 60..120 38.8 -> 34.1. 2 or 1 waves a workgroup, more of these on a CU: 44.9 / 52.5, 74.0 / 76.0, 32.6 / 33.3.
 // A token's visible tiles are cut in NP equal partitions, so a captured launch with a fixed NP balances every
-// length. Image rows are an odd number of 16-B chunks (row reads conflict-free).
+// length; of one partition the workgroup writes the result. Chunk c of image row r lies in slot c ^ r, or rows are an odd number of 16-B chunks (conflict-free either way).
 struct DecArgs {
   const bf16_t* q; long ldq;  // [T, ldq], head h at h * D
   const bf16_t* pool; const int* tab; int max_pages, n_pages, n_rows;
   const int* row; const int* pos;
   float* part; float* ml;     // [T, H, NP, V], [T, H, NP, 2] (max in log2 units, sum)
+  bf16_t* out; long ldo; float out_scale;  // of one partition: the result itself, as partition_merge makes it (else null)
   int H, G, D, V, NP;
   Mask mask;
   Score score;
@@ -197,178 +202,194 @@ struct DecArgs {
 
 template <int QS, int RT, int NH>
 __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
-  constexpr int CPR = 8 * QS + 8 * RT + 1, ROWB = CPR * 16;
-  constexpr int NI = (32 * CPR + 255) / 256;         // LDS-DMA instructions per wave and tile
-  constexpr int NIT = (32 * CPR + 63) / 64;          // of the workgroup (the last one may be half used)
-  constexpr int BUFB = NIT * 1024;
-  constexpr int QF = NH == 1 ? QS : 2 * QS;          // query fragments per wave
-  __shared__ __attribute__((aligned(16))) char smem[2 * BUFB + 4096];
-  float* sx = (float*)(smem + 2 * BUFB);             // [4 waves][64 lanes][4]
+  constexpr int NW = 4;
+  constexpr int CH = 8 * QS + 8 * RT;
+  constexpr bool SWZ = CH % 16 == 0;
+  constexpr int CPR = SWZ ? CH : CH + 1, ROWB = CPR * 16;
+  constexpr int NIT = (16 * CPR + 63) / 64, BUFB = NIT * 1024;  // LDS-DMA instructions of a tile (the last one may be part used)
+  constexpr int QF = 2 * QS, LDP = 64 * RT + 4;
+  constexpr int RING = NW * 2 * BUFB;                 // two images a wave; at the end 16 heads' O of each
+  static_assert(NW * 16 * LDP * 4 <= RING, "the merge fits the images");
+  __shared__ __attribute__((aligned(16))) char smem[RING + NW * NH * 16 * 8 + 64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
   const int part = bid % a.NP, gh = bid / a.NP % a.G, t = bid / (a.NP * a.G);
   const int HG = a.H / a.G, h0 = gh * HG;            // query heads h0 .. h0 + HG - 1
-  const int row = min(max(a.row[t], 0), a.n_rows - 1);
-  const int pos = min(max(a.pos[t], 0), a.max_pages * PAGE - 1);
-  const Tiles<32> tl(a.mask, pos, pos);
+  int row = a.row[t], pos = a.pos[t];
+  asm volatile("" : "+s"(row), "+s"(pos));           // in one trip, also if the partition is empty
+  row = min(max(row, 0), a.n_rows - 1);
+  pos = min(max(pos, 0), a.max_pages * PAGE - 1);
+  const Tiles<16> tl(a.mask, pos, pos);
   const int per = (tl.n + a.NP - 1) / a.NP;
   const int i0 = part * per, i1 = min(tl.n, i0 + per);
   if (i0 >= i1) {  // nothing for this partition (uniform over the workgroup)
-    if (tid < HG) {
-      float* m = a.ml + (((long)t * a.H + h0 + tid) * a.NP + part) * 2;
+    for (int h = tid; h < HG; h += 64 * NW) {
+      float* m = a.ml + (((long)t * a.H + h0 + h) * a.NP + part) * 2;
       m[0] = -INFINITY;
       m[1] = 0.f;
     }
     return;
   }
-  // query fragments: lane holds Q[head r16][32 s + 8 g ..]; heads past the last repeat it (not stored)
-  const int kt = w & 1, hi = w >> 1;                 // key half; K-dim half (NH = 1) or head tile (NH = 2)
-  const int qh = h0 + min((NH == 2 ? hi * 16 : 0) + r16, HG - 1);
-  const int sbase = NH == 1 ? hi * QS : 0;
-  bf16x8 qf[QF];
-  const bf16_t* qp = a.q + (long)t * a.ldq + (long)qh * a.D;
-#pragma unroll
-  for (int s = 0; s < QF; ++s) qf[s] = *(const bf16x8*)(qp + min(32 * (sbase + s) + 8 * g, a.D - 8));
+  const int n = i1 - i0 > w ? (i1 - i0 - w + NW - 1) / NW : 0;  // this wave's tiles: i0 + w + NW j
+  auto key_of = [&](int j) { return tl.key(min(i0 + w + NW * j, i1 - 1)); };
   const int* tab = a.tab + (long)row * a.max_pages;
+  int pages = tab[key_of(lane) / PAGE];              // of 64 tiles, a tile a lane
+  // query fragments: lane holds Q[head r16][32 s + 8 g ..]; heads past the last repeat it (not stored)
+  bf16x8 qf[NH][QF];
+#pragma unroll
+  for (int u = 0; u < NH; ++u) {
+    const bf16_t* qp = a.q + (long)t * a.ldq + (long)(h0 + min(16 * u + r16, HG - 1)) * a.D;
+#pragma unroll
+    for (int s = 0; s < QF; ++s) qf[u][s] = *(const bf16x8*)(qp + min(32 * s + 8 * g, a.D - 8));
+  }
   const int W = a.D + a.V;
 
-  // LDS-DMA sources: instruction j of wave w covers image chunks (4 j + w) * 64 + lane; columns past D (V)
+  // LDS-DMA sources: instruction j covers image chunks 64 j + lane; columns past D (V)
   // repeat the last chunk (the query is zero there, the sums are not stored)
-  uint32_t src[NI];  // element offset from the tile's first cache row
+  uint32_t src[NIT];  // element offset from the tile's first cache row
 #pragma unroll
-  for (int j = 0; j < NI; ++j) {
-    const int c = (4 * j + w) * 64 + lane, cc = c % CPR;
+  for (int j = 0; j < NIT; ++j) {
+    const int c = 64 * j + lane, r = min(c / CPR, 15), cc = SWZ ? c % CPR ^ r : c % CPR;
     const int col = cc < 8 * QS ? min(8 * cc, a.D - 8) : a.D + min(8 * (cc - 8 * QS), a.V - 8);
-    src[j] = (uint32_t)(min(c / CPR, 31) * W + col);
+    src[j] = (uint32_t)(r * W + col);
   }
-  auto page_of = [&](int i) { return min(max(tab[tl.key(i) / PAGE], 0), a.n_pages - 1); };
-  auto stage = [&](int i, int page, int buf) {
-    const bf16_t* base = a.pool + (((long)page * a.G + gh) * PAGE + tl.key(i) % PAGE) * W;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      if (4 * j + w < NIT)  // wave-uniform
-        __builtin_amdgcn_global_load_lds((const void*)(base + src[j]), (lds_void*)(smem + buf * BUFB + (4 * j + w) * 1024),
-                                         16, 0, 0);
+  char* const mine = smem + w * 2 * BUFB;
+  auto stage = [&](int j) {
+    if (j % 64 == 0 && j > 0) {
+      pages = tab[key_of(j + lane) / PAGE];
+      asm volatile("" : "+v"(pages));                // waited for here, not by every tile
     }
+    const int page = min(max(__builtin_amdgcn_readlane(pages, j % 64), 0), a.n_pages - 1);
+    const bf16_t* base = a.pool + (((long)page * a.G + gh) * PAGE + key_of(j) % PAGE) * W;
+    char* to = mine + (j & 1) * BUFB;
+#pragma unroll
+    for (int k = 0; k < NIT; ++k)
+      __builtin_amdgcn_global_load_lds((const void*)(base + src[k]), (lds_void*)(to + k * 1024), 16, 0, 0);
   };
 
-  f32x4 o[NH][RT];
+  f32x4 o[NH][4 * RT];
 #pragma unroll
-  for (int n = 0; n < NH; ++n)
+  for (int u = 0; u < NH; ++u)
 #pragma unroll
-    for (int c = 0; c < RT; ++c) o[n][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < 4 * RT; ++c) o[u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m[NH], l[NH];
 #pragma unroll
-  for (int n = 0; n < NH; ++n) { m[n] = -INFINITY; l[n] = 0.f; }
-
-  const bool more = w < NIT % 4;  // this wave issues NIT / 4 + 1 instructions per tile, else NIT / 4
-  stage(i0, page_of(i0), 0);
-  if (i0 + 1 < i1) stage(i0 + 1, page_of(i0 + 1), 1);
+  for (int u = 0; u < NH; ++u) { m[u] = -INFINITY; l[u] = 0.f; }
   if (a.D < 64 * QS) {
 #pragma unroll
-    for (int s = 0; s < QF; ++s)
-      if (32 * (sbase + s) + 8 * g >= a.D) qf[s] = bf16x8{};
+    for (int u = 0; u < NH; ++u)
+#pragma unroll
+      for (int s = 0; s < QF; ++s)
+        if (32 * s + 8 * g >= a.D) qf[u][s] = bf16x8{};
   }
 #pragma unroll
-  for (int s = 0; s < QF; ++s) asm volatile("" : "+v"(qf[s]));
-  int buf = 0;
-  for (int i = i0; i < i1; ++i, buf ^= 1) {
-    const bool n1 = i + 1 < i1, n2 = i + 2 < i1;
-    const int page2 = n2 ? page_of(i + 2) : 0;
-    const int key0 = tl.key(i);
+  for (int u = 0; u < NH; ++u)
+#pragma unroll
+    for (int s = 0; s < QF; ++s) asm volatile("" : "+v"(qf[u][s]));  // waited for ahead of the tiles
+  asm volatile("" : "+v"(pages));
+  auto slot = [](int r, int c) { return r * ROWB + (SWZ ? c ^ r : c) * 16; };
+  const int vr = 4 * g + ((lane >> 2) & 3);          // this lane's part of the transposed reads
+  if (n > 0) stage(0);
+  if (n > 1) stage(1);
+  for (int j = 0; j < n; ++j) {
+    const int key0 = key_of(j);
     // this tile's image; the next tile's instructions stay in flight
-    if (!n1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4 + 1) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT / 4) : "memory");
-    asm volatile("s_barrier" ::: "memory");           // ... of every wave
-    const char* img = smem + buf * BUFB;
-    // ---- scores ----
-    f32x4 sp[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two independent MFMA chains
-    {
-      const char* kp = img + (16 * kt + r16) * ROWB + (4 * sbase + g) * 16;
+    if (j + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NIT) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const char* img = mine + (j & 1) * BUFB;
+    f32x4 sp[NH][2];
 #pragma unroll
-      for (int s = 0; s < QF; ++s) {
-        const bf16x8 kf = *(const bf16x8*)(kp + s * 64);
-        sp[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], sp[s & 1], 0, 0, 0);
-      }
+    for (int u = 0; u < NH; ++u) sp[u][0] = sp[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < QF; ++s) {
+      const bf16x8 kf = *(const bf16x8*)(img + slot(r16, 4 * s + g));
+#pragma unroll
+      for (int u = 0; u < NH; ++u) sp[u][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[u][s], sp[u][s & 1], 0, 0, 0);
     }
-    *(f32x4*)(sx + (w * 64 + lane) * 4) = sp[0] + sp[1];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
-    // ---- softmax (identical in every wave) ----
-    const bool whole = key0 + 31 <= pos && (pos - key0 < a.mask.size || key0 + 31 < a.mask.keep);
-    bf16x8 pa[NH];
+    const bool whole = key0 + 15 <= pos && (pos - key0 < a.mask.size || key0 + 15 < a.mask.keep);
+    rt_s16x4 pa[NH];
 #pragma unroll
-    for (int n = 0; n < NH; ++n) {
-      f32x4 s2[2];
+    for (int u = 0; u < NH; ++u) {
+      f32x4 x = sp[u][0] + sp[u][1];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if constexpr (NH == 1)
-          s2[k] = *(const f32x4*)(sx + (k * 64 + lane) * 4) + *(const f32x4*)(sx + ((k + 2) * 64 + lane) * 4);
-        else
-          s2[k] = *(const f32x4*)(sx + ((k + 2 * n) * 64 + lane) * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s2[k][e] = a.score(s2[k][e]);
-      }
+      for (int e = 0; e < 4; ++e) x[e] = a.score(x[e]);
       if (!whole) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (!a.mask.sees(pos, key0 + 16 * k + 4 * g + e)) s2[k][e] = -INFINITY;
+        for (int e = 0; e < 4; ++e)
+          if (!a.mask.sees(pos, key0 + 4 * g + e)) x[e] = -INFINITY;
       }
-      float mx = fmaxf(fmaxf(fmaxf(s2[0][0], s2[0][1]), fmaxf(s2[0][2], s2[0][3])),
-                       fmaxf(fmaxf(s2[1][0], s2[1][1]), fmaxf(s2[1][2], s2[1][3])));
-      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
-      const float mn = fmaxf(m[n], mx);  // finite: every listed tile holds a visible key
-      const float alpha = fexp2(m[n] - mn);
-      m[n] = mn;
-      float rs = 0.f;
+      const float mx = over_groups(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), [](float p, float q) { return fmaxf(p, q); });
+      const float mn = fmaxf(m[u], mx);  // finite: every listed tile holds a visible key
+      const float alpha = fexp2(m[u] - mn);
+      m[u] = mn;
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float p = fexp2(s2[k][e] - mn);
-          s2[k][e] = p;
-          rs += p;
-        }
-      rs = over_groups(rs, [](float x, float y) { return x + y; });
-      l[n] = l[n] * alpha + rs;
-      pa[n] = pack_p(s2[0], s2[1]);
+      for (int e = 0; e < 4; ++e) x[e] = fexp2(x[e] - mn);
+      l[u] = l[u] * alpha + over_groups((x[0] + x[1]) + (x[2] + x[3]), [](float p, float q) { return p + q; });
+      pa[u] = __builtin_bit_cast(rt_s16x4, make_uint2(pack2bf(x[0], x[1]), pack2bf(x[2], x[3])));
       // O^T: the head is the lane's column, as in the scores (most tiles bring no new maximum)
       if (__any(alpha != 1.f)) {
 #pragma unroll
-        for (int c = 0; c < RT; ++c) o[n][c] *= alpha;
+        for (int c = 0; c < 4 * RT; ++c) o[u][c] *= alpha;
       }
     }
-    // ---- O += P V: value columns [16 RT w, 16 RT (w + 1)) ----
-    const uint32_t va = lds_addr(img + (4 * g + ((lane >> 2) & 3)) * ROWB + 128 * QS + w * RT * 32 + (lane & 3) * 8);
-    rt_s16x4 v[2 * RT];
-    if constexpr (RT == 4) ds_tr16_frag2<16 * ROWB, 32, 32 + 16 * ROWB>(va, va + 64, v);
-    else ds_tr16_x4<16 * ROWB, 32, 32 + 16 * ROWB>(va, v[0], v[1], v[2], v[3]);
 #pragma unroll
-    for (int c = 0; c < RT; ++c) {
-      const bf16x8 vf = cat4(v[2 * c], v[2 * c + 1]);
+    for (int c0 = 0; c0 < 4 * RT; c0 += 8) {
+      uint32_t va[8];
+      rt_s16x4 v[8];
 #pragma unroll
-      for (int n = 0; n < NH; ++n) o[n][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pa[n], o[n][c], 0, 0, 0);
+      for (int c = 0; c < 8; ++c) va[c] = lds_addr(img + slot(vr, 8 * QS + 2 * (c0 + c) + ((lane >> 1) & 1)) + (lane & 1) * 8);
+      ds_tr16_at8(va, v);
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int u = 0; u < NH; ++u) o[u][c0 + c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[c], pa[u], o[u][c0 + c], 0, 0, 0);
     }
-    if (n2) {  // every wave is done with this image: the tile after the next one takes its place
-      asm volatile("s_barrier" ::: "memory");
-      stage(i + 2, page2, buf);
-    }
+    if (j + 2 < n) stage(j + 2);  // this image has been read
   }
-  // o[n][c][e]: head h0 + 16 n + r16, value column 16 (RT w + c) + 4 g + e
+  // ---- the waves' sums: o[u][c][e] is head h0 + 16 u + r16, value column 16 c + 4 g + e ----
+  float2* const mls = (float2*)(smem + RING);        // [wave][head]
+  if (g == 0)
 #pragma unroll
-  for (int n = 0; n < NH; ++n) {
-    if (16 * n + r16 >= HG) continue;
-    const long th = ((long)t * a.H + h0 + 16 * n + r16) * a.NP + part;
-    float* po = a.part + th * a.V + 16 * RT * w + 4 * g;
+    for (int u = 0; u < NH; ++u) mls[w * 16 * NH + 16 * u + r16] = make_float2(m[u], l[u]);
+  __syncthreads();
+  float* const os = (float*)smem;                    // [wave][16 heads][LDP]
+  float* const invs = (float*)(smem + RING + NW * NH * 16 * 8);  // [16 heads]
 #pragma unroll
-    for (int c = 0; c < RT; ++c)
-      if (16 * (RT * w + c) + 4 * g < a.V) *(f32x4*)(po + 16 * c) = o[n][c];  // V % 8 == 0
-    if (w == 0 && g == 0) *(float2*)(a.ml + th * 2) = make_float2(m[n], l[n]);
+  for (int u = 0; u < NH; ++u) {
+    float M = -INFINITY, L = 0.f;                    // finite: wave 0 has a tile
+#pragma unroll
+    for (int k = 0; k < NW; ++k) M = fmaxf(M, mls[k * 16 * NH + 16 * u + r16].x);
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const float2 x = mls[k * 16 * NH + 16 * u + r16];
+      L += x.y * fexp2(x.x - M);
+    }
+    const float f = fexp2(m[u] - M);                 // 0 for a wave without tiles
+    if (u > 0) __syncthreads();
+    if (16 * u + r16 < HG) {
+#pragma unroll
+      for (int c = 0; c < 4 * RT; ++c) *(f32x4*)(os + (w * 16 + r16) * LDP + 16 * c + 4 * g) = o[u][c] * f;
+    }
+    if (w == 0 && g == 0 && 16 * u + r16 < HG) {
+      if (a.out) invs[r16] = a.out_scale / L;
+      else *(float2*)(a.ml + (((long)t * a.H + h0 + 16 * u + r16) * a.NP + part) * 2) = make_float2(M, L);
+    }
+    __syncthreads();
+    const int hn = min(HG - 16 * u, 16), V4 = a.V / 4;  // V % 8 == 0
+    for (int e = tid; e < hn * V4; e += 64 * NW) {
+      const int h = e / V4, c = e % V4 * 4;
+      f32x4 y = *(const f32x4*)(os + h * LDP + c);
+#pragma unroll
+      for (int k = 1; k < NW; ++k) y += *(const f32x4*)(os + (k * 16 + h) * LDP + c);
+      if (a.out) {
+        y *= invs[h];
+        *(uint2*)(a.out + (long)t * a.ldo + (long)(h0 + 16 * u + h) * a.V + c) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+      } else {
+        *(f32x4*)(a.part + (((long)t * a.H + h0 + 16 * u + h) * a.NP + part) * a.V + c) = y;
+      }
+    }
   }
 }
 
@@ -690,13 +711,25 @@ extern "C" int rt_window_decode_ok(int H, int G, int D, int V) {
   return G > 0 && H % G == 0 && H / G <= 32 && D % 8 == 0 && V % 8 == 0 && D >= 8 && V >= 8 && D <= 256 && V <= 256;
 }
 
+// Partitions of a token's tiles that a decode takes of the NP it may: a workgroup per CU. us (without the merge), 8 key heads of
+// 128, at 1 / 2 / 4 / 8 partitions: 4 rows of 3000..4000 keys 45 / 27 / 19 / 17, 16 of 300..1100 18.8 / 15.5 / 15.6 / 17.6, 32 24.5 / 26.1 /
+// 25.3 / 29.1, 64 43.5 / 44.2 / 44.0 / 50.0, 128 of 100..600 47.2 / 47.8 / 52.6 / 69.3, 256 of 60..120 34 / 42 / 63 / 106; and one needs
+// no merge (5 us).
+extern "C" int rt_window_decode_parts(int T, int G, int NP) {
+  const long groups = std::max(1L, (long)T * G);
+  return (int)std::min((long)NP, (256 + groups - 1) / groups);
+}
+
+// NP of one partition: to out (ldo % 4 == 0, 8-byte aligned), part and ml unused; of more: to part and ml, for partition_merge
 extern "C" int rt_window_decode(const void* q, long ldq, const void* pool, const int* tab, int max_pages, int n_pages,
-                                int n_rows, const int* row, const int* pos, float* part, float* ml, int T, int H, int G,
-                                int D, int V, int NP, int size, int keep, float scale, float cap, hipStream_t stream) {
+                                int n_rows, const int* row, const int* pos, float* part, float* ml, void* out, long ldo,
+                                float out_scale, int T, int H, int G, int D, int V, int NP, int size, int keep, float scale,
+                                float cap, hipStream_t stream) {
   if (T <= 0) return 0;
   if (!rt_window_decode_ok(H, G, D, V) || NP < 1 || ldq % 8) return -1;
-  DecArgs a{(const bf16_t*)q, ldq, (const bf16_t*)pool, tab, max_pages, n_pages, n_rows, row, pos, part, ml, H, G, D, V, NP,
-            make_mask(size, keep), make_score(scale, cap)};
+  if (NP == 1 && (ldo % 4 || (uintptr_t)out % 8)) return -1;
+  DecArgs a{(const bf16_t*)q, ldq, (const bf16_t*)pool, tab, max_pages, n_pages, n_rows, row, pos, part, ml,
+            NP == 1 ? (bf16_t*)out : nullptr, ldo, out_scale, H, G, D, V, NP, make_mask(size, keep), make_score(scale, cap)};
   dim3 grid((unsigned)((long)T * G * NP)), block(256);
 #define WD_(QS, RT)                                                                                        \
   do {                                                                                                     \

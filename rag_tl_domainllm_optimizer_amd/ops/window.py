@@ -49,12 +49,9 @@ class WindowDims:
 
 
 def _np_parts(T: int, d: WindowDims, max_len: int) -> int:
-    """Partitions of a token's visible tiles, at least 64 keys each: two workgroups per CU, and four of a token and key head
-    all the same. A partition is a chain of tiles (three barriers and a softmax each), so its CU needs others beside it, and
-    rows differ in length: decode steps of 16 / 32 / 64 rows of 300..1100 keys and 8 key heads took 557 / 656 / 888 us at 4 /
-    2 / 1 partitions, 556 / 637 / 847 at four, 550 / 640 / 847 at six. Of 96 / 128 rows of 100..600 keys 935 / 1133 us at one,
-    920 / 1122 at four; beyond 4096 workgroups a partition's own cost takes over (256 rows 1694 at one, 1682 at two,
-    1702 at eight)."""
+    """Partitions that a token's visible tiles may be cut in, at least 64 keys each: two workgroups per CU, and four of a token
+    and key head all the same up to 4096 workgroups. The kernel takes as many of them as give every CU a workgroup
+    (rt_window_decode_parts)."""
     keys = max_len if not d.window else min(max_len, d.window + d.keep + 64)
     groups = T * d.kv_heads
     return max(1, min(max((512 + groups - 1) // groups, min(4, 4096 // groups)), (keys + 63) // 64, 512))

@@ -278,6 +278,41 @@ def test_window_decode_partitions(T, parts, heads):
         assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, b
 
 
+@pytest.mark.parametrize("window,keep", [(0, 0), (5000, 100)])
+@pytest.mark.parametrize("D,V", [(8, 16), (136, 8)])
+def test_window_decode_of_many_pages(D, V, window, keep):
+    """one partition of more tiles than a wave holds page numbers of, and rows that end in each wave's tiles"""
+    T, G, most = 4, 64, 8300
+    d = ops.WindowDims(G, G, D, V, D ** -0.5, 30.0, window, keep)
+    g = torch.Generator(device=DEV).manual_seed(D + window)
+    n = torch.tensor([most, 4096 + 17, 4096 + 3 * 16, 5137])
+    cache = PagedCache([d.cache_width], T, most, T * (most + 63) // 64 * 64 + 64 * T, DEV, torch.bfloat16)
+    for b in range(T):
+        cache.reserve(b, int(n[b]))
+    cache.sync()
+    pool = cache.pool(0)
+    pool.normal_(generator=g)
+    proj = torch.randn(T, d.in_cols, generator=g, device=DEV).bfloat16()
+    cos, sin = torch.ones(cache.max_seq, D // 2, device=DEV), torch.zeros(cache.max_seq, D // 2, device=DEV)
+    out = torch.zeros(T, G * V, dtype=torch.bfloat16, device=DEV)
+    batch = RaggedBatch.single(torch.zeros(T, dtype=torch.long, device=DEV), torch.arange(T, dtype=torch.int32, device=DEV),
+                               (n - 1).int().to(DEV), most)
+    ops.window_attention(proj, 0, d, None, None, 1e-6, cos, sin, batch, pool, cache.table, out, 0.5)
+    for b in range(T):
+        k = int(n[b])
+        kv = pool.view(-1, G, 64, D + V)[cache.table[b].long()[:(k + 63) // 64]].transpose(1, 2).flatten(0, 1)[:k].double()
+        s = (proj[b, :G * D].view(G, D).double()[None] * kv[..., :D]).sum(-1).t() * d.scale
+        s = 30 * torch.tanh(s / 30)
+        if window:
+            at = torch.arange(k, device=DEV)
+            s = s.masked_fill((k - 1 - at >= window) & (at >= keep), -math.inf)
+        p = torch.softmax(s, -1)[..., None]
+        v = kv[..., D:].transpose(0, 1)
+        want, size = (0.5 * (p * x).sum(1).flatten() for x in (v, v.abs()))
+        # p and the result round to bf16 (half an ulp: 2^-8 each)
+        assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, b
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ch", [True, False])
 @pytest.mark.parametrize("H,K,D,V,taps", [(4, 2, 32, 64, 4), (6, 3, 9, 11, 3), (3, 1, 128, 128, 2), (2, 2, 200, 72, 4), (2, 1, 64, 256, 1),
