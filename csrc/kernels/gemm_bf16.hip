@@ -483,6 +483,10 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
       }
     }
   };
+  // the epilogue's element of this thread; its residual ahead of the weights, not a trip to memory behind them
+  const int row = tid >> 4, ci = tid & 15, col = grp * 16 + ci;
+  const bool has_r = !PAIR && p.R;
+  const bf16_t res = has_r ? p.R[(long)min(row, p.M - 1) * p.ldr + col] : (bf16_t)0;
   Regs r[DEPTH];
 #pragma unroll
   for (int i = 0; i < DEPTH - 1; ++i)
@@ -512,9 +516,7 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
     if (g == 0) rsq[wid][frow] = t;
   }
   __syncthreads();
-  const int row = tid >> 4, ci = tid & 15;
   if (row < p.M) {
-    const int col = grp * 16 + ci;
     // wave partials summed in wave order (NW = 4: the association of the original four-term sum)
     float ss = 0.f, yy = 0.f, uu = 0.f;
 #pragma unroll
@@ -535,7 +537,7 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
       if constexpr (W8) y *= p.sb[col];
       if (p.bias) y += bf2f(p.bias[col]);
       y = apply_act(y, p.act);
-      if (p.R) y += bf2f(p.R[(long)row * p.ldr + col]);
+      if (has_r) y += bf2f(res);
     }
     if constexpr (OUT_F32) ((float*)p.C)[(long)row * p.ldc + col] = y;
     else ((bf16_t*)p.C)[(long)row * p.ldc + col] = f2bf(y);
@@ -550,8 +552,8 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
 // and below get 2 to 4.6 TB/s of weights at these M: 64-column LDS rings re-read X as often as W, and the 256-row one
 // leaves slabs of half the weight bytes to a second launch. us a call with cold weights, M = 24 / 48 / 64, best
 // row-major form -> image form:
-//   6144 x 4096 with norm    21.6 / 21.5 / 22.5 -> 16.0 / 19.8 / 21.8     28672 x 4096, SwiGLU  55.5 / 53.4 / 56.0 -> 44.2 / 44.3 / 45.5
-//   4096 x 4096 + residual   14.8 / 16.4 / 17.3 -> 10.9 / 14.6 / 16.6     4096 x 14336          29.6 / 30.2 / 31.9 -> 25.5 / 27.6 / 31.0
+//   6144 x 4096 with norm    21.6 / 21.5 / 22.5 -> 14.9 / 17.2 / 19.4     28672 x 4096, SwiGLU  55.5 / 53.4 / 56.0 -> 44.2 / 44.3 / 45.5
+//   4096 x 4096 + residual   14.8 / 16.4 / 17.3 -> 10.9 / 13.9 / 15.4     4096 x 14336          29.6 / 30.2 / 31.9 -> 25.0 / 28.0 / 30.7
 //   10304 x 4096             36.0 / 37.4 / 38.8 -> 19.2 / 22.8 / 25.7     14336 x 4096, relu^2  29.8 / 31.3 / 32.6 -> 23.8 / 25.8 / 28.1
 //   32000 x 4096             59.0 / 58.9 / 60.8 -> 47.6 / 50.4 / 54.0     3072 x 2048 with norm 15.5 / 16.7 / 17.7 -> 7.1 / 9.9 / 11.7
 //
@@ -640,7 +642,11 @@ __global__ __launch_bounds__(64 * NW) void gemv64_kernel(GemmArgs p) {
 // through LDS in 64-deep chunks (8 KB, double-buffered, one barrier a chunk) and is read N / 64 times. Both X parts
 // and weights come in plain loads, DEPTH - 1 chunks ahead: with LDS-DMA for X the compiler waits for everything in flight
 // wherever it needs a weight register (SwiGLU 28672 x 4096 at M = 24: 49 us instead of 44). Few column groups are split
-// over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order.
+// over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order. It asks for the
+// tiles of all rows at once, and bias and residual are asked for ahead of the hand-off: a trip to memory a row tile, and one for
+// each element of a residual, were 2 to 3 us of every split product. us at M = 24 / 48 / 64: 6144 x 4096 with norm 15.8 / 19.6 / 21.9 ->
+// 14.9 / 17.2 / 19.4, 4096 x 4096 + residual 12.3 / 15.3 / 17.5 -> 12.1 / 13.9 / 15.4, 4096 x 14336 25.6 / 29.2 / 32.4 -> 25.0 / 28.0 /
+// 30.7, 2048 x 7168 14.0 / 17.5 / 20.7 -> 12.4 / 14.5 / 16.7. More chunks in flight (6, 8), fragments read a chunk ahead: nothing.
 template <bool OUT_F32, int RT, bool PAIR>
 __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __restrict__ slabs,
                                                            unsigned* __restrict__ tickets, int split) {
@@ -749,6 +755,19 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
       ss[t] = __shfl(v, frow + 16 * (frow >> 2), 64);
     }
   }
+  // the bias and residual of the epilogue: all at once, and beside the hand-off of a split
+  const int col = 16 * (4 * cg + cw) + 4 * g, n_out = PAIR ? p.N / 2 : p.N, lcol = min(col, n_out - 4);
+  const bool r4 = !PAIR && p.R && p.ldr % 4 == 0 && (uintptr_t)p.R % 8 == 0;
+  float bias[NG][4] = {};
+  if (p.bias)
+#pragma unroll
+    for (int j = 0; j < NG; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[j][e] = bf2f(p.bias[j * n_out + lcol + e]);
+  uint2 res[RT];
+  if (r4)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) res[t] = *(const uint2*)(p.R + (long)min(16 * t + frow, p.M - 1) * p.ldr + lcol);
   if (split > 1) {
     constexpr int SLAB = 16 * RT * COLS + 64;
     typedef unsigned long long u64;
@@ -774,51 +793,70 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
     __syncthreads();
     if (!*flag) return;
     if (tid == 0) __hip_atomic_store(tickets + cg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the last one adds all parts in their order, its own among them
-    u64* base = (u64*)(slabs + (long)cg * split * SLAB);
+    // the last one adds all parts in their order, its own among them; all row tiles' loads of AT_ONCE parts in flight
+    const u64* base = (const u64*)(slabs + (long)cg * split * SLAB);
+    constexpr int AT_ONCE = PAIR ? 2 : 4;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
+      if (normed) ss[t] = 0.f;
 #pragma unroll
-      for (int j = 0; j < NG; ++j) {
-        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int q = 0; q < split; ++q) {
-          const u64* d = base + (long)q * (SLAB / 2) + (((t * NG + j) * 4 + cw) * 64 + lane) * 2;
-          const u64 a = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          const u64 b = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          v += f32x4{__uint_as_float((unsigned)a), __uint_as_float((unsigned)(a >> 32)), __uint_as_float((unsigned)b),
-                     __uint_as_float((unsigned)(b >> 32))};
+      for (int j = 0; j < NG; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int q0 = 0; q0 < split; q0 += AT_ONCE) {
+      u64 v[AT_ONCE][RT][NG][2];
+      float s[AT_ONCE][RT];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const u64* part = base + (long)min(q0 + k, split - 1) * (SLAB / 2);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+#pragma unroll
+          for (int j = 0; j < NG; ++j)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+              v[k][t][j][e] = __hip_atomic_load(part + (((t * NG + j) * 4 + cw) * 64 + lane) * 2 + e, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+          s[k][t] = __hip_atomic_load((const float*)part + 16 * RT * COLS + 16 * t + frow, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);  // unused without a norm
         }
-        acc[t][j] = v;
       }
-      if (normed) {
-        float v = 0.f;
-        for (int q = 0; q < split; ++q)
-          v += __hip_atomic_load((const float*)base + (long)q * SLAB + 16 * RT * COLS + 16 * t + frow, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-        ss[t] = v;
-      }
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k)
+        if (q0 + k < split)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+#pragma unroll
+            for (int j = 0; j < NG; ++j)
+              acc[t][j] += f32x4{__uint_as_float((unsigned)v[k][t][j][0]), __uint_as_float((unsigned)(v[k][t][j][0] >> 32)),
+                                 __uint_as_float((unsigned)v[k][t][j][1]), __uint_as_float((unsigned)(v[k][t][j][1] >> 32))};
+            if (normed) ss[t] += s[k][t];
+          }
     }
   }
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const int row = 16 * t + frow;
-    if (row >= p.M) continue;
+    if (row >= p.M || col >= n_out) continue;
     const float rs = normed ? rsqrtf(ss[t] / (float)p.K + p.norm_eps) : 1.f;
-    const int col = 16 * (4 * cg + cw) + 4 * g;
-    if (col >= (PAIR ? p.N / 2 : p.N)) continue;
-    float y[4];
+    float y[4], r[4] = {};
+    if (r4) {
+      r[0] = __uint_as_float(res[t].x << 16); r[1] = __uint_as_float(res[t].x & 0xffff0000u);
+      r[2] = __uint_as_float(res[t].y << 16); r[3] = __uint_as_float(res[t].y & 0xffff0000u);
+    } else if (!PAIR && p.R) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = bf2f(p.R[(long)row * p.ldr + col + e]);
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       y[e] = acc[t][0][e] * rs;
-      if (p.bias) y[e] += bf2f(p.bias[col + e]);
+      if (p.bias) y[e] += bias[0][e];
       if constexpr (PAIR) {
         float up = acc[t][1][e] * rs;
-        if (p.bias) up += bf2f(p.bias[p.N / 2 + col + e]);
+        if (p.bias) up += bias[1][e];
         y[e] = glu(y[e], up, p.glu);
       } else {
         y[e] = apply_act(y[e], p.act);
-        if (p.R) y[e] += bf2f(p.R[(long)row * p.ldr + col + e]);
+        if (p.R) y[e] += r[e];
       }
     }
     if constexpr (OUT_F32) *(float4*)((float*)p.C + (long)row * p.ldc + col) = make_float4(y[0], y[1], y[2], y[3]);
@@ -1529,15 +1567,15 @@ static int decode_split(int N, int K) {
 
 // Image products of 16 < M <= 64 rows: re-reading X per 16-row group is the cheaper way while the product is small and its
 // groups fill the chip no more than once. us, direct | best split of the other, M = 24 / 48 / 64: 2048 x 2048 6.7 / 9.3 / 11.1
-// | 8.7 / 10.6 / 12.4; 3072 x 2048 7.1 / 9.9 / 11.7 | 10.1 / 12.8 / 14.3; 4096 x 4096 11.1 / 16.3 / 19.9 | 12.4 / 14.5 / 16.6
+// | 8.7 / 10.6 / 12.4 (before the hand-off took one trip); 3072 x 2048 7.1 / 9.9 / 11.7 | 10.1 / 12.8 / 14.3; 4096 x 4096 11.1 / 16.3 / 19.9 | 12.4 / 14.5 / 16.6
 // (M = 32: 12.1 | 12.4); 2048 x 7168, long K, 15.8 / 24 / 30 | 12.9 / 15.6 / 18.0.
 static bool gemm64_direct(int M, int N, int K) {
   return tuning().decode_split == 0 && N <= 4096 && K <= 4096 && (long)M * N * K <= 1L << 29;
 }
 // Split over K: up to one workgroup per CU, with at least 16 chunks each, 32 for the gated pairs whose partial tiles are
-// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 21.3 / 17.3 / 16.7 / 14.5 / 18.8 / 19.1;
-// 4096 x 14336 63.6 / 40.0 / 32.6 / 27.7 / 35.6 / 32.1; 6144 x 4096 22.1 / 19.3 / 24.3 / 21.7; 10304 x 4096 (161 groups)
-// 22.7 / 27.4; SwiGLU 14336 x 2048 18.0 / 20.8.
+// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 20.7 / 16.9 / 14.2 / 13.3 / 17.6 / 17.8;
+// 4096 x 14336 62.4 / 42.1 / 32.7 / 28.0 / 35.4 / 32.2; 6144 x 4096 21.7 / 17.3 / 21.5 / 19.1; 10304 x 4096 (161 groups)
+// 26.4 / 27.9; SwiGLU 14336 x 2048 18.0 / 17.4.
 static int gemm64_split(int groups, int K, bool pair) {
   if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
   int split = 1;
