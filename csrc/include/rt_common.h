@@ -287,6 +287,10 @@ __device__ __forceinline__ void sum_slabs8(const float* p, long stride, int ns, 
     lo[q] = *(const float4*)sp;
     hi[q] = *(const float4*)(sp + 4);
   }
+  // used here: else the compiler moves a slab's loads to its addition, behind the wait for the others
+#pragma unroll
+  for (int q = 1; q < 8; ++q)
+    asm volatile("" : "+v"(lo[q].x), "+v"(lo[q].y), "+v"(lo[q].z), "+v"(lo[q].w), "+v"(hi[q].x), "+v"(hi[q].y), "+v"(hi[q].z), "+v"(hi[q].w));
   out[0] = lo[0].x; out[1] = lo[0].y; out[2] = lo[0].z; out[3] = lo[0].w;
   out[4] = hi[0].x; out[5] = hi[0].y; out[6] = hi[0].z; out[7] = hi[0].w;
 #pragma unroll
@@ -362,7 +366,13 @@ __device__ __forceinline__ float block_sum(float v, float* sbuf) {
   if (lane == 0) sbuf[wid] = v;
   __syncthreads();
   float r = 0.f;
-  for (int i = 0; i < nw; ++i) r += sbuf[i];
+  for (int i0 = 0; i0 < nw; i0 += 8) {  // eight reads under way instead of a wait for each
+    float t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = sbuf[min(i0 + i, nw - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r += i0 + i < nw ? t[i] : -0.f;
+  }
   return r;
 }
 

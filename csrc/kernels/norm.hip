@@ -34,29 +34,39 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
   // weight (and bias) loads are issued with the row loads: one memory round trip before the
   // reduction instead of a second dependent one after it (decode rows are latency-bound)
   uint4 wraw[NV], braw[NV];
+  // and nothing stands between the loads: a branch for each was a trip for each (x, then res, and one slab's own: 256 rows of 4096
+  // over eight slabs 9.4 -> 8.6 us)
+  uint4 rraw[NV];
+  auto at = [&](int i) { return min((int)(threadIdx.x + i * blockDim.x), nv - 1) * 8; };
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = threadIdx.x + i * blockDim.x;
-    if (c < nv) {
-      wraw[i] = *(const uint4*)(w + c * 8);
-      if (LAYERNORM && b) braw[i] = *(const uint4*)(b + c * 8);
+  for (int i = 0; i < NV; ++i) wraw[i] = *(const uint4*)(w + at(i));
+  if (LAYERNORM && b)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) braw[i] = *(const uint4*)(b + at(i));
+  if (res)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) rraw[i] = *(const uint4*)(res + row * H + at(i));
+  if (xs) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      sum_slabs8(xs + row * H + at(i), sstride, nsplit, v[i]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[i][k] = bf2f(f2bf(v[i][k]));  // = the reduce kernel's bf16 output
     }
+  } else {
+    uint4 xraw[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) xraw[i] = *(const uint4*)(xr + at(i));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) unpack8(xraw[i], v[i]);
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * blockDim.x;
     if (c < nv) {
-      if (xs) {
-        float t8[8];
-        sum_slabs8(xs + row * H + c * 8, sstride, nsplit, t8);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[i][k] = bf2f(f2bf(t8[k]));  // = the reduce kernel's bf16 output
-      } else {
-        unpack8(*(const uint4*)(xr + c * 8), v[i]);
-      }
       if (res) {
         float r[8];
-        unpack8(*(const uint4*)(res + row * H + c * 8), r);
+        unpack8(rraw[i], r);
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[i][k] += r[k];
         // the residual stream is kept in bf16: round before normalising so fwd == what bwd sees
@@ -108,6 +118,8 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
 // sums' LDS exchanges and barriers were a good part of a short row's time. The NW partial sums are those of
 // norm_fwd_kernel's NW waves, added in its order: the same bits. LayerNorm with residual, us before -> now: 23000 x 384 16.7 ->
 // 13.8, 23000 x 768 31.3 -> 25.4 (5.6 TB/s), 4096 x 1024 7.9 -> 7.2, 15 x 384 3.0 -> 2.8
+// A row's loads all go out before the first is used (a branch for the residual and for each vector's end made each wait for its
+// own), on one machine: 23000 x 384 14.1 -> 13.5, 23000 x 768 31.8 -> 30.0, 80000 x 384 53.0 -> 49.6.
 template <bool LAYERNORM, int NW>
 __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                         const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
@@ -115,26 +127,30 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict
                                                         float* __restrict__ rstd_out, float* __restrict__ mean_out,
                                                         int T, int H, float eps) {
   const int lane = threadIdx.x & 63, nv = H / 8;
+  auto at = [&](int i) { return min(lane + 64 * i, nv - 1) * 8; };  // no branch between the loads: one trip for all
   uint4 wraw[NW], braw[NW];
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    const int c = lane + 64 * i;
-    if (c < nv) {
-      wraw[i] = *(const uint4*)(w + c * 8);
-      if (LAYERNORM && b) braw[i] = *(const uint4*)(b + c * 8);
-    }
+    wraw[i] = *(const uint4*)(w + at(i));
+    if (LAYERNORM && b) braw[i] = *(const uint4*)(b + at(i));
   }
   for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < T; row += (long)gridDim.x * 4) {
+    uint4 xraw[NW], rraw[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) xraw[i] = *(const uint4*)(x + row * H + at(i));
+    if (res)
+#pragma unroll
+      for (int i = 0; i < NW; ++i) rraw[i] = *(const uint4*)(res + row * H + at(i));
     float v[NW][8], s[NW];
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int c = lane + 64 * i;
       s[i] = 0.f;
       if (c < nv) {
-        unpack8(*(const uint4*)(x + row * H + c * 8), v[i]);
+        unpack8(xraw[i], v[i]);
         if (res) {
           float r[8];
-          unpack8(*(const uint4*)(res + row * H + c * 8), r);
+          unpack8(rraw[i], r);
 #pragma unroll
           for (int k = 0; k < 8; ++k) v[i][k] += r[k];
 #pragma unroll
@@ -430,7 +446,9 @@ __device__ __forceinline__ void act_stv(T* p, const float* o) {
   }
 }
 
-// V elements per access (4, or 1 when H % 4 != 0), NV accesses per thread
+// V elements per access (4, or 1 when H % 4 != 0), NV accesses per thread. A row of a decode step waits for trips to memory: x, y
+// and, up to NV = 4, the weights of both norms go out at once, with nothing between them (a row of 4096 in two accesses a thread,
+// 64 rows, 5.6 -> 4.8 us).
 template <typename T, int KIND, int V, int NV>
 __global__ __launch_bounds__(512) void branch_norm_kernel(BranchArgs a) {
   __shared__ float sbuf[8];
@@ -443,19 +461,52 @@ __global__ __launch_bounds__(512) void branch_norm_kernel(BranchArgs a) {
     tok = a.ids[row];
     tok = tok < 0 ? 0 : (tok >= a.vocab ? a.vocab - 1 : tok);
   }
+  constexpr bool AHEAD = NV <= 4;  // the weights, too
+  constexpr int NA = AHEAD ? NV : 1;
+  struct alignas(V * sizeof(T)) Raw { T v[V]; };
+  Raw wb[NA], ws[NA], wn[NA];
+  auto at = [&](int i) { return min((int)(threadIdx.x + i * blockDim.x), nvec - 1) * V; };
+  if (KIND == Y_NONE && a.table) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) act_ldv<T, V>((const T*)a.table + tok * a.H + at(i), x[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) act_ldv<float, V>(xr + at(i), x[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if constexpr (KIND == Y_ACT) {
+      act_ldv<T, V>((const T*)a.y + row * a.H + at(i), y[i]);
+    } else if constexpr (KIND == Y_SLABS) {
+      act_ldv<float, V>((const float*)a.y + row * a.H + at(i), y[i]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) y[i][e] = 0.f;
+    }
+  }
+  if constexpr (AHEAD) {  // of what is not given the row, unused
+    auto ahead = [&](const void* p, Raw (&w)[NA]) {
+      const T* from = p ? (const T*)p : (const T*)xr;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) w[i] = *(const Raw*)(from + at(i));
+    };
+    if constexpr (KIND != Y_NONE) {
+      ahead(a.w_branch, wb);
+      ahead(a.scale, ws);
+    }
+    ahead(a.w_next, wn);
+  }
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * blockDim.x;
+    if (c >= nvec) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) { x[i][e] = 0.f; y[i][e] = 0.f; }
-    if (c >= nvec) continue;
-    if (KIND == Y_NONE && a.table) act_ldv<T, V>((const T*)a.table + tok * a.H + c * V, x[i]);
-    else act_ldv<float, V>(xr + c * V, x[i]);
-    if constexpr (KIND == Y_ACT) {
-      act_ldv<T, V>((const T*)a.y + row * a.H + c * V, y[i]);
-    } else if constexpr (KIND == Y_SLABS) {
-      for (int q = 0; q < a.nsplit; ++q) {
+      for (int e = 0; e < V; ++e) { x[i][e] = 0.f; y[i][e] = 0.f; }
+      continue;
+    }
+    if constexpr (KIND == Y_SLABS) {
+      for (int q = 1; q < a.nsplit; ++q) {
         float t[V];
         act_ldv<float, V>((const float*)a.y + q * a.y_stride + row * a.H + c * V, t);
 #pragma unroll
@@ -506,10 +557,10 @@ __global__ __launch_bounds__(512) void branch_norm_kernel(BranchArgs a) {
       const int c = threadIdx.x + i * blockDim.x;
       if (c >= nvec) continue;
       float w[V];
-      act_ldv<T, V>((const T*)a.w_branch + c * V, w);
+      act_ldv<T, V>(AHEAD ? wb[i % NA].v : (const T*)a.w_branch + c * V, w);
       if (a.scale) {
         float f[V];
-        act_ldv<T, V>((const T*)a.scale + c * V, f);
+        act_ldv<T, V>(AHEAD ? ws[i % NA].v : (const T*)a.scale + c * V, f);
 #pragma unroll
         for (int e = 0; e < V; ++e) w[e] *= f[e];
       }
@@ -544,7 +595,7 @@ __global__ __launch_bounds__(512) void branch_norm_kernel(BranchArgs a) {
     const int c = threadIdx.x + i * blockDim.x;
     if (c >= nvec) continue;
     float w[V], o[V];
-    act_ldv<T, V>((const T*)a.w_next + c * V, w);
+    act_ldv<T, V>(AHEAD ? wn[i % NA].v : (const T*)a.w_next + c * V, w);
 #pragma unroll
     for (int e = 0; e < V; ++e) o[e] = x[i][e] * rstd * w[e];
     act_stv<T, V>((T*)a.h + row * a.H + c * V, o);
