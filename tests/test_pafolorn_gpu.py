@@ -278,6 +278,36 @@ def test_window_decode_partitions(T, parts, heads):
         assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, b
 
 
+@pytest.mark.parametrize("norms", [(True, True), (False, True), (False, False)])
+@pytest.mark.parametrize("H,G,D,V,half", [(32, 8, 128, 128, 64), (4, 2, 16, 8, 8), (40, 8, 136, 72, 64), (64, 32, 64, 64, 8), (1, 1, 256, 256, 128)])
+def test_window_prep_in_registers(H, G, D, V, half, norms):
+    """The form that holds a token in registers against the one that walks it (tables off 16 bytes): the same up to the order of
+    the norms' sums, one rounding to bf16; one lead a thread and two, chunks that do not turn, rows and positions out of range."""
+    T, rows, most = 9, 3, 130
+    g = torch.Generator(device=DEV).manual_seed(H * D + half)
+    d = ops.WindowDims(H, G, D, V, 1.0, 0.0, 0, 0)
+    proj = torch.randn(T, d.in_cols + 8, generator=g, device=DEV).bfloat16()
+    qn, kn = (torch.rand(n * D, generator=g, device=DEV).bfloat16() if on else None for n, on in zip((H, G), norms))
+    tab = torch.arange(1, 1 + rows * 3, dtype=torch.int32, device=DEV).view(rows, 3)
+    row = torch.tensor([0, 1, 2, 0, -1, 3, 1, 2, 2], dtype=torch.int32, device=DEV)  # every slot once
+    pos = torch.tensor([0, 63, 64, 129, 5, 7, 1000, -4, 191], dtype=torch.int32, device=DEV)
+    dims, fs = d.args()
+    got = []
+    for off in (0, 1):
+        flat = torch.Generator(device=DEV).manual_seed(1)
+        cos, sin = (torch.randn(most * half + off, generator=flat, device=DEV)[off:] for _ in range(2))
+        if off:
+            cos.copy_(first[0]), sin.copy_(first[1])
+        first = cos.clone(), sin.clone()
+        pool = torch.full((rows * 3 + 1, 64, G * (D + V)), 0.25, dtype=torch.bfloat16, device=DEV)
+        p = proj.clone()
+        ops.native().window_prep(p, 8, qn, kn, 1e-6, cos.view(most, half), sin.view(most, half), row, pos, pool, tab, dims, fs)
+        got.append((p.float(), pool.float()))
+    for a, b in zip(*got):
+        # a bf16 step, or what the order of the two products' sum is worth: 2^-23 of |u| |s| + |v| |c| < 32
+        assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 4e-6).all()
+
+
 @pytest.mark.parametrize("window,keep", [(0, 0), (5000, 100)])
 @pytest.mark.parametrize("D,V", [(8, 16), (136, 8)])
 def test_window_decode_of_many_pages(D, V, window, keep):
