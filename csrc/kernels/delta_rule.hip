@@ -160,6 +160,15 @@ __global__ __launch_bounds__(BLOCK) void delta_step_kernel(Args a) {
   const float dt = a.dt[a.channel ? (long)h * D + min(tid, D - 1) : h], A_log = a.A_log[h];
   const T* zp = (const T*)a.z + (long)t * a.ldz + (long)h * V;
   const uint32_t zw = word(zp + min(tid, V - 1)), nw = word((const T*)a.norm_w + min(tid, V - 1));
+  auto older = [&](int c, int j0) {  // taps from j0 tokens ago on
+    float y = 0.f;
+    for (int j = taps - 1; j >= j0; --j)
+      if (seen(j)) y = fmaf(ld(conv + (long)c * taps + taps - 1 - j), value<T>(past(c, j)), y);
+    return y;
+  };
+  float yo[PRE];  // the taps beyond: no load under a condition may stand behind the state's
+#pragma unroll
+  for (int k = 0; k < PRE; ++k) yo[k] = older(chan(min(tid + k * BLOCK, nch - 1)), TAP);
   asm volatile("" ::: "memory");
   float* Sp = a.S + (((long)row * a.H + h) * D) * V + (mine ? cg * VEC : 0);
   float s[NR][VEC];
@@ -179,29 +188,23 @@ __global__ __launch_bounds__(BLOCK) void delta_step_kernel(Args a) {
       }
     }
   }
-  auto put = [&](int i, int c, float y) {
+  auto put = [&](int i, int c, float y, float now) {  // now: the channel's input, not loaded again behind the state
     y *= sigmoid(y);
     (i < D ? qs[i] : (i < 2 * D ? ks[i - D] : vs[i - 2 * D])) = y;
     // the slot of this position is read by nobody at this position; heads that share a key head share the write
-    if (live && (i >= 2 * D || h % (a.H / a.K) == 0)) ring[(long)slot * C + c] = xt[c];
-  };
-  auto older = [&](int c, int j0) {  // taps from j0 tokens ago on
-    float y = 0.f;
-    for (int j = taps - 1; j >= j0; --j)
-      if (seen(j)) y = fmaf(ld(conv + (long)c * taps + taps - 1 - j), value<T>(past(c, j)), y);
-    return y;
+    if (live && (i >= 2 * D || h % (a.H / a.K) == 0)) st(ring + (long)slot * C + c, now);
   };
 #pragma unroll
   for (int k = 0; k < PRE; ++k) {
     const int i = tid + k * BLOCK;
     if (i >= nch) continue;
     const int c = chan(i);
-    float y = older(c, TAP);
+    float y = yo[k];
 #pragma unroll
     for (int j = TAP - 1; j >= 0; --j) y = seen(j) ? fmaf(value<T>(ww[k][j]), value<T>(xw[k][j]), y) : y;
-    put(i, c, y);
+    put(i, c, y, value<T>(xw[k][0]));
   }
-  for (int i = tid + PRE * BLOCK; i < nch; i += BLOCK) put(i, chan(i), older(chan(i), 0));
+  for (int i = tid + PRE * BLOCK; i < nch; i += BLOCK) put(i, chan(i), older(chan(i), 0), ld(xt + chan(i)));
   const float A = expf(A_log);
   if (a.channel) {
     if (tid < D) gs[tid] = expf(-A * softplus(value<T>(aw) + dt));
