@@ -880,6 +880,26 @@ __global__ __launch_bounds__(256, 2) void gemm_duo_kernel(Args p) {
   bf16_t* C = (bf16_t*)p.C;
   const int cc = tid & 15, gcol = n0 + cc * 8;
   if (gcol >= p.N) return;
+  // A whole tile without a residual: nothing between the reads of eight rows and their stores. With each row's
+  // check in between, a row's read was waited for before the next was issued: 16 LDS trips in a row at the end of
+  // a tile. Encoder forwards of 256 / 1024 texts 5554 / 4141 -> 5488 / 4064 us (duo products are about half of
+  // them). The last row of tiles and products with a residual keep the loop, which checks each row.
+  if (m0 + 256 <= p.M && !p.R) {
+#pragma unroll
+    for (int r0 = 0; r0 < 256; r0 += 128) {
+      uint2 v[8][2];
+      const bf16_t* from = tile + (r0 + (tid >> 4)) * LDT + cc * 8;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j][0] = *(const uint2*)(from + j * 16 * LDT);
+        v[j][1] = *(const uint2*)(from + j * 16 * LDT + 4);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        *(uint4*)(C + (long)(m0 + r0 + (tid >> 4) + j * 16) * p.ldc + gcol) = make_uint4(v[j][0].x, v[j][0].y, v[j][1].x, v[j][1].y);
+    }
+    return;
+  }
 #pragma unroll 4
   for (int row = tid >> 4; row < 256; row += 16) {
     const int grow = m0 + row;
