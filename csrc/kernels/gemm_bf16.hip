@@ -413,37 +413,31 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
   // NW waves split the group's K chunks (NW = 8: twice the weight bytes in flight per workgroup)
   __shared__ float red[NW][16][PAIR ? 33 : 17];
   __shared__ float rsq[NW][16];
-  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int frow = lane & 15, g = lane >> 4;
   const int grp = blockIdx.x;  // 16-row group (of the gate rows when PAIR)
   constexpr int KC = W8 ? 128 : 64;  // k per 2-KiB chunk
   const int nc = p.K / KC;
   const int c_begin = wid * nc / NW, c_end = (wid + 1) * nc / NW;
-  // this wave's chunks end the buffer: what is asked for beyond is 0 and no access
-  const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc((char*)p.B + (long)grp * nc * 2048, 0, c_end * 2048, 0x00020000);
-  const __amdgpu_buffer_rsrc_t ubase = __builtin_amdgcn_make_buffer_rsrc(
-      (char*)p.B + ((long)(PAIR ? p.N / 32 : 0) + grp) * nc * 2048, 0, c_end * 2048, 0x00020000);
-  auto nt16 = [&](__amdgpu_buffer_rsrc_t from, int off) {  // 2: non-temporal
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(from, off + lane * 16, 0, 2));
-  };
+  const char* wbase = (const char*)p.B + (long)grp * nc * 2048 + lane * 16;
+  const char* ubase = PAIR ? (const char*)p.B + ((long)(p.N / 32) + grp) * nc * 2048 + lane * 16 : wbase;
   const bf16_t* xrow = p.A + (long)min(frow, p.M - 1) * p.lda + g * (W8 ? 16 : 8);
   struct Regs { uint4 w0, w1, u0, u1, x0, x1, x2, x3; };
   auto ld = [&](Regs& r, int c) {
-    r.w0 = nt16(wbase, c * 2048);
-    r.w1 = nt16(wbase, c * 2048 + 1024);
+    r.w0 = load_nt16(wbase + (long)c * 2048);
+    r.w1 = load_nt16(wbase + (long)c * 2048 + 1024);
     if constexpr (PAIR) {
-      r.u0 = nt16(ubase, c * 2048);
-      r.u1 = nt16(ubase, c * 2048 + 1024);
+      r.u0 = load_nt16(ubase + (long)c * 2048);
+      r.u1 = load_nt16(ubase + (long)c * 2048 + 1024);
     }
-    const bf16_t* xc = c < c_end ? xrow + c * KC : p.A;  // beyond: one place for all lanes, unused
     if constexpr (W8) {  // k [128 c + 64 h + 16 g, +16) as two 8-element halves, h = 0, 1
-      r.x0 = *(const uint4*)(xc);
-      r.x1 = *(const uint4*)(xc + 8);
-      r.x2 = *(const uint4*)(xc + 64);
-      r.x3 = *(const uint4*)(xc + 72);
+      r.x0 = *(const uint4*)(xrow + c * 128);
+      r.x1 = *(const uint4*)(xrow + c * 128 + 8);
+      r.x2 = *(const uint4*)(xrow + c * 128 + 64);
+      r.x3 = *(const uint4*)(xrow + c * 128 + 72);
     } else {
-      r.x0 = *(const uint4*)(xc);
-      r.x1 = *(const uint4*)(xc + 32);
+      r.x0 = *(const uint4*)(xrow + c * 64);
+      r.x1 = *(const uint4*)(xrow + c * 64 + 32);
     }
   };
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, accu = acc;
@@ -494,21 +488,20 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
   const bool has_r = !PAIR && p.R;
   const bf16_t res = has_r ? p.R[(long)min(row, p.M - 1) * p.ldr + col] : (bf16_t)0;
   Regs r[DEPTH];
-  // No load under a condition, behind which the compiler would wait for all of them instead of counting. 1 row, us: SwiGLU
-  // 28672 x 4096 39.1 -> 38.3, 32000 x 4096 42.2 -> 41.0 (6.4 TB/s); at 16 rows, where X's loads take the address path as long
-  // as the weights take memory, nothing.
 #pragma unroll
-  for (int i = 0; i < DEPTH - 1; ++i) {
-    ld(r[i], c_begin + i);
-    __builtin_amdgcn_sched_barrier(0);  // in this order
-  }
-  for (int c = c_begin; c < c_end; c += DEPTH) {
+  for (int i = 0; i < DEPTH - 1; ++i)
+    if (c_begin + i < c_end) ld(r[i], c_begin + i);
+  int c = c_begin;
+  for (; c + DEPTH <= c_end; c += DEPTH) {
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) {
-      ld(r[(i + DEPTH - 1) % DEPTH], c + i + DEPTH - 1);
-      if (c + i < c_end) mma(r[i]);
+      if (c + i + DEPTH - 1 < c_end) ld(r[(i + DEPTH - 1) % DEPTH], c + i + DEPTH - 1);
+      mma(r[i]);
     }
   }
+#pragma unroll
+  for (int i = 0; i < DEPTH - 1; ++i)
+    if (c + i < c_end) mma(r[i]);
   // acc[r] of lane (frow, g) = C[row 4 g + r][16 grp + frow] over this wave's k range; the X row
   // sum of squares of row frow is spread over its 4 g lanes
 #pragma unroll
