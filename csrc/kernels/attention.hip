@@ -1467,9 +1467,16 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
     raw(row + (long)min(hk * G + r16, a.Hq - 1) * D, row + (long)(a.Hq + hk) * D, row + (long)(a.Hq + a.Hkv + hk) * D);
     __builtin_amdgcn_sched_barrier(0);
     load(ta, cfirst);
-    load(tb, cfirst + cstep);
+    if constexpr (W < 8) load(tb, cfirst + cstep);
   }
-  load(tc, cfirst + 2 * cstep);
+  if constexpr (W < 8) {
+    load(tc, cfirst + 2 * cstep);
+  } else if (cfirst + cstep < len) {
+    // Eight waves over one row: up to 128 keys none has a second tile, and 16 loads a wave of slot len - 1 are not free
+    // (3 rows of 95..133 keys, 40 pairs of heads a row: 8.7 us with them, 8.0 without; before either 8.3). Longer rows keep their 9.8.
+    load(tb, cfirst + cstep);
+    load(tc, cfirst + 2 * cstep);
+  }
   __builtin_amdgcn_sched_barrier(0);
   // x rotated with partner y: lo half (chunk < 8) x c - y s', hi half x c + y s' (s' = sign sin),
   // rounded to bf16 as the unfused rope kernel stores it
