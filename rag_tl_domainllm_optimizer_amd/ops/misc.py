@@ -26,7 +26,7 @@ def upload(src, device) -> torch.Tensor:
     device = torch.device(device)
     if device.type != "cuda" or t.is_cuda or t.numel() * t.element_size() > UPLOAD_PINNED or torch.cuda.is_current_stream_capturing():
         return t.to(device)
-    buf = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+    buf = torch.empty(t.shape, dtype=t.dtype, device="cpu", pin_memory=True)  # whatever the default device
     buf.copy_(t)
     return buf.to(device, non_blocking=True)
 

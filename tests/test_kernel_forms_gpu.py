@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from rag_tl_domainllm_optimizer_amd import ops
+from rag_tl_domainllm_optimizer_amd.generation.ragged import RaggedBatch
 from rag_tl_domainllm_optimizer_amd.ops import reference as ref
 
 pytestmark = pytest.mark.gpu
@@ -779,3 +780,14 @@ def test_upload_holds_the_source_of_the_call(n, dtype):
     src += 7
     for g in got:
         assert g.device.type == "cuda" and g.is_contiguous() and np.array_equal(g.cpu().numpy(), want)
+
+
+def test_upload_under_a_default_device():
+    """ops.upload and the tables made with it where new tensors go to the GPU by default, numpy arrays and CPU tensors alike."""
+    src = np.arange(1000, dtype=np.int64)
+    with torch.device(DEV):
+        got = [ops.upload(src, DEV), ops.upload(torch.from_numpy(src), DEV), ops.upload(torch.arange(1000), DEV)]
+        batch = RaggedBatch.build([(0, [5, 6, 7], 0), (1, [8] * 40, 3)], DEV)
+    for g in got:
+        assert g.device.type == "cuda" and torch.equal(g.cpu(), torch.from_numpy(src))
+    assert batch.ids.tolist() == [5, 6, 7] + [8] * 40 and batch.pos.tolist() == [0, 1, 2] + list(range(3, 43))
