@@ -118,9 +118,13 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
 // sums' LDS exchanges and barriers were a good part of a short row's time. The NW partial sums are those of
 // norm_fwd_kernel's NW waves, added in its order: the same bits. LayerNorm with residual, us before -> now: 23000 x 384 16.7 ->
 // 13.8, 23000 x 768 31.3 -> 25.4 (5.6 TB/s), 4096 x 1024 7.9 -> 7.2, 15 x 384 3.0 -> 2.8
-// A row's loads all go out before the first is used (a branch for the residual and for each vector's end made each wait for its
-// own), on one machine: 23000 x 384 14.1 -> 13.5, 23000 x 768 31.8 -> 30.0, 80000 x 384 53.0 -> 49.6.
-template <bool LAYERNORM, int NW>
+// ONCE: a row's loads all go out before the first is used (a branch for the residual and for each vector's end made each wait for
+// its own), and the residual stream is stored beside the result: stored between the loads' arrival and the sums it cost long rows
+// what the loads had gained. LayerNorm with residual, us, each vector for itself -> at once -> and stored at the end, on one machine:
+// 23000 x 384 13.9 -> 13.4 -> 12.4, 23000 x 768 30.9 -> 28.5 -> 25.3, 4096 x 1024 8.1 -> 8.9 -> 8.1. RMS with residual: 1024 x 1024
+// 3.6 -> 3.4 -> 3.2, but from about 4096 rows of two vectors on, when every SIMD has rows enough to hide the trips, a row's loads
+// side by side cost more than they save (4096 x 1024 7.0 -> 8.0, 8192 x 768 9.3 -> 10.0): not ONCE, each vector for itself.
+template <bool LAYERNORM, int NW, bool ONCE>
 __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                         const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
                                                         bf16_t* __restrict__ y, bf16_t* __restrict__ h_out,
@@ -136,26 +140,28 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict
   }
   for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < T; row += (long)gridDim.x * 4) {
     uint4 xraw[NW], rraw[NW];
+    if constexpr (ONCE) {
 #pragma unroll
-    for (int i = 0; i < NW; ++i) xraw[i] = *(const uint4*)(x + row * H + at(i));
-    if (res)
+      for (int i = 0; i < NW; ++i) xraw[i] = *(const uint4*)(x + row * H + at(i));
+      if (res)
 #pragma unroll
-      for (int i = 0; i < NW; ++i) rraw[i] = *(const uint4*)(res + row * H + at(i));
+        for (int i = 0; i < NW; ++i) rraw[i] = *(const uint4*)(res + row * H + at(i));
+    }
     float v[NW][8], s[NW];
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int c = lane + 64 * i;
       s[i] = 0.f;
       if (c < nv) {
-        unpack8(xraw[i], v[i]);
+        unpack8(ONCE ? xraw[i] : *(const uint4*)(x + row * H + c * 8), v[i]);
         if (res) {
           float r[8];
-          unpack8(rraw[i], r);
+          unpack8(ONCE ? rraw[i] : *(const uint4*)(res + row * H + c * 8), r);
 #pragma unroll
           for (int k = 0; k < 8; ++k) v[i][k] += r[k];
 #pragma unroll
           for (int k = 0; k < 8; ++k) v[i][k] = bf2f(f2bf(v[i][k]));
-          if (h_out) *(uint4*)(h_out + row * H + c * 8) = pack8(v[i]);
+          if (!ONCE && h_out) *(uint4*)(h_out + row * H + c * 8) = pack8(v[i]);
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) s[i] += LAYERNORM ? v[i][k] : v[i][k] * v[i][k];
@@ -186,6 +192,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict
       const int c = lane + 64 * i;
       if (c < nv) {
         float wv[8], bv[8], o[8];
+        if (ONCE && res && h_out) *(uint4*)(h_out + row * H + c * 8) = pack8(v[i]);
         unpack8(wraw[i], wv);
         if (LAYERNORM && b) unpack8(braw[i], bv);
 #pragma unroll
@@ -333,13 +340,18 @@ extern "C" int rt_norm_fwd(int layernorm, const void* x, const void* res, const 
   // beyond 1024 columns a workgroup a row was as fast (23000 x 2048: 85.3 and 86.5 us, RMS 74.5 and 68.4)
   if (!xs && (H <= 512 || (H <= 1024 && T >= 1024))) {
     const dim3 grid(std::min((T + 3) / 4, 2048)), block(256);
-#define NORM_ROWS(LN, NW)                                                                                           \
-  hipLaunchKernelGGL((norm_rows_kernel<LN, NW>), grid, block, 0, stream, (const bf16_t*)x, (const bf16_t*)res,      \
+#define NORM_ROWS(LN, NW, ONCE)                                                                                     \
+  hipLaunchKernelGGL((norm_rows_kernel<LN, NW, ONCE>), grid, block, 0, stream, (const bf16_t*)x, (const bf16_t*)res, \
                      (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean, T, H, eps)
-#define NORM_ROWS_LN(LN) \
-  if (H <= 512) NORM_ROWS(LN, 1); else NORM_ROWS(LN, 2)
-    if (layernorm) { NORM_ROWS_LN(true); } else { NORM_ROWS_LN(false); }
-#undef NORM_ROWS_LN
+    if (layernorm) {
+      if (H <= 512) NORM_ROWS(true, 1, true); else NORM_ROWS(true, 2, true);
+    } else if (H <= 512) {
+      NORM_ROWS(false, 1, true);
+    } else if (res && T >= 4096) {
+      NORM_ROWS(false, 2, false);
+    } else {
+      NORM_ROWS(false, 2, true);
+    }
 #undef NORM_ROWS
     RT_LAUNCH_CHECK();
     return 0;
