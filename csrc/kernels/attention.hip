@@ -1307,10 +1307,11 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 // (unbounded, the 4-wave form took 268 with its accumulators and ran one workgroup per CU: 48 rows of
 // 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every rotary-table / q /
 // k_new / v_new (or slab) load at once and the first tiles behind them: loads return in order, so the other way round
-// it waited for 24 KB a wave. All loads are unconditional, refills past the end too: behind a load under a condition
+// it waited for 24 KB a wave. Loads are unconditional, refills past the end too: behind a load under a condition
 // the compiler waits for every load at the join, and so had the three tiles arrive before the first was used, each time
-// (and lengths, slot and position one after the other: 3 trips). 1 row of 300 keys 10.5 -> 10.1 us, 48 rows of 150..1200
-// 37.9 -> 36.0, 256 rows of 173..301 (slabs) 58.9 -> 57.1. RoPE of q /
+// (and lengths, slot and position one after the other: 3 trips). But nothing is refilled unless a fourth tile follows: 128
+// rows of 2..15 keys, 40 key heads 19.0 -> 16.1 us, 48 of 20..60, 8 key heads 9.3 -> 8.8. 1 row of 300 keys 10.5 -> 10.1 us,
+// 48 rows of 150..1200 37.9 -> 36.0, 256 rows of 173..301 (slabs) 58.9 -> 57.1. RoPE of q /
 // k_new and the cache append are fused; lanes whose (clamped) key is the new token's slot use
 // k_new / v_new from registers. Measured at batch 256 (Mistral-7B, 174..301 keys): 51 us per
 // layer vs 80 us for the VALU kernel (profiles/decode_attn_r2_mfma.log).
@@ -1467,17 +1468,8 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
     raw(row + (long)min(hk * G + r16, a.Hq - 1) * D, row + (long)(a.Hq + hk) * D, row + (long)(a.Hq + a.Hkv + hk) * D);
     __builtin_amdgcn_sched_barrier(0);
     load(ta, cfirst);
-    if constexpr (W < 8) load(tb, cfirst + cstep);
+    if constexpr (W == 1) load(tb, cfirst + cstep);
   }
-  if constexpr (W < 8) {
-    load(tc, cfirst + 2 * cstep);
-  } else if (cfirst + cstep < len) {
-    // Eight waves over one row: up to 128 keys none has a second tile, and 16 loads a wave of slot len - 1 are not free
-    // (3 rows of 95..133 keys, 40 pairs of heads a row: 8.7 us with them, 8.0 without; before either 8.3). Longer rows keep their 9.8.
-    load(tb, cfirst + cstep);
-    load(tc, cfirst + 2 * cstep);
-  }
-  __builtin_amdgcn_sched_barrier(0);
   // x rotated with partner y: lo half (chunk < 8) x c - y s', hi half x c + y s' (s' = sign sin),
   // rounded to bf16 as the unfused rope kernel stores it
   auto rope8 = [&](const uint4& xv, const uint4& yv, const float4 (&c)[2], const float4 (&sn)[2], bool lo) -> uint4 {
@@ -1494,177 +1486,200 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
     }
     return pack8(o8);
   };
-  bf16x8 qf[DS];   // B operand of S^T = K·Q^T: Q[head r16][32 s + 8 g ..]
-  uint4 knew[DS];  // rotated k_new chunks 4 s + g (the lane's K-fragment chunks)
-#pragma unroll
-  for (int s2 = 0; s2 < DS; ++s2) {
-    const uint4 qv = rope8(qraw[s2], qraw[s2 ^ 2], cq[s2 & 1], sq[s2 & 1], s2 < 2);
-    qf[s2] = __builtin_bit_cast(bf16x8, r16 < G ? qv : make_uint4(0, 0, 0, 0));
-    knew[s2] = rope8(kraw[s2], kraw[s2 ^ 2], cq[s2 & 1], sq[s2 & 1], s2 < 2);
-  }
-  stamp(1);  // q / k_new / v_new / tables and the first tiles landed, RoPE done
-  // fp8 cache: quantise k_new / v_new per (token, kv head) (absmax / 448); this step attends over
-  // the quantised values too (knew / vxq hold them widened back to bf16, sk / sv their scales), so
-  // the step sees exactly what later steps read from the cache
-  uint4 vxq = vx;
-  float sk_new = 1.f, sv_new = 1.f;
-  uint2 kq[DS], vq = make_uint2(0, 0);
-  if constexpr (KV8) {
-    float amk = 0.f, amv = 0.f, f[8];
-#pragma unroll
-    for (int s2 = 0; s2 < DS; ++s2) {
-      unpack8(knew[s2], f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) amk = fmaxf(amk, fabsf(f[e]));
-    }
-    amk = over_groups(amk, [](float x, float y) { return fmaxf(x, y); });  // lane group g holds chunks 4 s + g
-    unpack8(vx, f);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) amv = fmaxf(amv, fabsf(f[e]));
-#pragma unroll
-    for (int o2 = 1; o2 < 16; o2 <<= 1) amv = fmaxf(amv, __shfl_xor(amv, o2, 64));  // chunk r16
-    sk_new = amk > 0.f ? amk / 448.f : 1.f;
-    sv_new = amv > 0.f ? amv / 448.f : 1.f;
-    const float ik = 1.f / sk_new, iv = 1.f / sv_new;
-#pragma unroll
-    for (int s2 = 0; s2 < DS; ++s2) {
-      unpack8(knew[s2], f);
-      kq[s2] = f32x8_to_fp8(f, ik);
-      knew[s2] = __builtin_bit_cast(uint4, fp8x8_to_bf16(kq[s2].x, kq[s2].y));
-    }
-    unpack8(vx, f);
-    vq = f32x8_to_fp8(f, iv);
-    vxq = __builtin_bit_cast(uint4, fp8x8_to_bf16(vq.x, vq.y));
-  }
-  // cache append: lane (g, 0) stores its 4 k chunks 4 s + g, lane group 1 the v chunks (wave 0)
-  if (has_new && w == 0) {
-    if constexpr (KV8) {
-      unsigned char* kdst = (unsigned char*)a.kc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
-      unsigned char* vdst = (unsigned char*)a.vc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
-      if (r16 == 0) {  // k-permuted: chunks 4 s + g at bytes 32 g + 8 s
-        *(uint4*)(kdst + 32 * g) = make_uint4(kq[0].x, kq[0].y, kq[1].x, kq[1].y);
-        *(uint4*)(kdst + 32 * g + 16) = make_uint4(kq[2].x, kq[2].y, kq[3].x, kq[3].y);
-      }
-      if (g == 1) *(uint2*)(vdst + r16 * 8) = vq;
-      if (lane == 0) {
-        a.ksc[((long)b * a.Hkv + hk) * a.SmaxP + s_new] = sk_new;
-        a.vsc[((long)b * a.Hkv + hk) * a.SmaxP + s_new] = sv_new;
-      }
-    } else {
-      bf16_t* kdst = a.kc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
-      bf16_t* vdst = a.vc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
-      if (r16 == 0) {
-#pragma unroll
-        for (int s2 = 0; s2 < DS; ++s2) *(uint4*)(kdst + (4 * s2 + g) * 8) = knew[s2];
-      }
-      if (g == 1) *(uint4*)(vdst + r16 * 8) = vx;
-    }
-  }
-
   f32x4 o[DT];
 #pragma unroll
   for (int c = 0; c < DT; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // of head r16 (identical over the 4 lane groups)
-  // P·V runs K = 32 MFMAs on 16-key tiles: k-slots 4..7 carry P = 0 against zero V rows 16..31
+  // Several waves over one row: up to 16 W keys none has a second tile, and 16 loads a wave of slot len - 1 are not free. The check
+  // for one stands around all that follows: behind a join of both the wait for q would have to be the shorter way's, and the
+  // longer's tiles arrive before it. us, tiles in any case -> check ahead of a join -> check around: 4 waves, 8 key heads, 48 rows of
+  // 20..60 keys 8.8 -> 7.8 -> 7.7, 32 of 300..600 16.0 -> 16.7 -> 15.9; 8 waves, 3 rows of 150..300 keys, 40 key heads (before any of
+  // it 10.8) 10.2 with the join, 9.2 now. One wave has nobody to fill its time: 96 rows of 20..60 keys 9.2 without a check, 9.8 with one.
+  auto attend = [&](auto more) {
+    bf16x8 qf[DS];   // B operand of S^T = K·Q^T: Q[head r16][32 s + 8 g ..]
+    uint4 knew[DS];  // rotated k_new chunks 4 s + g (the lane's K-fragment chunks)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) *(uint4*)(vimg + v_off<D>(16 + 4 * i + g, r16)) = make_uint4(0, 0, 0, 0);
-
-  auto consume = [&](Tile& T, int c0) {
-    // bf16 K fragments / V pieces of the tile (fp8: widened, unscaled e4m3 values; the per-key
-    // scales go on the scores and on P)
-    uint4 kf[DS], vf[4];
-    float ks[4] = {1.f, 1.f, 1.f, 1.f}, vs[4] = {1.f, 1.f, 1.f, 1.f};
+    for (int s2 = 0; s2 < DS; ++s2) {
+      const uint4 qv = rope8(qraw[s2], qraw[s2 ^ 2], cq[s2 & 1], sq[s2 & 1], s2 < 2);
+      qf[s2] = __builtin_bit_cast(bf16x8, r16 < G ? qv : make_uint4(0, 0, 0, 0));
+      knew[s2] = rope8(kraw[s2], kraw[s2 ^ 2], cq[s2 & 1], sq[s2 & 1], s2 < 2);
+    }
+    stamp(1);  // q / k_new / v_new / tables and the first tiles landed, RoPE done
+    // fp8 cache: quantise k_new / v_new per (token, kv head) (absmax / 448); this step attends over
+    // the quantised values too (knew / vxq hold them widened back to bf16, sk / sv their scales), so
+    // the step sees exactly what later steps read from the cache
+    uint4 vxq = vx;
+    float sk_new = 1.f, sv_new = 1.f;
+    uint2 kq[DS], vq = make_uint2(0, 0);
     if constexpr (KV8) {
+      float amk = 0.f, amv = 0.f, f[8];
 #pragma unroll
       for (int s2 = 0; s2 < DS; ++s2) {
-        const uint4& q = T.k8[s2 >> 1];
-        kf[s2] = __builtin_bit_cast(uint4, (s2 & 1) ? fp8x8_to_bf16(q.z, q.w) : fp8x8_to_bf16(q.x, q.y));
+        unpack8(knew[s2], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) amk = fmaxf(amk, fabsf(f[e]));
       }
+      amk = over_groups(amk, [](float x, float y) { return fmaxf(x, y); });  // lane group g holds chunks 4 s + g
+      unpack8(vx, f);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        vf[i] = __builtin_bit_cast(uint4, fp8x8_to_bf16(T.v8[i].x, T.v8[i].y));
-        ks[i] = T.ks[i];
-        vs[i] = T.vs[i];
+      for (int e = 0; e < 8; ++e) amv = fmaxf(amv, fabsf(f[e]));
+#pragma unroll
+      for (int o2 = 1; o2 < 16; o2 <<= 1) amv = fmaxf(amv, __shfl_xor(amv, o2, 64));  // chunk r16
+      sk_new = amk > 0.f ? amk / 448.f : 1.f;
+      sv_new = amv > 0.f ? amv / 448.f : 1.f;
+      const float ik = 1.f / sk_new, iv = 1.f / sv_new;
+#pragma unroll
+      for (int s2 = 0; s2 < DS; ++s2) {
+        unpack8(knew[s2], f);
+        kq[s2] = f32x8_to_fp8(f, ik);
+        knew[s2] = __builtin_bit_cast(uint4, fp8x8_to_bf16(kq[s2].x, kq[s2].y));
       }
-    } else {
-#pragma unroll
-      for (int s2 = 0; s2 < DS; ++s2) kf[s2] = T.k[s2];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) vf[i] = T.v[i];
+      unpack8(vx, f);
+      vq = f32x8_to_fp8(f, iv);
+      vxq = __builtin_bit_cast(uint4, fp8x8_to_bf16(vq.x, vq.y));
     }
-    if (has_new && s_new >= c0 && s_new < c0 + 16) {
-      if (min(c0 + r16, len - 1) == s_new) {
+    // cache append: lane (g, 0) stores its 4 k chunks 4 s + g, lane group 1 the v chunks (wave 0)
+    if (has_new && w == 0) {
+      if constexpr (KV8) {
+        unsigned char* kdst = (unsigned char*)a.kc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
+        unsigned char* vdst = (unsigned char*)a.vc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
+        if (r16 == 0) {  // k-permuted: chunks 4 s + g at bytes 32 g + 8 s
+          *(uint4*)(kdst + 32 * g) = make_uint4(kq[0].x, kq[0].y, kq[1].x, kq[1].y);
+          *(uint4*)(kdst + 32 * g + 16) = make_uint4(kq[2].x, kq[2].y, kq[3].x, kq[3].y);
+        }
+        if (g == 1) *(uint2*)(vdst + r16 * 8) = vq;
+        if (lane == 0) {
+          a.ksc[((long)b * a.Hkv + hk) * a.SmaxP + s_new] = sk_new;
+          a.vsc[((long)b * a.Hkv + hk) * a.SmaxP + s_new] = sv_new;
+        }
+      } else {
+        bf16_t* kdst = a.kc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
+        bf16_t* vdst = a.vc + (((long)b * a.Hkv + hk) * a.Smax + s_new) * D;
+        if (r16 == 0) {
 #pragma unroll
-        for (int s2 = 0; s2 < DS; ++s2) kf[s2] = knew[s2];
+          for (int s2 = 0; s2 < DS; ++s2) *(uint4*)(kdst + (4 * s2 + g) * 8) = knew[s2];
+        }
+        if (g == 1) *(uint4*)(vdst + r16 * 8) = vx;
       }
+    }
+
+    // P·V runs K = 32 MFMAs on 16-key tiles: k-slots 4..7 carry P = 0 against zero V rows 16..31
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (min(c0 + 4 * i + g, len - 1) == s_new) vf[i] = vxq;
-        if (KV8 && c0 + 4 * g + i == s_new) {  // this step's own scales (the prefetched ones may be stale)
-          ks[i] = sk_new;
-          vs[i] = sv_new;
+    for (int i = 0; i < 4; ++i) *(uint4*)(vimg + v_off<D>(16 + 4 * i + g, r16)) = make_uint4(0, 0, 0, 0);
+
+    auto consume = [&](Tile& T, int c0) {
+      // bf16 K fragments / V pieces of the tile (fp8: widened, unscaled e4m3 values; the per-key
+      // scales go on the scores and on P)
+      uint4 kf[DS], vf[4];
+      float ks[4] = {1.f, 1.f, 1.f, 1.f}, vs[4] = {1.f, 1.f, 1.f, 1.f};
+      if constexpr (KV8) {
+#pragma unroll
+        for (int s2 = 0; s2 < DS; ++s2) {
+          const uint4& q = T.k8[s2 >> 1];
+          kf[s2] = __builtin_bit_cast(uint4, (s2 & 1) ? fp8x8_to_bf16(q.z, q.w) : fp8x8_to_bf16(q.x, q.y));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          vf[i] = __builtin_bit_cast(uint4, fp8x8_to_bf16(T.v8[i].x, T.v8[i].y));
+          ks[i] = T.ks[i];
+          vs[i] = T.vs[i];
+        }
+      } else {
+#pragma unroll
+        for (int s2 = 0; s2 < DS; ++s2) kf[s2] = T.k[s2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vf[i] = T.v[i];
+      }
+      if (has_new && s_new >= c0 && s_new < c0 + 16) {
+        if (min(c0 + r16, len - 1) == s_new) {
+#pragma unroll
+          for (int s2 = 0; s2 < DS; ++s2) kf[s2] = knew[s2];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (min(c0 + 4 * i + g, len - 1) == s_new) vf[i] = vxq;
+          if (KV8 && c0 + 4 * g + i == s_new) {  // this step's own scales (the prefetched ones may be stale)
+            ks[i] = sk_new;
+            vs[i] = sv_new;
+          }
         }
       }
-    }
-    // V image rows 0..15 (the previous tile's transposed reads precede these writes in this
-    // wave's LDS queue)
+      // V image rows 0..15 (the previous tile's transposed reads precede these writes in this
+      // wave's LDS queue)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *(uint4*)(vimg + v_off<D>(4 * i + g, r16)) = vf[i];
-    // S^T: lane holds the scores of keys c0 + 4 g + i for head r16
-    f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4; ++i) *(uint4*)(vimg + v_off<D>(4 * i + g, r16)) = vf[i];
+      // S^T: lane holds the scores of keys c0 + 4 g + i for head r16
+      f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s2 = 0; s2 < DS; ++s2)
-      st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[s2]), qf[s2], st, 0, 0, 0);
-    float mx = -INFINITY;
+      for (int s2 = 0; s2 < DS; ++s2)
+        st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[s2]), qf[s2], st, 0, 0, 0);
+      float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float x = c0 + 4 * g + i < len ? st[i] * (KV8 ? ks[i] * a.scale_log2 : a.scale_log2) : -INFINITY;
-      st[i] = x;
-      mx = fmaxf(mx, x);
-    }
-    mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
-    const float mn = fmaxf(m, mx);  // finite: every tile holds >= 1 valid key
-    const float alpha = exp2_raw(m - mn);
-    m = mn;
-    float rs = 0.f;
+      for (int i = 0; i < 4; ++i) {
+        const float x = c0 + 4 * g + i < len ? st[i] * (KV8 ? ks[i] * a.scale_log2 : a.scale_log2) : -INFINITY;
+        st[i] = x;
+        mx = fmaxf(mx, x);
+      }
+      mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
+      const float mn = fmaxf(m, mx);  // finite: every tile holds >= 1 valid key
+      const float alpha = exp2_raw(m - mn);
+      m = mn;
+      float rs = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float pv = exp2_raw(st[i] - mn);
-      st[i] = KV8 ? pv * vs[i] : pv;  // fp8: the V scale of key c0 + 4 g + i rides on P
-      rs += pv;
-    }
-    rs = over_groups(rs, [](float x, float y) { return x + y; });
-    l = l * alpha + rs;
-    // O rows are heads 4 g + i: their factors live in lanes 4 g + i. Only rows < G are ever
-    // stored or merged (an O row depends on its own P row only), so G < 4 rescales G rows
+      for (int i = 0; i < 4; ++i) {
+        const float pv = exp2_raw(st[i] - mn);
+        st[i] = KV8 ? pv * vs[i] : pv;  // fp8: the V scale of key c0 + 4 g + i rides on P
+        rs += pv;
+      }
+      rs = over_groups(rs, [](float x, float y) { return x + y; });
+      l = l * alpha + rs;
+      // O rows are heads 4 g + i: their factors live in lanes 4 g + i. Only rows < G are ever
+      // stored or merged (an O row depends on its own P row only), so G < 4 rescales G rows
 #pragma unroll
-    for (int i = 0; i < (G < 4 ? G : 4); ++i) {
-      const float al = G <= 4 ? row_lane(alpha, i) : __shfl(alpha, 4 * g + i, 64);
+      for (int i = 0; i < (G < 4 ? G : 4); ++i) {
+        const float al = G <= 4 ? row_lane(alpha, i) : __shfl(alpha, 4 * g + i, 64);
 #pragma unroll
-      for (int c = 0; c < DT; ++c) o[c][i] *= al;
-    }
-    // O += P·V: P (A operand) = the packed S^T accumulators, V (B operand) by transposed reads
-    const bf16x8 pa = pack_bf16x8(st, f32x4{0.f, 0.f, 0.f, 0.f});
-    const int qrow_ = lane >> 2 & 3, pcol = lane & 3;
+        for (int c = 0; c < DT; ++c) o[c][i] *= al;
+      }
+      // O += P·V: P (A operand) = the packed S^T accumulators, V (B operand) by transposed reads
+      const bf16x8 pa = pack_bf16x8(st, f32x4{0.f, 0.f, 0.f, 0.f});
+      const int qrow_ = lane >> 2 & 3, pcol = lane & 3;
 #pragma unroll
-    for (int c = 0; c < DT; ++c) {
-      const int key_a = 4 * g + qrow_, col = 16 * c + 4 * pcol;
-      const s16x4 lo = ds_tr16(vimg + v_off<D>(key_a, col >> 3) + ((col & 7) << 1));
-      const s16x4 hi = ds_tr16(vimg + v_off<D>(key_a + 16, col >> 3) + ((col & 7) << 1));
-      o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, cat_tr(lo, hi), o[c], 0, 0, 0);
-    }
-  };
+      for (int c = 0; c < DT; ++c) {
+        const int key_a = 4 * g + qrow_, col = 16 * c + 4 * pcol;
+        const s16x4 lo = ds_tr16(vimg + v_off<D>(key_a, col >> 3) + ((col & 7) << 1));
+        const s16x4 hi = ds_tr16(vimg + v_off<D>(key_a + 16, col >> 3) + ((col & 7) << 1));
+        o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, cat_tr(lo, hi), o[c], 0, 0, 0);
+      }
+    };
 
-  // three tiles in flight (all of a wave's tiles at up to 48 W keys: one memory round trip); a register
-  // set is refilled right after its tile is consumed, behind the end with the last key: a load under a
-  // condition would make the compiler wait for all of them at every join
-  for (int c0 = cfirst; c0 < len; c0 += 3 * cstep) {
-    consume(ta, c0);
-    load(ta, c0 + 3 * cstep);
+    // three tiles in flight (all of a wave's tiles at up to 48 W keys: one memory round trip); while a fourth
+    // follows, a register set is refilled right after its tile is consumed, behind the end with the last key:
+    // a load under a condition would make the compiler wait for all of them at every join
+    int c0 = cfirst;
+    if constexpr (!decltype(more)::value) {
+      if (c0 < len) consume(ta, c0);
+      return;
+    }
+    for (; c0 + 3 * cstep < len; c0 += 3 * cstep) {
+      consume(ta, c0);
+      load(ta, c0 + 3 * cstep);
+      consume(tb, c0 + cstep);
+      load(tb, c0 + 4 * cstep);
+      consume(tc, c0 + 2 * cstep);
+      load(tc, c0 + 5 * cstep);
+    }
+    if (c0 < len) consume(ta, c0);
     if (c0 + cstep < len) consume(tb, c0 + cstep);
-    load(tb, c0 + 4 * cstep);
     if (c0 + 2 * cstep < len) consume(tc, c0 + 2 * cstep);
-    load(tc, c0 + 5 * cstep);
+  };
+  if (W == 1 || cfirst + cstep < len) {
+    if constexpr (W > 1) load(tb, cfirst + cstep);
+    load(tc, cfirst + 2 * cstep);
+    __builtin_amdgcn_sched_barrier(0);
+    attend(std::true_type());
+  } else {
+    attend(std::false_type());
   }
   if constexpr (W == 1) {
     // ---- normalise and store: lane holds O[head 4 g + i][d = 16 c + r16] ----

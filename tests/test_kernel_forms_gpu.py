@@ -124,6 +124,31 @@ def test_decode_attention_waves_per_pair(B, Hq, Hkv, Smax, window):
     assert torch.equal(kc.nan_to_num(), k2.nan_to_num()) and torch.equal(vc.nan_to_num(), v2.nan_to_num())
 
 
+@pytest.mark.parametrize("B,Hkv,G,W", [(70, 8, 4, 1), (70, 16, 16, 1), (34, 8, 4, 4), (34, 8, 8, 4), (34, 8, 1, 4), (32, 4, 4, 8), (32, 2, 2, 8)])
+def test_decode_attention_of_one_to_seven_tiles_a_wave(B, Hkv, G, W):
+    """Rows that end in each of a wave's first seven tiles of 16 keys and around their edges, waves of no tile, of one, of three and
+    of a refilled fourth among them, with keys that begin anywhere; slots behind the new token hold NaN."""
+    D, Smax, scale = 128, 16 * 7 * W + 8 * W, 128 ** -0.5
+    g = torch.Generator(device=DEV).manual_seed(B * W + G)
+    ends = [max(1, 16 * W * j + e) for j in range(8) for e in (-1, 0, 1, 8 * W)]
+    n = torch.tensor((ends * 3)[:B], dtype=torch.int32, device=DEV)
+    start = torch.minimum(torch.randint(0, 9, (B,), generator=g, device=DEV, dtype=torch.int32), n - 1)
+    kc, vc = torch.randn(2, B, Hkv, Smax, D, generator=g, device=DEV).bfloat16()
+    tail = torch.arange(Smax, device=DEV)[None, None, :, None] >= (n - 1).long()[:, None, None, None]
+    kc.masked_fill_(tail, float("nan"))
+    vc.masked_fill_(tail, float("nan"))
+    qkv = torch.randn(B, (G + 2) * Hkv * D, generator=g, device=DEV).bfloat16()
+    out = ops.decode_step_attention(qkv, kc, vc, n - 1, n, G * Hkv, kv_start=start).view(B, Hkv, G, D).double()
+    for b in range(B):
+        lo, hi = int(start[b]), int(n[b])
+        k, v = kc[b, :, lo:hi].double(), vc[b, :, lo:hi].double()
+        assert torch.equal(k[:, -1].flatten(), qkv[b, G * Hkv * D:(G + 1) * Hkv * D].double())
+        p = torch.softmax((qkv[b, :G * Hkv * D].view(Hkv, G, 1, D).double() * k[:, None]).sum(-1) * scale, -1)[..., None]
+        want, size = ((p * x[:, None]).sum(2) for x in (v, v.abs()))
+        # p and the result round to bf16 (half an ulp: 2^-8 each)
+        assert ((out[b] - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, (b, lo, hi)
+
+
 @pytest.mark.parametrize("B,Hkv,G", [(13, 40, 1), (33, 16, 2), (65, 8, 4), (65, 8, 8)])
 def test_decode_attention_form_whatever_the_free_slots(B, Hkv, G):
     """Beyond 512 (row, kv head) pairs short rows cost no more in a cache of many slots: the same form, so the same bits."""
