@@ -750,7 +750,6 @@ struct DecodeFusedArgs {
   // optional: qkv as nsplit fp32 split-K slabs [nsplit][B][ldq] (the qkv GEMM's reduce fused into
   // the MFMA kernel's prologue); qkv above is then unused
   const float* qkv_slabs; int qkv_nsplit; long qkv_sstride;
-  int kv_nt;                        // non-temporal K/V cache loads (each read once per step)
   long long* stamps;                // debug (W > 1 kernel): [blocks * W][8] s_memrealtime phase stamps, or null
   // fp8 K/V cache (config 5, MFMA kernels only): kc / vc hold OCP e4m3fn bytes, one fp32 scale per
   // (batch, kv head, slot) in ksc / vsc [B, Hkv, SmaxP]; K rows are stored k-permuted (element
@@ -791,7 +790,8 @@ __device__ __forceinline__ void rope_chunk(const bf16_t* head, int dl, const Dec
 }
 
 // One key chunk: CH = 4 waves x KPW keys x NK keys per lane. Loads of chunk j+1 are issued before
-// chunk j is consumed (two named register sets), softmax is online across chunks.
+// chunk j is consumed (two named register sets), softmax is online across chunks. Cache bytes are read
+// once a step: non-temporal.
 template <int D, int NK>
 struct KVChunk {
   uint4 k[NK], v[NK];
@@ -799,22 +799,13 @@ struct KVChunk {
 
 template <int D, int NK>
 __device__ __forceinline__ void load_chunk(KVChunk<D, NK>& c, const bf16_t* kbase, const bf16_t* vbase, int c0,
-                                           int p1, int wid, int sub, int dl, bool nt) {
+                                           int p1, int wid, int sub, int dl) {
   constexpr int KPW = 64 / (D / 8);
-  if (nt) {
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int key = min(c0 + (i * 4 + wid) * KPW + sub, p1 - 1);
-      c.k[i] = load_nt16(kbase + (long)key * D + dl * 8);
-      c.v[i] = load_nt16(vbase + (long)key * D + dl * 8);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int key = min(c0 + (i * 4 + wid) * KPW + sub, p1 - 1);
-      c.k[i] = *(const uint4*)(kbase + (long)key * D + dl * 8);
-      c.v[i] = *(const uint4*)(vbase + (long)key * D + dl * 8);
-    }
+  for (int i = 0; i < NK; ++i) {
+    const int key = min(c0 + (i * 4 + wid) * KPW + sub, p1 - 1);
+    c.k[i] = load_nt16(kbase + (long)key * D + dl * 8);
+    c.v[i] = load_nt16(vbase + (long)key * D + dl * 8);
   }
 }
 
@@ -904,10 +895,10 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(DecodeFusedArgs 
     const bf16_t* kbase = a.kc + ((long)b * a.Hkv + hk) * a.Smax * D;
     const bf16_t* vbase = a.vc + ((long)b * a.Hkv + hk) * a.Smax * D;
     KVChunk<D, NK> ca, cb;
-    load_chunk<D, NK>(ca, kbase, vbase, p0, p1, wid, sub, dl, a.kv_nt);
+    load_chunk<D, NK>(ca, kbase, vbase, p0, p1, wid, sub, dl);
     // the second chunk is issued with the first, before q (waiting for q drains both): a
     // partition of <= 2 chunks (the batch-1 partition plan) costs one memory round trip, not two
-    if (p0 + CH < p1) load_chunk<D, NK>(cb, kbase, vbase, p0 + CH, p1, wid, sub, dl, a.kv_nt);
+    if (p0 + CH < p1) load_chunk<D, NK>(cb, kbase, vbase, p0 + CH, p1, wid, sub, dl);
     float qv[G][8];
 #pragma unroll
     for (int gg = 0; gg < G; ++gg) rope_chunk<D>(row + (long)(hk * G + gg) * D, dl, a, p, qv[gg]);
@@ -933,10 +924,10 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(DecodeFusedArgs 
       for (int e = 0; e < 8; ++e) acc[gg][e] = 0.f;
     }
     for (int c0 = p0; c0 < p1; c0 += 2 * CH) {
-      if (c0 != p0 && c0 + CH < p1) load_chunk<D, NK>(cb, kbase, vbase, c0 + CH, p1, wid, sub, dl, a.kv_nt);
+      if (c0 != p0 && c0 + CH < p1) load_chunk<D, NK>(cb, kbase, vbase, c0 + CH, p1, wid, sub, dl);
       consume_chunk<D, G, NK>(ca, c0, p1, s_new, has_new, kp, vp, qv, m, l, acc, wid, sub, a.scale_log2);
       if (c0 + CH < p1) {
-        if (c0 + 2 * CH < p1) load_chunk<D, NK>(ca, kbase, vbase, c0 + 2 * CH, p1, wid, sub, dl, a.kv_nt);
+        if (c0 + 2 * CH < p1) load_chunk<D, NK>(ca, kbase, vbase, c0 + 2 * CH, p1, wid, sub, dl);
         consume_chunk<D, G, NK>(cb, c0 + CH, p1, s_new, has_new, kp, vp, qv, m, l, acc, wid, sub, a.scale_log2);
       }
     }
@@ -1388,7 +1379,9 @@ __global__ __launch_bounds__(64 * W, 2) void attn_decode_mfma_kernel(DecodeFused
         T.vs[i] = vsb[key];
       }
     } else {
-      // K plainly: both 64-B halves of a line are read, by two of these
+      // V, whole rows a load, is read once: non-temporal. K plainly: a load takes 64 B of each row, and the line's other
+      // half is the next one's. us, K plainly / non-temporal: 16 rows of 150..300 keys, 8 key heads 9.4 / 10.3, 48 of 300..600
+      // 24.2 / 25.0, 256 of 150..300 45.1 / 46.3 (96, one wave, 21.6 / 21.1)
 #pragma unroll
       for (int s2 = 0; s2 < DS; ++s2) T.k[s2] = *(const uint4*)(kbase + keyk * D + 32 * s2 + 8 * g);
 #pragma unroll
@@ -2381,9 +2374,6 @@ extern "C" int rt_attn_decode_fused(const void* qkv, long ldq, void* kc, void* v
   a.sign = sign; a.window = window; a.part = part; a.tickets = tickets; a.o = (bf16_t*)o; a.ldo = ldo;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.NP = NP; a.PS = PS; a.scale_log2 = scale * 1.4426950408889634f;
   a.qkv_slabs = qkv_slabs; a.qkv_nsplit = qkv_slabs ? qkv_nsplit : 0; a.qkv_sstride = (long)B * ldq;
-  // K/V cache bytes are read once per decode step: non-temporal loads (batch 256: 56 -> 50 us per
-  // layer, profiles/decode_nt_ab.log)
-  a.kv_nt = 1;
   a.stamps = stamps;
   a.ksc = ksc; a.vsc = vsc; a.SmaxP = ksc ? SmaxP : 0;
   const bool kv8 = ksc != nullptr;
