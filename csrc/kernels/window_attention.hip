@@ -811,9 +811,14 @@ extern "C" int rt_window_prep(int f32, void* proj, long ldp, int q_col, int k_co
              pool, tab, max_pages, n_pages, n_rows, H, G, D, V};
   const bool vec = !f32 && D % 8 == 0 && V % 8 == 0 && half % 8 == 0 && ldp % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 &&
                    v_col % 8 == 0 && ((uintptr_t)proj | (uintptr_t)pool | (uintptr_t)q_norm | (uintptr_t)k_norm) % 16 == 0;
-  const long leads = (long)H * ((D - half) / 8);  // a lead or two a thread; tables in 16-byte loads
-  const bool once = half >= 8 && G > 0 && leads <= 512 && (long)G * ((D - half) / 8) <= 256 && (long)G * V <= 2048 && n_rows > 0 &&
-                    max_pages > 0 && ((uintptr_t)cosT | (uintptr_t)sinT) % 16 == 0;
+  const long leads = (long)H * ((D - half) / 8), k_leads = (long)G * ((D - half) / 8);  // a lead or two a thread; tables in 16-byte loads
+  // Where tokens fill the chip several times over a workgroup's idle threads count, and a token of few heads leaves most idle. us,
+  // loops / registers: 4 heads and 2 key heads of 64, 700 / 2000 / 8000 tokens 5.7 / 7.4 / 17.4 and 5.2 / 8.5 / 24.0, without norms 4.3 /
+  // 5.6 / 11.6 and 4.3 / 6.9 / 19.4; 16 and 4 of 128 (224 items), 8000 tokens 27.9 and 26.9, without norms, where the loops read a
+  // row once, 19.9 and 21.5; 20 and 4 (256) 22.9 and 23.2, 24 and 8 37.7 and 33.5
+  const bool fills = T <= 768 || leads + k_leads + (long)G * V / 8 >= (q_norm || k_norm ? 224 : 256);
+  const bool once = half >= 8 && G > 0 && leads <= 512 && k_leads <= 256 && (long)G * V <= 2048 && n_rows > 0 && max_pages > 0 &&
+                    ((uintptr_t)cosT | (uintptr_t)sinT) % 16 == 0 && fills;
   if (f32) hipLaunchKernelGGL((window_prep_kernel<float, 1>), dim3(T), dim3(256), 0, stream, a);
   else if (vec && once) {
     if (leads <= 256) hipLaunchKernelGGL(window_prep_once_kernel<1>, dim3(T), dim3(256), 0, stream, a);

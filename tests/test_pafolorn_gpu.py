@@ -308,6 +308,31 @@ def test_window_prep_in_registers(H, G, D, V, half, norms):
         assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 4e-6).all()
 
 
+@pytest.mark.parametrize("norms", [True, False])
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 64, 64), (16, 4, 128, 128), (20, 4, 128, 128)])
+def test_window_prep_of_many_tokens(H, G, D, V, norms):
+    """The form that a call of 769 tokens takes against that of its parts of 768 and 1: the same up to the order of the norms' sums."""
+    T, half, most = 769, D // 2, 1024
+    g = torch.Generator(device=DEV).manual_seed(H)
+    d = ops.WindowDims(H, G, D, V, 1.0, 0.0, 0, 0)
+    proj = torch.randn(T, d.in_cols, generator=g, device=DEV).bfloat16()
+    qn, kn = (torch.rand(n * D, generator=g, device=DEV).bfloat16() if norms else None for n in (H, G))
+    cos, sin = (torch.randn(most, half, generator=g, device=DEV) for _ in range(2))
+    tab = torch.arange(32, dtype=torch.int32, device=DEV).flip(0).view(2, 16).contiguous()
+    tok = torch.arange(T, device=DEV)
+    row, pos = (tok % 2).int(), (tok // 2).int()
+    dims, fs = d.args()
+    got = []
+    for cuts in ((0, T), (0, 768, T)):
+        pool = torch.full((32, 64, G * (D + V)), 0.25, dtype=torch.bfloat16, device=DEV)
+        p = proj.clone()
+        for a, b in zip(cuts, cuts[1:]):
+            ops.native().window_prep(p[a:b], 0, qn, kn, 1e-6, cos, sin, row[a:b], pos[a:b], pool, tab, dims, fs)
+        got.append((p.float(), pool.float()))
+    for a, b in zip(*got):
+        assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 4e-6).all()  # as above
+
+
 @pytest.mark.parametrize("window,keep", [(0, 0), (5000, 100)])
 @pytest.mark.parametrize("D,V", [(8, 16), (136, 8)])
 def test_window_decode_of_many_pages(D, V, window, keep):
