@@ -41,7 +41,7 @@ int rt_window_prep(int, void*, long, int, int, int, const void*, const void*, fl
 int rt_window_decode_ok(int, int, int, int);
 int rt_window_decode(const void*, long, const void*, const int*, int, int, int, const int*, const int*, float*, float*, void*, long,
                      float, int, int, int, int, int, int, int, int, float, float, hipStream_t);
-int rt_window_decode_parts(int, int, int);
+int rt_window_decode_parts(int, int, int, int, int);
 int rt_window_prefill_ok(int, int);
 int rt_window_prefill(const void*, long, const void*, const int*, int, int, int, void*, long, const void*, const void*, int,
                       int, int, int, int, int, int, float, float, float, hipStream_t);
@@ -525,7 +525,7 @@ void window_decode(const Tensor& q, const Tensor& pool, const Tensor& tab, const
   TORCH_CHECK(pool.scalar_type() == at::kBFloat16 && q.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16 &&
                   q.is_cuda() && out.is_cuda() && q.size(1) == (int64_t)w.H * w.D && out.size(0) == T &&
                   out.size(1) == (int64_t)w.H * w.V && NP >= 1 && NP <= 1024 && al16(q), "window_decode: shapes");
-  const int np = rt_window_decode_parts((int)T, w.G, (int)NP);
+  const int np = rt_window_decode_parts((int)T, w.H, w.G, w.V, (int)NP);
   Tensor part, ml;
   if (np > 1) {
     part = at::empty({T, w.H, np, w.V}, q.options().dtype(at::kFloat));

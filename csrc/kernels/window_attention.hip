@@ -296,8 +296,10 @@ static CapScore make_cap_score(float scale, float cap) {
 // the waves' (m, l, O) meet in LDS. With a tile of 32 keys shared by the four waves every wave ran the same softmax
 // (H / G of 16 lanes of it needed: 38 of 46 us were its VALU work), with three barriers a tile; and a page's number, loaded
 // for each tile, waited for all LDS-DMA under way (loads return in order): the pages of 64 tiles now come at once.
-// us, before -> this (each at its partitions): 64 rows of 300..1100 keys 50.2 -> 43.5 and no merge, 16 22.6 -> 15.5, 4 of 3000..4000 30 -> 17,
+// us, 4 query heads a key head, 128 + 128 columns, before -> this (each at its partitions): 64 rows of 300..1100 keys 50.2 -> 43.5 and no merge, 16 22.6 -> 15.5, 4 of 3000..4000 30 -> 17,
 // 200 of 100..600 81.5 -> 70.8, 256 of 60..120 38.8 -> 34.1. 2 or 1 waves a workgroup, more of these on a CU: 44.9 / 52.5, 74.0 / 76.0, 32.6 / 33.3.
+// 16 heads of 256 + 256 columns, where every wave reads all of q for itself, are the form's worst: 1 row of 300 keys 9.9 -> 10.3, of
+// 4000 keys 17.8 -> 18.2, but 64 of 300..1100 33.9 -> 30.2 and 200 of 100..600 54 -> 41.
 // A token's visible tiles are cut in NP equal partitions, so a captured launch with a fixed NP balances every
 // length; of one partition the workgroup writes the result. Chunk c of image row r lies in slot c ^ r, or rows are an odd number of 16-B chunks (conflict-free either way).
 struct DecArgs {
@@ -306,7 +308,7 @@ struct DecArgs {
   const int* row; const int* pos;
   float* part; float* ml;     // [T, H, NP, V], [T, H, NP, 2] (max in log2 units, sum)
   bf16_t* out; long ldo; float out_scale;  // of one partition: the result itself, as partition_merge makes it (else null)
-  int H, G, D, V, NP;
+  int H, G, D, V, NP, S;      // S: workgroups that share a key head's query heads
   Mask mask;
   Score score;
 };
@@ -319,15 +321,15 @@ __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
   constexpr int CPR = SWZ ? CH : CH + 1, ROWB = CPR * 16;
   constexpr int NIT = (16 * CPR + 63) / 64, BUFB = NIT * 1024;  // LDS-DMA instructions of a tile (the last one may be part used)
   constexpr int QF = 2 * QS, LDP = 64 * RT + 4;
-  constexpr int RING = NW * 2 * BUFB;                 // two images a wave; at the end 16 heads' O of each
-  static_assert(NW * 16 * LDP * 4 <= RING, "the merge fits the images");
-  __shared__ __attribute__((aligned(16))) char smem[RING + NW * NH * 16 * 8 + 64];
+  constexpr int RING = NW * 2 * BUFB;                 // two images a wave; at the end 16 heads' O in their place
+  static_assert(16 * LDP * 4 <= 2 * BUFB, "a wave's sums fit its images");
+  __shared__ __attribute__((aligned(16))) char smem[RING + NW * NH * 16 * 8];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int part = bid % a.NP, gh = bid / a.NP % a.G, t = bid / (a.NP * a.G);
-  const int HG = a.H / a.G, h0 = gh * HG;            // query heads h0 .. h0 + HG - 1
+  const int sub = bid % a.S, part = bid / a.S % a.NP, gh = bid / (a.S * a.NP) % a.G, t = bid / (a.S * a.NP * a.G);
+  const int h0 = gh * (a.H / a.G) + 16 * NH * sub, HG = min(a.H / a.G - 16 * NH * sub, 16 * NH);  // query heads h0 .. h0 + HG - 1
   int row = a.row[t], pos = a.pos[t];
   asm volatile("" : "+s"(row), "+s"(pos));           // in one trip, also if the partition is empty
   row = min(max(row, 0), a.n_rows - 1);
@@ -459,46 +461,49 @@ __global__ __launch_bounds__(256, 2) void window_decode_kernel(DecArgs a) {
     }
     if (j + 2 < n) stage(j + 2);  // this image has been read
   }
-  // ---- the waves' sums: o[u][c][e] is head h0 + 16 u + r16, value column 16 c + 4 g + e ----
+  // ---- the waves' sums: o[u][c][e] is head h0 + 16 u + r16, value column 16 c + 4 g + e. A wave's go where its own images were,
+  // so the waves meet once a head tile, and whoever adds them up weighs them ----
   float2* const mls = (float2*)(smem + RING);        // [wave][head]
   if (g == 0)
 #pragma unroll
     for (int u = 0; u < NH; ++u) mls[w * 16 * NH + 16 * u + r16] = make_float2(m[u], l[u]);
-  __syncthreads();
-  float* const os = (float*)smem;                    // [wave][16 heads][LDP]
-  float* const invs = (float*)(smem + RING + NW * NH * 16 * 8);  // [16 heads]
+  constexpr int OS = 2 * BUFB / 4;                   // floats from wave to wave
 #pragma unroll
   for (int u = 0; u < NH; ++u) {
-    float M = -INFINITY, L = 0.f;                    // finite: wave 0 has a tile
-#pragma unroll
-    for (int k = 0; k < NW; ++k) M = fmaxf(M, mls[k * 16 * NH + 16 * u + r16].x);
-#pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      const float2 x = mls[k * 16 * NH + 16 * u + r16];
-      L += x.y * fexp2(x.x - M);
-    }
-    const float f = fexp2(m[u] - M);                 // 0 for a wave without tiles
     if (u > 0) __syncthreads();
     if (16 * u + r16 < HG) {
 #pragma unroll
-      for (int c = 0; c < 4 * RT; ++c) *(f32x4*)(os + (w * 16 + r16) * LDP + 16 * c + 4 * g) = o[u][c] * f;
-    }
-    if (w == 0 && g == 0 && 16 * u + r16 < HG) {
-      if (a.out) invs[r16] = a.out_scale / L;
-      else *(float2*)(a.ml + (((long)t * a.H + h0 + 16 * u + r16) * a.NP + part) * 2) = make_float2(M, L);
+      for (int c = 0; c < 4 * RT; ++c) *(f32x4*)((float*)mine + r16 * LDP + 16 * c + 4 * g) = o[u][c];
     }
     __syncthreads();
     const int hn = min(HG - 16 * u, 16), V4 = a.V / 4;  // V % 8 == 0
     for (int e = tid; e < hn * V4; e += 64 * NW) {
       const int h = e / V4, c = e % V4 * 4;
-      f32x4 y = *(const f32x4*)(os + h * LDP + c);
+      const long th = (long)t * a.H + h0 + 16 * u + h;
+      float2 ml[NW];
+      f32x4 x[NW];
 #pragma unroll
-      for (int k = 1; k < NW; ++k) y += *(const f32x4*)(os + (k * 16 + h) * LDP + c);
+      for (int k = 0; k < NW; ++k) {
+        ml[k] = mls[k * 16 * NH + 16 * u + h];
+        x[k] = *(const f32x4*)((float*)smem + k * OS + h * LDP + c);
+      }
+      float M = ml[0].x, L = 0.f;                    // finite: wave 0 has a tile
+#pragma unroll
+      for (int k = 1; k < NW; ++k) M = fmaxf(M, ml[k].x);
+      f32x4 y;
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+#pragma clang fp contract(off)
+        const float f = fexp2(ml[k].x - M);          // 0 for a wave without tiles
+        L = fmaf(ml[k].y, f, L);
+        y = k == 0 ? x[0] * f : y + x[k] * f;
+      }
       if (a.out) {
-        y *= invs[h];
+        y *= a.out_scale / L;
         *(uint2*)(a.out + (long)t * a.ldo + (long)(h0 + 16 * u + h) * a.V + c) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
       } else {
-        *(f32x4*)(a.part + (((long)t * a.H + h0 + 16 * u + h) * a.NP + part) * a.V + c) = y;
+        *(f32x4*)(a.part + (th * a.NP + part) * a.V + c) = y;
+        if (c == 0) *(float2*)(a.ml + (th * a.NP + part) * 2) = make_float2(M, L);
       }
     }
   }
@@ -833,12 +838,19 @@ extern "C" int rt_window_decode_ok(int H, int G, int D, int V) {
   return G > 0 && H % G == 0 && H / G <= 32 && D % 8 == 0 && V % 8 == 0 && D >= 8 && V >= 8 && D <= 256 && V <= 256;
 }
 
+// Workgroups that share the query heads of a key head: one, but one per 16 heads where there are more and more than 128 value
+// columns. With two tiles of heads over 256 columns a wave's sums take 256 registers, and the four waves' merge was the longer
+// part of a short row: us, a workgroup of 32 heads -> two of 16, 128 + 256 columns, 1 row of 300 keys 12.9 -> 10.1, 16 of 300..1100 17.8 ->
+// 14.5, 200 of 100..600 43.2 -> 31.1 (of 4 key heads of 64 + 256, where keys and values are the time, 68 -> 76; before the waves
+// had tiles of their own 89)
+static int head_groups(int H, int G, int V) { return V > 128 ? (H / G + 15) / 16 : 1; }
+
 // Partitions of a token's tiles that a decode takes of the NP it may: a workgroup per CU. us (without the merge), 8 key heads of
 // 128, at 1 / 2 / 4 / 8 partitions: 4 rows of 3000..4000 keys 45 / 27 / 19 / 17, 16 of 300..1100 18.8 / 15.5 / 15.6 / 17.6, 32 24.5 / 26.1 /
 // 25.3 / 29.1, 64 43.5 / 44.2 / 44.0 / 50.0, 128 of 100..600 47.2 / 47.8 / 52.6 / 69.3, 256 of 60..120 34 / 42 / 63 / 106; and one needs
 // no merge (5 us).
-extern "C" int rt_window_decode_parts(int T, int G, int NP) {
-  const long groups = std::max(1L, (long)T * G);
+extern "C" int rt_window_decode_parts(int T, int H, int G, int V, int NP) {
+  const long groups = std::max(1L, (long)T * G * head_groups(H, G, V));
   return (int)std::min((long)NP, (256 + groups - 1) / groups);
 }
 
@@ -851,14 +863,11 @@ extern "C" int rt_window_decode(const void* q, long ldq, const void* pool, const
   if (!rt_window_decode_ok(H, G, D, V) || NP < 1 || ldq % 8) return -1;
   if (NP == 1 && (ldo % 4 || (uintptr_t)out % 8)) return -1;
   DecArgs a{(const bf16_t*)q, ldq, (const bf16_t*)pool, tab, max_pages, n_pages, n_rows, row, pos, part, ml,
-            NP == 1 ? (bf16_t*)out : nullptr, ldo, out_scale, H, G, D, V, NP, make_mask(size, keep), make_score(scale, cap)};
-  dim3 grid((unsigned)((long)T * G * NP)), block(256);
-#define WD_(QS, RT)                                                                                        \
-  do {                                                                                                     \
-    if (H / G <= 16) hipLaunchKernelGGL((window_decode_kernel<QS, RT, 1>), grid, block, 0, stream, a);     \
-    else hipLaunchKernelGGL((window_decode_kernel<QS, RT, 2>), grid, block, 0, stream, a);                 \
-  } while (0)
-#define WD_V(QS) do { if (V <= 128) WD_(QS, 2); else WD_(QS, 4); } while (0)
+            NP == 1 ? (bf16_t*)out : nullptr, ldo, out_scale, H, G, D, V, NP, head_groups(H, G, V), make_mask(size, keep),
+            make_score(scale, cap)};
+  dim3 grid((unsigned)((long)T * G * NP * a.S)), block(256);
+#define WD_(QS, RT, NH) hipLaunchKernelGGL((window_decode_kernel<QS, RT, NH>), grid, block, 0, stream, a)
+#define WD_V(QS) do { if (V > 128) WD_(QS, 4, 1); else if (H / G > 16) WD_(QS, 2, 2); else WD_(QS, 2, 1); } while (0)
   if (D <= 64) WD_V(1);
   else if (D <= 128) WD_V(2);
   else if (D <= 192) WD_V(3);

@@ -308,6 +308,32 @@ def test_window_prep_in_registers(H, G, D, V, half, norms):
         assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 4e-6).all()
 
 
+@pytest.mark.parametrize("T", [3, 140])
+@pytest.mark.parametrize("H,G,D,V", [(16, 1, 64, 136), (17, 1, 8, 136), (64, 2, 136, 256), (96, 4, 256, 256), (62, 2, 64, 128)])
+def test_window_decode_of_many_query_heads(T, H, G, D, V):
+    """key heads of 16 to 32 query heads: one workgroup for all of them or, of wide values, one per 16; rows of 1 to 300 keys"""
+    d = ops.WindowDims(H, G, D, V, D ** -0.5, 0.0, 0, 0)
+    g = torch.Generator(device=DEV).manual_seed(H + V)
+    n = torch.randint(1, 301, (T,), generator=g, device=DEV, dtype=torch.int32)
+    n[:3] = torch.tensor([1, 300, 65], device=DEV)
+    pages = (300 + 63) // 64
+    pool = torch.randn(T * pages, 64, d.cache_width, generator=g, device=DEV).bfloat16()
+    tab = torch.randperm(T * pages, generator=g, device=DEV).int().view(T, pages)
+    q = torch.randn(T, H * D, generator=g, device=DEV).bfloat16()
+    dims, fs = d.args()
+    for parts in (1, 5):
+        out = torch.zeros(T, H * V, dtype=torch.bfloat16, device=DEV)
+        ops.native().window_decode(q, pool, tab, torch.arange(T, dtype=torch.int32, device=DEV), n - 1, out, parts, 0.5, dims, fs)
+        for b in range(0, T, 1 if T < 9 else 13):
+            k = int(n[b])
+            kv = pool.view(-1, G, 64, D + V)[tab[b].long()].transpose(1, 2).flatten(0, 1)[:k].double().transpose(0, 1)  # [G, k, D + V]
+            qb = q[b].view(G, H // G, D).double()
+            p = torch.softmax(torch.matmul(qb, kv[..., :D].transpose(1, 2).contiguous()) * d.scale, -1)
+            want, size = (0.5 * torch.matmul(p, v.contiguous()).flatten() for v in (kv[..., D:], kv[..., D:].abs()))
+            # p and the result round to bf16 (half an ulp: 2^-8 each)
+            assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, (parts, b)
+
+
 @pytest.mark.parametrize("norms", [True, False])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 64, 64), (16, 4, 128, 128), (20, 4, 128, 128)])
 def test_window_prep_of_many_tokens(H, G, D, V, norms):
