@@ -661,6 +661,8 @@ void bind_layered(py::module_& m) {
   m.def("window_prep", &window_prep, "q / k norm, rotation in halves, cache append");
   m.def("window_decode_ok", [](int H, int G, int D, int V) { return rt_window_decode_ok(H, G, D, V) != 0; });
   m.def("window_prefill_ok", [](int D, int V) { return rt_window_prefill_ok(D, V) != 0; });
+  m.def("window_decode_parts", [](int T, int H, int G, int V, int NP) { return rt_window_decode_parts(T, H, G, V, NP); },
+        "partitions that window_decode takes of the NP it may");
   m.def("window_decode", &window_decode, "windowed attention, few tokens per request");
   m.def("window_prefill", &window_prefill, "windowed flash attention of prompt portions from the pages");
   m.def("window_any", &window_any, "windowed attention, any size / type");

@@ -34,6 +34,17 @@
 
 namespace rt {
 
+// CUs of the device, a property computed once (thread-safe static initialisation)
+inline int num_cus() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      cus = 256;
+    return cus;
+  }();
+  return n;
+}
+
 typedef uint16_t bf16_t;  // raw bf16 bits; storage type for every bf16 tensor
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;   // MFMA A/B fragment

@@ -1397,18 +1397,6 @@ static bool bn128_supported(int layout_a, int layout_b, int act, int out) {
          (act == E_NONE && (key == 1 || key == 3 || key == 10 || key == 13)) || (key == 10 && act == E_DSWIGLU);
 }
 
-static int query_num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  return n;
-}
-// a device property, computed once (thread-safe static initialisation)
-static int num_cus() {
-  static const int n = query_num_cus();
-  return n;
-}
-
 // Ratio of a 256x128 tile's time to a 256x256 tile's (same K), for the wave planner below. With a K-contiguous A and a
 // column-contiguous B (NN) it is larger, 74 us to 120 at K = 4096: the transposed reads of B wait inside each phase. 4016 x 14336 x
 // 4096, which 0.55 put on seven rounds of 128 columns: 468 us, 391 on 256; with the SwiGLU backward 535, so 467.

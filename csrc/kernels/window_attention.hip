@@ -848,10 +848,13 @@ static int head_groups(int H, int G, int V) { return V > 128 ? (H / G + 15) / 16
 // Partitions of a token's tiles that a decode takes of the NP it may: a workgroup per CU. us (without the merge), 8 key heads of
 // 128, at 1 / 2 / 4 / 8 partitions: 4 rows of 3000..4000 keys 45 / 27 / 19 / 17, 16 of 300..1100 18.8 / 15.5 / 15.6 / 17.6, 32 24.5 / 26.1 /
 // 25.3 / 29.1, 64 43.5 / 44.2 / 44.0 / 50.0, 128 of 100..600 47.2 / 47.8 / 52.6 / 69.3, 256 of 60..120 34 / 42 / 63 / 106; and one needs
-// no merge (5 us).
+// no merge (5 us). The lengths are not known here, only the longest that the cache may hold, which is mostly far beyond them. A
+// long row among many short ones is then the time of one workgroup's tiles: 32 rows, one of 4000 keys and 31 of 50..150 41.9 at one
+// partition (the tiles of 32 keys shared by the waves took 47.1 with the merge, at four); 64 rows, one of 8000, 83 (93); 16 rows, one
+// of 4000, at two partitions 28 (47).
 extern "C" int rt_window_decode_parts(int T, int H, int G, int V, int NP) {
-  const long groups = std::max(1L, (long)T * G * head_groups(H, G, V));
-  return (int)std::min((long)NP, (256 + groups - 1) / groups);
+  const long groups = std::max(1L, (long)T * G * head_groups(H, G, V)), cus = num_cus();
+  return (int)std::min((long)NP, (cus + groups - 1) / groups);
 }
 
 // NP of one partition: to out (ldo % 4 == 0, 8-byte aligned), part and ml unused; of more: to part and ml, for partition_merge

@@ -49,9 +49,8 @@ class WindowDims:
 
 
 def _np_parts(T: int, d: WindowDims, max_len: int) -> int:
-    """Partitions that a token's visible tiles may be cut in, at least 64 keys each: two workgroups per CU, and four of a token
-    and key head all the same up to 4096 workgroups. The kernel takes as many of them as give every CU a workgroup
-    (rt_window_decode_parts)."""
+    """Partitions that a token's visible tiles may be cut in: the most that could help, of at least 64 keys each. What is launched
+    is decided beside the kernel (window_decode_parts: a workgroup per CU)."""
     keys = max_len if not d.window else min(max_len, d.window + d.keep + 64)
     groups = T * d.kv_heads
     return max(1, min(max((512 + groups - 1) // groups, min(4, 4096 // groups)), (keys + 63) // 64, 512))

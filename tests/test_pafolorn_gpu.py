@@ -308,6 +308,35 @@ def test_window_prep_in_registers(H, G, D, V, half, norms):
         assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 4e-6).all()
 
 
+@pytest.mark.parametrize("T,H,G,V,parts", [(1, 4, 1, 64, 7), (3, 32, 2, 64, 7), (8, 8, 8, 8, 4), (16, 72, 4, 64, 4), (40, 8, 2, 64, 4),
+                                           (127, 2, 1, 128, 3), (128, 2, 1, 128, 2), (255, 1, 1, 64, 2), (256, 1, 1, 64, 1),
+                                           (16, 64, 2, 256, 4)])
+def test_window_decode_launched_partitions(T, H, G, V, parts):
+    """The partitions that are launched, one to seven, and their merge: rows of 1 to 400 keys, most with empty partitions."""
+    D, most = 64, 400
+    d = ops.WindowDims(H, G, D, V, D ** -0.5, 0.0, 0, 0)
+    NP = ops.window._np_parts(T, d, most)
+    assert ops.native().window_decode_parts(T, H, G, V, NP) == parts
+    g = torch.Generator(device=DEV).manual_seed(T)
+    n = torch.randint(1, most + 1, (T,), generator=g, device=DEV, dtype=torch.int32)
+    n[0] = most
+    n[1::2] = torch.randint(1, 40, n[1::2].shape, generator=g, device=DEV, dtype=torch.int32)
+    pages = (most + 63) // 64
+    pool = torch.randn(T * pages, 64, d.cache_width, generator=g, device=DEV).bfloat16()
+    tab = torch.randperm(T * pages, generator=g, device=DEV).int().view(T, pages)
+    q = torch.randn(T, H * D, generator=g, device=DEV).bfloat16()
+    out = torch.zeros(T, H * V, dtype=torch.bfloat16, device=DEV)
+    dims, fs = d.args()
+    ops.native().window_decode(q, pool, tab, torch.arange(T, dtype=torch.int32, device=DEV), n - 1, out, NP, 1.0, dims, fs)
+    for b in range(T):
+        k = int(n[b])
+        kv = pool.view(-1, G, 64, D + V)[tab[b].long()].transpose(1, 2).flatten(0, 1)[:k].double().transpose(0, 1)  # [G, k, D + V]
+        p = torch.softmax(torch.matmul(q[b].view(G, H // G, D).double(), kv[..., :D].transpose(1, 2).contiguous()) * d.scale, -1)
+        want, size = (torch.matmul(p, v.contiguous()).flatten() for v in (kv[..., D:], kv[..., D:].abs()))
+        # p and the result round to bf16 (half an ulp: 2^-8 each)
+        assert ((out[b].double() - want).abs() - (2.0 ** -7 + 2.0 ** -11) * size).max() < 1e-6, b
+
+
 @pytest.mark.parametrize("T", [3, 140])
 @pytest.mark.parametrize("H,G,D,V", [(16, 1, 64, 136), (17, 1, 8, 136), (64, 2, 136, 256), (96, 4, 256, 256), (62, 2, 64, 128)])
 def test_window_decode_of_many_query_heads(T, H, G, D, V):
