@@ -66,7 +66,7 @@ int rt_attn_packed(const void*, long, const void*, long, const void*, long, void
 int rt_few_rows(const void*, long, const void*, long, const void*, const void*, void*, const void*, long, const void*, void*, long,
                 int, int, int, int, float, int, int, hipStream_t);
 int rt_gemm_nt_parts(int, int, int, int*);
-int rt_gemm_plan(int, int, int, int, int*);
+int rt_gemm_plan(int, int, int, int, int, int*);
 int rt_token_plan(int, int, int, int, int*);
 int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
@@ -1664,11 +1664,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   }, "parts of the K-steps and columns of a tile of an NN product");
   m.def("small_tiles", [](int64_t M, int64_t N, int64_t K, int64_t act) { return rt_small_tiles((int)M, (int)N, (int)K, (int)act) != 0; },
         "whether a product with a bias takes 64 x 64 tiles that sum the parts of K");
-  m.def("gemm_plan", [](int64_t M, int64_t N, int64_t K, int64_t act) {
+  m.def("gemm_plan", [](int64_t M, int64_t N, int64_t K, int64_t act, int64_t layout_b) {
     int form = 0;
-    const int rows = rt_gemm_plan((int)M, (int)N, (int)K, (int)act, &form);
+    const int rows = rt_gemm_plan((int)M, (int)N, (int)K, (int)act, (int)layout_b, &form);
     return std::make_pair(rows, form);
-  }, "rows of a plain NT product on 256 x 256 tiles (-1: two workgroups per CU) and the tiles of the rest");
+  }, "rows of a plain NT or an NN product on 256 x 256 tiles (-1: two workgroups per CU) and the tiles of the rest", py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("act"), py::arg("layout_b") = 0);
   m.def("gemm_big", &gemm_big, "token-parallel GEMM family (NT / NN / TN, LoRA K-extension, split-K, SwiGLU)",
         py::arg("a"), py::arg("b"), py::arg("layout_a"), py::arg("layout_b"), py::arg("a2") = py::none(),
         py::arg("b2") = py::none(), py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("out_mode") = 0,

@@ -46,7 +46,8 @@ struct Tuning {
   int m64_wide = 1;           // bf16 16 < M <= 64, N % 256 == 0, N <= 16384, no SwiGLU: 256 weight rows per workgroup
                               // (the wide kernel over row-major weights); 0: the 64-column ring gemm_m64_kernel
   // ---- token-parallel GEMMs (gemm_big.hip) ----
-  float gemm_bn128_cost = 0.55f;  // planner: time of a 256x128 tile / a 256x256 tile
+  float gemm_bn128_cost = 0.55f;  // planner: time of a 256x128 tile / a 256x256 tile; with a column-contiguous B (NN products) 1.127
+                                  // times as much, 0.62 (gemm_big.hip, bn128_cost)
   int gemm_duo = 1;           // NT products on two workgroups per CU: 0 never, 1 where they are short (gemm_big.hip), 2
                               // wherever the kernel takes them
   int gemm_mid = 1;           // ... and on smaller tiles: 0 never, 1 where the larger leave CUs idle, 2 / 3 / 4 always on 64 x 64 /

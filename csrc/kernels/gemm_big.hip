@@ -1400,7 +1400,7 @@ static bool bn128_supported(int layout_a, int layout_b, int act, int out) {
 // Ratio of a 256x128 tile's time to a 256x256 tile's (same K), for the wave planner below. With a K-contiguous A and a
 // column-contiguous B (NN) it is larger, 74 us to 120 at K = 4096: the transposed reads of B wait inside each phase. 4016 x 14336 x
 // 4096, which 0.55 put on seven rounds of 128 columns: 468 us, 391 on 256; with the SwiGLU backward 535, so 467.
-static float bn128_cost(int layout_b = ROW) { return layout_b == KMAJ ? 0.62f : tuning().gemm_bn128_cost; }
+static float bn128_cost(int layout_b = ROW) { return tuning().gemm_bn128_cost * (layout_b == KMAJ ? 0.62f / 0.55f : 1.f); }
 
 static int gemm_big_planned(const Args& p, int layout_a, int layout_b, int act, int out, int bn, hipStream_t stream);
 static int launch_mid(const Args& p, int form, int act, hipStream_t stream);
@@ -1559,9 +1559,10 @@ static Plan plan_tiles(int M, int N, int K, int act, bool plain, bool can128, in
   return p;
 }
 
-// how many rows of a plain product (see plan_tiles) go on 256 x 256 tiles, and the form of the rest; -1: gemm_duo_kernel
-extern "C" int rt_gemm_plan(int M, int N, int K, int act, int* form) {
-  const Plan p = plan_tiles(M, N, K, act, true, bn128_supported(ROW, ROW, act, O_BF16), ROW);
+// how many rows of a product with a bf16 result go on 256 x 256 tiles, and the form of the rest; -1: gemm_duo_kernel. A row-major B: a
+// plain product (see plan_tiles); a column-contiguous one: NN
+extern "C" int rt_gemm_plan(int M, int N, int K, int act, int layout_b, int* form) {
+  const Plan p = plan_tiles(M, N, K, act, layout_b == ROW, bn128_supported(ROW, layout_b, act, O_BF16), layout_b);
   *form = p.form;
   return p.m1 < 0 ? -1 : (int)std::min<long>(M, p.m1 * 256L);
 }
