@@ -45,6 +45,8 @@ __global__ __launch_bounds__(512, 2) void few_rows_kernel(Args p) {
   __shared__ __attribute__((aligned(16))) char ring[8 * D * CH];
   __shared__ __attribute__((aligned(16))) bf16_t xs[NW ? TR * 16 * LDX : 8];
   __shared__ f32x4 red[16][64];  // [part][column group][row tile]
+  // <2, 0, 0> takes the CU's LDS to the last byte: without a norm nothing names xs, and it gets no place
+  static_assert(sizeof(ring) + (NW ? sizeof(xs) : 0) + sizeof(red) <= 160 * 1024, "the LDS of a CU");
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, r16 = lane & 15;
   const int nc = p.K / 64, CG = 8 / (p.ks * p.rs), RTS = p.rs * RT;  // column groups, row tiles of the workgroup
