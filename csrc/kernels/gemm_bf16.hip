@@ -554,7 +554,7 @@ __global__ __launch_bounds__(64 * NW) void gemv16_kernel(GemmArgs p) {
 // row-major form -> image form:
 //   6144 x 4096 with norm    21.6 / 21.5 / 22.5 -> 14.9 / 17.2 / 19.4     28672 x 4096, SwiGLU  55.5 / 53.4 / 56.0 -> 44.2 / 44.3 / 45.5
 //   4096 x 4096 + residual   14.8 / 16.4 / 17.3 -> 10.9 / 13.9 / 15.4     4096 x 14336          29.6 / 30.2 / 31.9 -> 25.0 / 28.0 / 30.7
-//   10304 x 4096             36.0 / 37.4 / 38.8 -> 19.2 / 22.8 / 25.7     14336 x 4096, relu^2  29.8 / 31.3 / 32.6 -> 23.8 / 25.8 / 28.1
+//   10304 x 4096             36.0 / 37.4 / 38.8 -> 22.0 / 22.7 / 24.8     14336 x 4096, relu^2  29.8 / 31.3 / 32.6 -> 23.8 / 25.8 / 28.1
 //   32000 x 4096             59.0 / 58.9 / 60.8 -> 47.6 / 50.4 / 54.0     3072 x 2048 with norm 15.5 / 16.7 / 17.7 -> 7.1 / 9.9 / 11.7
 //
 // gemv64_kernel: gemv16_kernel with RT row tiles, for small products (see gemm64_direct): a workgroup owns one 16-row group
@@ -1566,16 +1566,17 @@ static int decode_split(int N, int K) {
 }
 
 // Image products of 16 < M <= 64 rows: re-reading X per 16-row group is the cheaper way while the product is small and its
-// groups fill the chip no more than once. us, direct | best split of the other, M = 24 / 48 / 64: 2048 x 2048 6.7 / 9.3 / 11.1
-// | 8.7 / 10.6 / 12.4 (before the hand-off took one trip); 3072 x 2048 7.1 / 9.9 / 11.7 | 10.1 / 12.8 / 14.3; 4096 x 4096 11.1 / 16.3 / 19.9 | 12.4 / 14.5 / 16.6
-// (M = 32: 12.1 | 12.4); 2048 x 7168, long K, 15.8 / 24 / 30 | 12.9 / 15.6 / 18.0.
+// groups fill the chip no more than once. us, direct | best split of the other, M = 24 / 48 / 64: 2048 x 2048 7.1 / 9.4 / 11.1
+// | 8.0 / 9.4 / 10.8; 3072 x 2048 7.4 / 10.1 / 11.9 | 8.8 / 10.3 / 11.9; 4096 x 4096 at M = 24 / 32 12.2 / 12.3 | 11.6 / 11.6 (the line
+// was drawn before the split's hand-off took one trip, when that was 12.4, and kept: before it 48 rows direct took 16.3, split 14.5).
 static bool gemm64_direct(int M, int N, int K) {
   return tuning().decode_split == 0 && N <= 4096 && K <= 4096 && (long)M * N * K <= 1L << 29;
 }
 // Split over K: up to one workgroup per CU, with at least 16 chunks each, 32 for the gated pairs whose partial tiles are
-// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 20.7 / 16.9 / 14.2 / 13.3 / 17.6 / 17.8;
-// 4096 x 14336 62.4 / 42.1 / 32.7 / 28.0 / 35.4 / 32.2; 6144 x 4096 21.7 / 17.3 / 21.5 / 19.1; 10304 x 4096 (161 groups)
-// 26.4 / 27.9; SwiGLU 14336 x 2048 18.0 / 17.4.
+// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 20.6 / 15.8 / 14.3 / 13.3 / 17.6 / 17.7;
+// 4096 x 14336 62.4 / 38.4 / 30.2 / 27.0 / 34.9 / 31.2; 6144 x 4096 21.7 / 17.3 / 21.5 / 19.2; 10304 x 4096 (161 groups)
+// 22.7 / 27.6. The pairs' line is older than the hand-off in one trip and lies too high now: SwiGLU 14336 x 2048 18.1 / 17.5 (at 64 rows
+// 19.5 / 19.6), 7168 x 4096 29.1 / 21.5 / 20.1 / 18.8, 10240 x 2560 22.1 / 17.8 / 17.8.
 static int gemm64_split(int groups, int K, bool pair) {
   if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
   int split = 1;
