@@ -285,32 +285,48 @@ __device__ __forceinline__ uint2 f32x8_to_fp8(const float* v, float inv) {
   return make_uint2(lo, hi);
 }
 
-// Sum of `ns` fp32 split-K slabs of 8 consecutive floats (slab q at p + q * stride), added in
-// slab order from slab 0 (bitwise equal to a rolled `for q` loop). The loads of the first 8 slabs
-// are issued unconditionally (indices clamped to ns - 1, the surplus ones hit cache) before the
-// first add: ONE L2/MALL round trip, where a rolled loop with a runtime trip count waits for every
-// slab's loads in turn.
-__device__ __forceinline__ void sum_slabs8(const float* p, long stride, int ns, float (&out)[8]) {
-  float4 lo[8], hi[8];
+// Sum of `ns` fp32 split-K slabs of 8 consecutive floats (slab q at p + q * stride), added in slab order from slab 0 (bitwise
+// equal to a rolled `for q` loop). Q slabs' loads are issued unconditionally (indices clamped to ns - 1, the surplus ones hit cache)
+// before the first add: ONE L2/MALL round trip, where a rolled loop with a runtime trip count waits for every slab's loads in turn.
+// Q by the number of slabs: eight loads whatever their number cost few slabs more than the trip (a reduction of 256 x 4096 over 1 /
+// 2 / 5 / 8 slabs 3.8 / 3.8 / 4.0 / 4.5 us, now 2.9 / 3.2 / 3.7 / 4.4).
+template <int Q>
+__device__ __forceinline__ void sum_slabs8_of(const float* p, long stride, int ns, float (&out)[8]) {
+  float4 lo[Q], hi[Q];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
+  for (int q = 0; q < Q; ++q) {
     const float* sp = p + (long)min(q, ns - 1) * stride;
     lo[q] = *(const float4*)sp;
     hi[q] = *(const float4*)(sp + 4);
   }
   // used here: else the compiler moves a slab's loads to its addition, behind the wait for the others
 #pragma unroll
-  for (int q = 1; q < 8; ++q)
+  for (int q = 1; q < Q; ++q)
     asm volatile("" : "+v"(lo[q].x), "+v"(lo[q].y), "+v"(lo[q].z), "+v"(lo[q].w), "+v"(hi[q].x), "+v"(hi[q].y), "+v"(hi[q].z), "+v"(hi[q].w));
   out[0] = lo[0].x; out[1] = lo[0].y; out[2] = lo[0].z; out[3] = lo[0].w;
   out[4] = hi[0].x; out[5] = hi[0].y; out[6] = hi[0].z; out[7] = hi[0].w;
 #pragma unroll
-  for (int q = 1; q < 8; ++q)
+  for (int q = 1; q < Q; ++q)
     if (q < ns) {
       out[0] += lo[q].x; out[1] += lo[q].y; out[2] += lo[q].z; out[3] += lo[q].w;
       out[4] += hi[q].x; out[5] += hi[q].y; out[6] += hi[q].z; out[7] += hi[q].w;
     }
-  for (int q = 8; q < ns; ++q) {
+}
+// MOST: of them in flight at most (4 where registers are short, else 8)
+template <int MOST = 8>
+__device__ __forceinline__ void sum_slabs8(const float* p, long stride, int ns, float (&out)[8]) {
+  if (ns == 1) {
+    sum_slabs8_of<1>(p, stride, ns, out);
+  } else if (ns <= 2) {
+    sum_slabs8_of<2>(p, stride, ns, out);
+  } else if (ns <= 4 || MOST == 4) {
+    sum_slabs8_of<4>(p, stride, ns, out);
+  } else if (ns <= 6) {
+    sum_slabs8_of<6>(p, stride, ns, out);
+  } else {
+    sum_slabs8_of<8>(p, stride, ns, out);
+  }
+  for (int q = MOST; q < ns; ++q) {
     const float4 a = *(const float4*)(p + (long)q * stride), b = *(const float4*)(p + (long)q * stride + 4);
     out[0] += a.x; out[1] += a.y; out[2] += a.z; out[3] += a.w;
     out[4] += b.x; out[5] += b.y; out[6] += b.z; out[7] += b.w;

@@ -16,15 +16,15 @@ namespace rt {
 
 constexpr int NORM_MAXV = 8;  // max 16-B vectors per thread -> H <= 256*8*8 = 16384
 
-template <bool LAYERNORM, int NV, int MAXT = 512>
+template <bool LAYERNORM, int NV, int MOST, int MAXT = 512>
 __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                        const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
                                                        bf16_t* __restrict__ y, bf16_t* __restrict__ h_out,
                                                        float* __restrict__ rstd_out, float* __restrict__ mean_out,
                                                        int H, float eps, const float* __restrict__ xs, int nsplit,
                                                        long sstride) {
-  // xs != null: x is the bf16-rounded sum of nsplit fp32 split-K slabs (stride sstride floats):
-  // the split-K reduce of the producing GEMM fused into this pass (decode at batch 65..512)
+  // MOST > 0: x is the bf16-rounded sum of nsplit fp32 split-K slabs xs (stride sstride floats), at most MOST of them in
+  // flight: the split-K reduce of the producing GEMM fused into this pass (decode at batch 65..512)
   __shared__ float sbuf[16];  // <= 16 waves
   const long row = blockIdx.x;
   const int nv = H / 8;
@@ -46,10 +46,10 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
   if (res)
 #pragma unroll
     for (int i = 0; i < NV; ++i) rraw[i] = *(const uint4*)(res + row * H + at(i));
-  if (xs) {
+  if constexpr (MOST > 0) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      sum_slabs8(xs + row * H + at(i), sstride, nsplit, v[i]);
+      sum_slabs8<MOST>(xs + row * H + at(i), sstride, nsplit, v[i]);
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[i][k] = bf2f(f2bf(v[i][k]));  // = the reduce kernel's bf16 output
     }
@@ -317,6 +317,10 @@ extern "C" int rt_norm_fwd(int layernorm, const void* x, const void* res, const 
   // split-K slab reduce (decode at batch 65..512: one row per block, rows <= CUs): twice the waves
   // per row (one 8-element chunk per thread) keep twice the slab loads in flight per CU
   const int sl = tuning().norm_slab_threads;
+  // More rows than CUs: two workgroups share a CU if their registers let them (48 with four slabs in flight, 111 with eight). us, RMS of
+  // 300 x 5120 over 1 / 5 / 8 slabs: 6.5 / 8.5 / 12.4 with a rolled loop, 7.7 / 9.2 / 12.8 with eight in flight, 5.0 / 7.8 / 11.9 now; 256 rows
+  // (rolled, now with eight) 5.0 / 6.1 / 10.0 and 4.1 / 5.4 / 9.5
+  const bool many = T > num_cus();
   if (xs && sl >= 512 && H / 8 >= 512 && H / 8 <= 512) {
     threads = 512;
     nvpt = 1;
@@ -325,14 +329,16 @@ extern "C" int rt_norm_fwd(int layernorm, const void* x, const void* res, const 
   // sums three chunks' slabs one memory round trip after another (19.6 us per norm at batch 256)
   if (xs && sl >= 512 && H / 8 > 512 && H / 8 <= 1024) {
     const int t = (H / 8 + 63) / 64 * 64;
-    if (layernorm)
-      hipLaunchKernelGGL((norm_fwd_kernel<true, 1, 1024>), dim3(T), dim3(t), 0, stream, (const bf16_t*)x,
-                         (const bf16_t*)res, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean,
-                         H, eps, xs, nsplit, (long)T * H);
-    else
-      hipLaunchKernelGGL((norm_fwd_kernel<false, 1, 1024>), dim3(T), dim3(t), 0, stream, (const bf16_t*)x,
-                         (const bf16_t*)res, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean,
-                         H, eps, xs, nsplit, (long)T * H);
+#define NORM_FWD_LONG(LN, MOST)                                                                                    \
+  hipLaunchKernelGGL((norm_fwd_kernel<LN, 1, MOST, 1024>), dim3(T), dim3(t), 0, stream, (const bf16_t*)x,          \
+                     (const bf16_t*)res, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean, \
+                     H, eps, xs, nsplit, (long)T * H)
+    if (layernorm) {
+      if (many) NORM_FWD_LONG(true, 4); else NORM_FWD_LONG(true, 8);
+    } else {
+      if (many) NORM_FWD_LONG(false, 4); else NORM_FWD_LONG(false, 8);
+    }
+#undef NORM_FWD_LONG
     RT_LAUNCH_CHECK();
     return 0;
   }
@@ -356,15 +362,24 @@ extern "C" int rt_norm_fwd(int layernorm, const void* x, const void* res, const 
     RT_LAUNCH_CHECK();
     return 0;
   }
-  if (layernorm) {
-    NORM_DISPATCH(true, norm_fwd_kernel, dim3(T), dim3(threads), 0, stream, (const bf16_t*)x, (const bf16_t*)res,
-                  (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean, H, eps, xs, nsplit,
-                  (long)T * H)
-  } else {
-    NORM_DISPATCH(false, norm_fwd_kernel, dim3(T), dim3(threads), 0, stream, (const bf16_t*)x, (const bf16_t*)res,
-                  (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean, H, eps, xs, nsplit,
-                  (long)T * H)
+#define NORM_FWD_NV(LN, NV, MOST)                                                                                  \
+  hipLaunchKernelGGL((norm_fwd_kernel<LN, NV, MOST>), dim3(T), dim3(threads), 0, stream, (const bf16_t*)x,         \
+                     (const bf16_t*)res, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, (bf16_t*)h_out, rstd, mean, \
+                     H, eps, xs, nsplit, (long)T * H)
+#define NORM_FWD(LN, NV)                                                                                           \
+  do {                                                                                                             \
+    if (!xs) NORM_FWD_NV(LN, NV, 0); else if (many) NORM_FWD_NV(LN, NV, 4); else NORM_FWD_NV(LN, NV, 8);           \
+  } while (0)
+#define NORM_FWD_LN(NV) do { if (layernorm) NORM_FWD(true, NV); else NORM_FWD(false, NV); } while (0)
+  switch (nvpt) {
+    case 1: NORM_FWD_LN(1); break;
+    case 2: NORM_FWD_LN(2); break;
+    case 4: NORM_FWD_LN(4); break;
+    default: if (H / 8 <= 6 * threads) NORM_FWD_LN(6); else NORM_FWD_LN(8);
   }
+#undef NORM_FWD_LN
+#undef NORM_FWD
+#undef NORM_FWD_NV
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -746,6 +746,29 @@ def test_weight_images_across_streams_captures_and_copies():
 
 
 # ---------------------------------------------------------------------------------------------- norms
+@pytest.mark.parametrize("H", [8, 520, 2048, 4096, 5120, 8192, 11008, 13312])
+@pytest.mark.parametrize("T", [5, 300])
+def test_slab_sums_by_their_number(T, H):
+    """One to ten slabs, on either side of the CUs' number: the sum in slab order, rounded once, in the reduction and ahead of a norm;
+    the norm of the rounded stream to one rounding (2^-8 of it, and 1e-5 for 32-bit sums)."""
+    from rag_tl_domainllm_optimizer_amd.ops.linear import SplitK
+
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    res, w = (torch.randn(n, H, generator=g, device=DEV).bfloat16() for n in (T, 1))
+    for ns in (1, 2, 3, 4, 5, 6, 7, 8, 9, 10):
+        slabs = torch.randn(ns, T, H, generator=g, device=DEV)
+        sk = SplitK(slabs.reshape(-1), ns, T, H, torch.bfloat16)
+        total = slabs[0].clone()
+        for q in range(1, ns):
+            total += slabs[q]
+        assert torch.equal(sk.reduce(), total.bfloat16())
+        y, h = ops.rms_norm(sk, w[0], 1e-5, res)
+        assert torch.equal(h, (total.bfloat16().float() + res.float()).bfloat16())
+        x = h.double()
+        want = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+        assert ((y.double() - want).abs() <= (2.0 ** -8 + 1e-5) * want.abs()).all()
+
+
 @pytest.mark.parametrize("H", [8, 384, 512, 520, 768, 1024, 1032])
 @pytest.mark.parametrize("T", [1, 5, 1023, 1024, 9001])
 def test_norm_wave_per_row_bits(H, T):
