@@ -88,6 +88,13 @@ def test_output_norm_with_scale(dtype, H):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H", [260, 1284, 2052, 3072, 4100, 5120, 6148, 8196, 16384])
+def test_output_norm_of_odd_widths(dtype, H):
+    """widths that leave part of a thread's last access unused, over two to eight accesses: stream and next norm"""
+    test_output_norm_with_scale(dtype, H)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 300, 700])
 def test_squared_relu_epilogues(M, dtype):
     for K, N in ((256, 512), (128, 192), (72, 144), (44, 30), (512, 136)):
