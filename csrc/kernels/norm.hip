@@ -119,7 +119,7 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
 // norm_fwd_kernel's NW waves, added in its order: the same bits. LayerNorm with residual, us before -> now: 23000 x 384 16.7 ->
 // 13.8, 23000 x 768 31.3 -> 25.4 (5.6 TB/s), 4096 x 1024 7.9 -> 7.2, 15 x 384 3.0 -> 2.8
 // ONCE: a row's loads all go out before the first is used (a branch for the residual and for each vector's end made each wait for
-// its own), and the residual stream is stored beside the result: stored between the loads' arrival and the sums it cost long rows
+// its own), and the residual stream is stored behind the result, under one check: stored between the loads' arrival and the sums it cost long rows
 // what the loads had gained. LayerNorm with residual, us, each vector for itself -> at once -> and stored at the end, on one machine:
 // 23000 x 384 13.9 -> 13.4 -> 12.4, 23000 x 768 30.9 -> 28.5 -> 25.3, 4096 x 1024 8.1 -> 8.9 -> 8.1. RMS with residual: 1024 x 1024
 // 3.6 -> 3.4 -> 3.2, but from about 4096 rows of two vectors on, when every SIMD has rows enough to hide the trips, a row's loads
@@ -192,7 +192,6 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict
       const int c = lane + 64 * i;
       if (c < nv) {
         float wv[8], bv[8], o[8];
-        if (ONCE && res && h_out) *(uint4*)(h_out + row * H + c * 8) = pack8(v[i]);
         unpack8(wraw[i], wv);
         if (LAYERNORM && b) unpack8(braw[i], bv);
 #pragma unroll
@@ -202,6 +201,11 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict
         }
         *(uint4*)(y + row * H + c * 8) = pack8(o);
       }
+    }
+    if (ONCE && res && h_out) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+        if (lane + 64 * i < nv) *(uint4*)(h_out + row * H + (lane + 64 * i) * 8) = pack8(v[i]);
     }
     if (lane == 0) {
       if (rstd_out) rstd_out[row] = rstd;
