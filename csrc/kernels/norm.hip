@@ -123,7 +123,8 @@ __global__ __launch_bounds__(MAXT) void norm_fwd_kernel(const bf16_t* __restrict
 // what the loads had gained. LayerNorm with residual, us, each vector for itself -> at once -> and stored at the end, on one machine:
 // 23000 x 384 13.9 -> 13.4 -> 12.4, 23000 x 768 30.9 -> 28.5 -> 25.3, 4096 x 1024 8.1 -> 8.9 -> 8.1. RMS with residual: 1024 x 1024
 // 3.6 -> 3.4 -> 3.2, but from about 4096 rows of two vectors on, when every SIMD has rows enough to hide the trips, a row's loads
-// side by side cost more than they save (4096 x 1024 7.0 -> 8.0, 8192 x 768 9.3 -> 10.0): not ONCE, each vector for itself.
+// side by side cost more than they save (4096 x 1024 7.0 -> 8.0, 8192 x 768 9.3 -> 10.0; without one from about 8192 on, 12000 x 768
+// 7.4 -> 7.9): not ONCE, each vector for itself.
 template <bool LAYERNORM, int NW, bool ONCE>
 __global__ __launch_bounds__(256) void norm_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                         const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
@@ -357,7 +358,7 @@ extern "C" int rt_norm_fwd(int layernorm, const void* x, const void* res, const 
       if (H <= 512) NORM_ROWS(true, 1, true); else NORM_ROWS(true, 2, true);
     } else if (H <= 512) {
       NORM_ROWS(false, 1, true);
-    } else if (res && T >= 4096) {
+    } else if (T >= (res ? 4096 : 8192)) {
       NORM_ROWS(false, 2, false);
     } else {
       NORM_ROWS(false, 2, true);
