@@ -19,7 +19,7 @@
 #define RT_LAUNCH_CHECK() RT_HIP_CHECK(hipGetLastError())
 
 // Device-side bounds checks of the debug build (python -m rag_tl_domainllm_optimizer_amd._build
-// --debug, SURVEY §5.2): a failed check prints the condition and traps the wave, which surfaces as
+// --debug): a failed check prints the condition and traps the wave, which surfaces as
 // a launch error on the next synchronisation instead of a silent out-of-bounds access.
 #ifndef RAGTL_DEBUG
 #define RAGTL_DEBUG 0
