@@ -70,7 +70,10 @@ int rt_gemm_plan(int, int, int, int, int, int*);
 int rt_token_plan(int, int, int, int, int*);
 int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
-                       float, hipStream_t);
+                       float, void*, long, void*, int, hipStream_t);
+long rt_encoder_few_bytes(int, int, int, int, int, int, const int*);
+int rt_encoder_few(const void* const*, void*, long, const long*, const float*, int, int, int, int, int, int, int, float, float, const int*, int,
+                   float*, const long*, long, hipStream_t);
 int rt_attn_decode(const void*, long, const void*, const void*, int, const int*, const int*, int, float*, int, int,
                    void*, long, int, int, int, int, float, hipStream_t);
 int rt_attn_decode_fused(const void*, long, void*, void*, int, const int*, const int*, const int*, const int*,
@@ -1408,11 +1411,35 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
                          (int)H, (float)eps, nullptr, 0, st),
              "encoder: norm");
   };
+  auto embed = [&](void* y, void* unset, long unset_bytes, void* zero) {
+    check_rc(rt_embed_norm_rows(word.data_ptr(), (const long*)ids.data_ptr(), ptab.data_ptr(), (const long*)pos.data_ptr(),
+                                emb[2] ? emb[2]->data_ptr() : nullptr, emb[3]->data_ptr(), emb[4]->data_ptr(), y, (int)M, (int)H,
+                                (float)eps, unset, unset_bytes, zero, (int)(M + 15) / 16 * 16, st),
+             "encoder: embedding");
+  };
+  // Up to 64 rows the layers in one launch: 64 rows of mpnet-base 517 -> 475 us, fewer or narrower more (see encoder_few.hip); beyond, a round of
+  // 16-row tasks no longer fits the CUs. The shapes that rt_encoder_few_bytes refuses (no bytes) go on below.
+  if (M <= 64 && H % 64 == 0 && F % 64 == 0) {
+    const KParts k[4] = {k_parts(M, 3 * H, H, 0), k_parts(M, H, H, 0), k_parts(M, F, H, 2), k_parts(M, H, F, 0)};
+    const int parts[8] = {k[0].n, k[0].grp, k[1].n, k[1].grp, k[2].n, k[2].grp, k[3].n, k[3].grp};
+    const int L = (int)(layers.size() / 12);
+    const long bytes = rt_encoder_few_bytes((int)M, (int)H, (int)F, (int)std::min<int64_t>(B, INT_MAX), L, (int)heads, parts);
+    if (bytes) {
+      Tensor ws = at::empty({bytes}, word.options().dtype(at::kByte));
+      char* const x0 = (char*)ws.data_ptr() + 256;
+      const int64_t x0_bytes = (M + 15) / 16 * 32 * H;
+      embed(x0, x0 + x0_bytes, bytes - 256 - x0_bytes, ws.data_ptr());
+      std::vector<const void*> w(layers.size());
+      for (size_t i = 0; i < w.size(); ++i) w[i] = layers[i].data_ptr();
+      check_rc(rt_encoder_few(w.data(), ws.data_ptr(), bytes, (const long*)off.data_ptr(), (const float*)opt_ptr(rel_bias), (int)rb_L, (int)M,
+                              (int)H, (int)F, (int)B, L, (int)heads, (float)eps, (float)(1.0 / std::sqrt((double)D)), parts,
+                              normalize ? 1 : 0, out.data_ptr<float>(), (const long*)to.data_ptr(), out.size(0), st),
+               "encoder: layers");
+      return true;
+    }
+  }
   Tensor x = rows(H), a = rows(H);
-  check_rc(rt_embed_norm_rows(word.data_ptr(), (const long*)ids.data_ptr(), ptab.data_ptr(), (const long*)pos.data_ptr(),
-                              emb[2] ? emb[2]->data_ptr() : nullptr, emb[3]->data_ptr(), emb[4]->data_ptr(), x.data_ptr(), (int)M,
-                              (int)H, (float)eps, st),
-           "encoder: embedding");
+  embed(x.data_ptr(), nullptr, 0, nullptr);
   const int64_t max_parts = M <= 16 ? 16 : 8;
   if (M <= 64 && H % 64 == 0 && F % 64 == 0 && k_parts(M, 3 * H, H, 0).n <= max_parts && k_parts(M, H, H, 0).n <= max_parts &&
       k_parts(M, F, H, 2).n <= max_parts && k_parts(M, H, F, 0).n <= max_parts) {

@@ -1,6 +1,6 @@
 // Products of few rows with weights of an encoder's size, for gfx950: y = act(x W^T + bias), where x may still be LN(d + res).
-// One query through all-MiniLM-L6-v2 is 24 such products of about 15 rows, each a few hundred KB of weights: what they take is
-// launch, one trip to memory and the reduction over K, not bandwidth.
+// For encoders that encoder_few.hip does not take (heads of 128, rows of 1024 with 4096 between): a query is four such products a layer, each
+// a few hundred KB of weights: what they take is launch, one trip to memory and the reduction over K, not bandwidth.
 //
 // K is summed in the parts, and the parts in the order, of the kernel that ops.gemm takes for the shape (see Args), so that the
 // bits are that kernel's: a text's embedding does not depend on the way it went. The 8 waves of a workgroup are parts x row tiles
@@ -210,14 +210,19 @@ __global__ __launch_bounds__(512, 2) void few_rows_kernel(Args p) {
 }
 
 // x[t] = LN(bf16(word[id] + pos[p]) + type): the embedding of an encoder in one pass, a wave a row. The sum is rounded to bf16
-// after each term, as embed_kernel and an addition do; the norm is norm_rows_kernel's without a residual.
+// after each term, as embed_kernel and an addition do; the norm is norm_rows_kernel's without a residual. `unset` and `zero` (see
+// encoder_few.hip): memory that is set to ones, and 256 bytes of zeros; with them the rows hold no word of ones, and lie in column groups
+// of 16 with `tile` rows each.
 template <int NW>
 __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __restrict__ word, const long* __restrict__ ids,
                                                               const bf16_t* __restrict__ pos, const long* __restrict__ pids,
                                                               const bf16_t* __restrict__ type, const bf16_t* __restrict__ w,
                                                               const bf16_t* __restrict__ b, bf16_t* __restrict__ y, int T, int H,
-                                                              float eps) {
+                                                              float eps, uint4* __restrict__ unset, long n_unset,
+                                                              unsigned* __restrict__ zero, int tile) {
   const int lane = threadIdx.x & 63, nv = H / 8;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n_unset; i += (long)gridDim.x * 256) unset[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (zero && blockIdx.x == 0 && threadIdx.x < 64) zero[threadIdx.x] = 0;
   for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < T; row += (long)gridDim.x * 4) {
     RT_ASSERT(ids[row] >= 0 && pids[row] >= 0);
     const bf16_t* const wp = word + ids[row] * H;
@@ -269,7 +274,13 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
         unpack8(*(const uint4*)(b + c * 8), bv);
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = fmaf((v[i][e] - mean) * rstd, wv[e], bv[e]);
-        *(uint4*)(y + row * H + c * 8) = pack8(o);
+        uint4 q = pack8(o);
+        if (zero) {
+          uint32_t* const u = (uint32_t*)&q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) u[e] = u[e] == ~0u ? 0xfffefffeu : u[e];
+        }
+        *(uint4*)(y + (zero ? ((c >> 1) * tile + row) * 16 + (c & 1) * 8 : row * H + c * 8)) = q;
       }
     }
   }
@@ -310,18 +321,19 @@ extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, c
   return 0;
 }
 
-// y[t] = LN(word[ids[t]] + pos[pids[t]] (+ type)); H % 8 == 0, H <= 1024
+// y[t] = LN(word[ids[t]] + pos[pids[t]] (+ type)); H % 8 == 0, H <= 1024. unset_bytes: a multiple of 16
 extern "C" int rt_embed_norm_rows(const void* word, const long* ids, const void* pos, const long* pids, const void* type,
-                                  const void* w, const void* b, void* y, int T, int H, float eps, hipStream_t stream) {
+                                  const void* w, const void* b, void* y, int T, int H, float eps, void* unset, long unset_bytes,
+                                  void* zero, int tile, hipStream_t stream) {
   if (T <= 0) return 0;
   if (H % 8 || H > 1024) return -1;
-  const dim3 grid(std::min((T + 3) / 4, 2048)), block(256);
-  if (H <= 512)
-    hipLaunchKernelGGL(fr::embed_norm_rows_kernel<1>, grid, block, 0, stream, (const bf16_t*)word, ids, (const bf16_t*)pos, pids,
-                       (const bf16_t*)type, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, T, H, eps);
-  else
-    hipLaunchKernelGGL(fr::embed_norm_rows_kernel<2>, grid, block, 0, stream, (const bf16_t*)word, ids, (const bf16_t*)pos, pids,
-                       (const bf16_t*)type, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, T, H, eps);
+  const long n = unset ? unset_bytes / 16 : 0;
+  const dim3 grid((unsigned)std::min(std::max((T + 3L) / 4, (n + 255) / 256), 2048L)), block(256);
+#define EN(W)                                                                                                                 \
+  hipLaunchKernelGGL(fr::embed_norm_rows_kernel<W>, grid, block, 0, stream, (const bf16_t*)word, ids, (const bf16_t*)pos, pids, \
+                     (const bf16_t*)type, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, T, H, eps, (uint4*)unset, n, (unsigned*)zero, tile)
+  if (H <= 512) EN(1); else EN(2);
+#undef EN
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -636,6 +636,85 @@ def test_native_encoder_forward_is_the_ops_forward(preset, lens):
     assert torch.equal(got[to], want)
 
 
+def _few_rows_encoder(heads, seed, **kw):
+    from rag_tl_domainllm_optimizer_amd import models
+    import dataclasses
+
+    cfg = dataclasses.replace(models.resolve_preset("minilm-l6"), num_layers=3, num_heads=heads, head_dim=384 // heads, **kw)
+    m = models.SentenceEncoder(cfg, device=DEV, dtype=torch.bfloat16, init=False).eval()
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            p.normal_(1.0 if "ln" in name and name.endswith("_w") else 0.0, 0.05, generator=g)
+
+    def inputs(lens, gap=0):
+        off = gap + torch.nn.functional.pad(torch.tensor(lens, device=DEV).cumsum(0), (1, 0))
+        rows = int(off[-1]) + gap
+        ids = torch.randint(4, cfg.vocab_size, (rows,), generator=g, device=DEV)
+        pos = torch.randint(0, 100, (rows,), generator=g, device=DEV)
+        return ids, pos, off, max(lens)
+    return m, inputs
+
+
+# 12 heads of 32, 6 of 64: one launch for the layers; 3 of 128: one by one
+@pytest.mark.parametrize("heads,kw", [(12, {}), (6, {}), (3, {}), (6, dict(intermediate_size=1472))])
+@pytest.mark.parametrize("lens,gap", [([15], 0), ([16], 0), ([31], 0), ([32], 0), ([48], 0), ([49], 0), ([64], 0), ([1] * 41, 0),
+                                      ([0, 5, 0, 33, 0], 0), ([17, 16, 30], 0), ([9, 20], 2), ([2], 31)])
+def test_encoder_of_few_rows(heads, kw, lens, gap):
+    """Up to 64 rows against the same forward op by op, the same bits: around the 16-row tiles and the 32-query blocks, many texts,
+    texts without rows, rows ahead of the first text and behind the last."""
+    m, inputs = _few_rows_encoder(heads, len(lens) + heads, **kw)
+    ids, pos, off, longest = inputs(lens, gap)
+    out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
+    assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(len(lens), device=DEV))
+    assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
+
+
+def test_encoder_of_few_rows_replayed_and_on_two_streams():
+    """A captured forward gives every replay's inputs their results, with eager calls between; two streams at once theirs."""
+    m, inputs = _few_rows_encoder(12, 3)
+    cases = [inputs(lens) for lens in ([40], [15], [40], [33, 7], [12, 28])]
+    want = [m.encode_packed(*c) for c in cases]
+    outs = [torch.zeros_like(w) for w in want]
+    tos = [torch.arange(len(w), device=DEV) for w in want]
+    ids, pos, off, longest = (t.clone() if torch.is_tensor(t) else t for t in cases[0])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        m._encode_native(ids, pos, off, longest, True, outs[0], tos[0])
+    for k in (0, 2, 0, 2):
+        ids.copy_(cases[k][0])
+        pos.copy_(cases[k][1])
+        m._encode_native(*cases[1], True, outs[1], tos[1])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], want[k]) and torch.equal(outs[1], want[1])
+    streams = [torch.cuda.Stream() for _ in cases]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for s, c, o, t in zip(streams, cases, outs, tos):
+            with torch.cuda.stream(s):
+                m._encode_native(*c, True, o, t)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
+@pytest.mark.parametrize("where", ["word_embed", "emb_ln_b", "layers.0.qkv_b", "layers.1.fc1_w", "layers.2.ln2_w"])
+def test_encoder_of_few_rows_with_all_ones(where):
+    """Words of all ones (NaN) among the parameters: NaN comes out, of no text that they do not reach."""
+    m, inputs = _few_rows_encoder(12, 4)
+    ids, pos, off, longest = inputs([15, 20])
+    ids[:20], ids[20:] = 5, 6
+    p = dict(m.named_parameters())[where]
+    with torch.no_grad():
+        (p[5] if where == "word_embed" else p).view(torch.int16).fill_(-1)
+    out = torch.zeros(2, m.cfg.hidden_size, device=DEV)
+    assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(2, device=DEV))
+    want = m.encode_packed(ids, pos, off, longest)
+    assert torch.equal(out.isnan(), want.isnan()) and out[0].isnan().any()
+    torch.testing.assert_close(out, want, rtol=0, atol=0, equal_nan=True)
+
+
 def test_native_encoder_writes_no_row_beyond_out():
     """Rows counted from the end go there, texts whose row does not exist go nowhere: the rows around out stay as they are."""
     from rag_tl_domainllm_optimizer_amd import models
