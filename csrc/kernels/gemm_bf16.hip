@@ -642,11 +642,13 @@ __global__ __launch_bounds__(64 * NW) void gemv64_kernel(GemmArgs p) {
 // through LDS in 64-deep chunks (8 KB, double-buffered, one barrier a chunk) and is read N / 64 times. Both X parts
 // and weights come in plain loads, DEPTH - 1 chunks ahead: with LDS-DMA for X the compiler waits for everything in flight
 // wherever it needs a weight register (SwiGLU 28672 x 4096 at M = 24: 49 us instead of 44). Few column groups are split
-// over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order. It asks for the
-// tiles of all rows at once, and bias and residual are asked for ahead of the hand-off: a trip to memory a row tile, and one for
-// each element of a residual, were 2 to 3 us of every split product. us at M = 24 / 48 / 64: 6144 x 4096 with norm 15.8 / 19.6 / 21.9 ->
-// 14.9 / 17.2 / 19.4, 4096 x 4096 + residual 12.3 / 15.3 / 17.5 -> 12.1 / 13.9 / 15.4, 4096 x 14336 25.6 / 29.2 / 32.4 -> 25.0 / 28.0 /
-// 30.7, 2048 x 7168 14.0 / 17.5 / 20.7 -> 12.4 / 14.5 / 16.7. More chunks in flight (6, 8), fragments read a chunk ahead: nothing.
+// over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order. A wave hands over for itself
+// (its columns are no other's), by 16-byte stores of whole lines and a ticket on a line of its own, and asks for all rows' tiles at once; bias and residual
+// are asked for ahead of it. Of 4096 x 4096 at 48 rows (11.7 us) 2.0 pass until the first chunk is there, 4.6 in the loop (7.3 TB/s), 1.4 until the
+// ticket is back, 1.2 until the parts are there, 0.7 in the epilogue, the rest between launches. us with the whole workgroup at one ticket and the
+// activations' code in the epilogue -> this, M = 24 / 48 / 64: 6144 x 4096 with norm 14.9 / 17.6 / 19.6 -> 13.8 / 15.6 / 16.8, 4096 x 4096 + residual
+// 10.9 / 13.5 / 15.2 -> 10.6 / 11.7 / 12.6, 4096 x 14336 23.5 / 26.2 / 28.9 -> 22.3 / 24.2 / 26.2, 2048 x 7168 12.1 / 14.5 / 16.5 -> 10.6 / 12.8 / 13.9.
+// More chunks in flight (6, 8), fragments read a chunk ahead: nothing.
 template <bool OUT_F32, int RT, bool PAIR>
 __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __restrict__ slabs,
                                                            unsigned* __restrict__ tickets, int split) {
@@ -764,37 +766,30 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
     for (int j = 0; j < NG; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) bias[j][e] = bf2f(p.bias[j * n_out + lcol + e]);
-  uint2 res[RT];
+  uint2 res[RT] = {};
   if (r4)
 #pragma unroll
     for (int t = 0; t < RT; ++t) res[t] = *(const uint2*)(p.R + (long)min(16 * t + frow, p.M - 1) * p.ldr + lcol);
   if (split > 1) {
-    constexpr int SLAB = 16 * RT * COLS + 64;
-    typedef unsigned long long u64;
-    auto bits = [](float a, float b) -> u64 { return (u64)__float_as_uint(a) | (u64)__float_as_uint(b) << 32; };
-    u64* slab = (u64*)(slabs + ((long)cg * split + sp) * SLAB);
-    // write-through stores, drained before the ticket
+    // a wave's columns are its own: it hands over to the same wave of the last workgroup, without the others. In 16-byte device-scope
+    // stores of whole lines, drained before the ticket
+    constexpr int SLAB = RT * NG * 256 + 64;  // floats of a wave: fragments, sums of squares
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(slabs, 0, -1, 0x00020000);
+    constexpr int SC1 = 16;
+    const uint32_t group = 4u * SLAB * (uint32_t)(split * (4 * cg + cw));  // bytes
+    const uint32_t own = group + 4u * SLAB * sp;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
 #pragma unroll
-      for (int j = 0; j < NG; ++j) {
-        u64* d = slab + (((t * NG + j) * 4 + cw) * 64 + lane) * 2;
-        __hip_atomic_store(d, bits(acc[t][j][0], acc[t][j][1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(d + 1, bits(acc[t][j][2], acc[t][j][3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (normed && cw == 0 && g == 0)
-        __hip_atomic_store((float*)slab + 16 * RT * COLS + 16 * t + frow, ss[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int j = 0; j < NG; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[t][j]), rs, own + 16 * (64 * (t * NG + j) + lane), 0, SC1);
+      if (normed && g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ss[t]), rs, own + 4 * (RT * NG * 256 + 16 * t + frow), 0, SC1);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    int* flag = (int*)smem;
-    if (tid == 0)
-      *flag = __hip_atomic_fetch_add(tickets + cg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(split - 1);
-    __syncthreads();
-    if (!*flag) return;
-    if (tid == 0) __hip_atomic_store(tickets + cg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(tickets + 32 * (4 * cg + cw), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(old) != (unsigned)(split - 1)) return;
+    if (lane == 0) __hip_atomic_store(tickets + 32 * (4 * cg + cw), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the last one adds all parts in their order, its own among them; all row tiles' loads of AT_ONCE parts in flight
-    const u64* base = (const u64*)(slabs + (long)cg * split * SLAB);
     constexpr int AT_ONCE = PAIR ? 2 : 4;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
@@ -803,21 +798,17 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
       for (int j = 0; j < NG; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     for (int q0 = 0; q0 < split; q0 += AT_ONCE) {
-      u64 v[AT_ONCE][RT][NG][2];
+      f32x4 v[AT_ONCE][RT][NG];
       float s[AT_ONCE][RT];
 #pragma unroll
       for (int k = 0; k < AT_ONCE; ++k) {
-        const u64* part = base + (long)min(q0 + k, split - 1) * (SLAB / 2);
+        const uint32_t part = group + 4u * SLAB * min(q0 + k, split - 1);
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
 #pragma unroll
           for (int j = 0; j < NG; ++j)
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-              v[k][t][j][e] = __hip_atomic_load(part + (((t * NG + j) * 4 + cw) * 64 + lane) * 2 + e, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-          s[k][t] = __hip_atomic_load((const float*)part + 16 * RT * COLS + 16 * t + frow, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);  // unused without a norm
+            v[k][t][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, part + 16 * (64 * (t * NG + j) + lane), 0, SC1));
+          s[k][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, part + 4 * (RT * NG * 256 + 16 * t + frow), 0, SC1));  // unused without a norm
         }
       }
 #pragma unroll
@@ -826,12 +817,36 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
 #pragma unroll
           for (int t = 0; t < RT; ++t) {
 #pragma unroll
-            for (int j = 0; j < NG; ++j)
-              acc[t][j] += f32x4{__uint_as_float((unsigned)v[k][t][j][0]), __uint_as_float((unsigned)(v[k][t][j][0] >> 32)),
-                                 __uint_as_float((unsigned)v[k][t][j][1]), __uint_as_float((unsigned)(v[k][t][j][1] >> 32))};
+            for (int j = 0; j < NG; ++j) acc[t][j] += v[k][t][j];
             if (normed) ss[t] += s[k][t];
           }
     }
+  }
+  // Linear and relu^2 on their own: the others' code, once an element, lies between what these run, and every jump over it is a
+  // wait for instructions that no cache holds (an epilogue of 1.25 us, now 0.7)
+  if (!PAIR && (p.act == ACT_NONE || p.act == ACT_RELU2) && (!p.R || r4)) {
+    const bool relu2 = p.act == ACT_RELU2;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int row = 16 * t + frow;
+      const float rs = normed ? rsqrtf(ss[t] / (float)p.K + p.norm_eps) : 1.f;
+      float y[4];
+      const float r[4] = {__uint_as_float(res[t].x << 16), __uint_as_float(res[t].x & 0xffff0000u), __uint_as_float(res[t].y << 16),
+                          __uint_as_float(res[t].y & 0xffff0000u)};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        y[e] = acc[t][0][e] * rs;
+        y[e] = p.bias ? y[e] + bias[0][e] : y[e];
+        const float q = fmaxf(y[e], 0.f);
+        y[e] = relu2 ? q * q : y[e];
+        y[e] = p.R ? y[e] + r[e] : y[e];
+      }
+      if (row < p.M && col < n_out) {
+        if constexpr (OUT_F32) *(float4*)((float*)p.C + (long)row * p.ldc + col) = make_float4(y[0], y[1], y[2], y[3]);
+        else *(uint2*)((bf16_t*)p.C + (long)row * p.ldc + col) = make_uint2(pack2bf(y[0], y[1]), pack2bf(y[2], y[3]));
+      }
+    }
+    return;
   }
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
@@ -1565,22 +1580,22 @@ static int decode_split(int N, int K) {
   return split;
 }
 
-// Image products of 16 < M <= 64 rows: re-reading X per 16-row group is the cheaper way while the product is small and its
-// groups fill the chip no more than once. us, direct | best split of the other, M = 24 / 48 / 64: 2048 x 2048 7.1 / 9.4 / 11.1
-// | 8.0 / 9.4 / 10.8; 3072 x 2048 7.4 / 10.1 / 11.9 | 8.8 / 10.3 / 11.9; 4096 x 4096 at M = 24 / 32 12.2 / 12.3 | 11.6 / 11.6 (the line
-// was drawn before the split's hand-off took one trip, when that was 12.4, and kept: before it 48 rows direct took 16.3, split 14.5).
+// Image products of 16 < M <= 64 rows: re-reading X per 16-row group, without a hand-off, is the cheaper way while X is small. us, direct | best
+// split of the other: 3072 x 1024 at M = 24 / 48 / 64 4.7 / 6.2 / 7.3 | 6.4 / 7.4 / 8.0; 2048 x 2048 at 24 / 32 / 48 6.8 / 7.5 / 9.4 | 7.1 / 7.2 / 8.2;
+// 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6.
 static bool gemm64_direct(int M, int N, int K) {
-  return tuning().decode_split == 0 && N <= 4096 && K <= 4096 && (long)M * N * K <= 1L << 29;
+  return tuning().decode_split == 0 && N <= 4096 && (long)M * K <= 1L << 16;
 }
-// Split over K: up to one workgroup per CU, with at least 16 chunks each, 32 for the gated pairs whose partial tiles are
-// twice as large. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 20.6 / 15.8 / 14.3 / 13.3 / 17.6 / 17.7;
-// 4096 x 14336 62.4 / 38.4 / 30.2 / 27.0 / 34.9 / 31.2; 6144 x 4096 21.7 / 17.3 / 21.5 / 19.2; 10304 x 4096 (161 groups)
-// 22.7 / 27.6. The pairs' line is older than the hand-off in one trip and lies too high now: SwiGLU 14336 x 2048 18.1 / 17.5 (at 64 rows
-// 19.5 / 19.6), 7168 x 4096 29.1 / 21.5 / 20.1 / 18.8, 10240 x 2560 22.1 / 17.8 / 17.8.
+// Split over K: up to one workgroup per CU (half a round more costs more than it balances), up to four parts of at least 8 chunks (10 for the
+// gated pairs, whose partial tiles are twice as large), more of at least 16. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 19.8 / 14.6 /
+// 12.6 / 11.7 / 14.3 / 14.6; 4096 x 14336 61.2 / 36.5 / 28.1 / 24.3 / 31.0 / 26.9; 6144 x 4096 20.9 / 15.8 / 19.2 / 16.5; 2048 x 7168 31.6 / 20.1 / 16.1 /
+// 13.7 / 12.6 / 12.8; 2048 x 2048 11.4 / 9.7 / 8.5 / 8.2 / 8.8 / 9.5; 10304 x 4096 (161 groups) 21.8 / 25.1 / 21.3; SwiGLU 14336 x 2048 17.9 / 16.0 / 20.2,
+// 7168 x 2048 17.1 / 13.7 / 12.8 / 13.1, 7168 x 4096 29.2 / 20.5 / 18.4 / 17.0.
 static int gemm64_split(int groups, int K, bool pair) {
   if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
+  auto least = [&](int parts) { return parts > 4 ? 16 : pair ? 10 : 8; };
   int split = 1;
-  while (split < 8 && groups * (split + 1) <= 256 && K / 64 >= (pair ? 32 : 16) * (split + 1)) ++split;
+  while (split < 8 && groups * (split + 1) <= 256 && K / 64 >= least(split + 1) * (split + 1)) ++split;
   return split;
 }
 
@@ -1675,7 +1690,9 @@ extern "C" int rt_gemm_nt_glu(const void* A, long lda, const void* B, long ldb, 
     const bool pair = act == ACT_SWIGLU;
     const int rt = (M + 15) / 16, groups = pair ? (N + 127) / 128 : (N + 63) / 64;
     const bool direct = !pair && gemm64_direct(M, N, K);
-    const int split = direct || !slabs || !tickets ? 1 : fit_split(gemm64_split(groups, K, pair), groups, 16 * rt * 64 * (pair ? 2 : 1) + 64);
+    // a ticket a wave, each on a line of its own
+    const int split = direct || !slabs || !tickets || 128 * groups > RT_SPLITK_TICKETS
+                          ? 1 : fit_split(gemm64_split(groups, K, pair), 4 * groups, 16 * rt * 16 * (pair ? 2 : 1) + 64);
     const dim3 grid(direct ? N / 16 : groups * split), block(direct ? 512 : 256);
 #define I64_CASE(F32, RTT)                                                                                              \
   if (direct) hipLaunchKernelGGL((gemv64_kernel<F32, RTT, 8, 3>), grid, block, 0, stream, p);                           \

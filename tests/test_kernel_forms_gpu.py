@@ -429,6 +429,29 @@ def test_image_products_17_to_64_rows(N, K, act):
                 assert (out[:, No:] == 7).all()
 
 
+@pytest.mark.parametrize("act", [0, ops.ACT_RELU2, 2, 4])
+@pytest.mark.parametrize("N,K,split", [(2064, 2176, 0), (4176, 1088, 0), (4176, 1088, 5), (208, 6144, 8)])
+def test_image_products_17_to_64_rows_epilogues(N, K, split, act):
+    """Linear and squared-relu results, whose epilogue is their own, and the others', behind parts of K and without: residuals that come
+    four at a time and ones that do not, with and without bias, a last column group that is not whole."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(N + act)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    img, bias = C.shuffle_decode_weight(w), torch.randn(N, generator=g, device=DEV).bfloat16()
+    for M in (17, 33, 64):
+        x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+        pre = x.double() @ w.double().t()
+        bound = (x.double().abs() @ w.double().abs().t()).max().item() * K * 2.0 ** -24 + 1e-6
+        for r, b in ((None, None), (torch.randn(M, N, generator=g, device=DEV).bfloat16(), bias),
+                     (torch.randn(M, N + 3, generator=g, device=DEV).bfloat16()[:, :N], None)):
+            with ops.tuning(decode_split=split):
+                y = C.gemm(x, img, None, None, b, act, False, None, r, 0.0, True)
+            z = pre if b is None else pre + b.double()
+            want = ref.apply_act(z, act) + (0 if r is None else r.double())
+            # a bf16 rounding of the result and, before a square, the fp32 sum's error
+            torch.testing.assert_close(y.double(), want, rtol=2.0 ** -8 + 1e-4, atol=2 * bound * (1 + z.abs().max().item()) + 1e-5)
+
+
 # ---------------------------------------------------------------------------------------------- GELU epilogue
 @pytest.mark.parametrize("M,N,res", [(65, 256, False), (300, 264, True), (4096, 8, False)])
 def test_gelu_epilogue_bits(M, N, res):
