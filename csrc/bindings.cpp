@@ -71,6 +71,8 @@ int rt_token_plan(int, int, int, int, int*);
 int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
                        float, void*, long, void*, int, hipStream_t);
+int rt_gemm_norm(const void*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, float, int, hipStream_t);
+int rt_gemm_norm_rows(int, int, int);
 long rt_encoder_few_bytes(int, int, int, int, int, int, const int*);
 int rt_encoder_few(const void* const*, void*, long, const long*, const float*, int, int, int, int, int, int, int, float, float, const int*, int,
                    float*, const long*, long, hipStream_t);
@@ -1361,6 +1363,24 @@ static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, 
   return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, 1, std::nullopt, std::nullopt, std::nullopt, bn, {});
 }
 
+// LN(x w^T + bias + res) in one launch, tiles of `rows` rows (0: as rt_gemm_norm_rows says); contiguous bf16
+static Tensor linear_norm(const Tensor& x, const Tensor& w, const Tensor& bias, const Tensor& res, const Tensor& lw, const Tensor& lb, double eps,
+                          int64_t rows) {
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  for (const Tensor* t : {&x, &w, &bias, &res, &lw, &lb})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->is_contiguous() && (uintptr_t)t->data_ptr() % 16 == 0,
+                "linear_norm: contiguous bf16 tensors, 16-byte aligned");
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && res.dim() == 2 && res.size(0) == M && res.size(1) == N && bias.numel() == N && lw.numel() == N &&
+                  lb.numel() == N && M <= INT_MAX, "linear_norm: sizes");
+  Tensor y = at::empty({M, N}, x.options());
+  if (!rows) rows = rt_gemm_norm_rows((int)M, (int)N, (int)K);
+  TORCH_CHECK(rows, "linear_norm: ", M, " x ", N, " x ", K, " is not faster in one launch");
+  check_rc(rt_gemm_norm(x.data_ptr(), w.data_ptr(), bias.data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M, (int)N, (int)K,
+                        (float)eps, (int)rows, cur_stream()),
+           "linear_norm");
+  return y;
+}
+
 // A sentence encoder's forward over texts without padding (see attn_packed), pooled and normalised, written to out[to[b]]:
 // one call for the 40 and more launches, which from Python take longer to issue than a short query's take to run. emb: word and
 // position tables, token type row or null, norm weight, norm bias; layers: qkv, o, ln1, fc1, fc2, ln2, a weight and a bias each.
@@ -1487,13 +1507,22 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
     norm(d, x, t[0], t[1], z);
     std::swap(x, z);
   } else {
+    // y = LN(in w^T + b + res): one launch where that is faster, the same bits
+    auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& y) {
+      const int tile = rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1));
+      if (tile)
+        check_rc(rt_gemm_norm(in.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M,
+                              (int)H, (int)in.size(1), (float)eps, tile, st),
+                 "encoder: product and norm");
+      else
+        norm(encoder_linear(in, t[0], t[1], 0), res, lw, lb, y);
+    };
+    Tensor y = rows(H);
     for (size_t l = 0; l < layers.size(); l += 12) {
       const Tensor* t = &layers[l];
       attend(encoder_linear(x, t[0], t[1], 0), a);
-      Tensor d = encoder_linear(a, t[2], t[3], 0), y = rows(H);
-      norm(d, x, t[4], t[5], y);
-      d = encoder_linear(encoder_linear(y, t[6], t[7], 2), t[8], t[9], 0);
-      norm(d, y, t[10], t[11], x);
+      product_norm(a, t + 2, t[4], t[5], x, y);
+      product_norm(encoder_linear(y, t[6], t[7], 2), t + 8, t[10], t[11], y, x);
     }
   }
   check_rc(rt_pool_norm(x.data_ptr(), nullptr, (const long*)off.data_ptr(), M, (int)B, 0, (int)H, normalize ? 1 : 0,
@@ -1736,6 +1765,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
         py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
         py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
+  m.def("linear_norm", &linear_norm, "LN(x w^T + b + res) in one launch", py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("res"), py::arg("lw"),
+        py::arg("lb"), py::arg("eps"), py::arg("rows") = 0);
   m.def("few_rows", &few_rows, "act(x w^T + b) of up to 32 rows, normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);

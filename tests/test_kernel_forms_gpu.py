@@ -738,6 +738,46 @@ def test_encoder_of_few_rows_with_all_ones(where):
     torch.testing.assert_close(out, want, rtol=0, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("M,K", [(1, 64), (63, 128), (64, 192), (65, 384), (127, 320), (128, 1536), (129, 64), (300, 448), (16400, 384)])
+def test_product_and_norm_in_one_launch(M, K, rows):
+    """LN(x w^T + b + res) with the bits of product and norm, and close to 64 bits: ends of tiles, fewer K-steps than are fetched ahead, odd
+    numbers of them, a NaN, an infinite and a huge row (whose variance overflows) among the others, rows around the result."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(M + K + rows)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(384, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    bias, lb = (torch.randn(384, generator=g, device=DEV).bfloat16() for _ in range(2))
+    lw = (1 + 0.1 * torch.randn(384, generator=g, device=DEV)).bfloat16()
+    res = torch.randn(M, 384, generator=g, device=DEV).bfloat16()
+    got = C.linear_norm(x, w, bias, res, lw, lb, 1e-12, rows)
+    want = ops.layer_norm(C.gemm_big(x, w, 0, 0, bias=bias), lw, lb, 1e-12, residual=res)[0]
+    assert torch.equal(got, want)
+    # product and sum are rounded to bf16 (2^-9 of values below 8) ahead of a division by about 1.4, the result (below 8) once more
+    h = x.double() @ w.double().t() + bias.double() + res.double()
+    ref = torch.nn.functional.layer_norm(h, (384,), lw.double(), lb.double(), 1e-12)
+    assert (got.double() - ref).abs().max().item() < 3 * 8 * 2 ** -9
+    if M < 60:
+        return
+    x[5, 3], res[17, 20], res[M - 1] = float("nan"), float("inf"), 1e30 * torch.sign(res[M - 1].float()).bfloat16()
+    got = C.linear_norm(x, w, bias, res, lw, lb, 1e-12, rows)
+    want2 = ops.layer_norm(C.gemm_big(x, w, 0, 0, bias=bias), lw, lb, 1e-12, residual=res)[0]
+    torch.testing.assert_close(got, want2, rtol=0, atol=0, equal_nan=True)
+    keep = [i for i in range(min(M - 1, 200)) if i not in (5, 17)]
+    assert got[5].isnan().all() and torch.equal(got[keep], want[keep])
+
+
+@pytest.mark.parametrize("lens", [[2951], [2952], [6407, 1], [5000, 11384], [9000, 7385], [1] * 500 + [17000]])
+def test_encoder_where_products_take_the_norm(lens):
+    """Around the row counts where the output and the second feed-forward product begin to end in the norm and where their tiles
+    grow, the bits of the forward op by op."""
+    m, inputs = _few_rows_encoder(12, sum(lens))
+    ids, pos, off, longest = inputs(lens)
+    out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
+    assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(len(lens), device=DEV))
+    assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
+
+
 def test_native_encoder_writes_no_row_beyond_out():
     """Rows counted from the end go there, texts whose row does not exist go nowhere: the rows around out stay as they are."""
     from rag_tl_domainllm_optimizer_amd import models
