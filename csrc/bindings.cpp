@@ -72,7 +72,7 @@ int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
                        float, void*, long, void*, int, hipStream_t);
 int rt_gemm_norm(const void*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, float, int, hipStream_t);
-int rt_gemm_norm_rows(int, int, int);
+int rt_gemm_norm_rows(int, int, int, int*);
 long rt_encoder_few_bytes(int, int, int, int, int, int, const int*);
 int rt_encoder_few(const void* const*, void*, long, const long*, const float*, int, int, int, int, int, int, int, float, float, const int*, int,
                    float*, const long*, long, hipStream_t);
@@ -1373,8 +1373,8 @@ static Tensor linear_norm(const Tensor& x, const Tensor& w, const Tensor& bias, 
   TORCH_CHECK(w.dim() == 2 && w.size(1) == K && res.dim() == 2 && res.size(0) == M && res.size(1) == N && bias.numel() == N && lw.numel() == N &&
                   lb.numel() == N && M <= INT_MAX, "linear_norm: sizes");
   Tensor y = at::empty({M, N}, x.options());
-  if (!rows) rows = rt_gemm_norm_rows((int)M, (int)N, (int)K);
-  TORCH_CHECK(rows, "linear_norm: ", M, " x ", N, " x ", K, " is not faster in one launch");
+  int first;
+  TORCH_CHECK(rows || rt_gemm_norm_rows((int)M, (int)N, (int)K, &first), "linear_norm: ", M, " x ", N, " x ", K, " is not faster in one launch");
   check_rc(rt_gemm_norm(x.data_ptr(), w.data_ptr(), bias.data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M, (int)N, (int)K,
                         (float)eps, (int)rows, cur_stream()),
            "linear_norm");
@@ -1509,10 +1509,10 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
   } else {
     // y = LN(in w^T + b + res): one launch where that is faster, the same bits
     auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& y) {
-      const int tile = rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1));
-      if (tile)
+      int first;
+      if (rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1), &first))
         check_rc(rt_gemm_norm(in.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M,
-                              (int)H, (int)in.size(1), (float)eps, tile, st),
+                              (int)H, (int)in.size(1), (float)eps, 0, st),
                  "encoder: product and norm");
       else
         norm(encoder_linear(in, t[0], t[1], 0), res, lw, lb, y);

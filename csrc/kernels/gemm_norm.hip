@@ -1,8 +1,11 @@
 // y = LN(x w^T + bias + res) of rows that a workgroup holds whole: the two products of a post-norm encoder layer that end in a layer norm.
 // As two launches the sum went out to memory and back between them, and 384 columns are one and a half tiles of 256: a quarter of the
-// matrix work was for columns that are not there. us, product and norm -> this, by 384 columns: 28100 rows x 384 33.7 -> 18.8, x 1536
-// 55.5 -> 35.8; 15000 rows 22.6 -> 12.0, 35.1 -> 23.8; 8960 rows 16.6 -> 10.4, 25.5 -> 22.0. Encoder forward of 1024 texts (MiniLM) 3775 -> 3446.
+// matrix work was for columns that are not there; 768 are three tiles of 256, whose rounds leave CUs idle. us, product and norm -> this, by 384 columns: 28100 rows x 384 33.7 -> 18.8, x 1536
+// 55.5 -> 35.8; 15000 rows 22.6 -> 12.0, 35.1 -> 23.8; 8960 rows 16.6 -> 10.4, 25.5 -> 22.0. By 768 columns, in an encoder: 24000 rows x 768 54.9 -> 37.5, x 3072 121 -> 99, 12000 rows 35.9 -> 24.4, 73.6 -> 67.
+// Encoder forward of 1024 texts (MiniLM) 3775 -> 3446, of mpnet-base over 12000 / 24000 / 49000 rows 3030 -> 2813 / 5150 -> 4790 / 10390 -> 9740.
 #include "rt_common.h"
+
+#include <algorithm>
 
 namespace rt {
 namespace gn {
@@ -60,13 +63,15 @@ __device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, uint4 v, uint3
 // stay for the step, each phase multiplies them by FG of its w fragments (a granule: 128 columns, 16 FG of every wave). While a phase is
 // multiplied the next one's fragments are read, and the places that are read out are asked for again: 7 granules and 3 x images ahead.
 // Behind the last step nothing is fetched: the same loads go out of range, which fills their places with zeros and keeps the counted waits.
-// Cycles a step of 128 / 64 rows by 384 columns: 2090 / 1300, of which the matrix cores work 1546 / 773 and the LDS pipe 1790 / 1310 (fragments
+// 96 rows by 768 columns (64 do not fill the matrix cores' time, of 128 neither sums nor rows fit): x fragments come in a burst of 12 a wave at the end of a
+// step, 3270 cycles of which the matrix cores work 2320. Cycles a step of 128 / 64 rows by 384 columns: 2090 / 1300, of which the matrix cores work 1546 / 773 and the LDS pipe 1790 / 1310 (fragments
 // and DMA), which bounds it. Waves 2 x 4 read the least of 128 rows, 1 x 8 of 64. w straight from memory to the one wave that
 // multiplies it (1 x 8) took 3200: its lanes lie 16 rows apart, one line a lane.
 template <int WC, int FM, int NP>
 __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
-  constexpr int TM = 8 / WC * 16 * FM, TN = 128 * NP, FG = 8 / WC, FN = FG * NP, NA = TM / 64, XI = TM * 128, GR = 128 * 128, LDT = TN + 8;
+  constexpr int TM = 8 / WC * 16 * FM, TN = 128 * NP, FG = 8 / WC, FN = FG * NP, NA = (TM + 63) / 64, XI = TM * 128, GR = 128 * 128, LDT = TN + 8;
   static_assert(TM * LDT * 2 <= AP * XI + BP * GR, "the tile fits the places");
+  constexpr bool LATE = NP > 4;  // no registers for the epilogue's operands beside the sums
   __shared__ __attribute__((aligned(16))) char smem[AP * XI + BP * GR];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -85,9 +90,9 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
     const uint32_t far = (uint32_t)(nk - 1 - t) & FAR;  // beyond the last step
 #pragma unroll
     for (int j = 0; j < NA; ++j) {
-      const int o = wid * NA + j;
+      const int o = TM == 96 && j ? 8 + (wid & 3) : TM == 128 ? 2 * wid + j : wid;  // 96 rows: the last four by two waves each, the same bytes
       const uint32_t base = (uint32_t)(o * 8 * (int)p.ldx * 2 + t * 128) | far;
-      dma16(Xr, smem + place * XI + o * 1024, (NA == 2 ? lx[j] : lx[wid & 1]) + base);
+      dma16(Xr, smem + place * XI + o * 1024, (TM == 128 ? lx[j] : lx[wid & 1]) + base);
     }
   };
   // granule of phase ph of step t: image row r is column (r / W) 16 FN + W ph + r % W, W = 16 FG
@@ -121,20 +126,30 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   // For the epilogue: 16 lanes a row, of which a lane has the 16-B vectors nq + 16 m; a wave four rows at a time
   const int nq = lane & 15, nrow = wid * (TM / 8) + (lane >> 4);
   uint2 bias[FN];
-#pragma unroll
-  for (int j = 0; j < FN; ++j) bias[j] = *(const uint2*)(p.bias + (FN * wc + j) * 16 + fq * 4);
   uint4 res[NP], lwr[NP], lbr[NP];
   auto residual = [&](int row) {
 #pragma unroll
     for (int m = 0; m < NP; ++m) res[m] = *(const uint4*)(p.res + (long)(m0 + min(row, rows - 1)) * p.ldr + (nq + 16 * m) * 8);
   };
-  residual(nrow);
+  auto operands = [&]() {
 #pragma unroll
-  for (int m = 0; m < NP; ++m) {
-    lwr[m] = *(const uint4*)(p.lw + (nq + 16 * m) * 8);
-    lbr[m] = *(const uint4*)(p.lb + (nq + 16 * m) * 8);
-  }
+    for (int j = 0; j < FN; ++j) bias[j] = *(const uint2*)(p.bias + (FN * wc + j) * 16 + fq * 4);
+    residual(nrow);
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {
+      lwr[m] = *(const uint4*)(p.lw + (nq + 16 * m) * 8);
+      lbr[m] = *(const uint4*)(p.lb + (nq + 16 * m) * 8);
+    }
+  };
+  if constexpr (!LATE) operands();
 
+  // All of w, each workgroup its share, in whole rows: the products that go through the caches between two of this one leave nothing of
+  // w there, and a K-step of it is a line of 128 B from each of TN rows, which all workgroups ask for at the same time, only 7 granules ahead. Its place is
+  // one that this wave fills itself later (loads come in in their order). In an encoder, 768 columns: 12000 rows x 3072 101 -> 67 us, x 768
+  // 32.2 -> 24.4, 24000 rows x 3072 123 -> 99.
+  const uint32_t share = (uint32_t)(((long)TN * p.ldw * 2 / gridDim.x + 8191) / 8192);
+  for (uint32_t k = 0; k < min(share, 6u); ++k)
+    dma16(Wr, smem + (AP - 1) * XI + (TM == 128 ? 2 * wid : wid) * 1024, ((blockIdx.x * share + k) * 8 + wid) * 1024 + lane * 16);
   // what the phases before the first would have asked for
   constexpr int B0 = AP * NP;
   static_assert(B0 - 1 >= BP, "x first");
@@ -195,6 +210,8 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
     if constexpr (NP > 1) phase(std::integral_constant<int, S ^ 1>{}, std::integral_constant<int, 1>{});
     if constexpr (NP > 2) phase(std::integral_constant<int, S>{}, std::integral_constant<int, 2>{});
     if constexpr (NP > 3) phase(std::integral_constant<int, S ^ 1>{}, std::integral_constant<int, 3>{});
+    if constexpr (NP > 4) phase(std::integral_constant<int, S>{}, std::integral_constant<int, 4>{});
+    if constexpr (NP > 5) phase(std::integral_constant<int, S ^ 1>{}, std::integral_constant<int, 5>{});
   };
   while (t + 1 < nk) {
     step(std::integral_constant<int, 0>{});
@@ -208,6 +225,7 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   // everything in registers in straight code 16200, this takes 9800.
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // nothing lands in the places any more
   __syncthreads();
+  if constexpr (LATE) operands();
   bf16_t* const tile = (bf16_t*)smem;
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
@@ -221,18 +239,21 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   __syncthreads();
   const __amdgpu_buffer_rsrc_t Yr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.y + (long)m0 * p.ldy), 0, ((rows - 1) * (int)p.ldy + TN) * 2, 0x00020000);
   auto row_sum = [&](const float (&x)[NP]) {
-    static_assert(NP == 2 || NP == 3 || NP == 4, "vectors of a lane");
-    float s;
-    if constexpr (NP == 4) s = (x[0] + x[2]) + (x[1] + x[3]);
+    static_assert(NP == 2 || NP == 3 || NP == 4 || NP == 6, "vectors of a lane");
+    float s, u = 0.f;  // of the first 64 vectors, of the others
+    if constexpr (NP >= 4) s = (x[0] + x[2]) + (x[1] + x[3]);
     else if constexpr (NP == 3) s = (x[0] + x[2]) + x[1];
     else s = x[0] + x[1];
-#define GN_DPP(ctrl) s += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(s), ctrl, 0xf, 0xf, false))
-    GN_DPP(0x128);  // row_ror:8
-    GN_DPP(0x124);  // row_ror:4: the exchange of lanes 4 apart, now that those 8 apart hold the same
-    GN_DPP(0x4e);   // quad_perm [2, 3, 0, 1]
-    GN_DPP(0xb1);   // quad_perm [1, 0, 3, 2]
+    if constexpr (NP == 6) u = x[4] + x[5];
+#define GN_DPP(v, ctrl) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), ctrl, 0xf, 0xf, false))
+#define GN_STEP(ctrl) do { GN_DPP(s, ctrl); if constexpr (NP > 4) GN_DPP(u, ctrl); } while (0)
+    GN_STEP(0x128);  // row_ror:8
+    GN_STEP(0x124);  // row_ror:4: the exchange of lanes 4 apart, now that those 8 apart hold the same
+    GN_STEP(0x4e);   // quad_perm [2, 3, 0, 1]
+    GN_STEP(0xb1);   // quad_perm [1, 0, 3, 2]
+#undef GN_STEP
 #undef GN_DPP
-    return s;
+    return NP > 4 ? s + u : s;
   };
 #pragma unroll 1
   for (int k = 0; k < TM / 8; k += 4) {
@@ -282,27 +303,60 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
 
 using namespace rt;
 
-// Rows of a tile with which rt_gemm_norm beats product and norm; 0: it doesn't, or the shape is not for it. A tile is one chain over K, 0.54 us a
-// step of 64 rows and 6 besides (128 rows: 0.9 and 8), however few there are: with few rows the product's small tiles in parallel are
-// faster. Even, by 384 columns: 2500 rows at K 128, 3000 at 384, 4500 at 768, 5300 at 1536, 10500 at 3072. Tiles of 64 while they are one
-// round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles of 64 42.6).
-extern "C" int rt_gemm_norm_rows(int M, int N, int K) {
-  if (N != 384 || K < 64 || K % 64 || (long)N * K * 2 >= 0x7fffffffL || M < 1800 + 3L * K) return 0;
-  return M <= 64 * num_cus() ? 64 : 128;
+static bool fits(int N, int K) { return (N == 384 || N == 768) && K >= 64 && K % 64 == 0 && (long)N * K * 2 < 0x7fffffffL; }
+
+// Rows of a tile with which rt_gemm_norm beats product and norm, `first` leading rows in larger ones; 0: it doesn't, or the shape is not for it.
+// A tile is one chain over K, however few there are: with few rows the product's small tiles in parallel are faster.
+// 384 columns: 0.54 us a step of 64 rows and 6 besides (128 rows: 0.9 and 8). Even: 2500 rows at K 128, 3000 at 384, 4500 at 768, 5300 at 1536,
+// 10500 at 3072; between an encoder's other kernels not below 4000 (a forward of 3000 rows 360 -> 368). Tiles of 64 while they are one round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles
+// of 64 42.6).
+// 768 columns, us within an encoder's forward (between other kernels: alone, with w in the caches, both are faster): a round of tiles of 64 takes
+// 10 and 1.18 a step, nearly full 14 and 1.25, one of several 6.4 and 1.53; of 96 18 and 1.72. Product and norm: tiles of 256 x 256, whole rounds of
+// them and a rest, and 0.78 ns a row. All of one size, or whole rounds of 96 and the rest in 64. Product and norm | this at K 768: 12000 rows 35.9 |
+// 24.4, 20000 42.7 | 34.0, 24000 54.9 | 37.5, 28000 59.3 | 49.4, 42000 88 | 73; at K 3072: 12000 73.6 | 67, 20000 89.6 | 90 (not taken), 24000 121 | 99, 28000
+// 146 | 160 (not taken), 49000 237 | 204.
+extern "C" int rt_gemm_norm_rows(int M, int N, int K, int* first) {
+  *first = 0;
+  if (!fits(N, K)) return 0;
+  if (N == 384) return M < std::max(4000L, 1800 + 3L * K) ? 0 : M <= 64 * num_cus() ? 64 : 128;
+  const int per64 = 64 * num_cus(), per96 = 96 * num_cus(), per256 = num_cus() / 3 * 256;
+  auto rounds = [](int rows, int per) { return (rows + per - 1) / per; };
+  const double steps = K / 64;
+  auto in64 = [&](int rows) {
+    const int n = rounds(rows, per64);
+    return n > 1 ? n * (6.4 + 1.53 * steps) : 4L * rows <= 3L * per64 ? 10 + 1.18 * steps : 14 + 1.25 * steps;
+  };
+  const double r96 = 18 + 1.72 * steps, large = 13 + 0.0203 * K, rest = std::min(1., 0.24 + 5e-5 * (M % per256));
+  const double apart = (M / per256 + rest) * large + 1.5 + 0.00078 * M;
+  const int whole = M / per96;
+  const double all64 = in64(M), all96 = rounds(M, per96) * r96, both = whole * r96 + in64(M - whole * per96);
+  if (std::min(std::min(all64, all96), both) > apart) return 0;
+  if (whole && both < all64 && both < all96) *first = whole * per96;
+  return all96 <= all64 && !*first ? 96 : 64;
 }
 
-// y = LN(x w^T + bias + res) * lw + lb of M rows, N = 384 columns, K % 64 == 0; contiguous 16-B aligned rows. rows: of a tile, 64 or 128.
-// -1: not for this kernel.
+// y = LN(x w^T + bias + res) * lw + lb of M rows, N = 384 or 768 columns, K % 64 == 0; contiguous 16-B aligned rows. rows: of a tile, 64 or 128
+// (384 columns) or 96 (768); 0: as rt_gemm_norm_rows says. -1: not for this kernel.
 extern "C" int rt_gemm_norm(const void* x, const void* w, const void* bias, const void* res, const void* lw, const void* lb, void* y, int M,
                             int N, int K, float eps, int rows, hipStream_t stream) {
-  if (N != 384 || K < 64 || K % 64 || (long)N * K * 2 >= 0x7fffffffL || (rows != 64 && rows != 128)) return -1;
+  const int large = N == 384 ? 128 : 96;
+  int first = 0;
+  if (!rows) rows = rt_gemm_norm_rows(M, N, K, &first);
+  if (!fits(N, K) || (rows != 64 && rows != large)) return -1;
   if (M <= 0) return 0;
-  gn::Args p;
-  p.x = (const bf16_t*)x; p.ldx = K; p.w = (const bf16_t*)w; p.ldw = K; p.bias = (const bf16_t*)bias; p.res = (const bf16_t*)res; p.ldr = N;
-  p.lw = (const bf16_t*)lw; p.lb = (const bf16_t*)lb; p.y = (bf16_t*)y; p.ldy = N; p.M = M; p.K = K; p.eps = eps;
-  const dim3 grid((M + rows - 1) / rows), block(512);
-  if (rows == 64) hipLaunchKernelGGL((gn::gemm_norm_kernel<8, 4, 3>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((gn::gemm_norm_kernel<4, 4, 3>), grid, block, 0, stream, p);
+  auto launch = [&](int m0, int n, int tile) {
+    gn::Args p;
+    p.x = (const bf16_t*)x + (long)m0 * K; p.ldx = K; p.w = (const bf16_t*)w; p.ldw = K; p.bias = (const bf16_t*)bias;
+    p.res = (const bf16_t*)res + (long)m0 * N; p.ldr = N; p.lw = (const bf16_t*)lw; p.lb = (const bf16_t*)lb; p.y = (bf16_t*)y + (long)m0 * N;
+    p.ldy = N; p.M = n; p.K = K; p.eps = eps;
+    const dim3 grid((n + tile - 1) / tile), block(512);
+    if (N == 768 && tile == 64) hipLaunchKernelGGL((gn::gemm_norm_kernel<8, 4, 6>), grid, block, 0, stream, p);
+    else if (N == 768) hipLaunchKernelGGL((gn::gemm_norm_kernel<8, 6, 6>), grid, block, 0, stream, p);
+    else if (tile == 64) hipLaunchKernelGGL((gn::gemm_norm_kernel<8, 4, 3>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((gn::gemm_norm_kernel<4, 4, 3>), grid, block, 0, stream, p);
+  };
+  if (first) launch(0, first, large);
+  if (M > first) launch(first, M - first, rows);
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -663,7 +663,7 @@ def _few_rows_encoder(heads, seed, **kw):
     from rag_tl_domainllm_optimizer_amd import models
     import dataclasses
 
-    cfg = dataclasses.replace(models.resolve_preset("minilm-l6"), num_layers=3, num_heads=heads, head_dim=384 // heads, **kw)
+    cfg = dataclasses.replace(models.resolve_preset("minilm-l6"), num_layers=3, num_heads=heads, **{"head_dim": 384 // heads, **kw})
     m = models.SentenceEncoder(cfg, device=DEV, dtype=torch.bfloat16, init=False).eval()
     g = torch.Generator(device=DEV).manual_seed(seed)
     with torch.no_grad():
@@ -981,3 +981,42 @@ def test_upload_under_a_default_device():
     for g in got:
         assert g.device.type == "cuda" and torch.equal(g.cpu(), torch.from_numpy(src))
     assert batch.ids.tolist() == [5, 6, 7] + [8] * 40 and batch.pos.tolist() == [0, 1, 2] + list(range(3, 43))
+
+
+@pytest.mark.parametrize("rows", [64, 96])
+@pytest.mark.parametrize("M,K", [(1, 64), (63, 128), (64, 192), (65, 384), (95, 320), (96, 768), (97, 64), (193, 448), (24580, 128)])
+def test_product_and_norm_of_768_columns_in_one_launch(M, K, rows):
+    """As with 384 columns: the bits of product and norm, close to 64 bits; NaN, infinite and huge rows stay their own."""
+    C = ops.native()
+    g = torch.Generator(device=DEV).manual_seed(M + K + rows)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(768, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    bias, lb = (torch.randn(768, generator=g, device=DEV).bfloat16() for _ in range(2))
+    lw = (1 + 0.1 * torch.randn(768, generator=g, device=DEV)).bfloat16()
+    res = torch.randn(M, 768, generator=g, device=DEV).bfloat16()
+    got = C.linear_norm(x, w, bias, res, lw, lb, 1e-12, rows)
+    want = ops.layer_norm(C.gemm_big(x, w, 0, 0, bias=bias), lw, lb, 1e-12, residual=res)[0]
+    assert torch.equal(got, want)
+    # product and sum are rounded to bf16 (2^-9 of values below 8) ahead of a division by about 1.4, the result (below 8) once more
+    h = x.double() @ w.double().t() + bias.double() + res.double()
+    ref = torch.nn.functional.layer_norm(h, (768,), lw.double(), lb.double(), 1e-12)
+    assert (got.double() - ref).abs().max().item() < 3 * 8 * 2 ** -9
+    if M < 60:
+        return
+    x[5, 3], res[17, 700], res[M - 1] = float("nan"), float("inf"), 1e30 * torch.sign(res[M - 1].float()).bfloat16()
+    got = C.linear_norm(x, w, bias, res, lw, lb, 1e-12, rows)
+    want2 = ops.layer_norm(C.gemm_big(x, w, 0, 0, bias=bias), lw, lb, 1e-12, residual=res)[0]
+    torch.testing.assert_close(got, want2, rtol=0, atol=0, equal_nan=True)
+    keep = [i for i in range(min(M - 1, 200)) if i not in (5, 17)]
+    assert got[5].isnan().all() and torch.equal(got[keep], want[keep])
+
+
+# 768 columns, K of 768 and 3072: around the row counts where the rule changes between product and norm, tiles of 64, of 96, and both
+@pytest.mark.parametrize("lens", [[7100], [7200], [10300], [10400], [16384], [16385], [21800], [20000, 4576], [24577], [34001], [41000], [46000]])
+def test_encoder_of_768_columns_where_products_take_the_norm(lens):
+    """The bits of the forward op by op."""
+    m, inputs = _few_rows_encoder(12, sum(lens), hidden_size=768, intermediate_size=3072, head_dim=64)
+    ids, pos, off, longest = inputs(lens)
+    out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
+    assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(len(lens), device=DEV))
+    assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
