@@ -101,6 +101,8 @@ int rt_adamw_mixed(float*, const void*, long, const float*, float*, float*, void
 int rt_pool_norm(const void*, const int*, const long*, long, int, int, int, int, float*, const long*, long, hipStream_t);
 int rt_scatter_scaled(const long*, int, long, hipStream_t);
 int rt_lora_grad_accum(const long*, int, long, hipStream_t);
+int rt_ivf_coarse(const float*, int, int, const void*, int, const float*, int, int, void*, float*, hipStream_t);
+int rt_topk_index(const float*, long, long, int, int, int*, hipStream_t);
 int rt_topk(const float*, long, long, int, int, const long*, long, int, float*, long*, hipStream_t);
 int rt_segment_mean(const float*, int, const long*, const int*, int, int, float*, hipStream_t);
 int rt_ivf_by_list(int, int, int, int, int, long);
@@ -1544,6 +1546,37 @@ std::vector<Tensor> topk(const Tensor& scores, int64_t k, const optional<Tensor>
   return {vals, ids};
 }
 
+// (q in bf16, scores [nq, nlist] q cen^T - pen) of up to 16 fp32 queries, with gemm's bits; empty where that takes another form
+std::vector<Tensor> ivf_coarse(const Tensor& q, const Tensor& cen, int64_t nlist, const optional<Tensor>& pen) {
+  CHECK_CUDA(q); CHECK_F32(q); CHECK_CUDA(cen); CHECK_BF16(cen);
+  TORCH_CHECK(q.dim() == 2 && cen.dim() == 2 && cen.size(1) == q.size(1) && nlist <= cen.size(0) && q.is_contiguous() && cen.is_contiguous(),
+              "ivf_coarse: operands");
+  const int64_t nq = q.size(0), d = q.size(1), rows = cen.size(0);
+  if (pen) {
+    CHECK_CUDA(*pen); CHECK_F32(*pen);
+    TORCH_CHECK(pen->is_contiguous() && pen->numel() == nlist, "ivf_coarse: pen");
+  }
+  if (nq < 1 || nq > 16 || rows % 16 || d % 64 || d > INT_MAX || rows > INT_MAX) return {};
+  int grp = 1;
+  const int parts = rt_gemm_nt_parts((int)nq, (int)rows, (int)d, &grp);
+  auto qb = at::empty({nq, d}, cen.options());
+  auto score = at::empty({nq, nlist}, q.options());
+  const int rc = rt_ivf_coarse(q.data_ptr<float>(), (int)nq, (int)d, cen.data_ptr(), (int)nlist, (const float*)opt_ptr(pen), parts, grp,
+                               qb.data_ptr(), score.data_ptr<float>(), cur_stream());
+  if (rc == -1) return {};
+  check_rc(rc, "ivf_coarse");
+  return {qb, score};
+}
+
+// the indices of topk, int32
+Tensor topk_index(const Tensor& scores, int64_t k) {
+  CHECK_CUDA(scores); CHECK_F32(scores); CHECK_ROWS(scores);
+  auto out = at::empty({scores.size(0), k}, scores.options().dtype(at::kInt));
+  check_rc(rt_topk_index(scores.data_ptr<float>(), scores.stride(0), scores.size(0), (int)scores.size(1), (int)k, out.data_ptr<int>(), cur_stream()),
+           "topk_index");
+  return out;
+}
+
 std::vector<Tensor> ivf_scan(const Tensor& q_, const Tensor& probes, const Tensor& lstart, const Tensor& lsize,
                              const Tensor& vecs, const Tensor& ids, const optional<Tensor>& sqnorm, bool l2,
                              int64_t maxlen) {
@@ -1788,6 +1821,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("adamw_apply", &adamw_apply);
   m.def("grad_sumsq", &grad_sumsq);
   m.def("pool_norm", &pool_norm, py::arg("x"), py::arg("lengths"), py::arg("normalize"), py::arg("off") = py::none());
+  m.def("ivf_coarse", &ivf_coarse, py::arg("q"), py::arg("cen"), py::arg("nlist"), py::arg("pen") = py::none());
+  m.def("topk_index", &topk_index, py::arg("scores"), py::arg("k"));
   m.def("topk", &topk, py::arg("scores"), py::arg("k"), py::arg("idmap") = py::none(), py::arg("finite") = false);
   m.def("ivf_scan", &ivf_scan);
   m.def("ivf_by_list", [](int64_t nq, int64_t nprobe, int64_t nlist, int64_t d, int64_t maxlen, int64_t total) {

@@ -83,14 +83,22 @@ struct TopkShared {
   int ci[TOPK_CAND];
 };
 
-__device__ __forceinline__ void topk_write(float v, int idx, int k, int at, long row, const long* idmap, long ldmap,
-                                           int finite, float* out_v, long* out_i) {
-  out_v[row * k + at] = v;
-  long id = idx == 0x7fffffff ? -1 : idx;
-  if (idmap && id >= 0) id = idmap[row * ldmap + id];
-  if (finite && !(fabsf(v) < INFINITY)) id = -1;
-  out_i[row * k + at] = id;
-}
+// where a row's k results go: values and ids, the candidate's index (-1: none) through idmap if there is one
+struct TopkOut {
+  const long* idmap; int finite;  // of the row
+  float* v; long* i;
+  __device__ __forceinline__ long id(int idx) const { return idx == 0x7fffffff ? -1 : idmap ? idmap[idx] : idx; }
+  __device__ __forceinline__ void put(int at, float val, long id) const {
+    v[at] = val;
+    i[at] = finite && !(fabsf(val) < INFINITY) ? -1 : id;
+  }
+};
+// the indices alone
+struct TopkIndices {
+  int* i;
+  __device__ __forceinline__ long id(int idx) const { return idx == 0x7fffffff ? -1 : idx; }
+  __device__ __forceinline__ void put(int at, float, long id) const { i[at] = (int)id; }
+};
 
 // A row with more candidates than the list holds (plateaus, fewer than K finite scores): 4-pass radix select of the K-th
 // key, then exactly K entries in cv / ci: the fewer than K above it, and of its ties those of the lowest indices
@@ -168,15 +176,11 @@ __device__ void topk_select(const float* s, int N, int K, TopkShared& sh) {
 // Rows with more than TOPK_CAND candidates go through topk_select first.
 // NT: a wave where its 64 maxima suffice (k <= 32) and hold 16 elements each at most (k-means assignment: 65536 rows
 // of 512), 1024 threads for long rows, 256 between.
-template <int NT>
-__global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scores, long ld, int N, int k,
-                                                  const long* __restrict__ idmap, long ldmap, int finite,
-                                                  float* __restrict__ out_v, long* __restrict__ out_i) {
+template <int NT, typename Out>
+__device__ __forceinline__ void topk_row(const float* s, int N, int k, const Out& out) {
   __shared__ TopkShared sh;
   __shared__ uint32_t tmax[NT];
   __shared__ unsigned char keep[TOPK_CAND];
-  const long row = blockIdx.x;
-  const float* s = scores + row * ld;
   const int tid = threadIdx.x, lane = tid & 63, K = min(k, N);
   uint32_t km = 0;
   // eight loads in flight, at the end four, those past it of the last element
@@ -247,13 +251,13 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
     topk_select<NT>(s, N, K, sh);
     n = K;
   }
-  for (int i = K + tid; i < k; i += NT) topk_write(-INFINITY, 0x7fffffff, k, i, row, idmap, ldmap, finite, out_v, out_i);
+  for (int i = K + tid; i < k; i += NT) out.put(i, -INFINITY, -1);
   if (n <= 64) {  // a candidate a lane, as below
     if (tid >= 64) return;
     const bool in = lane < n;
     const float v = in ? sh.cv[lane] : 0.f;
     const int idx = in ? sh.ci[lane] : 0;
-    const long id = idmap ? in ? idmap[row * ldmap + idx] : 0 : idx;
+    const long id = in ? out.id(idx) : 0;
     const uint32_t raw = okey(v), key = okey(v + 0.f);
     int above = 0, at = 0;
     for (int i = 0; i < n; ++i) above += (uint32_t)__builtin_amdgcn_readlane((int)raw, i) > raw;
@@ -264,10 +268,7 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
       const int oi = __builtin_amdgcn_readlane(idx, i);
       at += o > key || (o == key && oi < idx);
     }
-    if (keeps && at < K) {
-      out_v[row * k + at] = v;
-      out_i[row * k + at] = finite && !(fabsf(v) < INFINITY) ? -1 : id;
-    }
+    if (keeps && at < K) out.put(at, v, id);
     return;
   }
   // those with fewer than K keys above their own, then their places by value and index
@@ -289,8 +290,82 @@ __global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scor
         const uint32_t o = okey(sh.cv[i] + 0.f);
         at += keep[i] && (o > key || (o == key && sh.ci[i] < idx));
       }
-      if (at < K) topk_write(v, idx, k, at, row, idmap, ldmap, finite, out_v, out_i);
+      if (at < K) out.put(at, v, out.id(idx));
     }
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void topk_kernel(const float* __restrict__ scores, long ld, int N, int k,
+                                                  const long* __restrict__ idmap, long ldmap, int finite,
+                                                  float* __restrict__ out_v, long* __restrict__ out_i) {
+  const long row = blockIdx.x;
+  topk_row<NT>(scores + row * ld, N, k, TopkOut{idmap ? idmap + row * ldmap : nullptr, finite, out_v + row * k, out_i + row * k});
+}
+
+// The indices alone, in 32 bits: the lists that a scan probes
+template <int NT>
+__global__ __launch_bounds__(NT) void topk_index_kernel(const float* __restrict__ scores, long ld, int N, int k, int* __restrict__ out) {
+  const long row = blockIdx.x;
+  topk_row<NT>(scores + row * ld, N, k, TopkIndices{out + row * k});
+}
+
+// Scores of up to 16 queries with the centroids, q cen^T - pen, from fp32 queries, which go on in bf16 to the scan. A workgroup has 16 centroids,
+// a wave one of the product's parts of K; parts and groups are summed in the product's order: the same bits. Bound by one trip to
+// memory; rounding and product took two launches.
+struct CoarseArgs {
+  const float* q; int nq, d; const bf16_t* cen; int nlist; const float* pen;
+  int parts, grp;
+  bf16_t* qb; float* score;
+};
+__global__ __launch_bounds__(1024) void ivf_coarse_kernel(CoarseArgs a) {
+  __shared__ float red[16][4][65];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r16 = lane & 15;
+  const int part = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nc = a.d / 64, c0 = (int)((long)part * nc / a.parts), c1 = (int)((long)(part + 1) * nc / a.parts);
+  const bf16_t* const x = a.cen + (16L * blockIdx.x + r16) * a.d + 8 * g;  // rows up to a multiple of 16 are there
+  const long qrow = min(r16, a.nq - 1);
+  const float* const q = a.q + qrow * a.d + 8 * g;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  constexpr int U = 2;
+  for (int c = c0; c < c1; c += U) {
+    uint4 xv[U][2];
+    float4 qv[U][2][2];
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = 64 * min(c + i, c1 - 1) + 32 * h;
+        xv[i][h] = *(const uint4*)(x + k);
+        qv[i][h][0] = *(const float4*)(q + k);
+        qv[i][h][1] = *(const float4*)(q + k + 4);
+      }
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (c + i >= c1) continue;
+        const float4 lo = qv[i][h][0], hi = qv[i][h][1];
+        const uint4 y = make_uint4(pack2bf(lo.x, lo.y), pack2bf(lo.z, lo.w), pack2bf(hi.x, hi.y), pack2bf(hi.z, hi.w));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, y), __builtin_bit_cast(bf16x8, xv[i][h]), acc, 0, 0, 0);
+        if (blockIdx.x == 0 && r16 < a.nq) *(uint4*)(a.qb + qrow * a.d + 64 * (c + i) + 32 * h + 8 * g) = y;
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[part][r][lane] = acc[r];
+  __syncthreads();
+  // acc[r] of a lane: query 4 g + r, centroid r16
+  if (tid >= 256) return;
+  const int r = tid >> 6, query = 4 * g + r, c = 16 * (int)blockIdx.x + r16;
+  float v = 0.f, u = 0.f;
+  for (int p = 0, in = 0; p < a.parts; ++p) {
+    const float t = red[p][r][lane];
+    u = in ? u + t : t;
+    if (++in == a.grp) {
+      v = a.parts == a.grp ? u : v + u;
+      in = 0;
+    }
+  }
+  if (query < a.nq && c < a.nlist) a.score[(long)query * a.nlist + c] = a.pen ? v - a.pen[c] : v;
 }
 
 // IVF list scan: for query qi and its probe p (list L = probes[qi, p]), score every vector of the
@@ -622,6 +697,29 @@ extern "C" int rt_topk(const float* scores, long ld, long nq, int N, int k, cons
   else if (k <= 128 && N <= 4096) TOPK_LAUNCH(256);
   else TOPK_LAUNCH(1024);
 #undef TOPK_LAUNCH
+  RT_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int rt_topk_index(const float* scores, long ld, long nq, int N, int k, int* out, hipStream_t stream) {
+  if (k > TOPK_CAND / 2 || k > N) return -1;
+  if (nq == 0 || k <= 0) return 0;
+#define TOPK_LAUNCH(NT) hipLaunchKernelGGL(topk_index_kernel<NT>, dim3(nq), dim3(NT), 0, stream, scores, ld, N, k, out)
+  if (k <= 32 && N <= 1024) TOPK_LAUNCH(64);
+  else if (k <= 128 && N <= 4096) TOPK_LAUNCH(256);
+  else TOPK_LAUNCH(1024);
+#undef TOPK_LAUNCH
+  RT_LAUNCH_CHECK();
+  return 0;
+}
+
+// score [nq, nlist] and q in bf16, see ivf_coarse_kernel; cen: rows [nlist up to a multiple of 16, d]. -1: not for this kernel.
+extern "C" int rt_ivf_coarse(const float* q, int nq, int d, const void* cen, int nlist, const float* pen, int parts, int grp, void* qb,
+                             float* score, hipStream_t stream) {
+  if (nq < 1 || nq > 16 || d < 64 || d % 64 || nlist < 1 || parts < 4 || parts > 16 || grp < 1 || parts % grp) return -1;
+  if ((uintptr_t)q % 16 || (uintptr_t)cen % 16) return -1;
+  const CoarseArgs a{q, nq, d, (const bf16_t*)cen, nlist, pen, parts, grp, (bf16_t*)qb, score};
+  hipLaunchKernelGGL(ivf_coarse_kernel, dim3((nlist + 15) / 16), dim3(64 * parts), 0, stream, a);
   RT_LAUNCH_CHECK();
   return 0;
 }

@@ -9,6 +9,7 @@ import torch.nn.functional as F
 
 from . import reference as ref
 from ._ext import native, on_gpu
+from .linear import batch_invariant_on, gemm
 
 
 # ------------------------------------------------------------------------------------ tables made on the host
@@ -195,6 +196,22 @@ def topk(scores: torch.Tensor, k: int, idmap=None, finite: bool = False):
         return native().topk(scores if scores.stride(-1) == 1 else scores.contiguous(), k, idmap, finite)
     v, i = ref.topk(scores, k, idmap)
     return v, torch.where(torch.isfinite(v), i, torch.full_like(i, -1)) if finite else i
+
+
+def ivf_probes(q, cen, nlist: int, k: int, pen=None):
+    """The ``k`` lists that each query probes on a GPU, the best of its scores q cen[:nlist]^T - pen -> (q in bf16, int32 indices
+    [nq, k]). Up to 16 fp32 queries are rounded and multiplied in one launch, with :func:`gemm`'s bits."""
+    q = q.contiguous()
+    few = q.dtype == torch.float32 and q.dim() == 2 and 0 < q.shape[0] <= 16 and not batch_invariant_on()
+    both = native().ivf_coarse(q, cen, nlist, pen) if few else None
+    if both:
+        q, s = both
+    else:
+        q = q.to(torch.bfloat16)
+        s = gemm(q, cen, out_f32=True)[:, :nlist]  # the operand's padding rows stay out of the selection
+        if pen is not None:
+            s.sub_(pen)
+    return q, native().topk_index(s, k) if k <= 512 else topk(s, k)[1].int()
 
 
 def ivf_scan(q, probes, lstart, lsize, vecs, ids, maxlen, sqnorm=None, l2: bool = False):

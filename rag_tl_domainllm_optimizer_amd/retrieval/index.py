@@ -277,15 +277,16 @@ class IVFIndex:
         nprobe = min(nprobe or self.nprobe, self.nlist)
         q = q.to(self.device)
         l2 = self.metric == "l2"
-        probes = self._coarse(q, nprobe)
         maxlen = max(self.maxlen, 1)
         kk = min(k, nprobe * maxlen)
         if self.gpu:
-            cand, cid = ops.ivf_scan(q.to(self.dtype), probes, self.lstart, self.lsize, self.vecs, self.ids, maxlen,
+            qb, probes = ops.ivf_probes(q, self._cen_op, self.centroids.shape[0], nprobe, self._pen if l2 else None)
+            cand, cid = ops.ivf_scan(qb, probes, self.lstart, self.lsize, self.vecs, self.ids, maxlen,
                                      self.sqnorm, l2)
             v, out_ids = ops.topk(cand, kk, cid, finite=True)
         else:
             # same algorithm as the list-scan kernel: [nq, nprobe, maxlen] candidate slots
+            probes = self._coarse(q, nprobe)
             j = torch.arange(maxlen)
             slot = self.lstart.long()[probes][..., None] + j
             valid = j < self.lsize.long()[probes][..., None]

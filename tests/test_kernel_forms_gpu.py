@@ -1020,3 +1020,27 @@ def test_encoder_of_768_columns_where_products_take_the_norm(lens):
     out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
     assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(len(lens), device=DEV))
     assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
+
+
+@pytest.mark.parametrize("nlist,d", [(1, 64), (15, 128), (16, 256), (17, 320), (130, 384), (512, 384), (1000, 768), (300, 2048), (2000, 1088)])
+@pytest.mark.parametrize("l2", [False, True])
+def test_probes_of_few_queries(nlist, d, l2):
+    """The lists that product and top-k find, and the query that rounding alone gives, on both sides of the 16 queries of one launch: repeated
+    centroids (ties), a NaN query, queries that are not fp32 or not contiguous, all lists, more than the selection kernel takes."""
+    g = torch.Generator(device=DEV).manual_seed(nlist + d)
+    cen = torch.randn((nlist + 127) // 128 * 128, d, generator=g, device=DEV).bfloat16()
+    cen[nlist // 2] = cen[0]
+    pen = torch.randn(nlist, generator=g, device=DEV) if l2 else None
+    for nq in (1, 3, 16, 17):
+        q = torch.randn(nq, 2 * d, generator=g, device=DEV)
+        q[nq - 1, 0] = float("nan")
+        for x in (q[:, :d].contiguous(), q[:, :d], q[:, :d].bfloat16(), q[:, 1:d + 1]):
+            for k in {1, min(16, nlist), nlist}:
+                s = ops.gemm(x.contiguous().bfloat16(), cen, out_f32=True)[:, :nlist]
+                if l2:
+                    s = s - pen
+                qb, got = ops.ivf_probes(x, cen, nlist, k, pen)
+                assert torch.equal(qb.view(torch.int16), x.contiguous().bfloat16().view(torch.int16))
+                assert got.dtype == torch.int32
+                fine = slice(0, nq - 1) if x.isnan().any() else slice(0, nq)
+                assert torch.equal(got[fine].long(), ops.topk(s, k)[1][fine])
