@@ -59,7 +59,8 @@ int rt_swiglu_bwd(const void*, const void*, void*, long, int, hipStream_t);
 int rt_embed(const void*, const long*, const void*, const long*, void*, long, int, hipStream_t);
 int rt_rows_scatter(const void*, long, const int*, void*, long, int, long, hipStream_t);
 int rt_attn_fwd(const void*, long, const void*, long, const void*, long, void*, long, float*, const int*, const int*,
-                const float*, int, int, int, int, int, int, int, int, int, float, hipStream_t);
+                const float*, int, int, int, int, int, int, int, int, int, float, const int*, long, hipStream_t);
+int rt_kv_append_rows(const void*, long, const int*, int, int, int, int, int, void*, void*, int, long, hipStream_t);
 int rt_gemm_image(const void*, long, const void*, void*, long, int, int, int, int, int, int, const float*, hipStream_t);
 int rt_attn_packed(const void*, long, const void*, long, const void*, long, void*, long, const long*, const float*, int, int,
                    int, int, int, int, float, hipStream_t);
@@ -911,6 +912,21 @@ Tensor embed(const Tensor& table, const Tensor& ids, const optional<Tensor>& pta
 }
 
 // src [N, H] (row stride % 8 == 0) -> out [R, H]: out[r] = src[inv[r]] or zeros where inv[r] < 0
+// K and V of packed rows into cache slots [0, S) (see kv_append_rows_kernel); inv int32 [B S]
+void kv_append_rows(const Tensor& qkv, const Tensor& inv, int64_t S, int64_t Hq, Tensor kc, Tensor vc) {
+  CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_ROWS(qkv); CHECK_ALIGN16(qkv); CHECK_CUDA(inv); CHECK_I32(inv);
+  for (const Tensor* t : {&kc, &vc}) {
+    CHECK_CUDA(*t); CHECK_BF16(*t); CHECK_ALIGN16(*t);
+    TORCH_CHECK(t->dim() == 4 && t->is_contiguous() && t->sizes() == kc.sizes(), "kv_append_rows: caches [B, Hkv, Smax, D]");
+  }
+  const int64_t Hkv = kc.size(1), Smax = kc.size(2), D = kc.size(3);
+  TORCH_CHECK(S > 0 && S <= Smax && inv.is_contiguous() && inv.numel() % S == 0 && inv.numel() / S <= kc.size(0) && D % 8 == 0 &&
+                  qkv.stride(0) % 8 == 0 && qkv.size(1) >= (Hq + 2 * Hkv) * D, "kv_append_rows: sizes");
+  check_rc(rt_kv_append_rows(qkv.data_ptr(), qkv.stride(0), inv.data_ptr<int>(), (int)(inv.numel() / S), (int)S, (int)Hq, (int)Hkv, (int)D,
+                             kc.data_ptr(), vc.data_ptr(), (int)Smax, qkv.size(0), cur_stream()),
+           "kv_append_rows");
+}
+
 Tensor rows_scatter(const Tensor& src, const Tensor& inv, int64_t R) {
   CHECK_CUDA(src); CHECK_BF16(src); CHECK_CUDA(inv);
   TORCH_CHECK(src.dim() == 2 && src.stride(1) == 1 && src.stride(0) % 8 == 0, "rows_scatter: [N, H] rows expected");
@@ -928,12 +944,18 @@ Tensor rows_scatter(const Tensor& src, const Tensor& inv, int64_t R) {
 std::vector<Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, int64_t B, int64_t Sq, int64_t Sk,
                              int64_t Hq, int64_t Hkv, int64_t D, bool causal, int64_t window, double scale,
                              const optional<Tensor>& kv_start, const optional<Tensor>& kv_len,
-                             const optional<Tensor>& rel_bias, int64_t rb_L, bool need_lse) {
+                             const optional<Tensor>& rel_bias, int64_t rb_L, bool need_lse, const optional<Tensor>& first) {
   CHECK_CUDA(q); CHECK_BF16(q); CHECK_BF16(k); CHECK_BF16(v); CHECK_ROWS(q); CHECK_ROWS(k); CHECK_ROWS(v);
-  TORCH_CHECK(q.size(0) == B * Sq && k.size(0) == B * Sk && v.size(0) == B * Sk, "attn_fwd: row counts");
+  if (first) {  // rows of real positions only, see AttnArgs
+    CHECK_CUDA(*first); CHECK_I32(*first);
+    TORCH_CHECK(first->is_contiguous() && first->numel() == B && Sq == Sk && !need_lse && k.size(0) == q.size(0) && v.size(0) == q.size(0),
+                "attn_fwd: packed rows");
+  } else {
+    TORCH_CHECK(q.size(0) == B * Sq && k.size(0) == B * Sk && v.size(0) == B * Sk, "attn_fwd: row counts");
+  }
   TORCH_CHECK(Hq % Hkv == 0, "attn_fwd: Hq % Hkv");
   TORCH_CHECK(q.stride(0) % 8 == 0 && k.stride(0) % 8 == 0 && v.stride(0) % 8 == 0, "attn_fwd: strides % 8");
-  auto o = at::empty({B * Sq, Hq * D}, q.options());
+  auto o = at::empty({q.size(0), Hq * D}, q.options());
   Tensor lse = need_lse ? at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat)) : Tensor();
   if (kv_start.has_value() && kv_start->defined()) CHECK_I32(*kv_start);
   if (kv_len.has_value() && kv_len->defined()) CHECK_I32(*kv_len);
@@ -944,7 +966,8 @@ std::vector<Tensor> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, 
   check_rc(rt_attn_fwd(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), o.data_ptr(),
                        o.stride(0), need_lse ? lse.data_ptr<float>() : nullptr, (const int*)opt_ptr(kv_start),
                        (const int*)opt_ptr(kv_len), (const float*)opt_ptr(rel_bias), (int)rb_L, (int)B, (int)Sq,
-                       (int)Sk, (int)Hq, (int)Hkv, (int)D, causal ? 1 : 0, (int)window, (float)scale, cur_stream()),
+                       (int)Sk, (int)Hq, (int)Hkv, (int)D, causal ? 1 : 0, (int)window, (float)scale, (const int*)opt_ptr(first),
+                       q.size(0), cur_stream()),
            "attn_fwd");
   return {o, lse};
 }
@@ -1803,7 +1826,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows", &few_rows, "act(x w^T + b) of up to 32 rows, normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);
-  m.def("attn_fwd", &attn_fwd);
+  m.def("attn_fwd", &attn_fwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("B"), py::arg("Sq"), py::arg("Sk"), py::arg("Hq"), py::arg("Hkv"),
+        py::arg("D"), py::arg("causal"), py::arg("window"), py::arg("scale"), py::arg("kv_start"), py::arg("kv_len"), py::arg("rel_bias"),
+        py::arg("rb_L"), py::arg("need_lse"), py::arg("first") = py::none());
+  m.def("kv_append_rows", &kv_append_rows, py::arg("qkv"), py::arg("inv"), py::arg("S"), py::arg("Hq"), py::arg("k_cache"), py::arg("v_cache"));
   m.def("attn_decode", &attn_decode);
   m.def("attn_bwd", &attn_bwd, "flash attention backward (RoPE backward optionally fused into dQ / dK)",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("dout"), py::arg("lse"), py::arg("dq"),

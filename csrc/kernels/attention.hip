@@ -111,6 +111,7 @@ struct AttnArgs {
   int lpt;                    // heaviest-first dispatch order (attn_block_xyz; causal grids)
   int nx, gh, groups;         // packed form: query tiles, heads of a group, groups of all sequences
   const long* off;            // packed form: sequence b is rows [off[b], off[b + 1]) of Sq in all
+  const int* first; long rows; // forward without pad rows: position s >= kv_start[b] of sequence b is row first[b] + s of `rows` (else null)
 };
 
 // byte offset of 16-B chunk c of row r in a K-style (row-read) tile image
@@ -145,6 +146,10 @@ __device__ __forceinline__ int v_off(int r, int c) {
 //
 // Q64 (NU = 1, 4 waves of 16 rows): 64 positions of one head per workgroup — the same causal
 // saving for heads that share no K / V (MHA, e.g. Llama-2-13B), bitwise the 128-row form too.
+//
+// a.first: rows of real positions only, tiled by position all the same (masked keys are read from a real row instead of a pad's zeros: the
+// same bits). 32 prompts of 90 to 320 tokens had needed a grid filled, and read for the cache, and results gathered: 79 us a layer beside 87 here, now 13
+// beside 83 (Mistral-7B, four layers, 8247 -> 7985).
 template <int D, int NU = 2, bool HP = false, bool Q64 = false>
 __global__ __launch_bounds__(Q64 ? 256 : 64 * 8 / NU, D == 128 ? 2 : (D == 64 ? 3 : 4))
 void attn_fwd_kernel(AttnArgs a) {
@@ -179,13 +184,18 @@ void attn_fwd_kernel(AttnArgs a) {
   int kbeg = start;
   if (a.window > 0) kbeg = max(kbeg, qblk0 - a.window + 1);
   kbeg = max(kbeg, 0) & ~63;
+  // rows of position 0; the positions that have one
+  const long qbase = a.first ? (long)a.first[b] : (long)b * a.Sq, kbase = a.first ? qbase : (long)b * a.Sk;
+  const int plo = a.first ? (int)max((long)max(start, 0), -qbase) : 0;
+  const int qhi = a.first ? (int)min(a.Sq - 1L, a.rows - 1 - qbase) : a.Sq - 1, khi = a.first ? qhi : a.Sk - 1;
+  if (a.first && (qlast < plo || qhi < plo)) return;
 
   // Q fragments (B operand of S^T = K·Q^T): lane holds Q[q0+16u+r16][32s + 8g .. +8]
   bf16x8 qf[NU][DS];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int qrow = min(q0 + 16 * u + r16, a.Sq - 1);
-    const bf16_t* qp = a.q + ((long)b * a.Sq + qrow) * a.ldq + (long)h * D + 8 * g;
+    const int qrow = min(max(q0 + 16 * u + r16, plo), qhi);
+    const bf16_t* qp = a.q + (qbase + qrow) * a.ldq + (long)h * D + 8 * g;
 #pragma unroll
     for (int s = 0; s < DS; ++s) qf[u][s] = *(const bf16x8*)(qp + 32 * s);
   }
@@ -212,13 +222,13 @@ void attn_fwd_kernel(AttnArgs a) {
   constexpr int CPT = 64 * NCH / NT;  // chunks per thread per tensor (4 for D=128, 256 threads)
   constexpr int KSTEP = NT / NCH;     // key stride between a thread's chunks
   const int lc = tid % NCH, lkey = tid / NCH;
-  const bf16_t* kb = a.k + (long)b * a.Sk * a.ldk + (long)hk * D + lc * 8;
-  const bf16_t* vb = a.v + (long)b * a.Sk * a.ldv + (long)hk * D + lc * 8;
+  const bf16_t* kb = a.k + kbase * a.ldk + (long)hk * D + lc * 8;
+  const bf16_t* vb = a.v + kbase * a.ldv + (long)hk * D + lc * 8;
   u32x4 kreg[CPT], vreg[CPT];
   auto load_tile = [&](int kv0) {
 #pragma unroll
     for (int r = 0; r < CPT; ++r) {
-      const long kk = min(kv0 + lkey + KSTEP * r, a.Sk - 1);
+      const long kk = min(max(kv0 + lkey + KSTEP * r, plo), khi);
       kreg[r] = *(const u32x4*)(kb + kk * a.ldk);
       vreg[r] = *(const u32x4*)(vb + kk * a.ldv);
     }
@@ -378,8 +388,8 @@ void attn_fwd_kernel(AttnArgs a) {
     // HP: staging row 32 w + r = position qblk0 + r of head 4 hk + w
     const int qq = HP ? qblk0 + (row & 31) : qblk0 + row;
     const int hh = HP ? hk * 4 + (row >> 5) : h;
-    if (qq < a.Sq)
-      *(uint4*)(a.o + ((long)b * a.Sq + qq) * a.ldo + (long)hh * D + c * 8) = *(const uint4*)(Os + row * OROW + c * 8);
+    if (qq <= qhi && qq >= plo)
+      *(uint4*)(a.o + (qbase + qq) * a.ldo + (long)hh * D + c * 8) = *(const uint4*)(Os + row * OROW + c * 8);
   }
 }
 
@@ -2175,9 +2185,11 @@ static int attn_lpt_on(dim3 grid, int causal) {
 
 extern "C" int rt_attn_fwd(const void* q, long ldq, const void* k, long ldk, const void* v, long ldv, void* o, long ldo,
                            float* lse, const int* kv_start, const int* kv_len, const float* rel_bias, int rb_L, int B,
-                           int Sq, int Sk, int Hq, int Hkv, int D, int causal, int window, float scale,
-                           hipStream_t stream) {
-  AttnArgs a;
+                           int Sq, int Sk, int Hq, int Hkv, int D, int causal, int window, float scale, const int* first,
+                           long rows, hipStream_t stream) {
+  if (first && (Sq != Sk || lse || rel_bias)) return -1;
+  AttnArgs a = {};
+  a.first = first; a.rows = rows;
   a.q = (const bf16_t*)q; a.ldq = ldq; a.k = (const bf16_t*)k; a.ldk = ldk; a.v = (const bf16_t*)v; a.ldv = ldv;
   a.o = (bf16_t*)o; a.ldo = ldo; a.lse = lse; a.kv_start = kv_start; a.kv_len = kv_len; a.rel_bias = rel_bias;
   a.rb_L = rb_L; a.B = B; a.Sq = Sq; a.Sk = Sk; a.Hq = Hq; a.Hkv = Hkv; a.causal = causal; a.window = window;

@@ -148,6 +148,32 @@ __global__ __launch_bounds__(256) void rows_scatter_kernel(const bf16_t* __restr
   *(uint4*)(out + r * H + c * 8) = v;
 }
 
+// K / V of packed qkv rows into cache slots [0, S): slot s of row b from row inv[b S + s], zeros (a pad's) where that is negative. Two
+// 16-byte accesses a thread, whole cache rows; bound by their bytes: 32 x 320 slots of 8 heads of 128, 6250 of them with rows, 13.2 us, where the grid's fill and the append that
+// read it took 61.
+__global__ __launch_bounds__(256) void kv_append_rows_kernel(const bf16_t* __restrict__ qkv, long ld, const int* __restrict__ inv, int B, int S,
+                                                             int Hq, int Hkv, int D, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, int Smax,
+                                                             long N) {
+  const int nv = D / 8;
+  const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (gid >= (long)B * Hkv * S * nv) return;
+  const int c = gid % nv;
+  const long t = gid / nv;
+  const int s = t % S;
+  const long bh = t / S;
+  const int h = bh % Hkv, j = inv[bh / Hkv * S + s];
+  RT_ASSERT(j < N);
+  uint4 k = make_uint4(0, 0, 0, 0), v = k;
+  if (j >= 0) {
+    const bf16_t* const row = qkv + j * ld + (long)(Hq + h) * D + c * 8;
+    k = *(const uint4*)row;
+    v = *(const uint4*)(row + (long)Hkv * D);
+  }
+  const long to = (bh * Smax + s) * D + c * 8;
+  *(uint4*)(kc + to) = k;
+  *(uint4*)(vc + to) = v;
+}
+
 }  // namespace rt
 
 using namespace rt;
@@ -161,6 +187,17 @@ extern "C" int rt_rows_scatter(const void* src, long lds, const int* inv, void* 
   if (total == 0) return 0;
   hipLaunchKernelGGL(rows_scatter_kernel, dim3(nblocks(total)), dim3(256), 0, stream, (const bf16_t*)src, lds, inv,
                      (bf16_t*)out, R, H, N);
+  RT_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int rt_kv_append_rows(const void* qkv, long ld, const int* inv, int B, int S, int Hq, int Hkv, int D, void* kc, void* vc, int Smax,
+                                 long N, hipStream_t stream) {
+  if (D % 8 != 0 || ld % 8 != 0 || S > Smax) return -1;
+  const long total = (long)B * Hkv * S * (D / 8);
+  if (total == 0) return 0;
+  hipLaunchKernelGGL(kv_append_rows_kernel, dim3(nblocks(total)), dim3(256), 0, stream, (const bf16_t*)qkv, ld, inv, B, S, Hq, Hkv, D,
+                     (bf16_t*)kc, (bf16_t*)vc, Smax, N);
   RT_LAUNCH_CHECK();
   return 0;
 }

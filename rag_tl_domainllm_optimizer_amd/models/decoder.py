@@ -379,8 +379,9 @@ class CausalLM(nn.Module):
         position of every row [B, H] (rows are left-padded so all end at S-1).
 
         ``packed`` = (idx [N] device grid positions, off host row offsets) from ``packed_index``:
-        the projection GEMMs skip the left pads; each layer's qkv is scattered into the zeroed
-        [B*S] grid for RoPE + cache append + attention, and the outputs gathered back."""
+        the GEMMs skip the left pads, and on a GPU so do cache append and attention; on the CPU and with
+        an fp8 cache each layer's qkv is scattered into the zeroed [B*S] grid for RoPE + cache
+        append + attention, and the outputs gathered back."""
         cfg = self.cfg
         B, S = input_ids.shape
         dev = input_ids.device
@@ -395,8 +396,21 @@ class CausalLM(nn.Module):
             x = self.embed_tokens(input_ids.reshape(-1), pos)
         residual = None
         rows_pos = pos.index_select(0, idx) if (idx is not None and cos is not None) else pos
+        in_rows = idx is not None and x.is_cuda and x.dtype == torch.bfloat16 and not getattr(cache, "fp8", False)
+        if in_rows:
+            first = inv.view(B, S)[:, S - 1] - (S - 1)  # the packed row of a row's position 0, were there one
+            last_rows = ops.upload(packed[1][1:] - 1, dev)
         for li, layer in enumerate(self.layers):
             qkv, residual, rotated = layer.attn_in_rope(x, residual, (rows_pos, cos, sin) if cos is not None else None)
+            if in_rows:
+                if cos is not None and not rotated:
+                    ops.rope_qkv_(qkv, rows_pos, cos, sin, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim)
+                o = ops.prefill_attention_rows(qkv, first, inv, S, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim, cache.k[li],
+                                               cache.v[li], cfg.sliding_window, kv_start=ks)
+                if li == len(self.layers) - 1:  # see below
+                    o, residual = o.index_select(0, last_rows), residual.index_select(0, last_rows)
+                x, residual = layer.mlp(o, residual)
+                continue
             if idx is not None:
                 qkv = ops.scatter_rows(qkv, idx, inv, B * S)
             # rotated: q / k came out of the projection's epilogue already rotated (cache append only)

@@ -12,7 +12,7 @@ from .window import WindowDims, window_attention  # noqa: F401
 from .delta import delta_rule  # noqa: F401
 from .latent import LatentDims, latent_attention, yarn_rope_tables  # noqa: F401
 from .attention import (  # noqa: F401
-    attention, attention_packed, decode_attention, decode_step_attention, decode_workspace, flash_attention_packed, gather_rows, packed_inverse, scatter_rows,
+    attention, attention_packed, decode_attention, decode_step_attention, decode_workspace, flash_attention_packed, gather_rows, packed_inverse, prefill_attention_rows, scatter_rows,
     flash_attention_qkv, rope_qkv, rope_qkv_, FP8_KV_D, kv_dequantize, kv_quantize_rows, kv_store_fp8,
 )
 from .misc import (embedding, gae, ivf_probes, ivf_scan, ppo_advantages, pool_normalize, pool_normalize_packed, ppo_loss, row_dot, sample, segment_mean,  # noqa: F401

@@ -211,6 +211,16 @@ def flash_attention_packed(qkv_p, idx, B, S, Hq, Hkv, D, causal=True, window=0, 
     return gather_rows(o, idx, inv)
 
 
+def prefill_attention_rows(qkv, first, inv, S, Hq, Hkv, D, k_cache, v_cache, window=0, scale=None, kv_start=None):
+    """Prompt attention over packed rows where they lie (GPU, no grad): position s >= kv_start[b] of row b is row
+    first[b] + s of ``qkv`` (rotated already), and ``inv`` [B*S] the row of every position (-1: a pad). K and V go to cache
+    slots [0, S), zeros for pads, as from the grid that :func:`flash_attention_packed` fills; the outputs are packed rows, with the bits of the grid's."""
+    scale = scale if scale is not None else 1.0 / math.sqrt(D)
+    native().kv_append_rows(qkv, inv, S, Hq, k_cache, v_cache)
+    q, k, v = qkv[:, : Hq * D], qkv[:, Hq * D:(Hq + Hkv) * D], qkv[:, (Hq + Hkv) * D:(Hq + 2 * Hkv) * D]
+    return native().attn_fwd(q, k, v, first.numel(), S, S, Hq, Hkv, D, True, window, scale, kv_start, None, None, 0, False, first)[0]
+
+
 def attention(q, k, v, B, Sq, Sk, Hq, Hkv, D, causal=False, window=0, scale=None, kv_start=None, kv_len=None,
               rel_bias_lut: Optional[torch.Tensor] = None, rb_L: int = 0):
     """Inference attention on separate (strided) q/k/v row views; used by the encoders

@@ -1044,3 +1044,54 @@ def test_probes_of_few_queries(nlist, d, l2):
                 assert got.dtype == torch.int32
                 fine = slice(0, nq - 1) if x.isnan().any() else slice(0, nq)
                 assert torch.equal(got[fine].long(), ops.topk(s, k)[1][fine])
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 128), (4, 4, 128), (6, 2, 64), (3, 3, 32)])
+@pytest.mark.parametrize("S,lens,window", [(5, [5, 1, 3], 0), (64, [64, 63, 1, 0], 0), (129, [129, 0, 66, 128], 40), (300, [7, 300, 65, 200], 0),
+                                           (1100, [1100, 1, 900], 500)])
+def test_prompt_attention_over_rows_where_they_lie(Hq, Hkv, D, S, lens, window):
+    """The bits of the filled grid, attention and gather, and the caches' of its append, pads among them: tiles that are all pads or partly, rows of
+    one token and of none, head-packed and other tiles, a window."""
+    from rag_tl_domainllm_optimizer_amd.models import packed_index
+
+    B, W = len(lens), (Hq + 2 * Hkv) * D
+    g = torch.Generator(device=DEV).manual_seed(S + D)
+    start = np.array([S - n for n in lens])
+    idx, off = packed_index(start, np.full(B, S), S, torch.device(DEV))
+    qkv = torch.randn(int(off[-1]), W + 8, generator=g, device=DEV).bfloat16()[:, :W]
+    ks = torch.tensor(start, dtype=torch.int32, device=DEV)
+    inv = ops.packed_inverse(idx, B * S)
+    first = torch.tensor([int(off[b]) - int(start[b]) for b in range(B)], dtype=torch.int32, device=DEV)
+    kc, vc, kc0, vc0 = (torch.full((B, Hkv, S + 3, D), 5.0, device=DEV).bfloat16() for _ in range(4))
+    got = ops.prefill_attention_rows(qkv, first, inv, S, Hq, Hkv, D, kc, vc, window, kv_start=ks)
+    grid = ops.scatter_rows(qkv, idx, inv, B * S)
+    pos = torch.zeros(B * S, dtype=torch.int32, device=DEV)
+    ops.rope_qkv_(grid, pos, None, None, Hq, Hkv, D, S=S, k_cache=kc0, v_cache=vc0)
+    want = ops.gather_rows(ops.flash_attention_qkv(grid, B, S, Hq, Hkv, D, True, window, kv_start=ks), idx, inv)
+    assert torch.equal(got, want) and torch.equal(kc, kc0) and torch.equal(vc, vc0)
+
+
+@pytest.mark.parametrize("preset", ["tiny-mistral", "tiny-llama", "tiny-opt"])
+def test_packed_prefill_of_rows_equals_grid(preset):
+    """A whole prompt forward with pads left out and with pads worked on: close (products of other row counts sum in another order), caches of pads zero."""
+    from rag_tl_domainllm_optimizer_amd import models
+    from rag_tl_domainllm_optimizer_amd.generation import KVCache
+
+    if preset not in models.config.PRESETS:
+        pytest.skip("no such preset")
+    cfg = models.resolve_preset(preset)
+    m = models.CausalLM(cfg, device=torch.device(DEV), dtype=torch.bfloat16, seed=0)
+    lens, S = [30, 7, 1, 18], 30
+    g = torch.Generator().manual_seed(1)
+    ids = torch.randint(3, cfg.vocab_size, (len(lens), S), generator=g)
+    start = torch.tensor([S - n for n in lens], dtype=torch.int32)
+    out = []
+    for packed in (None, models.packed_index(start.numpy(), np.full(len(lens), S), S, torch.device(DEV))):
+        cache = KVCache(cfg.num_layers, len(lens), cfg.num_kv_heads, 64, cfg.head_dim, torch.device(DEV), torch.bfloat16)
+        cache.k.zero_()
+        cache.v.zero_()
+        out.append((m.prefill(ids.to(DEV), start.to(DEV), cache, packed=packed), cache))
+    _close(out[0][0], out[1][0])
+    for b, s in enumerate(start.tolist()):
+        _close(out[0][1].k[:, b, :, s:S], out[1][1].k[:, b, :, s:S])
+        assert not out[1][1].k[:, b, :, :s].any() and not out[1][1].v[:, b, :, :s].any()
