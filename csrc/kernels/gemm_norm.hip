@@ -309,7 +309,7 @@ static bool fits(int N, int K) { return (N == 384 || N == 768) && K >= 64 && K %
 // A tile is one chain over K, however few there are: with few rows the product's small tiles in parallel are faster.
 // 384 columns: 0.54 us a step of 64 rows and 6 besides (128 rows: 0.9 and 8). Even: 2500 rows at K 128, 3000 at 384, 4500 at 768, 5300 at 1536,
 // 10500 at 3072; between an encoder's other kernels not below 4000 (a forward of 3000 rows 360 -> 368). Tiles of 64 while they are one round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles
-// of 64 42.6).
+// of 64 42.6), whole rounds of these and the rest in 64 where that is one round more (MiniLM over 34000 rows 1434 -> 1396 us).
 // 768 columns, us within an encoder's forward (between other kernels: alone, with w in the caches, both are faster): a round of tiles of 64 takes
 // 10 and 1.18 a step, nearly full 14 and 1.25, one of several 6.4 and 1.53; of 96 18 and 1.72. Product and norm: tiles of 256 x 256, whole rounds of
 // them and a rest, and 0.78 ns a row. All of one size, or whole rounds of 96 and the rest in 64. Product and norm | this at K 768: 12000 rows 35.9 |
@@ -318,8 +318,15 @@ static bool fits(int N, int K) { return (N == 384 || N == 768) && K >= 64 && K %
 extern "C" int rt_gemm_norm_rows(int M, int N, int K, int* first) {
   *first = 0;
   if (!fits(N, K)) return 0;
-  if (N == 384) return M < std::max(4000L, 1800 + 3L * K) ? 0 : M <= 64 * num_cus() ? 64 : 128;
-  const int per64 = 64 * num_cus(), per96 = 96 * num_cus(), per256 = num_cus() / 3 * 256;
+  const int per64 = 64 * num_cus();
+  if (N == 384) {
+    if (M < std::max(4000L, 1800 + 3L * K)) return 0;
+    const int whole = M / (2 * per64) * 2 * per64;
+    if (M - whole > per64) return 128;
+    *first = M > whole ? whole : 0;
+    return M > whole ? 64 : 128;
+  }
+  const int per96 = 96 * num_cus(), per256 = num_cus() / 3 * 256;
   auto rounds = [](int rows, int per) { return (rows + per - 1) / per; };
   const double steps = K / 64;
   auto in64 = [&](int rows) {

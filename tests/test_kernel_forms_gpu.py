@@ -1095,3 +1095,29 @@ def test_packed_prefill_of_rows_equals_grid(preset):
     for b, s in enumerate(start.tolist()):
         _close(out[0][1].k[:, b, :, s:S], out[1][1].k[:, b, :, s:S])
         assert not out[1][1].k[:, b, :, :s].any() and not out[1][1].v[:, b, :, :s].any()
+
+
+@pytest.mark.parametrize("lens", [[32768], [32769], [34000], [20000, 20000], [49200]])
+def test_encoder_of_384_columns_in_tiles_of_two_sizes(lens):
+    """Around whole rounds of the larger tiles, whose rest goes in smaller ones: the bits of the forward op by op."""
+    m, inputs = _few_rows_encoder(12, sum(lens))
+    ids, pos, off, longest = inputs(lens)
+    out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
+    assert m._encode_native(ids, pos, off, longest, True, out, torch.arange(len(lens), device=DEV))
+    assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
+
+
+def test_encoder_batches_that_go_together(monkeypatch):
+    """Batches in one forward give what they give one by one; other row counts may sum products in another order: a bf16 rounding or two of
+    unit vectors of 384."""
+    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder, encoder
+    from rag_tl_domainllm_optimizer_amd.tokenizer import Tokenizer
+
+    m, _ = _few_rows_encoder(12, 5)
+    tok = Tokenizer.synthetic(m.cfg.vocab_size, m.cfg.arch)
+    words = tok.words()
+    texts = [" ".join(words[(7 * i + k) % len(words)] for k in range(i % 40)) for i in range(200)]
+    enc = Encoder(m, tok, max_length=64, batch_size=16)
+    got = enc.encode(texts)
+    monkeypatch.setattr(encoder, "MERGED_BYTES", 0)
+    assert (got - enc.encode(texts)).abs().max().item() < 4e-3
