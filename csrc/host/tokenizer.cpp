@@ -150,7 +150,7 @@ class Tokenizer {
   // so that a corpus of any size must not go through them.
   std::pair<at::Tensor, std::vector<std::tuple<int64_t, int64_t, int64_t>>> encode_sorted(
       const std::vector<std::string>& texts, const std::vector<int64_t>& front, const std::vector<int64_t>& back,
-      bool keep_last, int64_t max_length, int64_t batch, int64_t pos0, int64_t pin, int nthreads) const {
+      bool keep_last, int64_t max_length, int64_t batch, int64_t pos0, int64_t pin, int64_t most_rows, int nthreads) const {
     TORCH_CHECK(batch > 0 && max_length > 0, "encode_sorted: batch ", batch, ", max_length ", max_length);
     std::vector<std::vector<int64_t>> ids = encode_batch(texts, nthreads);
     py::gil_scoped_release release;
@@ -163,12 +163,19 @@ class Tokenizer {
     std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return len_of(a) < len_of(b); });
     std::vector<std::tuple<int64_t, int64_t, int64_t>> groups;
     int64_t total = N;
-    for (int64_t r = 0; r < N; r += batch) {
-      const int64_t n = std::min(batch, N - r);
-      int64_t rows = 0;
-      for (int64_t j = r; j < r + n; ++j) rows += len_of(order[j]);
+    for (int64_t r = 0; r < N;) {
+      int64_t n = 0, rows = 0;
+      do {  // further batches while their rows fit
+        const int64_t end = std::min(r + n + batch, N);
+        int64_t more = 0;
+        for (int64_t j = r + n; j < end; ++j) more += len_of(order[j]);
+        if (n && rows + more > most_rows) break;
+        n = end - r;
+        rows += more;
+      } while (r + n < N);
       groups.emplace_back(n, rows, len_of(order[r + n - 1]));
       total += n + 1 + 2 * rows;
+      r += n;
     }
     at::Tensor buf = at::empty({total}, at::TensorOptions().dtype(at::kLong).pinned_memory(pin > 0 && total <= pin));
     int64_t* p = buf.data_ptr<int64_t>();
@@ -397,7 +404,7 @@ void bind_tokenizer(py::module& m) {
       .def("encode_batch", &Tokenizer::encode_batch, py::arg("texts"), py::arg("nthreads") = 8)
       .def("encode_sorted", &Tokenizer::encode_sorted, py::arg("texts"), py::arg("front"), py::arg("back"),
            py::arg("keep_last"), py::arg("max_length"), py::arg("batch"), py::arg("pos0"), py::arg("pin"),
-           py::arg("nthreads") = 8)
+           py::arg("most_rows") = 0, py::arg("nthreads") = 8)
       .def("decode", &Tokenizer::decode, py::arg("ids"), py::arg("skip_special") = true)
       .def("token_to_id", &Tokenizer::token_to_id)
       .def("id_to_token", &Tokenizer::id_to_token)

@@ -16,6 +16,9 @@ from ..models.encoder import SentenceEncoder
 from ..tokenizer import Tokenizer, load_tokenizer
 
 
+MERGED_BYTES = 1 << 30  # of activations of batches that are encoded in one forward
+
+
 class Encoder:
     def __init__(self, model: SentenceEncoder, tokenizer: Tokenizer, max_length: int = 256, batch_size: int = 256):
         self.model = model
@@ -63,10 +66,16 @@ class Encoder:
                 out[torch.tensor(idx, device=self.device)] = emb.float()
             return out
         # every batch is tokenised and uploaded ahead of the first forward: between them the host only launches
-        order, batches = self.tokenizer.encode_sorted(texts, self.max_length, self.batch_size, self.device,
-                                                      self.model.first_position)
-        r, m = 0, self.model
+        r, m, tok = 0, self.model, self.tokenizer
         placed = type(m).encode_packed is SentenceEncoder.encode_packed and "encode_packed" not in vars(m)
+        # On a GPU batches go together while their activations stay within MERGED_BYTES: each product's last round of tiles leaves CUs
+        # idle once, not once a batch (1024 texts of 20 to 120 words, MiniLM, four batches
+        # 3231 -> 2869 us)
+        most = {}
+        if placed and self.device.type == "cuda" and type(tok).encode_sorted is Tokenizer.encode_sorted and "encode_sorted" not in vars(tok):
+            c = m.cfg
+            most = dict(most_rows=MERGED_BYTES // (2 * (7 * c.hidden_size + c.intermediate_size)))
+        order, batches = tok.encode_sorted(texts, self.max_length, self.batch_size, self.device, m.first_position, **most)
         for ids, pos, off, longest in batches:
             n = len(off) - 1
             if placed:

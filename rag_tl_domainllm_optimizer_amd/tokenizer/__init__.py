@@ -163,9 +163,9 @@ class Tokenizer:
             out.append(ids)
         return out
 
-    def encode_sorted(self, texts: Sequence[str], max_length: int, batch: int, device, first_position: int = 0):
+    def encode_sorted(self, texts: Sequence[str], max_length: int, batch: int, device, first_position: int = 0, most_rows: int = 0):
         """:meth:`encode_batch` for an encoder, natively and with one upload: the texts sorted by length in groups of
-        ``batch`` without padding -> (order [N]: the texts' indices, [(ids [rows], positions [rows] from
+        ``batch`` (several of them in one while they have no more than ``most_rows`` tokens) without padding -> (order [N]: the texts' indices, [(ids [rows], positions [rows] from
         ``first_position``, offsets [texts + 1]: each text's first row, the longest text's length)]), on ``device``; the
         copy is not waited for up to ``PINNED_TOKENS`` integers."""
         front, back = self._wrap([], True), []
@@ -173,7 +173,7 @@ class Tokenizer:
             front, back = front[:1], front[1:]
         pin = PINNED_TOKENS if torch.device(device).type == "cuda" else 0
         buf, groups = self._impl.encode_sorted(list(texts), front, back, self.template == "cls_sep", max_length, batch,
-                                               first_position, pin)
+                                               first_position, pin, most_rows)
         buf = buf.to(device, non_blocking=pin > 0 and buf.is_pinned())
         at, out = len(texts), []
         for n, rows, longest in groups:

@@ -79,3 +79,26 @@ def test_encoder_calls_parts_of_ones_own():
         torch.testing.assert_close(Encoder(model, t, 16, batch_size=4).encode(texts), padded(model, t), rtol=1e-5, atol=1e-6)
     plain.encode_ids = lambda ids, lengths, normalize=True: torch.full((len(ids), cfg.hidden_size), 0.5)
     assert bool((Encoder(plain, tok, 16).encode(texts) == 0.5).all())
+
+
+@pytest.mark.parametrize("most", [1, 40, 100, 10 ** 6])
+def test_encode_sorted_merges_batches(most):
+    """Batches go together while their rows fit, a single one whatever it has; the texts and their order are the same."""
+    tok = Tokenizer.synthetic(400, "bert")
+    words, r = tok.words(), random.Random(3)
+    texts = [" ".join(r.choices(words, k=r.randint(0, 12))) for _ in range(50)]
+    order, single = tok.encode_sorted(texts, 16, 8, "cpu", 2)
+    got, groups = tok.encode_sorted(texts, 16, 8, "cpu", 2, most)
+    assert torch.equal(got, order)
+    at = 0
+    for ids, pos, off, longest in groups:
+        parts = []
+        while sum(len(p[2]) - 1 for p in parts) < len(off) - 1:
+            parts.append(single[at + len(parts)])
+        at += len(parts)
+        assert torch.equal(ids, torch.cat([p[0] for p in parts])) and torch.equal(pos, torch.cat([p[1] for p in parts]))
+        assert longest == parts[-1][3] and off.diff().tolist() == sum((p[2].diff().tolist() for p in parts), [])
+        rows = len(ids)
+        assert len(parts) == 1 or rows <= most
+        assert at == len(single) or rows + len(single[at][0]) > most
+    assert at == len(single)
