@@ -1898,10 +1898,6 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnBwdArgs a) {
       vf[s] = *(const bf16x8*)(a.v + ((long)b * a.S + kk) * a.ldv + (long)hk * D + 32 * s + 8 * g);
     }
   }
-  // retire these loads once, here (else hipcc re-waits vmcnt(0) for them inside the loop, which
-  // also drains the Q/dO prefetch and the dQ atomics every iteration)
-#pragma unroll
-  for (int s = 0; s < DS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
   f32x4 dk[DT], dvv[DT];
 #pragma unroll
   for (int c = 0; c < DT; ++c) { dk[c] = f32x4{0.f, 0.f, 0.f, 0.f}; dvv[c] = f32x4{0.f, 0.f, 0.f, 0.f}; }
@@ -1939,7 +1935,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnBwdArgs a) {
       del_r = a.delta[li];
     }
   };
-  if (nit > 0) load_qdo(0);
+  if (nit > 0) load_qdo(0);  // beside the keys: one trip to memory for both
+  // retire these loads once, here (else hipcc re-waits vmcnt(0) for them inside the loop, which
+  // also drains the Q/dO prefetch every iteration)
+#pragma unroll
+  for (int s = 0; s < DS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
+  // queries that see this lane's key
+  const int vis_lo = a.causal ? mykey : 0;
+  const int vis_hi = !key_valid ? -1 : a.window > 0 ? min(a.S - 1, mykey + a.window - 1) : a.S - 1;
 
   for (int it = 0; it < nit; ++it) {
     const int h = hk * G + it / nqt, qt = qbeg + (it % nqt) * 64;
@@ -1971,19 +1974,23 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnBwdArgs a) {
           dp[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(oa, vf[s], dp[u], 0, 0, 0);
         }
       }
-      // P and dS (element (u,i) <-> q = qt + 16u + 4g + i, key = mykey)
+      // P and dS (element (u,i) <-> q = qt + 16u + 4g + i, key = mykey); nothing under a condition: each score waited for its
+      // lse from LDS behind a branch, 16 trips in a row
+      f32x4 ls[4], de[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        ls[u] = *(const f32x4*)(lse_s + 16 * u + 4 * g);
+        de[u] = *(const f32x4*)(del_s + 16 * u + 4 * g);
+      }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int ql = 16 * u + 4 * g + i;
-          const int qq = qt + ql;
-          bool ok = key_valid && qq < a.S;
-          if (a.causal) ok = ok && mykey <= qq;
-          if (a.window > 0) ok = ok && (qq - mykey) < a.window;
-          const float p = ok ? exp2_raw(sp[u][i] * a.scale_log2 - lse_s[ql]) : 0.f;
+          const int qq = qt + 16 * u + 4 * g + i;
+          const float x = sp[u][i] * a.scale_log2 - ls[u][i];
+          const float p = exp2_raw(qq >= vis_lo && qq <= vis_hi ? x : -INFINITY);
           sp[u][i] = p;
-          dp[u][i] = p * (dp[u][i] - del_s[ql]);
+          dp[u][i] = p * (dp[u][i] - de[u][i]);
         }
       // dV^T += dO^T · P ; dK^T += Q^T · dS  (A via transposed reads, B = accumulators)
       const int qrow = lane >> 2 & 3, pcol = lane & 3;
@@ -2085,10 +2092,6 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnBwdArgs a) {
   }
   const long li = ((long)b * a.Hq + h) * a.S + qrow;
   const float lse2 = a.lse[li] * 1.4426950408889634f, del = a.delta[li];
-  // retire these loads here (else hipcc re-waits vmcnt(0) for them inside the loop)
-#pragma unroll
-  for (int s2 = 0; s2 < DS; ++s2) asm volatile("" : "+v"(qf[s2]), "+v"(of[s2]));
-
   f32x4 dq[DT];
 #pragma unroll
   for (int c = 0; c < DT; ++c) dq[c] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -2114,13 +2117,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnBwdArgs a) {
       *(u32x4*)(Vs + k_off<D>(lkey + KSTEP * r, lc)) = vreg[r];
     }
   };
-  if (kbeg < kend) {
-    load_tile(kbeg);
-    store_tile();
-  }
+  if (kbeg < kend) load_tile(kbeg);
+  // retire the query's loads here (else hipcc re-waits vmcnt(0) for them inside the loop)
+#pragma unroll
+  for (int s2 = 0; s2 < DS; ++s2) asm volatile("" : "+v"(qf[s2]), "+v"(of[s2]));
+  if (kbeg < kend) store_tile();
   __syncthreads();
 
-  const int qq = q0 + r16;  // this lane's query row
+  const int qq = q0 + r16;  // this lane's query row, and the keys it sees
+  const int vis_lo = a.window > 0 ? max(start, qq - a.window + 1) : start;
+  const int vis_hi = qq >= a.S ? -1 : a.causal ? qq : a.S - 1;
   for (int kv0 = kbeg; kv0 < kend; kv0 += 64) {
     const bool has_next = kv0 + 64 < kend;
     if (has_next) load_tile(kv0 + 64);
@@ -2143,10 +2149,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(AttnBwdArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kk = kv0 + 16 * t + 4 * g + i;
-        bool ok = kk >= start && kk < a.S && qq < a.S;
-        if (a.causal) ok = ok && kk <= qq;
-        if (a.window > 0) ok = ok && (qq - kk) < a.window;
-        const float pv = ok ? exp2_raw(st[t][i] * a.scale_log2 - lse2) : 0.f;
+        const float x = st[t][i] * a.scale_log2 - lse2;
+        const float pv = exp2_raw(kk >= vis_lo && kk <= vis_hi ? x : -INFINITY);
         st[t][i] = pv * (dp[t][i] - del);  // dS^T
       }
     // dQ += dS · K: A = packed dS^T accumulators [q][keys], B = K^T by transposed reads
