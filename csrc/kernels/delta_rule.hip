@@ -326,7 +326,8 @@ __device__ __forceinline__ void stn(T* p, const float* o) {
 }
 
 // convolution and silu of channels c .. c + N - 1 at positions p .. p + 3, zeros from position p + n on. TAPS: their
-// number (every load issued ahead), 0: any
+// number (every load issued ahead, of a row that is there in place of one that counts as zero: with each under its condition they were seven
+// trips to memory in a row, and 16 or 32 branches around the silus), 0: any
 template <typename T, int N, int TAPS>
 __device__ __forceinline__ void conv4(const Conv<T>& cv, int p, int n, int c, float (&y)[4][N]) {
   const int taps = TAPS ? TAPS : cv.a.taps;
@@ -345,9 +346,20 @@ __device__ __forceinline__ void conv4(const Conv<T>& cv, int p, int n, int c, fl
   if constexpr (TAPS > 0) {
     __attribute__((aligned(16))) float v[TAPS + 3][N], f[TAPS][N];  // f: the weights as they lie, [channel][tap]
 #pragma unroll
-    for (int j = 0; j < TAPS + 3; ++j) row(p - (TAPS - 1) + j, v[j]);
+    for (int j = 0; j < TAPS + 3; ++j) {
+      const int q = min(p - (TAPS - 1) + j, p + n - 1);  // n may be 0 or less; the chunk's last token is there
+      const T* src = q >= cv.start ? cv.x + (long)(q - cv.start) * cv.a.ldx : cv.ring ? cv.ring + (long)(max(q, 0) % TAPS) * cv.C : cv.x;
+      ldn<T, N>(src + c, v[j]);
+    }
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) ldn<T, N>(w + j * N, f[j]);
+#pragma unroll
+    for (int j = 0; j < TAPS + 3; ++j) {
+      const int q = p - (TAPS - 1) + j;
+      const bool there = q < p + n && (q >= cv.start || (cv.ring && q >= 0));
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[j][e] = there ? v[j][e] : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -371,7 +383,10 @@ __device__ __forceinline__ void conv4(const Conv<T>& cv, int p, int n, int c, fl
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int e = 0; e < N; ++e) y[i][e] = i < n ? y[i][e] * sigmoid(y[i][e]) : 0.f;
+    for (int e = 0; e < N; ++e) {
+      const float x = i < n ? y[i][e] : 0.f;
+      y[i][e] = x * sigmoid(x);
+    }
 }
 
 // workgroup = (head, chunk); CHN: a decay per key channel, else per head. N: elements per access. With decays per channel
@@ -554,8 +569,12 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(Args a, Work w) {
       }
     } else if (tid < 2 * CH) {  // column of P
       const int c = tid - CH;
+      float col[CH];
 #pragma unroll
-      for (int i = 0; i < CH; ++i) ws[L::P + L::sq(i, c)] = i > c ? Ps[i][c] : (i == c ? dot[i] : 0.f);
+      for (int i = 0; i < CH; ++i) col[i] = Ps[i][c];
+      const float own = dot[c];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) ws[L::P + L::sq(i, c)] = i > c ? col[i] : (i == c ? own : 0.f);
     }
     return;
   }
