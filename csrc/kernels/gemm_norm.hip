@@ -162,18 +162,20 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   wait_but<newer(NP, NP - 1, NA)>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  read_w(std::integral_constant<int, 0>{}, 0);
+  asm volatile("" ::: "memory");  // w ahead of x, as a step's last phase
 #pragma unroll
   for (int i = 0; i < 2 * FM; ++i) read_x(i / FM, i % FM, 0);
-  read_w(std::integral_constant<int, 0>{}, 0);
   auto phase = [&](auto set, auto ph) {
     constexpr int P = decltype(ph)::value, S = decltype(set)::value;
     // the next fragments' images have landed and this wave has read this phase's granule (and, from the second phase on, the step's x): behind the
-    // barrier both hold for all
+    // barrier both hold for all. In the first phase the step's x, 2 FM reads, may be under way: they were asked for behind the granule's
     wait_but<newer(NP, P, NA), P == 0 ? 2 * FM : 0>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     const int wn = wp == BP - 1 ? 0 : wp + 1, xn = xp == AP - 1 ? 0 : xp + 1;
     read_w(std::integral_constant<int, S ^ 1>{}, wn);
+    if constexpr (P == NP - 1) asm volatile("" ::: "memory");  // no read of x ahead of these: the next phase's wait counts on it
     if constexpr (P == 1) stage_x(t + AP, xp);
     stage_w(t + (P + BP) / NP, (P + BP) % NP, wp);
 #pragma unroll
