@@ -14,6 +14,7 @@
 
 #include "host/tokenizer.h"
 #include "host/ivf_host.h"
+#include "host/settled.h"
 #include "rt_workspace.h"
 #include "rt_tuning.h"
 
@@ -216,8 +217,9 @@ struct GluArg {
 const void* opt_ptr(const optional<Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
 // Split-K workspace of the decode GEMM (fp32 slabs + self-resetting arrival tickets), one per
-// (device, stream) so GEMMs on concurrent streams never share tickets. Allocated on first use
-// (eager warm-up precedes graph capture); intentionally never freed.
+// (device, stream) so GEMMs on concurrent streams never share tickets. Allocated on first use, which may be while the stream is
+// capturing (torch captures on a stream of its own, whatever a warm-up ran on): the zeros are there at once, and no replay has to write
+// them. Intentionally never freed.
 struct DecodeWS {
   Tensor slabs, tickets;
 };
@@ -237,8 +239,10 @@ DecodeWS& decode_ws(const Tensor& like, hipStream_t st) {
   auto it = map->find(key);
   if (it != map->end()) return *it->second;
   auto* w = new DecodeWS();
+  rt::Settled settled(like);
   w->slabs = at::empty({RT_SPLITK_SLAB_FLOATS}, like.options().dtype(at::kFloat));
   w->tickets = at::zeros({RT_SPLITK_TICKETS}, like.options().dtype(at::kInt));
+  settled.settle();
   (*map)[key] = w;
   return *w;
 }

@@ -1121,3 +1121,43 @@ def test_encoder_batches_that_go_together(monkeypatch):
     got = enc.encode(texts)
     monkeypatch.setattr(encoder, "MERGED_BYTES", 0)
     assert (got - enc.encode(texts)).abs().max().item() < 4e-3
+
+
+@pytest.mark.parametrize("M", [8, 48])
+def test_products_captured_first_on_a_stream(M):
+    """A stream whose first split product is captured: the workspace it makes is ready for whichever graph is replayed first, beside
+    what the graphs' pool held before, and for eager products on the stream."""
+    import ctypes
+
+    C = ops.native()
+    hip = ctypes.CDLL("libamdhip64.so")
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(handle), 1) == 0  # one of torch's might have a workspace; 1: beside the default stream
+    s = torch.cuda.ExternalStream(handle.value)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, 4096, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(2048, 4096, generator=g, device=DEV) / 64).bfloat16()
+    img = C.shuffle_decode_weight(w)
+    with ops.tuning(decode_split=4):
+        want = C.gemm(x, img, None, None, None, 0, False, None, None, 0.0, True)
+        pool, junk = torch.cuda.graph_pool_handle(), []
+        torch.cuda.synchronize()
+        first, graphs, outs = torch.cuda.CUDAGraph(), [], []
+        with torch.cuda.graph(first, pool=pool, stream=s):
+            junk += [torch.full((1 << 16,), 7, dtype=torch.int32, device=DEV) for _ in range(8)]
+        first.replay()
+        torch.cuda.synchronize()
+        junk.clear()  # back to the pool, with the sevens
+        for _ in range(2):
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], pool=pool, stream=s):
+                outs.append(C.gemm(x, img, None, None, None, 0, False, None, None, 0.0, True))
+        assert not any(C.decode_ws_dirty_tickets())
+        for k in (1, 0, 1):
+            with torch.cuda.stream(s):
+                assert torch.equal(C.gemm(x, img, None, None, None, 0, False, None, None, 0.0, True), want)
+            torch.cuda.synchronize()
+            outs[k].fill_(5)
+            graphs[k].replay()
+            torch.cuda.synchronize()
+            assert torch.equal(outs[k], want)
