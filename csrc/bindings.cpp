@@ -18,6 +18,8 @@
 #include "rt_workspace.h"
 #include "rt_tuning.h"
 
+using rt::zero_page;
+
 extern "C" {
 int rt_gemm_nt_glu(const void*, long, const void*, long, const void*, long, const void*, long, int, const void*, void*,
                    long, int, int, int, int, int, float*, unsigned*, const void*, long, float, int, const float*,
@@ -356,16 +358,6 @@ Tensor shuffle_decode_weight_fp8(const Tensor& q, optional<Tensor> out) {
 // out_mode 0: bf16 (bias + act epilogue; act 5 = SwiGLU: b = [gate; up] (2F rows), C = [M, F],
 // out2 = optional [M, 2F] pre-activation), 1: fp32, 2: fp32 atomic accumulate into `out`
 // (split-K `nsplit`; `out` must be given and initialised).
-const Tensor& zero_page(const Tensor& like) {
-  static std::mutex mu;
-  static auto* map = new std::unordered_map<int, Tensor>();
-  std::lock_guard<std::mutex> g(mu);
-  auto it = map->find(like.get_device());
-  if (it != map->end()) return it->second;
-  (*map)[like.get_device()] = at::zeros({2048}, like.options().dtype(at::kBFloat16));
-  return (*map)[like.get_device()];
-}
-
 Tensor gemm_big(const Tensor& a, const Tensor& b, int64_t layout_a, int64_t layout_b, const optional<Tensor>& a2,
                 const optional<Tensor>& b2, const optional<Tensor>& bias, int64_t act, int64_t out_mode,
                 int64_t nsplit, optional<Tensor> out, const optional<Tensor>& out2, const optional<Tensor>& residual,

@@ -7,8 +7,11 @@
 #include <hip/hip_runtime_api.h>
 
 #include <mutex>
-#include <unordered_map>
 #include <vector>
+
+#include "host/settled.h"
+
+using rt::zero_page;
 
 extern "C" {
 int rt_branch_norm(int, int, float*, const void*, long, int, const void*, const void*, const void*, float, void*,
@@ -97,16 +100,6 @@ struct Glu {
     for (int i = 0; i < 3; ++i) v[i] = (float)g[i];
   }
 };
-const Tensor& zero_page(const Tensor& like) {
-  static std::mutex mu;
-  static auto* map = new std::unordered_map<int, Tensor>();
-  std::lock_guard<std::mutex> g(mu);
-  auto it = map->find(like.get_device());
-  if (it == map->end())
-    it = map->emplace(like.get_device(), at::zeros({2048}, like.options().dtype(at::kBFloat16))).first;
-  return it->second;
-}
-
 // x [T, H] fp32 in place; kind 0 none / embedding, 1 rows of the activation type, 2 fp32 slabs
 // [nsplit, T, H], 3 pairs (activation type), 4 pairs (fp32). Returns h (plain: x rounded, without w_next) or
 // None.

@@ -7,6 +7,9 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <mutex>
+#include <unordered_map>
+
 namespace rt {
 
 // While it lives the device's current stream is one that does not capture; settle() waits for what was given to it.
@@ -35,11 +38,19 @@ class Settled {
   c10::hip::HIPStream before_, side_;
 };
 
-inline at::Tensor settled_zeros(const at::Tensor& like, int64_t n, at::ScalarType type) {
-  Settled s(like);
-  at::Tensor t = at::zeros({n}, like.options().dtype(type));
-  s.settle();
-  return t;
+// 4 KiB of zeros of a device: what products read in place of rows and columns that are not there
+inline const at::Tensor& zero_page(const at::Tensor& like) {
+  static std::mutex mu;
+  static auto* map = new std::unordered_map<int, at::Tensor>();
+  std::lock_guard<std::mutex> g(mu);
+  auto it = map->find(like.get_device());
+  if (it == map->end()) {
+    Settled settled(like);
+    at::Tensor page = at::zeros({2048}, like.options().dtype(at::kBFloat16));
+    settled.settle();
+    it = map->emplace(like.get_device(), page).first;
+  }
+  return it->second;
 }
 
 }  // namespace rt

@@ -1161,3 +1161,32 @@ def test_products_captured_first_on_a_stream(M):
             graphs[k].replay()
             torch.cuda.synchronize()
             assert torch.equal(outs[k], want)
+
+
+def test_zeros_of_products_are_made_while_capturing():
+    """A process whose first product is captured: what products read in place of columns that are not there is zero before the graph is
+    replayed, whatever the graph's pool held."""
+    import subprocess
+    import sys
+
+    code = """
+import torch
+from rag_tl_domainllm_optimizer_amd import ops
+C, dev = ops.native(), "cuda"
+x, w = (torch.ones(200, 72, device=dev, dtype=torch.bfloat16) for _ in range(2))
+pool, graphs, s = torch.cuda.graph_pool_handle(), [torch.cuda.CUDAGraph() for _ in range(2)], torch.cuda.Stream()
+torch.cuda.synchronize()
+with torch.cuda.graph(graphs[0], pool=pool, stream=s):
+    junk = [torch.full((2048,), 7, dtype=torch.bfloat16, device=dev) for _ in range(512)]
+graphs[0].replay()
+torch.cuda.synchronize()
+del junk
+with torch.cuda.graph(graphs[1], pool=pool, stream=s):
+    y = C.gemm_big(x, w, 0, 0)
+print(C.gemm_big(x, w, 0, 0).unique().tolist())
+graphs[1].replay()
+torch.cuda.synchronize()
+print(y.unique().tolist())
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split() == ["[72.0]", "[72.0]"], r.stdout + r.stderr[-2000:]
