@@ -152,8 +152,8 @@ __device__ __forceinline__ int v_off(int r, int c) {
 // 98.8 -> 81.7 (in a forward 82.8 -> 67.1), 1 x 3700 165 -> 154, with a window 148 -> 124, 2 x 2000 of 40 heads 153 -> 128, 16 x 256 of 12 heads of
 // 64 20.0 -> 13.5, with a bias 32.4 -> 24.6.
 //
-// a.first: rows of real positions only, tiled by position all the same (masked keys are read from a real row instead of a pad's zeros: the
-// same bits). 32 prompts of 90 to 320 tokens had needed a grid filled, and read for the cache, and results gathered: 79 us a layer beside 87 here, now 13
+// a.first: rows of real positions only, tiled by position all the same (a pad's key is read from a real row and masked, its value
+// is zero as in a grid: the same bits). 32 prompts of 90 to 320 tokens had needed a grid filled, and read for the cache, and results gathered: 79 us a layer beside 87 here, now 13
 // beside 83 (Mistral-7B, four layers, 8247 -> 7985).
 template <int D, int NU = 2, bool HP = false, bool Q64 = false, bool RB = false>
 __global__ __launch_bounds__(Q64 ? 256 : 64 * 8 / NU, D == 128 ? 2 : (D == 64 ? 3 : 4))
@@ -253,6 +253,11 @@ void attn_fwd_kernel(AttnArgs a) {
   for (int u = 0; u < NU; ++u)
 #pragma unroll
     for (int s = 0; s < DS; ++s) asm volatile("" : "+v"(qf[u][s]));
+  if (kbeg < plo) {  // only a row's first tile: values of pads are zeros (a weight of 0 times an infinite value is none)
+#pragma unroll
+    for (int r = 0; r < CPT; ++r)
+      if (kbeg + lkey + KSTEP * r < plo) vreg[r] = u32x4{0, 0, 0, 0};
+  }
   if (kbeg < kend) store_tile(smem, smem + TILE_BYTES);
   __syncthreads();
 

@@ -1190,3 +1190,27 @@ print(y.unique().tolist())
 """
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.split() == ["[72.0]", "[72.0]"], r.stdout + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 128), (4, 4, 128), (6, 2, 64), (3, 3, 32)])
+@pytest.mark.parametrize("S,lens,window", [(70, [70, 3, 66, 1], 0), (200, [200, 130, 7, 64], 50)])
+def test_prompt_attention_over_rows_of_infinite_values(Hq, Hkv, D, S, lens, window):
+    """Infinite and NaN values at a row's first and last token: the grid's results, whose pads are zeros."""
+    from rag_tl_domainllm_optimizer_amd.models import packed_index
+
+    B, W = len(lens), (Hq + 2 * Hkv) * D
+    g = torch.Generator(device=DEV).manual_seed(S + D)
+    start = np.array([S - n for n in lens])
+    idx, off = packed_index(start, np.full(B, S), S, torch.device(DEV))
+    qkv = torch.randn(int(off[-1]), W, generator=g, device=DEV).bfloat16()
+    v = qkv[:, (Hq + Hkv) * D:]
+    v[off[:-1], 0], v[off[:-1], D - 1], v[off[1:] - 1, 1] = float("inf"), float("-inf"), float("nan")
+    ks = torch.tensor(start, dtype=torch.int32, device=DEV)
+    inv = ops.packed_inverse(idx, B * S)
+    first = torch.tensor([int(off[b]) - int(start[b]) for b in range(B)], dtype=torch.int32, device=DEV)
+    kc, vc = (torch.zeros(B, Hkv, S, D, device=DEV).bfloat16() for _ in range(2))
+    got = ops.prefill_attention_rows(qkv, first, inv, S, Hq, Hkv, D, kc, vc, window, kv_start=ks)
+    grid = ops.scatter_rows(qkv, idx, inv, B * S)
+    want = ops.gather_rows(ops.flash_attention_qkv(grid, B, S, Hq, Hkv, D, True, window, kv_start=ks), idx, inv)
+    assert want.isinf().any() and want.isnan().any()
+    torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
