@@ -16,22 +16,29 @@ from ..models.encoder import SentenceEncoder
 from ..tokenizer import Tokenizer, load_tokenizer
 
 
-MERGED_BYTES = 1 << 30  # of activations of batches that are encoded in one forward
+BATCH_SIZE = 256        # the default
+MERGED_BYTES = 1 << 30  # of activations of default batches that are encoded in one forward: what one of 256 long texts takes alone
 
 
 class Encoder:
-    def __init__(self, model: SentenceEncoder, tokenizer: Tokenizer, max_length: int = 256, batch_size: int = 256):
+    """``batch_size``: the most texts of a forward, where it is not the default. ``max_rows``: on a GPU batches go together up to so
+    many tokens (0: none do); None: those of the default size do, up to ``MERGED_BYTES`` of activations, others don't. A text's
+    last bits depend on the rows beside it in its forward, whose number chooses the order in which products are summed."""
+
+    def __init__(self, model: SentenceEncoder, tokenizer: Tokenizer, max_length: int = 256, batch_size: int = BATCH_SIZE,
+                 max_rows: Optional[int] = None):
         self.model = model
         self.tokenizer = tokenizer
         self.max_length = min(max_length, model.cfg.max_position - model.cfg.position_offset)
         self.batch_size = batch_size
+        self.max_rows = max_rows
 
     @classmethod
     def from_name(cls, name_or_path: str = "all-MiniLM-L6-v2:random", device="cpu", max_length: int = 256,
-                  batch_size: int = 256, seed: int = 0) -> "Encoder":
+                  batch_size: int = BATCH_SIZE, seed: int = 0, max_rows: Optional[int] = None) -> "Encoder":
         model = build_model(name_or_path, device=device, seed=seed)
         tok = load_tokenizer(name_or_path, model.cfg.vocab_size, model.cfg.arch)
-        return cls(model.eval(), tok, max_length, batch_size)
+        return cls(model.eval(), tok, max_length, batch_size, max_rows)
 
     @property
     def device(self):
@@ -47,6 +54,13 @@ class Encoder:
         return all(getattr(type(o), n, None) is getattr(c, n) and n not in vars(o) for o, c, names in (
             (self.model, SentenceEncoder, ("forward", "encode_ids")), (self.tokenizer, Tokenizer, ("encode_batch", "pad", "_wrap")))
             for n in names)
+
+    def _rows_together(self) -> int:
+        """Tokens up to which further batches go into a forward on a GPU."""
+        if self.max_rows is not None:
+            return self.max_rows
+        c = self.model.cfg
+        return MERGED_BYTES // (2 * (7 * c.hidden_size + c.intermediate_size)) if self.batch_size == BATCH_SIZE else 0
 
     @torch.no_grad()
     def encode(self, texts: Sequence[str], normalize: bool = True) -> torch.Tensor:
@@ -68,13 +82,11 @@ class Encoder:
         # every batch is tokenised and uploaded ahead of the first forward: between them the host only launches
         r, m, tok = 0, self.model, self.tokenizer
         placed = type(m).encode_packed is SentenceEncoder.encode_packed and "encode_packed" not in vars(m)
-        # On a GPU batches go together while their activations stay within MERGED_BYTES: each product's last round of tiles leaves CUs
-        # idle once, not once a batch (1024 texts of 20 to 120 words, MiniLM, four batches
-        # 3231 -> 2869 us)
+        # On a GPU batches go together: each product's last round of tiles leaves CUs idle once, not once a batch (1024 texts of
+        # 20 to 120 words, MiniLM, four batches 3231 -> 2869 us)
         most = {}
         if placed and self.device.type == "cuda" and type(tok).encode_sorted is Tokenizer.encode_sorted and "encode_sorted" not in vars(tok):
-            c = m.cfg
-            most = dict(most_rows=MERGED_BYTES // (2 * (7 * c.hidden_size + c.intermediate_size)))
+            most = dict(most_rows=self._rows_together())
         order, batches = tok.encode_sorted(texts, self.max_length, self.batch_size, self.device, m.first_position, **most)
         for ids, pos, off, longest in batches:
             n = len(off) - 1

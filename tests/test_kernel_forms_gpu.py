@@ -1107,20 +1107,18 @@ def test_encoder_of_384_columns_in_tiles_of_two_sizes(lens):
     assert torch.equal(out, m.encode_packed(ids, pos, off, longest))
 
 
-def test_encoder_batches_that_go_together(monkeypatch):
+def test_encoder_batches_that_go_together():
     """Batches in one forward give what they give one by one; other row counts may sum products in another order: a bf16 rounding or two of
     unit vectors of 384."""
-    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder, encoder
+    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder
     from rag_tl_domainllm_optimizer_amd.tokenizer import Tokenizer
 
     m, _ = _few_rows_encoder(12, 5)
     tok = Tokenizer.synthetic(m.cfg.vocab_size, m.cfg.arch)
     words = tok.words()
     texts = [" ".join(words[(7 * i + k) % len(words)] for k in range(i % 40)) for i in range(200)]
-    enc = Encoder(m, tok, max_length=64, batch_size=16)
-    got = enc.encode(texts)
-    monkeypatch.setattr(encoder, "MERGED_BYTES", 0)
-    assert (got - enc.encode(texts)).abs().max().item() < 4e-3
+    got = Encoder(m, tok, max_length=64, batch_size=16, max_rows=10 ** 6).encode(texts)
+    assert (got - Encoder(m, tok, max_length=64, batch_size=16).encode(texts)).abs().max().item() < 4e-3
 
 
 @pytest.mark.parametrize("M", [8, 48])
@@ -1214,3 +1212,25 @@ def test_prompt_attention_over_rows_of_infinite_values(Hq, Hkv, D, S, lens, wind
     want = ops.gather_rows(ops.flash_attention_qkv(grid, B, S, Hq, Hkv, D, True, window, kv_start=ks), idx, inv)
     assert want.isinf().any() and want.isnan().any()
     torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
+
+
+def test_encoder_batch_size_bounds_a_forward():
+    """A batch size of the caller's: no forward of more texts, unless rows are allowed; 256, the default: batches together."""
+    from rag_tl_domainllm_optimizer_amd.retrieval import Encoder
+    from rag_tl_domainllm_optimizer_amd.tokenizer import Tokenizer
+
+    m, _ = _few_rows_encoder(12, 6)
+    tok = Tokenizer.synthetic(m.cfg.vocab_size, m.cfg.arch)
+    words = tok.words()
+    texts = [" ".join(words[(7 * i + k) % len(words)] for k in range(1 + i % 9)) for i in range(600)]
+    forward, seen = m._encode_native, []
+    m._encode_native = lambda ids, pos, off, *a: seen.append((len(off) - 1, len(ids))) or forward(ids, pos, off, *a)
+
+    def forwards(**kw):
+        seen.clear()
+        Encoder(m, tok, max_length=64, **kw).encode(texts)
+        return list(seen)
+    assert max(n for n, _ in forwards(batch_size=16)) == 16
+    assert max(n for n, _ in forwards(batch_size=500)) == 500
+    assert [n for n, _ in forwards()] == [600] and [n for n, _ in forwards(max_rows=0)] == [256, 256, 88]
+    assert len(forwards(batch_size=16, max_rows=1000)) < 600 // 16 and all(r <= 1000 for _, r in forwards(batch_size=16, max_rows=1000))
