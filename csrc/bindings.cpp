@@ -14,6 +14,7 @@
 
 #include "host/tokenizer.h"
 #include "host/ivf_host.h"
+#include "host/lost.h"
 #include "host/settled.h"
 #include "rt_workspace.h"
 #include "rt_tuning.h"
@@ -74,7 +75,7 @@ int rt_gemm_plan(int, int, int, int, int, int*);
 int rt_token_plan(int, int, int, int, int*);
 int rt_small_tiles(int, int, int, int);
 int rt_embed_norm_rows(const void*, const long*, const void*, const long*, const void*, const void*, const void*, void*, int, int,
-                       float, void*, long, void*, int, hipStream_t);
+                       float, void*, long, void*, unsigned*, unsigned, hipStream_t);
 int rt_gemm_norm(const void*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, float, int, hipStream_t);
 int rt_gemm_norm_rows(int, int, int, int*);
 long rt_encoder_few_bytes(int, int, int, int, int, int, const int*);
@@ -160,6 +161,7 @@ static const TuningField kTuningFields[] = {
     {"gemm_group_m", &rt::Tuning::gemm_group_m, nullptr},
     {"sample_window", &rt::Tuning::sample_window, nullptr},
     {"sample_fast64", &rt::Tuning::sample_fast64, nullptr},
+    {"encoder_tries", &rt::Tuning::encoder_tries, nullptr},
 };
 
 py::dict get_tuning() {
@@ -1405,7 +1407,7 @@ static Tensor linear_norm(const Tensor& x, const Tensor& w, const Tensor& bias, 
 // A sentence encoder's forward over texts without padding (see attn_packed), pooled and normalised, written to out[to[b]]:
 // one call for the 40 and more launches, which from Python take longer to issue than a short query's take to run. emb: word and
 // position tables, token type row or null, norm weight, norm bias; layers: qkv, o, ln1, fc1, fc2, ln2, a weight and a bias each.
-// False where something is not as this path needs it (the caller goes op by op, which says what).
+// False where something is not as this path needs it (the caller goes op by op, which says what). Raises what raise_lost does.
 bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int64_t longest,
                     const std::vector<optional<Tensor>>& emb, const std::vector<Tensor>& layers, int64_t heads, double eps,
                     const optional<Tensor>& rel_bias, int64_t rb_L, bool normalize, Tensor out, const Tensor& to) {
@@ -1438,6 +1440,7 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
                     rel_bias->dim() == 2 && rel_bias->size(0) == heads && rel_bias->size(1) == 2 * rb_L - 1 && rb_L >= longest))
     return false;
 
+  rt::raise_lost(word.get_device());
   hipStream_t st = cur_stream();
   auto rows = [&](int64_t n) { return at::empty({M, n}, word.options()); };
   auto attend = [&](const Tensor& qkv, Tensor& a) {
@@ -1452,10 +1455,11 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
                          (int)H, (float)eps, nullptr, 0, st),
              "encoder: norm");
   };
-  auto embed = [&](void* y, void* unset, long unset_bytes, void* zero) {
+  const unsigned tries = (unsigned)std::max(0, rt::tuning().encoder_tries);
+  auto embed = [&](void* y, void* unset, long unset_bytes, void* head) {
     check_rc(rt_embed_norm_rows(word.data_ptr(), (const long*)ids.data_ptr(), ptab.data_ptr(), (const long*)pos.data_ptr(),
                                 emb[2] ? emb[2]->data_ptr() : nullptr, emb[3]->data_ptr(), emb[4]->data_ptr(), y, (int)M, (int)H,
-                                (float)eps, unset, unset_bytes, zero, (int)(M + 15) / 16 * 16, st),
+                                (float)eps, unset, unset_bytes, head, rt::lost_word(word.get_device()), tries, st),
              "encoder: embedding");
   };
   // Up to 64 rows the layers in one launch: 64 rows of mpnet-base 517 -> 475 us, fewer or narrower more (see encoder_few.hip); beyond, a round of
@@ -1817,6 +1821,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("encoder_packed", &encoder_packed, "sentence encoder over texts without padding", py::arg("ids"), py::arg("pos"),
         py::arg("off"), py::arg("longest"), py::arg("emb"), py::arg("layers"), py::arg("heads"), py::arg("eps"),
         py::arg("rel_bias"), py::arg("rb_L"), py::arg("normalize"), py::arg("out"), py::arg("to"));
+  m.def("raise_lost", &rt::raise_lost, "raise if a forward on the device gave up waiting", py::arg("device"));
   m.def("linear_norm", &linear_norm, "LN(x w^T + b + res) in one launch", py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("res"), py::arg("lw"),
         py::arg("lb"), py::arg("eps"), py::arg("rows") = 0);
   m.def("few_rows", &few_rows, "act(x w^T + b) of up to 32 rows, normalised first if asked", py::arg("x"), py::arg("w"),

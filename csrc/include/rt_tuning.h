@@ -58,6 +58,9 @@ struct Tuning {
                               // wave (0: 16 block-wide counting passes over the whole row; same draw)
   int sample_fast64 = 1;      // <= 64 survivors: sort / top-p / draw in wave 0's registers without a block
                               // barrier (0: the block-wide path; same draw)
+  // ---- encoders of few rows (encoder_few.hip) ----
+  int encoder_tries = 1 << 22;  // times a wave asks for rows of other workgroups before it gives up (seconds). 0, for tests: the first
+                                // task is left out, and those that wait for it give up at their first look
 };
 
 }  // namespace rt

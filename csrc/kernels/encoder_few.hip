@@ -13,13 +13,15 @@
 // stores to a line, an exchange took 0.7 to 2 us). Rows that feed a product without a norm lie as the MFMA takes them, and go from memory
 // to its operands. Asking more cheaply first (one word, or one wave of a workgroup), or all on one XCD, took longer (106 -> 115, 127).
 // A workgroup waits only for tasks that running workgroups have taken before it, so the launch ends with whatever number of them the
-// device runs at a time, beside other launches of its kind too; a wait of seconds gives up all the same, and the results are NaN.
+// device runs at a time, beside other launches of its kind too; a wait of seconds gives up all the same: the results are NaN, and a word of
+// host memory says so.
 //
 // The arithmetic, its parts of K and their order are few_rows.hip's, attn_packed_kernel's and pool_norm_kernel's: the same bits.
 // us, launch by launch -> this, with the embedding: MiniLM over 15 / 32 / 64 rows 133 -> 86 / 158 -> 103 / 190 -> 128, mpnet-base 344 -> 232 /
 // 451 -> 329 / 517 -> 475.
 #include "rt_common.h"
 #include "rt_gelu.h"
+#include "rt_few_head.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -48,7 +50,7 @@ struct Args {
   const long* off;
   bf16_t* ex;          // rows on their way: x0, then a layer's qkv, a, d1, x1, f, d2, x2; see place()
   unsigned ex_bytes;
-  unsigned* next;      // the next task
+  unsigned* next;      // the next task: FewHead, ahead of the rows
   int normalize;
   float* out; const long* to; long out_rows;
   int lds_x, lds_red;  // byte offsets behind the ring
@@ -60,7 +62,8 @@ __device__ __forceinline__ void dma16(const bf16_t* from, char* to) { __builtin_
 
 constexpr int SC1 = 16;
 __device__ __forceinline__ bool there(const u32x4& v) { return v[0] != NONE && v[1] != NONE && v[2] != NONE && v[3] != NONE; }
-// v[i] = load(i) until every lane's words are results; `lost`: set where somebody has given up
+// v[i] = load(i) until every lane's words are results. Waits are bounded: who has asked in vain `tries` times says so to the launch, which
+// gives up (each waiting wave looks every 1024 times), and to the host. Both are beside `lost` and not arguments: the kernel has no register for them.
 template <int N, typename F>
 __device__ __forceinline__ void await(unsigned* lost, u32x4 (&v)[N], F load) {
   for (int tries = 0;; ++tries) {
@@ -74,7 +77,12 @@ __device__ __forceinline__ void await(unsigned* lost, u32x4 (&v)[N], F load) {
     __builtin_amdgcn_s_sleep(1);
     if ((tries & 1023) == 1023) {
       if (__hip_atomic_load(lost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-      if (tries >> 22) __hip_atomic_store(lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      typedef __attribute__((address_space(4))) const FewHead Head;  // written by the launch before: by scalar loads, into no vector register
+      Head* const h = (Head*)(uintptr_t)(lost - 16);
+      if ((unsigned)tries >= h->tries) {
+        __hip_atomic_store(lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(h->report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
 }
@@ -527,7 +535,7 @@ static int red_bytes(const ef::Product& p) { return p.parts * p.cg * ef::RED * 1
 // normed rows of a task, or values of attention
 static int x_bytes(int H) { return std::max(16 * (H + 8) * 2, ef::UNITS * ef::VPLACE); }
 
-// Bytes of rows on their way (ahead of them the counter, 256 bytes); 0: not for this kernel. parts: n, grp of qkv, o, fc1, fc2.
+// Bytes of rows on their way (ahead of them a FewHead); 0: not for this kernel. parts: n, grp of qkv, o, fc1, fc2.
 extern "C" long rt_encoder_few_bytes(int M, int H, int F, int B, int L, int heads, const int* parts) {
   if (M < 1 || M > 64 || B < 1 || B > 1 << 12 || L < 1 || L > ef::MAX_LAYERS || heads < 1 || H % heads || H % 64 || F % 64 || H > 1024 || F > 1 << 14) return 0;
   if (H / heads != 32 && H / heads != 64) return 0;
@@ -542,7 +550,7 @@ extern "C" long rt_encoder_few_bytes(int M, int H, int F, int B, int L, int head
   return 256 + (M + 15) / 16 * 32L * (H + L * (8L * H + F));
 }
 
-// x0 in place at ex (behind the counter), everything else of it unset (see rt_embed_norm_rows)
+// x0 in place at ex (behind the head), everything else of it unset (see rt_embed_norm_rows)
 extern "C" int rt_encoder_few(const void* const* w, void* ws, long bytes, const long* off, const float* rel_bias, int rb_L, int M, int H, int F,
                               int B, int L, int heads, float eps, float scale, const int* parts, int normalize, float* out, const long* to,
                               long out_rows, hipStream_t stream) {

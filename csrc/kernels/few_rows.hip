@@ -13,6 +13,7 @@
 // 384 x 1536 9.8 -> 5.8 -> 4.4, and 2.9 of the norm with it. MiniLM over 15 / 32 rows 157 -> 141 / 201 -> 167, mpnet-base (and with
 // wave_reduce) 428 -> 345 / 620 -> 452. From 33 rows on gemm_mid_kernel's tiles are ahead.
 #include "rt_common.h"
+#include "rt_few_head.h"
 #include "rt_gelu.h"
 
 #include <algorithm>
@@ -210,19 +211,24 @@ __global__ __launch_bounds__(512, 2) void few_rows_kernel(Args p) {
 }
 
 // x[t] = LN(bf16(word[id] + pos[p]) + type): the embedding of an encoder in one pass, a wave a row. The sum is rounded to bf16
-// after each term, as embed_kernel and an addition do; the norm is norm_rows_kernel's without a residual. `unset` and `zero` (see
-// encoder_few.hip): memory that is set to ones, and 256 bytes of zeros; with them the rows hold no word of ones, and lie in column groups
-// of 16 with `tile` rows each.
+// after each term, as embed_kernel and an addition do; the norm is norm_rows_kernel's without a residual. `unset` and `head`
+// (see encoder_few.hip): memory that is set to ones, and a FewHead that is written; with them the rows hold no word of ones, and lie in
+// column groups of 16, T up to a multiple of 16 of them each. The arguments fill two lines: with a third it took 4.0 us instead of 3.6.
 template <int NW>
 __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __restrict__ word, const long* __restrict__ ids,
                                                               const bf16_t* __restrict__ pos, const long* __restrict__ pids,
                                                               const bf16_t* __restrict__ type, const bf16_t* __restrict__ w,
                                                               const bf16_t* __restrict__ b, bf16_t* __restrict__ y, int T, int H,
-                                                              float eps, uint4* __restrict__ unset, long n_unset,
-                                                              unsigned* __restrict__ zero, int tile) {
+                                                              float eps, int n_unset, uint4* __restrict__ unset,
+                                                              FewHead* __restrict__ head, unsigned* report, unsigned tries) {
   const int lane = threadIdx.x & 63, nv = H / 8;
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n_unset; i += (long)gridDim.x * 256) unset[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
-  if (zero && blockIdx.x == 0 && threadIdx.x < 64) zero[threadIdx.x] = 0;
+  if (head && blockIdx.x == gridDim.x - 1 && threadIdx.x < 64) {  // a workgroup that has no rows, as a rule
+    constexpr int TRIES = offsetof(FewHead, tries) / 4, REPORT = offsetof(FewHead, report) / 4;
+    const int t = threadIdx.x;
+    const unsigned long to = (unsigned long)report;
+    ((unsigned*)head)[t] = t == 0 ? tries == 0 : t == TRIES ? tries : t == REPORT ? (unsigned)to : t == REPORT + 1 ? (unsigned)(to >> 32) : 0;
+  }
   for (long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6); row < T; row += (long)gridDim.x * 4) {
     RT_ASSERT(ids[row] >= 0 && pids[row] >= 0);
     const bf16_t* const wp = word + ids[row] * H;
@@ -275,12 +281,12 @@ __global__ __launch_bounds__(256) void embed_norm_rows_kernel(const bf16_t* __re
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = fmaf((v[i][e] - mean) * rstd, wv[e], bv[e]);
         uint4 q = pack8(o);
-        if (zero) {
+        if (head) {
           uint32_t* const u = (uint32_t*)&q;
 #pragma unroll
           for (int e = 0; e < 4; ++e) u[e] = u[e] == ~0u ? 0xfffefffeu : u[e];
         }
-        *(uint4*)(y + (zero ? ((c >> 1) * tile + row) * 16 + (c & 1) * 8 : row * H + c * 8)) = q;
+        *(uint4*)(y + (head ? ((c >> 1) * ((T + 15) & ~15) + row) * 16 + (c & 1) * 8 : row * H + c * 8)) = q;
       }
     }
   }
@@ -324,14 +330,15 @@ extern "C" int rt_few_rows(const void* x, long ldx, const void* res, long ldr, c
 // y[t] = LN(word[ids[t]] + pos[pids[t]] (+ type)); H % 8 == 0, H <= 1024. unset_bytes: a multiple of 16
 extern "C" int rt_embed_norm_rows(const void* word, const long* ids, const void* pos, const long* pids, const void* type,
                                   const void* w, const void* b, void* y, int T, int H, float eps, void* unset, long unset_bytes,
-                                  void* zero, int tile, hipStream_t stream) {
+                                  void* head, unsigned* report, unsigned tries, hipStream_t stream) {
   if (T <= 0) return 0;
-  if (H % 8 || H > 1024) return -1;
+  if (H % 8 || H > 1024 || unset_bytes / 16 > 0x7fffffffL) return -1;
   const long n = unset ? unset_bytes / 16 : 0;
   const dim3 grid((unsigned)std::min(std::max((T + 3L) / 4, (n + 255) / 256), 2048L)), block(256);
 #define EN(W)                                                                                                                 \
   hipLaunchKernelGGL(fr::embed_norm_rows_kernel<W>, grid, block, 0, stream, (const bf16_t*)word, ids, (const bf16_t*)pos, pids, \
-                     (const bf16_t*)type, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, T, H, eps, (uint4*)unset, n, (unsigned*)zero, tile)
+                     (const bf16_t*)type, (const bf16_t*)w, (const bf16_t*)b, (bf16_t*)y, T, H, eps, (int)n, (uint4*)unset, (FewHead*)head, \
+                     report, tries)
   if (H <= 512) EN(1); else EN(2);
 #undef EN
   RT_LAUNCH_CHECK();

@@ -198,6 +198,14 @@ def topk(scores: torch.Tensor, k: int, idmap=None, finite: bool = False):
     return v, torch.where(torch.isfinite(v), i, torch.full_like(i, -1)) if finite else i
 
 
+def check_lost(device):
+    """Raise if an encoder's forward on ``device`` gave up a wait, which leaves its embeddings NaN: for where their results have been
+    waited for (the next forward raises, too)."""
+    device = torch.device(device)
+    if device.type == "cuda":
+        native().raise_lost(torch.cuda.current_device() if device.index is None else device.index)
+
+
 def ivf_probes(q, cen, nlist: int, k: int, pen=None):
     """The ``k`` lists that each query probes on a GPU, the best of its scores q cen[:nlist]^T - pen -> (q in bf16, int32 indices
     [nq, k]). Up to 16 fp32 queries are rounded and multiplied in one launch, with :func:`gemm`'s bits."""

@@ -13,6 +13,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 import torch
 
+from .. import ops
 from ..generation import Generator, SamplingParams
 from .prompt import build_prompt, extract_answer, encode_prompt
 
@@ -69,6 +70,7 @@ class RagPipeline:
             ids_l = [row[:k] for row, k in zip(ids.tolist(), ks)]
             scores = [row[:k] for row, k in zip(scores.tolist(), ks)]
             self._sync()
+            ops.check_lost(self.device)
             t1 = time.perf_counter()
             docs = [[self.docs[i] for i in row if i >= 0] for row in ids_l]
             prompts = [self._prompt_ids(q, d) for q, d in zip(qs, docs)]

@@ -256,7 +256,9 @@ class IVFIndex:
         a = self._assign(xq)
         cnt = torch.bincount(a, minlength=self.nlist).int()
         need = self.lsize + cnt
-        if bool((need > self.lcap).any()):
+        full = bool((need > self.lcap).any())
+        ops.check_lost(self.device)
+        if full:
             self._grow(need)
         srt, order = torch.sort(a, stable=True)
         first = (torch.cumsum(cnt, 0) - cnt).long()
@@ -339,6 +341,7 @@ def _save(index, path: str):
 
     os.makedirs(path, exist_ok=True)
     tensors, meta = index.state()
+    ops.check_lost(index.device)
     save_file({k: v.contiguous() for k, v in tensors.items()}, os.path.join(path, "index.safetensors"))
     with open(os.path.join(path, "index.json"), "w") as f:
         json.dump(meta, f, indent=2)

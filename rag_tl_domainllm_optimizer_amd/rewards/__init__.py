@@ -16,6 +16,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from .. import ops
+
 
 @dataclass
 class RewardConfig:
@@ -87,6 +89,7 @@ class RewardModel:
             a, b = self.cfg.gt_mix
             reward = torch.where(has_gt, a * reward + b * gsim, reward)
         gl = gsim.tolist()  # one device->host copy, not one per row
+        ops.check_lost(dev)
         comps = {"factual_accuracy": fact, "relevance": rel, "conciseness": conc,
                  "ground_truth_similarity": [gl[i] if g_i[i] >= 0 else None for i in range(B)],
                  "total_reward": reward}
