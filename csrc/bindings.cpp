@@ -1824,6 +1824,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("raise_lost", &rt::raise_lost, "raise if a forward on the device gave up waiting", py::arg("device"));
   m.def("linear_norm", &linear_norm, "LN(x w^T + b + res) in one launch", py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("res"), py::arg("lw"),
         py::arg("lb"), py::arg("eps"), py::arg("rows") = 0);
+  m.def("linear_norm_tiles", [](int64_t M, int64_t N, int64_t K) {
+    int first = 0;
+    const int rows = rt_gemm_norm_rows((int)M, (int)N, (int)K, &first);
+    return std::make_pair(rows, first);
+  }, "rows of linear_norm's tiles (0: two launches are faster), leading rows in larger ones", py::arg("M"), py::arg("N"), py::arg("K"));
   m.def("few_rows", &few_rows, "act(x w^T + b) of up to 32 rows, normalised first if asked", py::arg("x"), py::arg("w"),
         py::arg("bias") = py::none(), py::arg("act") = 0, py::arg("res") = py::none(), py::arg("lw") = py::none(),
         py::arg("lb") = py::none(), py::arg("eps") = 0.0);

@@ -767,10 +767,13 @@ def test_product_and_norm_in_one_launch(M, K, rows):
     assert got[5].isnan().all() and torch.equal(got[keep], want[keep])
 
 
-@pytest.mark.parametrize("lens", [[2951], [2952], [6407, 1], [5000, 11384], [9000, 7385], [1] * 500 + [17000]])
-def test_encoder_where_products_take_the_norm(lens):
+# rows of the tiles of the output product (K 384) and of the second feed-forward product (K 1536), 0: product and norm apart
+@pytest.mark.parametrize("lens,tiles", [([3999], (0, 0)), ([4000], (64, 0)), ([6407], (64, 0)), ([6407, 1], (64, 64)), ([5000, 11384], (64, 64)),
+                                        ([9000, 7385], (128, 128)), ([1] * 500 + [17000], (128, 128))])
+def test_encoder_where_products_take_the_norm(lens, tiles):
     """Around the row counts where the output and the second feed-forward product begin to end in the norm and where their tiles
     grow, the bits of the forward op by op."""
+    assert tuple(ops.native().linear_norm_tiles(sum(lens), 384, K)[0] for K in (384, 1536)) == tiles
     m, inputs = _few_rows_encoder(12, sum(lens))
     ids, pos, off, longest = inputs(lens)
     out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
@@ -1011,10 +1014,15 @@ def test_product_and_norm_of_768_columns_in_one_launch(M, K, rows):
     assert got[5].isnan().all() and torch.equal(got[keep], want[keep])
 
 
-# 768 columns, K of 768 and 3072: around the row counts where the rule changes between product and norm, tiles of 64, of 96, and both
-@pytest.mark.parametrize("lens", [[7100], [7200], [10300], [10400], [16384], [16385], [21800], [20000, 4576], [24577], [34001], [41000], [46000]])
-def test_encoder_of_768_columns_where_products_take_the_norm(lens):
+# 768 columns, K of 768 and 3072: around the row counts where the rule changes between product and norm (0), tiles of 64, of 96, and both (the
+# rest in 64 behind leading rows in 96)
+@pytest.mark.parametrize("lens,tiles", [([7150], (0, 0)), ([7151], (64, 0)), ([10345], (64, 0)), ([10346], (64, 64)), ([16384], (64, 64)),
+                                        ([16385], (96, 0)), ([21760], (96, 96)), ([20000, 4576], (96, 96)), ([24577], (64, 0)),
+                                        ([34001], ((64, 24576), (64, 24576))), ([41000], (64, 0)), ([46000], (64, 96))])
+def test_encoder_of_768_columns_where_products_take_the_norm(lens, tiles):
     """The bits of the forward op by op."""
+    for K, t in zip((768, 3072), tiles):
+        assert ops.native().linear_norm_tiles(sum(lens), 768, K) == (t if isinstance(t, tuple) else (t, 0))
     m, inputs = _few_rows_encoder(12, sum(lens), hidden_size=768, intermediate_size=3072, head_dim=64)
     ids, pos, off, longest = inputs(lens)
     out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
@@ -1077,8 +1085,6 @@ def test_packed_prefill_of_rows_equals_grid(preset):
     from rag_tl_domainllm_optimizer_amd import models
     from rag_tl_domainllm_optimizer_amd.generation import KVCache
 
-    if preset not in models.config.PRESETS:
-        pytest.skip("no such preset")
     cfg = models.resolve_preset(preset)
     m = models.CausalLM(cfg, device=torch.device(DEV), dtype=torch.bfloat16, seed=0)
     lens, S = [30, 7, 1, 18], 30
@@ -1097,9 +1103,11 @@ def test_packed_prefill_of_rows_equals_grid(preset):
         assert not out[1][1].k[:, b, :, :s].any() and not out[1][1].v[:, b, :, :s].any()
 
 
-@pytest.mark.parametrize("lens", [[32768], [32769], [34000], [20000, 20000], [49200]])
-def test_encoder_of_384_columns_in_tiles_of_two_sizes(lens):
+@pytest.mark.parametrize("lens,tiles", [([32768], (128, 0)), ([32769], (64, 32768)), ([34000], (64, 32768)), ([20000, 20000], (64, 32768)),
+                                        ([49152], (64, 32768)), ([49200], (128, 0))])
+def test_encoder_of_384_columns_in_tiles_of_two_sizes(lens, tiles):
     """Around whole rounds of the larger tiles, whose rest goes in smaller ones: the bits of the forward op by op."""
+    assert all(ops.native().linear_norm_tiles(sum(lens), 384, K) == tiles for K in (384, 1536))
     m, inputs = _few_rows_encoder(12, sum(lens))
     ids, pos, off, longest = inputs(lens)
     out = torch.full((len(lens), m.cfg.hidden_size), 7.0, device=DEV)
