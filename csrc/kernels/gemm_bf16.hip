@@ -1582,18 +1582,27 @@ static int decode_split(int N, int K) {
 
 // Image products of 16 < M <= 64 rows: re-reading X per 16-row group, without a hand-off, is the cheaper way while X is small. us, direct | best
 // split of the other: 3072 x 1024 at M = 24 / 48 / 64 4.7 / 6.2 / 7.3 | 6.4 / 7.4 / 8.0; 2048 x 2048 at 24 / 32 / 48 6.8 / 7.5 / 9.4 | 7.1 / 7.2 / 8.2;
-// 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6.
-static bool gemm64_direct(int M, int N, int K) {
-  return tuning().decode_split == 0 && N <= 4096 && (long)M * K <= 1L << 16;
+// 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6; 4096 x 2048 at 32 / 40 / 48
+// 8.1 / 9.2 / 9.9 | 8.3 / 9.3 / 9.3 (10.2 with the four parts that other sizes take).
+// Other activations than these linear ones (and squared relu) run their code behind the hand-off, row tile by row tile, where the direct form's eight waves share it: its
+// lines lie higher. GELU: 1024 x 1536 at 48 / 64 8.4 / 9.8 | 9.7 / 10.8; 4096 x 2048 at 48 / 64 10.2 / 12.0 | 11.5 / 12.8 (4 parts 12.4 / 13.5);
+// 1024 x 4096 at 17 / 24 9.4 / 10.6 | 10.2 / 9.8; 4096 x 4096 at 17 / 24 10.2 / 11.4 | 12.8 / 12.3. 30 of 882 sizes by act (1024 to 8192 x 1024 to 4096, 17 to 64
+// rows) are slower than the better of the two by more than 5 %.
+static bool gemm64_direct(int M, int N, int K, bool linear) {
+  if (tuning().decode_split || N > 4096) return false;
+  const long x = (long)M * K;
+  if (linear) return x <= (N > 3072 && K <= 2048 ? 5L << 14 : 1L << 16);
+  return N > 2048 ? x <= 5L << 14 || (K <= 2560 && x <= 1L << 17) : x <= 17L << 12 || (K <= 2048 && x <= 3L << 15);
 }
-// Split over K: up to one workgroup per CU (half a round more costs more than it balances), up to four parts of at least 8 chunks (10 for the
-// gated pairs, whose partial tiles are twice as large), more of at least 16. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 19.8 / 14.6 /
+// Split over K: up to one workgroup per CU (half a round more costs more than it balances), three or four parts of at least 8 chunks, two of at least
+// 10 (8192 x 1024 in one / two of 8 at 17 / 48 / 64 rows 7.2 / 8.0 / 8.7 | 8.1 / 8.9 / 9.8, with GELU 9 to 13 % too), gated pairs, whose partial tiles are twice as large,
+// 10, more parts of at least 16. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 19.8 / 14.6 /
 // 12.6 / 11.7 / 14.3 / 14.6; 4096 x 14336 61.2 / 36.5 / 28.1 / 24.3 / 31.0 / 26.9; 6144 x 4096 20.9 / 15.8 / 19.2 / 16.5; 2048 x 7168 31.6 / 20.1 / 16.1 /
 // 13.7 / 12.6 / 12.8; 2048 x 2048 11.4 / 9.7 / 8.5 / 8.2 / 8.8 / 9.5; 10304 x 4096 (161 groups) 21.8 / 25.1 / 21.3; SwiGLU 14336 x 2048 17.9 / 16.0 / 20.2,
 // 7168 x 2048 17.1 / 13.7 / 12.8 / 13.1, 7168 x 4096 29.2 / 20.5 / 18.4 / 17.0.
 static int gemm64_split(int groups, int K, bool pair) {
   if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
-  auto least = [&](int parts) { return parts > 4 ? 16 : pair ? 10 : 8; };
+  auto least = [&](int parts) { return parts > 4 ? 16 : pair || parts == 2 ? 10 : 8; };
   int split = 1;
   while (split < 8 && groups * (split + 1) <= 256 && K / 64 >= least(split + 1) * (split + 1)) ++split;
   return split;
@@ -1689,7 +1698,8 @@ extern "C" int rt_gemm_nt_glu(const void* A, long lda, const void* B, long ldb, 
   } else if (M > 16 && wshuf && p.Rp == 0 && ldc % 4 == 0) {
     const bool pair = act == ACT_SWIGLU;
     const int rt = (M + 15) / 16, groups = pair ? (N + 127) / 128 : (N + 63) / 64;
-    const bool direct = !pair && gemm64_direct(M, N, K);
+    const bool linear = (act == ACT_NONE || act == ACT_RELU2) && (!R || (ldr % 4 == 0 && (uintptr_t)R % 8 == 0));
+    const bool direct = !pair && gemm64_direct(M, N, K, linear);
     // a ticket a wave, each on a line of its own
     const int split = direct || !slabs || !tickets || 128 * groups > RT_SPLITK_TICKETS
                           ? 1 : fit_split(gemm64_split(groups, K, pair), 4 * groups, 16 * rt * 16 * (pair ? 2 : 1) + 64);
