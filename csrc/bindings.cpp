@@ -1532,22 +1532,28 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
     norm(d, x, t[0], t[1], z);
     std::swap(x, z);
   } else {
-    // y = LN(in w^T + b + res): one launch where that is faster, the same bits
-    auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& y) {
+    // y = LN(in w^T + b + res): one launch where that is faster, the same bits. The sum of two launches stays until the layer is done, and y comes
+    // behind it: where the allocator then puts them (in the rows of qkv) they are still in the caches. With y made once and the sum freed at
+    // once, 2000 rows of MiniLM took 288 us instead of 276.
+    auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& sum, Tensor& y) {
       int first;
-      if (rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1), &first))
+      if (rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1), &first)) {
+        if (!y.defined()) y = rows(H);
         check_rc(rt_gemm_norm(in.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M,
                               (int)H, (int)in.size(1), (float)eps, 0, st),
                  "encoder: product and norm");
-      else
-        norm(encoder_linear(in, t[0], t[1], 0), res, lw, lb, y);
+      } else {
+        sum = encoder_linear(in, t[0], t[1], 0);
+        if (!y.defined()) y = rows(H);
+        norm(sum, res, lw, lb, y);
+      }
     };
-    Tensor y = rows(H);
     for (size_t l = 0; l < layers.size(); l += 12) {
       const Tensor* t = &layers[l];
+      Tensor sum, y;
       attend(encoder_linear(x, t[0], t[1], 0), a);
-      product_norm(a, t + 2, t[4], t[5], x, y);
-      product_norm(encoder_linear(y, t[6], t[7], 2), t + 8, t[10], t[11], y, x);
+      product_norm(a, t + 2, t[4], t[5], x, sum, y);
+      product_norm(encoder_linear(y, t[6], t[7], 2), t + 8, t[10], t[11], y, sum, x);
     }
   }
   check_rc(rt_pool_norm(x.data_ptr(), nullptr, (const long*)off.data_ptr(), M, (int)B, 0, (int)H, normalize ? 1 : 0,
