@@ -909,7 +909,6 @@ Tensor embed(const Tensor& table, const Tensor& ids, const optional<Tensor>& pta
   return out;
 }
 
-// src [N, H] (row stride % 8 == 0) -> out [R, H]: out[r] = src[inv[r]] or zeros where inv[r] < 0
 // K and V of packed rows into cache slots [0, S) (see kv_append_rows_kernel); inv int32 [B S]
 void kv_append_rows(const Tensor& qkv, const Tensor& inv, int64_t S, int64_t Hq, Tensor kc, Tensor vc) {
   CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_ROWS(qkv); CHECK_ALIGN16(qkv); CHECK_CUDA(inv); CHECK_I32(inv);
@@ -925,6 +924,7 @@ void kv_append_rows(const Tensor& qkv, const Tensor& inv, int64_t S, int64_t Hq,
            "kv_append_rows");
 }
 
+// src [N, H] (row stride % 8 == 0) -> out [R, H]: out[r] = src[inv[r]] or zeros where inv[r] < 0
 Tensor rows_scatter(const Tensor& src, const Tensor& inv, int64_t R) {
   CHECK_CUDA(src); CHECK_BF16(src); CHECK_CUDA(inv);
   TORCH_CHECK(src.dim() == 2 && src.stride(1) == 1 && src.stride(0) % 8 == 0, "rows_scatter: [N, H] rows expected");

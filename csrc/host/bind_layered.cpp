@@ -6,7 +6,6 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
-#include <mutex>
 #include <vector>
 
 #include "host/settled.h"

@@ -15,7 +15,7 @@ from .attention import (  # noqa: F401
     attention, attention_packed, decode_attention, decode_step_attention, decode_workspace, flash_attention_packed, gather_rows, packed_inverse, prefill_attention_rows, scatter_rows,
     flash_attention_qkv, rope_qkv, rope_qkv_, FP8_KV_D, kv_dequantize, kv_quantize_rows, kv_store_fp8,
 )
-from .misc import (check_lost, embedding, gae, ivf_probes, ivf_scan, ppo_advantages, pool_normalize, pool_normalize_packed, ppo_loss, row_dot, sample, segment_mean,  # noqa: F401
+from .misc import (check_lost, embedding, gae, ivf_probes, ivf_scan, ivf_scores, ppo_advantages, pool_normalize, pool_normalize_packed, ppo_loss, row_dot, sample, segment_mean,  # noqa: F401
                    swiglu, token_logprobs, topk, upload)
 from .optim import FlatParams, FusedAdamW, MixedFlatParams, flat_params  # noqa: F401
 from .fp8 import Fp8Cache, dequantize_fp8, gemm_fp8, quantize_fp8  # noqa: F401

@@ -206,9 +206,9 @@ def check_lost(device):
         native().raise_lost(torch.cuda.current_device() if device.index is None else device.index)
 
 
-def ivf_probes(q, cen, nlist: int, k: int, pen=None):
-    """The ``k`` lists that each query probes on a GPU, the best of its scores q cen[:nlist]^T - pen -> (q in bf16, int32 indices
-    [nq, k]). Up to 16 fp32 queries are rounded and multiplied in one launch, with :func:`gemm`'s bits."""
+def ivf_scores(q, cen, nlist: int, pen=None):
+    """(q in bf16, q cen[:nlist]^T - pen in fp32) on a GPU. Up to 16 fp32 queries are rounded and multiplied in one launch, with
+    :func:`gemm`'s bits."""
     q = q.contiguous()
     few = q.dtype == torch.float32 and q.dim() == 2 and 0 < q.shape[0] <= 16 and not batch_invariant_on()
     both = native().ivf_coarse(q, cen, nlist, pen) if few else None
@@ -219,6 +219,12 @@ def ivf_probes(q, cen, nlist: int, k: int, pen=None):
         s = gemm(q, cen, out_f32=True)[:, :nlist]  # the operand's padding rows stay out of the selection
         if pen is not None:
             s.sub_(pen)
+    return q, s
+
+
+def ivf_probes(q, cen, nlist: int, k: int, pen=None):
+    """The ``k`` lists that each query probes on a GPU, the best of :func:`ivf_scores` -> (q in bf16, int32 indices [nq, k])."""
+    q, s = ivf_scores(q, cen, nlist, pen)
     return q, native().topk_index(s, k) if k <= 512 else topk(s, k)[1].int()
 
 

@@ -171,10 +171,7 @@ class IVFIndex:
     def _coarse(self, x: torch.Tensor, k: int) -> torch.Tensor:
         """indices [n, k] of the k best centroids per row (x already on device)."""
         if self.gpu:
-            # the operand's padding rows stay out of the selection
-            s = ops.gemm(x.to(self.dtype).contiguous(), self._cen_op, out_f32=True)[:, :self.centroids.shape[0]]
-            if self.metric == "l2":
-                s.sub_(self._pen)
+            s = ops.ivf_scores(x, self._cen_op, self.centroids.shape[0], self._pen if self.metric == "l2" else None)[1]
             return ops.topk(s, k)[1]
         s = x.float() @ self._cen_op.t() - self._pen
         return torch.topk(s, k, dim=-1).indices
