@@ -1,5 +1,5 @@
-// Forwards that gave up a bounded wait of theirs (encoder_few.hip). The kernel writes a word of pinned host memory, one a device, and the host looks at
-// it without waiting for anything: at the next forward, and wherever the package has just waited for results.
+// Forwards that gave up a bounded wait of theirs (encoder_few.hip). The kernel writes a word of pinned host memory, one a device, and the host
+// looks at it without waiting for anything: at the next forward, and wherever the package has just waited for results.
 #pragma once
 #include <c10/hip/HIPException.h>
 #include <c10/hip/HIPGraphsC10Utils.h>

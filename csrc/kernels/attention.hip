@@ -153,8 +153,8 @@ __device__ __forceinline__ int v_off(int r, int c) {
 // 64 20.0 -> 13.5, with a bias 32.4 -> 24.6.
 //
 // a.first: rows of real positions only, tiled by position all the same (a pad's key is read from a real row and masked, its value
-// is zero as in a grid: the same bits). 32 prompts of 90 to 320 tokens had needed a grid filled, and read for the cache, and results gathered: 79 us a layer beside 87 here, now 13
-// beside 83 (Mistral-7B, four layers, 8247 -> 7985).
+// is zero as in a grid: the same bits). 32 prompts of 90 to 320 tokens had needed a grid filled, and read for the cache, and results gathered:
+// 79 us a layer beside 87 here, now 13 beside 83 (Mistral-7B, four layers, 8247 -> 7985).
 template <int D, int NU = 2, bool HP = false, bool Q64 = false, bool RB = false>
 __global__ __launch_bounds__(Q64 ? 256 : 64 * 8 / NU, D == 128 ? 2 : (D == 64 ? 3 : 4))
 void attn_fwd_kernel(AttnArgs a) {
@@ -1332,8 +1332,8 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_g1_fp8_kernel(DecodeFused
 // counted waits keep the prefetch in flight). The launch bound holds every form to 256 registers, 2
 // waves per SIMD: all 2048 waves of a batch-256 layer, or two workgroups of 4 waves per CU, are resident
 // (unbounded, the 4-wave form took 268 with its accumulators and ran one workgroup per CU: 48 rows of
-// 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every rotary-table / q /
-// k_new / v_new (or slab) load at once and the first tiles behind them: loads return in order, so the other way round
+// 150..1200 keys 49 -> 41 us; the third tile: one wave, 48 rows 91 -> 71, 256 rows of 150..300 54 -> 52). The prologue issues every
+// rotary-table / q / k_new / v_new (or slab) load at once and the first tiles behind them: loads return in order, so the other way round
 // it waited for 24 KB a wave. Loads are unconditional, refills past the end too: behind a load under a condition
 // the compiler waits for every load at the join, and so had the three tiles arrive before the first was used, each time
 // (and lengths, slot and position one after the other: 3 trips). But nothing is refilled unless a fourth tile follows: 128

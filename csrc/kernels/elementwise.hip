@@ -149,8 +149,8 @@ __global__ __launch_bounds__(256) void rows_scatter_kernel(const bf16_t* __restr
 }
 
 // K / V of packed qkv rows into cache slots [0, S): slot s of row b from row inv[b S + s], zeros (a pad's) where that is negative. Two
-// 16-byte accesses a thread, whole cache rows; bound by their bytes: 32 x 320 slots of 8 heads of 128, 6250 of them with rows, 13.2 us, where the grid's fill and the append that
-// read it took 61.
+// 16-byte accesses a thread, whole cache rows; bound by their bytes: 32 x 320 slots of 8 heads of 128, 6250 of them with rows, 13.2 us, where
+// the grid's fill and the append that read it took 61.
 __global__ __launch_bounds__(256) void kv_append_rows_kernel(const bf16_t* __restrict__ qkv, long ld, const int* __restrict__ inv, int B, int S,
                                                              int Hq, int Hkv, int D, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, int Smax,
                                                              long N) {

@@ -63,7 +63,8 @@ __device__ __forceinline__ void dma16(const bf16_t* from, char* to) { __builtin_
 constexpr int SC1 = 16;
 __device__ __forceinline__ bool there(const u32x4& v) { return v[0] != NONE && v[1] != NONE && v[2] != NONE && v[3] != NONE; }
 // v[i] = load(i) until every lane's words are results. Waits are bounded: who has asked in vain `tries` times says so to the launch, which
-// gives up (each waiting wave looks every 1024 times), and to the host. Both are beside `lost` and not arguments: the kernel has no register for them.
+// gives up (each waiting wave looks every 1024 times), and to the host. Both are beside `lost` and not arguments: the kernel has no register
+// for them.
 template <int N, typename F>
 __device__ __forceinline__ void await(unsigned* lost, u32x4 (&v)[N], F load) {
   for (int tries = 0;; ++tries) {

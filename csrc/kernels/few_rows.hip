@@ -6,8 +6,8 @@
 // bits are that kernel's: a text's embedding does not depend on the way it went. The 8 waves of a workgroup are parts x row tiles
 // x column groups of 16; a wave has most of its weights (and of x) in flight at once, and partial sums meet in LDS. They come by
 // LDS-DMA, eight lanes to a row's 128 B, into places of the wave's own: loads straight in MFMA order, whose adjacent lanes are in
-// different rows, keep the CU's address path busy for 64 cycles each, these for 16 (profiles/calls/load_order.txt). With a norm ahead every workgroup normalises
-// the rows itself, two or four to a wave, over the weights' trip (12 KB from L2, where a kernel of its own costs a launch and
+// different rows, keep the CU's address path busy for 64 cycles each, these for 16 (profiles/calls/load_order.txt). With a norm ahead every
+// workgroup normalises the rows itself, two or four to a wave, over the weights' trip (12 KB from L2, where a kernel of its own costs a launch and
 // another trip); workgroup 0 also writes them.
 // Bound by latency. 15 rows, us, gemm_decode_kernel -> MFMA-order loads -> this: 1152 x 384 5.2 -> 4.5 -> 4.0, 384 x 384 (4.5 -> 4.0),
 // 384 x 1536 9.8 -> 5.8 -> 4.4, and 2.9 of the norm with it. MiniLM over 15 / 32 rows 157 -> 141 / 201 -> 167, mpnet-base (and with

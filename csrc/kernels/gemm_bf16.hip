@@ -643,12 +643,12 @@ __global__ __launch_bounds__(64 * NW) void gemv64_kernel(GemmArgs p) {
 // and weights come in plain loads, DEPTH - 1 chunks ahead: with LDS-DMA for X the compiler waits for everything in flight
 // wherever it needs a weight register (SwiGLU 28672 x 4096 at M = 24: 49 us instead of 44). Few column groups are split
 // over K (gemm64_split): partial tiles in write-through slabs, the last arriver adds them in their order. A wave hands over for itself
-// (its columns are no other's), by 16-byte stores of whole lines and a ticket on a line of its own, and asks for all rows' tiles at once; bias and residual
-// are asked for ahead of it. Of 4096 x 4096 at 48 rows (11.7 us) 2.0 pass until the first chunk is there, 4.6 in the loop (7.3 TB/s), 1.4 until the
-// ticket is back, 1.2 until the parts are there, 0.7 in the epilogue, the rest between launches. us with the whole workgroup at one ticket and the
-// activations' code in the epilogue -> this, M = 24 / 48 / 64: 6144 x 4096 with norm 14.9 / 17.6 / 19.6 -> 13.8 / 15.6 / 16.8, 4096 x 4096 + residual
-// 10.9 / 13.5 / 15.2 -> 10.6 / 11.7 / 12.6, 4096 x 14336 23.5 / 26.2 / 28.9 -> 22.3 / 24.2 / 26.2, 2048 x 7168 12.1 / 14.5 / 16.5 -> 10.6 / 12.8 / 13.9.
-// More chunks in flight (6, 8), fragments read a chunk ahead: nothing.
+// (its columns are no other's), by 16-byte stores of whole lines and a ticket on a line of its own, and asks for all rows' tiles at once; bias
+// and residual are asked for ahead of it. Of 4096 x 4096 at 48 rows (11.7 us) 2.0 pass until the first chunk is there, 4.6 in the loop (7.3
+// TB/s), 1.4 until the ticket is back, 1.2 until the parts are there, 0.7 in the epilogue, the rest between launches. us with the whole
+// workgroup at one ticket and the activations' code in the epilogue -> this, M = 24 / 48 / 64: 6144 x 4096 with norm 14.9 / 17.6 / 19.6 -> 13.8
+// / 15.6 / 16.8, 4096 x 4096 + residual 10.9 / 13.5 / 15.2 -> 10.6 / 11.7 / 12.6, 4096 x 14336 23.5 / 26.2 / 28.9 -> 22.3 / 24.2 / 26.2, 2048 x
+// 7168 12.1 / 14.5 / 16.5 -> 10.6 / 12.8 / 13.9. More chunks in flight (6, 8), fragments read a chunk ahead: nothing.
 template <bool OUT_F32, int RT, bool PAIR>
 __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __restrict__ slabs,
                                                            unsigned* __restrict__ tickets, int split) {
@@ -1581,13 +1581,13 @@ static int decode_split(int N, int K) {
 }
 
 // Image products of 16 < M <= 64 rows: re-reading X per 16-row group, without a hand-off, is the cheaper way while X is small. us, direct | best
-// split of the other: 3072 x 1024 at M = 24 / 48 / 64 4.7 / 6.2 / 7.3 | 6.4 / 7.4 / 8.0; 2048 x 2048 at 24 / 32 / 48 6.8 / 7.5 / 9.4 | 7.1 / 7.2 / 8.2;
-// 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6; 4096 x 2048 at 32 / 40 / 48
-// 8.1 / 9.2 / 9.9 | 8.3 / 9.3 / 9.3 (10.2 with the four parts that other sizes take).
-// Other activations than these (linear, relu, squared relu) run their code behind the hand-off, row tile by row tile, where the direct form's eight waves share it: its
-// lines lie higher. GELU: 1024 x 1536 at 48 / 64 8.4 / 9.8 | 9.7 / 10.8; 4096 x 2048 at 48 / 64 10.2 / 12.0 | 11.5 / 12.8 (4 parts 12.4 / 13.5);
-// 1024 x 4096 at 17 / 24 9.4 / 10.6 | 10.2 / 9.8; 4096 x 4096 at 17 / 24 10.2 / 11.4 | 12.8 / 12.3. 30 of 882 sizes by act (1024 to 8192 x 1024 to 4096, 17 to 64
-// rows) are slower than the better of the two by more than 5 %.
+// split of the other: 3072 x 1024 at M = 24 / 48 / 64 4.7 / 6.2 / 7.3 | 6.4 / 7.4 / 8.0; 2048 x 2048 at 24 / 32 / 48 6.8 / 7.5 / 9.4 | 7.1 /
+// 7.2 / 8.2; 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6; 4096 x 2048 at
+// 32 / 40 / 48 8.1 / 9.2 / 9.9 | 8.3 / 9.3 / 9.3 (10.2 with the four parts that other sizes take).
+// Other activations than these (linear, relu, squared relu) run their code behind the hand-off, row tile by row tile, where the direct form's
+// eight waves share it: its lines lie higher. GELU: 1024 x 1536 at 48 / 64 8.4 / 9.8 | 9.7 / 10.8; 4096 x 2048 at 48 / 64 10.2 / 12.0 | 11.5 /
+// 12.8 (4 parts 12.4 / 13.5); 1024 x 4096 at 17 / 24 9.4 / 10.6 | 10.2 / 9.8; 4096 x 4096 at 17 / 24 10.2 / 11.4 | 12.8 / 12.3. 7 of 588 forms
+// (GELU and silu, 1024 to 8192 x 1024 to 4096, 17 to 64 rows) are slower than the best of these and the splits by more than 5 %.
 static bool gemm64_direct(int M, int N, int K, bool linear) {
   if (tuning().decode_split || N > 4096) return false;
   const long x = (long)M * K;
@@ -1595,11 +1595,11 @@ static bool gemm64_direct(int M, int N, int K, bool linear) {
   return N > 2048 ? x <= 5L << 14 || (K <= 2560 && x <= 1L << 17) : x <= 17L << 12 || (K <= 2048 && x <= 3L << 15);
 }
 // Split over K: up to one workgroup per CU (half a round more costs more than it balances), three or four parts of at least 8 chunks, two of at least
-// 10 (8192 x 1024 in one / two of 8 at 17 / 48 / 64 rows 7.2 / 8.0 / 8.7 | 8.1 / 8.9 / 9.8, with GELU 9 to 13 % too), gated pairs, whose partial tiles are twice as large,
-// 10, more parts of at least 16. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 19.8 / 14.6 /
-// 12.6 / 11.7 / 14.3 / 14.6; 4096 x 14336 61.2 / 36.5 / 28.1 / 24.3 / 31.0 / 26.9; 6144 x 4096 20.9 / 15.8 / 19.2 / 16.5; 2048 x 7168 31.6 / 20.1 / 16.1 /
-// 13.7 / 12.6 / 12.8; 2048 x 2048 11.4 / 9.7 / 8.5 / 8.2 / 8.8 / 9.5; 10304 x 4096 (161 groups) 21.8 / 25.1 / 21.3; SwiGLU 14336 x 2048 17.9 / 16.0 / 20.2,
-// 7168 x 2048 17.1 / 13.7 / 12.8 / 13.1, 7168 x 4096 29.2 / 20.5 / 18.4 / 17.0.
+// 10 (8192 x 1024 in one / two of 8 at 17 / 48 / 64 rows 7.2 / 8.0 / 8.7 | 8.1 / 8.9 / 9.8, with GELU 9 to 13 % too), gated pairs, whose
+// partial tiles are twice as large, 10, more parts of at least 16. us unsplit / 2 / 3 / 4 / 6 / 8 parts at M = 48: 4096 x 4096 19.8 / 14.6 /
+// 12.6 / 11.7 / 14.3 / 14.6; 4096 x 14336 61.2 / 36.5 / 28.1 / 24.3 / 31.0 / 26.9; 6144 x 4096 20.9 / 15.8 / 19.2 / 16.5; 2048 x 7168 31.6 /
+// 20.1 / 16.1 / 13.7 / 12.6 / 12.8; 2048 x 2048 11.4 / 9.7 / 8.5 / 8.2 / 8.8 / 9.5; 10304 x 4096 (161 groups) 21.8 / 25.1 / 21.3; SwiGLU 14336
+// x 2048 17.9 / 16.0 / 20.2, 7168 x 2048 17.1 / 13.7 / 12.8 / 13.1, 7168 x 4096 29.2 / 20.5 / 18.4 / 17.0.
 static int gemm64_split(int groups, int K, bool pair) {
   if (tuning().decode_split > 0) return std::min(tuning().decode_split, K / 64);
   auto least = [&](int parts) { return parts > 4 ? 16 : pair || parts == 2 ? 10 : 8; };

@@ -1,8 +1,9 @@
 // y = LN(x w^T + bias + res) of rows that a workgroup holds whole: the two products of a post-norm encoder layer that end in a layer norm.
 // As two launches the sum went out to memory and back between them, and 384 columns are one and a half tiles of 256: a quarter of the
-// matrix work was for columns that are not there; 768 are three tiles of 256, whose rounds leave CUs idle. us, product and norm -> this, by 384 columns: 28100 rows x 384 33.7 -> 18.8, x 1536
-// 55.5 -> 35.8; 15000 rows 22.6 -> 12.0, 35.1 -> 23.8; 8960 rows 16.6 -> 10.4, 25.5 -> 22.0. By 768 columns, in an encoder: 24000 rows x 768 54.9 -> 37.5, x 3072 121 -> 99, 12000 rows 35.9 -> 24.4, 73.6 -> 67.
-// Encoder forward of 1024 texts (MiniLM) 3775 -> 3446, of mpnet-base over 12000 / 24000 / 49000 rows 3030 -> 2813 / 5150 -> 4790 / 10390 -> 9740.
+// matrix work was for columns that are not there; 768 are three tiles of 256, whose rounds leave CUs idle. us, product and norm -> this, by 384
+// columns: 28100 rows x 384 33.7 -> 18.8, x 1536 55.5 -> 35.8; 15000 rows 22.6 -> 12.0, 35.1 -> 23.8; 8960 rows 16.6 -> 10.4, 25.5 -> 22.0. By
+// 768 columns, in an encoder: 24000 rows x 768 54.9 -> 37.5, x 3072 121 -> 99, 12000 rows 35.9 -> 24.4, 73.6 -> 67. Encoder forward of 1024
+// texts (MiniLM) 3775 -> 3446, of mpnet-base over 12000 / 24000 / 49000 rows 3030 -> 2813 / 5150 -> 4790 / 10390 -> 9740.
 #include "rt_common.h"
 
 #include <algorithm>
@@ -63,10 +64,10 @@ __device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, uint4 v, uint3
 // stay for the step, each phase multiplies them by FG of its w fragments (a granule: 128 columns, 16 FG of every wave). While a phase is
 // multiplied the next one's fragments are read, and the places that are read out are asked for again: 7 granules and 3 x images ahead.
 // Behind the last step nothing is fetched: the same loads go out of range, which fills their places with zeros and keeps the counted waits.
-// 96 rows by 768 columns (64 do not fill the matrix cores' time, of 128 neither sums nor rows fit): x fragments come in a burst of 12 a wave at the end of a
-// step, 3270 cycles of which the matrix cores work 2320. Cycles a step of 128 / 64 rows by 384 columns: 2090 / 1300, of which the matrix cores work 1546 / 773 and the LDS pipe 1790 / 1310 (fragments
-// and DMA), which bounds it. Waves 2 x 4 read the least of 128 rows, 1 x 8 of 64. w straight from memory to the one wave that
-// multiplies it (1 x 8) took 3200: its lanes lie 16 rows apart, one line a lane.
+// 96 rows by 768 columns (64 do not fill the matrix cores' time, of 128 neither sums nor rows fit): x fragments come in a burst of 12 a wave at
+// the end of a step, 3270 cycles of which the matrix cores work 2320. Cycles a step of 128 / 64 rows by 384 columns: 2090 / 1300, of which the
+// matrix cores work 1546 / 773 and the LDS pipe 1790 / 1310 (fragments and DMA), which bounds it. Waves 2 x 4 read the least of 128 rows, 1 x 8
+// of 64. w straight from memory to the one wave that multiplies it (1 x 8) took 3200: its lanes lie 16 rows apart, one line a lane.
 template <int WC, int FM, int NP>
 __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   constexpr int TM = 8 / WC * 16 * FM, TN = 128 * NP, FG = 8 / WC, FN = FG * NP, NA = (TM + 63) / 64, XI = TM * 128, GR = 128 * 128, LDT = TN + 8;
@@ -144,9 +145,9 @@ __global__ __launch_bounds__(512, 2) void gemm_norm_kernel(Args p) {
   if constexpr (!LATE) operands();
 
   // All of w, each workgroup its share, in whole rows: the products that go through the caches between two of this one leave nothing of
-  // w there, and a K-step of it is a line of 128 B from each of TN rows, which all workgroups ask for at the same time, only 7 granules ahead. Its place is
-  // one that this wave fills itself later (loads come in in their order). In an encoder, 768 columns: 12000 rows x 3072 101 -> 67 us, x 768
-  // 32.2 -> 24.4, 24000 rows x 3072 123 -> 99.
+  // w there, and a K-step of it is a line of 128 B from each of TN rows, which all workgroups ask for at the same time, only 7 granules ahead.
+  // Its place is one that this wave fills itself later (loads come in in their order). In an encoder, 768 columns: 12000 rows x 3072 101 -> 67
+  // us, x 768 32.2 -> 24.4, 24000 rows x 3072 123 -> 99.
   const uint32_t share = (uint32_t)(((long)TN * p.ldw * 2 / gridDim.x + 8191) / 8192);
   for (uint32_t k = 0; k < min(share, 6u); ++k)
     dma16(Wr, smem + (AP - 1) * XI + (TM == 128 ? 2 * wid : wid) * 1024, ((blockIdx.x * share + k) * 8 + wid) * 1024 + lane * 16);
@@ -310,13 +311,14 @@ static bool fits(int N, int K) { return (N == 384 || N == 768) && K >= 64 && K %
 // Rows of a tile with which rt_gemm_norm beats product and norm, `first` leading rows in larger ones; 0: it doesn't, or the shape is not for it.
 // A tile is one chain over K, however few there are: with few rows the product's small tiles in parallel are faster.
 // 384 columns: 0.54 us a step of 64 rows and 6 besides (128 rows: 0.9 and 8). Even: 2500 rows at K 128, 3000 at 384, 4500 at 768, 5300 at 1536,
-// 10500 at 3072; between an encoder's other kernels not below 4000 (a forward of 3000 rows 360 -> 368). Tiles of 64 while they are one round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles
-// of 64 42.6), whole rounds of these and the rest in 64 where that is one round more (MiniLM over 34000 rows 1434 -> 1396 us).
-// 768 columns, us within an encoder's forward (between other kernels: alone, with w in the caches, both are faster): a round of tiles of 64 takes
-// 10 and 1.18 a step, nearly full 14 and 1.25, one of several 6.4 and 1.53; of 96 18 and 1.72. Product and norm: tiles of 256 x 256, whole rounds of
-// them and a rest, and 0.78 ns a row. All of one size, or whole rounds of 96 and the rest in 64. Product and norm | this at K 768: 12000 rows 35.9 |
-// 24.4, 20000 42.7 | 34.0, 24000 54.9 | 37.5, 28000 59.3 | 49.4, 42000 88 | 73; at K 3072: 12000 73.6 | 67, 20000 89.6 | 90 (not taken), 24000 121 | 99, 28000
-// 146 | 160 (not taken), 49000 237 | 204.
+// 10500 at 3072; between an encoder's other kernels not below 4000 (forwards of 3000 / 3600 / 3990 rows 362 / 387 / 392 -> 366 / 392 / 398).
+// Tiles of 64 while they are one round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles of 64 42.6),
+// whole rounds of these and the rest in 64 where that is one round more (MiniLM over 34000 rows 1434 -> 1396 us). 768 columns, us within an
+// encoder's forward (between other kernels: alone, with w in the caches, both are faster): a round of tiles of 64 takes 10 and 1.18 a step,
+// nearly full 14 and 1.25, one of several 6.4 and 1.53; of 96 18 and 1.72. Product and norm: tiles of 256 x 256, whole rounds of them and a
+// rest, and 0.78 ns a row. All of one size, or whole rounds of 96 and the rest in 64. Product and norm | this at K 768: 12000 rows 35.9 | 24.4,
+// 20000 42.7 | 34.0, 24000 54.9 | 37.5, 28000 59.3 | 49.4, 42000 88 | 73; at K 3072: 12000 73.6 | 67, 20000 89.6 | 90 (not taken), 24000 121 |
+// 99, 28000 146 | 160 (not taken), 49000 237 | 204.
 extern "C" int rt_gemm_norm_rows(int M, int N, int K, int* first) {
   *first = 0;
   if (!fits(N, K)) return 0;

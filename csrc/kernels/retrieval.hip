@@ -463,10 +463,10 @@ __global__ __launch_bounds__(64) void ivf_probe_kernel(const bf16_t* __restrict_
   }
 }
 
-// The same of 256 < d <= 384 and lists that are even or at most 4096 long: a wave per 16 vectors, whose pieces are all in flight as MFMA fragments at once, the query as the other
-// operand's sixteen rows. A single query over 16 lists of 200 and of 780, 7.3 -> 5.2 and 7.5 -> 5.8 us; many queries over
-// lists of 100 20.3 -> 16.4 (64 x 16 of 4096), 53 -> 49 (256 x 16). Smaller d leaves the wave with too little in flight (128: 1.3 to 1.5 times
-// the time), 768 takes half the waves away (1.0 to 1.15 times); one and two queries over skewed
+// The same of 256 < d <= 384 and lists that are even or at most 4096 long: a wave per 16 vectors, whose pieces are all in flight as MFMA
+// fragments at once, the query as the other operand's sixteen rows. A single query over 16 lists of 200 and of 780, 7.3 -> 5.2 and 7.5 -> 5.8
+// us; many queries over lists of 100 20.3 -> 16.4 (64 x 16 of 4096), 53 -> 49 (256 x 16). Smaller d leaves the wave with too little in flight
+// (128: 1.3 to 1.5 times the time), 768 takes half the waves away (1.0 to 1.15 times); one and two queries over skewed
 // lists of up to 7909 16.7 against 15.9 and 29.7 against 27.6, over even ones of up to 8735 11.1 against 12.3 and 18.5 against 19.6.
 constexpr int PF = 12;
 __global__ __launch_bounds__(256, 4) void ivf_probe16_kernel(ScanArgs a) {
