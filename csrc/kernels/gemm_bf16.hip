@@ -822,10 +822,10 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
           }
     }
   }
-  // Linear, relu and relu^2 on their own: the others' code, once an element, lies between what these run, and every jump over it is a
+  // Linear and relu^2 on their own: the others' code, once an element, lies between what these run, and every jump over it is a
   // wait for instructions that no cache holds (an epilogue of 1.25 us, now 0.7)
-  if (!PAIR && (p.act == ACT_NONE || p.act == ACT_RELU || p.act == ACT_RELU2) && (!p.R || r4)) {
-    const bool relu = p.act == ACT_RELU, relu2 = p.act == ACT_RELU2;
+  if (!PAIR && (p.act == ACT_NONE || p.act == ACT_RELU2) && (!p.R || r4)) {
+    const bool relu2 = p.act == ACT_RELU2;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       const int row = 16 * t + frow;
@@ -838,7 +838,7 @@ __global__ __launch_bounds__(256) void gemm64_image_kernel(GemmArgs p, float* __
         y[e] = acc[t][0][e] * rs;
         y[e] = p.bias ? y[e] + bias[0][e] : y[e];
         const float q = fmaxf(y[e], 0.f);
-        y[e] = relu2 ? q * q : relu ? q : y[e];
+        y[e] = relu2 ? q * q : y[e];
         y[e] = p.R ? y[e] + r[e] : y[e];
       }
       if (row < p.M && col < n_out) {
@@ -1584,7 +1584,7 @@ static int decode_split(int N, int K) {
 // split of the other: 3072 x 1024 at M = 24 / 48 / 64 4.7 / 6.2 / 7.3 | 6.4 / 7.4 / 8.0; 2048 x 2048 at 24 / 32 / 48 6.8 / 7.5 / 9.4 | 7.1 /
 // 7.2 / 8.2; 3072 x 3072 at 17 / 24 8.2 / 9.3 | 8.5 / 8.5; 4096 x 4096 at 17 / 24 / 32 9.7 / 10.8 / 12.0 | 10.4 / 10.4 / 10.6; 4096 x 2048 at
 // 32 / 40 / 48 8.1 / 9.2 / 9.9 | 8.3 / 9.3 / 9.3 (10.2 with the four parts that other sizes take).
-// Other activations than these (linear, relu, squared relu) run their code behind the hand-off, row tile by row tile, where the direct form's
+// Other activations than these (linear, squared relu) run their code behind the hand-off, row tile by row tile, where the direct form's
 // eight waves share it: its lines lie higher. GELU: 1024 x 1536 at 48 / 64 8.4 / 9.8 | 9.7 / 10.8; 4096 x 2048 at 48 / 64 10.2 / 12.0 | 11.5 /
 // 12.8 (4 parts 12.4 / 13.5); 1024 x 4096 at 17 / 24 9.4 / 10.6 | 10.2 / 9.8; 4096 x 4096 at 17 / 24 10.2 / 11.4 | 12.8 / 12.3. 7 of 588 forms
 // (GELU and silu, 1024 to 8192 x 1024 to 4096, 17 to 64 rows) are slower than the best of these and the splits by more than 5 %.
@@ -1698,7 +1698,7 @@ extern "C" int rt_gemm_nt_glu(const void* A, long lda, const void* B, long ldb, 
   } else if (M > 16 && wshuf && p.Rp == 0 && ldc % 4 == 0) {
     const bool pair = act == ACT_SWIGLU;
     const int rt = (M + 15) / 16, groups = pair ? (N + 127) / 128 : (N + 63) / 64;
-    const bool linear = (act == ACT_NONE || act == ACT_RELU || act == ACT_RELU2) && (!R || (ldr % 4 == 0 && (uintptr_t)R % 8 == 0));
+    const bool linear = (act == ACT_NONE || act == ACT_RELU2) && (!R || (ldr % 4 == 0 && (uintptr_t)R % 8 == 0));
     const bool direct = !pair && gemm64_direct(M, N, K, linear);
     // a ticket a wave, each on a line of its own
     const int split = direct || !slabs || !tickets || 128 * groups > RT_SPLITK_TICKETS

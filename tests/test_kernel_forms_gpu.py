@@ -429,10 +429,10 @@ def test_image_products_17_to_64_rows(N, K, act):
                 assert (out[:, No:] == 7).all()
 
 
-@pytest.mark.parametrize("act", [0, ops.ACT_RELU2, 1, 2, 4])
+@pytest.mark.parametrize("act", [0, ops.ACT_RELU2, 2, 4])
 @pytest.mark.parametrize("N,K,split", [(2064, 2176, 0), (4176, 1088, 0), (4176, 1088, 5), (208, 6144, 8), (3104, 2048, 0), (5136, 1024, 0)])
 def test_image_products_17_to_64_rows_epilogues(N, K, split, act):
-    """Linear, relu and squared-relu results, whose epilogue is their own, and the others', behind parts of K and without: residuals that come
+    """Linear and squared-relu results, whose epilogue is their own, and the others', behind parts of K and without: residuals that come
     four at a time and ones that do not, with and without bias, a last column group that is not whole."""
     C = ops.native()
     g = torch.Generator(device=DEV).manual_seed(N + act)
