@@ -1371,19 +1371,23 @@ std::vector<Tensor> few_rows(const Tensor& x, const Tensor& w, const optional<Te
   return {y, xo};
 }
 
-// y = act(x w^T + b), the kernel chosen as ops.gemm chooses it
-static Tensor encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act) {
+// y = act(x w^T + b) to a given y, the kernel chosen as ops.gemm chooses it
+static void encoder_linear(const Tensor& x, const Tensor& w, const Tensor& b, int64_t act, const Tensor& y) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  if (M <= 64 && N % 8 == 0) return gemm(x, w, std::nullopt, std::nullopt, b, act, false, std::nullopt, std::nullopt, 0.0, false, {});
+  if (M <= 64 && N % 8 == 0) {
+    gemm(x, w, std::nullopt, std::nullopt, b, act, false, y, std::nullopt, 0.0, false, {});
+    return;
+  }
   int bn = 0;
   const int split = rt_token_plan((int)M, (int)N, (int)K, (int)act, &bn);
-  if (rt_small_tiles((int)M, (int)N, (int)K, (int)act))
-    return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, split, std::nullopt, std::nullopt, std::nullopt, 0, {});
-  if (split > 1) {
+  if (rt_small_tiles((int)M, (int)N, (int)K, (int)act)) {
+    gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, split, y, std::nullopt, std::nullopt, 0, {});
+  } else if (split > 1) {
     auto slabs = at::empty({split * M * N}, x.options().dtype(at::kFloat));
-    return gemm_splitk(x, w, split, slabs, b, act, std::nullopt, std::nullopt, bn, {});
+    gemm_splitk(x, w, split, slabs, b, act, y, std::nullopt, bn, {});
+  } else {
+    gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, 1, y, std::nullopt, std::nullopt, bn, {});
   }
-  return gemm_big(x, w, 0, 0, std::nullopt, std::nullopt, b, act, 0, 1, std::nullopt, std::nullopt, std::nullopt, bn, {});
 }
 
 // LN(x w^T + bias + res) in one launch, tiles of `rows` rows (0: as rt_gemm_norm_rows says); contiguous bf16
@@ -1532,28 +1536,34 @@ bool encoder_packed(const Tensor& ids, const Tensor& pos, const Tensor& off, int
     norm(d, x, t[0], t[1], z);
     std::swap(x, z);
   } else {
-    // y = LN(in w^T + b + res): one launch where that is faster, the same bits. The sum of two launches stays until the layer is done, and y comes
-    // behind it: where the allocator then puts them (in the rows of qkv) they are still in the caches. With y made once and the sum freed at
-    // once, 2000 rows of MiniLM took 288 us instead of 276.
-    auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& sum, Tensor& y) {
+    // Every product's rows have a place of their own for the whole forward: a kernel that writes where the one before it read takes longer (the lines
+    // are still in other XCDs' L2, it seems). Buffers that the allocator handed on within a layer cost 4 to 10 % of MiniLM's forwards of 1000 to 4500
+    // rows (2000: 271 to 288 us by their order, now 263) and 1 to 5 % of mpnet-base's of 400 to 3000. From 56 MiB on the feed-forward rows take those
+    // of qkv, as a smaller whole counts for more: mpnet-base over 3900 / 5500 / 6500 rows 1488 / 2012 / 2108 apart, 1473 / 1983 / 2069 together.
+    const bool apart = M * (7 * H + F) * 2 <= 56L << 20;
+    const Tensor qkv_f = at::empty({M * (apart ? 3 * H : std::max(3 * H, F))}, word.options());
+    const Tensor qkv = qkv_f.narrow(0, 0, M * 3 * H).view({M, 3 * H}), f = apart ? rows(F) : qkv_f.narrow(0, 0, M * F).view({M, F});
+    const Tensor sum = rows(H);
+    Tensor y = rows(H);
+    // into = LN(in w^T + b + res): one launch where that is faster, the same bits
+    auto product_norm = [&](const Tensor& in, const Tensor* t, const Tensor& lw, const Tensor& lb, const Tensor& res, Tensor& into) {
       int first;
       if (rt_gemm_norm_rows((int)M, (int)H, (int)in.size(1), &first)) {
-        if (!y.defined()) y = rows(H);
-        check_rc(rt_gemm_norm(in.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), y.data_ptr(), (int)M,
+        check_rc(rt_gemm_norm(in.data_ptr(), t[0].data_ptr(), t[1].data_ptr(), res.data_ptr(), lw.data_ptr(), lb.data_ptr(), into.data_ptr(), (int)M,
                               (int)H, (int)in.size(1), (float)eps, 0, st),
                  "encoder: product and norm");
       } else {
-        sum = encoder_linear(in, t[0], t[1], 0);
-        if (!y.defined()) y = rows(H);
-        norm(sum, res, lw, lb, y);
+        encoder_linear(in, t[0], t[1], 0, sum);
+        norm(sum, res, lw, lb, into);
       }
     };
     for (size_t l = 0; l < layers.size(); l += 12) {
       const Tensor* t = &layers[l];
-      Tensor sum, y;
-      attend(encoder_linear(x, t[0], t[1], 0), a);
-      product_norm(a, t + 2, t[4], t[5], x, sum, y);
-      product_norm(encoder_linear(y, t[6], t[7], 2), t + 8, t[10], t[11], y, sum, x);
+      encoder_linear(x, t[0], t[1], 0, qkv);
+      attend(qkv, a);
+      product_norm(a, t + 2, t[4], t[5], x, y);
+      encoder_linear(y, t[6], t[7], 2, f);
+      product_norm(f, t + 8, t[10], t[11], y, x);
     }
   }
   check_rc(rt_pool_norm(x.data_ptr(), nullptr, (const long*)off.data_ptr(), M, (int)B, 0, (int)H, normalize ? 1 : 0,
