@@ -311,7 +311,7 @@ static bool fits(int N, int K) { return (N == 384 || N == 768) && K >= 64 && K %
 // Rows of a tile with which rt_gemm_norm beats product and norm, `first` leading rows in larger ones; 0: it doesn't, or the shape is not for it.
 // A tile is one chain over K, however few there are: with few rows the product's small tiles in parallel are faster.
 // 384 columns: 0.54 us a step of 64 rows and 6 besides (128 rows: 0.9 and 8). Even: 2500 rows at K 128, 3000 at 384, 4500 at 768, 5300 at 1536,
-// 10500 at 3072; between an encoder's other kernels not below 4000 (forwards of 3000 / 3600 / 3990 rows 362 / 387 / 392 -> 366 / 392 / 398).
+// 10500 at 3072; between an encoder's other kernels of 4000 to 5000 rows both are even at K 384 (a forward of 4500 403 us), 5500 / 8000 464 / 530 -> 456 / 510.
 // Tiles of 64 while they are one round of the CUs (16384 rows x 1536 24.7 us, tiles of 128 32.1), then 128 (17000 rows 31.7, tiles of 64 42.6),
 // whole rounds of these and the rest in 64 where that is one round more (MiniLM over 34000 rows 1434 -> 1396 us). 768 columns, us within an
 // encoder's forward (between other kernels: alone, with w in the caches, both are faster): a round of tiles of 64 takes 10 and 1.18 a step,
